@@ -1,0 +1,69 @@
+"""The choice of a token where the kernel's bins, lists and runs have their edges."""
+
+import pytest
+import torch
+
+import plain_qwen2 as plain
+
+pytestmark = pytest.mark.gpu
+
+PARAMS = [(1.0, 0, 1.0), (0.7, 1, 1.0), (0.8, 3, 1.0), (1.3, 50, 1.0), (1.0, 0, 0.0), (1.0, 0, 1e-6), (0.7, 0, 0.5),
+          (1.0, 0, 0.999999), (2.0, 40, 0.9), (0.5, 10 ** 9, 0.3), (1.0, 1, 0.5)]
+
+
+def rows_of(kind, n, vocab):
+    g = torch.Generator().manual_seed(vocab + len(kind))
+    x = torch.randn((n, vocab), generator=g)
+    if kind == "narrow":      # all within a thousandth
+        return x * 1e-3 + 7.0
+    if kind == "wide":        # most of them far below the bins' range
+        return x * 60.0
+    if kind == "equal":       # one bin cannot be told from another
+        return torch.full_like(x, -3.25)
+    if kind == "ties":        # a handful of values: more tokens in a bin than the list holds where the vocabulary is large
+        return (x * 2).round() + 0.0  # (no negative zeros: the order of the keys tells them from zero)
+    if kind == "masked":      # a few tokens allowed, the others at -inf
+        keep = torch.rand((n, vocab), generator=g) < 0.02
+        keep[:, vocab // 2] = True
+        return torch.where(keep, x, torch.tensor(float("-inf")))
+    return x * 2.5
+
+
+@pytest.mark.parametrize("kind", ["plain", "narrow", "wide", "equal", "ties", "masked"])
+@pytest.mark.parametrize("vocab", [1, 2, 63, 65, 2047, 4096, 16385, 40007])
+def test_kept_sets_and_draws(kind, vocab):
+    from from_scratch_inference_engine_amd import ops
+
+    ops.load(build_if_missing=False)
+    cases = [(t, k, p, u) for t, k, p in PARAMS for u in (0.003, 0.4999, 0.99999)]
+    logits = rows_of(kind, len(cases), vocab)
+    dev = lambda v, dt: torch.tensor(v, dtype=dt).cuda()
+    t, k, p, u = zip(*cases)
+    args = (dev(t, torch.float32), dev(k, torch.int32), dev(p, torch.float32), dev(u, torch.float64))
+    got = ops.sample(logits.cuda(), *args).cpu().tolist()
+    assert got == ops.sample(logits.cuda(), *args).cpu().tolist()  # (nothing depends on the order of the threads)
+    for i, (temp, top_k, top_p, number) in enumerate(cases):
+        want = plain.sample(logits[i], temp, top_k, top_p, number)
+        if got[i] != want:
+            # the oracle's weights are float64, the kernel's float32 exponentials of at most 2^-22 relative error
+            # (|logit difference| / temperature times 2^-24 and the function's own): a draw or an edge of the kept
+            # set within that of a boundary may fall on its other side
+            alt = {plain.sample(logits[i], temp, top_k, min(max(top_p + dp, 0.0), 1.0) if top_p < 1.0 else 1.0,
+                                min(max(number + d, 0.0), 1.0 - 1e-12))
+                   for d in (-1e-5, 0.0, 1e-5) for dp in (-1e-6, 0.0, 1e-6)}
+            assert got[i] in alt, (kind, vocab, cases[i], got[i], want)
+
+
+def test_rows_that_are_no_numbers_end():
+    """A NaN, an infinite maximum and a row of -inf give some token of the vocabulary."""
+    from from_scratch_inference_engine_amd import ops
+
+    ops.load(build_if_missing=False)
+    x = torch.randn((4, 5000), generator=torch.Generator().manual_seed(0))
+    x[0, 17] = float("nan")
+    x[1, 99] = float("inf")
+    x[2, :] = float("-inf")
+    ones = torch.ones(4).cuda()
+    out = ops.sample(x.cuda(), ones, torch.full((4,), 20, dtype=torch.int32).cuda(), 0.9 * ones,
+                     torch.full((4,), 0.5, dtype=torch.float64).cuda()).cpu()
+    assert ((out >= 0) & (out < 5000)).all() and out[1] == 99
