@@ -306,6 +306,11 @@ int fsie_attention_split_static(const void* q, int64_t q_stride, const void* k_p
 
 int fsie_sample(const float* logits, int n_rows, int vocab, const float* temperature, const int32_t* top_k,
                 const float* top_p, const double* uniform, int32_t* out, hipStream_t stream);
+// The same with every row shared by several workgroups, for vocabularies of 16,384 tokens and more:
+// `workspace` = fsie_sample_workspace(n_rows, vocab) bytes on the device (0: the call is fsie_sample's), uninitialised.
+int64_t fsie_sample_workspace(int n_rows, int vocab);
+int fsie_sample_split(const float* logits, int n_rows, int vocab, const float* temperature, const int32_t* top_k,
+                      const float* top_p, const double* uniform, void* workspace, int32_t* out, hipStream_t stream);
 
 // ---- RMS norm in groups, over a stream with up to two pending deltas ----------------------------
 // x = residual + delta_scale * (delta1 + delta2) (either delta may be null; each is [total_rows, hidden] in its own

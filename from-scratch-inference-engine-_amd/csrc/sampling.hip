@@ -18,6 +18,7 @@
 #include "api.h"
 
 #include <math.h>
+#include <stddef.h>
 
 namespace {
 
@@ -375,6 +376,71 @@ __device__ uint32_t cut_by_bisection(const float* row, int vocab, float mx, floa
     return cut;
 }
 
+// The first token, in vocabulary order, at which the running sum of the kept weights passes uniform * their sum, from the
+// sums of the runs: every wave finds the run, and the wave that owns it (`own_runs` runs a wave; -1: there is one wave)
+// walks it.
+__device__ void draw_from_runs(const float* __restrict__ row, int vocab, Best top, float inv_temp, uint32_t cut, double uniform,
+                               const double* run_sum, int own_runs, int32_t* out) {
+    const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
+    const int rows = ((vocab + FSIE_WAVE - 1) / FSIE_WAVE + kRuns - 1) / kRuns;  // 64 tokens each
+    const float mx = top.value;
+    // four neighbouring runs a lane
+    double part[kRuns / FSIE_WAVE], upto = 0.0;
+#pragma unroll
+    for (int q = 0; q < kRuns / FSIE_WAVE; ++q) {
+        part[q] = run_sum[lane * (kRuns / FSIE_WAVE) + q];
+        upto += part[q];
+    }
+#pragma unroll
+    for (int off = 1; off < FSIE_WAVE; off <<= 1) {
+        const double other = __shfl_up(upto, off, FSIE_WAVE);
+        if (lane >= off) upto += other;
+    }
+    const double total = __shfl(upto, FSIE_WAVE - 1, FSIE_WAVE);
+    const double threshold = uniform * total;
+    double before = __shfl_up(upto, 1, FSIE_WAVE);
+    if (lane == 0) before = 0.0;
+    // the first lane whose running sum passes the threshold, then the first of its runs
+    const unsigned long long past = __ballot(threshold < upto);
+    if (past == 0) {  // a NaN or no weight at all
+        if (threadIdx.x == 0) *out = top.index;
+        return;
+    }
+    const int owner = __ffsll(past) - 1;
+    int run = lane * (kRuns / FSIE_WAVE);
+    double cum = before;
+#pragma unroll
+    for (int q = 0; q < kRuns / FSIE_WAVE - 1; ++q) {
+        if (run == lane * (kRuns / FSIE_WAVE) + q && threshold >= cum + part[q]) {
+            cum += part[q];
+            ++run;
+        }
+    }
+    run = __shfl(run, owner, FSIE_WAVE);
+    cum = __shfl(cum, owner, FSIE_WAVE);
+    if (own_runs > 0 && wave != run / own_runs) return;
+    int last_kept = -1;
+    for (int j = 0; j < rows; ++j) {
+        const int64_t i = (static_cast<int64_t>(run) * rows + j) * FSIE_WAVE + lane;
+        const float v = row[i < vocab ? i : vocab - 1];
+        const bool kept = i < vocab && order_key(v) >= cut;
+        double w = kept ? token_weight(v, mx, inv_temp) : 0.0;
+#pragma unroll
+        for (int off = 1; off < FSIE_WAVE; off <<= 1) {
+            const double other = __shfl_up(w, off, FSIE_WAVE);
+            if (lane >= off) w += other;
+        }
+        const unsigned long long hit = __ballot(kept && threshold < cum + w), any = __ballot(kept);
+        if (hit) {
+            if (lane == __ffsll(hit) - 1) *out = static_cast<int>(i);
+            return;
+        }
+        if (any) last_kept = static_cast<int>((static_cast<int64_t>(run) * rows + j) * FSIE_WAVE) + 63 - __clzll(any);
+        cum += __shfl(w, FSIE_WAVE - 1, FSIE_WAVE);
+    }
+    if (lane == 0) *out = last_kept >= 0 ? last_kept : top.index;  // rounding at the run's end
+}
+
 __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restrict__ logits, int vocab,
                                                           const float* __restrict__ temperature,
                                                           const int32_t* __restrict__ top_k,
@@ -435,64 +501,495 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
         if (lane == 0) run_sum[run] = mine;
     }
     __syncthreads();
-    // every wave finds the run by itself: four neighbouring runs a lane
-    double part[kRuns / FSIE_WAVE], upto = 0.0;
+    draw_from_runs(row, vocab, top, inv_temp, cut, uniform[r], run_sum, kRunsOfWave, out + r);
+}
+
+// ---- a row shared by several workgroups -------------------------------------------------------
+// One workgroup a row leaves three quarters of the chip idle at 64 rows and all but one unit at one row, and a unit
+// needs some 10 us for every pass over 152,064 tokens (their exponentials and the adds in float64).  From kSplitFrom
+// tokens on the row's runs are dealt to up to 64 workgroups, and the passes become launches: the maximum; bins (or,
+// for rows without a threshold, the draw's sums); the threshold bins' tokens; the cut; the draw's sums; the draw.
+// What a launch leaves for the next lies in a workspace of the row.
+constexpr int kSplitFrom = 16384;
+constexpr int kPart = 256;          // threads of a shared row's workgroups
+constexpr int kMaxParts = 64;
+constexpr int kPairs = 512;         // so many listed tokens are compared with each other, more are bisected
+constexpr int kKeep = 4096;         // tokens that the list holds
+
+struct SplitRow {
+    unsigned long long hi[kBins], lo[kBins];
+    double run_sum[kRuns];
+    unsigned int count[kBins];
+    unsigned int n_listed, cut;     // (behind the bins: cleared with them)
+    unsigned int pad[2];
+    float listed[kKeep];
+    float part_max[kMaxParts], part_low[kMaxParts];
+    int part_index[kMaxParts], part_nan[kMaxParts];
+};
+static_assert(sizeof(SplitRow) % 16 == 0, "rows of the workspace stay aligned");
+
+struct RowParams {
+    float temp, inv_temp, p;
+    int k;
+    bool cuts;
+};
+__device__ __forceinline__ RowParams row_params(int r, int vocab, const float* temperature, const int32_t* top_k,
+                                                const float* top_p) {
+    RowParams q;
+    q.temp = temperature ? temperature[r] : 0.f;
+    q.inv_temp = 1.0f / q.temp;
+    q.k = top_k && top_k[r] > 0 && top_k[r] < vocab ? top_k[r] : 0;
+    q.p = top_p ? top_p[r] : 1.f;
+    q.cuts = q.temp > 0.f && (q.k > 0 || q.p < 1.f);
+    return q;
+}
+
+// The row's maximum and its place, the smallest value above -inf, whether a NaN is in it: from the parts', by a wave.
+struct RowTop {
+    Best best;
+    float low;
+    bool nan;
+    // whether the row's thresholds can be found by bins, and their scale
+    __device__ bool binned(int vocab, float* scale) const {
+        const float range = fminf(best.value - low, kRange);
+        if (vocab > kMaxBinned || nan || !(fabsf(best.value) < INFINITY) || !(range > 1e-30f)) return false;
+        *scale = static_cast<float>(kBins - 1) / range;
+        return true;
+    }
+};
+__device__ RowTop row_top(const SplitRow* w, int parts) {
+    const int lane = threadIdx.x & (FSIE_WAVE - 1), at = min(lane, parts - 1);
+    RowTop t{Best{w->part_max[at], w->part_index[at]}, w->part_low[at], w->part_nan[at] != 0};
 #pragma unroll
-    for (int q = 0; q < kRuns / FSIE_WAVE; ++q) {
-        part[q] = run_sum[lane * (kRuns / FSIE_WAVE) + q];
-        upto += part[q];
+    for (int off = FSIE_WAVE / 2; off > 0; off >>= 1) {
+        t.best = better(t.best, Best{__shfl_xor(t.best.value, off, FSIE_WAVE), __shfl_xor(t.best.index, off, FSIE_WAVE)});
+        t.low = fminf(t.low, __shfl_xor(t.low, off, FSIE_WAVE));
+    }
+    t.nan = __any(t.nan);
+    return t;
+}
+
+// 64-token lines of a run, and the tokens of part `part`
+__device__ __forceinline__ int run_lines(int vocab) {
+    return ((vocab + FSIE_WAVE - 1) / FSIE_WAVE + kRuns - 1) / kRuns;
+}
+__device__ __forceinline__ void part_range(int vocab, int parts, int part, int* begin, int* end) {
+    const int64_t tokens = static_cast<int64_t>(run_lines(vocab)) * FSIE_WAVE * (kRuns / parts);
+    *begin = static_cast<int>(min(static_cast<int64_t>(vocab), tokens * part));
+    *end = static_cast<int>(min(static_cast<int64_t>(vocab), tokens * (part + 1)));
+}
+
+template <typename F>
+__device__ __forceinline__ void for_part(const float* __restrict__ row, int begin, int end, F body) {
+    for (int i0 = begin + threadIdx.x; i0 < end; i0 += kPart * kUnroll) {
+        float v[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) v[u] = row[min(i0 + u * kPart, end - 1)];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u)
+            if (i0 + u * kPart < end) body(v[u], i0 + u * kPart);
+    }
+}
+
+// The kept weights of the part's runs, a run a wave at a time, in the order of the lanes.
+__device__ void add_runs(const float* __restrict__ row, int vocab, int parts, int part, float mx, float inv_temp,
+                         uint32_t cut, double* run_sum) {
+    const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
+    const int lines = run_lines(vocab), per_part = kRuns / parts;
+    for (int q = wave; q < per_part; q += kPart / FSIE_WAVE) {
+        const int run = part * per_part + q;
+        const int64_t first = static_cast<int64_t>(run) * lines * FSIE_WAVE + lane;
+        double mine = 0.0;
+        for (int j0 = 0; j0 < lines; j0 += kUnroll) {
+            float v[kUnroll];
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u)
+                v[u] = row[min(first + static_cast<int64_t>(min(j0 + u, lines - 1)) * FSIE_WAVE, static_cast<int64_t>(vocab - 1))];
+#pragma unroll
+            for (int u = 0; u < kUnroll; ++u)
+                if (j0 + u < lines && first + static_cast<int64_t>(j0 + u) * FSIE_WAVE < vocab && order_key(v[u]) >= cut)
+                    mine += token_weight(v[u], mx, inv_temp);
+        }
+        mine = wave_sum_f64(mine);
+        if (lane == 0) run_sum[run] = mine;
+    }
+}
+
+__global__ __launch_bounds__(kPart) void split_top_kernel(const float* __restrict__ logits, int vocab, int parts, SplitRow* ws) {
+    __shared__ float sval[kPart / FSIE_WAVE], slow[kPart / FSIE_WAVE];
+    __shared__ int sidx[kPart / FSIE_WAVE], snan[kPart / FSIE_WAVE];
+    SplitRow* w = ws + blockIdx.y;
+    const int part = blockIdx.x, lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
+    // the bins and counters of the row are this launch's to clear
+    uint32_t* bins = reinterpret_cast<uint32_t*>(w->hi);
+    constexpr int kClear = static_cast<int>(offsetof(SplitRow, listed) / 4);
+    for (int i = part * kPart + threadIdx.x; i < kClear; i += parts * kPart) bins[i] = 0;
+    int begin, end;
+    part_range(vocab, parts, part, &begin, &end);
+    Best best{-INFINITY, 0x7fffffff};
+    float low = INFINITY;
+    bool nan = false;
+    for_part(logits + static_cast<int64_t>(blockIdx.y) * vocab, begin, end, [&](float v, int i) {
+        nan |= v != v;
+        if (v > -INFINITY) low = fminf(low, v);
+        if (best.index == 0x7fffffff || v > best.value) best = Best{v, i};
+    });
+#pragma unroll
+    for (int off = FSIE_WAVE / 2; off > 0; off >>= 1) {
+        best = better(best, Best{__shfl_xor(best.value, off, FSIE_WAVE), __shfl_xor(best.index, off, FSIE_WAVE)});
+        low = fminf(low, __shfl_xor(low, off, FSIE_WAVE));
+    }
+    nan = __any(nan);
+    if (lane == 0) {
+        sval[wave] = best.value;
+        sidx[wave] = best.index;
+        slow[wave] = low;
+        snan[wave] = nan;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < kPart / FSIE_WAVE; ++i) {
+            best = better(best, Best{sval[i], sidx[i]});
+            low = fminf(low, slow[i]);
+            nan = nan || snan[i];
+        }
+        w->part_max[part] = best.value;
+        w->part_index[part] = best.index;
+        w->part_low[part] = low;
+        w->part_nan[part] = nan;
+    }
+}
+
+__global__ __launch_bounds__(kPart) void split_bins_kernel(const float* __restrict__ logits, int vocab, int parts,
+                                                           const float* __restrict__ temperature,
+                                                           const int32_t* __restrict__ top_k,
+                                                           const float* __restrict__ top_p, SplitRow* ws) {
+    __shared__ unsigned long long hi[kBins], lo[kBins];
+    __shared__ unsigned int count[kBins];
+    const int r = blockIdx.y;
+    const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
+    if (!(q.temp > 0.f)) return;
+    SplitRow* w = ws + r;
+    const RowTop top = row_top(w, parts);
+    const float* row = logits + static_cast<int64_t>(r) * vocab;
+    const float mx = top.best.value;
+    if (!q.cuts) {
+        add_runs(row, vocab, parts, blockIdx.x, mx, q.inv_temp, 0, w->run_sum);
+        return;
+    }
+    float scale;
+    if (!top.binned(vocab, &scale)) return;
+    for (int b = threadIdx.x; b < kBins; b += kPart) {
+        hi[b] = lo[b] = 0;
+        count[b] = 0;
+    }
+    __syncthreads();
+    const int hi_bits = 63 - (32 - __clz(vocab));  // vocab < 2^(32 - clz): the sum of all weights stays below 2^63
+    int begin, end;
+    part_range(vocab, parts, blockIdx.x, &begin, &end);
+    for_part(row, begin, end, [&](float v, int) {
+        const int b = bin_of(v, mx, scale);
+        atomicAdd(&count[b], 1u);
+        if (q.p < 1.f) {
+            const Limbs m = limbs_of(expf((v - mx) * q.inv_temp), hi_bits);
+            if (m.hi) atomicAdd(&hi[b], m.hi);
+            if (m.lo) atomicAdd(&lo[b], m.lo);
+        }
+    });
+    __syncthreads();
+    for (int b = threadIdx.x; b < kBins; b += kPart) {
+        if (!count[b]) continue;
+        atomicAdd(&w->count[b], count[b]);
+        if (hi[b]) atomicAdd(&w->hi[b], hi[b]);
+        if (lo[b]) atomicAdd(&w->lo[b], lo[b]);
+    }
+}
+
+// The running sums of the bins' values from the maximum down, found by a workgroup of THREADS: where `target` is first
+// reached, and the sum above that bin.
+struct Found {
+    int bin;       // -1: nowhere
+    double above, total;
+};
+template <int THREADS, typename F>
+__device__ Found find_in_bins(double target, F value) {
+    constexpr int PER = kBins / THREADS;
+    __shared__ double wave_sum[THREADS / FSIE_WAVE];
+    __shared__ Found found;
+    const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
+    double v[PER], run = 0.0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        v[i] = value(static_cast<int>(threadIdx.x) * PER + i);
+        run += v[i];
     }
 #pragma unroll
     for (int off = 1; off < FSIE_WAVE; off <<= 1) {
-        const double other = __shfl_up(upto, off, FSIE_WAVE);
-        if (lane >= off) upto += other;
+        const double other = __shfl_up(run, off, FSIE_WAVE);
+        if (lane >= off) run += other;
     }
-    const double total = __shfl(upto, FSIE_WAVE - 1, FSIE_WAVE);
-    const double threshold = uniform[r] * total;
-    double before = __shfl_up(upto, 1, FSIE_WAVE);
-    if (lane == 0) before = 0.0;
-    // the first lane whose running sum passes the threshold, then the first of its runs
-    const unsigned long long past = __ballot(threshold < upto);
-    if (past == 0) {  // a NaN or no weight at all
+    __syncthreads();
+    if (lane == FSIE_WAVE - 1) wave_sum[wave] = run;
+    if (threadIdx.x == 0) found.bin = -1;
+    __syncthreads();
+    double base = 0.0, total = 0.0;
+    for (int i = 0; i < THREADS / FSIE_WAVE; ++i) {
+        if (i == wave) base = total;
+        total += wave_sum[i];
+    }
+    const double left = __shfl_up(run, 1, FSIE_WAVE);  // (all lanes together: a shuffle reads active lanes only)
+    double before = base + (lane ? left : 0.0);
+    if (before < target && target <= base + run) {
+        int bin = static_cast<int>(threadIdx.x) * PER;
+#pragma unroll
+        for (int i = 0; i < PER - 1; ++i)
+            if (bin == static_cast<int>(threadIdx.x) * PER + i && target > before + v[i]) {
+                before += v[i];
+                ++bin;
+            }
+        found.bin = bin;
+        found.above = before;
+    }
+    __syncthreads();
+    const Found out{found.bin, found.above, total};
+    __syncthreads();
+    return out;
+}
+
+__global__ __launch_bounds__(kPart) void split_list_kernel(const float* __restrict__ logits, int vocab, int parts,
+                                                           const float* __restrict__ temperature,
+                                                           const int32_t* __restrict__ top_k,
+                                                           const float* __restrict__ top_p, SplitRow* ws) {
+    const int r = blockIdx.y;
+    const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
+    if (!q.cuts) return;
+    SplitRow* w = ws + r;
+    const RowTop top = row_top(w, parts);
+    float scale;
+    if (!top.binned(vocab, &scale)) return;
+    const int hi_bits = 63 - (32 - __clz(vocab));
+    const auto weight = [&](int b) { return value_of(Limbs{w->hi[b], w->lo[b]}, hi_bits); };
+    int k_bin = -1, from = 0, upto = -1;
+    if (q.k > 0) k_bin = find_in_bins<kPart>(q.k, [&](int b) { return static_cast<double>(w->count[b]); }).bin;
+    if (q.p < 1.f) {
+        // top p of what top k keeps: all of the bins above its own and some of that one, so the last kept token lies
+        // between the bins that the least and the most of it give
+        const double most = find_in_bins<kPart>(INFINITY, [&](int b) { return k_bin < 0 || b <= k_bin ? weight(b) : 0.0; }).total;
+        double least = most;
+        if (k_bin >= 0) least = find_in_bins<kPart>(INFINITY, [&](int b) { return b < k_bin ? weight(b) : 0.0; }).total;
+        const double p = static_cast<double>(q.p);
+        if (p > 0.0) {
+            from = max(0, find_in_bins<kPart>(p * least, weight).bin);
+            upto = find_in_bins<kPart>(p * most, weight).bin;
+        }
+    }
+    int begin, end;
+    part_range(vocab, parts, blockIdx.x, &begin, &end);
+    for_part(logits + static_cast<int64_t>(r) * vocab, begin, end, [&](float v, int) {
+        const int b = bin_of(v, top.best.value, scale);
+        if (b == k_bin || (from <= b && b <= upto)) {
+            const unsigned int at = atomicAdd(&w->n_listed, 1u);
+            if (at < kKeep) w->listed[at] = v;
+        }
+    });
+}
+
+// The key of the first listed token, from the largest down, at which reached(key's tokens and all larger) holds, by
+// bisection over the keys; what is summed are integers, so the list's order does not matter.
+template <typename S, typename F>
+__device__ uint32_t bisect_list(const uint32_t* keys, int n, uint32_t key_max, S value, F reached) {
+    __shared__ unsigned long long sum_hi, sum_lo;
+    uint32_t lo = 0, hi = key_max;
+    while (lo < hi) {
+        const uint32_t mid = lo + (hi - lo) / 2 + ((hi - lo) & 1);
+        __syncthreads();
+        if (threadIdx.x == 0) sum_hi = sum_lo = 0;
+        __syncthreads();
+        Limbs mine{0, 0};
+        for (int i = threadIdx.x; i < n; i += kThreads)
+            if (keys[i] >= mid) {
+                const Limbs v = value(i);
+                mine.hi += v.hi;
+                mine.lo += v.lo;
+            }
+        if (mine.hi) atomicAdd(&sum_hi, mine.hi);
+        if (mine.lo) atomicAdd(&sum_lo, mine.lo);
+        __syncthreads();
+        if (reached(Limbs{sum_hi, sum_lo})) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+__global__ __launch_bounds__(kThreads) void split_cut_kernel(const float* __restrict__ logits, int vocab, int parts,
+                                                             const float* __restrict__ temperature,
+                                                             const int32_t* __restrict__ top_k,
+                                                             const float* __restrict__ top_p, SplitRow* ws) {
+    __shared__ uint32_t keys[kKeep];
+    __shared__ short bin_of_key[kKeep];
+    __shared__ unsigned long long w_hi[kPairs], w_lo[kPairs];
+    __shared__ double sdbl[kWaves];
+    __shared__ unsigned long long kept_hi, kept_lo;
+    __shared__ uint32_t cut_found;
+    __shared__ unsigned int of_bin;
+    const int r = blockIdx.x;
+    const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
+    if (!q.cuts) return;
+    SplitRow* w = ws + r;
+    const RowTop top = row_top(w, parts);
+    const float* row = logits + static_cast<int64_t>(r) * vocab;
+    const float mx = top.best.value;
+    const uint32_t key_max = order_key(mx);
+    const int n = static_cast<int>(min(w->n_listed, static_cast<unsigned int>(kKeep + 1)));
+    float scale = 0.f;
+    bool fits = top.binned(vocab, &scale) && n <= kKeep;  // (the same in every thread)
+    uint32_t cut = 0;
+    if (fits) {
+        const int hi_bits = 63 - (32 - __clz(vocab));
+        for (int i = threadIdx.x; i < n; i += kThreads) {
+            const float v = w->listed[i];
+            keys[i] = order_key(v);
+            bin_of_key[i] = static_cast<short>(bin_of(v, mx, scale));
+            if (i < kPairs) {
+                const Limbs m = limbs_of(expf((v - mx) * q.inv_temp), hi_bits);
+                w_hi[i] = m.hi;
+                w_lo[i] = m.lo;
+            }
+        }
+        const auto listed_weight = [&](int i) {
+            if (i < kPairs) return Limbs{w_hi[i], w_lo[i]};
+            return limbs_of(expf((w->listed[i] - mx) * q.inv_temp), hi_bits);
+        };
+        if (threadIdx.x == 0) {
+            kept_hi = kept_lo = 0;
+            cut_found = 0;
+            of_bin = 0;
+        }
+        __syncthreads();
+        int k_bin = -1;
+        if (q.k > 0) {
+            const Found at = find_in_bins<kThreads>(q.k, [&](int b) { return static_cast<double>(w->count[b]); });
+            k_bin = at.bin;
+            const long long want = q.k - static_cast<long long>(at.above);
+            if (k_bin < 0) {
+                fits = false;
+            } else if (n <= kPairs) {
+                if (static_cast<int>(threadIdx.x) < n && bin_of_key[threadIdx.x] == k_bin) {
+                    const uint32_t mine = keys[threadIdx.x];
+                    int over = 0, upto = 0;
+                    for (int j = 0; j < n; ++j) {
+                        const bool same = bin_of_key[j] == k_bin;
+                        over += same && keys[j] > mine;
+                        upto += same && keys[j] >= mine;
+                    }
+                    if (over < want && want <= upto) cut_found = mine;  // (equal keys write the same)
+                }
+                __syncthreads();
+                cut = cut_found;
+            } else {
+                cut = bisect_list(keys, n, key_max, [&](int i) { return Limbs{bin_of_key[i] == k_bin, 0}; },
+                                  [&](Limbs s) { return static_cast<long long>(s.hi) >= want; });
+            }
+            if (cut == 0) fits = false;
+        }
+        if (fits && q.p < 1.f) {
+            __syncthreads();
+            Limbs kept{0, 0};  // of top k's bin
+            for (int i = threadIdx.x; i < n; i += kThreads)
+                if (bin_of_key[i] == k_bin && keys[i] >= cut) {
+                    const Limbs m = listed_weight(i);
+                    kept.hi += m.hi;
+                    kept.lo += m.lo;
+                }
+            if (kept.hi) atomicAdd(&kept_hi, kept.hi);
+            if (kept.lo) atomicAdd(&kept_lo, kept.lo);
+            if (threadIdx.x == 0) cut_found = 0;
+            __syncthreads();
+            const auto weight = [&](int b) {
+                if (k_bin >= 0 && b >= k_bin) return b == k_bin ? value_of(Limbs{kept_hi, kept_lo}, hi_bits) : 0.0;
+                return value_of(Limbs{w->hi[b], w->lo[b]}, hi_bits);
+            };
+            const double target = static_cast<double>(q.p) * find_in_bins<kThreads>(INFINITY, weight).total;
+            if (!(target > 0.0)) {
+                cut = key_max;
+            } else {
+                const Found at = find_in_bins<kThreads>(target, weight);
+                const auto counts = [&](int i) { return bin_of_key[i] == at.bin && keys[i] >= cut; };
+                const auto reaches = [&](Limbs s) { return target <= at.above + value_of(s, hi_bits); };
+                // (rounding may have put the target outside the bins that were listed)
+                unsigned int mine_of_bin = 0;
+                for (int i = threadIdx.x; i < n; i += kThreads) mine_of_bin += bin_of_key[i] == at.bin;
+                if (mine_of_bin) atomicAdd(&of_bin, mine_of_bin);
+                __syncthreads();
+                uint32_t found = 0;
+                if (at.bin < 0 || of_bin != w->count[max(at.bin, 0)]) {
+                    fits = false;
+                } else if (n <= kPairs) {
+                    if (static_cast<int>(threadIdx.x) < n && counts(threadIdx.x)) {
+                        const uint32_t mine = keys[threadIdx.x];
+                        Limbs over{0, 0}, upto{0, 0};
+                        for (int j = 0; j < n; ++j) {
+                            if (!counts(j) || keys[j] < mine) continue;
+                            upto.hi += w_hi[j];
+                            upto.lo += w_lo[j];
+                            if (keys[j] > mine) {
+                                over.hi += w_hi[j];
+                                over.lo += w_lo[j];
+                            }
+                        }
+                        if (!reaches(over) && reaches(upto)) cut_found = mine;
+                    }
+                    __syncthreads();
+                    found = cut_found;
+                } else {
+                    found = bisect_list(keys, n, key_max, [&](int i) { return counts(i) ? listed_weight(i) : Limbs{0, 0}; }, reaches);
+                }
+                if (found == 0) fits = false;
+                cut = found;
+            }
+        }
+    }
+    if (!fits) {
+        __syncthreads();
+        cut = cut_by_bisection(row, vocab, mx, q.inv_temp, q.k, q.p, sdbl);
+    }
+    if (threadIdx.x == 0) w->cut = cut;
+}
+
+__global__ __launch_bounds__(kPart) void split_runs_kernel(const float* __restrict__ logits, int vocab, int parts,
+                                                           const float* __restrict__ temperature,
+                                                           const int32_t* __restrict__ top_k,
+                                                           const float* __restrict__ top_p, SplitRow* ws) {
+    const int r = blockIdx.y;
+    const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
+    if (!q.cuts) return;  // (rows without a threshold have their sums already)
+    SplitRow* w = ws + r;
+    add_runs(logits + static_cast<int64_t>(r) * vocab, vocab, parts, blockIdx.x, row_top(w, parts).best.value, q.inv_temp,
+             w->cut, w->run_sum);
+}
+
+__global__ __launch_bounds__(FSIE_WAVE) void split_draw_kernel(const float* __restrict__ logits, int vocab, int parts,
+                                                               const float* __restrict__ temperature,
+                                                               const int32_t* __restrict__ top_k,
+                                                               const float* __restrict__ top_p,
+                                                               const double* __restrict__ uniform, const SplitRow* ws,
+                                                               int32_t* __restrict__ out) {
+    const int r = blockIdx.x;
+    const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
+    const SplitRow* w = ws + r;
+    const Best top = row_top(w, parts).best;
+    if (!(q.temp > 0.f)) {
         if (threadIdx.x == 0) out[r] = top.index;
         return;
     }
-    const int owner = __ffsll(past) - 1;
-    int run = lane * (kRuns / FSIE_WAVE);
-    double cum = before;
-#pragma unroll
-    for (int q = 0; q < kRuns / FSIE_WAVE - 1; ++q) {
-        if (run == lane * (kRuns / FSIE_WAVE) + q && threshold >= cum + part[q]) {
-            cum += part[q];
-            ++run;
-        }
-    }
-    run = __shfl(run, owner, FSIE_WAVE);
-    cum = __shfl(cum, owner, FSIE_WAVE);
-    if (wave != run / kRunsOfWave) return;
-    int last_kept = -1;
-    for (int j = 0; j < rows; ++j) {
-        const int64_t i = (static_cast<int64_t>(run) * rows + j) * FSIE_WAVE + lane;
-        const float v = row[i < vocab ? i : vocab - 1];
-        const bool kept = i < vocab && order_key(v) >= cut;
-        double w = kept ? token_weight(v, mx, inv_temp) : 0.0;
-#pragma unroll
-        for (int off = 1; off < FSIE_WAVE; off <<= 1) {
-            const double other = __shfl_up(w, off, FSIE_WAVE);
-            if (lane >= off) w += other;
-        }
-        const unsigned long long hit = __ballot(kept && threshold < cum + w), any = __ballot(kept);
-        if (hit) {
-            if (lane == __ffsll(hit) - 1) out[r] = static_cast<int>(i);
-            return;
-        }
-        if (any) last_kept = static_cast<int>((static_cast<int64_t>(run) * rows + j) * FSIE_WAVE) + 63 - __clzll(any);
-        cum += __shfl(w, FSIE_WAVE - 1, FSIE_WAVE);
-    }
-    if (lane == 0) out[r] = last_kept >= 0 ? last_kept : top.index;  // rounding at the run's end
+    draw_from_runs(logits + static_cast<int64_t>(r) * vocab, vocab, top, q.inv_temp, q.cuts ? w->cut : 0, uniform[r],
+                   w->run_sum, -1, out + r);
 }
 
 }  // namespace
+
+extern "C" int64_t fsie_sample_workspace(int n_rows, int vocab) {
+    return vocab >= kSplitFrom && n_rows > 0 ? static_cast<int64_t>(n_rows) * static_cast<int64_t>(sizeof(SplitRow)) : 0;
+}
 
 extern "C" int fsie_sample(const float* logits, int n_rows, int vocab, const float* temperature,
                            const int32_t* top_k, const float* top_p, const double* uniform, int32_t* out,
@@ -502,5 +999,31 @@ extern "C" int fsie_sample(const float* logits, int n_rows, int vocab, const flo
     if (n_rows == 0) return 0;
     sample_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, temperature, top_k, top_p, uniform, out);
     FSIE_CHECK_LAUNCH("sample");
+    return 0;
+}
+
+extern "C" int fsie_sample_split(const float* logits, int n_rows, int vocab, const float* temperature, const int32_t* top_k,
+                                 const float* top_p, const double* uniform, void* workspace, int32_t* out,
+                                 hipStream_t stream) {
+    FSIE_REQUIRE(n_rows > 0 && n_rows <= 65535 && vocab > 0, "sample_split: bad sizes rows=%d vocab=%d", n_rows, vocab);
+    FSIE_REQUIRE(!temperature || uniform, "sample_split: temperatures given without uniform numbers");
+    FSIE_REQUIRE(workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
+                 "sample_split: a workspace on 16 bytes is needed");
+    SplitRow* ws = static_cast<SplitRow*>(workspace);
+    // a power of two of parts that gives every compute unit about four workgroups
+    int parts = 1;
+    while (parts < kMaxParts && n_rows * parts < 1024) parts *= 2;
+    const dim3 grid(parts, n_rows);
+    split_top_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, ws);
+    if (temperature) {
+        split_bins_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
+        if (top_k || top_p) {
+            split_list_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
+            split_cut_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
+            split_runs_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
+        }
+    }
+    split_draw_kernel<<<n_rows, FSIE_WAVE, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, uniform, ws, out);
+    FSIE_CHECK_LAUNCH("sample_split");
     return 0;
 }

@@ -940,6 +940,12 @@ def sample(logits: torch.Tensor, temperature: Optional[torch.Tensor] = None,
     if out is None:
         out = torch.empty((n,), dtype=torch.int32, device=logits.device)
     _need(out, "sample out", dtype=torch.int32, shape=(n,))
+    size = int(load().fsie_sample_workspace(n, v))
+    if size:  # a large vocabulary: every row is shared by several workgroups, which meet in a workspace
+        work = torch.empty((size,), dtype=torch.uint8, device=logits.device)
+        check(load().fsie_sample_split(logits.data_ptr(), n, v, _ptr(temperature), _ptr(top_k), _ptr(top_p),
+                                       _ptr(uniform), work.data_ptr(), out.data_ptr(), _stream()))
+        return out
     check(load().fsie_sample(logits.data_ptr(), n, v, _ptr(temperature), _ptr(top_k), _ptr(top_p),
                              _ptr(uniform), out.data_ptr(), _stream()))
     return out

@@ -120,6 +120,8 @@ _SIGNATURES = {
     "fsie_moe_tile_rows": ([c_int, c_int], c_int),
     "fsie_moe_combine": ([_P, _P, _P, c_int, c_int, c_int, _P, c_int, c_int, _P], c_int),
     "fsie_sample": ([_P, c_int, c_int, _P, _P, _P, _P, _P, _P], c_int),
+    "fsie_sample_workspace": ([c_int, c_int], c_int64),
+    "fsie_sample_split": ([_P, c_int, c_int, _P, _P, _P, _P, _P, _P, _P], c_int),
 }
 
 

@@ -22,6 +22,8 @@ def rows_of(kind, n, vocab):
         return torch.full_like(x, -3.25)
     if kind == "ties":        # a handful of values: more tokens in a bin than the list holds where the vocabulary is large
         return (x * 2).round() + 0.0  # (no negative zeros: the order of the keys tells them from zero)
+    if kind == "coarse":      # hundreds of tokens of one value: more than are compared with each other
+        return (x * 10).round() / 4 + 0.0
     if kind == "masked":      # a few tokens allowed, the others at -inf
         keep = torch.rand((n, vocab), generator=g) < 0.02
         keep[:, vocab // 2] = True
@@ -29,7 +31,7 @@ def rows_of(kind, n, vocab):
     return x * 2.5
 
 
-@pytest.mark.parametrize("kind", ["plain", "narrow", "wide", "equal", "ties", "masked"])
+@pytest.mark.parametrize("kind", ["plain", "narrow", "wide", "equal", "ties", "coarse", "masked"])
 @pytest.mark.parametrize("vocab", [1, 2, 63, 65, 2047, 4096, 16385, 40007])
 def test_kept_sets_and_draws(kind, vocab):
     from from_scratch_inference_engine_amd import ops
@@ -67,3 +69,20 @@ def test_rows_that_are_no_numbers_end():
     out = ops.sample(x.cuda(), ones, torch.full((4,), 20, dtype=torch.int32).cuda(), 0.9 * ones,
                      torch.full((4,), 0.5, dtype=torch.float64).cuda()).cpu()
     assert ((out >= 0) & (out < 5000)).all() and out[1] == 99
+
+
+@pytest.mark.parametrize("rows", [1, 3, 64, 1100])
+def test_a_row_does_not_depend_on_how_many_workgroups_share_it(rows):
+    from from_scratch_inference_engine_amd import ops
+
+    ops.load(build_if_missing=False)
+    g = torch.Generator().manual_seed(rows)
+    x = (torch.randn((rows, 16500), generator=g) * 2.5).cuda()
+    kinds = [(0.0, 0, 1.0), (1.0, 0, 1.0), (0.8, 50, 1.0), (0.7, 0, 0.9), (1.0, 200, 0.95)]
+    t, k, p = zip(*[kinds[i % 5] for i in range(rows)])
+    args = [torch.tensor(t).cuda(), torch.tensor(k, dtype=torch.int32).cuda(), torch.tensor(p).cuda(),
+            torch.rand((rows,), generator=g, dtype=torch.float64).cuda()]
+    got = ops.sample(x, *args)
+    for i in sorted({0, rows // 2, rows - 1, min(rows - 1, 4)}):
+        assert got[i] == ops.sample(x[i:i + 1].contiguous(), *[a[i:i + 1].contiguous() for a in args])[0]
+    assert torch.equal(ops.sample(x), x.argmax(1).to(torch.int32))
