@@ -221,6 +221,16 @@ int fsie_gemm_mfma_skinny_act(const void* x, const void* w, const float* bias, v
 int fsie_gemm_mfma_wide_act(const void* x, const void* w, const float* bias, void* y, int M, int N, int K, int waves,
                             int blocks, int frags, int act, float act_pos, float act_neg, hipStream_t stream);
 int fsie_gemm_mfma_wide_act_takes(int M, int N, int K);
+
+// Products of many rows (prompts), bfloat16 x [M, K] and w [N, K], N a multiple of 16, K of 64, 16-byte aligned:
+//   result 1: gate and up rows of w in turn, y bfloat16 [M, N/2] (act as for fsie_gemm_mfma_wide_gated)
+//   result 2: y float32 partial sums [splits][M][N] of slices of K;  result 0: y bfloat16 [M, N]
+// tile 0 .. 3: 128 x 256, 256 x 192, 256 x 256, 256 x 320 rows of x by rows of w a workgroup.
+// fsie_gemm_mfma_tile_plan: tile + 256 * splits, or -1 where the library's product is the faster one.
+int fsie_gemm_mfma_tile_plan(int M, int N, int K, int result, int units);
+int fsie_gemm_mfma_tile(const void* x, const void* w, void* y, int M, int N, int K, int result, int splits, int tile,
+                        int act, float act_pos, float act_neg, hipStream_t stream);
+
 int64_t fsie_fragment_order_size(int N, int K);
 int fsie_fragment_order(const void* w, void* out, int N, int K, hipStream_t stream);
 

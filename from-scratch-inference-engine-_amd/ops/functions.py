@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import ctypes
 
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -552,6 +553,45 @@ def gemm_mfma_wide_swiglu(x: torch.Tensor, weight: torch.Tensor, waves: int = 0,
     _need(out, "gemm out", dtype=torch.bfloat16, shape=(m, n // 2))
     check(load().fsie_gemm_mfma_wide_gated(x.data_ptr(), wptr, out.data_ptr(), m, n, k, waves, blocks, frags,
                                            *gate_act(act).args, _stream()))
+    return out
+
+
+def gemm_mfma_tile(x: torch.Tensor, weight: torch.Tensor, splits: int = 1, tile: int = 2) -> torch.Tensor:
+    """Float32 partial sums [splits, M, N] of x [M, K] . weight [N, K]^T (bfloat16) over slices of K, by the kernel for
+    many rows (N a multiple of 16, K of 64); ``tile``: its tile's shape (``gemm_tile_plan`` chooses both)."""
+    return _gemm_tile(x, weight, GEMM_TILE_SUMS, splits, tile, None)
+
+
+def gemm_mfma_tile_gated(x: torch.Tensor, weight: torch.Tensor, act="silu", tile: int = 2) -> torch.Tensor:
+    """The products of gate and up value (``act``: a ``GateAct`` or its name) [M, N/2] in bfloat16 of x [M, K] and a weight
+    [N, K] whose rows are gate and up in turn, by the kernel for many rows (N a multiple of 16, K of 64)."""
+    return _gemm_tile(x, weight, GEMM_TILE_PAIR, 1, tile, gate_act(act))
+
+
+GEMM_TILE_PAIR, GEMM_TILE_SUMS = 1, 2
+
+
+@lru_cache(maxsize=4096)
+def gemm_tile_plan(m: int, n: int, k: int, result: int):
+    """(tile, slices of K) for ``gemm_mfma_tile_gated`` (``result`` = GEMM_TILE_PAIR) or ``gemm_mfma_tile`` (GEMM_TILE_SUMS) at
+    these sizes; None where the library's product is faster or the kernel does not take them."""
+    choice = int(load().fsie_gemm_mfma_tile_plan(m, n, k, result, compute_units()))
+    return None if choice < 0 else (choice % 256, choice // 256)
+
+
+def _gemm_tile(x, weight, result: int, splits: int, tile: int, act) -> torch.Tensor:
+    _need(x, "gemm x", dtype=torch.bfloat16, ndim=2)
+    _need(weight, "gemm weight", dtype=torch.bfloat16, ndim=2)
+    m, k = x.shape
+    n = weight.shape[0]
+    if weight.shape[1] != k:
+        raise KernelError(f"gemm_mfma_tile: x has {k} columns, weight has {weight.shape[1]}")
+    if result == GEMM_TILE_SUMS:
+        out = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+    else:
+        out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
+    check(load().fsie_gemm_mfma_tile(x.data_ptr(), weight.data_ptr(), out.data_ptr(), m, n, k, result, splits, tile,
+                                     *(act.args if act is not None else (0, 0.0, 0.0)), _stream()))
     return out
 
 

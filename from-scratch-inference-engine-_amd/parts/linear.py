@@ -160,6 +160,12 @@ class Linear:
             splits = self.residual_splits(m)
             if splits > 1:
                 return ops.gemm_mfma_skinny(x, self.weight, splits=splits)
+        if (getattr(ctx, "partial_sums_ok", False) and x.dtype == torch.bfloat16 and self.bias is None
+                and m > GEMM_MFMA_WIDE_MAX_M):
+            # prompts and a long K: the product for many rows in slices of K
+            plan = ops.gemm_tile_plan(m, self.out_features, self.in_features, ops.GEMM_TILE_SUMS)
+            if plan is not None:
+                return ops.gemm_mfma_tile(x, self.weight, splits=plan[1], tile=plan[0])
         return None
 
     def partial_sums(self, x: torch.Tensor, few_rows: bool = False) -> Optional[torch.Tensor]:
