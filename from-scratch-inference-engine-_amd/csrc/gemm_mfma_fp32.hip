@@ -119,7 +119,129 @@ int launch_mt(int waves, const float* x, const float* w, const float* bias, floa
     return 0;
 }
 
+// ---- many rows (prompts) ----------------------------------------------------------------------
+// A workgroup of four waves makes 64 rows of X by 64 of W, a wave 32 by 32; 32 values of K at a time go through two
+// stages of LDS (the next one's loads are under way while this one is multiplied), a row's eight 16-byte units permuted
+// by the row so that eight rows' reads meet different banks.  A wave's read of 16 bytes a lane feeds four instructions
+// of 32 cycles each, so the matrix cores are the bound, and the small tile is what fills the chip: a unit holds five
+// workgroups, and N = 896 at 682 rows still makes 154 of them (in slices of K as many times that).
+// Two levels of float32 sums as above, runs of kTileFlush values of K.  108 TFLOP/s at 2,048 x
+// 3584 x 18944 (154 is what the library reaches at 8,192 cubed); against the vector kernel before it 5,090 -> 2,580 us there,
+// 211 -> 136 at 682 x 9728 x 896, and in seven slices 822 -> 77 at 682 x 896 x 4864.
+constexpr int kTileEdge = 64, kTileK = 32, kTileFlush = 256;
+
+template <bool SUMS>
+__global__ __launch_bounds__(256) void gemm_fp32_tile_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                            const float* __restrict__ bias, float* __restrict__ y, int M,
+                                                            int N, int K, int k_slice) {
+    __shared__ float4 lds[2][2][kTileEdge][kTileK / 4];
+    const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
+    const int n0 = blockIdx.x * kTileEdge, m0 = blockIdx.y * kTileEdge;
+    const int k_begin = blockIdx.z * k_slice, k_end = min(K, k_begin + k_slice);
+    // this thread's units of a stage: rows r and r + 32 of W and of X, values 4 u .. 4 u + 4
+    const int r = threadIdx.x >> 3, u = threadIdx.x & 7;
+    const float* from[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {  // rows past the end repeat the last one and are never written
+        from[i] = w + static_cast<int64_t>(min(n0 + r + 32 * i, N - 1)) * K;
+        from[2 + i] = x + static_cast<int64_t>(min(m0 + r + 32 * i, M - 1)) * K;
+    }
+    float4 held[4];
+    const auto bring = [&](int k0) {
+        const int k = k0 + 4 * u;  // K and the slices are multiples of 4: four values are all in or all out
+        const bool in = k < k_end;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            held[i] = *reinterpret_cast<const float4*>(from[i] + (in ? k : k_begin));
+            if (!in) held[i] = float4{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    const int row = lane & 15, kg = lane >> 4;
+    const int nw = (wave & 1) * 32, mw = (wave >> 1) * 32;
+    floatx4 acc[2][2], total[2][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[j][t] = total[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    bring(k_begin);
+    int buf = 0, run = 0;
+    for (int k0 = k_begin; k0 < k_end; k0 += kTileK, buf ^= 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lds[buf][i >> 1][r + 32 * (i & 1)][u ^ (r & 7)] = held[i];
+        __syncthreads();  // (one a step: the stage written next was read before the last one)
+        if (k0 + kTileK < k_end) bring(k0 + kTileK);
+        float4 a[2][2], b[2][2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                a[j][h] = lds[buf][0][nw + 16 * j + row][(4 * h + kg) ^ (row & 7)];
+                b[j][h] = lds[buf][1][mw + 16 * j + row][(4 * h + kg) ^ (row & 7)];
+            }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+                        acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(reinterpret_cast<const float*>(&a[j][h])[i],
+                                                                        reinterpret_cast<const float*>(&b[t][h])[i], acc[j][t], 0, 0, 0);
+        if (++run == kTileFlush / kTileK) {
+            run = 0;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    total[j][t] += acc[j][t];
+                    acc[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+    }
+    // lane holds D[n .. n + 4][m]
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int m = m0 + mw + 16 * t + row;
+        if (m >= M) continue;
+        float* to = y + ((SUMS ? static_cast<int64_t>(blockIdx.z) * M : 0) + m) * N;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int n = n0 + nw + 16 * j + 4 * kg;
+            const floatx4 v = acc[j][t] + total[j][t];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (n + i < N) to[n + i] = !SUMS && bias ? v[i] + bias[n + i] : v[i];
+        }
+    }
+}
+
 }  // namespace
+
+// float32 operands and result, any number of rows, K a multiple of 4, x and w 16-byte aligned.  splits > 1: y holds
+// that many partial sums [splits][M][N] of slices of K, without bias.
+extern "C" int fsie_gemm_fp32_tile(const float* x, const float* w, const float* bias, float* y, int M, int N, int K,
+                                   int splits, hipStream_t stream) {
+    FSIE_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_fp32_tile: bad sizes M=%d N=%d K=%d", M, N, K);
+    FSIE_REQUIRE(K % 4 == 0, "gemm_fp32_tile: K=%d must be a multiple of 4", K);
+    FSIE_REQUIRE(splits >= 1 && splits <= 64 && (splits == 1 || !bias), "gemm_fp32_tile: %d slices", splits);
+    FSIE_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0,
+                 "gemm_fp32_tile: operands must be 16-byte aligned");
+    if (M == 0) return 0;
+    const int64_t tiles_m = ceil_div64(M, kTileEdge);
+    FSIE_REQUIRE(tiles_m <= 65535, "gemm_fp32_tile: %d rows", M);
+    // slices of whole flushes where K gives them, so that a slice's runs are those of the uncut sum; else of whole steps
+    int64_t slice = ceil_div64(ceil_div64(K, splits), kTileFlush) * kTileFlush;
+    if (slice * (splits - 1) >= K) slice = ceil_div64(ceil_div64(K, splits), kTileK) * kTileK;
+    FSIE_REQUIRE(splits == 1 || slice * (splits - 1) < K, "gemm_fp32_tile: K=%d does not give %d slices", K, splits);
+    const dim3 grid(static_cast<unsigned>((N + kTileEdge - 1) / kTileEdge), static_cast<unsigned>(tiles_m), static_cast<unsigned>(splits));
+    if (splits > 1)
+        gemm_fp32_tile_kernel<true><<<grid, 256, 0, stream>>>(x, w, nullptr, y, M, N, K, static_cast<int>(slice));
+    else
+        gemm_fp32_tile_kernel<false><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K, static_cast<int>(ceil_div64(K, kTileK) * kTileK));
+    FSIE_CHECK_LAUNCH("gemm_fp32_tile");
+    return 0;
+}
 
 // float32 operands and result.  1 <= M <= 64, K a multiple of 4, x and w 16-byte aligned.
 // waves: 1, 2, 4 or 8 waves of a workgroup split K; 0 = choose.

@@ -407,6 +407,34 @@ def gemm_mfma_fp32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     return out
 
 
+def gemm_fp32_tile(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, splits: int = 1) -> torch.Tensor:
+    """The same for any number of rows (prompts).  ``splits`` > 1: float32 partial sums [splits, M, N] of slices of K (no
+    bias), for ``rmsnorm`` to add up."""
+    _need(x, "gemm x", dtype=torch.float32, ndim=2)
+    _need(weight, "gemm weight", dtype=torch.float32, ndim=2)
+    m, k = x.shape
+    n = weight.shape[0]
+    if weight.shape[1] != k:
+        raise KernelError(f"gemm: weight inner size {weight.shape[1]} does not match x's {k}")
+    if bias is not None:
+        _need(bias, "gemm bias", dtype=torch.float32, shape=(n,))
+    out = torch.empty((m, n) if splits == 1 else (splits, m, n), dtype=torch.float32, device=x.device)
+    check(load().fsie_gemm_fp32_tile(x.data_ptr(), weight.data_ptr(), _ptr(bias), out.data_ptr(), m, n, k, splits, _stream()))
+    return out
+
+
+@lru_cache(maxsize=4096)
+def gemm_fp32_tile_splits(m: int, n: int, k: int) -> int:
+    """Slices of K for ``gemm_fp32_tile``: whole runs of 256 values (the kernel's own), as many as bring its tiles of 64 x 64
+    to four a compute unit."""
+    tiles = -(-m // 64) * -(-n // 64)
+    wanted = min(GEMM_MAX_SPLITS, 4 * compute_units() // tiles, k // 256)
+    if wanted < 2:
+        return 1
+    run = -(-(-(-k // wanted)) // 256) * 256
+    return -(-k // run)
+
+
 def gemm_mfma_skinny(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
                      out_dtype: Optional[torch.dtype] = None, waves: int = 0, blocks: int = 0,
                      out: Optional[torch.Tensor] = None, epilogue: str = "plain", splits: int = 1) -> torch.Tensor:

@@ -94,6 +94,8 @@ class Linear:
                 # decoding in the 32-bit path: W streams once into true float32 matrix instructions
                 # (several times faster than the vector kernels from 8 rows on, no faster at one or two)
                 return ops.gemm_mfma_fp32(x, w, bias)
+            if self.float32_on_matrix_cores and m > GEMM_MFMA_SKINNY_MAX_M and self.in_features % 4 == 0:
+                return ops.gemm_fp32_tile(x, w, bias)  # prompts: the same instruction, both operands through LDS
             return ops.gemm(x, w, bias, out_dtype=out_dtype)
         wants_f32 = out_dtype is not None and out_dtype != x.dtype
         if wants_f32 and out_dtype == torch.float32 and self.out_features <= self.narrow_to:
@@ -160,6 +162,12 @@ class Linear:
             splits = self.residual_splits(m)
             if splits > 1:
                 return ops.gemm_mfma_skinny(x, self.weight, splits=splits)
+        if (getattr(ctx, "partial_sums_ok", False) and x.dtype == torch.float32 and self.bias is None
+                and self.float32_on_matrix_cores and m > GEMM_MFMA_SKINNY_MAX_M and self.in_features % 4 == 0):
+            # prompts of the 32-bit path: slices of K where the tiles alone leave the chip idle
+            splits = ops.gemm_fp32_tile_splits(m, self.out_features, self.in_features)
+            if splits > 1:
+                return ops.gemm_fp32_tile(x, self.weight, splits=splits)
         if (getattr(ctx, "partial_sums_ok", False) and x.dtype == torch.bfloat16 and self.bias is None
                 and m > GEMM_MFMA_WIDE_MAX_M):
             # prompts and a long K: the product for many rows in slices of K

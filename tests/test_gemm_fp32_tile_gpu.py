@@ -1,0 +1,41 @@
+"""The 32-bit product for many rows at the edges of its tiles, steps, runs and slices."""
+
+import pytest
+import torch
+
+import from_scratch_inference_engine_amd.ops as ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("k", [4, 28, 32, 36, 256, 260, 1100])
+@pytest.mark.parametrize("m,n", [(65, 1), (64, 64), (63, 65), (129, 130), (200, 3)])
+def test_against_64_bits(m, n, k):
+    ops.load(build_if_missing=False)
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn((m, k), generator=g).cuda(), torch.randn((n, k), generator=g).cuda()
+    bias = torch.randn((n,), generator=g).cuda()
+    want = x.double() @ w.double().t()
+    # a product and a sum of k of them in float32, in any order: at most k + 1 roundings of 2^-24 of the magnitudes' sum
+    bound = (k + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t() + bias.double().abs())
+    assert ((ops.gemm_fp32_tile(x, w).double() - want).abs() <= bound).all()
+    assert ((ops.gemm_fp32_tile(x, w, bias).double() - (want + bias.double())).abs() <= bound).all()
+    for slices in range(2, 6):
+        run = -(-k // slices)
+        if -(-run // 32) * 32 * (slices - 1) >= k:
+            with pytest.raises(ops.KernelError):
+                ops.gemm_fp32_tile(x, w, splits=slices)
+            continue
+        got = ops.gemm_fp32_tile(x, w, splits=slices)
+        assert got.shape == (slices, m, n) and ((got.double().sum(0) - want).abs() <= bound).all()
+
+
+def test_slices_are_ones_the_kernel_takes():
+    ops.load(build_if_missing=False)
+    for m in (65, 200, 682, 2048):
+        for n, k in ((896, 4864), (896, 896), (3584, 18944), (64, 256), (64, 300), (16, 512), (40, 2000)):
+            slices = ops.gemm_fp32_tile_splits(m, n, k)
+            assert 1 <= slices <= 16
+            if slices > 1:
+                x, w = torch.zeros((m, k), device="cuda"), torch.zeros((n, k), device="cuda")
+                assert ops.gemm_fp32_tile(x, w, splits=slices).shape[0] == slices
