@@ -228,8 +228,11 @@ __global__ __launch_bounds__(512, 2) void gemm_tile_kernel(const bf16_t* __restr
 #pragma unroll
             for (int j = 0; j < J; ++j) {
                 if (RESULT == kPair) {
-                    out[j] = pack2_bf16(gate_pair(acc[j][t][0], acc[j][t][1], ACT, act_pos, act_neg),
-                                        gate_pair(acc[j][t][2], acc[j][t][3], ACT, act_pos, act_neg));
+                    // gate and up are rounded to 16 bits first, as the library's product leaves them for the pass that
+                    // multiplies them: what a token of a prompt gets does not depend on which of the two its portion takes
+                    const uint32_t a = pack2_bf16(acc[j][t][0], acc[j][t][1]), b = pack2_bf16(acc[j][t][2], acc[j][t][3]);
+                    out[j] = pack2_bf16(gate_pair(__uint_as_float(a << 16), __uint_as_float(a & 0xffff0000u), ACT, act_pos, act_neg),
+                                        gate_pair(__uint_as_float(b << 16), __uint_as_float(b & 0xffff0000u), ACT, act_pos, act_neg));
                 } else {
                     out[2 * j] = pack2_bf16(acc[j][t][0], acc[j][t][1]);
                     out[2 * j + 1] = pack2_bf16(acc[j][t][2], acc[j][t][3]);
