@@ -361,10 +361,12 @@ void launch_shape(int mt, int N, int splits, int& waves, int& blocks, bool gate_
         // slices 39.6 against 38.1); with two blocks a wave, four waves (N = 152064: 236 against 260)
         const int64_t groups4 = static_cast<int64_t>((N + 63) / 64) * splits;
         waves = (groups4 >= 1024 && blocks == 1) ? 8 : 4;
-        // one tile of X at a large N of a fragment-ordered W: nothing to share, and two waves a workgroup stream best (N = 152064,
-        // K = 3584, fragment-ordered: 8 rows 168 us with two waves, 171 with four, 179 with eight; one row
-        // 164 / 168 / 177; N = 152064, K = 5120, 8 rows: 247 / 249 / 259)
-        if (frags && mt == 1 && groups4 >= 1024 && blocks == 1) waves = 2;  // (on rows: 215 / 195 / 194)
+        // one tile of X and a fragment-ordered W: nothing to share, and two waves a workgroup stream best (N = 152064,
+        // K = 3584: 8 rows 168 us with two waves, 171 with four, 179 with eight; one row
+        // 164 / 168 / 177; N = 152064, K = 5120, 8 rows: 247 / 249 / 259; gate and up of 8 rows: N = 16384, K = 2048 13.1 us with two,
+        // 15.1 with four, N = 9728, K = 896 6.7 / 7.4; sums of 8 rows: N = K = 3584 in seven slices 6.4 / 6.8, N = 4608, K = 3584
+        // 7.1 / 7.3, N = 6144, K = 2048 in four 6.1 / 7.0)
+        if (frags && mt == 1 && blocks == 1) waves = 2;  // (on rows, N = 152064: 215 / 195 / 194)
         // two waves a workgroup where that deals the waves more evenly to the compute units (N =
         // 5120 in 8 slices: 640 workgroups of four waves put 12 waves on the fullest of 256 units,
         // 1280 of two put 10; K = 13824, 8 rows: 26.7 against 29.8 us)
@@ -409,16 +411,30 @@ extern "C" int fsie_gemm_mfma_wide_best_splits(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0) return 1;
     const int mt = (M + 15) / 16;
     const int units = fsie_compute_units();
+    const int stage = 32 * FSIE_WIDE_STEPS;
     if (mt <= 1 || units <= 0) {
-        for (int s = 8; s >= 2; --s)
-            if (K / s >= 512 && fsie_gemm_mfma_wide_slice(K, s) > 0) return s;
-        return 1;
+        int best = 1;
+        for (int s = 8; s >= 2 && best == 1; --s)
+            if (K / s >= 512 && fsie_gemm_mfma_wide_slice(K, s) > 0) best = s;
+        // where that gives a unit one workgroup of 64 rows of W or less, shorter slices, down to one stage, while the
+        // workgroups stay fewer than two a unit (8 rows: N = K = 896 in seven slices 2.4 us, whole 5.6; N = 896, K = 4864 in
+        // 13 4.2, in eight 5.0; N = K = 2048 in eight 3.7, in four 4.3; N = 2048, K = 8192 in 13 7.6, in eight 8.5, in 16 9.0;
+        // but N = 6144, K = 2048, 384 workgroups in four slices, 6.1 against 6.3 in eight)
+        const int64_t groups = (N + 63) / 64;
+        if (units > 0 && groups * best <= units) {
+            for (int s = FSIE_GEMM_MAX_SPLITS; s > best; --s)
+                if (K / s >= stage && groups * s < 2 * static_cast<int64_t>(units) && fsie_gemm_mfma_wide_slice(K, s) > 0) return s;
+        }
+        return best;
     }
+    // a K too short for two slices of 512 is cut finer, for the matrices of small models (40 rows, N = K = 896: 3.4 us in
+    // seven slices, 6.1 whole)
+    const int shortest = K >= 2 * 512 ? 512 : stage;
     int best = 1;
     int64_t best_groups = 0;
     bool best_fits = false;
     for (int s = 2; s <= FSIE_GEMM_MAX_SPLITS; ++s) {
-        if (K / s < 512 || fsie_gemm_mfma_wide_slice(K, s) <= 0) continue;
+        if (K / s < shortest || fsie_gemm_mfma_wide_slice(K, s) <= 0) continue;
         int waves = 0, blocks = 0;
         launch_shape(mt, N, s, waves, blocks);
         const int rows = 16 * blocks * waves;
@@ -437,7 +453,7 @@ extern "C" int fsie_gemm_mfma_wide_best_splits(int M, int N, int K) {
     // K = 5120 the sums of the rule's four slices are a tenth and the rule's choice the fastest).
     if (mt == 4 && best > 2 && 4.0 * best * 64 * N > 0.2 * 2.0 * N * K) {
         for (int s = 2; s < best; ++s) {
-            if (K / s < 512 || fsie_gemm_mfma_wide_slice(K, s) <= 0) continue;
+            if (K / s < shortest || fsie_gemm_mfma_wide_slice(K, s) <= 0) continue;
             int waves = 0, blocks = 0;
             launch_shape(mt, N, s, waves, blocks);
             const int rows = 16 * blocks * waves;

@@ -32,12 +32,12 @@ class Linear:
     # A bfloat16 weight of at least this many bytes is kept a second time, in the order of the matrix
     # instruction's fragments, for the engine's own products (decoding): a wave then loads 1 KB in one
     # piece with streaming loads, where rows give it 16 pieces of 64 bytes (a compute unit draws about
-    # half as much when a wave's load is pieces of rows).  From 16 MB on: the q/k/v and output
-    # projections of a 7B model (33 and 26 MB) gain by it.  The rows stay for the library's products of
-    # many rows.  None: no copies.
+    # half as much when a wave's load is pieces of rows).  From 8 MB on (8 rows: N = 896, K = 4864, 8.7 MB,
+    # 4.2 us against 4.8; N = K = 2048 3.7 / 4.2; N = 3072, K = 2048 4.2 / 4.9; below that a launch is most of
+    # the time).  The rows stay for the library's products of many rows.  None: no copies.
     # A copy that would leave less than ``streamed_copy_reserve`` of the device's memory free is not
     # made: a model that large keeps copies of its first layers only and runs the rest from rows.
-    streamed_copy_from = 16 << 20
+    streamed_copy_from = 8 << 20
     streamed_copy_reserve = 0.25
 
     def __init__(self, in_features: int, out_features: int, bias: bool = False):
