@@ -184,6 +184,8 @@ int fsie_gemm(const void* x, const void* w, const float* bias, void* y, int M, i
 // True float32 on the matrix cores (v_mfma_f32_16x16x4_f32) for up to 64 rows: the 32-bit path's decoding.
 int fsie_gemm_mfma_fp32(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int waves,
                         hipStream_t stream);
+// The same as partial sums [splits][M][N] of slices of K.
+int fsie_gemm_mfma_fp32_sums(const float* x, const float* w, float* y, int M, int N, int K, int splits, hipStream_t stream);
 // The same for any number of rows (prompts); splits > 1: y = partial sums [splits][M][N] of slices of K, no bias.
 int fsie_gemm_fp32_tile(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int splits,
                         hipStream_t stream);

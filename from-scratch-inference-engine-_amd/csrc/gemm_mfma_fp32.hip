@@ -19,7 +19,8 @@ template <int MT, int WAVES>
 __global__ __launch_bounds__(WAVES * FSIE_WAVE) void gemm_mfma_fp32_kernel(const float* __restrict__ x,
                                                                           const float* __restrict__ w,
                                                                           const float* __restrict__ bias,
-                                                                          float* __restrict__ y, int M, int N, int K) {
+                                                                          float* __restrict__ y, int M, int N, int K,
+                                                                          int slice_steps) {
     constexpr int U = MT >= 3 ? 2 : 4;
     __shared__ float red[WAVES > 1 ? (WAVES - 1) * MT * FSIE_WAVE * 4 : 1];
     const int lane = threadIdx.x & (FSIE_WAVE - 1);
@@ -41,9 +42,12 @@ __global__ __launch_bounds__(WAVES * FSIE_WAVE) void gemm_mfma_fp32_kernel(const
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = total[t] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    const int n_steps = (K + 15) / 16;
+    // blockIdx.y: a slice of K of `slice_steps` steps, whose sums are a plane of y of their own
+    const int first_step = blockIdx.y * slice_steps;
+    const int n_steps = min((K + 15) / 16, first_step + slice_steps);
+    y += static_cast<int64_t>(blockIdx.y) * M * N;
     int pass = 0;
-    for (int s0 = wave; s0 < n_steps; s0 += WAVES * U, ++pass) {
+    for (int s0 = first_step + wave; s0 < n_steps; s0 += WAVES * U, ++pass) {
         if (pass > 0 && pass % kFlush == 0) {
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
@@ -57,7 +61,7 @@ __global__ __launch_bounds__(WAVES * FSIE_WAVE) void gemm_mfma_fp32_kernel(const
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int k0 = (s0 + u * WAVES) * 16 + kg * 4;
-            ok[u] = k0 < K;  // K is a multiple of 4: a lane's four values are all in or all out
+            ok[u] = k0 < K && s0 + u * WAVES < n_steps;  // K is a multiple of 4: a lane's four values are all in or all out
             const int k0c = ok[u] ? k0 : 0;
             a[u] = *reinterpret_cast<const float4*>(wp + k0c);
 #pragma unroll
@@ -106,14 +110,15 @@ __global__ __launch_bounds__(WAVES * FSIE_WAVE) void gemm_mfma_fp32_kernel(const
 }
 
 template <int MT>
-int launch_mt(int waves, const float* x, const float* w, const float* bias, float* y, int M, int N, int K,
+int launch_mt(int waves, const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int splits,
               hipStream_t stream) {
-    const unsigned groups = static_cast<unsigned>((N + 15) / 16);
+    const int steps = (K + 15) / 16, slice = (steps + splits - 1) / splits;
+    const dim3 groups(static_cast<unsigned>((N + 15) / 16), static_cast<unsigned>(splits));
     switch (waves) {
-        case 1: gemm_mfma_fp32_kernel<MT, 1><<<groups, 64, 0, stream>>>(x, w, bias, y, M, N, K); break;
-        case 2: gemm_mfma_fp32_kernel<MT, 2><<<groups, 128, 0, stream>>>(x, w, bias, y, M, N, K); break;
-        case 4: gemm_mfma_fp32_kernel<MT, 4><<<groups, 256, 0, stream>>>(x, w, bias, y, M, N, K); break;
-        default: gemm_mfma_fp32_kernel<MT, 8><<<groups, 512, 0, stream>>>(x, w, bias, y, M, N, K); break;
+        case 1: gemm_mfma_fp32_kernel<MT, 1><<<groups, 64, 0, stream>>>(x, w, bias, y, M, N, K, slice); break;
+        case 2: gemm_mfma_fp32_kernel<MT, 2><<<groups, 128, 0, stream>>>(x, w, bias, y, M, N, K, slice); break;
+        case 4: gemm_mfma_fp32_kernel<MT, 4><<<groups, 256, 0, stream>>>(x, w, bias, y, M, N, K, slice); break;
+        default: gemm_mfma_fp32_kernel<MT, 8><<<groups, 512, 0, stream>>>(x, w, bias, y, M, N, K, slice); break;
     }
     FSIE_CHECK_LAUNCH("gemm_mfma_fp32");
     return 0;
@@ -244,9 +249,10 @@ extern "C" int fsie_gemm_fp32_tile(const float* x, const float* w, const float* 
 }
 
 // float32 operands and result.  1 <= M <= 64, K a multiple of 4, x and w 16-byte aligned.
-// waves: 1, 2, 4 or 8 waves of a workgroup split K; 0 = choose.
-extern "C" int fsie_gemm_mfma_fp32(const float* x, const float* w, const float* bias, float* y, int M, int N, int K,
-                                   int waves, hipStream_t stream) {
+// waves: 1, 2, 4 or 8 waves of a workgroup split K; 0 = choose.  splits > 1: y = partial sums [splits][M][N] of slices of K,
+// no bias.
+static int few_rows(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int waves, int splits,
+                    hipStream_t stream) {
     FSIE_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_mfma_fp32: bad sizes M=%d N=%d K=%d", M, N, K);
     FSIE_REQUIRE(M <= FSIE_GEMM_MFMA_SKINNY_MAX_M, "gemm_mfma_fp32: at most %d rows, got %d",
                  FSIE_GEMM_MFMA_SKINNY_MAX_M, M);
@@ -257,18 +263,31 @@ extern "C" int fsie_gemm_mfma_fp32(const float* x, const float* w, const float* 
                  "gemm_mfma_fp32: operands must be 16-byte aligned");
     FSIE_REQUIRE(waves == 0 || waves == 1 || waves == 2 || waves == 4 || waves == 8,
                  "gemm_mfma_fp32: waves must be 0, 1, 2, 4 or 8");
+    const int steps = (K + 15) / 16;
+    FSIE_REQUIRE(splits >= 1 && splits <= FSIE_GEMM_MAX_SPLITS &&
+                     (splits == 1 || ((steps + splits - 1) / splits) * (splits - 1) < steps),
+                 "gemm_mfma_fp32: K=%d does not give %d slices", K, splits);
     if (M == 0) return 0;
     if (waves == 0) {
-        const int groups = (N + 15) / 16;
-        const int steps = (K + 15) / 16;
+        const int groups = (N + 15) / 16 * splits;
         waves = 1;
         while (waves < 8 && groups * waves < 1024) waves *= 2;
-        while (waves > 1 && steps < 4 * waves) waves /= 2;
+        while (waves > 1 && steps / splits < 4 * waves) waves /= 2;
     }
     switch ((M + 15) / 16) {
-        case 1: return launch_mt<1>(waves, x, w, bias, y, M, N, K, stream);
-        case 2: return launch_mt<2>(waves, x, w, bias, y, M, N, K, stream);
-        case 3: return launch_mt<3>(waves, x, w, bias, y, M, N, K, stream);
-        default: return launch_mt<4>(waves, x, w, bias, y, M, N, K, stream);
+        case 1: return launch_mt<1>(waves, x, w, bias, y, M, N, K, splits, stream);
+        case 2: return launch_mt<2>(waves, x, w, bias, y, M, N, K, splits, stream);
+        case 3: return launch_mt<3>(waves, x, w, bias, y, M, N, K, splits, stream);
+        default: return launch_mt<4>(waves, x, w, bias, y, M, N, K, splits, stream);
     }
+}
+
+extern "C" int fsie_gemm_mfma_fp32(const float* x, const float* w, const float* bias, float* y, int M, int N, int K,
+                                   int waves, hipStream_t stream) {
+    return few_rows(x, w, bias, y, M, N, K, waves, 1, stream);
+}
+
+extern "C" int fsie_gemm_mfma_fp32_sums(const float* x, const float* w, float* y, int M, int N, int K, int splits,
+                                        hipStream_t stream) {
+    return few_rows(x, w, nullptr, y, M, N, K, 0, splits, stream);
 }

@@ -407,6 +407,30 @@ def gemm_mfma_fp32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     return out
 
 
+def gemm_mfma_fp32_sums(x: torch.Tensor, weight: torch.Tensor, splits: int) -> torch.Tensor:
+    """The same as float32 partial sums [splits, M, N] of slices of K, for ``rmsnorm`` to add up."""
+    _need(x, "gemm x", dtype=torch.float32, ndim=2)
+    _need(weight, "gemm weight", dtype=torch.float32, ndim=2)
+    m, k = x.shape
+    n = weight.shape[0]
+    if weight.shape[1] != k:
+        raise KernelError(f"gemm: weight inner size {weight.shape[1]} does not match x's {k}")
+    out = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+    check(load().fsie_gemm_mfma_fp32_sums(x.data_ptr(), weight.data_ptr(), out.data_ptr(), m, n, k, splits, _stream()))
+    return out
+
+
+def gemm_mfma_fp32_splits(k: int) -> int:
+    """Slices of K for ``gemm_mfma_fp32_sums``: eight, each at least 224 long (4 rows, us whole and in the rule's slices:
+    N = 896, K = 4864 17.6 and 7.3, N = K = 896 5.2 and 3.7, N = 3584, K = 18944 74 and 53, N = 2048, K = 8192 27 and 22;
+    workgroups of 16 rows of W that walk all of K wait for one trip to memory after the other)."""
+    splits = max(1, min(8, k // 224))
+    steps = -(-k // 16)
+    while splits > 1 and -(-steps // splits) * (splits - 1) >= steps:
+        splits -= 1
+    return splits
+
+
 def gemm_fp32_tile(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, splits: int = 1) -> torch.Tensor:
     """The same for any number of rows (prompts).  ``splits`` > 1: float32 partial sums [splits, M, N] of slices of K (no
     bias), for ``rmsnorm`` to add up."""

@@ -163,11 +163,16 @@ class Linear:
             if splits > 1:
                 return ops.gemm_mfma_skinny(x, self.weight, splits=splits)
         if (getattr(ctx, "partial_sums_ok", False) and x.dtype == torch.float32 and self.bias is None
-                and self.float32_on_matrix_cores and m > GEMM_MFMA_SKINNY_MAX_M and self.in_features % 4 == 0):
-            # prompts of the 32-bit path: slices of K where the tiles alone leave the chip idle
-            splits = ops.gemm_fp32_tile_splits(m, self.out_features, self.in_features)
-            if splits > 1:
-                return ops.gemm_fp32_tile(x, self.weight, splits=splits)
+                and self.float32_on_matrix_cores and m > 2 and self.in_features % 4 == 0):
+            # the 32-bit path: slices of K where the rows of W alone (or a prompt's tiles) leave the chip idle
+            if m <= GEMM_MFMA_SKINNY_MAX_M:
+                splits = ops.gemm_mfma_fp32_splits(self.in_features)
+                if splits > 1:
+                    return ops.gemm_mfma_fp32_sums(x, self.weight, splits)
+            else:
+                splits = ops.gemm_fp32_tile_splits(m, self.out_features, self.in_features)
+                if splits > 1:
+                    return ops.gemm_fp32_tile(x, self.weight, splits=splits)
         if (getattr(ctx, "partial_sums_ok", False) and x.dtype == torch.bfloat16 and self.bias is None
                 and m > GEMM_MFMA_WIDE_MAX_M):
             # prompts and a long K: the product for many rows in slices of K

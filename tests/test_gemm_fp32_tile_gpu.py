@@ -39,3 +39,22 @@ def test_slices_are_ones_the_kernel_takes():
             if slices > 1:
                 x, w = torch.zeros((m, k), device="cuda"), torch.zeros((n, k), device="cuda")
                 assert ops.gemm_fp32_tile(x, w, splits=slices).shape[0] == slices
+
+
+@pytest.mark.parametrize("m", [3, 16, 17, 64])
+@pytest.mark.parametrize("n,k", [(896, 896), (40, 448), (17, 4864), (64, 452), (896, 2000)])
+def test_few_rows_in_slices(m, n, k):
+    ops.load(build_if_missing=False)
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn((m, k), generator=g).cuda(), torch.randn((n, k), generator=g).cuda()
+    want = x.double() @ w.double().t()
+    bound = (k + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    for slices in {2, 3, ops.gemm_mfma_fp32_splits(k)} - {1}:
+        got = ops.gemm_mfma_fp32_sums(x, w, slices)
+        assert got.shape == (slices, m, n) and ((got.double().sum(0) - want).abs() <= bound).all()
+
+
+def test_slices_of_few_rows_are_never_empty():
+    for k in list(range(4, 1200, 4)) + [4864, 8192, 18944]:
+        slices, steps = ops.gemm_mfma_fp32_splits(k), -(-k // 16)
+        assert 1 <= slices <= 8 and -(-steps // slices) * (slices - 1) < steps
