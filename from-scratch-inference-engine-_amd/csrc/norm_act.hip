@@ -168,7 +168,10 @@ __global__ __launch_bounds__(kThreads) void stream_out_kernel(float* __restrict_
 // One wave per (token, head): o [tokens][heads * width] float32 is normalised over the `width` values of
 // the head (plain weight [width], shared by the heads) and multiplied by act(gate) of the same place;
 // gate [tokens][gate_stride] of T (the columns of the head start at h * width).
-template <typename T>
+// HELD > 0: heads of up to 64 * HELD values, which a lane keeps in registers: the planes, the gate and the weight are all
+// asked for at once, where the loop waits for each plane of each run of 64 and reads o twice.  A launch of few tokens is
+// nothing but those trips to memory (8 tokens of 8 heads of 256, two planes: 4.7 us, 6.9 before; the same sums in the same order).
+template <typename T, int HELD>
 __global__ __launch_bounds__(kThreads) void gated_headnorm_kernel(const float* __restrict__ o, const T* __restrict__ gate,
                                                                   int64_t gate_stride, const float* __restrict__ weight,
                                                                   T* __restrict__ out, int64_t n_runs, int heads, int width,
@@ -182,6 +185,36 @@ __global__ __launch_bounds__(kThreads) void gated_headnorm_kernel(const float* _
     const float* src = o + (t * heads + h) * width;
     const T* g = gate + t * gate_stride + static_cast<int64_t>(h) * width;
     T* dst = out + t * out_stride + static_cast<int64_t>(h) * width;  // (rows of out may be columns of wider rows)
+    if (HELD > 0) {
+        constexpr int AHEAD = 4;  // planes asked for together
+        float x[HELD > 0 ? HELD : 1], w[HELD > 0 ? HELD : 1], gate_value[HELD > 0 ? HELD : 1];
+#pragma unroll
+        for (int j = 0; j < HELD; ++j) {
+            const int i = min(lane + FSIE_WAVE * j, width - 1);
+            w[j] = weight[i];
+            gate_value[j] = to_float(g[i]);
+            float part[AHEAD];
+#pragma unroll
+            for (int p = 0; p < AHEAD; ++p) part[p] = src[min(p, n_planes - 1) * plane + i];
+            x[j] = part[0];
+#pragma unroll
+            for (int p = 1; p < AHEAD; ++p)
+                if (p < n_planes) x[j] += part[p];
+        }
+        for (int p = AHEAD; p < n_planes; ++p)
+#pragma unroll
+            for (int j = 0; j < HELD; ++j) x[j] += src[p * plane + min(lane + FSIE_WAVE * j, width - 1)];
+        float total = 0.f;
+#pragma unroll
+        for (int j = 0; j < HELD; ++j)
+            if (lane + FSIE_WAVE * j < width) total += x[j] * x[j];
+        const float by = 1.0f / sqrtf(wave_sum(total) / static_cast<float>(width) + eps);
+#pragma unroll
+        for (int j = 0; j < HELD; ++j)
+            if (lane + FSIE_WAVE * j < width)
+                dst[lane + FSIE_WAVE * j] = from_float<T>((((x[j] * by) * w[j]) * gate_act(gate_value[j], act)) * out_scale);
+        return;
+    }
     // o comes as n_planes arrays a `plane` apart, added in order (the shares of a state kernel's row splits)
     auto value = [&](int i) {
         float x = src[i];
@@ -313,15 +346,19 @@ extern "C" int fsie_gated_headnorm(const float* o, int n_planes, const void* gat
     if (n_tokens == 0) return 0;
     const int64_t runs = static_cast<int64_t>(n_tokens) * heads;
     const unsigned grid = static_cast<unsigned>(ceil_div64(runs, kThreads / FSIE_WAVE));
+#define FSIE_HEADNORM(T, HELD)                                                                                              \
+    gated_headnorm_kernel<T, HELD><<<grid, kThreads, 0, stream>>>(o, static_cast<const T*>(gate), gate_stride, weight,      \
+                                                                static_cast<T*>(out), runs, heads, width, eps, act,         \
+                                                                n_planes, plane, out_stride, out_scale)
+    const bool held = width <= 4 * FSIE_WAVE;
     if (dtype == FSIE_F32) {
-        gated_headnorm_kernel<float><<<grid, kThreads, 0, stream>>>(o, static_cast<const float*>(gate), gate_stride, weight,
-                                                                  static_cast<float*>(out), runs, heads, width, eps, act, n_planes, plane,
-                                                                  out_stride, out_scale);
+        if (held) FSIE_HEADNORM(float, 4);
+        else FSIE_HEADNORM(float, 0);
     } else {
-        gated_headnorm_kernel<bf16_t><<<grid, kThreads, 0, stream>>>(o, static_cast<const bf16_t*>(gate), gate_stride, weight,
-                                                                   static_cast<bf16_t*>(out), runs, heads, width, eps, act, n_planes, plane,
-                                                                   out_stride, out_scale);
+        if (held) FSIE_HEADNORM(bf16_t, 4);
+        else FSIE_HEADNORM(bf16_t, 0);
     }
+#undef FSIE_HEADNORM
     FSIE_CHECK_LAUNCH("gated_headnorm");
     return 0;
 }
