@@ -711,18 +711,16 @@ struct Found {
     int bin;       // -1: nowhere
     double above, total;
 };
-template <int THREADS, typename F>
-__device__ Found find_in_bins(double target, F value) {
+// `v`: the values of this thread's own kBins / THREADS neighbouring bins (read from memory once for all searches).
+template <int THREADS>
+__device__ Found find_in_bins(double target, const double (&v)[kBins / THREADS]) {
     constexpr int PER = kBins / THREADS;
     __shared__ double wave_sum[THREADS / FSIE_WAVE];
     __shared__ Found found;
     const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
-    double v[PER], run = 0.0;
+    double run = 0.0;
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        v[i] = value(static_cast<int>(threadIdx.x) * PER + i);
-        run += v[i];
-    }
+    for (int i = 0; i < PER; ++i) run += v[i];
 #pragma unroll
     for (int off = 1; off < FSIE_WAVE; off <<= 1) {
         const double other = __shfl_up(run, off, FSIE_WAVE);
@@ -768,19 +766,33 @@ __global__ __launch_bounds__(kPart) void split_list_kernel(const float* __restri
     float scale;
     if (!top.binned(vocab, &scale)) return;
     const int hi_bits = 63 - (32 - __clz(vocab));
-    const auto weight = [&](int b) { return value_of(Limbs{w->hi[b], w->lo[b]}, hi_bits); };
+    constexpr int PER = kBins / kPart;
+    const int b0 = static_cast<int>(threadIdx.x) * PER;
+    double counts[PER], weights[PER], some[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        counts[i] = static_cast<double>(w->count[b0 + i]);
+        weights[i] = value_of(Limbs{w->hi[b0 + i], w->lo[b0 + i]}, hi_bits);
+    }
     int k_bin = -1, from = 0, upto = -1;
-    if (q.k > 0) k_bin = find_in_bins<kPart>(q.k, [&](int b) { return static_cast<double>(w->count[b]); }).bin;
+    if (q.k > 0) k_bin = find_in_bins<kPart>(q.k, counts).bin;
     if (q.p < 1.f) {
         // top p of what top k keeps: all of the bins above its own and some of that one, so the last kept token lies
         // between the bins that the least and the most of it give
-        const double most = find_in_bins<kPart>(INFINITY, [&](int b) { return k_bin < 0 || b <= k_bin ? weight(b) : 0.0; }).total;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) some[i] = k_bin < 0 || b0 + i <= k_bin ? weights[i] : 0.0;
+        const double most = find_in_bins<kPart>(INFINITY, some).total;
         double least = most;
-        if (k_bin >= 0) least = find_in_bins<kPart>(INFINITY, [&](int b) { return b < k_bin ? weight(b) : 0.0; }).total;
+        if (k_bin >= 0) {
+#pragma unroll
+            for (int i = 0; i < PER; ++i) some[i] = b0 + i < k_bin ? weights[i] : 0.0;
+            least = find_in_bins<kPart>(INFINITY, some).total;
+        }
         const double p = static_cast<double>(q.p);
         if (p > 0.0) {
-            from = max(0, find_in_bins<kPart>(p * least, weight).bin);
-            upto = find_in_bins<kPart>(p * most, weight).bin;
+            upto = find_in_bins<kPart>(p * most, weights).bin;
+            from = k_bin < 0 ? upto : find_in_bins<kPart>(p * least, weights).bin;
+            from = max(0, from);
         }
     }
     int begin, end;
@@ -866,8 +878,13 @@ __global__ __launch_bounds__(kThreads) void split_cut_kernel(const float* __rest
         }
         __syncthreads();
         int k_bin = -1;
+        constexpr int PER = kBins / kThreads;
+        const int b0 = static_cast<int>(threadIdx.x) * PER;
+        double values[PER];
         if (q.k > 0) {
-            const Found at = find_in_bins<kThreads>(q.k, [&](int b) { return static_cast<double>(w->count[b]); });
+#pragma unroll
+            for (int i = 0; i < PER; ++i) values[i] = static_cast<double>(w->count[b0 + i]);
+            const Found at = find_in_bins<kThreads>(q.k, values);
             k_bin = at.bin;
             const long long want = q.k - static_cast<long long>(at.above);
             if (k_bin < 0) {
@@ -904,15 +921,17 @@ __global__ __launch_bounds__(kThreads) void split_cut_kernel(const float* __rest
             if (kept.lo) atomicAdd(&kept_lo, kept.lo);
             if (threadIdx.x == 0) cut_found = 0;
             __syncthreads();
-            const auto weight = [&](int b) {
-                if (k_bin >= 0 && b >= k_bin) return b == k_bin ? value_of(Limbs{kept_hi, kept_lo}, hi_bits) : 0.0;
-                return value_of(Limbs{w->hi[b], w->lo[b]}, hi_bits);
-            };
-            const double target = static_cast<double>(q.p) * find_in_bins<kThreads>(INFINITY, weight).total;
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                const int b = b0 + i;
+                values[i] = value_of(Limbs{w->hi[b], w->lo[b]}, hi_bits);
+                if (k_bin >= 0 && b >= k_bin) values[i] = b == k_bin ? value_of(Limbs{kept_hi, kept_lo}, hi_bits) : 0.0;
+            }
+            const double target = static_cast<double>(q.p) * find_in_bins<kThreads>(INFINITY, values).total;
             if (!(target > 0.0)) {
                 cut = key_max;
             } else {
-                const Found at = find_in_bins<kThreads>(target, weight);
+                const Found at = find_in_bins<kThreads>(target, values);
                 const auto counts = [&](int i) { return bin_of_key[i] == at.bin && keys[i] >= cut; };
                 const auto reaches = [&](Limbs s) { return target <= at.above + value_of(s, hi_bits); };
                 // (rounding may have put the target outside the bins that were listed)

@@ -36,6 +36,29 @@ def uniform_for(seed: int, request_id: int, index: int) -> float:
     return (z >> 11) / float(1 << 53)
 
 
+_VECTOR_FROM = 12  # rows from which the array form below is the faster one (a row alone takes 1.5 us, the arrays 15)
+
+
+def _splitmix64_array(x: np.ndarray) -> np.ndarray:
+    x = x + np.uint64(0x9E3779B97F4A7C15)
+    z = (x ^ (x >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+    z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+    return z ^ (z >> np.uint64(31))
+
+
+def uniforms_for(seed: int, request_ids: Sequence[int], indices: Sequence[int]):
+    """``uniform_for`` of every pair, the same numbers: in uint64 arithmetic (which wraps as the masks do) for many rows."""
+    if len(request_ids) < _VECTOR_FROM:
+        return [uniform_for(seed, r, i) for r, i in zip(request_ids, indices)]
+    try:
+        r, i = np.array(request_ids, dtype=np.uint64), np.array(indices, dtype=np.uint64)
+    except (OverflowError, ValueError):  # (an id that is negative or beyond 64 bits)
+        return [uniform_for(seed, r, i) for r, i in zip(request_ids, indices)]
+    with np.errstate(over="ignore"):
+        z = _splitmix64_array(_splitmix64_array(np.uint64(_splitmix64(seed & _MASK)) ^ r) ^ i)
+    return (z >> np.uint64(11)).astype(np.float64) / float(1 << 53)
+
+
 class Sampler:
     def __init__(self, seed: int = 0):
         self.seed = int(seed)
@@ -80,7 +103,7 @@ class Sampler:
         if all(p.greedy for p in params):
             return ops.sample(logits)
         uniform, temperature, top_k, top_p = self._upload(
-            [uniform_for(self.seed, r, i) for r, i in zip(request_ids, indices)],
+            uniforms_for(self.seed, request_ids, indices),
             [max(float(p.temperature), 0.0) for p in params], [int(p.top_k) for p in params],
             [float(p.top_p) for p in params], logits.device)
         return ops.sample(logits, temperature, top_k, top_p, uniform)

@@ -313,3 +313,14 @@ def test_no_more_running_requests_than_a_step_has_tokens_for():
     assert seen[0] == ids[:3] and seen[-1] == ids[3:]
     assert all(len(s.sequences[i].output) == 4 for i in ids)
     m.check_invariants()
+
+
+@pytest.mark.parametrize("n", [1, 11, 12, 64])
+def test_uniform_numbers_of_many_rows_are_those_of_each(n):
+    from from_scratch_inference_engine_amd.sampling.sampler import uniform_for, uniforms_for
+
+    ids, places = [(7919 * i) ** 3 for i in range(n)], [i * i for i in range(n)]
+    for seed in (0, 5, -1, 2 ** 63 + 11, 2 ** 70):
+        assert list(uniforms_for(seed, ids, places)) == [uniform_for(seed, r, i) for r, i in zip(ids, places)]
+    odd = [-3] + ids  # (what does not fit 64 bits unsigned is masked, as for a row alone)
+    assert list(uniforms_for(1, odd, [0] + places)) == [uniform_for(1, r, i) for r, i in zip(odd, [0] + places)]
