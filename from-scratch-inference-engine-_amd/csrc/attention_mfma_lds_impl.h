@@ -158,7 +158,6 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
     // capped scores: a product p becomes (softcap / scale) * tanh(p * scale / softcap), still in the products' units
     const bool capped = softcap > 0.f;
     const float cap_in = capped ? scale / softcap : 0.f, cap_out = capped ? softcap / scale : 0.f;
-    auto score_of = [&](float product) { return capped ? cap_out * tanh_by_exp(product * cap_in) : product; };
     // BIASED: the row's factor, and its head's slope in the units of the products
     float r_in[NT], r_slope[NT];
 
@@ -212,11 +211,20 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
     const int cpp = page_size >> 3;
     const int t = threadIdx.x;
     uint4 kreg[PER_THREAD], vreg[PER_THREAD];
-    int k_dst[PER_THREAD], v_dst[PER_THREAD];
-    int k_key[PER_THREAD], k_pg[PER_THREAD], v_pg[PER_THREAD];
-    int k_in_page[PER_THREAD], v_in_page[PER_THREAD];
+    // Heads of 256 in pages of 16 fill the registers (the accumulators alone are 128, the queries 64, a block under way 64): with
+    // the seven numbers a piece that the general copy keeps, and a branch for the cap at every score, the compiler moved 219
+    // registers to memory and back in each block.  Here the places of piece i follow from those of piece 0: K's key t / 32 + 8 i
+    // (row 32 (i / 4) + 4 (i % 4) beyond piece 0's), V's dimension t / 2 + 128 (i % 2), both in page i / 2 of the block; with that,
+    // the cap as one branch a block and the wide heads' fragments in turn (below) it is 151 registers, most of them outside the loop
+    // over whole blocks.  16 query heads on one kv head of 256, 2,048 tokens: 390 us before, 169 us now, 5.3 us a block in the
+    // longest workgroup, of which the matrix cores need 1.1: with one wave a SIMD what bounds it is the wait on LDS.
+    constexpr bool AFFINE = HDT == 16 && PS == 16;
+    constexpr int PLACES = AFFINE ? 1 : PER_THREAD;
+    int k_dst[PLACES], v_dst[PLACES];
+    int k_key[PLACES], k_pg[PLACES], v_pg[PLACES];
+    int k_in_page[PLACES], v_in_page[PLACES];
 #pragma unroll
-    for (int i = 0; i < PER_THREAD; ++i) {
+    for (int i = 0; i < PLACES; ++i) {
         const int p = t + kLdsThreads * i;
         k_key[i] = p / (2 * HDT);
         const int k_part = p - k_key[i] * (2 * HDT);
@@ -239,6 +247,20 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
         // probability zero.  Keys past the end inside an existing page are read as they are (the
         // scores of such keys are replaced, not multiplied, and the pools hold finite values only).
         const int kb_page = kb >> page_shift;
+        if constexpr (AFFINE) {
+#pragma unroll
+            for (int j = 0; j < PER_THREAD / 2; ++j) {
+                const int page = table[min(kb_page + j, max_pages - 1)];
+                const bool ok = kb_page + j < max_pages && page >= 0;
+                const uint64_t at = static_cast<uint64_t>(ok ? page : 0) * page_stride;
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    kreg[2 * j + half] = ld16(k_pool + at + 8 * HD * half + static_cast<uint32_t>(k_in_page[0]));
+                    vreg[2 * j + half] = ld16(v_pool + at + 128 * 16 * half + static_cast<uint32_t>(v_in_page[0]));
+                }
+            }
+            return;
+        }
         if constexpr (one_page_per_step<HDT, PS>()) {
             int page[PER_THREAD];
 #pragma unroll
@@ -252,14 +274,14 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
             }
             return;
         }
-        int kpage[PER_THREAD], vpage[PER_THREAD];
+        int kpage[PLACES], vpage[PLACES];
 #pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i) {
+        for (int i = 0; i < PLACES; ++i) {
             kpage[i] = table[min(kb_page + k_pg[i], max_pages - 1)];
             vpage[i] = table[min(kb_page + v_pg[i], max_pages - 1)];
         }
 #pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i) {
+        for (int i = 0; i < PLACES; ++i) {
             const bool kok = kb_page + k_pg[i] < max_pages && kpage[i] >= 0;
             kreg[i] = ld16(k_pool + static_cast<uint64_t>(kok ? kpage[i] : 0) * page_stride + k_in_page[i]);
             const bool vok = kb_page + v_pg[i] < max_pages && vpage[i] >= 0;
@@ -267,8 +289,16 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
         }
     };
     auto stash = [&](int buf) {
+        if constexpr (AFFINE) {
 #pragma unroll
-        for (int i = 0; i < PER_THREAD; ++i) {
+            for (int i = 0; i < PER_THREAD; ++i) {
+                *reinterpret_cast<uint4*>(&k_lds[buf][k_dst[0] + (32 * (i / 4) + 4 * (i % 4)) * KS]) = kreg[i];
+                *reinterpret_cast<uint4*>(&v_lds[buf][v_dst[0] + 128 * VS * (i % 2) + 16 * (i / 2)]) = vreg[i];
+            }
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < PLACES; ++i) {
             *reinterpret_cast<uint4*>(&k_lds[buf][k_dst[i]]) = kreg[i];
             *reinterpret_cast<uint4*>(&v_lds[buf][v_dst[i]]) = vreg[i];
         }
@@ -288,7 +318,7 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
     auto compute_block = [&](int kb, const bf16_t* kbuf, const bf16_t* vbuf, auto inner, bool kept_block) {
         constexpr bool INNER = decltype(inner)::value;
         bool use[2];
-        floatx4 st[2][NT][2];
+        floatx4 st[2][NT][2] = {};  // (a half that the wave does not see stays zero and goes nowhere)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int kh = kb + 32 * h;
@@ -296,6 +326,25 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
             use[h] = INNER || (kept_block ? kh < kept_before
                                           : (kh <= my_last && ((kh < key_end && kh + 32 > key_begin) || kh < kept_in_range)));
             if (!use[h]) continue;
+            if constexpr (HDT > 12) {  // wide heads: one run of 16 keys in registers at a time
+#pragma unroll
+                for (int tt = 0; tt < 2; ++tt) {
+                    const bf16_t* kr = kbuf + (32 * h + 16 * tt + c) * KS + 8 * G;
+                    F16B kf[S32];
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int s = 0; s < S32; ++s) kf[s].raw = *reinterpret_cast<const uint4*>(kr + s * 32);
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt) {
+                        floatx4 a = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int s = 0; s < S32; ++s)
+                            a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s].v, qf[nt][s].v, a, 0, 0, 0);
+                        st[h][nt][tt] = a;
+                    }
+                }
+                continue;
+            }
             F16B kf[2][S32];
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt) {
@@ -314,11 +363,25 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
                     st[h][nt][tt] = a;
                 }
         }
-        // mask and maximum
+        // mask and maximum.  The cap is one branch a block and not one a score.
         float sv[2][NT][8];
         float m_loc[NT];
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) m_loc[nt] = -INFINITY;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) sv[h][nt][i] = BIASED ? st[h][nt][i >> 2][i & 3] * r_in[nt] : st[h][nt][i >> 2][i & 3];
+        if (capped) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) sv[h][nt][i] = cap_out * tanh_by_exp(sv[h][nt][i] * cap_in);
+        }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             if (!use[h]) continue;
@@ -327,17 +390,13 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
                                         (window <= 0 || kh > pos0 + n_q - 1 - window));
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
-                // the score of the i-th of this lane's eight keys
-                const float at_first = BIASED ? r_slope[nt] * static_cast<float>(kh + 8 * G - rpos[nt]) : 0.f;
-                auto score_at = [&](int i) {
-                    const float product = st[h][nt][i >> 2][i & 3];
-                    if constexpr (BIASED) return score_of(product * r_in[nt]) + fmaf(r_slope[nt], static_cast<float>(i), at_first);
-                    else return score_of(product);
-                };
-                if (full) {
+                if constexpr (BIASED) {
+                    // the i-th of this lane's eight keys
+                    const float at_first = r_slope[nt] * static_cast<float>(kh + 8 * G - rpos[nt]);
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) sv[h][nt][i] = score_at(i);
-                } else {
+                    for (int i = 0; i < 8; ++i) sv[h][nt][i] = sv[h][nt][i] + fmaf(r_slope[nt], static_cast<float>(i), at_first);
+                }
+                if (!full) {
 #pragma unroll
                     for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
@@ -347,7 +406,7 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
                                                              : ((key >= key_begin && key < key_end) || key < kept_in_range);
                             const bool vis = rvalid[nt] && in_range && key <= rpos[nt] &&
                                              (window <= 0 || key > rpos[nt] - window || key < keep);
-                            sv[h][nt][tt * 4 + r] = vis ? score_at(tt * 4 + r) : -INFINITY;
+                            sv[h][nt][tt * 4 + r] = vis ? sv[h][nt][tt * 4 + r] : -INFINITY;
                         }
                 }
 #pragma unroll
@@ -403,6 +462,24 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             if (!use[h]) continue;
+            if constexpr (HDT > 12) {  // (32 dimensions at a time)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+                    l_acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones.v, pb[h][nt].v, l_acc[nt], 0, 0, 0);
+#pragma unroll
+                for (int d0 = 0; d0 < HDT; d0 += 2) {
+                    F16B vf[2];
+                    if (d0 % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) vf[i].raw = *reinterpret_cast<const uint4*>(vbuf + ((d0 + i) * 16 + c) * VS + 32 * h + 8 * G);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int nt = 0; nt < NT; ++nt)
+                            acc[nt][d0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[i].v, pb[h][nt].v, acc[nt][d0 + i], 0, 0, 0);
+                }
+                continue;
+            }
             F16B vf[HDT];
 #pragma unroll
             for (int dt = 0; dt < HDT; ++dt)

@@ -683,6 +683,13 @@ def test_attention_over_pages(ops, dtype, scalar, heads, kv, hd, page, window):
         assert (alone - out).abs().max() <= 2.0 ** -7 * out.abs().max()
 
 
+@pytest.mark.parametrize("heads, kv, hd, window", [(8, 1, 256, None), (5, 1, 256, 100), (6, 2, 224, None)])
+def test_attention_of_wide_heads_in_pages_of_16(ops, heads, kv, hd, window):
+    """Heads of 256 in pages of 16 copy their blocks by places that follow from the first piece's, and heads of more
+    than 192 hold fewer fragments at a time: the same sequences and bounds as the other sizes."""
+    test_attention_over_pages(ops, torch.bfloat16, False, heads, kv, hd, 16, window)
+
+
 @pytest.mark.parametrize("heads, kv, seqs", [
     (28, 4, [(0, 4096)]),                # a whole long prompt: 32 groups of four tiles a kv head on the die-mapped grid
     (28, 4, [(4096, 2048), (17000, 1)]),  # a portion behind thousands of cached keys; a decode of 67 splits and their merge
