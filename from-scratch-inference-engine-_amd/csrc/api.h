@@ -229,7 +229,7 @@ int fsie_gemm_mfma_wide_act_takes(int M, int N, int K);
 
 // Products of many rows (prompts), bfloat16 x [M, K] and w [N, K], N a multiple of 16, K of 64, 16-byte aligned:
 //   result 1: gate and up rows of w in turn, y bfloat16 [M, N/2] (act as for fsie_gemm_mfma_wide_gated)
-//   result 2: y float32 partial sums [splits][M][N] of slices of K;  result 0: y bfloat16 [M, N]
+//   result 2: y float32 partial sums [splits][M][N] of slices of K
 // tile 0 .. 3: 128 x 256, 256 x 192, 256 x 256, 256 x 320 rows of x by rows of w a workgroup.
 // fsie_gemm_mfma_tile_plan: tile + 256 * splits, or -1 where the library's product is the faster one.
 int fsie_gemm_mfma_tile_plan(int M, int N, int K, int result, int units);
@@ -321,7 +321,7 @@ int fsie_attention_split_static(const void* q, int64_t q_stride, const void* k_p
 
 int fsie_sample(const float* logits, int n_rows, int vocab, const float* temperature, const int32_t* top_k,
                 const float* top_p, const double* uniform, int32_t* out, hipStream_t stream);
-// The same with every row shared by several workgroups, for vocabularies of 16,384 tokens and more:
+// The same at temperatures with every row shared by several workgroups, where fsie_sample_workspace says so:
 // `workspace` = fsie_sample_workspace(n_rows, vocab) bytes on the device (0: the call is fsie_sample's), uninitialised.
 int64_t fsie_sample_workspace(int n_rows, int vocab);
 int fsie_sample_split(const float* logits, int n_rows, int vocab, const float* temperature, const int32_t* top_k,

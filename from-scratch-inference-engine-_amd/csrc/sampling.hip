@@ -13,7 +13,8 @@
 // the threshold's bin) are bisected over the order-preserving integer image of the logits, a pass a probe.
 // What bounds it is how often a compute unit reads a row of 600 KB from the caches: 2 passes for greedy and
 // plain temperature, 4 with a threshold, where the bisection alone took 32 a threshold (64 rows of 152,064, a fifth
-// of them each greedy, at a temperature, top k, top p and both: 183 us, 1,504 with the bisection alone).
+// of them each greedy, at a temperature, top k, top p and both: 183 us, 1,504 with the bisection alone).  Long rows
+// are shared by several workgroups where the call has few of them (below): 88 us for the same call.
 #include "common.h"
 #include "api.h"
 
@@ -58,13 +59,16 @@ __device__ __forceinline__ Best better(Best a, Best b) {
 }
 
 // `low`, `nan`: this thread's smallest value above -inf, and whether it met a NaN.
+template <bool RANGE>
 __device__ Best block_argmax(const float* row, int vocab, float* sval, int* sidx, float* low, bool* nan) {
     Best best{-INFINITY, 0x7fffffff};
     *low = INFINITY;
     *nan = false;
     auto take = [&](float v, int i) {
-        *nan |= v != v;
-        if (v > -INFINITY) *low = fminf(*low, v);
+        if (RANGE) {
+            *nan |= v != v;
+            if (v > -INFINITY) *low = fminf(*low, v);
+        }
         if (best.index == 0x7fffffff || v > best.value) best = Best{v, i};  // strict: lowest index of a stripe wins
     };
     int done = 0;
@@ -441,6 +445,17 @@ __device__ void draw_from_runs(const float* __restrict__ row, int vocab, Best to
     if (lane == 0) *out = last_kept >= 0 ? last_kept : top.index;  // rounding at the run's end
 }
 
+// Without temperatures: the maximum alone.  A kernel of its own, since the other one's extremes and registers cost this pass
+// twice its time (1 row of 151,936: 9.5 us, 18 in the other; 64 rows: 14 and 21).
+__global__ __launch_bounds__(kThreads) void sample_greedy_kernel(const float* __restrict__ logits, int vocab, int32_t* __restrict__ out) {
+    __shared__ float sval[kWaves];
+    __shared__ int sidx[kWaves];
+    float low;
+    bool nan;
+    const Best top = block_argmax<false>(logits + static_cast<int64_t>(blockIdx.x) * vocab, vocab, sval, sidx, &low, &nan);
+    if (threadIdx.x == 0) out[blockIdx.x] = top.index;
+}
+
 __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restrict__ logits, int vocab,
                                                           const float* __restrict__ temperature,
                                                           const int32_t* __restrict__ top_k,
@@ -457,8 +472,8 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
     const float* row = logits + static_cast<int64_t>(r) * vocab;
     float low;
     bool nan;
-    const Best top = block_argmax(row, vocab, sval, sidx, &low, &nan);
-    const float temp = temperature ? temperature[r] : 0.f;
+    const Best top = block_argmax<true>(row, vocab, sval, sidx, &low, &nan);
+    const float temp = temperature[r];
     if (!(temp > 0.f)) {
         if (threadIdx.x == 0) out[r] = top.index;
         return;
@@ -510,7 +525,16 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
 // tokens on the row's runs are dealt to up to 64 workgroups, and the passes become launches: the maximum; bins (or,
 // for rows without a threshold, the draw's sums); the threshold bins' tokens; the cut; the draw's sums; the draw.
 // What a launch leaves for the next lies in a workspace of the row.
+// A workgroup a row takes the same time up to 256 rows and grows with the row; shared, six launches' ends cost some 30 us
+// and the rest grows with the tokens of all rows.  Alone / shared, us, at 1, 8, 64 and 256 rows:
+//    16,384 tokens   44 / 32    44 / 35    45 /  50    45 /  81
+//    32,000          56 / 33    57 / 37    58 /  52    59 /  94
+//    65,536          84 / 35    84 / 39    86 /  59    90 / 115
+//   152,064         170 / 39   168 / 49   176 /  88   190 / 193
+// so rows are shared from kSplitFrom tokens on while each of them has kTokensForRow for every row of the call.  (Without
+// temperatures it is one pass over the row, and a workgroup a row is the faster one.)
 constexpr int kSplitFrom = 16384;
+constexpr int kTokensForRow = 400;
 constexpr int kPart = 256;          // threads of a shared row's workgroups
 constexpr int kMaxParts = 64;
 constexpr int kPairs = 512;         // so many listed tokens are compared with each other, more are bisected
@@ -536,7 +560,7 @@ struct RowParams {
 __device__ __forceinline__ RowParams row_params(int r, int vocab, const float* temperature, const int32_t* top_k,
                                                 const float* top_p) {
     RowParams q;
-    q.temp = temperature ? temperature[r] : 0.f;
+    q.temp = temperature[r];
     q.inv_temp = 1.0f / q.temp;
     q.k = top_k && top_k[r] > 0 && top_k[r] < vocab ? top_k[r] : 0;
     q.p = top_p ? top_p[r] : 1.f;
@@ -1007,7 +1031,7 @@ __global__ __launch_bounds__(FSIE_WAVE) void split_draw_kernel(const float* __re
 }  // namespace
 
 extern "C" int64_t fsie_sample_workspace(int n_rows, int vocab) {
-    return vocab >= kSplitFrom && n_rows > 0 ? static_cast<int64_t>(n_rows) * static_cast<int64_t>(sizeof(SplitRow)) : 0;
+    return vocab >= kSplitFrom && n_rows > 0 && vocab / n_rows >= kTokensForRow ? static_cast<int64_t>(n_rows) * static_cast<int64_t>(sizeof(SplitRow)) : 0;
 }
 
 extern "C" int fsie_sample(const float* logits, int n_rows, int vocab, const float* temperature,
@@ -1016,7 +1040,8 @@ extern "C" int fsie_sample(const float* logits, int n_rows, int vocab, const flo
     FSIE_REQUIRE(n_rows >= 0 && vocab > 0, "sample: bad sizes rows=%d vocab=%d", n_rows, vocab);
     FSIE_REQUIRE(!temperature || uniform, "sample: temperatures given without uniform numbers");
     if (n_rows == 0) return 0;
-    sample_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, temperature, top_k, top_p, uniform, out);
+    if (temperature) sample_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, temperature, top_k, top_p, uniform, out);
+    else sample_greedy_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, out);
     FSIE_CHECK_LAUNCH("sample");
     return 0;
 }
@@ -1025,7 +1050,7 @@ extern "C" int fsie_sample_split(const float* logits, int n_rows, int vocab, con
                                  const float* top_p, const double* uniform, void* workspace, int32_t* out,
                                  hipStream_t stream) {
     FSIE_REQUIRE(n_rows > 0 && n_rows <= 65535 && vocab > 0, "sample_split: bad sizes rows=%d vocab=%d", n_rows, vocab);
-    FSIE_REQUIRE(!temperature || uniform, "sample_split: temperatures given without uniform numbers");
+    FSIE_REQUIRE(temperature && uniform, "sample_split: temperatures and uniform numbers are needed");
     FSIE_REQUIRE(workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
                  "sample_split: a workspace on 16 bytes is needed");
     SplitRow* ws = static_cast<SplitRow*>(workspace);
@@ -1034,13 +1059,11 @@ extern "C" int fsie_sample_split(const float* logits, int n_rows, int vocab, con
     while (parts < kMaxParts && n_rows * parts < 1024) parts *= 2;
     const dim3 grid(parts, n_rows);
     split_top_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, ws);
-    if (temperature) {
-        split_bins_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
-        if (top_k || top_p) {
-            split_list_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
-            split_cut_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
-            split_runs_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
-        }
+    split_bins_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
+    if (top_k || top_p) {
+        split_list_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
+        split_cut_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
+        split_runs_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
     }
     split_draw_kernel<<<n_rows, FSIE_WAVE, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, uniform, ws, out);
     FSIE_CHECK_LAUNCH("sample_split");
