@@ -5,7 +5,8 @@
 // cache itself; for a long portion the same block is then fetched by every tile of the request,
 // and the kernel is bound by those fetches (L2 to compute unit), far from the matrix cores' rate.
 // Here a workgroup takes up to four consecutive tiles of one request and kv head (32 query rows
-// each: tokens x heads of the group), one per wave.  All 256 threads copy a block of 64 keys and
+// each: tokens x heads of the group), one per wave (two waves a tile for heads of more than 128).
+// All threads copy a block of 64 keys and
 // values from the cache pages into LDS with fully coalesced 16-byte loads (the next block's loads
 // are in flight while the present one is computed: two LDS buffers, one barrier per block); every
 // wave then takes its A operands from LDS.
@@ -43,17 +44,28 @@
 namespace fsie_attn {
 
 constexpr int kLdsKeys = 64;   // keys per block
-constexpr int kLdsWaves = 4;   // waves = tiles per workgroup
-constexpr int kLdsThreads = 64 * kLdsWaves;
+constexpr int kLdsTiles = 4;   // tiles of 32 rows per workgroup
 
-// Whether, with a page size known at compile time, all 256 threads copy from one page in each of
+// Heads of more than 128: two waves a tile, 16 of its rows each.  One wave a tile of a head of 256 holds 128 accumulators,
+// 64 registers of queries and 64 of the block under way, and there is one such wave a SIMD: the compiler moved 219 registers
+// to memory and back in each block of 64 keys, and nothing ran while the wave waited for LDS.  Half the rows a wave leave
+// two waves a SIMD and no register moved; each reads all keys and values, so LDS gives out twice the bytes.  One kv head,
+// 16 query heads, 2,048 tokens, us before / now: heads of 256 360 / 104, 224 322 / 100, 192 195 / 86, 160 114 / 78; a
+// portion of 512 tokens behind 3,000 keys, 256: 590 / 164.  What bounds it now is LDS: 512 KB a block at heads of 256 is
+// 1.7 us of the 3.2 that a block takes, 1.1 of which the matrix cores need.
+template <int HDT>
+constexpr bool two_waves_a_tile() { return HDT > 8; }
+template <int HDT>
+constexpr int lds_threads() { return 64 * kLdsTiles * (two_waves_a_tile<HDT>() ? 2 : 1); }
+
+// Whether, with a page size known at compile time, all threads copy from one page in each of
 // their steps: step i of K and step i of V then both read page i of the block.
 template <int HDT, int PS>
 constexpr bool one_page_per_step() {
     if (PS <= 0) return false;
-    for (int i = 0; i < HDT / 2; ++i)
-        for (int t = 0; t < kLdsThreads; ++t) {
-            const int p = t + kLdsThreads * i;
+    for (int i = 0; i < 128 * HDT / lds_threads<HDT>(); ++i)
+        for (int t = 0; t < lds_threads<HDT>(); ++t) {
+            const int p = t + lds_threads<HDT>() * i;
             if ((p / (2 * HDT)) / PS != i || (p / (PS / 8)) / (HDT * 16) != i) return false;
         }
     return true;
@@ -66,7 +78,7 @@ constexpr bool one_page_per_step() {
 // BIASED: the scores of a token take a factor of its own (row_scale, or null) and a distance bias by the head's slope
 // (slopes, or null): an instantiation of its own, so that the others spend no instruction on it.
 template <int HDT, int PS, bool BIASED>
-__global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT <= 8 ? 2 : 1, HDT <= 8 ? 2 : 1))) void attention_mfma_lds_kernel(
+__global__ __launch_bounds__(lds_threads<HDT>()) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_mfma_lds_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_pool,
     const bf16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_pages,
     const int32_t* __restrict__ items, const int32_t* __restrict__ groups, bf16_t* __restrict__ out, int n_heads,
@@ -76,10 +88,12 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
     constexpr int HD = HDT * 16;
     const int page_size = PS > 0 ? PS : page_size_arg;
     constexpr int S32 = HDT / 2;       // 32-wide steps over the head dimension
-    constexpr int NT = 2;              // query tiles of 16 rows per wave
+    constexpr int THREADS = lds_threads<HDT>();
+    constexpr int NT = two_waves_a_tile<HDT>() ? 1 : 2;  // query tiles of 16 rows per wave
     constexpr int KS = HD + FSIE_LDS_KPAD;         // elements per key row in LDS (padded against bank conflicts)
     constexpr int VS = kLdsKeys + FSIE_LDS_VPAD;   // elements per dimension row of V^T in LDS
-    constexpr int PER_THREAD = HDT / 2;  // 16-byte pieces of K, and of V, per thread and block
+    constexpr int PIECES = 128 * HDT;                     // 16-byte pieces of K, and of V, per block
+    constexpr int PER_THREAD = (PIECES + THREADS - 1) / THREADS;  // 16-byte pieces of K, and of V, per thread and block
     __shared__ __attribute__((aligned(16))) bf16_t k_lds[2][kLdsKeys * KS];
     __shared__ __attribute__((aligned(16))) bf16_t v_lds[2][HD * VS];
 
@@ -115,9 +129,10 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
     const int g_idx = n_groups - 1 - g_lin;
     const int first = groups[2 * g_idx], n_tiles = groups[2 * g_idx + 1];
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
-    const bool active = wave < n_tiles;
-    const int32_t* item = items + static_cast<int64_t>(first + (active ? wave : 0)) * FSIE_ATTN_ITEM_INTS;
+    const int tile = threadIdx.x / (64 * 2 / NT);                           // the wave's tile of the group
+    const int row_base = NT == 1 ? (threadIdx.x >> 6 & 1) * 16 : 0;         // and its rows of the tile
+    const bool active = tile < n_tiles;
+    const int32_t* item = items + static_cast<int64_t>(first + (active ? tile : 0)) * FSIE_ATTN_ITEM_INTS;
     // the same for every lane of the wave: kept in scalar registers, so that what is decided by
     // them is a scalar branch and not a masked region
     const int q_row0 = __builtin_amdgcn_readfirstlane(item[FSIE_ATTN_ITEM_QROW]);
@@ -167,7 +182,7 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
     F16B qf[NT][S32];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-        const int rg = nt * 16 + c;
+        const int rg = row_base + nt * 16 + c;
         const int tq = rg / gh, hh = rg - tq * gh;
         rvalid[nt] = active && rg < n_rows && hh < gh_here;
         rtok[nt] = tq;
@@ -211,21 +226,13 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
     const int cpp = page_size >> 3;
     const int t = threadIdx.x;
     uint4 kreg[PER_THREAD], vreg[PER_THREAD];
-    // Heads of 256 in pages of 16 fill the registers (the accumulators alone are 128, the queries 64, a block under way 64): with
-    // the seven numbers a piece that the general copy keeps, and a branch for the cap at every score, the compiler moved 219
-    // registers to memory and back in each block.  Here the places of piece i follow from those of piece 0: K's key t / 32 + 8 i
-    // (row 32 (i / 4) + 4 (i % 4) beyond piece 0's), V's dimension t / 2 + 128 (i % 2), both in page i / 2 of the block; with that,
-    // the cap as one branch a block and the wide heads' fragments in turn (below) it is 151 registers, most of them outside the loop
-    // over whole blocks.  16 query heads on one kv head of 256, 2,048 tokens: 390 us before, 169 us now, 5.3 us a block in the
-    // longest workgroup, of which the matrix cores need 1.1: with one wave a SIMD what bounds it is the wait on LDS.
-    constexpr bool AFFINE = HDT == 16 && PS == 16;
-    constexpr int PLACES = AFFINE ? 1 : PER_THREAD;
-    int k_dst[PLACES], v_dst[PLACES];
-    int k_key[PLACES], k_pg[PLACES], v_pg[PLACES];
-    int k_in_page[PLACES], v_in_page[PLACES];
+    int k_dst[PER_THREAD], v_dst[PER_THREAD];
+    int k_key[PER_THREAD], k_pg[PER_THREAD], v_pg[PER_THREAD];
+    int k_in_page[PER_THREAD], v_in_page[PER_THREAD];
 #pragma unroll
-    for (int i = 0; i < PLACES; ++i) {
-        const int p = t + kLdsThreads * i;
+    for (int i = 0; i < PER_THREAD; ++i) {
+        // (heads of 160 and 224 leave the last step's second half without a piece: it copies the last one again)
+        const int p = PIECES % THREADS ? min(t + THREADS * i, PIECES - 1) : t + THREADS * i;
         k_key[i] = p / (2 * HDT);
         const int k_part = p - k_key[i] * (2 * HDT);
         // in LDS the keys of a group of 32 lie in the order the lanes read them: key
@@ -247,20 +254,6 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
         // probability zero.  Keys past the end inside an existing page are read as they are (the
         // scores of such keys are replaced, not multiplied, and the pools hold finite values only).
         const int kb_page = kb >> page_shift;
-        if constexpr (AFFINE) {
-#pragma unroll
-            for (int j = 0; j < PER_THREAD / 2; ++j) {
-                const int page = table[min(kb_page + j, max_pages - 1)];
-                const bool ok = kb_page + j < max_pages && page >= 0;
-                const uint64_t at = static_cast<uint64_t>(ok ? page : 0) * page_stride;
-#pragma unroll
-                for (int half = 0; half < 2; ++half) {
-                    kreg[2 * j + half] = ld16(k_pool + at + 8 * HD * half + static_cast<uint32_t>(k_in_page[0]));
-                    vreg[2 * j + half] = ld16(v_pool + at + 128 * 16 * half + static_cast<uint32_t>(v_in_page[0]));
-                }
-            }
-            return;
-        }
         if constexpr (one_page_per_step<HDT, PS>()) {
             int page[PER_THREAD];
 #pragma unroll
@@ -274,14 +267,14 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
             }
             return;
         }
-        int kpage[PLACES], vpage[PLACES];
+        int kpage[PER_THREAD], vpage[PER_THREAD];
 #pragma unroll
-        for (int i = 0; i < PLACES; ++i) {
+        for (int i = 0; i < PER_THREAD; ++i) {
             kpage[i] = table[min(kb_page + k_pg[i], max_pages - 1)];
             vpage[i] = table[min(kb_page + v_pg[i], max_pages - 1)];
         }
 #pragma unroll
-        for (int i = 0; i < PLACES; ++i) {
+        for (int i = 0; i < PER_THREAD; ++i) {
             const bool kok = kb_page + k_pg[i] < max_pages && kpage[i] >= 0;
             kreg[i] = ld16(k_pool + static_cast<uint64_t>(kok ? kpage[i] : 0) * page_stride + k_in_page[i]);
             const bool vok = kb_page + v_pg[i] < max_pages && vpage[i] >= 0;
@@ -289,16 +282,8 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
         }
     };
     auto stash = [&](int buf) {
-        if constexpr (AFFINE) {
 #pragma unroll
-            for (int i = 0; i < PER_THREAD; ++i) {
-                *reinterpret_cast<uint4*>(&k_lds[buf][k_dst[0] + (32 * (i / 4) + 4 * (i % 4)) * KS]) = kreg[i];
-                *reinterpret_cast<uint4*>(&v_lds[buf][v_dst[0] + 128 * VS * (i % 2) + 16 * (i / 2)]) = vreg[i];
-            }
-            return;
-        }
-#pragma unroll
-        for (int i = 0; i < PLACES; ++i) {
+        for (int i = 0; i < PER_THREAD; ++i) {
             *reinterpret_cast<uint4*>(&k_lds[buf][k_dst[i]]) = kreg[i];
             *reinterpret_cast<uint4*>(&v_lds[buf][v_dst[i]]) = vreg[i];
         }
@@ -326,25 +311,6 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
             use[h] = INNER || (kept_block ? kh < kept_before
                                           : (kh <= my_last && ((kh < key_end && kh + 32 > key_begin) || kh < kept_in_range)));
             if (!use[h]) continue;
-            if constexpr (HDT > 12) {  // wide heads: one run of 16 keys in registers at a time
-#pragma unroll
-                for (int tt = 0; tt < 2; ++tt) {
-                    const bf16_t* kr = kbuf + (32 * h + 16 * tt + c) * KS + 8 * G;
-                    F16B kf[S32];
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int s = 0; s < S32; ++s) kf[s].raw = *reinterpret_cast<const uint4*>(kr + s * 32);
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt) {
-                        floatx4 a = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                        for (int s = 0; s < S32; ++s)
-                            a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[s].v, qf[nt][s].v, a, 0, 0, 0);
-                        st[h][nt][tt] = a;
-                    }
-                }
-                continue;
-            }
             F16B kf[2][S32];
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt) {
@@ -363,7 +329,8 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
                     st[h][nt][tt] = a;
                 }
         }
-        // mask and maximum.  The cap is one branch a block and not one a score.
+        // mask and maximum.  The cap is one branch a block and not one a score: 28 heads on 4 kv heads of 128, 2,048 tokens,
+        // 84 us with a branch at each score, 73 so.
         float sv[2][NT][8];
         float m_loc[NT];
 #pragma unroll
@@ -462,24 +429,6 @@ __global__ __launch_bounds__(kLdsThreads) __attribute__((amdgpu_waves_per_eu(HDT
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             if (!use[h]) continue;
-            if constexpr (HDT > 12) {  // (32 dimensions at a time)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-                    l_acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones.v, pb[h][nt].v, l_acc[nt], 0, 0, 0);
-#pragma unroll
-                for (int d0 = 0; d0 < HDT; d0 += 2) {
-                    F16B vf[2];
-                    if (d0 % 4 == 0) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) vf[i].raw = *reinterpret_cast<const uint4*>(vbuf + ((d0 + i) * 16 + c) * VS + 32 * h + 8 * G);
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-#pragma unroll
-                        for (int nt = 0; nt < NT; ++nt)
-                            acc[nt][d0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[i].v, pb[h][nt].v, acc[nt][d0 + i], 0, 0, 0);
-                }
-                continue;
-            }
             F16B vf[HDT];
 #pragma unroll
             for (int dt = 0; dt < HDT; ++dt)
@@ -548,7 +497,7 @@ int launch_lds(const bf16_t* q, int64_t q_stride, const bf16_t* k_pool, const bf
     const bool by_die = ys <= 8 && 8 % ys == 0;
     // by die: every die gets the same number of workgroups, the last ones of which may be empty
     const dim3 grid = by_die ? dim3(static_cast<unsigned>((n_groups + 8 / ys - 1) / (8 / ys)) * 8) : dim3(n_groups, ys);
-    attention_mfma_lds_kernel<HDT, PS, BIASED><<<grid, kLdsThreads, 0, stream>>>(q, q_stride, k_pool, v_pool, block_tables, max_pages,
+    attention_mfma_lds_kernel<HDT, PS, BIASED><<<grid, lds_threads<HDT>(), 0, stream>>>(q, q_stride, k_pool, v_pool, block_tables, max_pages,
                                                                      items, groups, out, n_heads, n_kv, page_size,
                                                                      window, scale, gh, head_chunks, n_groups,
                                                                      by_die ? ys : 0, max(1, fsie_compute_units() / 8), sinks, softcap,

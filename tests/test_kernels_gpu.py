@@ -683,11 +683,13 @@ def test_attention_over_pages(ops, dtype, scalar, heads, kv, hd, page, window):
         assert (alone - out).abs().max() <= 2.0 ** -7 * out.abs().max()
 
 
-@pytest.mark.parametrize("heads, kv, hd, window", [(8, 1, 256, None), (5, 1, 256, 100), (6, 2, 224, None)])
-def test_attention_of_wide_heads_in_pages_of_16(ops, heads, kv, hd, window):
-    """Heads of 256 in pages of 16 copy their blocks by places that follow from the first piece's, and heads of more
-    than 192 hold fewer fragments at a time: the same sequences and bounds as the other sizes."""
-    test_attention_over_pages(ops, torch.bfloat16, False, heads, kv, hd, 16, window)
+@pytest.mark.parametrize("heads, kv, hd, page, window", [(8, 1, 256, 16, None), (5, 1, 256, 16, 100), (16, 1, 192, 16, None),
+                                                         (6, 2, 192, 32, 37), (6, 2, 224, 16, None),
+                                                         (10, 1, 224, 64, 90), (4, 2, 160, 16, None), (3, 1, 160, 8, 61)])
+def test_attention_of_wide_heads(ops, heads, kv, hd, page, window):
+    """Heads of more than 128 give a tile two waves, and those of 160 and 224 copy blocks that are no multiple of the
+    workgroup: the same sequences and bounds as the other sizes."""
+    test_attention_over_pages(ops, torch.bfloat16, False, heads, kv, hd, page, window)
 
 
 @pytest.mark.parametrize("heads, kv, seqs", [
