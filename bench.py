@@ -98,6 +98,8 @@ def kernel_classes(runner, cfg, batch: int, prompt_len: int, itemsize: int) -> d
         "gemm_mfma_skinny": lambda a, k: matrix_class(a[1]), "gemm_mfma_wide": lambda a, k: matrix_class(a[1]),
         "gemm_mfma_wide_swiglu": lambda a, k: "gate_up",
         "gemm": lambda a, k: matrix_class(a[1]), "gemm_mfma_fp32": lambda a, k: matrix_class(a[1]),
+        "gemm_mfma_fp32_sums": lambda a, k: matrix_class(a[1]), "gemm_fp32_tile": lambda a, k: matrix_class(a[1]),
+        "gemm_mfma_tile": lambda a, k: matrix_class(a[1]), "gemm_mfma_tile_gated": lambda a, k: "gate_up",
         "library_mm": lambda a, k: matrix_class(a[1]),
         "swiglu": lambda a, k: "gate_up", "rmsnorm": lambda a, k: "norms", "embedding": lambda a, k: "other",
         "rope_table": lambda a, k: "other", "residual_add": lambda a, k: "other",

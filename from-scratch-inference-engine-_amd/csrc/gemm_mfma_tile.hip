@@ -18,8 +18,8 @@
 // have arrived.
 // What bounds it: a step of 256 x 256 x 64 takes 1.38 us where its matrix instructions alone take 1.04 (v_mfma_f32_16x16x32
 // at 2.07 PFLOP/s over the chip); the LDS is busy for nine tenths of that (24 KB of fragments a wave and step, 64 KB
-// written).  1,320 TFLOP/s at 2,048 x 37888 x 3584 with gate and up multiplied, 1,366 at 8,192 cubed.  The
-// instruction of 32 x 32 x 16, faster by itself, reads the same bytes in a worse pattern: 1,150 and 1,215.
+// written).  1,320 TFLOP/s at 2,048 x 37888 x 3584 with gate and up multiplied.  The instruction
+// of 32 x 32 x 16, faster by itself, reads the same bytes in a worse pattern: 1,150.
 #include "common.h"
 #include "api.h"
 
@@ -45,7 +45,7 @@ struct Shape {
     static constexpr int kUnderWay = kWLoads + 2 * kXLoads;  // loads that are younger than those a wait is for
 };
 
-enum Result { kPlain = 0, kPair = 1, kSums = 2 };
+enum Result { kPair = 1, kSums = 2 };
 
 // 16 bytes a lane from memory to LDS, lane i's at lds + 16 i.  The instruction takes the LDS address from m0.
 __device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t lds, uint32_t offset, uint32_t k_offset) {
@@ -224,32 +224,24 @@ __global__ __launch_bounds__(512, 2) void gemm_tile_kernel(const bf16_t* __restr
             for (int j = 0; j < J; ++j)
                 if (n + 4 * j < N) *reinterpret_cast<floatx4*>(to + 4 * j) = acc[j][t];
         } else {
-            uint32_t out[2 * J];  // J values of a pair's product, or 2 J of the plain one
+            uint32_t out[J];  // two values each, of 4 rows of W
 #pragma unroll
             for (int j = 0; j < J; ++j) {
-                if (RESULT == kPair) {
-                    // gate and up are rounded to 16 bits first, as the library's product leaves them for the pass that
-                    // multiplies them: what a token of a prompt gets does not depend on which of the two its portion takes
-                    const uint32_t a = pack2_bf16(acc[j][t][0], acc[j][t][1]), b = pack2_bf16(acc[j][t][2], acc[j][t][3]);
-                    out[j] = pack2_bf16(gate_pair(__uint_as_float(a << 16), __uint_as_float(a & 0xffff0000u), ACT, act_pos, act_neg),
-                                        gate_pair(__uint_as_float(b << 16), __uint_as_float(b & 0xffff0000u), ACT, act_pos, act_neg));
-                } else {
-                    out[2 * j] = pack2_bf16(acc[j][t][0], acc[j][t][1]);
-                    out[2 * j + 1] = pack2_bf16(acc[j][t][2], acc[j][t][3]);
-                }
+                // gate and up are rounded to 16 bits first, as the library's product leaves them for the pass that
+                // multiplies them: what a token of a prompt gets does not depend on which of the two its portion takes
+                const uint32_t a = pack2_bf16(acc[j][t][0], acc[j][t][1]), b = pack2_bf16(acc[j][t][2], acc[j][t][3]);
+                out[j] = pack2_bf16(gate_pair(__uint_as_float(a << 16), __uint_as_float(a & 0xffff0000u), ACT, act_pos, act_neg),
+                                    gate_pair(__uint_as_float(b << 16), __uint_as_float(b & 0xffff0000u), ACT, act_pos, act_neg));
             }
-            constexpr int kWords = RESULT == kPair ? J : 2 * J;      // of two values, for 4 J rows of W
-            constexpr int kRowsOfWord = RESULT == kPair ? 4 : 2;
-            uint32_t* to = reinterpret_cast<uint32_t*>(static_cast<bf16_t*>(y) + (RESULT == kPair ? static_cast<int64_t>(m) * (N / 2) + n / 2
-                                                                                                 : static_cast<int64_t>(m) * N + n));
-            if (kWords % 4 == 0) {  // (N is a multiple of 16: 16 neighbours are all in or all out)
+            uint32_t* to = reinterpret_cast<uint32_t*>(static_cast<bf16_t*>(y) + static_cast<int64_t>(m) * (N / 2) + n / 2);
+            if constexpr (J % 4 == 0) {  // (N is a multiple of 16: 16 neighbours are all in or all out)
 #pragma unroll
-                for (int i = 0; i < kWords; i += 4)
-                    if (n + i * kRowsOfWord < N) *reinterpret_cast<uint4*>(to + i) = uint4{out[i], out[i + 1], out[i + 2], out[i + 3]};
+                for (int j = 0; j < J; j += 4)
+                    if (n + 4 * j < N) *reinterpret_cast<uint4*>(to + j) = uint4{out[j], out[j + 1], out[j + 2], out[j + 3]};
             } else {
 #pragma unroll
-                for (int i = 0; i < kWords; ++i)
-                    if (n + i * kRowsOfWord < N) to[i] = out[i];
+                for (int j = 0; j < J; ++j)
+                    if (n + 4 * j < N) to[j] = out[j];
             }
         }
     }
@@ -306,7 +298,7 @@ int launch_shape(int tile, const Call& c) {
 // (208 / 226 at 2,048 x 4096 x 14336), and where the tiles alone fill the units too (427 / 456 at 4,096 x 4096 x 18944).
 // The sums' own bytes, written here and read by the norm, count at 4.5 TB/s.
 extern "C" int fsie_gemm_mfma_tile_plan(int M, int N, int K, int result, int units) {
-    if (M <= 0 || N <= 0 || K <= 0 || units <= 0 || N % 16 || K % kStep || result == kPlain) return -1;
+    if (M <= 0 || N <= 0 || K <= 0 || units <= 0 || N % 16 || K % kStep || (result != kPair && result != kSums)) return -1;
     if (static_cast<int64_t>(M) * K * 2 >= (int64_t{1} << 31) || static_cast<int64_t>(N) * K * 2 >= (int64_t{1} << 31)) return -1;
     const int rows[4] = {128, 256, 256, 256}, cols[4] = {256, 192, 256, 320};
     const double us_a_step[4] = {0.90, 1.10, 1.38, 1.78};
@@ -338,7 +330,7 @@ extern "C" int fsie_gemm_mfma_tile(const void* x, const void* w, void* y, int M,
                                    int tile, int act, float act_pos, float act_neg, hipStream_t stream) {
     FSIE_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_mfma_tile: bad sizes M=%d N=%d K=%d", M, N, K);
     FSIE_REQUIRE(N % 16 == 0 && K % kStep == 0, "gemm_mfma_tile: N=%d must be a multiple of 16, K=%d of %d", N, K, kStep);
-    FSIE_REQUIRE(result == kPlain || result == kPair || result == kSums, "gemm_mfma_tile: unknown result %d", result);
+    FSIE_REQUIRE(result == kPair || result == kSums, "gemm_mfma_tile: unknown result %d", result);
     FSIE_REQUIRE(splits >= 1 && splits <= K / kStep && (splits == 1 || result == kSums), "gemm_mfma_tile: %d slices", splits);
     FSIE_REQUIRE(tile >= 0 && tile <= 3, "gemm_mfma_tile: unknown tile %d", tile);
     FSIE_REQUIRE(result != kPair || FSIE_PAIR_KNOWN(act), "gemm_mfma_tile: unknown activation %d", act);
@@ -348,7 +340,6 @@ extern "C" int fsie_gemm_mfma_tile(const void* x, const void* w, void* y, int M,
                      reinterpret_cast<uintptr_t>(y) % 16 == 0, "gemm_mfma_tile: operands must be 16-byte aligned");
     if (M == 0) return 0;
     const Call c{static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), y, M, N, K, splits, act_pos, act_neg, stream};
-    if (result == kPlain) return launch_shape<kPlain, 0>(tile, c);
     if (result == kSums) return launch_shape<kSums, 0>(tile, c);
     switch (act) {
         case FSIE_ACT_SILU: return launch_shape<kPair, FSIE_ACT_SILU>(tile, c);
