@@ -7,7 +7,7 @@
 // tokens of one request, a range of keys, and where the result goes: the output (normalised), or a
 // partial record (unnormalised sum, running maximum, denominator) that attention_merge combines
 // when a key range was split over several items.  grid = (items, kv_heads * head_chunks); a block
-// holds rows = tokens x heads of one kv head's group (gh heads per chunk), four rows per wave.
+// holds rows = tokens x heads of one kv head's group (gh heads per chunk), two rows of each eight per wave.
 //
 // Page layout: keys [page][kv_head][slot][head_dim], values [page][kv_head][head_dim][slot]; block_tables[seq * max_pages + i] = page id of the
 // request's i-th page, or -1 where a window has passed.
@@ -48,6 +48,10 @@ __device__ __forceinline__ void load4(const bf16_t* p, float (&f)[4]) {
 // VEC: the head size and the page size are multiples of 4 and the pools are aligned for load4, so a
 // thread copies four values of a key (along the head) or of a dimension (four consecutive slots of a
 // page; only for items whose first key is a multiple of 4, else element by element) with one load.
+// What bounds it is LDS: a score reads two values a product, and an item's chain of tiles is serial.  16-byte reads
+// of both, the rows of a pass spread over all four waves (a decode's 7 heads take one pass, not two in two waves) and passes
+// without rows left out halved it, with the same sums in the same order.  Float32, us before / now: 4 requests of 300 keys,
+// 14 heads on 2 of 64 24 / 12, 28 on 4 of 128 39 / 18, 16 on 1 of 256 71 / 39; a prompt of 300 tokens 99 / 62, 180 / 106, 322 / 160.
 template <typename T, bool VEC, int MAXC>
 __global__ __launch_bounds__(256) void attention_scalar_kernel(
     const T* __restrict__ q, int64_t q_stride, const T* __restrict__ k_pool, const T* __restrict__ v_pool,
@@ -57,11 +61,12 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
     const T* __restrict__ k_pooled, const T* __restrict__ v_pooled, const int32_t* __restrict__ pooled_tables,
     int pooled_max_pages, int pooled_page_size, int pooled_tokens, const float* __restrict__ slopes,
     const float* __restrict__ row_scale) {
-    extern __shared__ float lds[];
+    extern __shared__ __attribute__((aligned(16))) float lds[];
     float* qs = lds;                          // [kRows][hd]
-    float* kv = qs + kRows * hd;              // [kKeys][hd + 1]
-    float* ps = kv + kKeys * (hd + 1);        // [kRows][kKeys]
-    const int kv_stride = hd + 1;
+    // rows of keys and values: with 16-byte accesses four floats apart, so that eight lanes' rows meet eight groups of banks
+    const int kv_stride = VEC ? hd + 4 : hd + 1;
+    float* kv = qs + kRows * hd;              // [kKeys][kv_stride]
+    float* ps = kv + kKeys * kv_stride;       // [kRows][kKeys]
 
     const int32_t* item = items + static_cast<int64_t>(blockIdx.x) * FSIE_ATTN_ITEM_INTS;
     const int seq = item[FSIE_ATTN_ITEM_SEQ];
@@ -111,7 +116,7 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
     float m_run[2], l_run[2], acc[2][MAXC];
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-        const int r = wave * 4 + p * 2 + sub;
+        const int r = p * 8 + wave * 2 + sub;
         const bool row_ok = r < n_rows && (r % gh) < gh_here;
         r_scale[p] = row_ok && row_scale ? scale * row_scale[q_row0 + r / gh] : scale;
         r_slope[p] = row_ok && slopes ? slopes[h_base + (r % gh)] : 0.f;
@@ -149,7 +154,7 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
                         load4(k_pool + ((static_cast<int64_t>(page) * n_kv + kvh) * page_size + kj % page_size) * hd + d, f);
                 }
                 float* dst = kv + j * kv_stride + d;
-                dst[0] = f[0], dst[1] = f[1], dst[2] = f[2], dst[3] = f[3];
+                *reinterpret_cast<float4*>(dst) = float4{f[0], f[1], f[2], f[3]};
             }
         } else {
             for (int e = tid; e < kKeys * hd; e += blockDim.x) {
@@ -169,7 +174,8 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
         float corr[2];
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
-            const int r = wave * 4 + p * 2 + sub;
+            if (p * 8 >= n_rows) continue;  // the same for the whole workgroup
+            const int r = p * 8 + wave * 2 + sub;
             const bool row_ok = r < n_rows && (r % gh) < gh_here;
             const int pos = pos0 + r / gh;
             const int kj = kt + lane32;
@@ -181,7 +187,18 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
                 const float* qr = qs + r * hd;
                 const float* kr = kv + lane32 * kv_stride;
                 float dot = 0.f;
-                for (int d = 0; d < hd; ++d) dot = fmaf(qr[d], kr[d], dot);
+                if (VEC) {
+#pragma unroll 8
+                    for (int d = 0; d < hd; d += 4) {
+                        const float4 a = *reinterpret_cast<const float4*>(qr + d), b = *reinterpret_cast<const float4*>(kr + d);
+                        dot = fmaf(a.x, b.x, dot);
+                        dot = fmaf(a.y, b.y, dot);
+                        dot = fmaf(a.z, b.z, dot);
+                        dot = fmaf(a.w, b.w, dot);
+                    }
+                } else {
+                    for (int d = 0; d < hd; ++d) dot = fmaf(qr[d], kr[d], dot);
+                }
                 s = dot * r_scale[p];
                 if (softcap > 0.f) s = softcap * tanhf(s / softcap);  // capped scores: softcap * tanh(s / softcap)
                 if (slopes) s = fmaf(r_slope[p], static_cast<float>(kj - pos), s);
@@ -226,14 +243,21 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
         __syncthreads();
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
-            const int r = wave * 4 + p * 2 + sub;
-            const float* pr = ps + r * kKeys;
+            if (p * 8 >= n_rows) continue;
+            const int r = p * 8 + wave * 2 + sub;
+            float pr[kKeys];
+#pragma unroll
+            for (int j = 0; j < kKeys; j += 4) {
+                const float4 four = *reinterpret_cast<const float4*>(ps + r * kKeys + j);
+                pr[j] = four.x, pr[j + 1] = four.y, pr[j + 2] = four.z, pr[j + 3] = four.w;
+            }
 #pragma unroll
             for (int i = 0; i < MAXC; ++i) {
                 if (i < n_chunks) {
                     const int d = lane32 + 32 * i;
                     float a = acc[p][i] * corr[p];
                     if (d < hd) {
+#pragma unroll
                         for (int j = 0; j < kKeys; ++j) a = fmaf(pr[j], kv[j * kv_stride + d], a);
                     }
                     acc[p][i] = a;
@@ -246,7 +270,7 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
     // results
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-        const int r = wave * 4 + p * 2 + sub;
+        const int r = p * 8 + wave * 2 + sub;
         if (!(r < n_rows && (r % gh) < gh_here)) continue;
         const int tq = r / gh, hq = h_base + (r % gh);
         if (partial_base < 0) {
@@ -483,7 +507,7 @@ extern "C" int fsie_attention_scalar(const void* q, int64_t q_stride, const void
     const int gh = group < kRows ? group : kRows;
     const int head_chunks = (group + gh - 1) / gh;
     const dim3 grid(n_items, n_kv * head_chunks);
-    const size_t lds = sizeof(float) * (static_cast<size_t>(kRows) * head_dim + kKeys * (head_dim + 1) + kRows * kKeys);
+    const size_t lds = sizeof(float) * (static_cast<size_t>(kRows) * head_dim + kKeys * (head_dim + 4) + kRows * kKeys);
     const bool vec = head_dim % 4 == 0 && page_size % 4 == 0 && reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(v_pool) % 16 == 0 && reinterpret_cast<uintptr_t>(k_pooled) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(v_pooled) % 16 == 0;
