@@ -20,7 +20,7 @@ namespace {
 
 constexpr int kRows = 16;      // query rows per block
 constexpr int kKeys = 32;      // keys per tile
-constexpr int kMaxChunks = 8;       // head_dim <= 32 * 8: the usual instantiation
+constexpr int kMaxChunks = 8;       // head_dim <= 32 * 8 (with 16-byte accesses 2 and 4 have instantiations of their own)
 constexpr int kMaxChunksWide = 16;  // head_dim <= 32 * 16
 
 __device__ __forceinline__ float half_wave_max(float v) {
@@ -50,8 +50,10 @@ __device__ __forceinline__ void load4(const bf16_t* p, float (&f)[4]) {
 // page; only for items whose first key is a multiple of 4, else element by element) with one load.
 // What bounds it is LDS: a score reads two values a product, and an item's chain of tiles is serial.  16-byte reads
 // of both, the rows of a pass spread over all four waves (a decode's 7 heads take one pass, not two in two waves) and passes
-// without rows left out halved it, with the same sums in the same order.  Float32, us before / now: 4 requests of 300 keys,
-// 14 heads on 2 of 64 24 / 12, 28 on 4 of 128 39 / 18, 16 on 1 of 256 71 / 39; a prompt of 300 tokens 99 / 62, 180 / 106, 322 / 160.
+// without rows left out halved it, with the same sums in the same order; and an instantiation for heads of up to 64 and
+// 128 values has the registers to keep the next loads under way.  Float32, us at the start / with the reads / now: 4 requests of
+// 300 keys, 14 heads on 2 of 64 24 / 12 / 11, 28 on 4 of 128 39 / 18 / 16, 16 on 1 of 256 71 / 39 / 33; a prompt of 300 tokens
+// 99 / 62 / 54, 181 / 106 / 95, 322 / 160 / 135.
 template <typename T, bool VEC, int MAXC>
 __global__ __launch_bounds__(256) void attention_scalar_kernel(
     const T* __restrict__ q, int64_t q_stride, const T* __restrict__ k_pool, const T* __restrict__ v_pool,
@@ -61,6 +63,7 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
     const T* __restrict__ k_pooled, const T* __restrict__ v_pooled, const int32_t* __restrict__ pooled_tables,
     int pooled_max_pages, int pooled_page_size, int pooled_tokens, const float* __restrict__ slopes,
     const float* __restrict__ row_scale) {
+    constexpr bool AHEAD = MAXC <= 4;  // (heads of more than 128 fetch where they store: their registers bound the occupancy)
     extern __shared__ __attribute__((aligned(16))) float lds[];
     float* qs = lds;                          // [kRows][hd]
     // rows of keys and values: with 16-byte accesses four floats apart, so that eight lanes' rows meet eight groups of banks
@@ -126,6 +129,18 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
         for (int i = 0; i < MAXC; ++i) acc[p][i] = 0.f;
     }
     const int n_chunks = (hd + 31) / 32;
+    // VEC: the i-th four values that a thread copies of a tile's keys (four values of a key each; key kKeys: none)
+    int k_key[MAXC], k_dim[MAXC];
+    if (VEC) {
+        const int per_key = hd >> 2, step_keys = 256 / per_key, step_dims = 256 - step_keys * per_key;
+        int j = tid / per_key, d = tid - j * per_key;
+#pragma unroll
+        for (int i = 0; i < MAXC; ++i) {
+            k_key[i] = min(j, kKeys), k_dim[i] = 4 * d;
+            j += step_keys, d += step_dims;
+            if (d >= per_key) d -= per_key, ++j;
+        }
+    }
     const int32_t* own_table = block_tables + static_cast<int64_t>(seq) * max_pages;
     const int own_page_size = page_size;
     const T* const own_k = k_pool;
@@ -140,22 +155,46 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
     const T* const k_pool = pooled ? k_pooled : own_k;
     const T* const v_pool = pooled ? v_pooled : own_v;
     const bool slots_by_four = VEC && (seg_begin & 3) == 0 && (page_size & 3) == 0;
+    const int page_shift = (page_size & (page_size - 1)) == 0 ? __ffs(page_size) - 1 : -1;
+    auto page_of = [&](int kj) { return page_shift >= 0 ? kj >> page_shift : kj / page_size; };
+    // VEC: what a thread copies of a tile's keys, and then of its values, passes through these registers, and (AHEAD) is
+    // under way there: the values while the tile is scored, the next tile's keys while its values are added up.
+    float ahead[MAXC][4];
+    auto fetch_keys = [&](int kt) {
+#pragma unroll
+        for (int i = 0; i < MAXC; ++i) {
+            if (i >= n_chunks) continue;
+            const int j = k_key[i], kj = kt + j;
+            ahead[i][0] = ahead[i][1] = ahead[i][2] = ahead[i][3] = 0.f;
+            if (j < kKeys && kj < seg_end) {
+                const int pg = page_of(kj), page = table[pg];
+                if (page >= 0)
+                    load4(k_pool + ((static_cast<int64_t>(page) * n_kv + kvh) * page_size + (kj - pg * page_size)) * hd + k_dim[i], ahead[i]);
+            }
+        }
+    };
+    auto fetch_values = [&](int kt) {
+        const int kj = kt + 4 * (tid & (kKeys / 4 - 1));  // a multiple of 4: the four slots lie in one page
+        const int pg = page_of(kj), page = kj < seg_end ? table[pg] : -1;
+        const T* from = v_pool + ((static_cast<int64_t>(page) * n_kv + kvh) * hd) * page_size + (kj - pg * page_size);
+#pragma unroll
+        for (int i = 0; i < MAXC; ++i) {
+            if (i >= n_chunks) continue;
+            const int d = tid / (kKeys / 4) + 32 * i;
+            ahead[i][0] = ahead[i][1] = ahead[i][2] = ahead[i][3] = 0.f;
+            if (page >= 0 && d < hd) load4(from + static_cast<int64_t>(d) * page_size, ahead[i]);
+        }
+    };
+    if (VEC && AHEAD) fetch_keys(seg_begin);
     for (int kt = seg_begin; kt < seg_end; kt += kKeys) {
         __syncthreads();  // previous tile's values are no longer read (first pass: qs is written)
         if (VEC) {
-            const int per_key = hd >> 2;
-            for (int e = tid; e < kKeys * per_key; e += blockDim.x) {
-                const int j = e / per_key, d = (e - j * per_key) * 4;
-                const int kj = kt + j;
-                float f[4] = {0.f, 0.f, 0.f, 0.f};
-                if (kj < seg_end) {
-                    const int page = table[kj / page_size];
-                    if (page >= 0)
-                        load4(k_pool + ((static_cast<int64_t>(page) * n_kv + kvh) * page_size + kj % page_size) * hd + d, f);
-                }
-                float* dst = kv + j * kv_stride + d;
-                *reinterpret_cast<float4*>(dst) = float4{f[0], f[1], f[2], f[3]};
-            }
+            if (!AHEAD) fetch_keys(kt);
+#pragma unroll
+            for (int i = 0; i < MAXC; ++i)
+                if (i < n_chunks && k_key[i] < kKeys)
+                    *reinterpret_cast<float4*>(kv + k_key[i] * kv_stride + k_dim[i]) = float4{ahead[i][0], ahead[i][1], ahead[i][2], ahead[i][3]};
+            if (AHEAD && slots_by_four) fetch_values(kt);
         } else {
             for (int e = tid; e < kKeys * hd; e += blockDim.x) {
                 const int j = e / hd, d = e - j * hd;
@@ -181,7 +220,7 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
             const int kj = kt + lane32;
             bool visible = row_ok && kj < seg_end && kj <= pos && (window <= 0 || kj > pos - window || kj < keep);
             if (pooled) visible = row_ok && kj < seg_end && (kj + 1) * pooled_tokens <= pos - window + 1;
-            if (visible) visible = table[kj / page_size] >= 0;
+            if (visible) visible = table[page_of(kj)] >= 0;
             float s = -INFINITY;
             if (visible) {
                 const float* qr = qs + r * hd;
@@ -214,17 +253,14 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
         if (slots_by_four) {
             // a page of values is [head_dim][page_size]: consecutive threads take the eight groups of
             // four keys of a dimension, then the next dimension
-            for (int e = tid; e < (kKeys / 4) * hd; e += blockDim.x) {
-                const int g = e & (kKeys / 4 - 1), d = e / (kKeys / 4);
-                const int kj = kt + 4 * g;  // a multiple of 4: the four slots lie in one page
-                float f[4] = {0.f, 0.f, 0.f, 0.f};
-                if (kj < seg_end) {
-                    const int page = table[kj / page_size];
-                    if (page >= 0)
-                        load4(v_pool + ((static_cast<int64_t>(page) * n_kv + kvh) * hd + d) * page_size + kj % page_size, f);
-                }
+            if (!AHEAD) fetch_values(kt);
+            const int g = tid & (kKeys / 4 - 1);
 #pragma unroll
-                for (int t = 0; t < 4; ++t) kv[(4 * g + t) * kv_stride + d] = kj + t < seg_end ? f[t] : 0.f;
+            for (int i = 0; i < MAXC; ++i) {
+                const int d = tid / (kKeys / 4) + 32 * i;
+                if (i >= n_chunks || d >= hd) continue;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) kv[(4 * g + t) * kv_stride + d] = kt + 4 * g + t < seg_end ? ahead[i][t] : 0.f;
             }
         } else {
             for (int e = tid; e < kKeys * hd; e += blockDim.x) {
@@ -240,6 +276,7 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
                 kv[j * kv_stride + d] = v;
             }
         }
+        if (VEC && AHEAD && kt + kKeys < seg_end) fetch_keys(kt + kKeys);
         __syncthreads();
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
@@ -529,13 +566,13 @@ extern "C" int fsie_attention_scalar(const void* q, int64_t q_stride, const void
                                            pooled_page_size, pooled_tokens, slopes, row_scale);                      \
     } while (0)
 #define FSIE_SCALAR_ATTENTION_OF(T)                                          \
-    if (wide) {                                                              \
-        if (vec) FSIE_SCALAR_ATTENTION(T, true, kMaxChunksWide);             \
-        else FSIE_SCALAR_ATTENTION(T, false, kMaxChunksWide);                \
-    } else {                                                                 \
-        if (vec) FSIE_SCALAR_ATTENTION(T, true, kMaxChunks);                 \
+    if (!vec) {                                                              \
+        if (wide) FSIE_SCALAR_ATTENTION(T, false, kMaxChunksWide);           \
         else FSIE_SCALAR_ATTENTION(T, false, kMaxChunks);                    \
-    }
+    } else if (wide) FSIE_SCALAR_ATTENTION(T, true, kMaxChunksWide);         \
+    else if (head_dim > 128) FSIE_SCALAR_ATTENTION(T, true, kMaxChunks);     \
+    else if (head_dim > 64) FSIE_SCALAR_ATTENTION(T, true, 4);               \
+    else FSIE_SCALAR_ATTENTION(T, true, 2);
     if (dtype == FSIE_F32) {
         FSIE_SCALAR_ATTENTION_OF(float)
     } else {

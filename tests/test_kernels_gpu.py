@@ -683,6 +683,15 @@ def test_attention_over_pages(ops, dtype, scalar, heads, kv, hd, page, window):
         assert (alone - out).abs().max() <= 2.0 ** -7 * out.abs().max()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads, kv, hd, page, window", [(3, 1, 4, 4, None), (20, 2, 36, 16, 21), (9, 1, 64, 12, None),
+                                                         (4, 2, 68, 8, 50), (6, 3, 124, 20, None), (2, 1, 132, 4, None), (2, 1, 252, 16, 90)])
+def test_attention_in_float32_arithmetic_copies_any_head_by_fours(ops, dtype, heads, kv, hd, page, window):
+    """Heads around the instantiations' 64 and 128 values and of no whole run of 32, pages of no power of two, up to
+    eight rows of a workgroup and more: the same sequences and bounds as the other sizes."""
+    test_attention_over_pages(ops, dtype, True, heads, kv, hd, page, window)
+
+
 @pytest.mark.parametrize("heads, kv, hd, page, window", [(8, 1, 256, 16, None), (5, 1, 256, 16, 100), (16, 1, 192, 16, None),
                                                          (6, 2, 192, 32, 37), (6, 2, 224, 16, None),
                                                          (10, 1, 224, 64, 90), (4, 2, 160, 16, None), (3, 1, 160, 8, 61)])
