@@ -15,15 +15,17 @@ from ..ops.functions import (GEMM_MFMA_SKINNY_BEST_M, GEMM_MFMA_SKINNY_MAX_M, GE
 class Linear:
     """Holds ``weight`` [N, K] in the compute dtype and an optional float32 ``bias`` [N].
 
-    float32: the engine's own kernels only (true 32-bit products and sums): vector FMA kernels,
-    and for 3 to 64 rows (decoding) the matrix cores' float32 instruction, which rounds nothing.
+    float32: the engine's own kernels only (true 32-bit products and sums): vector FMA kernels for 1 and 2
+    rows, and from 3 rows on the matrix cores' float32 instruction, which rounds nothing: a kernel that
+    streams W up to 64 rows, one of 64 x 64 tiles beyond; residual projections leave partial sums.
     bfloat16: up to 16 rows (decoding) the engine's matrix-core kernel that streams the weight
     once; its sibling that shares x through LDS for float32 results of 8 to 64 rows (the logits;
     beyond 64 rows the library with a float32 result), for the residual projections
     (``for_residual``: 17 to 64 rows, and any number where K is long) and for the partial sums of
-    other projections of 17 to 64 rows (``partial_sums``); everything else the library product
-    (hipBLASLt through torch, where the reference's engine calls cuBLAS) with float32
-    accumulation, the bias added by a kernel of the engine.  A large weight has a second copy in
+    other projections of 17 to 64 rows (``partial_sums``); residual projections of more than 128 rows whose K is 16,384
+    and more the engine's kernel for many rows, in slices of K (``ops.gemm_tile_plan``); everything else
+    the library product (hipBLASLt through torch, where the reference's engine calls cuBLAS) with
+    float32 accumulation, the bias added by a kernel of the engine.  A large weight has a second copy in
     the order of the matrix instruction's fragments (``prepare``, ``streamed``), from which the
     sibling takes every product of up to 64 rows."""
 
