@@ -324,7 +324,7 @@ __global__ __launch_bounds__(256) void fragment_order_kernel(const u32x4* __rest
 }
 
 // Waves a workgroup and row blocks a wave where the caller leaves them open (0).
-void launch_shape(int mt, int N, int splits, int& waves, int& blocks, bool gate_up = false, bool frags = false) {
+void launch_shape(int mt, int N, int splits, int& waves, int& blocks, bool gate_up = false, bool frags = false, int k_slice = 0) {
     if (gate_up && mt >= 2 && waves == 0 && blocks == 0) {
         // 17 rows and more, one slice: the products and the reads of x from LDS bound a workgroup, so
         // a compute unit with two workgroups takes twice as long as one with one, and a unit draws
@@ -365,8 +365,11 @@ void launch_shape(int mt, int N, int splits, int& waves, int& blocks, bool gate_
         // K = 3584: 8 rows 168 us with two waves, 171 with four, 179 with eight; one row
         // 164 / 168 / 177; N = 152064, K = 5120, 8 rows: 247 / 249 / 259; gate and up of 8 rows: N = 16384, K = 2048 13.1 us with two,
         // 15.1 with four, N = 9728, K = 896 6.7 / 7.4; sums of 8 rows: N = K = 3584 in seven slices 6.4 / 6.8, N = 4608, K = 3584
-        // 7.1 / 7.3, N = 6144, K = 2048 in four 6.1 / 7.0)
-        if (frags && mt == 1 && blocks == 1) waves = 2;  // (on rows, N = 152064: 215 / 195 / 194)
+        // 7.1 / 7.3, N = 6144, K = 2048 in four 6.1 / 7.0).  Not between the many and the
+        // few workgroups, two or three a unit, where they walk a long slice: N = 3584, K = 18944 in eight slices of 2,432
+        // 22.4 us with four waves, 23.3 with two; N = 4096, K = 14336 in eight of 1,792 20.7 / 21.1.
+        const bool few = groups4 <= fsie_compute_units();
+        if (frags && mt == 1 && blocks == 1 && (groups4 >= 1024 || k_slice <= 1024 || few)) waves = 2;  // (on rows, N = 152064: 215 / 195 / 194)
         // two waves a workgroup where that deals the waves more evenly to the compute units (N =
         // 5120 in 8 slices: 640 workgroups of four waves put 12 waves on the fullest of 256 units,
         // 1280 of two put 10; K = 13824, 8 rows: 26.7 against 29.8 us)
@@ -482,7 +485,7 @@ extern "C" int fsie_gemm_mfma_wide(const void* x, const void* w, float* y, int M
     FSIE_REQUIRE(blocks == 0 || blocks == 1 || blocks == 2, "gemm_mfma_wide: blocks must be 0, 1 or 2");
     if (M == 0) return 0;
     const int mt = (M + 15) / 16;
-    launch_shape(mt, N, splits, waves, blocks, false, frags != 0);
+    launch_shape(mt, N, splits, waves, blocks, false, frags != 0, k_slice);
     const bf16_t* xp = static_cast<const bf16_t*>(x);
     const bf16_t* wq = static_cast<const bf16_t*>(w);
     if (frags) return launch_shape_of<SUMS, true>(mt, waves, blocks, xp, wq, y, M, N, K, splits, k_slice, 0, PointEpilogue{}, stream);
@@ -511,7 +514,7 @@ extern "C" int fsie_gemm_mfma_wide_gated(const void* x, const void* w, void* y, 
     FSIE_REQUIRE(blocks == 0 || blocks == 1 || blocks == 2, "gemm_mfma_wide_swiglu: blocks must be 0, 1 or 2");
     if (M == 0) return 0;
     const int mt = (M + 15) / 16;
-    launch_shape(mt, N, 1, waves, blocks, true, frags != 0);
+    launch_shape(mt, N, 1, waves, blocks, true, frags != 0, k_slice);
     const bf16_t* xp = static_cast<const bf16_t*>(x);
     const bf16_t* wq = static_cast<const bf16_t*>(w);
     float* yp = static_cast<float*>(y);
