@@ -590,6 +590,10 @@ __device__ RowTop row_top(const SplitRow* w, int parts) {
         t.low = fminf(t.low, __shfl_xor(t.low, off, FSIE_WAVE));
     }
     t.nan = __any(t.nan);
+    // A NaN is neither larger nor smaller, so lanes that met one may have ended elsewhere than the others: lane 0's answer
+    // (part 0 always has tokens) is the row's, in every wave and every launch, since loops with barriers depend on it.
+    t.best = Best{__shfl(t.best.value, 0, FSIE_WAVE), __shfl(t.best.index, 0, FSIE_WAVE)};
+    t.low = __shfl(t.low, 0, FSIE_WAVE);
     return t;
 }
 

@@ -56,19 +56,27 @@ def test_kept_sets_and_draws(kind, vocab):
             assert got[i] in alt, (kind, vocab, cases[i], got[i], want)
 
 
-def test_rows_that_are_no_numbers_end():
-    """A NaN, an infinite maximum and a row of -inf give some token of the vocabulary."""
+@pytest.mark.parametrize("vocab", [5000, 16500, 40007])  # (a workgroup a row, and rows shared by 64 of them)
+@pytest.mark.parametrize("top_k, top_p", [(20, 0.9), (0, 0.9), (20, 1.0), (0, 1.0)])
+def test_rows_that_are_no_numbers_end(vocab, top_k, top_p):
+    """A NaN (at the first token, inside the row, and first and last of what a workgroup of a shared row has: 512 and 768
+    tokens at these sizes), an infinite maximum and a row of -inf give some token of the vocabulary."""
     from from_scratch_inference_engine_amd import ops
 
     ops.load(build_if_missing=False)
-    x = torch.randn((4, 5000), generator=torch.Generator().manual_seed(0))
+    rows = 8
+    x = torch.randn((rows, vocab), generator=torch.Generator().manual_seed(0))
     x[0, 17] = float("nan")
     x[1, 99] = float("inf")
     x[2, :] = float("-inf")
-    ones = torch.ones(4).cuda()
-    out = ops.sample(x.cuda(), ones, torch.full((4,), 20, dtype=torch.int32).cuda(), 0.9 * ones,
-                     torch.full((4,), 0.5, dtype=torch.float64).cuda()).cpu()
-    assert ((out >= 0) & (out < 5000)).all() and out[1] == 99
+    x[4, 0] = float("nan")
+    x[5, 3072] = x[5, 1536] = float("nan")
+    x[6, 767] = x[6, 511] = x[6, 768] = float("nan")
+    x[7, :] = float("nan")
+    ones = torch.ones(rows).cuda()
+    out = ops.sample(x.cuda(), ones, torch.full((rows,), top_k, dtype=torch.int32).cuda(), top_p * ones,
+                     torch.full((rows,), 0.5, dtype=torch.float64).cuda()).cpu()
+    assert ((out >= 0) & (out < vocab)).all() and out[1] == 99
 
 
 @pytest.mark.parametrize("rows, vocab", [(1, 16500), (3, 16500), (41, 16500), (42, 16500), (64, 40007), (1100, 16500)])
