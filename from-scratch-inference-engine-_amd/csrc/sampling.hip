@@ -9,8 +9,8 @@
 // the row adds up every bin's count and weight in LDS, a scan finds the bin in which the threshold lies, a second pass
 // lays that bin's few hundred tokens side by side, and comparing those with each other gives the token at which the
 // kept set ends.  The bins' weights are integers (two limbs of the float's own bits), so the order in which the threads
-// add them changes nothing.  Rows that do not fit this (a maximum that is not finite, a NaN, more than 2,048 tokens in
-// the threshold's bin) are bisected over the order-preserving integer image of the logits, a pass a probe.
+// add them changes nothing.  Rows that do not fit this (a maximum that is not finite, a NaN, a temperature whose inverse
+// is zero or infinite, so that a weight may be a NaN, more than 2,048 tokens in the threshold's bin) are bisected over the order-preserving integer image of the logits, a pass a probe.
 // What bounds it is how often a compute unit reads a row of 600 KB from the caches: 2 passes for greedy and
 // plain temperature, 4 with a threshold, where the bisection alone took 32 a threshold (64 rows of 152,064, a fifth
 // of them each greedy, at a temperature, top k, top p and both: 183 us, 1,504 with the bisection alone).  Long rows
@@ -118,6 +118,9 @@ __device__ Best block_argmax(const float* row, int vocab, float* sval, int* sidx
 __device__ __forceinline__ double token_weight(float logit, float mx, float inv_temp) {
     return static_cast<double>(expf((logit - mx) * inv_temp));
 }
+
+// whether every token of a row without NaN and with a finite maximum has a weight that is a number
+__device__ __forceinline__ bool weighs(float inv_temp) { return inv_temp > 0.f && inv_temp < INFINITY; }
 
 constexpr int kBins = 2048;        // two a thread
 constexpr int kListed = 2048;      // tokens of one bin that are compared with each other
@@ -245,7 +248,7 @@ __device__ bool cut_by_bins(Binned& s, const float* row, int vocab, float mx, fl
     __syncthreads();
     for (int w = 0; w < kWaves; ++w) low = fminf(low, lowest[w]);
     const float range = fminf(mx - low, kRange);
-    if (odd || !(range > 1e-30f)) return false;
+    if (odd || !(range > 1e-30f) || !weighs(inv_temp)) return false;
     const float scale = static_cast<float>(kBins - 1) / range;
     const int hi_bits = 63 - (32 - __clz(vocab));  // vocab < 2^(32 - clz): the sum of all weights stays below 2^63
     for_row(row, vocab, [&](float v, int) {
@@ -574,9 +577,9 @@ struct RowTop {
     float low;
     bool nan;
     // whether the row's thresholds can be found by bins, and their scale
-    __device__ bool binned(int vocab, float* scale) const {
+    __device__ bool binned(int vocab, float inv_temp, float* scale) const {
         const float range = fminf(best.value - low, kRange);
-        if (vocab > kMaxBinned || nan || !(fabsf(best.value) < INFINITY) || !(range > 1e-30f)) return false;
+        if (vocab > kMaxBinned || nan || !(fabsf(best.value) < INFINITY) || !(range > 1e-30f) || !weighs(inv_temp)) return false;
         *scale = static_cast<float>(kBins - 1) / range;
         return true;
     }
@@ -706,7 +709,7 @@ __global__ __launch_bounds__(kPart) void split_bins_kernel(const float* __restri
         return;
     }
     float scale;
-    if (!top.binned(vocab, &scale)) return;
+    if (!top.binned(vocab, q.inv_temp, &scale)) return;
     for (int b = threadIdx.x; b < kBins; b += kPart) {
         hi[b] = lo[b] = 0;
         count[b] = 0;
@@ -792,7 +795,7 @@ __global__ __launch_bounds__(kPart) void split_list_kernel(const float* __restri
     SplitRow* w = ws + r;
     const RowTop top = row_top(w, parts);
     float scale;
-    if (!top.binned(vocab, &scale)) return;
+    if (!top.binned(vocab, q.inv_temp, &scale)) return;
     const int hi_bits = 63 - (32 - __clz(vocab));
     constexpr int PER = kBins / kPart;
     const int b0 = static_cast<int>(threadIdx.x) * PER;
@@ -881,7 +884,7 @@ __global__ __launch_bounds__(kThreads) void split_cut_kernel(const float* __rest
     const uint32_t key_max = order_key(mx);
     const int n = static_cast<int>(min(w->n_listed, static_cast<unsigned int>(kKeep + 1)));
     float scale = 0.f;
-    bool fits = top.binned(vocab, &scale) && n <= kKeep;  // (the same in every thread)
+    bool fits = top.binned(vocab, q.inv_temp, &scale) && n <= kKeep;  // (the same in every thread)
     uint32_t cut = 0;
     if (fits) {
         const int hi_bits = 63 - (32 - __clz(vocab));

@@ -79,6 +79,24 @@ def test_rows_that_are_no_numbers_end(vocab, top_k, top_p):
     assert ((out >= 0) & (out < vocab)).all() and out[1] == 99
 
 
+@pytest.mark.parametrize("vocab", [300, 5000, 16500])
+@pytest.mark.parametrize("temperature", [float("inf"), 1e-45])
+def test_weights_that_are_no_numbers_leave_the_maximum(vocab, temperature):
+    """At a temperature whose inverse is zero a token at -inf weighs (-inf) * 0, at one whose inverse is infinite the
+    largest weighs 0 * inf: no sum of the row is a number then, and the choice is the largest token."""
+    from from_scratch_inference_engine_amd import ops
+
+    ops.load(build_if_missing=False)
+    rows = 6
+    g = torch.Generator().manual_seed(vocab)
+    x = torch.randn((rows, vocab), generator=g)
+    x = torch.where(torch.rand((rows, vocab), generator=g) < 0.5, x, torch.tensor(float("-inf")))
+    for top_p in (0.1, 0.9, 1.0):
+        out = ops.sample(x.cuda(), torch.full((rows,), temperature).cuda(), torch.zeros(rows, dtype=torch.int32).cuda(),
+                         torch.full((rows,), top_p).cuda(), torch.linspace(0.0, 0.99, rows, dtype=torch.float64).cuda())
+        assert out.cpu().tolist() == x.argmax(1).tolist()
+
+
 @pytest.mark.parametrize("rows, vocab", [(1, 16500), (3, 16500), (41, 16500), (42, 16500), (64, 40007), (1100, 16500)])
 def test_a_row_does_not_depend_on_how_many_workgroups_share_it(rows, vocab):
     from from_scratch_inference_engine_amd import ops
