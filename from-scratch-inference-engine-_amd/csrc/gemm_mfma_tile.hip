@@ -47,14 +47,14 @@ struct Shape {
 
 enum Result { kPair = 1, kSums = 2 };
 
-// 16 bytes a lane from memory to LDS, lane i's at lds + 16 i.  The instruction takes the LDS address from m0.
+// 16 bytes a lane from memory to LDS, lane i's at lds + 16 i.  The instruction takes the LDS address from m0, which is an
+// operand here and written by the compiler; the wait state between that and the load is not, inside an asm statement.
 __device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t lds, uint32_t offset, uint32_t k_offset) {
     asm volatile(
-        "s_mov_b32 m0, %0\n\t"
         "s_nop 0\n\t"
         "buffer_load_dwordx4 %1, %2, %3 offen lds"
         :
-        : "s"(lds), "v"(offset), "s"(rsrc), "s"(k_offset)
+        : "{m0}"(lds), "v"(offset), "s"(rsrc), "s"(k_offset)
         : "memory");
 }
 #define FSIE_TILE_FENCE() __builtin_amdgcn_sched_barrier(0)
