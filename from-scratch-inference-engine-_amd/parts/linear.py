@@ -72,6 +72,12 @@ class Linear:
             if free - w.numel() * 2 >= self.streamed_copy_reserve * total:
                 self.streamed = ops.fragment_order(w)
 
+    def kernel_reads(self, x: torch.Tensor) -> bool:
+        """Whether the engine's 16-byte loads can read ``x`` and the weight as they lie: rows without gaps, on 16 bytes.
+        Where not, a product of many rows goes to the library or the vector kernels, which take any."""
+        w = self._weight
+        return x.is_contiguous() and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
+
     def drop_copy(self) -> int:
         """Forget the fragment-ordered copy (the products then read rows); returns its bytes."""
         if self.streamed is None:
@@ -96,7 +102,8 @@ class Linear:
                 # decoding in the 32-bit path: W streams once into true float32 matrix instructions
                 # (several times faster than the vector kernels from 8 rows on, no faster at one or two)
                 return ops.gemm_mfma_fp32(x, w, bias)
-            if self.float32_on_matrix_cores and m > GEMM_MFMA_SKINNY_MAX_M and self.in_features % 4 == 0:
+            if (self.float32_on_matrix_cores and m > GEMM_MFMA_SKINNY_MAX_M and self.in_features % 4 == 0
+                    and self.kernel_reads(x) and out_dtype in (None, x.dtype)):
                 return ops.gemm_fp32_tile(x, w, bias)  # prompts: the same instruction, both operands through LDS
             return ops.gemm(x, w, bias, out_dtype=out_dtype)
         wants_f32 = out_dtype is not None and out_dtype != x.dtype
@@ -152,14 +159,14 @@ class Linear:
             # 65 to 128 rows of a fragment-ordered weight: the same kernel with five to eight tiles of x,
             # where its launch shape has one
             splits = self.wide_splits(m)
-            if splits > 1 and self.wide_takes(m, splits):
+            if splits > 1 and self.wide_takes(m, splits) and self.kernel_reads(x):
                 return ops.gemm_mfma_wide(x, self.streamed, splits=splits)
         if (getattr(ctx, "partial_sums_ok", False) and x.dtype == torch.bfloat16 and self.bias is None
                 and self.in_features % 8 == 0 and 0 < m <= GEMM_MFMA_SKINNY_MAX_M):
             # the kernel that shares x through LDS: above 16 rows, and at any number of rows where
             # K is long enough for six slices or more
             splits = self.wide_splits(m)
-            if splits > 1 and (m > GEMM_MFMA_SKINNY_BEST_M or splits >= 6 or self.streamed is not None):
+            if splits > 1 and (self.kernel_reads(x) if m > GEMM_MFMA_SKINNY_BEST_M else splits >= 6 or self.streamed is not None):
                 return ops.gemm_mfma_wide(x, self.wide_weight, splits=splits)
             splits = self.residual_splits(m)
             if splits > 1:
@@ -173,13 +180,13 @@ class Linear:
                     return ops.gemm_mfma_fp32_sums(x, self.weight, splits)
             else:
                 splits = ops.gemm_fp32_tile_splits(m, self.out_features, self.in_features)
-                if splits > 1:
+                if splits > 1 and self.kernel_reads(x):
                     return ops.gemm_fp32_tile(x, self.weight, splits=splits)
         if (getattr(ctx, "partial_sums_ok", False) and x.dtype == torch.bfloat16 and self.bias is None
                 and m > GEMM_MFMA_WIDE_MAX_M):
             # prompts and a long K: the product for many rows in slices of K
             plan = ops.gemm_tile_plan(m, self.out_features, self.in_features, ops.GEMM_TILE_SUMS)
-            if plan is not None:
+            if plan is not None and self.kernel_reads(x):
                 return ops.gemm_mfma_tile(x, self.weight, splits=plan[1], tile=plan[0])
         return None
 
@@ -195,6 +202,8 @@ class Linear:
         splits = self.wide_splits(m)
         if splits < 2 or not self.wide_takes(m, splits):
             return None
+        if m > GEMM_MFMA_SKINNY_BEST_M and not self.kernel_reads(x):
+            return None  # (the library's)
         return ops.gemm_mfma_wide(x, self.wide_weight, splits=splits)
 
     def wide_takes(self, m: int, splits: int, gate_up: bool = False) -> bool:

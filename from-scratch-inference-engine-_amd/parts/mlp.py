@@ -82,7 +82,8 @@ class SwiGLU(FeedForward):
         else:
             # prompts: where its tiles fill the chip, the product for many rows with act(gate) * up in its epilogue
             plan = (ops.gemm_tile_plan(m, self.gate_up.out_features, self.hidden_size, ops.GEMM_TILE_PAIR)
-                    if x.dtype == torch.bfloat16 and m > self.streamed_swiglu_max_rows else None)
+                    if x.dtype == torch.bfloat16 and m > self.streamed_swiglu_max_rows and self.gate_up.kernel_reads(x)
+                    else None)
             act = (ops.swiglu(self.gate_up(x), act=self._gate_act) if plan is None else
                    ops.gemm_mfma_tile_gated(x, self.gate_up.weight, act=self._gate_act, tile=plan[0]))
         return self.down.for_residual(act, ctx)

@@ -240,3 +240,57 @@ def test_schedules_and_windows(model_dirs, tmp_path, dtype, calls, window):
         assert rc.pages_held(0) <= -(-(window + 25) // 4) + 1 < 90 // 4
     runner.manager.close(rc)
     runner.manager.check_invariants()
+
+
+@pytest.mark.parametrize("dtype, m, n, k", [
+    (torch.float32, 100, 96, 512),     # tiles of 64 x 64, whole and in slices
+    (torch.bfloat16, 40, 1152, 896),   # slices of a stage of K
+    (torch.bfloat16, 200, 256, 16384), # a prompt's long K in slices
+    (torch.bfloat16, 300, 256, 512),   # the library's
+])
+def test_products_of_many_rows_take_rows_as_they_lie(dtype, m, n, k):
+    """Rows that do not start on 16 bytes, or (bfloat16) lie apart, give what the same rows give packed: within the
+    rounding of float32 sums in another order, and of the result to the type."""
+    from from_scratch_inference_engine_amd import ops
+    from from_scratch_inference_engine_amd.parts.linear import Linear
+
+    ops.load(build_if_missing=False)
+    ctx = Ctx(dtype)
+    ctx.partial_sums_ok = True
+    x, w = rnd((m, k), 1).to(dtype).cuda(), rnd((n, k), 2, scale=0.1).to(dtype).cuda()
+    shifted = torch.empty(m * k + 1, dtype=dtype, device="cuda")[1:].view(m, k).copy_(x)
+    apart = torch.empty((m, k + 8), dtype=dtype, device="cuda")[:, :k].copy_(x)
+    lin = Linear(k, n)
+    whole = x.double() @ w.double().t()
+    bound = (k + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    if dtype == torch.bfloat16:
+        bound = bound + 2.0 ** -8 * whole.abs()
+    for rows in (x, shifted) + ((apart,) if dtype == torch.bfloat16 else ()):
+        lin.weight = w
+        sums = lin.for_residual(rows, ctx).double()
+        assert ((sums.sum(0) if sums.dim() == 3 else sums) - whole).abs().le(bound).all()
+        assert (lin(rows).double() - whole).abs().le(bound).all()
+    lin.weight = torch.empty(n * k + 1, dtype=dtype, device="cuda")[1:].view(n, k).copy_(w)
+    assert (lin(x).double() - whole).abs().le(bound).all() if m > 64 else True
+    if dtype == torch.float32:
+        with pytest.raises(ops.KernelError):
+            lin(x, out_dtype=torch.bfloat16)  # a type that is not offered
+
+
+def test_feed_forward_of_many_rows_takes_rows_as_they_lie():
+    from from_scratch_inference_engine_amd import ops
+    from from_scratch_inference_engine_amd.parts.mlp import SwiGLU
+
+    ops.load(build_if_missing=False)
+    m, h, f = 2048, 896, 4864
+    assert ops.gemm_tile_plan(m, 2 * f, h, ops.GEMM_TILE_PAIR) is not None
+    part = SwiGLU(h, f)
+    part.gate_up_weight, part.down_weight = (rnd(s, i, torch.bfloat16, 0.05).cuda() for i, s in enumerate([(2 * f, h), (h, f)]))
+    x = rnd((m, h), 3, torch.bfloat16).cuda()
+    want = part.forward(x, Ctx(torch.bfloat16)).float()
+    shifted = torch.empty(m * h + 1, dtype=torch.bfloat16, device="cuda")[1:].view(m, h).copy_(x)
+    apart = torch.empty((m, h + 8), dtype=torch.bfloat16, device="cuda")[:, :h].copy_(x)
+    for rows in (shifted, apart):
+        got = part.forward(rows, Ctx(torch.bfloat16)).float()
+        # two products and an activation, each rounded to 8 bits after sums in another order
+        assert (got - want).norm() <= 2.0 ** -7 * want.norm()
