@@ -39,7 +39,10 @@ class Linear:
     # the time).  The rows stay for the library's products of many rows.  None: no copies.
     # A copy that would leave less than ``streamed_copy_reserve`` of the device's memory free is not
     # made: a model that large keeps copies of its first layers only and runs the rest from rows.
+    # From 17 rows on the copy is read of weights of 16 MB and more: where the copies of 8 to 16 MB were read too, decode steps of
+    # 20 and 32 rows at hidden size 2,048 took 2 % longer and at 2,560 1 %, and 65 to 128 rows left the library's faster products.
     streamed_copy_from = 8 << 20
+    streamed_many_rows_from = 16 << 20
     streamed_copy_reserve = 0.25
 
     def __init__(self, in_features: int, out_features: int, bias: bool = False):
@@ -87,10 +90,16 @@ class Linear:
         self._wide_takes = {}
         return freed
 
-    @property
-    def wide_weight(self):
-        """What the products that share x through LDS read: the fragment-ordered copy if there is one."""
-        return self.weight if self.streamed is None else self.streamed
+    def copy_for(self, m: int):
+        """The fragment-ordered copy, if there is one that products of ``m`` rows read."""
+        if self.streamed is None or (m > GEMM_MFMA_SKINNY_BEST_M and self._weight.numel() * 2 < self.streamed_many_rows_from):
+            return None
+        return self.streamed
+
+    def wide_weight(self, m: int):
+        """What the products of ``m`` rows that share x through LDS read: the fragment-ordered copy if there is one for them."""
+        copy = self.copy_for(m)
+        return self.weight if copy is None else copy
 
     def __call__(self, x: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
                  skip_bias: bool = False) -> torch.Tensor:
@@ -114,7 +123,7 @@ class Linear:
                 and ops.gemm_mfma_wide_splits_ok(self.in_features, 1)):
             # float32 results (logits) of 8 to 64 rows: x shared through LDS; from the fragment-ordered
             # copy at any number of rows
-            return ops.gemm_mfma_wide(x, self.wide_weight)
+            return ops.gemm_mfma_wide(x, self.wide_weight(m))
         if (wants_f32 and bias is None and m > GEMM_MFMA_SKINNY_MAX_M and out_dtype == torch.float32
                 and self.in_features % 8 == 0 and self.out_features % 8 == 0):
             # logits of more rows than the engine's kernels take (a decode batch beyond 64, a replay
@@ -153,49 +162,50 @@ class Linear:
 
     def residual_sums(self, x: torch.Tensor, ctx) -> Optional[torch.Tensor]:
         """The partial sums of ``for_residual``, or None where the product is better left whole."""
+        if self.bias is not None or not getattr(ctx, "partial_sums_ok", False):
+            return None
         m = x.shape[0]
-        if (getattr(ctx, "partial_sums_ok", False) and x.dtype == torch.bfloat16 and self.bias is None
-                and GEMM_MFMA_SKINNY_MAX_M < m <= GEMM_MFMA_WIDE_MAX_M and self.streamed is not None):
-            # 65 to 128 rows of a fragment-ordered weight: the same kernel with five to eight tiles of x,
-            # where its launch shape has one
-            splits = self.wide_splits(m)
-            if splits > 1 and self.wide_takes(m, splits) and self.kernel_reads(x):
-                return ops.gemm_mfma_wide(x, self.streamed, splits=splits)
-        if (getattr(ctx, "partial_sums_ok", False) and x.dtype == torch.bfloat16 and self.bias is None
-                and self.in_features % 8 == 0 and 0 < m <= GEMM_MFMA_SKINNY_MAX_M):
-            # the kernel that shares x through LDS: above 16 rows, and at any number of rows where
-            # K is long enough for six slices or more
-            splits = self.wide_splits(m)
-            if splits > 1 and (self.kernel_reads(x) if m > GEMM_MFMA_SKINNY_BEST_M else splits >= 6 or self.streamed is not None):
-                return ops.gemm_mfma_wide(x, self.wide_weight, splits=splits)
-            splits = self.residual_splits(m)
-            if splits > 1:
-                return ops.gemm_mfma_skinny(x, self.weight, splits=splits)
-        if (getattr(ctx, "partial_sums_ok", False) and x.dtype == torch.float32 and self.bias is None
-                and self.float32_on_matrix_cores and m > 2 and self.in_features % 4 == 0):
+        if x.dtype == torch.float32:
             # the 32-bit path: slices of K where the rows of W alone (or a prompt's tiles) leave the chip idle
+            if not self.float32_on_matrix_cores or m <= 2 or self.in_features % 4:
+                return None
             if m <= GEMM_MFMA_SKINNY_MAX_M:
                 splits = ops.gemm_mfma_fp32_splits(self.in_features)
-                if splits > 1:
-                    return ops.gemm_mfma_fp32_sums(x, self.weight, splits)
-            else:
-                splits = ops.gemm_fp32_tile_splits(m, self.out_features, self.in_features)
-                if splits > 1 and self.kernel_reads(x):
-                    return ops.gemm_fp32_tile(x, self.weight, splits=splits)
-        if (getattr(ctx, "partial_sums_ok", False) and x.dtype == torch.bfloat16 and self.bias is None
-                and m > GEMM_MFMA_WIDE_MAX_M):
+                return ops.gemm_mfma_fp32_sums(x, self.weight, splits) if splits > 1 else None
+            splits = ops.gemm_fp32_tile_splits(m, self.out_features, self.in_features)
+            return ops.gemm_fp32_tile(x, self.weight, splits=splits) if splits > 1 and self.kernel_reads(x) else None
+        if x.dtype != torch.bfloat16 or m == 0:
+            return None
+        if m > GEMM_MFMA_WIDE_MAX_M:
             # prompts and a long K: the product for many rows in slices of K
             plan = ops.gemm_tile_plan(m, self.out_features, self.in_features, ops.GEMM_TILE_SUMS)
-            if plan is not None and self.kernel_reads(x):
-                return ops.gemm_mfma_tile(x, self.weight, splits=plan[1], tile=plan[0])
-        return None
+            return (ops.gemm_mfma_tile(x, self.weight, splits=plan[1], tile=plan[0])
+                    if plan is not None and self.kernel_reads(x) else None)
+        if m > GEMM_MFMA_SKINNY_MAX_M:
+            # 65 to 128 rows of a fragment-ordered weight: the same kernel with five to eight tiles of x,
+            # where its launch shape has one
+            if self.copy_for(m) is None:
+                return None
+            splits = self.wide_splits(m)
+            return (ops.gemm_mfma_wide(x, self.streamed, splits=splits)
+                    if splits > 1 and self.wide_takes(m, splits) and self.kernel_reads(x) else None)
+        if self.in_features % 8:
+            return None
+        # the kernel that shares x through LDS: above 16 rows, and at any number of rows where
+        # K is long enough for six slices or more
+        splits = self.wide_splits(m)
+        if splits > 1 and (self.kernel_reads(x) if m > GEMM_MFMA_SKINNY_BEST_M
+                           else self.streamed is not None or splits >= 6):
+            return ops.gemm_mfma_wide(x, self.wide_weight(m), splits=splits)
+        splits = self.residual_splits(m)
+        return ops.gemm_mfma_skinny(x, self.weight, splits=splits) if splits > 1 else None
 
     def partial_sums(self, x: torch.Tensor, few_rows: bool = False) -> Optional[torch.Tensor]:
         """x . W^T (no bias) of 17 to 64 rows (to 128 from a fragment-ordered copy) as float32 partial
         sums [S, T, N] of slices of K, for a consumer that adds them up itself; None where the engine's
         kernel for that does not take the sizes.  ``few_rows``: also for up to 16 rows."""
         m = x.shape[0]
-        most = GEMM_MFMA_SKINNY_MAX_M if self.streamed is None else GEMM_MFMA_WIDE_MAX_M
+        most = GEMM_MFMA_SKINNY_MAX_M if self.copy_for(m) is None else GEMM_MFMA_WIDE_MAX_M
         least = 0 if few_rows else GEMM_MFMA_SKINNY_BEST_M  # (fewer rows: for a consumer that spares a launch by it)
         if x.dtype != torch.bfloat16 or not least < m <= most:
             return None
@@ -204,14 +214,15 @@ class Linear:
             return None
         if m > GEMM_MFMA_SKINNY_BEST_M and not self.kernel_reads(x):
             return None  # (the library's)
-        return ops.gemm_mfma_wide(x, self.wide_weight, splits=splits)
+        return ops.gemm_mfma_wide(x, self.wide_weight(m), splits=splits)
 
     def wide_takes(self, m: int, splits: int, gate_up: bool = False) -> bool:
         """Whether the kernel that shares x through LDS takes ``m`` rows of this weight (beyond 64 rows
         it has kernels for some launch shapes only)."""
-        key = (-(-m // 16), splits, gate_up, self.streamed is not None)
+        weight = self.wide_weight(m)
+        key = (-(-m // 16), splits, gate_up, weight is self.streamed)
         if key not in self._wide_takes:
-            self._wide_takes[key] = ops.gemm_mfma_wide_takes(m, self.wide_weight, splits, gate_up)
+            self._wide_takes[key] = ops.gemm_mfma_wide_takes(m, weight, splits, gate_up)
         return self._wide_takes[key]
 
     def wide_splits(self, m: int) -> int:

@@ -67,7 +67,7 @@ class SwiGLU(FeedForward):
 
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         m = x.shape[0]
-        if (x.dtype == torch.bfloat16 and self.gate_up.streamed is not None and 0 < m <= self.streamed_swiglu_max_rows
+        if (x.dtype == torch.bfloat16 and self.gate_up.copy_for(m) is not None and 0 < m <= self.streamed_swiglu_max_rows
                 and self.gate_up.wide_takes(m, 1, gate_up=True)):
             # from the fragment-ordered copy at any number of rows up to 64, and up to 128 where the
             # kernel has the launch shape for it: SiLU*up in the product's epilogue
@@ -82,10 +82,9 @@ class SwiGLU(FeedForward):
         else:
             # prompts: where its tiles fill the chip, the product for many rows with act(gate) * up in its epilogue
             plan = (ops.gemm_tile_plan(m, self.gate_up.out_features, self.hidden_size, ops.GEMM_TILE_PAIR)
-                    if x.dtype == torch.bfloat16 and m > self.streamed_swiglu_max_rows and self.gate_up.kernel_reads(x)
-                    else None)
-            act = (ops.swiglu(self.gate_up(x), act=self._gate_act) if plan is None else
-                   ops.gemm_mfma_tile_gated(x, self.gate_up.weight, act=self._gate_act, tile=plan[0]))
+                    if x.dtype == torch.bfloat16 and m > self.streamed_swiglu_max_rows else None)
+            act = (ops.gemm_mfma_tile_gated(x, self.gate_up.weight, act=self._gate_act, tile=plan[0])
+                   if plan is not None and self.gate_up.kernel_reads(x) else ops.swiglu(self.gate_up(x), act=self._gate_act))
         return self.down.for_residual(act, ctx)
 
 
@@ -154,7 +153,7 @@ class PlainFeedForward(FeedForward):
     def _activated(self, x: torch.Tensor) -> torch.Tensor:
         m, up = x.shape[0], self.up
         if x.dtype == torch.bfloat16 and m > 0:
-            if (up.streamed is not None and ops.gemm_mfma_wide_act_takes(m, up.streamed)
+            if (up.copy_for(m) is not None and ops.gemm_mfma_wide_act_takes(m, up.streamed)
                     and (m <= 48 or self.intermediate_size <= 32 * ops.compute_units())):
                 # (a full fourth tile of x keeps a unit busy by itself: with more than a workgroup a unit the product in
                 # slices of K, 64 rows of N = 14336, K = 4096 30.7 us against 34.1)
