@@ -430,9 +430,11 @@ extern "C" int fsie_gemm_mfma_wide_best_splits(int M, int N, int K) {
         }
         return best;
     }
-    // a K too short for two slices of 512 is cut finer, for the matrices of small models (40 rows, N = K = 896: 3.4 us in
-    // seven slices, 6.1 whole)
-    const int shortest = K >= 2 * 512 ? 512 : stage;
+    // A K too short for two slices of 512 is cut finer for up to 64 rows of the matrices of small models: with the norm that
+    // adds them up 0.5 to 0.9 of the time that the library's product takes (N = 512 to 4,096, K = 256 to 896; N = K = 896,
+    // 40 rows: 6.6 us, 11.1).  Not beyond: the sums of 9,728 rows of W weigh more than its product (K = 896, 64 rows 15.5 us,
+    // the library's 11.8), and at 65 to 128 rows they lose at 6,144 (K = 896, 128 rows 21 / 12).
+    const int shortest = K >= 2 * 512 || mt > 4 || N > 4096 ? 512 : stage;
     int best = 1;
     int64_t best_groups = 0;
     bool best_fits = false;

@@ -209,6 +209,10 @@ class Linear:
         least = 0 if few_rows else GEMM_MFMA_SKINNY_BEST_M  # (fewer rows: for a consumer that spares a launch by it)
         if x.dtype != torch.bfloat16 or not least < m <= most:
             return None
+        if m > GEMM_MFMA_SKINNY_BEST_M and self.in_features < 2 * 512 and (self.in_features < 7 * 128 or self.out_features < 1024):
+            # slices of one stage of K: added up by a launch of their own they pay from seven slices and 1,024 rows of W on
+            # (N = 1024, K = 896: 17 rows 6.2 us, 64 8.0, the library's 6.6 and 10.4; K = 768: 5.8 and 7.3 against 5.0 and 7.0)
+            return None
         splits = self.wide_splits(m)
         if splits < 2 or not self.wide_takes(m, splits):
             return None

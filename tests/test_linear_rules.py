@@ -14,3 +14,20 @@ def test_copies_of_small_weights_are_for_sixteen_rows(n, k, rows, copy):
     assert lin.copy_for(rows) is None and lin.wide_weight(rows) is lin.weight
     lin.streamed = object()
     assert (lin.copy_for(rows) is lin.streamed) == copy and (lin.wide_weight(rows) is lin.weight) == (not copy)
+
+
+@pytest.mark.parametrize("m, n, k", [(17, 1024, 768), (64, 9728, 640), (40, 512, 896), (128, 14336, 512)])
+def test_partial_sums_of_a_short_k_are_not_taken(m, n, k):
+    lin = Linear(k, n)
+    lin.weight = torch.empty((n, k), dtype=torch.bfloat16, device="meta")
+    assert lin.partial_sums(torch.empty((m, k), dtype=torch.bfloat16, device="meta")) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m, n, k, cut", [(40, 896, 896, True), (64, 4096, 256, True), (32, 4096, 896, True), (64, 9728, 896, False),
+                                          (80, 6144, 896, False), (128, 1024, 896, False), (40, 2048, 1024, True)])
+def test_slices_of_a_short_k(m, n, k, cut):
+    from from_scratch_inference_engine_amd import ops
+
+    ops.load(build_if_missing=False)
+    assert (ops.gemm_mfma_wide_best_splits(m, n, k) > 1) == cut
