@@ -395,7 +395,7 @@ extern "C" int fsie_gemm_mfma_wide_slice(int K, int splits) {
 }
 
 // Into how many slices of K a product of M rows that leaves partial sums is best cut (1: not at
-// all, or this kernel does not take K).  A slice is at least 512 long.
+// all, or this kernel does not take K).  A slice is at least 512 long, but for small matrices (below).
 // Up to 16 rows: as many slices as K gives, up to 8: many short workgroups, several a compute unit
 // (N = K = 3584 on MI355X, 8 rows: 7 slices 7.4 us, 6 7.2, 4 9.3, the few-rows kernel's 4 8.4; the
 // norm that then adds 7 parts instead of 4 takes 0.6 us longer, which leaves 0.03 ms of a decode
@@ -419,13 +419,15 @@ extern "C" int fsie_gemm_mfma_wide_best_splits(int M, int N, int K) {
         int best = 1;
         for (int s = 8; s >= 2 && best == 1; --s)
             if (K / s >= 512 && fsie_gemm_mfma_wide_slice(K, s) > 0) best = s;
-        // where that gives a unit one workgroup of 64 rows of W or less, shorter slices, down to one stage, while the
-        // workgroups stay fewer than two a unit (8 rows: N = K = 896 in seven slices 2.4 us, whole 5.6; N = 896, K = 4864 in
-        // 13 4.2, in eight 5.0; N = K = 2048 in eight 3.7, in four 4.3; N = 2048, K = 8192 in 13 7.6, in eight 8.5, in 16 9.0;
-        // but N = 6144, K = 2048, 384 workgroups in four slices, 6.1 against 6.3 in eight)
+        // Where that gives a unit one workgroup of 64 rows of W or less, shorter slices, down to one stage: up to eight, and up
+        // to 14 where eight would walk 1,024 values or more, while the workgroups stay fewer than two a unit.  With the norm
+        // that adds them up, 8 rows, us: N = K = 896 in seven slices 5.6, whole 7.1; N = K = 2048 (a copy) in eight 7.3, in four
+        // 7.5; N = 896, K = 3072 (a copy) in eight 6.4, in six 6.9; N = 1024, K = 8192 (a copy) in 13 8.9, in eight 9.5; N = 2048,
+        // K = 8192 11.8 / 12.2.  More slices than that cost the norm more than the product gains: N = 1536, K = 2048 in 16
+        // 10.6, in eight 7.8; N = 1536, K = 4096 (a copy) 11.2 / 8.2; N = 1536, K = 8192 (a copy) in 16 13.8, in 13 11.1.
         const int64_t groups = (N + 63) / 64;
         if (units > 0 && groups * best <= units) {
-            for (int s = FSIE_GEMM_MAX_SPLITS; s > best; --s)
+            for (int s = K >= 8 * 1024 ? 14 : 8; s > best; --s)
                 if (K / s >= stage && groups * s < 2 * static_cast<int64_t>(units) && fsie_gemm_mfma_wide_slice(K, s) > 0) return s;
         }
         return best;

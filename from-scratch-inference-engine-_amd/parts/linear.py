@@ -195,7 +195,7 @@ class Linear:
         # K is long enough for six slices or more
         splits = self.wide_splits(m)
         if splits > 1 and (self.kernel_reads(x) if m > GEMM_MFMA_SKINNY_BEST_M
-                           else self.streamed is not None or splits >= 6):
+                           else self.streamed is not None or self.slices_beat_few_rows(splits)):
             return ops.gemm_mfma_wide(x, self.wide_weight(m), splits=splits)
         splits = self.residual_splits(m)
         return ops.gemm_mfma_skinny(x, self.weight, splits=splits) if splits > 1 else None
@@ -238,6 +238,20 @@ class Linear:
         if tiles not in self._wide_splits:
             self._wide_splits[tiles] = ops.gemm_mfma_wide_best_splits(m, self.out_features, self.in_features)
         return self._wide_splits[tiles]
+
+    def slices_beat_few_rows(self, splits: int) -> bool:
+        """Up to 16 rows of a weight without a copy: whether the kernel that shares x through LDS, in ``splits`` slices of K,
+        is faster than the few-rows kernel in two, four or eight.  Six slices or more, of 512 and more values of K; or shorter
+        ones that the other kernel has no even cut for, as long as the workgroups are not too many (with the norm, 8 rows, us,
+        this kernel / the other: N = K = 896 5.6 / 6.4, N = 3072, K = 896 7.6 / 7.8, N = 3584 8.1 / 8.0; N = K = 1536
+        7.5 / 8.1).  At K = 1024 the other's halves are as good from N = 1,536 on (16 rows 7.4 / 7.0, N = 1024 6.0 / 6.4), and
+        at K = 2048 its quarters at any N (N = 512 6.2 / 6.1, N = 1024 6.7 / 6.5)."""
+        if splits < 6:
+            return False
+        groups = -(-self.out_features // 64) * splits
+        if self.in_features < 2048:
+            return groups <= (128 if self.in_features == 1024 else 384)
+        return self.in_features >= 6 * 512
 
     def residual_splits(self, m: int) -> int:
         """Slices of K for ``for_residual`` (1 = do not cut): as many as bring the workgroups to

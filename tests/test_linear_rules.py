@@ -31,3 +31,23 @@ def test_slices_of_a_short_k(m, n, k, cut):
 
     ops.load(build_if_missing=False)
     assert (ops.gemm_mfma_wide_best_splits(m, n, k) > 1) == cut
+
+
+@pytest.mark.parametrize("n, k, splits, wide", [
+    (896, 896, 7, True), (1024, 1024, 8, True), (1536, 1536, 6, True), (4096, 768, 6, True), (896, 3072, 8, True), (512, 4096, 8, True),
+    (3584, 896, 7, False), (1536, 1024, 8, False), (512, 2048, 8, False), (1536, 2048, 8, False), (2048, 640, 5, False)])
+def test_few_rows_without_a_copy(n, k, splits, wide):
+    assert Linear(k, n).slices_beat_few_rows(splits) == wide
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n, k, splits", [
+    (896, 896, 7), (1536, 1536, 6), (896, 2048, 8), (1536, 2048, 8), (896, 3072, 8), (1536, 4096, 8), (896, 4864, 8), (2048, 2048, 8),
+    (1536, 8192, 13), (2048, 8192, 13), (1024, 13824, 14), (4096, 8192, 8), (3584, 3584, 7), (6144, 2048, 4), (3584, 18944, 8)])
+def test_slices_of_sixteen_rows(n, k, splits):
+    """Up to eight slices, 14 of a long K: more cost the norm that adds them up more than the product gains."""
+    from from_scratch_inference_engine_amd import ops
+
+    ops.load(build_if_missing=False)
+    if ops.compute_units() == 256:
+        assert ops.gemm_mfma_wide_best_splits(8, n, k) == splits
