@@ -361,15 +361,16 @@ void launch_shape(int mt, int N, int splits, int& waves, int& blocks, bool gate_
         // slices 39.6 against 38.1); with two blocks a wave, four waves (N = 152064: 236 against 260)
         const int64_t groups4 = static_cast<int64_t>((N + 63) / 64) * splits;
         waves = (groups4 >= 1024 && blocks == 1) ? 8 : 4;
-        // one tile of X and a fragment-ordered W: nothing to share, and two waves a workgroup stream best (N = 152064,
+        // one tile of X and a fragment-ordered W: nothing to share, and two waves a workgroup stream best where the workgroups
+        // are very many, at most one a unit, or walk 512 values of K at most (N = 152064,
         // K = 3584: 8 rows 168 us with two waves, 171 with four, 179 with eight; one row
         // 164 / 168 / 177; N = 152064, K = 5120, 8 rows: 247 / 249 / 259; gate and up of 8 rows: N = 16384, K = 2048 13.1 us with two,
         // 15.1 with four, N = 9728, K = 896 6.7 / 7.4; sums of 8 rows: N = K = 3584 in seven slices 6.4 / 6.8, N = 4608, K = 3584
-        // 7.1 / 7.3, N = 6144, K = 2048 in four 6.1 / 7.0).  Not between the many and the
-        // few workgroups, two or three a unit, where they walk a long slice: N = 3584, K = 18944 in eight slices of 2,432
-        // 22.4 us with four waves, 23.3 with two; N = 4096, K = 14336 in eight of 1,792 20.7 / 21.1.
+        // 7.1 / 7.3, N = 6144, K = 2048 in four 6.1 / 7.0).  Two or three workgroups a unit that walk longer slices keep four:
+        // N = 3584, K = 18944 in eight slices of 2,432 22.4 us with four waves, 23.3 with two; N = 4096, K = 14336 in eight of
+        // 1,792 20.7 / 21.1; with the norm behind it, N = 4096, K = 8192 in eight of 1,024 19.1 / 21.1.
         const bool few = groups4 <= fsie_compute_units();
-        if (frags && mt == 1 && blocks == 1 && (groups4 >= 1024 || k_slice <= 1024 || few)) waves = 2;  // (on rows, N = 152064: 215 / 195 / 194)
+        if (frags && mt == 1 && blocks == 1 && (groups4 >= 1024 || (k_slice > 0 && k_slice <= 512) || few)) waves = 2;  // (on rows, N = 152064: 215 / 195 / 194)
         // two waves a workgroup where that deals the waves more evenly to the compute units (N =
         // 5120 in 8 slices: 640 workgroups of four waves put 12 waves on the fullest of 256 units,
         // 1280 of two put 10; K = 13824, 8 rows: 26.7 against 29.8 us)
