@@ -45,6 +45,7 @@ __global__ __launch_bounds__(WAVES * FSIE_WAVE) void gemm_mfma_fp32_kernel(const
     // blockIdx.y: a slice of K of `slice_steps` steps, whose sums are a plane of y of their own
     const int first_step = blockIdx.y * slice_steps;
     const int n_steps = min((K + 15) / 16, first_step + slice_steps);
+    const int k_end = min(K, n_steps * 16);
     y += static_cast<int64_t>(blockIdx.y) * M * N;
     int pass = 0;
     for (int s0 = first_step + wave; s0 < n_steps; s0 += WAVES * U, ++pass) {
@@ -61,7 +62,7 @@ __global__ __launch_bounds__(WAVES * FSIE_WAVE) void gemm_mfma_fp32_kernel(const
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int k0 = (s0 + u * WAVES) * 16 + kg * 4;
-            ok[u] = k0 < K && s0 + u * WAVES < n_steps;  // K is a multiple of 4: a lane's four values are all in or all out
+            ok[u] = k0 < k_end;  // K is a multiple of 4: a lane's four values are all in or all out
             const int k0c = ok[u] ? k0 : 0;
             a[u] = *reinterpret_cast<const float4*>(wp + k0c);
 #pragma unroll
