@@ -420,10 +420,21 @@ def gemm_mfma_fp32_sums(x: torch.Tensor, weight: torch.Tensor, splits: int) -> t
     return out
 
 
-def gemm_mfma_fp32_splits(k: int) -> int:
-    """Slices of K for ``gemm_mfma_fp32_sums``: eight, each at least 224 long (4 rows, us whole and in the rule's slices:
-    N = 896, K = 4864 17.6 and 7.3, N = K = 896 5.2 and 3.7, N = 3584, K = 18944 74 and 53, N = 2048, K = 8192 27 and 22;
-    workgroups of 16 rows of W that walk all of K wait for one trip to memory after the other)."""
+def gemm_mfma_fp32_splits(k: int, n: Optional[int] = None) -> int:
+    """Slices of K for ``gemm_mfma_fp32_sums`` (``n``: rows of W, where known): eight, each about 224 long or more, the last
+    one may be shorter.  With the norm that adds them up, us whole / in slices at 4 and 64 rows: N = 896, K = 4864 20.4 / 10.4 and
+    56 / 21, N = K = 896 8.2 / 7.1 and 16.8 / 11.4, N = 3584, K = 18944 70 / 55 and 201 / 181, N = 2048, K = 8192 30 / 25 and
+    84 / 51; workgroups of 16 rows of W that walk all of K wait for one trip to memory after the other.
+
+    One where the whole product keeps nine tenths of the units busy in every round of its workgroups and K is not very long
+    (N = 4096, K = 2048 16.3 / 17.3 at 16 rows and 28.8 / 32.2 at 64, N = 8192, K = 2048 32.6 / 38.2 at 32, K = 8192 80 / 92
+    at 8; but N = 4096, K = 14336 68 / 49 at 4, 162 / 163 at 64), and where its only round keeps three quarters of them busy
+    and K is short (N = 3072, K = 1536 10.5 / 11.8 at 3)."""
+    if n is not None:
+        groups, units = -(-n // 16), max(1, compute_units())
+        places = -(-groups // units) * units
+        if (10 * groups >= 9 * places and k < 12288) or (places == units and 4 * groups >= 3 * units and k < 2048):
+            return 1
     splits = max(1, min(8, k // 224))
     steps = -(-k // 16)
     while splits > 1 and -(-steps // splits) * (splits - 1) >= steps:

@@ -170,7 +170,7 @@ class Linear:
             if not self.float32_on_matrix_cores or m <= 2 or self.in_features % 4:
                 return None
             if m <= GEMM_MFMA_SKINNY_MAX_M:
-                splits = ops.gemm_mfma_fp32_splits(self.in_features)
+                splits = ops.gemm_mfma_fp32_splits(self.in_features, self.out_features)
                 return ops.gemm_mfma_fp32_sums(x, self.weight, splits) if splits > 1 else None
             splits = ops.gemm_fp32_tile_splits(m, self.out_features, self.in_features)
             return ops.gemm_fp32_tile(x, self.weight, splits=splits) if splits > 1 and self.kernel_reads(x) else None

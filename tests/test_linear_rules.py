@@ -51,3 +51,12 @@ def test_slices_of_sixteen_rows(n, k, splits):
     ops.load(build_if_missing=False)
     if ops.compute_units() == 256:
         assert ops.gemm_mfma_wide_best_splits(8, n, k) == splits
+
+
+@pytest.mark.parametrize("n, k, whole", [(896, 896, False), (3584, 18944, False), (5120, 5120, False), (6144, 896, False), (4096, 14336, False),
+                                         (4096, 2048, True), (8192, 8192, True), (3072, 1536, True), (3072, 2048, False)])
+def test_float32_slices_of_few_rows(n, k, whole, monkeypatch):
+    from from_scratch_inference_engine_amd.ops import functions
+
+    monkeypatch.setattr(functions, "compute_units", lambda: 256)
+    assert (functions.gemm_mfma_fp32_splits(k, n) == 1) == whole
