@@ -284,18 +284,23 @@ int launch_shape(int tile, const Call& c) {
 // Which tile, and how many slices of K, a product of M rows should take; -1: the library's product (and the pass that
 // follows it) is faster, or the sizes are not the kernel's.  Returns tile + 256 * slices.
 //
-// The rule is the time that a count of rounds gives: workgroups (one a compute unit) in rounds over the units, a step of
+// The rule is the time that a count of rounds gives: workgroups (one a compute unit) in rounds over the units of a die, which
+// gets every eighth column of tiles with all of its tiles of X (20 columns of 12 tiles are 36 workgroups for the 32 units of four
+// of the dies: two rounds, not one), a step of
 // 64 values of K in 0.90, 1.10, 1.38 and 1.78 us for the tiles of 128 x 256, 256 x 192, 256 x 256 and 256 x 320, and 8 us
 // a round for filling the stages and writing the result (each within 8 % of what 11 numbers of rows from 144 to 4,096 took
 // at N x K = 37888 x 3584, 27648 x 5120, 28672 x 4096, 16384 x 2048 and 9728 x 896).
 // Gate and up: against the library's product at 1.2 PFLOP/s (or its weights at 5.5 TB/s) and 8 us, and the pass that
 // multiplies gate and up (3 bytes an output of the product at 4.8 TB/s, and 3 us): the two together took 554 us at 2,048 x
 // 37888 x 3584 where this kernel takes 423, 316 / 213 at 978 rows, 149 / 108 at 512; 121 / 106 at 2,048 x 16384 x 2048; but
-// 48 / 63 at 144 x 28672 x 4096, 25 / 32 at 144 x 16384 x 2048, where the tiles do not fill the chip.
-// Partial sums: from K = 16384 on, as long as the tiles of 256 x 256 are fewer than the units.  The library has to cut such a
-// product along K as well and does it badly (with the norm that follows: 387 us at 2,048 x 3584 x 18944 against 242, 175 / 79
-// at 512 rows, 122 / 49 at 144; 300 / 89 at 512 x 5120 x 27648), while at K = 14336 and below it is the faster one
-// (208 / 226 at 2,048 x 4096 x 14336), and where the tiles alone fill the units too (427 / 456 at 4,096 x 4096 x 18944).
+// 48 / 63 at 144 x 28672 x 4096, 25 / 32 at 144 x 16384 x 2048, where the tiles do not fill the chip.  Over 14 matrices and 18
+// numbers of rows from 129 to 4,096 the choice takes 0.89 of the library's time, and at none more than 1.03.
+// Partial sums: the library has to cut a long K as well and does it badly.  With the norm that follows, library / this kernel, us:
+// 378 / 243 at 2,048 x 3584 x 18944, 281 / 197 at 1,500 rows, 204 / 81 at 512, 106 / 51 at 129; 288 / 140 at 512 x 5120 x
+// 27648.  At K = 14336 and below it is the faster one (208 / 226 at 2,048 x 4096 x 14336), and at K = 16384 from some 32 tiles of
+// 256 x 256 on (2,048 x 2048 136 / 145, 4,096 x 1024 133 / 152; 1,024 x 2048 97 / 86).  From three quarters as many tiles as
+// units on the library fills the chip by itself at 1.2 to 1.45 PFLOP/s (3,000 x 4096 x 18944 383 / 426, 1,500 x 8192 x 18944
+// 377 / 421, 3,000 x 5120 x 27648 607 / 669), so a plan must promise 1.25 in one slice there (4,096 x 3584 x 18944 548 / 464).
 // The sums' own bytes, written here and read by the norm, count at 4.5 TB/s.
 extern "C" int fsie_gemm_mfma_tile_plan(int M, int N, int K, int result, int units) {
     if (M <= 0 || N <= 0 || K <= 0 || units <= 0 || N % 16 || K % kStep || (result != kPair && result != kSums)) return -1;
@@ -303,13 +308,14 @@ extern "C" int fsie_gemm_mfma_tile_plan(int M, int N, int K, int result, int uni
     const int rows[4] = {128, 256, 256, 256}, cols[4] = {256, 192, 256, 320};
     const double us_a_step[4] = {0.90, 1.10, 1.38, 1.78};
     const int64_t steps = K / kStep;
-    if (result == kSums && (K < 16384 || ceil_div64(M, 256) * ceil_div64(N, 256) >= units)) return -1;
+    const int64_t tiles = ceil_div64(M, 256) * ceil_div64(N, 256);
+    if (result == kSums && (K < 16384 || tiles >= units || (K < 17408 && tiles > 32))) return -1;
     double best = 1e30;
     int choice = -1;
     for (int tile = 0; tile < 4; ++tile) {
         for (int slices = 1; slices <= (result == kSums ? 16 : 1); ++slices) {
-            const int64_t groups = ceil_div64(M, rows[tile]) * ceil_div64(N, cols[tile]) * slices;
-            double us = static_cast<double>(ceil_div64(groups, units)) *
+            const int64_t columns = ceil_div64(ceil_div64(N, cols[tile]) * slices, 8);  // of a die
+            double us = static_cast<double>(ceil_div64(columns * ceil_div64(M, rows[tile]), ceil_div64(units, 8))) *
                         (static_cast<double>(ceil_div64(steps, slices)) * us_a_step[tile] + 8.0);
             if (result == kSums) us += 8.0 * slices * M * static_cast<double>(N) / 4.5e6;
             if (us < best) {
@@ -318,8 +324,10 @@ extern "C" int fsie_gemm_mfma_tile_plan(int M, int N, int K, int result, int uni
             }
         }
     }
+    const double flops = 2.0 * M * static_cast<double>(N) * K;
+    if (result == kSums && 4 * tiles >= 3 * static_cast<int64_t>(units) && (choice / 256 > 1 || flops / best < 1.25e9)) return -1;
     if (result == kPair) {
-        const double flops = 2.0 * M * static_cast<double>(N) * K, weights = 2.0 * N * static_cast<double>(K);
+        const double weights = 2.0 * N * static_cast<double>(K);
         const double product = flops / 1.2e9 > weights / 5.5e6 ? flops / 1.2e9 : weights / 5.5e6;
         if (best > product + 8.0 + 3.0 * M * static_cast<double>(N) / 4.8e6 + 3.0) return -1;
     }

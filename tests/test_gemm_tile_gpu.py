@@ -91,3 +91,16 @@ def test_plan_names_a_tile_and_slices_that_the_kernel_takes():
     for n, k in ((37880, 3584), (37888, 3592)):      # rows that the stores or the steps of K do not fit
         assert plan(2048, n, k, 1, 256) == -1
     assert plan(2048, 1 << 20, 4096, 1, 256) == -1   # beyond the 32-bit offsets
+
+
+def test_plan_deals_the_columns_of_tiles_to_eight_dies():
+    """A die has an eighth of the units and gets every eighth column with all of its tiles: no plan whose fullest die takes
+    more rounds than another plan's, at the same work a round."""
+    plan = ops.load(build_if_missing=False).fsie_gemm_mfma_tile_plan
+    assert plan(850, 1536, 18944, 2, 256) == 1 + 256 * 8    # (six slices of 128 x 256: 36 columns, 35 workgroups for 32 units)
+    assert plan(1500, 3584, 18944, 2, 256) == 1 + 256 * 2   # (three of 256 x 256: 42 columns, 36 workgroups)
+    assert plan(700, 3584, 18944, 2, 256) == 1 + 256 * 4
+    assert plan(3000, 768 * 8, 768, 1, 256) == 1 + 256      # (20 columns of 256 x 320, 36 workgroups)
+    for m, n, k in ((3000, 5120, 27648), (1500, 8192, 18944), (3000, 4096, 20480), (4096, 1024, 16384), (2048, 2048, 16384)):
+        assert plan(m, n, k, 2, 256) == -1                  # the library fills the chip by itself
+    assert plan(4096, 3584, 18944, 2, 256) >= 0 and plan(1024, 1024, 16384, 2, 256) >= 0
