@@ -170,7 +170,10 @@ __global__ __launch_bounds__(kThreads) void stream_out_kernel(float* __restrict_
 // gate [tokens][gate_stride] of T (the columns of the head start at h * width).
 // HELD > 0: heads of up to 64 * HELD values, which a lane keeps in registers: the planes, the gate and the weight are all
 // asked for at once, where the loop waits for each plane of each run of 64 and reads o twice.  A launch of few tokens is
-// nothing but those trips to memory (8 tokens of 8 heads of 256, two planes: 4.7 us, 6.9 before; the same sums in the same order).
+// nothing but those trips to memory (8 tokens of 4 heads of 256, two planes: 3.6 us, 4.5 before; the same sums in the same order).
+// A launch of many is the instructions of its waves: a head of 64 takes one value a lane and only the planes there are
+// (2,048 tokens of 16 heads of 64, one plane: 11.8 us with the loop, 14.6 with four values a lane and four planes, 10.9 so; of 128
+// 16.3, 17 and 14.4; of 256 23.9 and 19.1).
 template <typename T, int HELD>
 __global__ __launch_bounds__(kThreads) void gated_headnorm_kernel(const float* __restrict__ o, const T* __restrict__ gate,
                                                                   int64_t gate_stride, const float* __restrict__ weight,
@@ -187,19 +190,26 @@ __global__ __launch_bounds__(kThreads) void gated_headnorm_kernel(const float* _
     T* dst = out + t * out_stride + static_cast<int64_t>(h) * width;  // (rows of out may be columns of wider rows)
     if (HELD > 0) {
         constexpr int AHEAD = 4;  // planes asked for together
-        float x[HELD > 0 ? HELD : 1], w[HELD > 0 ? HELD : 1], gate_value[HELD > 0 ? HELD : 1];
+        constexpr int N = HELD > 0 ? HELD : 1;
+        float x[N], w[N], gate_value[N], part[AHEAD][N];
+#pragma unroll
+        for (int p = 0; p < AHEAD; ++p) {
+            if (p >= n_planes) continue;  // (the same for the whole launch)
+#pragma unroll
+            for (int j = 0; j < HELD; ++j) part[p][j] = src[p * plane + min(lane + FSIE_WAVE * j, width - 1)];
+        }
 #pragma unroll
         for (int j = 0; j < HELD; ++j) {
             const int i = min(lane + FSIE_WAVE * j, width - 1);
             w[j] = weight[i];
             gate_value[j] = to_float(g[i]);
-            float part[AHEAD];
+            x[j] = part[0][j];
+        }
 #pragma unroll
-            for (int p = 0; p < AHEAD; ++p) part[p] = src[min(p, n_planes - 1) * plane + i];
-            x[j] = part[0];
+        for (int p = 1; p < AHEAD; ++p) {
+            if (p >= n_planes) continue;
 #pragma unroll
-            for (int p = 1; p < AHEAD; ++p)
-                if (p < n_planes) x[j] += part[p];
+            for (int j = 0; j < HELD; ++j) x[j] += part[p][j];
         }
         for (int p = AHEAD; p < n_planes; ++p)
 #pragma unroll
@@ -350,14 +360,17 @@ extern "C" int fsie_gated_headnorm(const float* o, int n_planes, const void* gat
     gated_headnorm_kernel<T, HELD><<<grid, kThreads, 0, stream>>>(o, static_cast<const T*>(gate), gate_stride, weight,      \
                                                                 static_cast<T*>(out), runs, heads, width, eps, act,         \
                                                                 n_planes, plane, out_stride, out_scale)
-    const bool held = width <= 4 * FSIE_WAVE;
+#define FSIE_HEADNORM_OF(T)                                  \
+    if (width <= FSIE_WAVE) FSIE_HEADNORM(T, 1);             \
+    else if (width <= 2 * FSIE_WAVE) FSIE_HEADNORM(T, 2);    \
+    else if (width <= 4 * FSIE_WAVE) FSIE_HEADNORM(T, 4);    \
+    else FSIE_HEADNORM(T, 0)
     if (dtype == FSIE_F32) {
-        if (held) FSIE_HEADNORM(float, 4);
-        else FSIE_HEADNORM(float, 0);
+        FSIE_HEADNORM_OF(float);
     } else {
-        if (held) FSIE_HEADNORM(bf16_t, 4);
-        else FSIE_HEADNORM(bf16_t, 0);
+        FSIE_HEADNORM_OF(bf16_t);
     }
+#undef FSIE_HEADNORM_OF
 #undef FSIE_HEADNORM
     FSIE_CHECK_LAUNCH("gated_headnorm");
     return 0;

@@ -107,6 +107,21 @@ def test_softcap_and_gated_headnorm(ops):
         assert rel(got.float().cpu(), ref) <= tol(dtype, bf16=2.0 ** -7)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [1, 16, 63, 64, 65, 127, 128, 129, 255, 256, 257, 300])
+def test_gated_headnorm_of_every_width_and_number_of_planes(ops, dtype, width):
+    """One, two and four values a lane and the loop, at their edges; as many planes as are asked for together and more."""
+    heads, t = 3, 5
+    w = 1 + rnd((width,), 3, 0.3)
+    g = rnd((t, heads * width), 4).to(dtype)
+    for planes in (1, 2, 4, 5, 8):
+        o = rnd((planes, t, heads * width), 2 + planes, 4.0)
+        ref = plain.norm_plain_weight(o.double().sum(0).reshape(t, heads, width), w.double(), 1e-5).reshape(t, -1)
+        ref = ref * g.double() * torch.sigmoid(g.double())
+        got = ops.gated_headnorm(o.cuda(), g.cuda(), w.cuda(), 1e-5, heads)
+        assert got.dtype == dtype and rel(got.float().cpu(), ref) <= tol(dtype, bf16=2.0 ** -7), planes
+
+
 def oracle_gla_states(q, k, v, z, tau, state):
     """The recurrence on given q (already scaled), k, v [T, H, *] and decay logits z: returns o and the state."""
     alpha = torch.pow(torch.sigmoid(z), 1.0 / tau)
