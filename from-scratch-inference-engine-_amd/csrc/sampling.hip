@@ -11,10 +11,10 @@
 // kept set ends.  The bins' weights are integers (two limbs of the float's own bits), so the order in which the threads
 // add them changes nothing.  Rows that do not fit this (a maximum that is not finite, a NaN, a temperature whose inverse
 // is zero or infinite, so that a weight may be a NaN, more than 2,048 tokens in the threshold's bin) are bisected over the order-preserving integer image of the logits, a pass a probe.
-// What bounds it is how often a compute unit reads a row of 600 KB from the caches: 2 passes for greedy and
-// plain temperature, 4 with a threshold, where the bisection alone took 32 a threshold (64 rows of 152,064, a fifth
-// of them each greedy, at a temperature, top k, top p and both: 183 us, 1,504 with the bisection alone).  Long rows
-// are shared by several workgroups where the call has few of them (below): 88 us for the same call.
+// What bounds it is how often a compute unit reads a row of 600 KB from the caches: one pass for greedy, two at a plain
+// temperature, 4 with a threshold and 5 with two whose bins differ, where the bisection alone took 32 a threshold (64 rows of
+// 152,064, a fifth of them each greedy, at a temperature, top k, top p and both: 152 us, 1,504 with the bisection alone).
+// Long rows are shared by several workgroups where the call has few of them (below): 89 us for the same call.
 #include "common.h"
 #include "api.h"
 
@@ -459,6 +459,9 @@ __global__ __launch_bounds__(kThreads) void sample_greedy_kernel(const float* __
     if (threadIdx.x == 0) out[blockIdx.x] = top.index;
 }
 
+// CUTS: some row may have a threshold.  Without, the kernel is rid of the bins (60 KB of LDS, with which a compute unit holds one
+// workgroup): 380 rows of 1,000 tokens at a temperature 19 us with them, 16.5 without; 64 of 32,000 22 and 18.
+template <bool CUTS>
 __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restrict__ logits, int vocab,
                                                           const float* __restrict__ temperature,
                                                           const int32_t* __restrict__ top_k,
@@ -467,16 +470,17 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
                                                           int32_t* __restrict__ out) {
     __shared__ float sval[kWaves];
     __shared__ int sidx[kWaves];
-    __shared__ double sdbl[kWaves];
     __shared__ double run_sum[kRuns];
-    __shared__ Binned binned;
 
     const int r = blockIdx.x;
     const float* row = logits + static_cast<int64_t>(r) * vocab;
+    const float temp = temperature[r];
+    const int k = CUTS && top_k && top_k[r] > 0 && top_k[r] < vocab ? top_k[r] : 0;
+    const float p = CUTS && top_p ? top_p[r] : 1.f;
+    const bool cuts = CUTS && temp > 0.f && (k > 0 || p < 1.f);  // (only these rows need the smallest value and look for a NaN)
     float low;
     bool nan;
-    const Best top = block_argmax<true>(row, vocab, sval, sidx, &low, &nan);
-    const float temp = temperature[r];
+    const Best top = cuts ? block_argmax<true>(row, vocab, sval, sidx, &low, &nan) : block_argmax<false>(row, vocab, sval, sidx, &low, &nan);
     if (!(temp > 0.f)) {
         if (threadIdx.x == 0) out[r] = top.index;
         return;
@@ -484,39 +488,49 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
     const float mx = top.value;
     const float inv_temp = 1.0f / temp;
     uint32_t cut = 0;  // tokens with key >= cut are kept
-    const int k = top_k && top_k[r] > 0 && top_k[r] < vocab ? top_k[r] : 0;
-    const float p = top_p ? top_p[r] : 1.f;
-    if (k > 0 || p < 1.f) {
-        if (vocab > kMaxBinned || !(fabsf(mx) < INFINITY) || !cut_by_bins(binned, row, vocab, mx, low, nan, inv_temp, k, p, &cut)) {
+    if constexpr (CUTS) {
+        __shared__ double sdbl[kWaves];
+        __shared__ Binned binned;
+        if (cuts && (vocab > kMaxBinned || !(fabsf(mx) < INFINITY) || !cut_by_bins(binned, row, vocab, mx, low, nan, inv_temp, k, p, &cut))) {
             __syncthreads();
             cut = cut_by_bisection(row, vocab, mx, inv_temp, k, p, sdbl);
         }
     }
 
     // inverse CDF in vocabulary order.  The vocabulary is cut into kRuns runs of whole 64 tokens; a wave adds up the
-    // kept weights of kRuns / kWaves neighbouring ones, then the wave whose run holds the threshold walks it.
+    // kept weights of kRuns / kWaves neighbouring ones, kAbreast of them at a time (a run alone is a chain of one trip to
+    // memory and six exchanges between lanes, 1 us), then the wave whose run holds the threshold walks it.
     const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
     const int rows = ((vocab + FSIE_WAVE - 1) / FSIE_WAVE + kRuns - 1) / kRuns;  // 64 tokens each
-    constexpr int kRunsOfWave = kRuns / kWaves;
-    const auto kept_weight = [&](float v, int i) { return i < vocab && order_key(v) >= cut ? token_weight(v, mx, inv_temp) : 0.0; };
-    for (int q = 0; q < kRunsOfWave; ++q) {
+    constexpr int kRunsOfWave = kRuns / kWaves, kAbreast = 4;
+    for (int q = 0; q < kRunsOfWave; q += kAbreast) {
         const int run = wave * kRunsOfWave + q;
-        double mine = 0.0;
-        for (int j0 = 0; j0 < rows; j0 += kUnroll) {
-            float v[kUnroll];
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                const int64_t i = (static_cast<int64_t>(run) * rows + min(j0 + u, rows - 1)) * FSIE_WAVE + lane;
-                v[u] = row[i < vocab ? i : vocab - 1];
-            }
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                const int64_t i = (static_cast<int64_t>(run) * rows + j0 + u) * FSIE_WAVE + lane;
-                if (j0 + u < rows && i < vocab) mine += kept_weight(v[u], static_cast<int>(i));
-            }
+        if (static_cast<int64_t>(run) * rows * FSIE_WAVE >= vocab) {  // (a small vocabulary has fewer runs)
+            if (lane < kAbreast) run_sum[run + lane] = 0.0;
+            continue;
         }
-        mine = wave_sum_f64(mine);
-        if (lane == 0) run_sum[run] = mine;
+        double mine[kAbreast] = {};
+        for (int j0 = 0; j0 < rows; j0 += kUnroll / kAbreast) {
+            float v[kAbreast][kUnroll / kAbreast];
+            const auto token = [&](int a, int u) { return (static_cast<int64_t>(run + a) * rows + j0 + u) * FSIE_WAVE + lane; };
+#pragma unroll
+            for (int a = 0; a < kAbreast; ++a)
+#pragma unroll
+                for (int u = 0; u < kUnroll / kAbreast; ++u) v[a][u] = row[min(token(a, u), static_cast<int64_t>(vocab - 1))];
+#pragma unroll
+            for (int a = 0; a < kAbreast; ++a)
+#pragma unroll
+                for (int u = 0; u < kUnroll / kAbreast; ++u)
+                    if (j0 + u < rows && token(a, u) < vocab && order_key(v[a][u]) >= cut) mine[a] += token_weight(v[a][u], mx, inv_temp);
+        }
+#pragma unroll
+        for (int off = FSIE_WAVE / 2; off > 0; off >>= 1)
+#pragma unroll
+            for (int a = 0; a < kAbreast; ++a) mine[a] += __shfl_xor(mine[a], off, FSIE_WAVE);
+        if (lane == 0) {
+#pragma unroll
+            for (int a = 0; a < kAbreast; ++a) run_sum[run + a] = mine[a];
+        }
     }
     __syncthreads();
     draw_from_runs(row, vocab, top, inv_temp, cut, uniform[r], run_sum, kRunsOfWave, out + r);
@@ -529,15 +543,18 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
 // for rows without a threshold, the draw's sums); the threshold bins' tokens; the cut; the draw's sums; the draw.
 // What a launch leaves for the next lies in a workspace of the row.
 // A workgroup a row takes the same time up to 256 rows and grows with the row; shared, six launches' ends cost some 30 us
-// and the rest grows with the tokens of all rows.  Alone / shared, us, at 1, 8, 64 and 256 rows:
-//    16,384 tokens   44 / 32    44 / 35    45 /  50    45 /  81
-//    32,000          56 / 33    57 / 37    58 /  52    59 /  94
-//    65,536          84 / 35    84 / 39    86 /  59    90 / 115
-//   152,064         170 / 39   168 / 49   176 /  88   190 / 193
-// so rows are shared from kSplitFrom tokens on while each of them has kTokensForRow for every row of the call.  (Without
-// temperatures it is one pass over the row, and a workgroup a row is the faster one.)
+// and the rest grows with the tokens of all rows.  Alone / shared, us, a fifth of the rows each greedy, plain, top k, top p and
+// both, at 1, 8, 32, 64, 128 and 256 rows:
+//    16,384 tokens   34 /  31    34 / 33    35 / 43    35 / 50     35 /  63     36 /  82
+//    32,000          45 /  32    46 / 34    46 / 45    46 / 51     46 /  65     48 /  94
+//    65,536          69 /  34    69 / 39    70 / 49    71 / 58     72 /  77     75 / 114
+//   152,064         137 /  38   138 / 47   144 / 66   152 / 89    153 / 127    159 / 193
+// so rows are shared from kSplitFrom tokens on while each of them has kTokensForRow for every row of the call.  Without
+// thresholds it is three launches, and the same line (32,000 tokens 16 / 9, 17 / 11, 17 / 14, 17 / 17, 17 / 24, 19 / 40).
+// (Without temperatures it is one pass over the row, and a workgroup a row is the faster one; with temperatures that all
+// say greedy too, but that only the device knows.)
 constexpr int kSplitFrom = 16384;
-constexpr int kTokensForRow = 400;
+constexpr int kTokensForRow = 800;
 constexpr int kPart = 256;          // threads of a shared row's workgroups
 constexpr int kMaxParts = 64;
 constexpr int kPairs = 512;         // so many listed tokens are compared with each other, more are bisected
@@ -1047,7 +1064,9 @@ extern "C" int fsie_sample(const float* logits, int n_rows, int vocab, const flo
     FSIE_REQUIRE(n_rows >= 0 && vocab > 0, "sample: bad sizes rows=%d vocab=%d", n_rows, vocab);
     FSIE_REQUIRE(!temperature || uniform, "sample: temperatures given without uniform numbers");
     if (n_rows == 0) return 0;
-    if (temperature) sample_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, temperature, top_k, top_p, uniform, out);
+    if (temperature && (top_k || top_p))
+        sample_kernel<true><<<n_rows, kThreads, 0, stream>>>(logits, vocab, temperature, top_k, top_p, uniform, out);
+    else if (temperature) sample_kernel<false><<<n_rows, kThreads, 0, stream>>>(logits, vocab, temperature, nullptr, nullptr, uniform, out);
     else sample_greedy_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, out);
     FSIE_CHECK_LAUNCH("sample");
     return 0;
