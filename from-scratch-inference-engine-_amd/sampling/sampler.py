@@ -106,4 +106,7 @@ class Sampler:
             uniforms_for(self.seed, request_ids, indices),
             [max(float(p.temperature), 0.0) for p in params], [int(p.top_k) for p in params],
             [float(p.top_p) for p in params], logits.device)
-        return ops.sample(logits, temperature, top_k, top_p, uniform)
+        # (a threshold that no row has is not passed: the kernels then spare what finds it)
+        vocab = logits.shape[1]
+        return ops.sample(logits, temperature, top_k if any(0 < p.top_k < vocab for p in params) else None,
+                          top_p if any(p.top_p < 1.0 for p in params) else None, uniform)

@@ -97,7 +97,7 @@ def test_weights_that_are_no_numbers_leave_the_maximum(vocab, temperature):
         assert out.cpu().tolist() == x.argmax(1).tolist()
 
 
-@pytest.mark.parametrize("rows, vocab", [(1, 16500), (3, 16500), (41, 16500), (42, 16500), (64, 40007), (1100, 16500)])
+@pytest.mark.parametrize("rows, vocab", [(1, 16500), (3, 16500), (20, 16500), (21, 16500), (41, 16500), (42, 16500), (50, 40007), (64, 40007), (1100, 16500)])
 def test_a_row_does_not_depend_on_how_many_workgroups_share_it(rows, vocab):
     from from_scratch_inference_engine_amd import ops
 
@@ -112,3 +112,22 @@ def test_a_row_does_not_depend_on_how_many_workgroups_share_it(rows, vocab):
     for i in sorted({0, rows // 2, rows - 1, min(rows - 1, 4)}):
         assert got[i] == ops.sample(x[i:i + 1].contiguous(), *[a[i:i + 1].contiguous() for a in args])[0]
     assert torch.equal(ops.sample(x), x.argmax(1).to(torch.int32))
+
+
+@pytest.mark.parametrize("rows, vocab", [(3, 700), (20, 5000), (3, 16500), (50, 16500)])
+@pytest.mark.parametrize("top_k, top_p", [(0, 1.0), (40, 1.0), (0, 0.8), (40, 0.8), (10 ** 6, 1.0)])
+def test_thresholds_that_no_row_has_are_not_passed(rows, vocab, top_k, top_p, monkeypatch):
+    """The sampler leaves out an array that says nothing, and the tokens are those that the arrays give."""
+    from from_scratch_inference_engine_amd import SamplingParams, ops
+    from from_scratch_inference_engine_amd.sampling.sampler import Sampler, uniforms_for
+
+    ops.load(build_if_missing=False)
+    x = (torch.randn((rows, vocab), generator=torch.Generator().manual_seed(rows)) * 2.5).cuda()
+    params = [SamplingParams(0.0 if i == 1 else 0.9, top_k, top_p) for i in range(rows)]
+    passed, sample = [], ops.sample
+    monkeypatch.setattr(ops, "sample", lambda *a: (passed.append(a), sample(*a))[1])
+    got = Sampler(5).sample(x, params, list(range(rows)), [3] * rows)
+    assert (passed[0][2] is not None) == (0 < top_k < vocab) and (passed[0][3] is not None) == (top_p < 1.0)
+    dev = lambda v, dt: torch.tensor(v, dtype=dt).cuda()
+    assert got == sample(x, dev([p.temperature for p in params], torch.float32), dev([top_k] * rows, torch.int32),
+                         dev([top_p] * rows, torch.float32), dev(list(uniforms_for(5, range(rows), [3] * rows)), torch.float64)).tolist()
