@@ -64,6 +64,8 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
     int pooled_max_pages, int pooled_page_size, int pooled_tokens, const float* __restrict__ slopes,
     const float* __restrict__ row_scale) {
     constexpr bool AHEAD = MAXC <= 4;  // (heads of more than 128 fetch where they store: their registers bound the occupancy)
+    constexpr bool HELD = MAXC <= 8;   // (heads of more than 256 four values at a time: with a tile's in registers, 342 of them, one
+                                       // wave a SIMD was left: 32 requests of 700 keys, 2 heads of 320 on 1, 79 us / 102)
     extern __shared__ __attribute__((aligned(16))) float lds[];
     float* qs = lds;                          // [kRows][hd]
     // rows of keys and values: with 16-byte accesses four floats apart, so that eight lanes' rows meet eight groups of banks
@@ -131,7 +133,7 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
     const int n_chunks = (hd + 31) / 32;
     // VEC: the i-th four values that a thread copies of a tile's keys (four values of a key each; key kKeys: none)
     int k_key[MAXC], k_dim[MAXC];
-    if (VEC) {
+    if (VEC && HELD) {
         const int per_key = hd >> 2, step_keys = 256 / per_key, step_dims = 256 - step_keys * per_key;
         int j = tid / per_key, d = tid - j * per_key;
 #pragma unroll
@@ -188,7 +190,19 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
     if (VEC && AHEAD) fetch_keys(seg_begin);
     for (int kt = seg_begin; kt < seg_end; kt += kKeys) {
         __syncthreads();  // previous tile's values are no longer read (first pass: qs is written)
-        if (VEC) {
+        if (VEC && !HELD) {
+            const int per_key = hd >> 2;
+            for (int e = tid; e < kKeys * per_key; e += blockDim.x) {
+                const int j = e / per_key, d = 4 * (e - j * per_key), kj = kt + j;
+                float f[4] = {0.f, 0.f, 0.f, 0.f};
+                if (kj < seg_end) {
+                    const int pg = page_of(kj), page = table[pg];
+                    if (page >= 0)
+                        load4(k_pool + ((static_cast<int64_t>(page) * n_kv + kvh) * page_size + (kj - pg * page_size)) * hd + d, f);
+                }
+                *reinterpret_cast<float4*>(kv + j * kv_stride + d) = float4{f[0], f[1], f[2], f[3]};
+            }
+        } else if (VEC) {
             if (!AHEAD) fetch_keys(kt);
 #pragma unroll
             for (int i = 0; i < MAXC; ++i)
@@ -250,7 +264,19 @@ __global__ __launch_bounds__(256) void attention_scalar_kernel(
             ps[r * kKeys + lane32] = pe;
         }
         __syncthreads();  // scores done: the tile buffer can take the values
-        if (slots_by_four) {
+        if (slots_by_four && !HELD) {
+            for (int e = tid; e < (kKeys / 4) * hd; e += blockDim.x) {
+                const int g = e & (kKeys / 4 - 1), d = e / (kKeys / 4);
+                const int kj = kt + 4 * g, pg = page_of(kj);  // a multiple of 4: the four slots lie in one page
+                float f[4] = {0.f, 0.f, 0.f, 0.f};
+                if (kj < seg_end) {
+                    const int page = table[pg];
+                    if (page >= 0) load4(v_pool + ((static_cast<int64_t>(page) * n_kv + kvh) * hd + d) * page_size + (kj - pg * page_size), f);
+                }
+#pragma unroll
+                for (int t = 0; t < 4; ++t) kv[(4 * g + t) * kv_stride + d] = kj + t < seg_end ? f[t] : 0.f;
+            }
+        } else if (slots_by_four) {
             // a page of values is [head_dim][page_size]: consecutive threads take the eight groups of
             // four keys of a dimension, then the next dimension
             if (!AHEAD) fetch_values(kt);

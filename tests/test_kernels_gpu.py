@@ -692,6 +692,13 @@ def test_attention_in_float32_arithmetic_copies_any_head_by_fours(ops, dtype, he
     test_attention_over_pages(ops, dtype, True, heads, kv, hd, page, window)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("heads, kv, hd, page, window", [(2, 1, 260, 16, None), (9, 1, 320, 8, 50), (4, 2, 384, 12, None), (2, 1, 512, 16, 70)])
+def test_attention_in_float32_arithmetic_of_heads_beyond_256(ops, dtype, heads, kv, hd, page, window):
+    """Heads whose keys and values a thread copies four values at a time: the same sequences and bounds as the other sizes."""
+    test_attention_over_pages(ops, dtype, True, heads, kv, hd, page, window)
+
+
 @pytest.mark.parametrize("heads, kv, hd, page, window", [(8, 1, 256, 16, None), (5, 1, 256, 16, 100), (16, 1, 192, 16, None),
                                                          (6, 2, 192, 32, 37), (6, 2, 224, 16, None),
                                                          (10, 1, 224, 64, 90), (4, 2, 160, 16, None), (3, 1, 160, 8, 61)])
