@@ -695,8 +695,18 @@ def test_attention_in_float32_arithmetic_copies_any_head_by_fours(ops, dtype, he
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("heads, kv, hd, page, window", [(2, 1, 260, 16, None), (9, 1, 320, 8, 50), (4, 2, 384, 12, None), (2, 1, 512, 16, 70)])
 def test_attention_in_float32_arithmetic_of_heads_beyond_256(ops, dtype, heads, kv, hd, page, window):
-    """Heads whose keys and values a thread copies four values at a time: the same sequences and bounds as the other sizes."""
-    test_attention_over_pages(ops, dtype, True, heads, kv, hd, page, window)
+    """Heads whose keys and values a thread copies four values at a time."""
+    seqs = [(7, 5), (19, 1), (600, 1), (0, 33), (300, 2), (123, 70), (0, 1), (40, 200)]
+    case = paged_case(seqs, heads, kv, hd, page, dtype, seed=hd + heads, window=window, scalar=True)
+    out = run_attention(ops, case, heads, kv, hd, window)
+    row = 0
+    for (p, n), q, k, v in zip(seqs, case["qs"], case["ks"], case["vs"]):
+        ref = plain.attention(q, k, v, heads, kv, hd, query_offset=p, window=window)
+        # a score is a sum of hd products whose running values, scaled, stay below some 6; its hd roundings, independent of
+        # each other, move it by sqrt(hd) * 2^-24 * 6, a probability by as much, the output by twice that of the largest value
+        bound = 12 * math.sqrt(hd) * 2.0 ** -24 * v.abs().max().item() if dtype == torch.float32 else 2.0 ** -7 * ref.abs().max().item()
+        assert (out[row:row + n] - ref).abs().max().item() <= bound, f"seq past {p} new {n}"
+        row += n
 
 
 @pytest.mark.parametrize("heads, kv, hd, page, window", [(8, 1, 256, 16, None), (5, 1, 256, 16, 100), (16, 1, 192, 16, None),
