@@ -458,11 +458,17 @@ def gemm_fp32_tile(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     return out
 
 
+_FP32_TILE_ROWS = 512  # rows of a prompt's step that the slices below are made for
+
+
 @lru_cache(maxsize=4096)
 def gemm_fp32_tile_splits(m: int, n: int, k: int) -> int:
     """Slices of K for ``gemm_fp32_tile``: whole runs of 256 values (the kernel's own), as many as bring its tiles of 64 x 64
-    to four a compute unit."""
-    tiles = -(-m // 64) * -(-n // 64)
+    to four a compute unit at 512 rows.  By N and K alone, whatever ``m``: a row's sums are then the same in a step of any
+    number of rows that takes this kernel.  Slices by the step's own rows gain at few rows of a wide W and lose at others
+    (with the norm, us by 512 rows / by the step's: N = 896, K = 4864 30 / 28 at 65 rows, 80 / 90 at 700; N = K = 2048 24 / 24 and
+    82 / 77, 202 / 183 at 2,048; N = K = 5120 143 / 95 at 65; the vector kernel before took two to seven times as long)."""
+    tiles = -(-_FP32_TILE_ROWS // 64) * -(-n // 64)
     wanted = min(GEMM_MAX_SPLITS, 4 * compute_units() // tiles, k // 256)
     if wanted < 2:
         return 1

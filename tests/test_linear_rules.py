@@ -60,3 +60,23 @@ def test_float32_slices_of_few_rows(n, k, whole, monkeypatch):
 
     monkeypatch.setattr(functions, "compute_units", lambda: 256)
     assert (functions.gemm_mfma_fp32_splits(k, n) == 1) == whole
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n, k", [(896, 4864), (896, 896), (2048, 2048), (5120, 5120), (512, 2048)])
+def test_a_float32_row_of_a_prompt_does_not_depend_on_the_rows_beside_it(n, k):
+    """Whole and as a residual projection in slices: the first rows of 700 are the bits that 70 and 300 of them give."""
+    from from_scratch_inference_engine_amd import ops
+
+    ops.load(build_if_missing=False)
+
+    class Ctx:
+        partial_sums_ok = True
+
+    lin = Linear(k, n)
+    lin.weight = torch.randn((n, k), generator=torch.Generator().manual_seed(n)).cuda()
+    x = torch.randn((700, k), generator=torch.Generator().manual_seed(k)).cuda()
+    whole, sums = lin(x), lin.for_residual(x, Ctx)
+    for m in (70, 300):
+        assert torch.equal(lin(x[:m].contiguous()), whole[:m])
+        assert torch.equal(lin.for_residual(x[:m].contiguous(), Ctx), sums[..., :m, :])
