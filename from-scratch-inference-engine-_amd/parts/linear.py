@@ -41,6 +41,7 @@ class Linear:
     # made: a model that large keeps copies of its first layers only and runs the rest from rows.
     # From 17 rows on the copy is read of weights of 16 MB and more: where the copies of 8 to 16 MB were read too, decode steps of
     # 20 and 32 rows at hidden size 2,048 took 2 % longer and at 2,560 1 %, and 65 to 128 rows left the library's faster products.
+    # (Where ``streamed_copy_from`` is set lower, from twice that size on.)
     streamed_copy_from = 8 << 20
     streamed_many_rows_from = 16 << 20
     streamed_copy_reserve = 0.25
@@ -92,9 +93,10 @@ class Linear:
 
     def copy_for(self, m: int):
         """The fragment-ordered copy, if there is one that products of ``m`` rows read."""
-        if self.streamed is None or (m > GEMM_MFMA_SKINNY_BEST_M and self._weight.numel() * 2 < self.streamed_many_rows_from):
-            return None
-        return self.streamed
+        if self.streamed is None or m <= GEMM_MFMA_SKINNY_BEST_M:
+            return self.streamed
+        least = min(self.streamed_many_rows_from, 2 * (self.streamed_copy_from or 0))
+        return self.streamed if self._weight.numel() * 2 >= least else None
 
     def wide_weight(self, m: int):
         """What the products of ``m`` rows that share x through LDS read: the fragment-ordered copy if there is one for them."""

@@ -16,6 +16,17 @@ def test_copies_of_small_weights_are_for_sixteen_rows(n, k, rows, copy):
     assert (lin.copy_for(rows) is lin.streamed) == copy and (lin.wide_weight(rows) is lin.weight) == (not copy)
 
 
+@pytest.mark.parametrize("copies_from, size, copy", [(0, 64, True), (None, 64, True), (1 << 20, 1 << 20, False), (1 << 20, 2 << 20, True),
+                                                     (48 << 20, 16 << 20, True)])
+def test_copies_where_their_least_size_is_set(copies_from, size, copy, monkeypatch):
+    monkeypatch.setattr(Linear, "streamed_copy_from", copies_from)
+    lin = Linear(size // 2, 1)
+    lin.weight = torch.empty((1, size // 2), dtype=torch.bfloat16, device="meta")
+    lin.streamed = object()
+    assert lin.copy_for(16) is lin.streamed
+    assert (lin.copy_for(17) is lin.streamed) == copy and (lin.copy_for(128) is lin.streamed) == copy
+
+
 @pytest.mark.parametrize("m, n, k", [(17, 1024, 768), (64, 9728, 640), (40, 512, 896), (128, 14336, 512)])
 def test_partial_sums_of_a_short_k_are_not_taken(m, n, k):
     lin = Linear(k, n)
