@@ -298,9 +298,13 @@ int launch_shape(int tile, const Call& c) {
 // Partial sums: the library has to cut a long K as well and does it badly.  With the norm that follows, library / this kernel, us:
 // 378 / 243 at 2,048 x 3584 x 18944, 281 / 197 at 1,500 rows, 204 / 81 at 512, 106 / 51 at 129; 288 / 140 at 512 x 5120 x
 // 27648.  At K = 14336 and below it is the faster one (208 / 226 at 2,048 x 4096 x 14336), and at K = 16384 from some 32 tiles of
-// 256 x 256 on (2,048 x 2048 136 / 145, 4,096 x 1024 133 / 152; 1,024 x 2048 97 / 86).  From three quarters as many tiles as
-// units on the library fills the chip by itself at 1.2 to 1.45 PFLOP/s (3,000 x 4096 x 18944 383 / 426, 1,500 x 8192 x 18944
-// 377 / 421, 3,000 x 5120 x 27648 607 / 669), so a plan must promise 1.25 in one slice there (4,096 x 3584 x 18944 548 / 464).
+// 256 x 256 on (2,048 x 2048 136 / 145, 4,096 x 1024 133 / 152; 1,024 x 2048 97 / 86).  Up to half as many tiles as units
+// this kernel is the faster one (K = 18944 to 28672, N = 1536 to 8192, 576 to 5,000 rows: 0.4 to 0.9 of the library's time, 1.03 once).
+// Beyond, the library fills the chip by itself and runs at 1.2 to 1.45 PFLOP/s at most numbers of rows: only a plan of one round
+// is as fast (2,560 x 3584 x 18944 in two slices 280, 542; 2,048 x 5120 x 27648 412 / 455), not one of two (2,816 x 3584 x 18944
+// 362 / 310, 2,560 x 4096 339 / 309, 2,816 x 4096 419 / 348, 2,304 x 5120 x 27648 547 / 504; where the library's choice is a slow
+// one, two rounds would still gain: 3,072 x 3584 373 / 573), and from three quarters as many tiles as units on only in one slice that
+// promises 1.25 (4,096 x 3584 x 18944 446 / 563; 3,840 x 4096 440 / 410).
 // The sums' own bytes, written here and read by the norm, count at 4.5 TB/s.
 extern "C" int fsie_gemm_mfma_tile_plan(int M, int N, int K, int result, int units) {
     if (M <= 0 || N <= 0 || K <= 0 || units <= 0 || N % 16 || K % kStep || (result != kPair && result != kSums)) return -1;
@@ -310,13 +314,15 @@ extern "C" int fsie_gemm_mfma_tile_plan(int M, int N, int K, int result, int uni
     const int64_t steps = K / kStep;
     const int64_t tiles = ceil_div64(M, 256) * ceil_div64(N, 256);
     if (result == kSums && (K < 16384 || tiles >= units || (K < 17408 && tiles > 32))) return -1;
+    const bool one_round = result == kSums && 2 * tiles > units;
     double best = 1e30;
     int choice = -1;
     for (int tile = 0; tile < 4; ++tile) {
         for (int slices = 1; slices <= (result == kSums ? 16 : 1); ++slices) {
             const int64_t columns = ceil_div64(ceil_div64(N, cols[tile]) * slices, 8);  // of a die
-            double us = static_cast<double>(ceil_div64(columns * ceil_div64(M, rows[tile]), ceil_div64(units, 8))) *
-                        (static_cast<double>(ceil_div64(steps, slices)) * us_a_step[tile] + 8.0);
+            const int64_t rounds = ceil_div64(columns * ceil_div64(M, rows[tile]), ceil_div64(units, 8));
+            if (one_round && rounds > 1) continue;
+            double us = static_cast<double>(rounds) * (static_cast<double>(ceil_div64(steps, slices)) * us_a_step[tile] + 8.0);
             if (result == kSums) us += 8.0 * slices * M * static_cast<double>(N) / 4.5e6;
             if (us < best) {
                 best = us;
@@ -325,7 +331,8 @@ extern "C" int fsie_gemm_mfma_tile_plan(int M, int N, int K, int result, int uni
         }
     }
     const double flops = 2.0 * M * static_cast<double>(N) * K;
-    if (result == kSums && 4 * tiles >= 3 * static_cast<int64_t>(units) && (choice / 256 > 1 || flops / best < 1.25e9)) return -1;
+    if (choice < 0 || (one_round && flops / best < (choice / 256 > 1 ? 1.05e9 : 1.25e9))) return -1;
+    if (result == kSums && 4 * tiles >= 3 * static_cast<int64_t>(units) && choice / 256 > 1) return -1;
     if (result == kPair) {
         const double weights = 2.0 * N * static_cast<double>(K);
         const double product = flops / 1.2e9 > weights / 5.5e6 ? flops / 1.2e9 : weights / 5.5e6;

@@ -104,3 +104,12 @@ def test_plan_deals_the_columns_of_tiles_to_eight_dies():
     for m, n, k in ((3000, 5120, 27648), (1500, 8192, 18944), (3000, 4096, 20480), (4096, 1024, 16384), (2048, 2048, 16384)):
         assert plan(m, n, k, 2, 256) == -1                  # the library fills the chip by itself
     assert plan(4096, 3584, 18944, 2, 256) >= 0 and plan(1024, 1024, 16384, 2, 256) >= 0
+
+
+def test_plan_of_many_tiles_is_one_round():
+    """Sums from half as many tiles as units on: one round of workgroups, or the library's product."""
+    plan = ops.load(build_if_missing=False).fsie_gemm_mfma_tile_plan
+    for m, n, k in ((2816, 3584, 18944), (3328, 3584, 18944), (2304, 4096, 18944), (2816, 4096, 18944), (2304, 5120, 27648), (1128, 8192, 28672)):
+        assert plan(m, n, k, 2, 256) == -1
+    assert plan(2560, 3584, 18944, 2, 256) == 3 + 256 * 2 and plan(2048, 5120, 27648, 2, 256) == 3 + 256 * 2
+    assert plan(2048, 4096, 18944, 2, 256) == 2 + 256 * 2   # 128 tiles

@@ -73,6 +73,22 @@ def test_float32_slices_of_few_rows(n, k, whole, monkeypatch):
     assert (functions.gemm_mfma_fp32_splits(k, n) == 1) == whole
 
 
+@pytest.mark.parametrize("slices, timed, own", [(1, False, True), (1, True, False), (2, False, True), (2, True, True)])
+def test_a_whole_product_of_many_rows_is_left_to_the_librarys_timed_kernels(slices, timed, own, monkeypatch):
+    from from_scratch_inference_engine_amd import ops
+    from from_scratch_inference_engine_amd.parts import linear
+
+    class Ctx:
+        partial_sums_ok = True
+
+    monkeypatch.setattr(ops, "gemm_tile_plan", lambda *a: (2, slices))
+    monkeypatch.setattr(ops, "gemm_mfma_tile", lambda *a, **kw: "sums")
+    monkeypatch.setattr(linear, "library_tuning_enabled", lambda: timed)
+    lin = Linear(18944, 64)
+    lin.weight = torch.empty((64, 18944), dtype=torch.bfloat16, device="meta")
+    assert (lin.residual_sums(torch.empty((256, 18944), dtype=torch.bfloat16, device="meta"), Ctx) == "sums") == own
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n, k", [(896, 4864), (896, 896), (2048, 2048), (5120, 5120), (512, 2048)])
 def test_a_float32_row_of_a_prompt_does_not_depend_on_the_rows_beside_it(n, k):
