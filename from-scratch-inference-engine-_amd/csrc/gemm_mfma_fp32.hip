@@ -5,7 +5,8 @@
 // operands (16 bytes, four values of k, per lane), X comes from cache through a buffer descriptor
 // that ends with its last row, the waves of a workgroup split K and their partial tiles are added
 // through LDS in the fixed order of the waves: a row's sums depend on K and on the launch shape
-// that N and K give, never on the other rows of the batch.
+// that N, K and the number of tiles of 16 rows give (runs of a length for up to 32 rows, of half of it beyond), never on
+// what the other rows hold.
 #include "common.h"
 #include "api.h"
 
@@ -129,8 +130,9 @@ int launch_mt(int waves, const float* x, const float* w, const float* bias, floa
 // A workgroup of four waves makes 64 rows of X by 64 of W, a wave 32 by 32; 32 values of K at a time go through two
 // stages of LDS (the next one's loads are under way while this one is multiplied), a row's eight 16-byte units permuted
 // by the row so that eight rows' reads meet different banks.  A wave's read of 16 bytes a lane feeds four instructions
-// of 32 cycles each, so the matrix cores are the bound, and the small tile is what fills the chip: a unit holds five
-// workgroups, and N = 896 at 682 rows still makes 154 of them (in slices of K as many times that).
+// of 32 cycles each, so the matrix cores are the bound (busy in 0.71 of the units' cycles at 2,048 x 3584 x 18944, 0.66 at
+// 682 x 9728 x 896, where the LDS is in 0.17, without bank conflicts), and the small tile is what fills the chip: a unit holds
+// five workgroups, and N = 896 at 682 rows still makes 154 of them (in slices of K as many times that).
 // Two levels of float32 sums as above, runs of kTileFlush values of K.  108 TFLOP/s at 2,048 x
 // 3584 x 18944 (154 is what the library reaches at 8,192 cubed); against the vector kernel before it 5,090 -> 2,580 us there,
 // 211 -> 136 at 682 x 9728 x 896, and in seven slices 822 -> 77 at 682 x 896 x 4864.

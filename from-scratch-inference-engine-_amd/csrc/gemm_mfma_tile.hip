@@ -14,8 +14,8 @@
 // and while one group is in an M phase the other is in a C phase.  What M1 reads of a stage (W and half of X) is free
 // for the step after next as soon as both groups have read it, the other half of X a phase pair later: each is asked for
 // then, four phases (some 2,000 cycles) before it is waited for.  A wave has the same number of loads under way at
-// every wait (the last steps' are asked for again when there are no more), so "all but the last eight" is what has to
-// have arrived.
+// every wait (the last steps' are asked for again when there are no more), so "all but the last kUnderWay of the shape" is
+// what has to have arrived.
 // What bounds it: a step of 256 x 256 x 64 takes 1.38 us where its matrix instructions alone take 1.04 (v_mfma_f32_16x16x32
 // at 2.07 PFLOP/s over the chip); the LDS is busy for nine tenths of that (24 KB of fragments a wave and step, 64 KB
 // written).  1,320 TFLOP/s at 2,048 x 37888 x 3584 with gate and up multiplied.  The instruction
@@ -228,7 +228,8 @@ __global__ __launch_bounds__(512, 2) void gemm_tile_kernel(const bf16_t* __restr
 #pragma unroll
             for (int j = 0; j < J; ++j) {
                 // gate and up are rounded to 16 bits first, as the library's product leaves them for the pass that
-                // multiplies them: what a token of a prompt gets does not depend on which of the two its portion takes
+                // multiplies them: what a token of a prompt gets does not depend on which of the two its portion takes, up to the
+                // order of the float32 sums (which now and then round to neighbouring 16-bit values)
                 const uint32_t a = pack2_bf16(acc[j][t][0], acc[j][t][1]), b = pack2_bf16(acc[j][t][2], acc[j][t][3]);
                 out[j] = pack2_bf16(gate_pair(__uint_as_float(a << 16), __uint_as_float(a & 0xffff0000u), ACT, act_pos, act_neg),
                                     gate_pair(__uint_as_float(b << 16), __uint_as_float(b & 0xffff0000u), ACT, act_pos, act_neg));
