@@ -752,7 +752,11 @@ class GQAttention(Mixer):
                 and plan.n_small and not plan.n_large and not plan.n_long and x.dtype == torch.bfloat16
                 and ops.attention_mfma_qkv_ok(self.head_dim, cache.page_size)):
             return None
-        sums = self.qkv.partial_sums(x, few_rows=True)
+        # (heads of more than 128 add up their slices more slowly than short ones make the product faster: product and attention of
+        # 1 and 8 requests at hidden size 896 in seven slices, with a product that rotates and writes instead: heads of 160 14.1 and
+        # 15.4 us, 13.0 and 13.7; of 256 20.1 and 20.6, 16.6 and 18.2; at 1,536 in six slices and in three: 160 14.6 and 15.1,
+        # 13.6 and 14.7; 256 18.8 and 20.1, 16.5 and 17.8)
+        sums = self.qkv.partial_sums(x, few_rows=True, long_slices=self.head_dim > 128)
         if sums is None:
             return None
         out = torch.empty((x.shape[0], self.q_dim), dtype=x.dtype, device=x.device)

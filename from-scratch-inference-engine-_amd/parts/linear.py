@@ -205,10 +205,11 @@ class Linear:
         splits = self.residual_splits(m)
         return ops.gemm_mfma_skinny(x, self.weight, splits=splits) if splits > 1 else None
 
-    def partial_sums(self, x: torch.Tensor, few_rows: bool = False) -> Optional[torch.Tensor]:
+    def partial_sums(self, x: torch.Tensor, few_rows: bool = False, long_slices: bool = False) -> Optional[torch.Tensor]:
         """x . W^T (no bias) of 17 to 64 rows (to 128 from a fragment-ordered copy) as float32 partial
         sums [S, T, N] of slices of K, for a consumer that adds them up itself; None where the engine's
-        kernel for that does not take the sizes.  ``few_rows``: also for up to 16 rows."""
+        kernel for that does not take the sizes.  ``few_rows``: also for up to 16 rows.  ``long_slices``: only in
+        slices of 512 values of K and more, for a consumer to whom a slice more costs what shorter ones bring."""
         m = x.shape[0]
         most = GEMM_MFMA_SKINNY_MAX_M if self.copy_for(m) is None else GEMM_MFMA_WIDE_MAX_M
         least = 0 if few_rows else GEMM_MFMA_SKINNY_BEST_M  # (fewer rows: for a consumer that spares a launch by it)
@@ -218,8 +219,8 @@ class Linear:
             # slices of one stage of K: added up by a launch of their own they pay from seven slices and 1,024 rows of W on
             # (N = 1024, K = 896: 17 rows 6.2 us, 64 8.0, the library's 6.6 and 10.4; K = 768: 5.8 and 7.3 against 5.0 and 7.0)
             return None
-        splits = self.wide_splits(m)
-        if splits < 2 or not self.wide_takes(m, splits):
+        splits = self.long_splits() if long_slices and m <= GEMM_MFMA_SKINNY_BEST_M else self.wide_splits(m)
+        if splits < 2 or (long_slices and self.in_features < 2 * 512) or not self.wide_takes(m, splits):
             return None
         if m > GEMM_MFMA_SKINNY_BEST_M and not self.kernel_reads(x):
             return None  # (the library's)
@@ -243,6 +244,10 @@ class Linear:
         if tiles not in self._wide_splits:
             self._wide_splits[tiles] = ops.gemm_mfma_wide_best_splits(m, self.out_features, self.in_features)
         return self._wide_splits[tiles]
+
+    def long_splits(self) -> int:
+        """Up to eight slices of 512 values of K and more (1: K gives none)."""
+        return next((s for s in range(8, 1, -1) if self.in_features >= 512 * s and ops.gemm_mfma_wide_splits_ok(self.in_features, s)), 1)
 
     def slices_beat_few_rows(self, splits: int) -> bool:
         """Up to 16 rows of a weight without a copy: whether the kernel that shares x through LDS, in ``splits`` slices of K,

@@ -64,6 +64,27 @@ def test_slices_of_sixteen_rows(n, k, splits):
         assert ops.gemm_mfma_wide_best_splits(8, n, k) == splits
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("k, short, long", [(512, 4, 0), (896, 7, 0), (1024, 8, 2), (1536, 6, 3), (2048, 8, 4), (3072, 8, 6)])
+@pytest.mark.parametrize("rows", [1, 16])
+def test_long_slices_for_those_who_pay_for_each(k, short, long, rows):
+    """The sums of both cuts are the product's: within a float32 rounding of 2^-24 for each of K additions of each term."""
+    from from_scratch_inference_engine_amd import ops
+
+    ops.load(build_if_missing=False)
+    lin = Linear(k, 512)
+    lin.weight = torch.randn((512, k), generator=torch.Generator().manual_seed(k)).to(torch.bfloat16).cuda()
+    x = torch.randn((rows, k), generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).cuda()
+    exact, size = x.double() @ lin.weight.double().t(), x.double().abs() @ lin.weight.double().abs().t()
+    for sums, slices in ((lin.partial_sums(x, few_rows=True), short), (lin.partial_sums(x, few_rows=True, long_slices=True), long)):
+        if slices == 0:
+            assert sums is None
+            continue
+        if ops.compute_units() == 256:
+            assert sums.shape[0] == slices
+        assert ((sums.double().sum(0) - exact).abs() <= k * 2.0 ** -24 * size).all()
+
+
 @pytest.mark.parametrize("n, k, whole", [(896, 896, False), (3584, 18944, False), (5120, 5120, False), (6144, 896, False), (4096, 14336, False),
                                          (4096, 2048, True), (8192, 8192, True), (3072, 1536, True), (3072, 2048, False)])
 def test_float32_slices_of_few_rows(n, k, whole, monkeypatch):
