@@ -745,6 +745,16 @@ class GQAttention(Mixer):
         table = self.position.rotation_table(self.head_dim, ctx)
         return table is not None, table
 
+    @property
+    def wants_long_slices(self) -> bool:
+        """Whether the attention that adds up q/k/v itself takes no slices of less than 512 values of K."""
+        # Heads of more than 128 add up their slices more slowly than short ones make the product faster: product and attention of
+        # 1 and 8 requests at hidden size 896 in seven slices, with a product that rotates and writes instead: heads of 160 14.1 and
+        # 15.4 us, 13.0 and 13.7; of 256 20.1 and 20.6, 16.6 and 18.2; at 1,536 in six slices and in three: 160 14.6 and 15.1,
+        # 13.6 and 14.7; 256 18.8 and 20.1, 16.5 and 17.8.  Narrower heads gain from 640 values of K on (28 heads of 128: at 768 12.9
+        # and 14.0, 13.7 and 16.8; 14 of 64 at 640 10.4 and 11.3, 10.3 and 11.1, at 512 10.5 and 11.3, 9.8 and 10.3).
+        return self.head_dim > 128 or self.qkv.in_features < 640
+
     def _from_sums(self, x: torch.Tensor, ctx, cache, plan, fuse: bool, table) -> Optional[torch.Tensor]:
         """Attention of a step of one token a request straight from the q/k/v product's partial sums
         (None: not such a step, or the kernels do not take the sizes)."""
@@ -752,11 +762,7 @@ class GQAttention(Mixer):
                 and plan.n_small and not plan.n_large and not plan.n_long and x.dtype == torch.bfloat16
                 and ops.attention_mfma_qkv_ok(self.head_dim, cache.page_size)):
             return None
-        # (heads of more than 128 add up their slices more slowly than short ones make the product faster: product and attention of
-        # 1 and 8 requests at hidden size 896 in seven slices, with a product that rotates and writes instead: heads of 160 14.1 and
-        # 15.4 us, 13.0 and 13.7; of 256 20.1 and 20.6, 16.6 and 18.2; at 1,536 in six slices and in three: 160 14.6 and 15.1,
-        # 13.6 and 14.7; 256 18.8 and 20.1, 16.5 and 17.8)
-        sums = self.qkv.partial_sums(x, few_rows=True, long_slices=self.head_dim > 128)
+        sums = self.qkv.partial_sums(x, few_rows=True, long_slices=self.wants_long_slices)
         if sums is None:
             return None
         out = torch.empty((x.shape[0], self.q_dim), dtype=x.dtype, device=x.device)

@@ -128,3 +128,12 @@ def test_a_float32_row_of_a_prompt_does_not_depend_on_the_rows_beside_it(n, k):
     for m in (70, 300):
         assert torch.equal(lin(x[:m].contiguous()), whole[:m])
         assert torch.equal(lin.for_residual(x[:m].contiguous(), Ctx), sums[..., :m, :])
+
+
+@pytest.mark.parametrize("head, hidden, long", [(64, 896, False), (128, 640, False), (128, 512, True), (64, 256, True), (160, 896, True), (256, 2048, True)])
+def test_slices_that_attention_adds_up(head, hidden, long):
+    from types import SimpleNamespace
+
+    from from_scratch_inference_engine_amd.parts.attention import GQAttention
+
+    assert GQAttention.wants_long_slices.fget(SimpleNamespace(head_dim=head, qkv=Linear(hidden, 4 * head))) == long
