@@ -39,9 +39,11 @@ class Linear:
     # the time).  The rows stay for the library's products of many rows.  None: no copies.
     # A copy that would leave less than ``streamed_copy_reserve`` of the device's memory free is not
     # made: a model that large keeps copies of its first layers only and runs the rest from rows.
-    # From 17 rows on the copy is read of weights of 16 MB and more: where the copies of 8 to 16 MB were read too, decode steps of
-    # 20 and 32 rows at hidden size 2,048 took 2 % longer and at 2,560 1 %, and 65 to 128 rows left the library's faster products.
-    # (Where ``streamed_copy_from`` is set lower, from twice that size on.)
+    # Up to 64 rows read any copy: 0.86 to 1.0 of the time from rows at 15 sizes of 8 to 15 MB, with the norm.  (A model of few layers
+    # has such matrices in the Infinity Cache as rows, which the copies' streaming loads pass by: steps of 20 rows of
+    # 8 layers at hidden size 2,048 13.2 ms of 24 from copies, 13.1 from rows, but of 28 layers 41.8 and 43.3, 32 layers at 2,560 50.4 and
+    # 51.6; the 0.5B shape, 64 rows, 29.3 and 30.7.)  Beyond 64 rows copies of 16 MB and more are read: those of 8 to 16 MB are no
+    # faster than the library's product there.  (Where ``streamed_copy_from`` is set lower, from twice that size on.)
     streamed_copy_from = 8 << 20
     streamed_many_rows_from = 16 << 20
     streamed_copy_reserve = 0.25
@@ -93,7 +95,7 @@ class Linear:
 
     def copy_for(self, m: int):
         """The fragment-ordered copy, if there is one that products of ``m`` rows read."""
-        if self.streamed is None or m <= GEMM_MFMA_SKINNY_BEST_M:
+        if self.streamed is None or m <= GEMM_MFMA_SKINNY_MAX_M:
             return self.streamed
         least = min(self.streamed_many_rows_from, 2 * (self.streamed_copy_from or 0))
         return self.streamed if self._weight.numel() * 2 >= least else None

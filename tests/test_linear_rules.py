@@ -6,9 +6,9 @@ import torch
 from from_scratch_inference_engine_amd.parts.linear import Linear
 
 
-@pytest.mark.parametrize("n, k, rows, copy", [(2048, 2048, 16, True), (2048, 2048, 17, False), (2048, 2048, 128, False),
+@pytest.mark.parametrize("n, k, rows, copy", [(2048, 2048, 16, True), (2048, 2048, 64, True), (2048, 2048, 65, False), (2048, 2048, 128, False),
                                               (4096, 2048, 17, True), (4096, 2048, 128, True)])
-def test_copies_of_small_weights_are_for_sixteen_rows(n, k, rows, copy):
+def test_copies_of_small_weights_are_for_sixty_four_rows(n, k, rows, copy):
     lin = Linear(k, n)
     lin.weight = torch.empty((n, k), dtype=torch.bfloat16, device="meta")
     assert lin.copy_for(rows) is None and lin.wide_weight(rows) is lin.weight
@@ -23,8 +23,8 @@ def test_copies_where_their_least_size_is_set(copies_from, size, copy, monkeypat
     lin = Linear(size // 2, 1)
     lin.weight = torch.empty((1, size // 2), dtype=torch.bfloat16, device="meta")
     lin.streamed = object()
-    assert lin.copy_for(16) is lin.streamed
-    assert (lin.copy_for(17) is lin.streamed) == copy and (lin.copy_for(128) is lin.streamed) == copy
+    assert lin.copy_for(64) is lin.streamed
+    assert (lin.copy_for(65) is lin.streamed) == copy and (lin.copy_for(128) is lin.streamed) == copy
 
 
 @pytest.mark.parametrize("m, n, k", [(17, 1024, 768), (64, 9728, 640), (40, 512, 896), (128, 14336, 512)])
