@@ -30,7 +30,7 @@ class Linear:
     sibling takes every product of up to 64 rows."""
 
     narrow_to = 64  # float32 results of at most this many outputs from bfloat16 operands: the narrow kernel
-    float32_on_matrix_cores = True  # up to 64 rows of float32: v_mfma_f32_16x16x4_f32 instead of vector FMAs
+    float32_on_matrix_cores = True  # 3 rows of float32 and more: v_mfma_f32_16x16x4_f32 instead of vector FMAs
     # A bfloat16 weight of at least this many bytes is kept a second time, in the order of the matrix
     # instruction's fragments, for the engine's own products (decoding): a wave then loads 1 KB in one
     # piece with streaming loads, where rows give it 16 pieces of 64 bytes (a compute unit draws about
