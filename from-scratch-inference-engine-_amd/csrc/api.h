@@ -227,6 +227,16 @@ int fsie_gemm_mfma_wide_act(const void* x, const void* w, const float* bias, voi
                             int blocks, int frags, int act, float act_pos, float act_neg, hipStream_t stream);
 int fsie_gemm_mfma_wide_act_takes(int M, int N, int K);
 
+// Up to 16 rows and a K so short that all of it is under way at once; K a multiple of 32, operands 16-byte aligned, the result 8-byte:
+//   result 0: y float32 partial sums [slices][M][N] (w in fragment order)
+//   result 1: gate and up rows of w in turn, y bfloat16 [M, N/2] (w in fragment order; act as for fsie_gemm_mfma_wide_gated)
+//   result 2: y bfloat16 [M, N] = act(sum + bias), act a FsiePointAct
+// fsie_gemm_mfma_stream_plan: waves + 256 * blocks of 16 rows of w a workgroup + 65536 * slices of K, or -1 where another product
+// is the better one (result 3: as 2, where fsie_gemm_mfma_wide_act is the other product).
+int fsie_gemm_mfma_stream_plan(int M, int N, int K, int result, int frags);
+int fsie_gemm_mfma_stream(const void* x, const void* w, const float* bias, void* y, int M, int N, int K, int result,
+                          int plan, int frags, int act, float pos, float neg, hipStream_t stream);
+
 // Products of many rows (prompts), bfloat16 x [M, K] and w [N, K], N a multiple of 16, K of 64, 16-byte aligned:
 //   result 1: gate and up rows of w in turn, y bfloat16 [M, N/2] (act as for fsie_gemm_mfma_wide_gated)
 //   result 2: y float32 partial sums [splits][M][N] of slices of K

@@ -608,15 +608,19 @@ def gemm_mfma_wide_splits_ok(k: int, splits: int) -> bool:
 
 
 def gemm_mfma_wide_swiglu(x: torch.Tensor, weight: torch.Tensor, waves: int = 0, blocks: int = 0,
-                          out: Optional[torch.Tensor] = None, act="silu") -> torch.Tensor:
+                          out: Optional[torch.Tensor] = None, act="silu", few_rows: bool = False) -> torch.Tensor:
     """silu(gate) * up, or what ``act`` (a ``GateAct`` or its name) makes of them, [M, N/2] (bfloat16) of x [M, K] and a weight [N, K] whose rows are gate and up
     in turn (or its ``FragmentOrdered`` copy), by the kernel that shares x through LDS; up to 64
-    rows, N a multiple of 4, K of 128."""
+    rows, N a multiple of 4, K of 128.  ``few_rows``: up to 16 rows go to ``gemm_mfma_stream`` where that is faster (the same
+    sums in another order)."""
     _need(x, "gemm x", dtype=torch.bfloat16, ndim=2)
     m, k = x.shape
     wptr, n, frags = _wide_weight(weight, k)
     if n % 4:
         raise KernelError(f"gemm_mfma_wide_swiglu: the number of weight rows {n} must be a multiple of 4")
+    plan = gemm_stream_plan(m, n, k, GEMM_STREAM_GATED, bool(frags)) if few_rows and out is None and not waves and not blocks else None
+    if plan is not None:
+        return gemm_mfma_stream(x, weight, GEMM_STREAM_GATED, plan, act=act)
     if out is None:
         out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
     _need(out, "gemm out", dtype=torch.bfloat16, shape=(m, n // 2))
@@ -661,6 +665,40 @@ def _gemm_tile(x, weight, result: int, splits: int, tile: int, act) -> torch.Ten
         out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
     check(load().fsie_gemm_mfma_tile(x.data_ptr(), weight.data_ptr(), out.data_ptr(), m, n, k, result, splits, tile,
                                      *(act.args if act is not None else (0, 0.0, 0.0)), _stream()))
+    return out
+
+
+GEMM_STREAM_SUMS, GEMM_STREAM_GATED, GEMM_STREAM_POINT, GEMM_STREAM_PLAN_ACT = 0, 1, 2, 3
+
+
+@lru_cache(maxsize=4096)
+def gemm_stream_plan(m: int, n: int, k: int, result: int, frags: bool) -> Optional[int]:
+    """How ``gemm_mfma_stream`` takes ``m`` rows of a weight of these sizes (``frags``: its ``FragmentOrdered`` copy); None where
+    another product is faster or it does not take them.  GEMM_STREAM_PLAN_ACT: GEMM_STREAM_POINT for a product with an activation."""
+    plan = int(load().fsie_gemm_mfma_stream_plan(m, n, k, result, int(frags)))
+    return None if plan < 0 else plan
+
+
+def gemm_mfma_stream(x: torch.Tensor, weight, result: int, plan: int, bias: Optional[torch.Tensor] = None, act=None) -> torch.Tensor:
+    """x [M, K] . weight [N, K]^T for bfloat16 operands and up to 16 rows, by the kernel that has all of a short K under way at once.
+    ``result``: GEMM_STREAM_SUMS, float32 partial sums [slices, M, N] (a ``FragmentOrdered`` weight); GEMM_STREAM_GATED, the products of gate
+    and up value (``act``: a ``GateAct`` or its name) [M, N/2] in bfloat16 (a ``FragmentOrdered`` weight); GEMM_STREAM_POINT, act(sum +
+    bias) [M, N] in bfloat16 (``act``: a ``PointAct`` or None).  ``plan`` is ``gemm_stream_plan``'s."""
+    _need(x, "gemm x", dtype=torch.bfloat16, ndim=2)
+    m, k = x.shape
+    wptr, n, frags = _wide_weight(weight, k)
+    if bias is not None:
+        _need(bias, "gemm bias", dtype=torch.float32, shape=(n,))
+    if result == GEMM_STREAM_SUMS:
+        out = torch.empty((plan >> 16, m, n), dtype=torch.float32, device=x.device)
+        args = (0, 0.0, 0.0)
+    elif result == GEMM_STREAM_GATED:
+        out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
+        args = gate_act(act).args
+    else:
+        out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+        args = (0, 0.0, 0.0) if act is None else (act.code, act.pos, act.neg)
+    check(load().fsie_gemm_mfma_stream(x.data_ptr(), wptr, _ptr(bias), out.data_ptr(), m, n, k, result, plan, frags, *args, _stream()))
     return out
 
 

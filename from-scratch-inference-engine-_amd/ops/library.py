@@ -56,6 +56,8 @@ _SIGNATURES = {
     "fsie_gemm_mfma_wide_best_splits": ([c_int, c_int, c_int], c_int),
     "fsie_gemm_mfma_wide": ([_P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P], c_int),
     "fsie_gemm_mfma_wide_swiglu": ([_P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P], c_int),
+    "fsie_gemm_mfma_stream_plan": ([c_int, c_int, c_int, c_int, c_int], c_int),
+    "fsie_gemm_mfma_stream": ([_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, _P], c_int),
     "fsie_gemm_mfma_skinny_act": ([_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, _P], c_int),
     "fsie_gemm_mfma_wide_act": ([_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, _P], c_int),
     "fsie_gemm_mfma_wide_act_takes": ([c_int, c_int, c_int], c_int),

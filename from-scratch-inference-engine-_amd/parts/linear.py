@@ -22,7 +22,8 @@ class Linear:
     once; its sibling that shares x through LDS for float32 results of 8 to 64 rows (the logits;
     beyond 64 rows the library with a float32 result), for the residual projections
     (``for_residual``: 17 to 64 rows, and any number where K is long) and for the partial sums of
-    other projections of 17 to 64 rows (``partial_sums``); residual projections of more than 128 rows whose K is 16,384
+    other projections of 17 to 64 rows (``partial_sums``); a third for up to 16 rows and a K so short that all of it is under
+    way at once (``ops.gemm_stream_plan``); residual projections of more than 128 rows whose K is 16,384
     and more the engine's kernel for many rows, in slices of K (``ops.gemm_tile_plan``); everything else
     the library product (hipBLASLt through torch, where the reference's engine calls cuBLAS) with
     float32 accumulation, the bias added by a kernel of the engine.  A large weight has a second copy in
@@ -133,6 +134,10 @@ class Linear:
             # logits of more rows than the engine's kernels take (a decode batch beyond 64, a replay
             # that wants every position): the library with a float32 result
             return library_mm(x, w, float32_result=True)
+        if not wants_f32 and 0 < m <= GEMM_MFMA_SKINNY_BEST_M:
+            plan = self.stream_plan(m, ops.GEMM_STREAM_POINT)
+            if plan is not None and self.kernel_reads(x):
+                return ops.gemm_mfma_stream(x, self.wide_weight(m), ops.GEMM_STREAM_POINT, plan, bias)
         if self.in_features % 8 == 0 and m <= (GEMM_MFMA_SKINNY_MAX_M if wants_f32 else GEMM_MFMA_SKINNY_BEST_M):
             return ops.gemm_mfma_skinny(x, w, bias, out_dtype=out_dtype)
         if not wants_f32 and self.out_features % 4 == 0:
@@ -198,6 +203,9 @@ class Linear:
                     if splits > 1 and self.wide_takes(m, splits) and self.kernel_reads(x) else None)
         if self.in_features % 8:
             return None
+        plan = self.stream_plan(m, ops.GEMM_STREAM_SUMS) if m <= GEMM_MFMA_SKINNY_BEST_M else None
+        if plan is not None and self.kernel_reads(x):
+            return ops.gemm_mfma_stream(x, self.streamed, ops.GEMM_STREAM_SUMS, plan)
         # the kernel that shares x through LDS: above 16 rows, and at any number of rows where
         # K is long enough for six slices or more
         splits = self.wide_splits(m)
@@ -227,6 +235,10 @@ class Linear:
         if m > GEMM_MFMA_SKINNY_BEST_M and not self.kernel_reads(x):
             return None  # (the library's)
         return ops.gemm_mfma_wide(x, self.wide_weight(m), splits=splits)
+
+    def stream_plan(self, m: int, result: int):
+        """How the kernel for few rows and a short K takes ``m`` rows of this weight, or None."""
+        return ops.gemm_stream_plan(m, self.out_features, self.in_features, result, self.streamed is not None)
 
     def wide_takes(self, m: int, splits: int, gate_up: bool = False) -> bool:
         """Whether the kernel that shares x through LDS takes ``m`` rows of this weight (beyond 64 rows

@@ -71,7 +71,7 @@ class SwiGLU(FeedForward):
                 and self.gate_up.wide_takes(m, 1, gate_up=True)):
             # from the fragment-ordered copy at any number of rows up to 64, and up to 128 where the
             # kernel has the launch shape for it: SiLU*up in the product's epilogue
-            act = ops.gemm_mfma_wide_swiglu(x, self.gate_up.streamed, act=self._gate_act)
+            act = ops.gemm_mfma_wide_swiglu(x, self.gate_up.streamed, act=self._gate_act, few_rows=self.gate_up.kernel_reads(x))
         elif (x.dtype == torch.bfloat16 and 3 <= m <= GEMM_MFMA_SKINNY_BEST_M and self.hidden_size % 128 == 0
                 and self.gate_up.out_features % 4 == 0 and self.gate_up.out_features // 64 >= ops.compute_units()):
             # three rows and more of a matrix that gives every compute unit a workgroup: the kernel that
@@ -153,6 +153,9 @@ class PlainFeedForward(FeedForward):
     def _activated(self, x: torch.Tensor) -> torch.Tensor:
         m, up = x.shape[0], self.up
         if x.dtype == torch.bfloat16 and m > 0:
+            plan = up.stream_plan(m, ops.GEMM_STREAM_PLAN_ACT) if m <= GEMM_MFMA_SKINNY_BEST_M else None
+            if plan is not None and up.kernel_reads(x):
+                return ops.gemm_mfma_stream(x, up.wide_weight(m), ops.GEMM_STREAM_POINT, plan, up.bias, self._act)
             if (up.copy_for(m) is not None and ops.gemm_mfma_wide_act_takes(m, up.streamed)
                     and (m <= 48 or self.intermediate_size <= 32 * ops.compute_units())):
                 # (a full fourth tile of x keeps a unit busy by itself: with more than a workgroup a unit the product in

@@ -1,0 +1,78 @@
+"""The product of up to 16 rows whose K is under way at once: against float64, at the edges of its blocks, steps and slices."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from from_scratch_inference_engine_amd import ops as module
+
+    module.load(build_if_missing=False)
+    return module
+
+
+def operands(m, n, k):
+    gen = torch.Generator().manual_seed(1000 * m + n + k)
+    x, w = (torch.randn(s, generator=gen).to(torch.bfloat16).cuda() for s in ((m, k), (n, k)))
+    exact, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    return x, w, exact, k * 2.0 ** -24 * size  # a float32 rounding for each of K additions of each term
+
+
+# one step of K; a step fewer and more than the waves hold evenly; the most a workgroup of 4, 8 and 16 waves holds; N that ends inside
+# a block of 16 rows and inside a pair of blocks
+@pytest.mark.parametrize("m, n, k", [(1, 4, 32), (16, 36, 96), (3, 52, 1024), (7, 1168, 1056), (16, 80, 2048), (2, 20, 2080), (9, 100, 4064), (16, 48, 4096)])
+@pytest.mark.parametrize("frags", [True, False])
+def test_whole_products(ops, m, n, k, frags):
+    x, w, exact, bound = operands(m, n, k)
+    weight, bias = ops.fragment_order(w) if frags else w, torch.randn(n, generator=torch.Generator().manual_seed(n)).cuda()
+    steps = k // 32
+    for waves in (4, 8, 16):
+        for blocks in (1, 2):
+            if -(-steps // waves) > 8 or (waves == 4 and blocks == 2):
+                continue
+            got = ops.gemm_mfma_stream(x, weight, ops.GEMM_STREAM_POINT, waves + 256 * blocks + 65536, bias).double()
+            want = exact + bias.double()
+            assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2 * bound).all(), (waves, blocks)  # one rounding to bfloat16
+            if frags:
+                got = ops.gemm_mfma_stream(x, weight, ops.GEMM_STREAM_GATED, waves + 256 * blocks + 65536, act="relu").double()
+                gate, up = exact[:, 0::2], exact[:, 1::2]
+                want, off = gate.clamp(min=0) * up, bound[:, 0::2] * up.abs() + bound[:, 1::2] * gate.abs()
+                assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2 * off).all(), (waves, blocks)
+
+
+@pytest.mark.parametrize("m, n, k, splits", [(1, 17, 1024, 1), (16, 33, 2048, 2), (5, 896, 4864, 4), (8, 31, 4864, 3), (16, 1536, 8960, 5), (2, 100, 1056, 2)])
+def test_partial_sums(ops, m, n, k, splits):
+    x, w, exact, bound = operands(m, n, k)
+    f = ops.fragment_order(w)
+    for blocks in (1, 2):
+        got = ops.gemm_mfma_stream(x, f, ops.GEMM_STREAM_SUMS, 8 + 256 * blocks + 65536 * splits)
+        assert got.shape == (splits, m, n) and got.dtype == torch.float32
+        assert ((got.double().sum(0) - exact).abs() <= bound).all(), blocks
+    k_slice = -(-(k // 32) // splits) * 32  # a slice holds its own part of K only
+    first = x[:, :k_slice].double() @ w[:, :k_slice].double().t()
+    assert ((got[0].double() - first).abs() <= bound).all()
+
+
+def test_what_the_plan_takes(ops):
+    """A plan is one the kernel takes; where it stops: rows, K, steps of K, and for one or two rows the widest gate and up matrices."""
+    if ops.compute_units() != 256:
+        pytest.skip("the figures are those of 256 units")
+    plan = ops.gemm_stream_plan
+    assert plan(8, 896, 4864, ops.GEMM_STREAM_SUMS, True) == 8 + 256 + 4 * 65536
+    assert plan(8, 2048, 8192, ops.GEMM_STREAM_SUMS, True) == 8 + 512 + 4 * 65536
+    assert plan(8, 3584, 3584, ops.GEMM_STREAM_SUMS, True) == 8 + 512 + 2 * 65536
+    for n, k, frags in ((3584, 18944, True), (4608, 3584, True), (896, 896, True), (896, 4864, False)):
+        assert plan(8, n, k, ops.GEMM_STREAM_SUMS, frags) is None
+    assert plan(8, 9728, 896, ops.GEMM_STREAM_GATED, True) == 4 + 256 + 65536 and plan(9, 9728, 896, ops.GEMM_STREAM_GATED, True) is None
+    assert plan(16, 8192, 1024, ops.GEMM_STREAM_GATED, True) and plan(2, 22016, 2048, ops.GEMM_STREAM_GATED, True) is None
+    assert plan(4, 14336, 4096, ops.GEMM_STREAM_PLAN_ACT, True) and plan(5, 14336, 4096, ops.GEMM_STREAM_PLAN_ACT, True) is None
+    assert plan(5, 14336, 4096, ops.GEMM_STREAM_POINT, True) and plan(5, 4112, 896, ops.GEMM_STREAM_POINT, False) is None
+    assert plan(2, 16384, 2048, ops.GEMM_STREAM_GATED, True) and plan(3, 16384, 2048, ops.GEMM_STREAM_GATED, True) is None
+    assert plan(17, 896, 896, ops.GEMM_STREAM_POINT, True) is None and plan(0, 896, 896, ops.GEMM_STREAM_POINT, True) is None
+    assert plan(8, 896, 4128, ops.GEMM_STREAM_POINT, True) is None and plan(8, 898, 896, ops.GEMM_STREAM_POINT, True) is None
+    x = torch.zeros((4, 100), dtype=torch.bfloat16, device="cuda")
+    with pytest.raises(ops.KernelError, match="bad sizes"):
+        ops.gemm_mfma_stream(x, torch.zeros((8, 100), dtype=torch.bfloat16, device="cuda"), ops.GEMM_STREAM_POINT, 4 + 256 + 65536)
