@@ -199,6 +199,19 @@ def test_graph_bucket_pads_plans_of_decode_steps():
     assert planner.graph_bucket(Host([(10, 1), (0, 40)], 16, torch.bfloat16)) is None
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("lens, whole", [([30], True), ([60, 5, 63], True), ([3000, 5], False)])
+def test_a_graph_of_whole_requests_has_no_merge(dtype, lens, whole):
+    planner = AttentionPlanner(28, 4, 128, None)
+    planner.compute_units = 256
+    host = Host([(p, 1) for p in lens], 16, dtype)
+    bucket = planner.graph_bucket(host)
+    host.pad = {planner.key: bucket}
+    plan = planner.plan(host)
+    assert (bucket[0] == len(lens)) == whole and plan["n_small"] == bucket[0]
+    assert plan["n_merges"] == (0 if whole else len(lens)) and (plan["n_partial"] == 0) == whole
+
+
 def test_the_short_tile_at_the_end_of_a_long_portion_stays_with_its_group():
     """40 query heads on 8 kv heads give tiles of six tokens: a portion of 2,048 tokens ends with a tile
     of two.  That tile is the last of its group of four, not a small item of its own (which would
