@@ -97,6 +97,13 @@ int fsie_gla_scan(const void* proj, int64_t proj_stride, int q_off, int k_off, i
                   float* chunk_work, int max_chunks, int heads, int dim, int vdim, float q_scale, float inv_tau,
                   int n_slots, int dtype, const float* head_decay, const void* qk, int64_t qk_stride, const float* cos_sin,
                   int rot_pairs, hipStream_t stream);
+// The same for a step of one token a request (bfloat16), with what stands before and behind it: the decays' second product (the
+// bottleneck's values stand in proj too), the norm of every head's o and its gate.
+int fsie_gla_step_takes(int heads, int dim, int vdim, int rank);
+int fsie_gla_step(const void* proj, int64_t proj_stride, int q_off, int k_off, int v_off, int g_off, int a_off, int rank,
+                  const void* a2, const float* a2_bias, float* state, const int32_t* q_starts, const int32_t* seq_slots,
+                  int n_seqs, const float* norm, void* out, int heads, int dim, int vdim, float q_scale, float inv_tau, float eps,
+                  int act, int n_slots, hipStream_t stream);
 // cos_sin [n_tokens][rot_pairs][2] (or null and 0): the first 2 * rot_pairs channels of every q and k head are turned,
 // channel i with channel i + rot_pairs, by the token's cosines and sines as they are read (float32).
 // qk (or null): q and k are read from rows of their own, qk_stride values apart, at the same column offsets.

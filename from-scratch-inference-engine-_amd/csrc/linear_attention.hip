@@ -29,6 +29,7 @@
 #include "common.h"
 #include "api.h"
 #include "chunk_scan_impl.h"
+#include "log_sigmoid.h"
 
 #include <math.h>
 
@@ -40,9 +41,6 @@ constexpr int kGlaCols = 64;
 constexpr int kGlaTokens = 8;  // tokens whose shares of o are added up at once
 constexpr int kGlaChunkThreads = 256;
 
-
-// log(sigmoid(z)) without overflow: min(z, 0) - log(1 + exp(-|z|))
-__device__ __forceinline__ float log_sigmoid(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 
 // Channel i of a head's q or k (x points at it), turned by the token's angles where a rotation is given: the first
 // 2 * pairs channels of a head rotate, channel i with channel i + pairs, by cs[i mod pairs] = (cos, sin); float32.

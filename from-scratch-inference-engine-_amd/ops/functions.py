@@ -1273,6 +1273,41 @@ def gla_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, z: torch.Te
     return out
 
 
+def gla_step_takes(heads: int, dim: int, vdim: int, rank: int) -> bool:
+    """Whether ``gla_step`` takes a layer of these sizes."""
+    return bool(load().fsie_gla_step_takes(int(heads), int(dim), int(vdim), int(rank)))
+
+
+def gla_step(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, g_off: int, a_off: int, a2: torch.Tensor,
+             a2_bias: torch.Tensor, state: torch.Tensor, q_starts: torch.Tensor, seq_slots: torch.Tensor, norm_weight: torch.Tensor,
+             heads: int, dim: int, vdim: int, q_scale: float, inv_tau: float, eps: float, act: str) -> torch.Tensor:
+    """Gated linear attention of a step of one token a request, one launch: ``gla_scan`` with the decays made from the bottleneck
+    (the columns from ``a_off`` of ``proj``, bfloat16) by ``a2`` [heads * dim, rank] and ``a2_bias`` (float32), then ``gated_headnorm``
+    with the gates from column ``g_off``: y [T, heads * vdim] in bfloat16.  The row of a token that is not its request's only one
+    in the step, or whose request has no slot, stays unwritten."""
+    _need(proj, "gla proj", dtype=torch.bfloat16, ndim=2)
+    t, w = proj.shape
+    _need(a2, "gla a2", dtype=torch.bfloat16, ndim=2)
+    rank = a2.shape[1]
+    _need(a2, "gla a2", dtype=torch.bfloat16, shape=(heads * dim, rank))
+    _need(a2_bias, "gla a2 bias", dtype=torch.float32, shape=(heads * dim,))
+    _need(norm_weight, "gla norm", dtype=torch.float32, shape=(vdim,))
+    _need(state, "gla state", dtype=torch.float32, ndim=4)
+    if tuple(state.shape[1:]) != (heads, dim, vdim):
+        raise KernelError(f"gla state: shape {tuple(state.shape)} is not [slots, {heads}, {dim}, {vdim}]")
+    _need(q_starts, "gla q_starts", dtype=torch.int32, ndim=1)
+    _need(seq_slots, "gla seq_slots", dtype=torch.int32, ndim=1)
+    n = seq_slots.shape[0]
+    if q_starts.shape[0] != n + 1 or n > t:
+        raise KernelError("gla: q_starts must have one entry more than seq_slots, and every request a token")
+    out = torch.empty((t, heads * vdim), dtype=torch.bfloat16, device=proj.device)
+    check(load().fsie_gla_step(proj.data_ptr(), w, q_off, k_off, v_off, g_off, a_off, rank, a2.data_ptr(), a2_bias.data_ptr(),
+                               state.data_ptr(), q_starts.data_ptr(), seq_slots.data_ptr(), n, norm_weight.data_ptr(), out.data_ptr(),
+                               heads, dim, vdim, float(q_scale), float(inv_tau), float(eps), gate_act_code(act), state.shape[0],
+                               _stream()))
+    return out
+
+
 # ---------------------------------------------------------------------------------------------
 # attention through a latent
 # ---------------------------------------------------------------------------------------------
