@@ -23,16 +23,8 @@ constexpr int kKeys = 32;      // keys per tile
 constexpr int kMaxChunks = 8;       // head_dim <= 32 * 8 (with 16-byte accesses 2 and 4 have instantiations of their own)
 constexpr int kMaxChunksWide = 16;  // head_dim <= 32 * 16
 
-__device__ __forceinline__ float half_wave_max(float v) {
-#pragma unroll
-    for (int off = 16; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, FSIE_WAVE));
-    return v;
-}
-__device__ __forceinline__ float half_wave_sum(float v) {
-#pragma unroll
-    for (int off = 16; off > 0; off >>= 1) v += __shfl_xor(v, off, FSIE_WAVE);
-    return v;
-}
+__device__ __forceinline__ float half_wave_max(float v) { return max_of_sixteen(max_xor16(v)); }
+__device__ __forceinline__ float half_wave_sum(float v) { return sum_of_sixteen(sum_xor16(v)); }
 
 // Four consecutive elements as floats: one 16-byte (float32) or 8-byte (bfloat16) load.
 __device__ __forceinline__ void load4(const float* p, float (&f)[4]) {

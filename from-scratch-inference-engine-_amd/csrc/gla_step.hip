@@ -15,7 +15,6 @@
 #include "log_sigmoid.h"
 
 #include <math.h>
-#include <type_traits>
 
 namespace {
 
@@ -47,17 +46,6 @@ __device__ __forceinline__ float dot8(uint4 a, uint4 b, float z) {
         z = fmaf(__uint_as_float(x[i] & 0xffff0000u), __uint_as_float(y[i] & 0xffff0000u), z);
     }
     return z;
-}
-
-// The sum over eight consecutive lanes, in all of them.
-__device__ __forceinline__ float sum_of_eight(float v) {
-    auto from = [](float v, auto ctrl) {
-        return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), decltype(ctrl)::value, 0xf, 0xf, true));
-    };
-    v += from(v, std::integral_constant<int, 0xB1>{});   // the neighbour
-    v += from(v, std::integral_constant<int, 0x4E>{});   // the other pair of the four
-    v += from(v, std::integral_constant<int, 0x141>{});  // mirrored within eight: the other four
-    return v;
 }
 
 // CPL consecutive floats, one access
