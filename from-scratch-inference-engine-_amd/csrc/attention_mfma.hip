@@ -107,6 +107,8 @@ extern "C" int fsie_attention_mfma_qkv(const float* sums, int n_parts, int n_tok
     f.slopes = slopes;
     f.row_scale = row_scale;
     f.n_parts = n_parts;
+    f.group = n_heads / n_kv;
+    f.page_magic = fsie_attn::magic_of(page_size);
     return fn(f, k_pool, v_pool, block_tables, max_pages, items, n_items, out, partials, n_heads, n_kv, page_size,
               window, scale, waves, stream);
 }

@@ -1,6 +1,6 @@
 // Causal grouped-query attention over the pages of the cache on the matrix cores (bfloat16).
 //
-// One wave per work item and kv head (chunk).  Everything is computed transposed so that no
+// One workgroup per work item and kv head (chunk).  Everything is computed transposed so that no
 // operand ever has to change lanes or pass through LDS:
 //
 //   S^T[key, row] = K[key, :] . Q[row, :]      A = K rows from the cache (16 B per lane),
@@ -26,11 +26,14 @@
 // kv head's group).  Requires page_size % 4 == 0; with a page size that is a multiple of 8 a
 // lane's 8 values of a dimension come with one load instead of two.
 //
-// A workgroup may have several waves (up to MAXW; 4 when NT > 1): they split the item's key range
-// into contiguous runs of blocks, and their partial results are combined inside the workgroup:
-// maxima and sums through LDS, then the first wave adds the others' rescaled accumulators to its
-// own in the fixed order of the waves.  Decoding against a long context therefore needs neither partial
-// records in memory nor a second kernel, and the result does not depend on timing.
+// One query tile: an item's blocks are dealt to the waves of its workgroup, a block a wave where the item is short, and the
+// waves' results meet in LDS, in the fixed order of the waves, behind one barrier.  Decoding against a long context needs
+// neither partial records in memory nor a second kernel, and the result does not depend on timing.
+// Such a step is bound by the chain inside a workgroup: the item, the block table, the keys, one trip to memory each, then
+// products and exponentials that wait for each other.  So no wave takes two blocks where another has none, masks are selects (no
+// branch a value), and little code is run once: 10 KB of instructions, not 31.  One request of the 0.5B shape and 60 to 110
+// keys 7.2 -> 4.5 us from a workgroup's first instruction to its last, eight of the 7B shape and 64 to 550 6.6 -> 5.0.
+// Several query tiles (NT > 1, up to 4 waves): a wave per 512 keys, combined by the first wave.
 //
 // QKV: the variant for steps of one token a request takes q, k and v as the float32 partial sums
 // that a product in slices of K leaves, and finishes them itself: every workgroup adds up the
@@ -42,6 +45,7 @@
 #include "common.h"
 #include "api.h"
 
+#include <limits.h>
 #include <math.h>
 
 namespace fsie_attn {
@@ -84,7 +88,11 @@ struct QkvSums {
     const float* slopes;     // [n_heads] or null: slopes[h] * (query position - key position) is taken off the (capped)
                              // scores of head h (any variant)
     const float* row_scale;  // [n_tokens] or null: a factor on all scores of a token, before the cap (any variant)
+    int group;               // heads a kv head (any variant)
+    uint32_t page_magic;     // 2^32 / page_size, rounded up: a key's page by one multiplication (any variant)
 };
+
+inline uint32_t magic_of(int page_size) { return 0xFFFFFFFFu / static_cast<uint32_t>(page_size) + 1u; }
 
 // Element d of a head after the rotation of the pairs (i, i + HD / 2) by the angles whose
 // cosines and sines are cs[i].  One fixed sequence of roundings, whoever asks: the key that a
@@ -115,6 +123,11 @@ __device__ __forceinline__ uint4 rotated8(const float* head, const float2* cs, i
                  pack2_bf16(rotated_by(a1.z, b1.z, t3.x, t3.y, hi), rotated_by(a1.w, b1.w, t3.z, t3.w, hi))};
 }
 
+// A bit for each of eight consecutive keys that is among the first n (n of any sign).
+__device__ __forceinline__ uint32_t keys_below(int n) { return (1u << min(max(n, 0), 8)) - 1u; }
+
+constexpr int kFarBelow = INT_MIN / 2;  // below every key
+
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
@@ -122,15 +135,18 @@ template <int HDT>
 constexpr int max_waves() {
     return HDT <= 4 ? 16 : (HDT <= 8 ? 8 : 4);  // registers per wave grow with the head size
 }
+// The variant for items of up to four blocks of keys (what a step with idle compute units is cut into): a wave a block, and
+// with QKV one more for the new key.
+constexpr int kShortWaves = 4;
 
 // BIASED false: no distance bias and no factor a token, known when the kernel is compiled (the QKV variants have no
 // registers to spare for them); true: whatever slopes and row_scale say.
 template <int HDT, int NT, int MAXW, bool V16, bool QKV = false, bool BIASED = true>
-__global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW == 1 && NT > 1 ? 2 : 1))) void attention_mfma_kernel(
+__global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW == 1 && NT > 1 ? 2 : 1))) void attention_mfma_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_pool,
     const bf16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_pages,
     const int32_t* __restrict__ items, bf16_t* __restrict__ out, float* __restrict__ partials, int n_heads,
-    int n_kv, int page_size, int window, float scale, int gh, int head_chunks, QkvSums f) {
+    int n_kv, int page_size, int window, float scale, int gh, QkvSums f) {
     static_assert(!QKV || (NT == 1 && HDT % 2 == 0), "the QKV variant: one query tile, head_dim a multiple of 32");
     constexpr int HD = HDT * 16;
     // scores: 32-wide steps over the head dimension when head_dim is a multiple of 32, else
@@ -142,19 +158,23 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
     constexpr int S16A = S16 > 0 ? S16 : 1;
 
     const int32_t* item = items + static_cast<int64_t>(blockIdx.x) * FSIE_ATTN_ITEM_INTS;
-    const int seq = item[FSIE_ATTN_ITEM_SEQ];
-    const int q_row0 = item[FSIE_ATTN_ITEM_QROW];
-    const int n_q = item[FSIE_ATTN_ITEM_NQ];
-    const int pos0 = item[FSIE_ATTN_ITEM_POS];
-    const int key_begin = item[FSIE_ATTN_ITEM_KBEGIN];
-    int key_end = item[FSIE_ATTN_ITEM_KEND];
-    const int partial_base = item[FSIE_ATTN_ITEM_PARTIAL];
+    // (the item in one scalar load: its fields one by one are trips of their own, each behind the last one's use)
+    typedef int ItemInts __attribute__((ext_vector_type(8), aligned(4)));
+    static_assert(FSIE_ATTN_ITEM_INTS == 8, "an item is eight numbers");
+    const ItemInts it = *reinterpret_cast<const ItemInts*>(item);
+    const int seq = it[FSIE_ATTN_ITEM_SEQ];
+    const int q_row0 = it[FSIE_ATTN_ITEM_QROW];
+    const int n_q = it[FSIE_ATTN_ITEM_NQ];
+    const int pos0 = it[FSIE_ATTN_ITEM_POS];
+    const int key_begin = it[FSIE_ATTN_ITEM_KBEGIN];
+    int key_end = it[FSIE_ATTN_ITEM_KEND];
+    const int partial_base = it[FSIE_ATTN_ITEM_PARTIAL];
     if (n_q <= 0) return;  // padding item
     // The first keys of the request that a window keeps: seen whatever the window says.  An item told to
     // (FSIE_ATTN_KEEP_WALK) reads those that lie before its own range too, [0, prefix_end), as blocks of
     // their own ahead of the range's blocks.
-    const int keep = item[FSIE_ATTN_ITEM_KEEP] & ~FSIE_ATTN_KEEP_WALK;
-    const int prefix_end = (item[FSIE_ATTN_ITEM_KEEP] & FSIE_ATTN_KEEP_WALK) ? min(keep, key_begin) : 0;
+    const int keep = it[FSIE_ATTN_ITEM_KEEP] & ~FSIE_ATTN_KEEP_WALK;
+    const int prefix_end = (it[FSIE_ATTN_ITEM_KEEP] & FSIE_ATTN_KEEP_WALK) ? min(keep, key_begin) : 0;
     // QKV: the item whose keys end with the request's new one walks the cache up to it and takes
     // the new key and value from the sums
     const bool owner = QKV && pos0 >= key_begin && pos0 < key_end;
@@ -162,60 +182,50 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
     int new_slot = -1;
     if constexpr (QKV) new_slot = f.slots[q_row0];
 
-    const int group = n_heads / n_kv;
-    const int kvh = blockIdx.y / head_chunks;
-    const int chunk = blockIdx.y - kvh * head_chunks;
+    const int group = f.group;
+    const int kvh = blockIdx.y, chunk = blockIdx.z;
     const int gh_here = min(gh, group - chunk * gh);
     const int h_base = kvh * group + chunk * gh;
     const int n_rows = n_q * gh;
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    // (the QKV variant of one wave is launched with four: three only help to add up the sums)
-    const int n_waves = QKV && MAXW == 1 ? 1 : blockDim.x >> 6;
+    const int n_waves = blockDim.x >> 6;
     const int c = lane & 15;  // column of S^T and O^T (query row of a tile); row of the A tiles
     const int G = lane >> 4;  // lane group: which 4 (or 8) of the reduction indices this lane holds
     const int32_t* table = block_tables + static_cast<int64_t>(seq) * max_pages;
     const float scale2 = scale * kLog2e;  // scores in units of log2 e: exp() becomes exp2()
     // capped scores: softcap * tanh(product * scale / softcap), in the same units
-    const bool capped = f.softcap > 0.f;
+    const bool capped = !QKV && f.softcap > 0.f;
     const float cap2 = f.softcap * kLog2e, cap_in = capped ? scale / f.softcap : scale2;
-    auto scaled = [&](float product, float in) { return capped ? cap2 * tanh_by_exp(product * in) : product * in; };
     // the distance bias, in the same units: slope (key - query), added to the scaled scores
     const bool sloped = BIASED && f.slopes != nullptr;
 
-    // LDS: the accumulators that the waves after the first hand over at the end; before that, in
-    // the QKV variant, the heads added up from the sums (up to 16 of queries, a key, a value) and
-    // the cosines and sines
-    constexpr int kCombine = MAXW > 1 ? (MAXW - 1) * NT * HDT * 64 : 0;
+    // LDS: the accumulators that the waves hand over at the end; and in the QKV variant the heads added up from
+    // the sums (up to 16 of queries, a key, a value) and the cosines and sines, which a wave may still read when another
+    // hands over: apart, where a unit's LDS holds two workgroups of both, else in the same place behind a barrier
+    constexpr int kCombine = MAXW == 1 ? 0 : NT == 1 ? MAXW * HDT * 64 : (MAXW - 1) * NT * HDT * 64;
     // a head's row in LDS is four floats longer than the head, so that the 16 rows that a wave reads
     // at once, 16 bytes each, fall into different banks
     constexpr int RS = HD + 4;
     constexpr int kHeads = QKV ? (18 * RS + HD) / 4 : 0;
-    constexpr int kLds = kCombine > kHeads ? kCombine : (kHeads > 0 ? kHeads : 1);
-    __shared__ floatx4 s_o[kLds];
-    float* s_row = reinterpret_cast<float*>(s_o);
+    constexpr bool kApart = HDT <= 8;
+    constexpr int kLds = kApart ? kCombine + kHeads : (kCombine > kHeads ? kCombine : kHeads);
+    __shared__ floatx4 s_o[kLds > 0 ? kLds : 1];
+    float* s_row = reinterpret_cast<float*>(s_o + (kApart ? kCombine : 0));
     float2* s_cs = reinterpret_cast<float2*>(s_row + 18 * RS);
     // The heads this workgroup needs, added up over the slices, with the bias, into LDS.  In two
     // steps: first all the reads of up to eight slices, in straight-line code (a slice past the last
     // reads the last one again, a thread without a column reads column 0), so that they are under
-    // way together, and with the reads of the first keys where the same wave walks keys; then the
+    // way together, and with the reads of the first keys; then the
     // additions.  A loop of one read and one addition a slice would be a trip to memory a slice.
-    // The variant of one wave is launched with four: the other three add up the sums and leave
-    // after the barrier, so that the first has only its keys under way.  The hardware counts 63
-    // reads of a wave at most, and a wait for one of 27 reads of sums behind 64 of keys would wait
-    // for most of the keys too.
-    constexpr int kThreadsLeast = MAXW == 1 ? 192 : 64 * MAXW;  // threads that add up sums
-    constexpr int NJ = QKV ? (18 * HD / 4 + kThreadsLeast - 1) / kThreadsLeast : 1;  // columns of four a thread
+    constexpr int NJ = QKV ? (18 * HD / 4 + 64 * MAXW - 1) / (64 * MAXW) : 1;  // columns of four a thread
     constexpr int PC = NJ <= 3 ? 8 : 4;                                              // slices read at once
     float4 part[NJ][PC], bias_of[NJ];
     float2 angle = float2{1.f, 0.f};
     int lds_at[NJ];
     const float* col_at[NJ];
-    const int sum_thread = MAXW == 1 ? static_cast<int>(threadIdx.x) - 64 : static_cast<int>(threadIdx.x);
-    const int sum_threads = MAXW == 1 ? static_cast<int>(blockDim.x) - 64 : static_cast<int>(blockDim.x);
-    const bool helper = QKV && MAXW == 1 && wave > 0;  // a wave that only adds up sums
-    const bool sums_here = MAXW > 1 || wave > 0;
+    const int sum_thread = static_cast<int>(threadIdx.x), sum_threads = static_cast<int>(blockDim.x);
     auto issue_sums = [&]() {
         const int q_dim = n_heads * HD, kv_dim = n_kv * HD;
         const int n_cols = (gh_here + 2) * HD;
@@ -227,7 +237,7 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
                 continue;
             }
             const int i = (sum_thread + j * sum_threads) * 4;
-            const bool has = i >= 0 && i < n_cols;
+            const bool has = i < n_cols;
             const int ic = has ? i : 0;
             const int seg = ic / HD, d = ic - seg * HD;
             lds_at[j] = has ? seg * RS + d : -1;
@@ -240,7 +250,7 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
         }
         if (f.cos_sin) {
             const float2* cs = reinterpret_cast<const float2*>(f.cos_sin) + static_cast<int64_t>(q_row0) * (HD / 2);
-            angle = cs[min(max(sum_thread, 0), HD / 2 - 1)];
+            angle = cs[min(sum_thread, HD / 2 - 1)];
         }
     };
     auto finish_sums = [&]() {
@@ -259,7 +269,7 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
             if (f.bias) a = float4{a.x + bias_of[j].x, a.y + bias_of[j].y, a.z + bias_of[j].z, a.w + bias_of[j].w};
             if (lds_at[j] >= 0) *reinterpret_cast<float4*>(s_row + lds_at[j]) = a;
         }
-        for (int i = max(sum_thread, 0); i < HD / 2; i += sum_threads) {
+        for (int i = sum_thread; i < HD / 2; i += sum_threads) {
             if (i == sum_thread || !f.cos_sin) s_cs[i] = angle;  // (without a table: cosine 1, sine 0)
             else s_cs[i] = (reinterpret_cast<const float2*>(f.cos_sin) + static_cast<int64_t>(q_row0) * (HD / 2))[i];
         }
@@ -274,7 +284,7 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         const int rg = nt * 16 + c;
-        const int tq = rg / gh, hh = rg - tq * gh;
+        const int tq = QKV ? 0 : rg / gh, hh = rg - tq * gh;
         rvalid[nt] = rg < n_rows && hh < gh_here;
         rtok[nt] = tq;
         rhead[nt] = h_base + hh;
@@ -310,9 +320,8 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
 
     const int64_t head_stride = static_cast<int64_t>(page_size) * HD;  // one kv head of one page
     // key / page_size as one multiplication (the host has checked that keys * page_size < 2^32): a
-    // division by a size known only at run time costs some thirty vector instructions, four times
-    // per block of 32 keys
-    const uint32_t page_magic = 0xFFFFFFFFu / static_cast<uint32_t>(page_size) + 1u;
+    // division by a size known only at run time costs some thirty vector instructions
+    const uint32_t page_magic = f.page_magic;
     // this wave's run of key blocks
     const int kb_first = key_begin & ~31;
     // The walk runs over block coordinates: from kb_first on a coordinate is the key itself; the blocks of
@@ -320,12 +329,13 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
     const int pre_len = (prefix_end + 31) & ~31;
     const int walk_first = kb_first - pre_len;
     const int n_blocks = ((key_end - kb_first + 31) >> 5) + (pre_len >> 5);
-    // an item uses one wave per 4 blocks (128 keys) of its own when it has one query tile, per 16
-    // blocks (512 keys) when it has several, however many waves the launch has: how its keys are
-    // split depends on the item alone
-    constexpr int kBlocksPerWave = NT == 1 ? 4 : 16;
-    const int n_active = min(n_waves, max(1, (n_blocks + kBlocksPerWave - 1) / kBlocksPerWave));
-    const int per_wave = (n_blocks + n_active - 1) / n_active;
+    // One query tile: an item's blocks are dealt to as many waves as it has blocks, up to what the head size allows, in runs
+    // of equal length; several tiles: a wave per 16 blocks (512 keys).  How its keys are split depends on the item alone: the
+    // variant for short items has fewer waves, but only where every one of them has a block of its own either way.
+    constexpr int kKeyWaves = QKV && MAXW == kShortWaves + 1 ? kShortWaves : MAXW;
+    const int n_run_of = NT == 1 ? (n_blocks + kKeyWaves - 1) / kKeyWaves : 0;
+    const int n_active = NT == 1 ? max(1, n_run_of > 0 ? (n_blocks + n_run_of - 1) / n_run_of : 1) : min(n_waves, max(1, (n_blocks + 15) / 16));
+    const int per_wave = NT == 1 ? n_run_of : (n_blocks + n_active - 1) / n_active;
     // QKV: the request's new key is a run of its own, for a wave that the keys of the cache leave
     // idle if there is one (else for the first); n_runs = waves whose results are combined
     const int new_key_wave = owner && n_active < n_waves ? n_active : 0;
@@ -340,39 +350,43 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
     };
     // V16: the page size is a multiple of 8, so the keys 8 G .. 8 G + 7 of a block lie in one page,
     // 16-byte aligned (a template flag: a run-time branch around the loads costs a third of the speed)
-    // Where the four runs of a block's keys lie: the two tiles of 16 keys of the scores (one key
-    // per lane, c) and the two runs of 4 consecutive keys per lane group of the second product
-    // (never across a page: page_size % 4 == 0).  A key without a page (past the end, or behind a
-    // window) points at page 0: what is read there is finite and its probability is zero.
+    // Where a block's keys lie: for the scores the two tiles of 16 keys (one key per lane, c), for the second product the two
+    // runs of 4 consecutive keys per lane group (never across a page: page_size % 4 == 0; with V16 eight keys from a multiple
+    // of eight on lie in one page, so one table entry serves both runs).  A key without a page (past the end, or behind a
+    // window) points at page 0: what is read there is finite and its probability is zero; so it is with the keys behind the
+    // last one in that one's page.
+    constexpr int RUN = V16 ? 1 : 2;
     struct Where {
-        int64_t k[2], v[2];  // element offsets into the pools
+        int64_t k[RUN], v[RUN];  // element offsets into the pools
     };
     struct Asked {
-        int page[4], idx[4], key[4];
+        int page[2 * RUN], idx[2 * RUN], key[2 * RUN];
         int limit;  // keys from here on do not belong to the block's range
     };
     auto ask_pages = [&](int kb, Asked& p) {
-        p.limit = kb >= kb_first ? key_end : prefix_end;
+        const int of_range = key_end, of_kept = prefix_end;
+        p.limit = kb >= kb_first ? of_range : of_kept;
         kb = kb >= kb_first ? kb : kb - walk_first;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            p.key[t] = kb + 8 * (c >> 2) + 4 * t + (c & 3);
-            p.key[2 + t] = kb + 8 * G + 4 * t;
+        for (int t = 0; t < RUN; ++t) {
+            p.key[t] = kb + 8 * (c >> 2) + 4 * t;
+            p.key[RUN + t] = kb + 8 * G + 4 * t;
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {  // the four table reads go out together
+        for (int i = 0; i < 2 * RUN; ++i) {  // the table reads go out together
             p.idx[i] = static_cast<int>(__umulhi(static_cast<uint32_t>(p.key[i]), page_magic));
             p.page[i] = table[min(p.idx[i], max_pages - 1)];
         }
     };
+    const int64_t page_stride = n_kv * head_stride, kv_base = kvh * head_stride;
     auto place = [&](const Asked& p, Where& at) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const bool ok = p.key[i] < p.limit && p.idx[i] < max_pages && p.page[i] >= 0;
-            const int64_t head = (static_cast<int64_t>(ok ? p.page[i] : 0) * n_kv + kvh) * head_stride;
+        for (int i = 0; i < 2 * RUN; ++i) {
+            const bool ok = (p.key[i] < p.limit) & (p.idx[i] < max_pages) & (p.page[i] >= 0);
+            const int64_t head = static_cast<int64_t>(static_cast<uint32_t>(ok ? p.page[i] : 0)) * page_stride + kv_base;
             const int off = ok ? p.key[i] - p.idx[i] * page_size : 0;
-            if (i < 2) at.k[i] = head + static_cast<int64_t>(off) * HD + (X32 ? 8 : 4) * G;
-            else at.v[i - 2] = head + off + static_cast<int64_t>(c) * page_size;
+            if (i < RUN) at.k[i] = head + static_cast<uint32_t>((off + (c & 3)) * HD + (X32 ? 8 : 4) * G);
+            else at.v[i - RUN] = head + static_cast<uint32_t>(off + c * page_size);
         }
     };
     auto locate = [&](int kb, Where& at) {
@@ -383,7 +397,7 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
     auto load_block = [&](const Where& at, Block& blk) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const bf16_t* kp = k_pool + at.k[t];
+            const bf16_t* kp = k_pool + at.k[V16 ? 0 : t] + (V16 ? 4 * t * HD : 0);
 #pragma unroll
             for (int s = 0; s < S32; ++s) blk.kf[t][s].raw = ld16(kp + s * 32);
 #pragma unroll
@@ -395,10 +409,10 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
             for (int dt = 0; dt < HDT; ++dt) {
                 // (streaming loads where several waves walk long runs of keys; the short items of one wave are slower with them)
                 const bf16_t* vp = v0 + static_cast<int64_t>(dt * 16) * page_size;
-                blk.vf[dt].raw = MAXW > 1 ? ld16_once(vp) : ld16(vp);
+                blk.vf[dt].raw = MAXW > kShortWaves + 1 ? ld16_once(vp) : ld16(vp);
             }
         } else {
-            const bf16_t* v1 = v_pool + at.v[1];
+            const bf16_t* v1 = v_pool + at.v[RUN - 1];
 #pragma unroll
             for (int dt = 0; dt < HDT; ++dt) {
                 const uint2 lo = ld8(v0 + static_cast<int64_t>(dt * 16) * page_size);
@@ -410,6 +424,8 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
     auto compute_block = [&](int kb, const Block& blk) {
         const bool kept_block = kb < kb_first;  // a block of the kept first keys (the same for the whole wave)
         if (kept_block) kb -= walk_first;
+        const int of_range = key_end, of_kept = prefix_end;  // (values: a choice between the variables themselves is one of addresses)
+        const int range_begin = kept_block ? 0 : key_begin, range_end = kept_block ? of_kept : of_range;
         const bool full = !kept_block && kb >= key_begin && kb + 32 <= key_end && kb + 31 <= pos0 &&
                           (window <= 0 || kb > pos0 + n_q - 1 - window);  // the same for the whole wave
 #pragma unroll
@@ -426,41 +442,43 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
                 for (int s = 0; s < S16; ++s)
                     st[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(blk.kt[t][s].v, qt[nt][s].v, st[t], 0, 0, 0);
             }
-            // ---- mask, running maximum.  A block that every row of the item sees whole (below
-            // the diagonal, inside the key range and the window) needs no mask; in a long
-            // portion that is nearly every block.
+            // ---- scores, mask, running maximum; no branch a value (a mask of 64 branches was 3 of the 8.5 us of a step of one
+            // request: each an exec mask and cold instructions).  A block that every row of the item sees whole (below the
+            // diagonal, inside the key range and the window) needs no mask; in a long portion that is nearly every block.
             float sv[8];
-            float m_loc = -INFINITY;
-            if (full) {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) sv[i] = scaled(st[i >> 2][i & 3], r_in[nt]);
-            } else {
+            for (int i = 0; i < 8; ++i) sv[i] = st[i >> 2][i & 3] * r_in[nt];
+            if (capped) {  // (the same for the whole launch)
 #pragma unroll
-                for (int t = 0; t < 2; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int key = kb + 8 * G + 4 * t + r;
-                        const bool in_range = kept_block ? key < prefix_end : (key >= key_begin && key < key_end);
-                        const bool vis = rvalid[nt] && in_range && key <= rpos[nt] &&
-                                         (window <= 0 || key > rpos[nt] - window || key < keep);
-                        sv[t * 4 + r] = vis ? scaled(st[t][r], r_in[nt]) : -INFINITY;
-                    }
+                for (int i = 0; i < 8; ++i) sv[i] = cap2 * tanh_by_exp(sv[i]);
             }
-            if (sloped) {  // (the same for the whole launch; hidden keys stay at minus infinity)
-                const float at_first = r_slope[nt] * static_cast<float>(kb + 8 * G - rpos[nt]);
+            const int first = kb + 8 * G;  // this lane's keys: first .. first + 7
+            if (sloped) {  // (the same for the whole launch)
+                const float at_first = r_slope[nt] * static_cast<float>(first - rpos[nt]);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) sv[i] += fmaf(r_slope[nt], static_cast<float>(i), at_first);
             }
+            if (!full) {
+                // of the block's range, up to the row's own position: the keys inside the window, and the kept first ones
+                const int upto = min(range_end, rpos[nt] + 1), hi = rvalid[nt] ? upto : kFarBelow;
+                const int in_window = rpos[nt] - window + 1, seen = window > 0 ? in_window : kFarBelow;
+                const uint32_t vis = keys_below(hi - first) & ~keys_below(range_begin - first) &
+                                     (~keys_below(seen - first) | keys_below(keep - first));
 #pragma unroll
-            for (int i = 0; i < 8; ++i) m_loc = fmaxf(m_loc, sv[i]);
+                for (int i = 0; i < 8; ++i) sv[i] = (vis & (1u << i)) != 0u ? sv[i] : -INFINITY;
+            }
+            float m_loc = sv[0];
+#pragma unroll
+            for (int i = 1; i < 8; ++i) m_loc = fmaxf(m_loc, sv[i]);
             m_loc = max_xor32(max_xor16(m_loc));
             const float m_new = fmaxf(m_run[nt], m_loc);
-            const float corr = (m_run[nt] == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_run[nt] - m_new);
+            const float m_of = m_new == -INFINITY ? 0.f : m_new;  // (a row without a key so far: all its probabilities zero)
+            const float corr = (m_run[nt] == -INFINITY) ? 1.f : __builtin_amdgcn_exp2f(m_run[nt] - m_of);
             float p[8];
             float p_sum = 0.f;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                p[i] = (sv[i] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(sv[i] - m_new);
+                p[i] = __builtin_amdgcn_exp2f(sv[i] - m_of);
                 p_sum += p[i];
             }
             l_run[nt] = l_run[nt] * corr + p_sum;  // this lane's keys only; lane groups are summed at the end
@@ -488,12 +506,8 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
     // its data is in flight while the matrix cores work on the present one (few waves run here,
     // so occupancy does not hide the latency).
     constexpr bool PREFETCH = NT == 1 && HDT <= 8;
-    // A workgroup of one wave (items of up to 128 keys, what a step with idle compute units is cut
-    // into) has all 512 registers of its SIMD: the table reads of its four blocks go out together,
-    // then all their data reads, and the products follow; one trip to memory for the addresses and
-    // one for the data, where fetching a block ahead costs a trip per block (8.0 -> 7.3 us a layer for
-    // eight requests of 640 keys).
-    constexpr bool ALL_AHEAD = PREFETCH && MAXW == 1;
+    // (the variant for short items has one block a wave, as a rule)
+    constexpr bool SHORT = NT == 1 && MAXW <= kShortWaves + 1 && HDT <= 8;
     // QKV: the new key and value, from the sums: a block of their own whose first key they are (the
     // mask hides the rest), and into the pools for the steps to come.  An idle wave does it, or the
     // first one before its walk, while its first keys from the cache are under way.
@@ -519,77 +533,56 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
             nb.vf[dt].raw = uint4{G == 0 ? pack2_bf16(vh[dt * 16 + c], 0.f) : 0u, 0u, 0u, 0u};
         compute_block(pos0, nb);
         key_end = pos0;
-        if (chunk == 0 && new_slot >= 0 && new_slot < f.pool_slots) {
-            const int page = new_slot / page_size;
-            const int off = new_slot - page * page_size;
-            bf16_t* kd = f.k_out + ((static_cast<int64_t>(page) * n_kv + kvh) * page_size + off) * HD;
-            for (int d = 2 * lane; d < HD; d += 128)
-                *reinterpret_cast<uint32_t*>(kd + d) = pack2_bf16(rotated<HD>(kh, s_cs, d), rotated<HD>(kh, s_cs, d + 1));
-            bf16_t* vd = f.v_out + (static_cast<int64_t>(page) * n_kv + kvh) * head_stride + off;
-            for (int d = lane; d < HD; d += 64) vd[static_cast<int64_t>(d) * page_size] = from_float<bf16_t>(vh[d]);
-        }
+    };
+    // ... and into the pools, by a wave that has the least to do
+    auto keep_new_key = [&]() {
+        if (!(owner && chunk == 0 && new_slot >= 0 && new_slot < f.pool_slots)) return;
+        const float* kh = s_row + gh_here * RS;
+        const float* vh = kh + RS;
+        const int page = new_slot / page_size;
+        const int off = new_slot - page * page_size;
+        bf16_t* kd = f.k_out + ((static_cast<int64_t>(page) * n_kv + kvh) * page_size + off) * HD;
+        for (int d = 2 * lane; d < HD; d += 128)
+            *reinterpret_cast<uint32_t*>(kd + d) = pack2_bf16(rotated<HD>(kh, s_cs, d), rotated<HD>(kh, s_cs, d + 1));
+        bf16_t* vd = f.v_out + (static_cast<int64_t>(page) * n_kv + kvh) * head_stride + off;
+        for (int d = lane; d < HD; d += 64) vd[static_cast<int64_t>(d) * page_size] = from_float<bf16_t>(vh[d]);
     };
 
     // QKV: the block table (warm in the L2) is read first, then the reads of the sums (which come from
     // further away) and of the first keys go out together; the queries are built from LDS while the keys
     // are under way
-    if constexpr (ALL_AHEAD) {
-        Where at[4];
-        Block blk[4];
-        auto locate4 = [&](int kb0) {
-#pragma unroll
-            for (int d = 0; d < 4; ++d) locate(kb0 + 32 * d, at[d]);  // past the end: page 0, masked below
-        };
-        auto load4 = [&]() {
-#pragma unroll
-            for (int d = 0; d < 4; ++d) load_block(at[d], blk[d]);
-        };
-        const bool any = !helper && kb_begin < kb_end;
-        if (any) locate4(kb_begin);
-        if (any) load4();
-        if constexpr (QKV) {
-            if (sums_here) {
-                issue_sums();
-                finish_sums();
-            }
-            __syncthreads();
-            if (helper) return;
-            build_queries();
-            score_new_key();
-        }
-        for (int kb0 = kb_begin; kb0 < kb_end; kb0 += 4 * 32) {
-            if (kb0 > kb_begin) {
-                locate4(kb0);
-                load4();
-            }
-#pragma unroll
-            for (int d = 0; d < 4; ++d)
-                if (kb0 + 32 * d < kb_end) compute_block(kb0 + 32 * d, blk[d]);
-        }
-    } else {
-        const bool any = !helper && kb_begin < kb_end;
+    {
+        const bool any = kb_begin < kb_end;
         Where at;
         Block cur, nxt;
         // (QKV: the reads of the sums, which come from further away than the table, go out before the
         // wait for the table)
         Asked first;
         if (any) ask_pages(kb_begin, first);
-        if constexpr (QKV)
-            if (sums_here) issue_sums();
+        if constexpr (QKV) issue_sums();
         if (any) place(first, at);
         if (PREFETCH && any) {
             load_block(at, cur);
-            locate(kb_begin + 32, at);
+            if (!SHORT) locate(kb_begin + 32, at);
         }
         if constexpr (QKV) {
-            if (sums_here) finish_sums();
+            finish_sums();
             __syncthreads();
-            if (helper) return;
             build_queries();
             score_new_key();
+            if (wave == (new_key_wave == n_waves - 1 ? 0 : n_waves - 1)) keep_new_key();
+            if (!kApart) __syncthreads();
         }
         constexpr bool IN_TURN = QKV && MAXW <= 8;  // (16 waves a workgroup have 128 registers each: not enough)
-        if (PREFETCH && any && !IN_TURN) {
+        if (SHORT && any) {
+            for (int kb = kb_begin;;) {
+                compute_block(kb, cur);
+                kb += 32;
+                if (kb >= kb_end) break;
+                locate(kb, at);
+                load_block(at, cur);
+            }
+        } else if (PREFETCH && any && !IN_TURN) {
             for (int kb = kb_begin; kb < kb_end; kb += 32) {
                 if (kb + 32 < kb_end) {
                     load_block(at, nxt);
@@ -628,7 +621,83 @@ __global__ __launch_bounds__(QKV && MAXW == 1 ? 256 : 64 * MAXW) __attribute__((
         }
     }
 
-    // ---- the denominator and maximum of every query row; several waves combine inside the
+    // ---- one query tile: every wave with keys lays its accumulators, maxima and sums into LDS, and behind a barrier
+    // the waves deal the sixteens of the head's values among themselves, each adding the runs up in their fixed order, relative to the
+    // common maximum, and writing its part of the result (one barrier, no atomics).  By the first wave alone, behind two
+    // barriers, the runs of eight waves would be 64 reads of LDS in a row.
+    if constexpr (NT == 1) {
+        constexpr int MW = (MAXW + 3) / 4 * 4;
+        __shared__ float s_m1[16][MW + 4], s_l1[16][MW + 4];  // [column][wave]: a lane reads its column's waves four at a time
+        if (wave < n_runs) {
+#pragma unroll
+            for (int dt = 0; dt < HDT; ++dt) s_o[(wave * HDT + dt) * 64 + lane] = acc[0][dt];
+        }
+        const float l_w = sum_xor32(sum_xor16(l_run[0]));
+        if (G == 0) {  // (a wave without keys: minus infinity and zero)
+            s_m1[c][wave] = m_run[0];
+            s_l1[c][wave] = l_w;
+        }
+        __syncthreads();
+        if (!rvalid[0]) return;
+        float m_of_run[MW], l_of_run[MW], factor[MW];
+#pragma unroll
+        for (int w = 0; w < MW; w += 4) {
+            const floatx4 m4 = *reinterpret_cast<const floatx4*>(&s_m1[c][w]), l4 = *reinterpret_cast<const floatx4*>(&s_l1[c][w]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bool is = w + i < MAXW && w + i < n_runs;
+                m_of_run[w + i] = is ? m4[i] : -INFINITY;
+                l_of_run[w + i] = is ? l4[i] : 0.f;
+            }
+        }
+        float m_all = m_of_run[0];
+#pragma unroll
+        for (int w = 1; w < MAXW; ++w) m_all = fmaxf(m_all, m_of_run[w]);
+        const float m_of = m_all == -INFINITY ? 0.f : m_all;
+        float denom = 0.f;
+#pragma unroll
+        for (int w = 0; w < MW; ++w) {
+            factor[w] = __builtin_amdgcn_exp2f(m_of_run[w] - m_of);
+            denom = fmaf(l_of_run[w], factor[w], denom);
+        }
+        float inv = 1.f;
+        if (partial_base < 0) {
+            float whole = denom;
+            if (f.sinks && m_all != -INFINITY) whole += __builtin_amdgcn_exp2f(f.sinks[rhead[0]] * kLog2e - m_all);
+            inv = whole > 0.f ? 1.0f / whole : 0.f;
+        }
+        bf16_t* o = out + (static_cast<int64_t>(q_row0 + rtok[0]) * n_heads + rhead[0]) * HD + 4 * G;
+        // (a cut item's record: unnormalised sums, their maximum in natural units and denominator, for attention_merge)
+        float* rec = partials + (static_cast<int64_t>(max(partial_base, 0) + rtok[0]) * n_heads + rhead[0]) * (HD + 2);
+        for (int dt = wave; dt < HDT; dt += n_waves) {
+            // lane holds O^T[d = 16 dt + 4 G + r][row c]
+            floatx4 a{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w0 = 0; w0 < MAXW; w0 += 4) {
+                if (w0 >= n_runs) break;  // (the same for the whole workgroup)
+                floatx4 v[4];  // four at once, past the last run the last one again, not added
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = s_o[(min(w0 + i, n_runs - 1) * HDT + dt) * 64 + lane];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) a[r] = w0 + i < n_runs ? fmaf(v[i][r], factor[w0 + i], a[r]) : a[r];
+            }
+            if (partial_base < 0) {
+                *reinterpret_cast<uint2*>(o + dt * 16) = uint2{pack2_bf16(a[0] * inv, a[1] * inv), pack2_bf16(a[2] * inv, a[3] * inv)};
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) rec[dt * 16 + 4 * G + r] = a[r];
+            }
+        }
+        if (partial_base >= 0 && wave == 0 && G == 0) {
+            rec[HD] = m_all * kLn2;
+            rec[HD + 1] = denom;
+        }
+        return;
+    }
+
+    // ---- several query tiles: the denominator and maximum of every query row; several waves combine inside the
     // workgroup: maxima and sums through LDS, then the waves after the first lay their
     // accumulators, rescaled to the common maximum, into LDS, and the first wave adds them to its
     // own in the fixed order of the waves and writes the result (two barriers, no atomics)
@@ -737,18 +806,29 @@ int launch(const void* q, int64_t q_stride, const void* k_pool, const void* v_po
     const int rows = 16 * NT;
     const int gh = group < rows ? group : rows;
     const int head_chunks = (group + gh - 1) / gh;
-    const dim3 grid(n_items, n_kv * head_chunks);
+    const dim3 grid(n_items, n_kv, head_chunks);
+    scores.group = group;
+    scores.page_magic = magic_of(page_size);
     if (waves < 1) waves = 1;
     if (waves > MAXW) waves = MAXW;
-    // a launch of one wave per workgroup takes the instantiation without the LDS of the
-    // combination, which would otherwise limit how many workgroups a compute unit holds
+    // Several query tiles: a launch of one wave per workgroup takes the instantiation without the LDS of the
+    // combination, which would otherwise limit how many workgroups a compute unit holds.  One: the variant for short items,
+    // or all the waves the kernel has
 #define FSIE_ATTN_LAUNCH(W, THREADS, V)                                                                              \
     attention_mfma_kernel<HDT, NT, W, V><<<grid, THREADS, 0, stream>>>(                                              \
         static_cast<const bf16_t*>(q), q_stride, static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool), \
         block_tables, max_pages, items, static_cast<bf16_t*>(out), partials, n_heads, n_kv, page_size, window, scale, \
-        gh, head_chunks, scores)
+        gh, scores)
     const bool v16 = page_size % 8 == 0;
-    if (waves == 1) {
+    if constexpr (NT == 1) {
+        if (waves == 1) {
+            if (v16) FSIE_ATTN_LAUNCH(kShortWaves, 64 * kShortWaves, true);
+            else FSIE_ATTN_LAUNCH(kShortWaves, 64 * kShortWaves, false);
+        } else {
+            if (v16) FSIE_ATTN_LAUNCH(MAXW, 64 * MAXW, true);
+            else FSIE_ATTN_LAUNCH(MAXW, 64 * MAXW, false);
+        }
+    } else if (waves == 1) {
         if (v16) FSIE_ATTN_LAUNCH(1, 64, true);
         else FSIE_ATTN_LAUNCH(1, 64, false);
     } else {
@@ -768,20 +848,16 @@ int launch_qkv(const QkvSums& f, const void* k_pool, const void* v_pool, const i
     constexpr int MAXW = max_waves<HDT>();
     const int group = n_heads / n_kv;
     const int gh = group < 16 ? group : 16;
-    const int head_chunks = (group + gh - 1) / gh;
-    const dim3 grid(n_items, n_kv * head_chunks);
-    if (waves < 1) waves = 1;
-    if (waves > MAXW) waves = MAXW;
+    const dim3 grid(n_items, n_kv, (group + gh - 1) / gh);
 #define FSIE_ATTN_LAUNCH(W, THREADS)                                                                                 \
     if (f.slopes || f.row_scale) FSIE_ATTN_LAUNCH_AS(W, THREADS, true); else FSIE_ATTN_LAUNCH_AS(W, THREADS, false)
 #define FSIE_ATTN_LAUNCH_AS(W, THREADS, B)                                                                           \
     attention_mfma_kernel<HDT, 1, W, true, true, B><<<grid, THREADS, 0, stream>>>(                                      \
         nullptr, 0, static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool), block_tables, max_pages, \
-        items, static_cast<bf16_t*>(out), partials, n_heads, n_kv, page_size, window, scale, gh, head_chunks, f)
-    // one wave and three that only help with the sums; or all the waves the kernel has (those that an
-    // item's keys leave idle help with the sums too)
-    if (waves == 1) {
-        FSIE_ATTN_LAUNCH(1, 256);
+        items, static_cast<bf16_t*>(out), partials, n_heads, n_kv, page_size, window, scale, gh, f)
+    constexpr int SHORTW = HDT <= 8 ? kShortWaves + 1 : MAXW;
+    if (waves <= 1) {
+        FSIE_ATTN_LAUNCH(SHORTW, 64 * SHORTW);
     } else {
         FSIE_ATTN_LAUNCH(MAXW, 64 * MAXW);
     }

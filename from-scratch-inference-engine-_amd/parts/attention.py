@@ -26,10 +26,9 @@ class AttentionPlanner:
     keys (decoding against a long context) is split over the keys into several items and merged
     afterwards in the order of the splits: 256 keys an item for the float32-arithmetic kernel (128
     or 64 by the same rule as below); for
-    the matrix-core kernel, which gives every 128 keys to a wave of the item's workgroup and
+    the matrix-core kernel, which deals an item's keys to the waves of its workgroup and
     combines those inside, 1,024 keys, or 512, 256 or 128 while that leaves the step with at most
-    as many workgroups as the device has compute units (every wave still sums the same 128 keys;
-    only where their sums meet changes).  Longer portions are cut into *large* tiles of ``large_tokens``; how they are
+    as many workgroups as the device has compute units.  Longer portions are cut into *large* tiles of ``large_tokens``; how they are
     cut depends on the portion alone, never on what else is in the batch.  The item table lists
     the small items first.
 

@@ -748,6 +748,32 @@ def test_attention_over_pages_at_the_lengths_that_are_timed(ops, heads, kv, seqs
         assert max(m[2] for m in plan["merges"]) > (64 if heads == 28 else 40)  # splits of the long decode
 
 
+@pytest.mark.parametrize("heads, kv, hd, page, window", [(14, 2, 64, 16, None), (6, 2, 128, 24, 70), (4, 4, 48, 4, None), (20, 1, 256, 8, None)])
+def test_attention_of_items_by_few_and_by_many_waves(ops, heads, kv, hd, page, window):
+    """The variant for short items (a wave a block of 32 keys) and the one with all the waves the head size allows: the same bits
+    for an item of up to four blocks, and within rounding (probabilities in bfloat16) of the plain one for longer items, which
+    the first walks in runs of several blocks a wave."""
+    from from_scratch_inference_engine_amd.parts.attention import AttentionPlanner
+
+    seqs = [(p, 1) for p in (0, 31, 32, 96, 127, 128, 131, 255, 256, 700, 1023)]
+    AttentionPlanner.compute_units = 8  # whole requests
+    try:
+        case = paged_case(seqs, heads, kv, hd, page, torch.bfloat16, seed=hd, window=window)
+    finally:
+        AttentionPlanner.compute_units = None
+    plan = case["plan"]
+    assert not plan["n_merges"] and plan["n_small"] == len(seqs)
+    many = run_attention(ops, dict(case, plan=dict(plan, waves=16)), heads, kv, hd, window)
+    few = run_attention(ops, dict(case, plan=dict(plan, waves=1)), heads, kv, hd, window)
+    for row, ((p, _), q, k, v) in enumerate(zip(seqs, case["qs"], case["ks"], case["vs"])):
+        ref = plain.attention(q, k, v, heads, kv, hd, query_offset=p, window=window)
+        for out in (many, few):
+            assert (out[row:row + 1] - ref).abs().max() <= 2.0 ** -7 * ref.abs().max(), p
+        first = 0 if window is None else max(0, p - window + 1)
+        if p // 32 - first // 32 < 4:
+            assert torch.equal(many[row], few[row]), p
+
+
 @pytest.mark.parametrize("units", [4096, 8])  # items of 128 keys, one wave each, and a merge; whole requests, up to 8 waves
 @pytest.mark.parametrize("heads, kv, hd, page, window, n_parts, bias", [
     (28, 4, 128, 16, None, 8, True),   # a large model's geometry
