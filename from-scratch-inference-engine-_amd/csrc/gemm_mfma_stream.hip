@@ -52,7 +52,10 @@ struct StreamCall {
 // of W.  blockIdx.y: the slice.  Steps past the slice's end read the last step of K again and are not multiplied; rows of W past
 // the end repeat the last one (a fragment-ordered copy is filled up to whole blocks) and are not written.
 template <int WAVES, int S, int NB, int RESULT, bool FRAGS>
-__global__ __launch_bounds__(WAVES * 64) void gemm_mfma_stream_kernel(const StreamCall c) {
+__global__ __launch_bounds__(WAVES * 64) void gemm_mfma_stream_kernel(const bf16_t* x, const bf16_t* w, void* y, int M, int N, int K,
+                                                                         int slice_steps, int act, float pos, float neg,
+                                                                         const float* bias) {
+    const StreamCall c{x, w, y, M, N, K, slice_steps, act, pos, neg, bias};  // (one by one they come with the launch, a struct would not)
     __shared__ floatx4 red[WAVES * NB * 64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -127,7 +130,8 @@ template <int WAVES, int S, int NB, int RESULT, bool FRAGS>
 int launch(const StreamCall& c, hipStream_t stream) {
     const int blocks = (c.N + 15) / 16;
     const dim3 grid((blocks + NB - 1) / NB, (c.K / 32 + c.slice_steps - 1) / c.slice_steps);
-    gemm_mfma_stream_kernel<WAVES, S, NB, RESULT, FRAGS><<<grid, WAVES * 64, 0, stream>>>(c);
+    gemm_mfma_stream_kernel<WAVES, S, NB, RESULT, FRAGS><<<grid, WAVES * 64, 0, stream>>>(c.x, c.w, c.y, c.M, c.N, c.K, c.slice_steps, c.act,
+                                                                                       c.pos, c.neg, c.bias);
     FSIE_CHECK_LAUNCH("gemm_mfma_stream");
     return 0;
 }

@@ -56,7 +56,13 @@ struct alignas(4 * CPL) Cols {
 
 // ROWS = dim / 16 (key channels a wave), CPL = vdim / 64 (value columns a lane).  grid = (requests, heads)
 template <int ROWS, int CPL>
-__global__ __launch_bounds__(kStepThreads) void gla_step_kernel(const StepCall c) {
+__global__ __launch_bounds__(kStepThreads) void gla_step_kernel(
+    const int32_t* q_starts, const int32_t* seq_slots, const bf16_t* proj, int64_t proj_stride, const bf16_t* a2, float* state,
+    int n_slots, int heads, int rank, int a_off, int q_off, int k_off, int v_off, int g_off, const float* a2_bias,
+    const float* norm, bf16_t* out, float q_scale, float inv_tau, float eps, int act) {
+    // (one by one the first of them come with the launch, a struct would not)
+    const StepCall c{proj, proj_stride, q_off, k_off, v_off, g_off, a_off, rank, a2, a2_bias, state, q_starts, seq_slots,
+                     norm, out, heads, n_slots, q_scale, inv_tau, eps, act};
     constexpr int DIM = 16 * ROWS, VDIM = 64 * CPL;
     typedef Cols<CPL> Vec;
     __shared__ float s_q[DIM], s_k[DIM], s_a[DIM];
@@ -149,7 +155,9 @@ __global__ __launch_bounds__(kStepThreads) void gla_step_kernel(const StepCall c
 
 template <int ROWS, int CPL>
 void launch_step(const StepCall& c, int n_seqs, hipStream_t stream) {
-    gla_step_kernel<ROWS, CPL><<<dim3(n_seqs, c.heads), kStepThreads, 0, stream>>>(c);
+    gla_step_kernel<ROWS, CPL><<<dim3(n_seqs, c.heads), kStepThreads, 0, stream>>>(
+        c.q_starts, c.seq_slots, c.proj, c.proj_stride, c.a2, c.state, c.n_slots, c.heads, c.rank, c.a_off, c.q_off, c.k_off,
+        c.v_off, c.g_off, c.a2_bias, c.norm, c.out, c.q_scale, c.inv_tau, c.eps, c.act);
 }
 
 template <int ROWS>
