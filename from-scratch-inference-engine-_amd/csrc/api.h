@@ -277,6 +277,13 @@ int fsie_attention_scalar(const void* q, int64_t q_stride, const void* k_pool, c
 // Items that leave partial records ignore it; the merge that combines them adds it once.
 int fsie_attention_merge(const float* partials, const int32_t* merges, int n_merges, void* out, int n_heads,
                          int head_dim, int dtype, const float* sinks, hipStream_t stream);
+// The same for float32 storage on the float32 matrix instruction; fsie_attention_scalar goes there where fsie_attention_f32_ok
+// says so and nothing is pooled.
+int fsie_attention_f32_ok(int head_dim, int page_size);
+int fsie_attention_f32(const float* q, int64_t q_stride, const float* k_pool, const float* v_pool, const int32_t* block_tables,
+                       int max_pages, const int32_t* items, int n_items, float* out, float* partials, int n_heads, int n_kv,
+                       int head_dim, int page_size, int window, float scale, const float* sinks, float softcap, const float* slopes,
+                       const float* row_scale, hipStream_t stream);
 int fsie_attention_scalar_tile_tokens(int n_heads, int n_kv);
 // The mean key and value of blocks of `block_tokens` consecutive positions, from the pages of keys and values to the
 // pools of pooled blocks: jobs [n_jobs][2] = (request of the step, block), a request of -1: nothing.  Block b's

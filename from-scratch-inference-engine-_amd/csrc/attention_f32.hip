@@ -1,0 +1,312 @@
+// Causal grouped-query attention over the pages of the cache on the float32 matrix instruction, for float32 storage: products,
+// softmax and sums in float32, no operand rounded.
+//
+// As in the bfloat16 kernel everything is computed transposed, so that no operand changes lanes or passes through LDS:
+//   S^T[key, row] = K[key, :] . Q[row, :]       A = K, B = Q
+//   O^T[d, row]  += V^T[d, key] . P^T[key, row] A = V^T (the cache stores values as [head_dim][slot]), B = P^T
+// v_mfma_f32_16x16x4_f32 takes one value of four reduction indices from each lane (lane = 16 G + c: row c, index G).  Which indices
+// a step of four takes is free as long as both operands agree: step i of a run of sixteen takes 4 G + i, so a lane's four values
+// of a run are neighbours, one 16-byte load.  The first product leaves the scores of the keys 4 G .. 4 G + 3 in a lane, which is
+// the B operand of the second one's four steps over those keys.
+//
+// A workgroup takes an item (a tile of up to 16 query rows, a range of keys) of a kv head; the item's blocks of 16 keys are
+// dealt to its waves in runs of equal length, and the waves' sums meet in LDS, in the order of the waves, behind one barrier.
+// What bounds it is the chain: the item, the block table, keys and values, a trip to memory each, then 32 matrix instructions a
+// block and head of 64 at 32 cycles.  With the merge where items are cut, us, the kernel on the vector units (attention_scalar) /
+// this one: 4 requests of 300 keys, 14 heads on 2 of 64 12.1 / 8.3, 28 on 4 of 128 16.9 / 8.6, 16 on 1 of 256 35.0 / 12.5; one
+// of 100 keys 15.1 / 6.9, 23.1 / 7.7, 54 / 13.8; 32 of 700 20.7 / 15.3, 56 / 26, 48 / 24; a prompt of 300 tokens 49 / 16, 88 / 29,
+// 130 / 37, of 1,000 185 / 59, 537 / 155, 636 / 203.
+#include "common.h"
+#include "api.h"
+
+#include <limits.h>
+#include <math.h>
+
+namespace {
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+constexpr int kFarBelow = INT_MIN / 2;  // below every key
+
+template <int HDT>
+constexpr int f32_waves() {
+    return HDT <= 4 ? 16 : (HDT <= 8 ? 8 : 4);  // registers a wave grow with the head size
+}
+
+struct F32Call {
+    const float *q, *k_pool, *v_pool;
+    int64_t q_stride;
+    const int32_t *block_tables, *items;
+    float *out, *partials;
+    int n_items, max_pages, n_heads, n_kv, page_size, window;
+    float scale, softcap;
+    const float *sinks, *slopes, *row_scale;
+};
+
+template <int HDT>
+__global__ __launch_bounds__(64 * f32_waves<HDT>()) void attention_f32_kernel(
+    const int32_t* __restrict__ items, const int32_t* __restrict__ block_tables, int max_pages, int page_size, uint32_t page_magic,
+    int n_kv, const float* __restrict__ k_pool, const float* __restrict__ v_pool, const float* __restrict__ q, int64_t q_stride,
+    float* __restrict__ out, float* __restrict__ partials, int n_heads, int group, int gh, int window, float scale, float softcap,
+    const float* __restrict__ sinks, const float* __restrict__ slopes, const float* __restrict__ row_scale) {
+    constexpr int HD = HDT * 16, W = f32_waves<HDT>(), MW = (W + 3) / 4 * 4;
+    __shared__ floatx4 s_o[W * HDT * 64];
+    __shared__ float s_m[16][MW + 4], s_l[16][MW + 4];  // [column][wave]: a lane reads its column's waves four at a time
+
+    typedef int ItemInts __attribute__((ext_vector_type(8), aligned(4)));
+    static_assert(FSIE_ATTN_ITEM_INTS == 8, "an item is eight numbers");
+    const ItemInts it = *reinterpret_cast<const ItemInts*>(items + static_cast<int64_t>(blockIdx.x) * FSIE_ATTN_ITEM_INTS);
+    const int seq = it[FSIE_ATTN_ITEM_SEQ], q_row0 = it[FSIE_ATTN_ITEM_QROW], n_q = it[FSIE_ATTN_ITEM_NQ], pos0 = it[FSIE_ATTN_ITEM_POS];
+    const int key_begin = it[FSIE_ATTN_ITEM_KBEGIN], key_end = it[FSIE_ATTN_ITEM_KEND], partial_base = it[FSIE_ATTN_ITEM_PARTIAL];
+    if (n_q <= 0) return;  // padding item
+    // the first keys that a window keeps: seen whatever the window says, and read, as blocks ahead of the item's own
+    // range, where the item is told to
+    const int keep = it[FSIE_ATTN_ITEM_KEEP] & ~(FSIE_ATTN_KEEP_WALK | FSIE_ATTN_POOL_WALK);
+    const int prefix_end = (it[FSIE_ATTN_ITEM_KEEP] & FSIE_ATTN_KEEP_WALK) ? min(keep, key_begin) : 0;
+
+    const int kvh = blockIdx.y, chunk = blockIdx.z;
+    const int gh_here = min(gh, group - chunk * gh), h_base = kvh * group + chunk * gh;
+    const int lane = threadIdx.x & 63, c = lane & 15, G = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int32_t* table = block_tables + static_cast<int64_t>(seq) * max_pages;
+
+    // the blocks, in coordinates that are the keys themselves from kb_first on; those of the kept first keys stand before
+    const int kb_first = key_begin & ~15;
+    const int pre_len = (prefix_end + 15) & ~15;
+    const int walk_first = kb_first - pre_len;
+    const int n_blocks = ((key_end - kb_first + 15) >> 4) + (pre_len >> 4);
+    const int per_wave = (n_blocks + W - 1) / W;
+    const int n_runs = per_wave > 0 ? (n_blocks + per_wave - 1) / per_wave : 1;
+    const int kb_begin = walk_first + wave * per_wave * 16;
+    const int kb_end = min(key_end, kb_begin + per_wave * 16);
+
+    const int64_t head_stride = static_cast<int64_t>(page_size) * HD;
+    const int64_t page_stride = n_kv * head_stride, kv_base = kvh * head_stride;
+    // A key without a page (past the end, or behind a window) is read from page 0 and masked.
+    struct Asked {
+        int k_page, v_page, k_idx, v_idx, k_key, v_key, limit;
+    };
+    auto ask = [&](int kb, Asked& p) {
+        p.limit = kb >= kb_first ? key_end : prefix_end;
+        kb = kb >= kb_first ? kb : kb - walk_first;
+        p.k_key = kb + c, p.v_key = kb + 4 * G;
+        p.k_idx = static_cast<int>(__umulhi(static_cast<uint32_t>(p.k_key), page_magic));
+        p.v_idx = static_cast<int>(__umulhi(static_cast<uint32_t>(p.v_key), page_magic));
+        p.k_page = table[min(p.k_idx, max_pages - 1)];
+        p.v_page = table[min(p.v_idx, max_pages - 1)];
+    };
+    struct Block {
+        floatx4 k[HDT], v[HDT];
+        bool v_ok;  // the keys 4 G .. 4 G + 3 have a page
+    };
+    auto load = [&](const Asked& p, Block& b) {
+        const bool k_ok = (p.k_key < p.limit) & (p.k_idx < max_pages) & (p.k_page >= 0);
+        b.v_ok = (p.v_key < p.limit) & (p.v_idx < max_pages) & (p.v_page >= 0);
+        const float* kp = k_pool + static_cast<uint32_t>(k_ok ? p.k_page : 0) * page_stride + kv_base +
+                          static_cast<uint32_t>((k_ok ? p.k_key - p.k_idx * page_size : 0) * HD + 4 * G);
+        const float* vp = v_pool + static_cast<uint32_t>(b.v_ok ? p.v_page : 0) * page_stride + kv_base +
+                          static_cast<uint32_t>((b.v_ok ? p.v_key - p.v_idx * page_size : 0) + c * page_size);
+#pragma unroll
+        for (int j = 0; j < HDT; ++j) b.k[j] = *reinterpret_cast<const floatx4*>(kp + 16 * j);
+#pragma unroll
+        for (int j = 0; j < HDT; ++j) b.v[j] = *reinterpret_cast<const floatx4*>(vp + static_cast<int64_t>(16 * j) * page_size);
+    };
+
+    const bool any = kb_begin < kb_end;
+    Asked asked;
+    if (any) ask(kb_begin, asked);
+    // this lane's query row; a row that does not exist reads the item's first one and is masked
+    const int tq = c / gh, hh = c - tq * gh;
+    const bool row_ok = tq < n_q && hh < gh_here;
+    const int head = h_base + (row_ok ? hh : 0), row = q_row0 + (row_ok ? tq : 0), pos = pos0 + tq;
+    floatx4 qf[HDT];
+    {
+        const float* qp = q + static_cast<int64_t>(row) * q_stride + static_cast<int64_t>(head) * HD + 4 * G;
+#pragma unroll
+        for (int j = 0; j < HDT; ++j) qf[j] = *reinterpret_cast<const floatx4*>(qp + 16 * j);
+    }
+    const float factor_in = row_scale ? scale * row_scale[row] : scale;
+    const float slope = slopes ? slopes[head] : 0.f;
+
+    float m_run = -INFINITY, l_run = 0.f;
+    floatx4 acc[HDT];
+#pragma unroll
+    for (int j = 0; j < HDT; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    Block b;
+    if (any) load(asked, b);
+    for (int kb = kb_begin; kb < kb_end;) {
+        floatx4 st{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < HDT; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) st = __builtin_amdgcn_mfma_f32_16x16x4f32(b.k[j][i], qf[j][i], st, 0, 0, 0);
+        const bool kept = kb < kb_first;  // a block of the kept first keys (the same for the whole wave)
+        const int of_range = key_end, of_kept = prefix_end;
+        const int range_begin = kept ? 0 : key_begin, range_end = kept ? of_kept : of_range;
+        const int first = (kept ? kb - walk_first : kb) + 4 * G;  // this lane's keys: first .. first + 3
+        const int upto = min(range_end, pos + 1), hi = (row_ok & b.v_ok) ? upto : kFarBelow;
+        const int in_window = pos - window + 1, seen = window > 0 ? in_window : kFarBelow;
+        float s[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            s[i] = st[i] * factor_in;
+            if (softcap > 0.f) s[i] = softcap * tanhf(s[i] / softcap);  // (the same for the whole launch, as the next)
+            if (slopes) s[i] = fmaf(slope, static_cast<float>(first + i - pos), s[i]);
+            const int key = first + i;
+            const bool vis = (key < hi) & (key >= range_begin) & ((key >= seen) | (key < keep));
+            s[i] = vis ? s[i] : -INFINITY;
+        }
+        if (__any(!b.v_ok | (first + 3 >= range_end))) {
+            // values outside the range need not be numbers: they must not meet their probabilities of zero
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bool held = b.v_ok & (first + i < range_end);
+#pragma unroll
+                for (int j = 0; j < HDT; ++j) b.v[j][i] = held ? b.v[j][i] : 0.f;
+            }
+        }
+        const float m_loc = max_xor32(max_xor16(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]))));
+        const float m_new = fmaxf(m_run, m_loc);
+        const float m_of = m_new == -INFINITY ? 0.f : m_new;  // (a row without a key so far: all its probabilities zero)
+        const float corr = m_run == -INFINITY ? 1.f : expf(m_run - m_of);
+        float p[4], p_sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            p[i] = expf(s[i] - m_of);
+            p_sum += p[i];
+        }
+        l_run = l_run * corr + p_sum;  // this lane's keys only; the lane groups are summed at the end
+        m_run = m_new;
+        if (__any(corr != 1.f)) {
+#pragma unroll
+            for (int j = 0; j < HDT; ++j) acc[j] *= corr;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < HDT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(b.v[j][i], p[i], acc[j], 0, 0, 0);
+        kb += 16;
+        if (kb >= kb_end) break;
+        ask(kb, asked);
+        load(asked, b);
+    }
+
+    if (wave < n_runs) {
+#pragma unroll
+        for (int j = 0; j < HDT; ++j) s_o[(wave * HDT + j) * 64 + lane] = acc[j];
+    }
+    const float l_w = sum_xor32(sum_xor16(l_run));
+    if (G == 0) {  // (a wave without keys: minus infinity and zero)
+        s_m[c][wave] = m_run;
+        s_l[c][wave] = l_w;
+    }
+    __syncthreads();
+    if (!row_ok) return;
+    float m_of_run[MW], l_of_run[MW], factor[MW];
+#pragma unroll
+    for (int w = 0; w < MW; w += 4) {
+        const floatx4 m4 = *reinterpret_cast<const floatx4*>(&s_m[c][w]), l4 = *reinterpret_cast<const floatx4*>(&s_l[c][w]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool is = w + i < n_runs;
+            m_of_run[w + i] = is ? m4[i] : -INFINITY;
+            l_of_run[w + i] = is ? l4[i] : 0.f;
+        }
+    }
+    float m_all = m_of_run[0];
+#pragma unroll
+    for (int w = 1; w < W; ++w) m_all = fmaxf(m_all, m_of_run[w]);
+    const float m_of = m_all == -INFINITY ? 0.f : m_all;
+    float denom = 0.f;
+#pragma unroll
+    for (int w = 0; w < MW; ++w) {
+        factor[w] = expf(m_of_run[w] - m_of);
+        denom = fmaf(l_of_run[w], factor[w], denom);
+    }
+    float inv = 1.f;
+    if (partial_base < 0) {
+        // a sink is one more term of the denominator, exp(sink) relative to the maximum; it has no value
+        const float whole = denom + ((sinks && m_all != -INFINITY) ? expf(sinks[head] - m_all) : 0.f);
+        inv = whole > 0.f ? 1.0f / whole : 0.f;
+    }
+    float* o = out + (static_cast<int64_t>(row) * n_heads + head) * HD + 4 * G;
+    // (a cut item's record: unnormalised sums, their maximum and denominator, for attention_merge)
+    float* rec = partials + (static_cast<int64_t>(max(partial_base, 0) + tq) * n_heads + head) * (HD + 2);
+    for (int j = wave; j < HDT; j += W) {
+        floatx4 a{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w0 = 0; w0 < W; w0 += 4) {
+            if (w0 >= n_runs) break;  // (the same for the whole workgroup)
+            floatx4 v[4];  // four at once, past the last run the last one again, not added
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = s_o[(min(w0 + i, n_runs - 1) * HDT + j) * 64 + lane];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) a[r] = w0 + i < n_runs ? fmaf(v[i][r], factor[w0 + i], a[r]) : a[r];
+        }
+        if (partial_base < 0) {
+            *reinterpret_cast<floatx4*>(o + 16 * j) = a * inv;
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) rec[16 * j + 4 * G + r] = a[r];
+        }
+    }
+    if (partial_base >= 0 && wave == 0 && G == 0) {
+        rec[HD] = m_all;
+        rec[HD + 1] = denom;
+    }
+}
+
+template <int HDT>
+int launch(const F32Call& a, hipStream_t stream) {
+    const int group = a.n_heads / a.n_kv, gh = group < 16 ? group : 16;
+    const dim3 grid(a.n_items, a.n_kv, (group + gh - 1) / gh);
+    attention_f32_kernel<HDT><<<grid, 64 * f32_waves<HDT>(), 0, stream>>>(
+        a.items, a.block_tables, a.max_pages, a.page_size, 0xFFFFFFFFu / static_cast<uint32_t>(a.page_size) + 1u, a.n_kv, a.k_pool,
+        a.v_pool, a.q, a.q_stride, a.out, a.partials, a.n_heads, group, gh, a.window, a.scale, a.softcap, a.sinks, a.slopes,
+        a.row_scale);
+    FSIE_CHECK_LAUNCH("attention_f32");
+    return 0;
+}
+
+template <int HDT>
+int launch_from(int hdt, const F32Call& a, hipStream_t stream) {
+    if (hdt == HDT) return launch<HDT>(a, stream);
+    if constexpr (HDT < 16) return launch_from<HDT + 1>(hdt, a, stream);
+    fsie_set_error("attention_f32: no kernel for head_dim %d", 16 * hdt);
+    return 1;
+}
+
+}  // namespace
+
+// Whether fsie_attention_f32 takes these sizes (float32 storage).
+extern "C" int fsie_attention_f32_ok(int head_dim, int page_size) {
+    return head_dim > 0 && head_dim % 16 == 0 && head_dim <= 256 && page_size > 0 && page_size % 4 == 0;
+}
+
+// Attention of float32 queries over float32 pools: items of at most 16 rows (tokens x heads of a group, as
+// fsie_attention_scalar's), records and the other operands as there.  Rows of q, and the pools, on 16 bytes.
+extern "C" int fsie_attention_f32(const float* q, int64_t q_stride, const float* k_pool, const float* v_pool,
+                                  const int32_t* block_tables, int max_pages, const int32_t* items, int n_items, float* out,
+                                  float* partials, int n_heads, int n_kv, int head_dim, int page_size, int window, float scale,
+                                  const float* sinks, float softcap, const float* slopes, const float* row_scale,
+                                  hipStream_t stream) {
+    FSIE_REQUIRE(n_items >= 0 && n_heads > 0 && n_kv > 0 && n_heads % n_kv == 0,
+                 "attention: heads %d must be a positive multiple of kv heads %d", n_heads, n_kv);
+    FSIE_REQUIRE(fsie_attention_f32_ok(head_dim, page_size),
+                 "attention_f32: head_dim %d must be a multiple of 16 up to 256 and page_size %d of 4", head_dim, page_size);
+    FSIE_REQUIRE(max_pages > 0 && (static_cast<int64_t>(max_pages) + 8) * page_size * page_size < (int64_t{1} << 32),
+                 "attention_f32: %d pages of %d keys are more than the kernel can address", max_pages, page_size);
+    FSIE_REQUIRE(q && k_pool && v_pool && block_tables && items && out, "attention_f32: missing operand");
+    FSIE_REQUIRE(q_stride % 4 == 0 && reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 &&
+                     reinterpret_cast<uintptr_t>(v_pool) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0,
+                 "attention_f32: rows of q, the pools and the result must be 16-byte aligned");
+    if (n_items == 0) return 0;
+    F32Call a{};
+    a.q = q, a.k_pool = k_pool, a.v_pool = v_pool, a.q_stride = q_stride, a.block_tables = block_tables, a.items = items;
+    a.out = out, a.partials = partials, a.n_items = n_items, a.max_pages = max_pages, a.n_heads = n_heads, a.n_kv = n_kv;
+    a.page_size = page_size, a.window = window, a.scale = scale, a.softcap = softcap;
+    a.sinks = sinks, a.slopes = slopes, a.row_scale = row_scale;
+    return launch_from<1>(head_dim / 16, a, stream);
+}

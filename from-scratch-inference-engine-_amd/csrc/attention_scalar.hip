@@ -1,6 +1,6 @@
 // Causal grouped-query attention over the pages of the cache: float32 arithmetic throughout
 // (products, softmax, sums), for float32 or bfloat16 storage.  It is the attention of the 32-bit
-// path and takes any head size up to 512 (beyond 256 in an instantiation with twice the accumulators
+// path where the kernel on the matrix instruction (attention_f32.hip) does not take the sizes, and takes any head size up to 512 (beyond 256 in an instantiation with twice the accumulators
 // and more shared memory than a launch gets by default).
 //
 // The host cuts the step into work items (api.h: FSIE_ATTN_ITEM_*): a tile of up to 16/gh query
@@ -558,6 +558,16 @@ extern "C" int fsie_attention_scalar(const void* q, int64_t q_stride, const void
     FSIE_REQUIRE(page_size > 0 && max_pages > 0, "attention: bad page geometry");
     FSIE_REQUIRE(dtype == FSIE_F32 || dtype == FSIE_BF16, "attention: unknown dtype %d", dtype);
     if (n_items == 0) return 0;
+    // float32 storage: the kernel on the matrix instruction where it takes the sizes; this one for the rest (heads of other
+    // sizes and of more than 256, pooled blocks, odd pages and addresses) and for bfloat16 storage in float32 arithmetic
+    if (dtype == FSIE_F32 && !k_pooled && fsie_attention_f32_ok(head_dim, page_size) && q_stride % 4 == 0 &&
+        (static_cast<int64_t>(max_pages) + 8) * page_size * page_size < (int64_t{1} << 32) &&
+        (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pool) | reinterpret_cast<uintptr_t>(v_pool) |
+         reinterpret_cast<uintptr_t>(out)) % 16 == 0)
+        return fsie_attention_f32(static_cast<const float*>(q), q_stride, static_cast<const float*>(k_pool),
+                                  static_cast<const float*>(v_pool), block_tables, max_pages, items, n_items,
+                                  static_cast<float*>(out), partials, n_heads, n_kv, head_dim, page_size, window, scale, sinks,
+                                  softcap, slopes, row_scale, stream);
     const int group = n_heads / n_kv;
     const int gh = group < kRows ? group : kRows;
     const int head_chunks = (group + gh - 1) / gh;

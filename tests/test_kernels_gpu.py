@@ -748,6 +748,37 @@ def test_attention_over_pages_at_the_lengths_that_are_timed(ops, heads, kv, seqs
         assert max(m[2] for m in plan["merges"]) > (64 if heads == 28 else 40)  # splits of the long decode
 
 
+@pytest.mark.parametrize("heads, kv, hd, page, window, units", [(14, 2, 64, 16, None, None), (6, 3, 16, 4, 21, 8), (20, 1, 128, 24, 70, None),
+                                                                (2, 2, 240, 8, None, 8), (3, 1, 256, 64, 300, 4096)])
+def test_attention_on_the_float32_matrix_instruction(ops, heads, kv, hd, page, window, units):
+    """Positions at the edges of the blocks of 16 keys and of the runs that waves take, whole and cut, prompts; values that are
+    no numbers where nothing has been written; and the kernel for other addresses, which gets queries that do not lie on 16 bytes."""
+    from from_scratch_inference_engine_amd.parts.attention import AttentionPlanner
+
+    seqs = [(0, 1), (15, 1), (16, 1), (17, 5), (63, 1), (64, 1), (255, 1), (256, 1), (700, 1), (0, 37), (250, 19)]
+    AttentionPlanner.compute_units = units
+    try:
+        case = paged_case(seqs, heads, kv, hd, page, torch.float32, seed=hd, window=window)
+    finally:
+        AttentionPlanner.compute_units = None
+    case["v_pool"][case["v_pool"] == -9.0] = float("nan")
+    out = run_attention(ops, case, heads, kv, hd, window)
+    row = 0
+    for (p, n), q, k, v in zip(seqs, case["qs"], case["ks"], case["vs"]):
+        ref = plain.attention(q, k, v, heads, kv, hd, query_offset=p, window=window)
+        assert (out[row:row + n] - ref).abs().max() <= 2e-6, (p, n)
+        row += n
+    t, width = case["q"].shape
+    shifted = torch.empty(t * width + 1).cuda()[1:].view(t, width).copy_(case["q"])
+    plan, other = case["plan"], torch.zeros(t, width).cuda()
+    partials = torch.empty(max(plan["n_partial"], 1) * heads * (hd + 2)).cuda()
+    ops.attention_scalar(shifted, width, case["k_pool"].cuda(), case["v_pool"].cuda(), case["tables"].cuda(), torch.from_numpy(plan["items"]).cuda(),
+                         plan["n_small"] + plan["n_large"], other, partials, heads, kv, hd, window, 1.0 / math.sqrt(hd), t)
+    if plan["n_merges"]:
+        ops.attention_merge(partials, torch.from_numpy(plan["merges"]).cuda(), plan["n_merges"], other, heads, hd)
+    assert (other.cpu() - out).abs().max() <= 4e-6
+
+
 @pytest.mark.parametrize("heads, kv, hd, page, window", [(14, 2, 64, 16, None), (6, 2, 128, 24, 70), (4, 4, 48, 4, None), (20, 1, 256, 8, None)])
 def test_attention_of_items_by_few_and_by_many_waves(ops, heads, kv, hd, page, window):
     """The variant for short items (a wave a block of 32 keys) and the one with all the waves the head size allows: the same bits
