@@ -1,4 +1,4 @@
-// The walk over chunks of sixteen tokens that the recurrent mixers share: a state S [dim][vdim] per request and
+// The walk over chunks of sixteen tokens of the matrix memory (mlstm.hip): a state S [dim][vdim] per request and
 // head that every chunk multiplies by a decay per key channel and adds a product of sixteen keys and values to,
 //   o_t   = qd_t^T S_in + sum_{j <= t} A[t][j] v_j,      S_out = diag(g) S_in + sum_j kd_j v_j^T,
 // from a work array that the mixer's own kernel has filled for every chunk and head: qd [16][dp], kd transposed
@@ -40,16 +40,16 @@ __host__ __device__ inline int64_t gla_chunk_floats(int dp) { return static_cast
 // renumbering of the inner index (the tokens 4 g + m at step m) lets v, kdT and A be read in vectors of four.
 // A wave's chain per chunk is nine matrix instructions; the waves' shares of the chunks' o (and the four steps
 // of A v, dealt to the waves in turn) meet in shared memory, a barrier every few chunks, and are added in the
-// order of the waves.  The shares of o that the token-by-token kernel would leave in further planes of `out` are zero here.
+// order of the waves.
 //
-// ONES: the grid has one more tile of columns after the head's last, and that tile carries a single further column
+// The grid has one more tile of columns after the head's last, and that tile carries a single further column
 // of S whose values v are all one: a normaliser n_t = diag(g) n_(t-1) + k_t, with o = q . n.  It lies at
 // `ones_at` floats into the head's record, its channels side by side, and its o goes to ones_out [tokens][heads].
-template <typename T, int NW, bool ONES>
+template <typename T, int NW>
 __global__ __launch_bounds__(64 * NW) void gla_chunk_scan_kernel(
     const T* __restrict__ proj, int64_t proj_stride, int v_off, const float* __restrict__ work,
     float* __restrict__ state, const int32_t* __restrict__ q_starts, const int32_t* __restrict__ seq_slots,
-    float* __restrict__ out, int64_t out_plane, int heads, int dim, int vdim, int dp, int planes, int n_slots,
+    float* __restrict__ out, int heads, int dim, int vdim, int dp, int n_slots,
     int64_t state_head_stride, int64_t ones_at, float* __restrict__ ones_out) {
     constexpr int G = NW <= 8 ? 4 : 2;  // chunks between two barriers: their shares of o lie in LDS side by side
     __shared__ float part[2][G][NW][4][64];
@@ -62,7 +62,7 @@ __global__ __launch_bounds__(64 * NW) void gla_chunk_scan_kernel(
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g4 = lane >> 4;
-    const bool ones_tile = ONES && blockIdx.z == gridDim.z - 1;  // the same for the whole workgroup
+    const bool ones_tile = blockIdx.z == gridDim.z - 1;  // the same for the whole workgroup
     const int col = blockIdx.z * 16 + n;
     const bool col_ok = ones_tile ? n == 0 : col < vdim;
     const int64_t row_stride = ones_tile ? 1 : vdim;
@@ -120,7 +120,7 @@ __global__ __launch_bounds__(64 * NW) void gla_chunk_scan_kernel(
         a4[slot_] = *reinterpret_cast<const floatx4*>(wc + a_at);
     };
     // o of the `count` chunks of group gi (G chunks between two barriers) from the waves' shares, added in the
-    // order of the waves, a value a thread and round.  Further planes of `out`: zeros.
+    // order of the waves, a value a thread and round.
     auto finish = [&](int gi, int count, bool really) {
         const int t0 = lo + gi * G * kGlaChunk;
         float* oc = ones_tile ? ones_out + static_cast<int64_t>(t0) * heads + h
@@ -136,10 +136,7 @@ __global__ __launch_bounds__(64 * NW) void gla_chunk_scan_kernel(
                 for (int ww = 1; ww < NW; ++ww) sum += part[gi & 1][j][ww][i][l];
                 const int tok = j * kGlaChunk + 4 * (l >> 4) + i, c = l & 15;
                 if (really && t0 + tok < hi && (ones_tile ? c == 0 : blockIdx.z * 16 + c < vdim)) {
-                    float* dst = oc + tok * o_stride + c;
-                    *dst = sum;
-                    if (!ones_tile)
-                        for (int pl = 1; pl < planes; ++pl) dst[pl * out_plane] = 0.f;
+                    oc[tok * o_stride + c] = sum;
                 }
             }
         }

@@ -1,0 +1,476 @@
+// Gated linear attention over portions of prompts: chunks of sixteen tokens on the float32 matrix instruction, runs of eight
+// to 32 chunks (segments) side by side.  The recurrence and what a chunk makes of it stand in linear_attention.hip; with B_t the
+// sum of log alpha over the chunk's tokens up to and including t, per channel,
+//   o_t   = (q_t * exp(B_t))^T S_in + sum_{j <= t} A[t][j] v_j,   A[t][j] = sum_c q_t[c] k_j[c] exp(B_t[c] - B_j[c]),
+//   S_out = diag(exp(B_last)) S_in + sum_j (k_j * exp(B_last - B_j)) v_j^T.
+// A first kernel lays the scaled q and k, the chunk's decay and A out for every chunk and head.  The walk over a portion's chunks
+// is a chain, 128 chunks for a prompt of 2,048 tokens; it is cut into segments, in two launches:
+//   1  a portion's first segment, whole, from the request's state; of the segments between first and last what they
+//      make of a state: S_end = diag(G) S_begin + L, with L their walk from zero and G the product of their decays
+//   2  the segments after the first, each from the state that the ones before it leave, L + G (L' + G' (..)), and the last one's end
+//      is the request's state.
+// A wave has sixteen value columns and all key channels of a head: dim / 16 tiles of S in accumulators, whose layout is that
+// of the instruction's second operand if step i of a tile takes the channels 4 g + i (g = 0 .. 3).  A chunk is 68 instructions of
+// 32 cycles for a wave and 128 channels, 0.9 us; its operands, which other dies have written, take some 2 us to come.  So a chunk's
+// record lies in memory as the waves read it and goes straight to LDS, three chunks ahead, for the four waves of a workgroup
+// together.  (In registers, three chunks ahead, the operands are 400 of them a lane and the copies between the two halves of
+// the register file took longer than the products; one ahead, a chunk waited 1.7 us.)
+// Two workgroups share a unit, whose matrix cores are then busy most of the time (a chunk of each 1.6 us).  With the kernel in
+// front and the norm behind, us, one wave per sixteen channels and columns with all chunks in a row / this: 8 heads of 128 x 256,
+// 2,048 tokens 125 / 84, 8,192 507 / 249, eight prompts of 40 to 200 80 / 50, one of 500 49 / 51, of 200 33 / 36; 4 of 64 x 64,
+// 2,048 93 / 39; 4 of 256 x 512 231 / 159.
+#include "common.h"
+#include "api.h"
+#include "log_sigmoid.h"
+
+#include <math.h>
+
+namespace {
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+constexpr int kChunk = 16;     // tokens of a chunk: one tile of the matrix instruction
+constexpr int kLeastSegment = 8;  // chunks of the shortest segment
+
+// Chunks of a segment of a portion of n chunks, by that number alone: the chain is a segment in each launch, and a segment of the
+// second one starts with a pass over the records of those before it.  Up to sixteen chunks one segment: a second launch costs
+// more than the half of the chain that it spares.
+constexpr int kWhole = 16;
+__device__ __forceinline__ int segment_of(int n) { return n <= kWhole ? n : n <= 128 ? kLeastSegment : (n <= 512 ? 16 : 32); }
+constexpr int kPrepThreads = 256;
+
+__device__ __forceinline__ int chunks_of(const int32_t* q_starts, const int32_t* seq_slots, int s, int n_slots) {
+    const int len = q_starts[s + 1] - q_starts[s], slot = seq_slots[s];
+    return (len > 0 && slot >= 0 && slot < n_slots) ? (len + kChunk - 1) / kChunk : 0;
+}
+
+// Work array of one chunk and head, each operand as the lanes 16 g + n of a wave read it, four floats a lane: q * exp(B_t)
+// [channels / 16][g][n][4], the token n and the channels 4 g ..; k * exp(B_last - B_t) [channels / 16][g][n][4], the channel n and the
+// tokens 4 g ..; exp(B_last) [channels]; A (zero above the diagonal) [g][n][4], the token n and the earlier ones 4 g ..; from a
+// multiple of 256 floats on v in float32, [columns / 16][g][n][4], the column n and the tokens 4 g ..
+__host__ __device__ constexpr int operand_floats_of(int dp) { return ((2 * kChunk + 1) * dp + kChunk * kChunk + 255) / 256 * 256; }
+__host__ __device__ inline int64_t chunk_floats_of(int dp, int vdim) { return operand_floats_of(dp) + (vdim + 15) / 16 * 256; }
+__device__ __forceinline__ int a_place(int t, int j) { return ((j >> 2) * 16 + t) * 4 + (j & 3); }
+// ... and of a segment: L as the accumulators lie, and G.
+__host__ __device__ inline int64_t segment_floats_of(int dp, int vdim) { return static_cast<int64_t>(dp) * ((vdim + 15) / 16 * 16) + dp; }
+
+struct ChunksCall {
+    const void *proj, *qk;
+    int64_t proj_stride, qk_stride;
+    int q_off, k_off, v_off;
+    const float* z;
+    float *work, *state, *out;
+    const int32_t *q_starts, *seq_slots;
+    int n_seqs, n_tokens, max_chunks, heads, dim, vdim, n_slots;
+    float q_scale, inv_tau;
+    const float* head_decay;
+    const float2* cos_sin;
+    int pairs;
+    hipStream_t stream;
+};
+
+// grid = (heads, upper bound of the step's chunks): a head's records are written on the die (workgroup number modulo 8) that reads
+// them.  The logarithms are kept to the base two (the hardware's exponential is
+// 2^x).  Every load of a thread goes out before the first is used (the trips one after the other were most of the kernel).  A's
+// pairs below the diagonal are two threads each, the diagonal (exponents of zero) the last sixteen threads.
+template <typename T, int DP>
+__global__ __launch_bounds__(kPrepThreads) void gla_chunk_prep_kernel(
+    const int32_t* __restrict__ q_starts, const int32_t* __restrict__ seq_slots, const T* __restrict__ rows, int64_t row_stride,
+    const float* __restrict__ z, float* __restrict__ work, int n_seqs, int n_slots, int q_off, int k_off, int heads, int dim,
+    const T* __restrict__ v_rows, int64_t v_stride, int vdim, float q_scale, float inv_tau, const float* __restrict__ head_decay, const float2* __restrict__ cos_sin, int pairs) {
+    constexpr int LD = DP + 4, PER = kChunk * DP / kPrepThreads;
+    __shared__ __attribute__((aligned(16))) float qs[kChunk * LD], ks[kChunk * LD], bs[kChunk * LD];
+    const int h = blockIdx.x, chunk = blockIdx.y, tid = threadIdx.x;
+    int first = 0, seq = -1;
+    for (int s = 0; s < n_seqs; ++s) {
+        const int n = chunks_of(q_starts, seq_slots, s, n_slots);
+        if (chunk < first + n) { seq = s; break; }
+        first += n;
+    }
+    if (seq < 0) return;  // the same for the whole workgroup
+    const int t0 = q_starts[seq] + (chunk - first) * kChunk;
+    const int nt = min(kChunk, q_starts[seq + 1] - t0);
+    float* w = work + (static_cast<int64_t>(h) * gridDim.y + chunk) * chunk_floats_of(DP, vdim);
+    float* kdT = w + kChunk * DP;
+    float* g = kdT + kChunk * DP;
+    float* A = g + DP;
+    const float to_log2 = inv_tau * 1.44269504088896340736f;
+
+    float q[PER], k[PER], la[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {  // (places past the portion's end or the head read a neighbour's value and are zeroed below)
+        const int e = tid + i * kPrepThreads, t = t0 + min(e / DP, nt - 1), c = min(e % DP, dim - 1);
+        const T* row = rows + static_cast<int64_t>(t) * row_stride + h * dim + c;
+        q[i] = to_float(row[q_off]);
+        k[i] = to_float(row[k_off]);
+        la[i] = head_decay ? head_decay[h] : z[(static_cast<int64_t>(t) * heads + h) * dim + c];
+    }
+    if (cos_sin) {
+        // the first 2 * pairs channels of a head are turned, channel c with channel c + pairs, by (cos, sin); float32
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int e = tid + i * kPrepThreads, t = t0 + min(e / DP, nt - 1), c = min(e % DP, dim - 1);
+            if (c < 2 * pairs) {
+                const bool low = c < pairs;
+                const T* other = rows + static_cast<int64_t>(t) * row_stride + h * dim + (low ? c + pairs : c - pairs);
+                const float2 turn = cos_sin[static_cast<int64_t>(t) * pairs + (low ? c : c - pairs)];
+                const float qo = to_float(other[q_off]), ko = to_float(other[k_off]);
+                q[i] = low ? fmaf(q[i], turn.x, -(qo * turn.y)) : fmaf(q[i], turn.x, qo * turn.y);
+                k[i] = low ? fmaf(k[i], turn.x, -(ko * turn.y)) : fmaf(k[i], turn.x, ko * turn.y);
+            }
+        }
+    }
+    for (int c = tid; c < (vdim + 15) / 16 * 16; c += kPrepThreads) {  // v, a column a thread
+        const T* from = v_rows + static_cast<int64_t>(t0) * v_stride + h * vdim + min(c, vdim - 1);
+        float v[kChunk];
+#pragma unroll
+        for (int t = 0; t < kChunk; ++t) v[t] = to_float(from[min(t, nt - 1) * v_stride]);
+        floatx4* to = reinterpret_cast<floatx4*>(w + operand_floats_of(DP)) + (c >> 4) * 64 + (c & 15);
+#pragma unroll
+        for (int t = 0; t < kChunk; t += 4) {
+            floatx4 v4;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v4[u] = t + u < nt && c < vdim ? v[t + u] : 0.f;
+            to[t * 4] = v4;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int e = tid + i * kPrepThreads, t = e / DP, c = e % DP;
+        const bool is = t < nt && c < dim;
+        const float log2_alpha = head_decay ? log2f(la[i]) : to_log2 * log_sigmoid(la[i]);
+        qs[t * LD + c] = is ? q[i] * q_scale : 0.f;
+        ks[t * LD + c] = is ? k[i] : 0.f;
+        bs[t * LD + c] = is ? log2_alpha : 0.f;
+    }
+    __syncthreads();
+    if (tid < DP) {
+        float b[kChunk], sum = 0.f;
+#pragma unroll
+        for (int t = 0; t < kChunk; ++t) b[t] = bs[t * LD + tid];
+#pragma unroll
+        for (int t = 0; t < kChunk; ++t) {
+            sum += b[t];
+            bs[t * LD + tid] = sum;
+        }
+        float whole = __builtin_amdgcn_exp2f(sum);
+        if (head_decay && tid < dim) {
+            // a fixed decay: the chunk's decay is its power, by multiplications (it is what the state carries from
+            // chunk to chunk, so its rounding adds up over a long prompt)
+            whole = 1.f;
+            for (int t = 0; t < nt; ++t) whole *= head_decay[h];
+        }
+        g[tid] = whole;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = tid; e < kChunk * DP / 4; e += kPrepThreads) {  // four neighbouring channels of a token
+        const int t = e & 15, c = (e >> 6) * 16 + ((e >> 4) & 3) * 4;
+        const floatx4 q4 = *reinterpret_cast<const floatx4*>(qs + t * LD + c), b4 = *reinterpret_cast<const floatx4*>(bs + t * LD + c);
+        floatx4 v;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = q4[u] * __builtin_amdgcn_exp2f(b4[u]);
+        *reinterpret_cast<floatx4*>(w + 4 * e) = v;
+    }
+#pragma unroll
+    for (int e = tid; e < kChunk * DP / 4; e += kPrepThreads) {  // four neighbouring tokens of a channel
+        const int c = (e >> 6) * 16 + (e & 15), t4 = ((e >> 4) & 3) * 4;
+        const float last = bs[(kChunk - 1) * LD + c];
+        floatx4 v;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = ks[(t4 + u) * LD + c] * __builtin_amdgcn_exp2f(last - bs[(t4 + u) * LD + c]);
+        *reinterpret_cast<floatx4*>(kdT + 4 * e) = v;
+    }
+    if (tid < 240) {
+        // pair p = tid / 2 of the rows and columns i > j, this thread every other four channels
+        const int p = tid >> 1, half = tid & 1;
+        int i = static_cast<int>((1.f + sqrtf(static_cast<float>(1 + 8 * p))) * 0.5f);
+        i = i * (i - 1) / 2 > p ? i - 1 : ((i + 1) * i / 2 <= p ? i + 1 : i);
+        const int j = p - i * (i - 1) / 2;
+        float a = 0.f;
+#pragma unroll 4
+        for (int c = 4 * half; c < DP; c += 8) {  // (channels past dim, tokens past the end: q = k = 0)
+            const floatx4 q4 = *reinterpret_cast<const floatx4*>(qs + i * LD + c), k4 = *reinterpret_cast<const floatx4*>(ks + j * LD + c);
+            const floatx4 x4 = *reinterpret_cast<const floatx4*>(bs + i * LD + c) - *reinterpret_cast<const floatx4*>(bs + j * LD + c);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) a = fmaf(q4[u] * k4[u], __builtin_amdgcn_exp2f(x4[u]), a);
+        }
+        a += lane_of<kLaneNeighbour>(a);
+        if (half == 0) A[a_place(i, j)] = i < nt ? a : 0.f;
+        else A[a_place(j, i)] = 0.f;  // above the diagonal
+    } else {
+        const int i = tid - 240;
+        float a = 0.f;
+#pragma unroll 4
+        for (int c = 0; c < DP; c += 4) {
+            const floatx4 q4 = *reinterpret_cast<const floatx4*>(qs + i * LD + c), k4 = *reinterpret_cast<const floatx4*>(ks + i * LD + c);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) a = fmaf(q4[u], k4[u], a);
+        }
+        A[a_place(i, i)] = i < nt ? a : 0.f;
+    }
+}
+
+// 16 bytes a lane from memory to LDS, lane i's at lds + 16 i.  The instruction takes the LDS address from m0, which is an
+// operand here and written by the compiler; the wait state between that and the load is not, inside an asm statement.
+__device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t lds, uint32_t offset, uint32_t base) {
+    asm volatile(
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, %3 offen lds"
+        :
+        : "{m0}"(lds), "v"(offset), "s"(rsrc), "s"(base)
+        : "memory");
+}
+
+template <int NT>
+struct Stages {
+    static constexpr int kOperands = operand_floats_of(16 * NT) / 256;    // loads of 1 KB (256 floats) of a chunk's record: the operands,
+    static constexpr int kLoads = (kOperands + 4 + 3) / 4;                // v of four tiles; a wave's share (the last ones twice)
+    static constexpr int kFloats = 4 * kLoads * 256;                      // a stage
+    static constexpr int kStages = 3;  // (two workgroups of 72 KB a unit, for heads of 128)
+    static constexpr int kBytes = kStages * kFloats * 4;
+};
+
+// grid = (heads, value columns / 64, upper bound of the launch's segments), a wave sixteen columns: workgroups without a segment come
+// last (one in two among the others, they left half of every die's units to them, and the rest in two rounds).  NT: tiles of sixteen
+// channels.  LATER: the second launch.
+template <int NT, bool LATER>
+__global__ __launch_bounds__(256, NT <= 8 ? 2 : 1) void gla_segment_kernel(
+    const int32_t* __restrict__ q_starts, const int32_t* __restrict__ seq_slots, const float* __restrict__ work, float* segments,
+    float* __restrict__ state, float* __restrict__ out, int n_seqs, int n_slots, int max_chunks, int heads, int dim, int vdim) {
+    constexpr int DP = 16 * NT;
+    using St = Stages<NT>;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int h = blockIdx.x, place = blockIdx.z, lane = threadIdx.x & 63, n = lane & 15, g4 = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tiles = (vdim + 15) / 16, tile0 = static_cast<int>(blockIdx.y) * 4, tile = min(tile0 + wave, tiles - 1);
+    const int col = tile * 16 + n;
+    const bool tile_ok = tile0 + wave < tiles;  // (waves past the last tile repeat it and write nothing)
+    const bool col_ok = tile_ok && col < vdim;
+    // the request and the segment
+    int first = 0, before = 0, seq = -1, seg = 0, n_chunks = 0;
+    for (int s = 0; s < n_seqs; ++s) {
+        const int chunks = chunks_of(q_starts, seq_slots, s, n_slots), len = max(1, segment_of(chunks));
+        const int segs = (chunks + len - 1) / len, here = LATER ? max(0, segs - 1) : (segs > 1 ? segs - 1 : segs);
+        if (place < before + here) {
+            seq = s, seg = place - before + (LATER ? 1 : 0), n_chunks = chunks;
+            break;
+        }
+        before += here, first += chunks;
+    }
+    if (seq < 0) return;  // the same for the whole workgroup
+    const int length = segment_of(n_chunks), begin = seg * length, end = min(n_chunks, begin + length);
+    const bool last = end == n_chunks;
+    const bool whole = LATER || seg == 0;  // o too, not only what the segment makes of a state
+    const int lo = q_starts[seq], hi = q_starts[seq + 1], slot = seq_slots[seq];
+
+    // the chunks' records to LDS: this wave's share of the loads
+    const int64_t per_chunk = chunk_floats_of(DP, vdim);
+    const float* w = work + (static_cast<int64_t>(h) * max_chunks + first) * per_chunk;
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds);
+    uint32_t from[St::kLoads];
+#pragma unroll
+    for (int i = 0; i < St::kLoads; ++i) {
+        const int j = wave * St::kLoads + i;
+        from[i] = (j < St::kOperands ? j : St::kOperands + min(tile0 + j - St::kOperands, tiles - 1)) * 1024u + lane * 16u;
+    }
+    auto bring = [&](int ci) {  // (past the end the last chunk once more)
+        const uint64_t at = reinterpret_cast<uint64_t>(w + min(ci, end - 1) * per_chunk);
+        u32x4 rsrc;
+        rsrc[0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at));
+        rsrc[1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at >> 32));
+        rsrc[2] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(chunk_floats_of(DP, vdim) * 4));
+        rsrc[3] = 0x00020000u;
+        const uint32_t to = lds0 + static_cast<uint32_t>(ci % St::kStages) * (St::kFloats * 4);
+#pragma unroll
+        for (int i = 0; i < St::kLoads; ++i) load_to_lds(rsrc, to + (wave * St::kLoads + i) * 1024u, from[i], 0u);
+    };
+
+    // Segment records: that of the segment that starts at chunk c of the step is number c / 8 (segments that are not a portion's
+    // last are eight chunks and longer, so no two have the same).
+    const int64_t record = segment_floats_of(DP, vdim);
+    const int64_t my_l = (static_cast<int64_t>(tile) * NT * 64 + lane) * 4, my_g = static_cast<int64_t>(tiles) * 16 * DP + 4 * g4;
+    auto record_of = [&](int s) { return segments + (static_cast<int64_t>((first + s * length) / kLeastSegment) * heads + h) * record; };
+    float* my_state = state + (static_cast<int64_t>(slot) * heads + h) * dim * vdim + min(col, vdim - 1);
+    floatx4 S[NT];  // the channels 16 t + 4 g4 + i of the column n
+    if (LATER || !whole) {
+#pragma unroll
+        for (int u = 0; u < St::kStages - 1; ++u) bring(begin + u);
+    }
+    if (!LATER && whole) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) S[t][i] = my_state[static_cast<int64_t>(min(16 * t + 4 * g4 + i, dim - 1)) * vdim];
+        // (every load stands for itself: left to the choice between it and zero, it would move behind it, a branch and a trip each)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(S[t]));
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) S[t][i] = (col_ok && 16 * t + 4 * g4 + i < dim) ? S[t][i] : 0.f;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < St::kStages - 1; ++u) bring(begin + u);
+    } else if (!LATER) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) S[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    } else {
+        const float* r = record_of(0) + my_l;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) S[t] = *reinterpret_cast<const floatx4*>(r + t * 256);
+#pragma unroll 2
+        for (int s = 1; s < seg; ++s) {
+            const float* of = record_of(s);
+            floatx4 l4[NT], d4[NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                l4[t] = *reinterpret_cast<const floatx4*>(of + my_l + t * 256);
+                d4[t] = *reinterpret_cast<const floatx4*>(of + my_g + 16 * t);
+            }
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) S[t][i] = fmaf(d4[t][i], S[t][i], l4[t][i]);
+        }
+    }
+    floatx4 decays[NT];  // of the chunks so far (a segment between first and last)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) decays[t] = floatx4{1.f, 1.f, 1.f, 1.f};
+
+    const int64_t out_stride = static_cast<int64_t>(heads) * vdim;
+    float* mine = out + (lo + 4 * g4) * out_stride + h * vdim + min(col, vdim - 1);
+    for (int ci = begin; ci < end; ++ci) {
+        // All but the youngest kStages - 2 chunks' loads have arrived (stores are counted too: then it is a little more that has)
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(St::kLoads * (St::kStages - 2)) : "memory");
+        bring(ci + St::kStages - 1);  // into the stage that every wave has read before this barrier
+        const float* c = lds + (ci % St::kStages) * St::kFloats;
+        // all of the chunk's operands asked for before the first product
+        floatx4 q4[NT], k4[NT], g[NT], a4{0.f, 0.f, 0.f, 0.f};
+        const floatx4 v4 = *reinterpret_cast<const floatx4*>(c + St::kOperands * 256 + wave * 256 + 4 * lane);
+        if (whole) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) q4[t] = *reinterpret_cast<const floatx4*>(c + t * 256 + 4 * lane);
+            a4 = *reinterpret_cast<const floatx4*>(c + (2 * kChunk + 1) * DP + 4 * lane);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            g[t] = *reinterpret_cast<const floatx4*>(c + 2 * kChunk * DP + 16 * t + 4 * g4);
+            k4[t] = *reinterpret_cast<const floatx4*>(c + kChunk * DP + t * 256 + 4 * lane);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (whole) {
+            floatx4 o[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};  // two sums that do not wait for each other
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(q4[t][i], S[t][i], o[i & 1], 0, 0, 0);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) o[m & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[m], v4[m], o[m & 1], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) S[t] *= g[t];
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[t][m], v4[m], S[t], 0, 0, 0);
+            const floatx4 sum = o[0] + o[1];
+            float* to = mine + ci * kChunk * out_stride;
+            const int left = hi - lo - ci * kChunk - 4 * g4;  // tokens from this lane's first on
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (col_ok && i < left) to[i * out_stride] = sum[i];
+        } else {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) S[t] *= g[t], decays[t] *= g[t];
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) S[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[t][m], v4[m], S[t], 0, 0, 0);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (no load may still write LDS when the workgroup's is given away)
+    if (!tile_ok) return;
+    if (last) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = 16 * t + 4 * g4 + i;
+                if (col_ok && row < dim) my_state[static_cast<int64_t>(row) * vdim] = S[t][i];
+            }
+    } else if (!LATER) {
+        float* of = record_of(seg);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) *reinterpret_cast<floatx4*>(of + my_l + t * 256) = S[t];
+        if (!whole && tile == 0 && n == 0) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) *reinterpret_cast<floatx4*>(of + my_g + 16 * t) = decays[t];
+        }
+    }
+}
+
+template <int NT, bool LATER>
+int launch_segments(const ChunksCall& c, int n) {
+    constexpr int bytes = Stages<NT>::kBytes;
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gla_segment_kernel<NT, LATER>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    FSIE_REQUIRE(allowed == hipSuccess, "gla_scan: %d bytes of LDS: %s", bytes, hipGetErrorString(allowed));
+    gla_segment_kernel<NT, LATER><<<dim3(c.heads, (c.vdim + 63) / 64, n), 256, bytes, c.stream>>>(
+        c.q_starts, c.seq_slots, c.work, c.work + c.max_chunks * chunk_floats_of(16 * NT, c.vdim) * c.heads, c.state, c.out, c.n_seqs,
+        c.n_slots, c.max_chunks, c.heads, c.dim, c.vdim);
+    return 0;
+}
+
+template <typename T, int NT>
+int launch(const ChunksCall& c) {
+    constexpr int DP = 16 * NT;
+    const T* rows = static_cast<const T*>(c.qk ? c.qk : c.proj);
+    gla_chunk_prep_kernel<T, DP><<<dim3(c.heads, c.max_chunks), kPrepThreads, 0, c.stream>>>(
+        c.q_starts, c.seq_slots, rows, c.qk ? c.qk_stride : c.proj_stride, c.z, c.work, c.n_seqs, c.n_slots, c.q_off, c.k_off, c.heads,
+        c.dim, static_cast<const T*>(c.proj) + c.v_off, c.proj_stride, c.vdim, c.q_scale, c.inv_tau, c.head_decay, c.cos_sin, c.pairs);
+    // segments that are not a portion's last are eight chunks and longer: at most max_chunks / 8 of them, and none where no
+    // portion can have more than sixteen chunks
+    const int inner = c.n_tokens > kWhole * kChunk ? c.max_chunks / kLeastSegment : 0;
+    int status = launch_segments<NT, false>(c, c.n_seqs + inner);
+    if (status == 0 && inner > 0) status = launch_segments<NT, true>(c, inner);
+    if (status) return status;
+    FSIE_CHECK_LAUNCH("gla_chunks");
+    return 0;
+}
+
+template <typename T>
+int launch_dim(const ChunksCall& c) {
+    if (c.dim <= 16) return launch<T, 1>(c);
+    if (c.dim <= 32) return launch<T, 2>(c);
+    if (c.dim <= 64) return launch<T, 4>(c);
+    if (c.dim <= 128) return launch<T, 8>(c);
+    return launch<T, 16>(c);
+}
+
+}  // namespace
+
+// Floats of work that a chunk of sixteen tokens needs for a layer of these sizes, its share of the segments' records included.
+extern "C" int64_t fsie_gla_chunk_floats(int heads, int dim, int vdim) {
+    int dp = 16;
+    while (dp < dim) dp *= 2;
+    return heads * chunk_floats_of(dp, vdim) + (heads * segment_floats_of(dp, vdim) + kLeastSegment - 1) / kLeastSegment;
+}
+
+// All portions of the step, chunk by chunk, for fsie_gla_scan (which has checked the operands): work has room for max_chunks
+// chunks, out is [n_tokens][heads * vdim].
+extern "C" int fsie_gla_chunks(const void* proj, int64_t proj_stride, int q_off, int k_off, int v_off, const float* z, float* state,
+                               const int32_t* q_starts, const int32_t* seq_slots, int n_seqs, int n_tokens, float* out, float* work,
+                               int max_chunks, int heads, int dim, int vdim, float q_scale, float inv_tau, int n_slots, int dtype,
+                               const float* head_decay, const void* qk, int64_t qk_stride, const float* cos_sin, int rot_pairs,
+                               hipStream_t stream) {
+    FSIE_REQUIRE(max_chunks >= n_tokens / kChunk + n_seqs, "gla_scan: room for %d chunks, the step may have %d", max_chunks,
+                 n_tokens / kChunk + n_seqs);
+    FSIE_REQUIRE(n_seqs <= 65535 && heads <= 65535 && (vdim + 63) / 64 <= 65535, "gla_scan: too many requests, heads or columns");
+    FSIE_REQUIRE(reinterpret_cast<uintptr_t>(work) % 16 == 0 && dim <= 256, "gla_scan: the work array must be 16-byte aligned");
+    const ChunksCall c{proj, qk, proj_stride, qk_stride, q_off, k_off, v_off, z, work, state, out, q_starts, seq_slots, n_seqs,
+                       n_tokens, n_tokens / kChunk + n_seqs, heads, dim, vdim, n_slots, q_scale, inv_tau, head_decay,
+                       rot_pairs > 0 ? reinterpret_cast<const float2*>(cos_sin) : nullptr, rot_pairs, stream};
+    return dtype == FSIE_F32 ? launch_dim<float>(c) : launch_dim<bf16_t>(c);
+}

@@ -14,21 +14,10 @@
 // padding with decay 1 and k = q = 0), and the walk reads them with addresses that are uniform over the
 // wave, which the compiler turns into scalar loads: no lane-wide traffic for them at all.
 //
-// A portion of kGlaChunkMin tokens or more does not walk token by token.  It is cut into chunks of sixteen
-// tokens (counted from the portion's first token), and with B_t the sum of log alpha over the chunk's tokens
-// up to and including t, per channel,
-//   o_t   = (q_t * exp(B_t))^T S_in + sum_{j <= t} A[t][j] v_j,   A[t][j] = sum_c q_t[c] k_j[c] exp(B_t[c] - B_j[c]),
-//   S_out = diag(exp(B_last)) S_in + sum_j (k_j * exp(B_last - B_j)) v_j^T,
-// which is the same recurrence with its sums taken in another order: every exponent is a sum of logarithms of
-// decays, none is positive, nothing can overflow whatever the decays are.  A first kernel computes the scaled
-// q and k, the chunk's decay and A for every chunk and head at once (float32 on the vector units); the walk
-// over chunks then is three small matrix products a chunk on the float32 matrix instruction
-// (v_mfma_f32_16x16x4_f32, no rounding of operands), one wave per sixteen key channels and sixteen value
-// columns with its tile of S in an accumulator; the waves of a head's columns meet every few chunks to add
-// their shares of o.
+// A step with a portion of a prompt does not walk token by token: gla_chunks.hip takes it, chunk by chunk on the matrix
+// instruction (the same recurrence with its sums in another order).
 #include "common.h"
 #include "api.h"
-#include "chunk_scan_impl.h"
 #include "log_sigmoid.h"
 
 #include <math.h>
@@ -39,8 +28,12 @@ constexpr int kGlaWaves = 16;
 constexpr int kGlaThreads = 64 * kGlaWaves;
 constexpr int kGlaCols = 64;
 constexpr int kGlaTokens = 8;  // tokens whose shares of o are added up at once
-constexpr int kGlaChunkThreads = 256;
+constexpr int kGlaChunk = 16;     // tokens of a chunk
+constexpr int kGlaChunkMin = 16;  // steps of fewer tokens walk token by token
 
+// A workgroup barrier that waits for this wave's shared-memory traffic only: __syncthreads also waits for its loads and stores
+// of global memory, and the walk has both in flight at every barrier.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Channel i of a head's q or k (x points at it), turned by the token's angles where a rotation is given: the first
 // 2 * pairs channels of a head rotate, channel i with channel i + pairs, by cs[i mod pairs] = (cos, sin); float32.
@@ -54,20 +47,12 @@ __device__ __forceinline__ float turned_channel(const T* __restrict__ x, int i, 
     return low ? fmaf(a, t.x, -(b * t.y)) : fmaf(a, t.x, b * t.y);
 }
 
-// prep [3][tokens][heads][dp]: scaled q, k, decay.  Grid: blocks of 256 elements over all tokens of the step,
-// or (with short_only > 0) over the first tokens of every request (grid.y), and only for requests of at most
-// short_only tokens: the others go chunk by chunk and need none of this.
+// prep [3][tokens][heads][dp]: scaled q, k, decay.  Grid: blocks of 256 elements over all tokens of the step.
 template <typename T>
 __global__ void gla_prep_kernel(const T* __restrict__ proj, int64_t proj_stride, int q_off, int k_off,
                                 const float* __restrict__ z, float* __restrict__ prep, int64_t total, int heads, int dim,
-                                int dp, float q_scale, float inv_tau, const int32_t* __restrict__ q_starts, int short_only,
-                                const float* __restrict__ head_decay, const float2* __restrict__ cos_sin, int pairs) {
-    int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (short_only > 0) {
-        const int lo = q_starts[blockIdx.y], len = q_starts[blockIdx.y + 1] - lo;
-        if (len > short_only || e >= static_cast<int64_t>(len) * heads * dp) return;
-        e += static_cast<int64_t>(lo) * heads * dp;
-    }
+                                int dp, float q_scale, float inv_tau, const float* __restrict__ head_decay, const float2* __restrict__ cos_sin, int pairs) {
+    const int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (e >= total) return;
     const int i = static_cast<int>(e % dp);
     const int64_t th = e / dp;
@@ -92,8 +77,7 @@ template <typename T, int ROWS>
 __global__ __launch_bounds__(kGlaThreads) void gla_scan_kernel(
     const T* __restrict__ proj, int64_t proj_stride, int v_off, const float* __restrict__ prep, int64_t prep_plane,
     float* __restrict__ state, const int32_t* __restrict__ q_starts, const int32_t* __restrict__ seq_slots,
-    float* __restrict__ out, int64_t out_plane, int heads, int dim, int vdim, int dp, int row_splits, int n_slots,
-    int skip_from) {
+    float* __restrict__ out, int64_t out_plane, int heads, int dim, int vdim, int dp, int row_splits, int n_slots) {
     constexpr int TT = kGlaTokens;
     __shared__ float part[kGlaWaves][TT][kGlaCols];
     const int seq = blockIdx.x, h = blockIdx.y;
@@ -104,7 +88,6 @@ __global__ __launch_bounds__(kGlaThreads) void gla_scan_kernel(
     const int lo = q_starts[seq], hi = q_starts[seq + 1];
     const int slot = seq_slots[seq];
     if (hi <= lo || slot < 0 || slot >= n_slots) return;  // the same for the whole workgroup
-    if (hi - lo >= skip_from) return;                     // the chunk kernels' portion
     const bool col_ok = col < vdim;
     const int row0 = (split * kGlaWaves + wave) * ROWS;  // this wave's first key channel
 
@@ -159,111 +142,6 @@ __global__ __launch_bounds__(kGlaThreads) void gla_scan_kernel(
     }
 }
 
-// The chunks of a step are numbered request by request, in the order of the requests; a request whose portion
-// is shorter than kGlaChunkMin, or that has no slot, has none.  (A handful of scalar loads per workgroup.)
-// grid = (upper bound of the step's chunks, heads).  The logarithms are kept to the base two (the hardware's
-// exponential is 2^x).  Every (token, channel) of the chunk is one thread's in the loads and in the stores; only
-// the running sums over the chunk's tokens are a thread a channel.  A's pairs (j <= i) are dealt to the first
-// 136 threads, row i together with row 15 - i, so that no wave carries the empty half of the square.
-template <typename T>
-__global__ __launch_bounds__(kGlaChunkThreads) void gla_chunk_prep_kernel(
-    const T* __restrict__ proj, int64_t proj_stride, int q_off, int k_off, const float* __restrict__ z,
-    float* __restrict__ work, const int32_t* __restrict__ q_starts, const int32_t* __restrict__ seq_slots, int n_seqs,
-    int heads, int dim, int dp, float q_scale, float inv_tau, int n_slots, const float* __restrict__ head_decay,
-    const float2* __restrict__ cos_sin, int pairs) {
-    extern __shared__ float lds[];  // [3][16][dp + 4]: q, k, B
-    const int ld = dp + 4;
-    float* qs = lds;
-    float* ks = qs + kGlaChunk * ld;
-    float* bs = ks + kGlaChunk * ld;
-    const int h = blockIdx.y, tid = threadIdx.x;
-    int first = 0, seq = -1;
-    for (int s = 0; s < n_seqs; ++s) {
-        const int n = gla_chunks_of(q_starts, seq_slots, s, n_slots);
-        if (static_cast<int>(blockIdx.x) < first + n) { seq = s; break; }
-        first += n;
-    }
-    if (seq < 0) return;  // the same for the whole workgroup
-    const int t0 = q_starts[seq] + (static_cast<int>(blockIdx.x) - first) * kGlaChunk;
-    const int nt = min(kGlaChunk, q_starts[seq + 1] - t0);
-    float* w = work + (static_cast<int64_t>(blockIdx.x) * heads + h) * gla_chunk_floats(dp);
-    float* qd = w;
-    float* kdT = qd + kGlaChunk * dp;
-    float* g = kdT + kGlaChunk * dp;
-    float* A = g + dp;
-    const float to_log2 = inv_tau * 1.44269504088896340736f;
-
-    for (int e = tid; e < kGlaChunk * dp; e += kGlaChunkThreads) {
-        const int t = e / dp, c = e - t * dp;
-        float q = 0.f, k = 0.f, la = 0.f;
-        if (t < nt && c < dim) {
-            const T* row = proj + static_cast<int64_t>(t0 + t) * proj_stride + h * dim + c;
-            const float2* cs = cos_sin ? cos_sin + static_cast<int64_t>(t0 + t) * pairs : nullptr;
-            q = turned_channel(row + q_off, c, pairs, cs) * q_scale;
-            k = turned_channel(row + k_off, c, pairs, cs);
-            la = head_decay ? log2f(head_decay[h])
-                            : to_log2 * log_sigmoid(z[(static_cast<int64_t>(t0 + t) * heads + h) * dim + c]);
-        }
-        qs[t * ld + c] = q;
-        ks[t * ld + c] = k;
-        bs[t * ld + c] = la;
-    }
-    __syncthreads();
-    for (int c = tid; c < dp; c += kGlaChunkThreads) {
-        float sum = 0.f;
-#pragma unroll
-        for (int t = 0; t < kGlaChunk; ++t) {
-            sum += bs[t * ld + c];
-            bs[t * ld + c] = sum;
-        }
-        float whole = __builtin_amdgcn_exp2f(sum);
-        if (head_decay && c < dim) {
-            // a fixed decay: the chunk's decay is its power, by multiplications (it is what the state carries from
-            // chunk to chunk, so its rounding adds up over a long prompt)
-            whole = 1.f;
-            for (int t = 0; t < nt; ++t) whole *= head_decay[h];
-        }
-        g[c] = whole;
-    }
-    __syncthreads();
-    for (int e = tid; e < kGlaChunk * dp; e += kGlaChunkThreads) {
-        const int t = e / dp, c = e - t * dp;
-        qd[e] = qs[t * ld + c] * __builtin_amdgcn_exp2f(bs[t * ld + c]);
-    }
-    for (int e = tid; e < dp * (kGlaChunk / 4); e += kGlaChunkThreads) {
-        const int c = e >> 2, t4 = (e & 3) * 4;
-        const float last = bs[(kGlaChunk - 1) * ld + c];
-        floatx4 kd;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) kd[i] = ks[(t4 + i) * ld + c] * __builtin_amdgcn_exp2f(last - bs[(t4 + i) * ld + c]);
-        *reinterpret_cast<floatx4*>(kdT + c * kGlaChunk + t4) = kd;
-    }
-    // A: thread p < 136 has the pair number p of the rows (r, 15 - r) put side by side, r = p / 17
-    if (tid < kGlaChunk * (kGlaChunk + 1) / 2) {
-        const int r = tid / (kGlaChunk + 1), o = tid - r * (kGlaChunk + 1);
-        const int i = o <= r ? r : kGlaChunk - 1 - r;
-        const int j = o <= r ? o : o - r - 1;
-        float a = 0.f;
-        if (i < nt) {
-            const float* qi = qs + i * ld;
-            const float* kj = ks + j * ld;
-            const float* bi = bs + i * ld;
-            const float* bj = bs + j * ld;
-            for (int c = 0; c < dp; c += 4) {  // (channels past dim: q = k = 0)
-                const floatx4 q4 = *reinterpret_cast<const floatx4*>(qi + c), k4 = *reinterpret_cast<const floatx4*>(kj + c);
-                const floatx4 x4 = *reinterpret_cast<const floatx4*>(bi + c) - *reinterpret_cast<const floatx4*>(bj + c);
-#pragma unroll
-                for (int u = 0; u < 4; ++u) a = fmaf(q4[u] * k4[u], __builtin_amdgcn_exp2f(x4[u]), a);
-            }
-        }
-        A[i * kGlaChunk + j] = a;
-    }
-    // above the diagonal: zeros
-    for (int e = tid; e < kGlaChunk * kGlaChunk; e += kGlaChunkThreads) {
-        if ((e & 15) > (e >> 4)) A[e] = 0.f;
-    }
-}
-
 // Key channels a wave holds and the splits of a head's channels over workgroups: as many splits (1, 2, 4)
 // as still leave a wave four channels, while the workgroups of one request number fewer than 128.  A
 // function of the layer's sizes alone, never of the step.
@@ -281,8 +159,8 @@ void gla_shape(int heads, int dim, int vdim, int* rows, int* splits) {
 }  // namespace
 
 // Sizes of the work arrays of fsie_gla_scan for a layer of these sizes: floats of `prep` a token, the planes
-// of `out` (row splits), and for the portions that go chunk by chunk the tokens of a chunk, the shortest such
-// portion and the floats of `chunk_work` a chunk.  A step of n_tokens tokens in n_seqs requests has at most
+// of `out` (row splits), and for the steps that go chunk by chunk the tokens of a chunk, the least tokens of such a
+// step and the floats of `chunk_work` a chunk.  A step of n_tokens tokens in n_seqs requests has at most
 // n_tokens / chunk_tokens + n_seqs chunks, and none if n_tokens < chunk_min.
 extern "C" int fsie_gla_scan_shape(int heads, int dim, int vdim, int* prep_floats_per_token, int* out_planes,
                                    int* chunk_tokens, int* chunk_min, int64_t* chunk_floats) {
@@ -293,7 +171,7 @@ extern "C" int fsie_gla_scan_shape(int heads, int dim, int vdim, int* prep_float
     *out_planes = splits;
     *chunk_tokens = kGlaChunk;
     *chunk_min = kGlaChunkMin;
-    *chunk_floats = gla_chunk_floats(kGlaWaves * splits * rows) * heads;
+    *chunk_floats = fsie_gla_chunk_floats(heads, dim, vdim);
     return 0;
 }
 
@@ -303,10 +181,9 @@ extern "C" int fsie_gla_scan_shape(int heads, int dim, int vdim, int* prep_float
 // q_starts[s] .. q_starts[s + 1] and the slot seq_slots[s] (a slot outside the table: the request is
 // skipped).  q is multiplied by q_scale; alpha = sigmoid(z)^inv_tau.  prep: work array of n_tokens *
 // prep_floats_per_token floats; out: out_planes arrays [n_tokens][heads * vdim] float32 whose sum, in order,
-// is o (fsie_gla_scan_shape gives both numbers).  chunk_work: room for max_chunks chunks, or null: with it, the
-// portions of at least chunk_min tokens go chunk by chunk (max_chunks must be the bound that fsie_gla_scan_shape
-// names, or more); without it every portion is walked token by token.  Which way a portion goes depends on
-// its own length alone, and the two ways differ by rounding only.
+// is o (fsie_gla_scan_shape gives both numbers).  chunk_work: room for max_chunks chunks, or null: with it every portion of
+// the step goes chunk by chunk, prep is not used and out is one array (max_chunks must be the bound that fsie_gla_scan_shape
+// names, or more); without it every portion is walked token by token.  The two ways differ by rounding only.
 extern "C" int fsie_gla_scan(const void* proj, int64_t proj_stride, int q_off, int k_off, int v_off, const float* z,
                              float* state, const int32_t* q_starts, const int32_t* seq_slots, int n_seqs, int n_tokens,
                              float* prep, float* out, float* chunk_work, int max_chunks, int heads, int dim, int vdim,
@@ -324,67 +201,37 @@ extern "C" int fsie_gla_scan(const void* proj, int64_t proj_stride, int q_off, i
     FSIE_REQUIRE(n_seqs >= 0 && n_tokens >= 0 && heads > 0 && dim > 0 && vdim > 0 && n_slots > 0, "gla_scan: bad sizes");
     FSIE_REQUIRE(dim <= 256, "gla_scan: %d key channels a head are more than the kernel takes (256)", dim);
     FSIE_REQUIRE(dtype == FSIE_F32 || dtype == FSIE_BF16, "gla_scan: unknown dtype %d", dtype);
-    FSIE_REQUIRE(proj && (z || head_decay) && state && q_starts && seq_slots && out && prep, "gla_scan: missing operand");
+    FSIE_REQUIRE(proj && (z || head_decay) && state && q_starts && seq_slots && out && (prep || chunk_work), "gla_scan: missing operand");
     FSIE_REQUIRE(q_off >= 0 && k_off >= 0 && v_off >= 0 && (qk || (q_off + heads * dim <= proj_stride &&
                      k_off + heads * dim <= proj_stride)) && v_off + heads * vdim <= proj_stride,
                  "gla_scan: the q, k and v columns do not fit a row of %lld", static_cast<long long>(proj_stride));
     if (n_seqs == 0 || n_tokens == 0) return 0;
+    if (chunk_work)
+        return fsie_gla_chunks(proj, proj_stride, q_off, k_off, v_off, z, state, q_starts, seq_slots, n_seqs, n_tokens, out, chunk_work,
+                               max_chunks, heads, dim, vdim, q_scale, inv_tau, n_slots, dtype, head_decay, qk, qk_stride, cos_sin,
+                               rot_pairs, stream);
     int rows, splits;
     gla_shape(heads, dim, vdim, &rows, &splits);
     const int dp = kGlaWaves * splits * rows;
     const int col_blocks = (vdim + kGlaCols - 1) / kGlaCols;
-    FSIE_REQUIRE(heads <= 65535 && col_blocks * splits <= 65535 && (vdim + 15) / 16 <= 65535, "gla_scan: too many heads or columns");
+    FSIE_REQUIRE(heads <= 65535 && col_blocks * splits <= 65535, "gla_scan: too many heads or columns");
     const int64_t plane = static_cast<int64_t>(n_tokens) * heads * dp;
     const int64_t out_plane = static_cast<int64_t>(n_tokens) * heads * vdim;
     const dim3 grid(n_seqs, heads, col_blocks * splits);
-    const bool chunks = chunk_work != nullptr && n_tokens >= kGlaChunkMin;
-    if (chunks) {
-        FSIE_REQUIRE(max_chunks >= n_tokens / kGlaChunk + n_seqs, "gla_scan: room for %d chunks, the step may have %d",
-                     max_chunks, n_tokens / kGlaChunk + n_seqs);
-        FSIE_REQUIRE(max_chunks <= 0x7fffffff / kGlaChunk, "gla_scan: too many chunks");
-        FSIE_REQUIRE(proj_stride <= 0x7fffffff / kGlaChunk && qk_step <= 0x7fffffff / kGlaChunk && static_cast<int64_t>(heads) * vdim <= 0x7fffffff / kGlaChunk,
-                     "gla_scan: rows too long for the chunk kernels' 32-bit offsets");
-    }
-    const int skip_from = chunks ? kGlaChunkMin : 0x7fffffff;
-    // with the chunk kernels at work only portions below their length are walked: their first tokens, request by request
-    const int short_only = chunks ? kGlaChunkMin - 1 : 0;
-    const dim3 prep_grid(static_cast<unsigned>(chunks ? ceil_div64(static_cast<int64_t>(short_only) * heads * dp, 256)
-                                                      : ceil_div64(plane, 256)),
-                         chunks ? n_seqs : 1);
-    FSIE_REQUIRE(n_seqs <= 65535 || !chunks, "gla_scan: too many requests");
-    const dim3 chunk_grid(chunks ? max_chunks : 1, heads);
-    const size_t chunk_lds = 3 * kGlaChunk * (dp + 4) * sizeof(float);
-    const dim3 scan_grid(n_seqs, heads, (vdim + 15) / 16);
-    int scan_waves = 1;  // a wave for every sixteen key channels, rounded up to a power of two: at most sixteen
-    while (scan_waves * 16 < dim) scan_waves *= 2;
-#define FSIE_GLA_CHUNKS(T, NW)                                                                                        \
-    gla_chunk_scan_kernel<T, NW, false><<<scan_grid, 64 * NW, 0, stream>>>(static_cast<const T*>(proj), proj_stride, v_off,    \
-                                                                    chunk_work, state, q_starts, seq_slots, out,        \
-                                                                    out_plane, heads, dim, vdim, dp, splits, n_slots,           \
-                                                                    static_cast<int64_t>(dim) * vdim, 0, nullptr)
+    const dim3 prep_grid(static_cast<unsigned>(ceil_div64(plane, 256)));
 #define FSIE_GLA_LAUNCH(T, ROWS)                                                                                       \
     gla_scan_kernel<T, ROWS><<<grid, kGlaThreads, 0, stream>>>(static_cast<const T*>(proj), proj_stride, v_off, prep, plane, \
                                                                state, q_starts, seq_slots, out, out_plane, heads, dim, vdim, \
-                                                               dp, splits, n_slots, skip_from)
+                                                               dp, splits, n_slots)
 #define FSIE_GLA_BY_ROWS(T)                                                                                          \
     gla_prep_kernel<T><<<prep_grid, 256, 0, stream>>>(static_cast<const T*>(qk_rows), qk_step, q_off, k_off, z, prep, \
-                                                      plane, heads, dim, dp, q_scale, inv_tau, q_starts, short_only, head_decay,  \
+                                                      plane, heads, dim, dp, q_scale, inv_tau, head_decay,  \
                                                       turn, rot_pairs);                                              \
     if (rows == 1) FSIE_GLA_LAUNCH(T, 1);                                                                            \
     else if (rows == 2) FSIE_GLA_LAUNCH(T, 2);                                                                       \
     else if (rows == 4) FSIE_GLA_LAUNCH(T, 4);                                                                       \
     else if (rows == 8) FSIE_GLA_LAUNCH(T, 8);                                                                       \
-    else FSIE_GLA_LAUNCH(T, 16);                                                                                     \
-    if (chunks) {                                                                                                    \
-        gla_chunk_prep_kernel<T><<<chunk_grid, kGlaChunkThreads, chunk_lds, stream>>>(                                \
-            static_cast<const T*>(qk_rows), qk_step, q_off, k_off, z, chunk_work, q_starts, seq_slots, n_seqs, heads, dim, \
-            dp, q_scale, inv_tau, n_slots, head_decay, turn, rot_pairs);                                             \
-        if (scan_waves == 1) FSIE_GLA_CHUNKS(T, 1);                                                                  \
-        else if (scan_waves == 2) FSIE_GLA_CHUNKS(T, 2);                                                             \
-        else if (scan_waves == 4) FSIE_GLA_CHUNKS(T, 4);                                                             \
-        else if (scan_waves == 8) FSIE_GLA_CHUNKS(T, 8);                                                             \
-        else FSIE_GLA_CHUNKS(T, 16);                                                                                 \
-    }
+    else FSIE_GLA_LAUNCH(T, 16)
     if (dtype == FSIE_F32) {
         FSIE_GLA_BY_ROWS(float);
     } else {
@@ -392,7 +239,6 @@ extern "C" int fsie_gla_scan(const void* proj, int64_t proj_stride, int q_off, i
     }
 #undef FSIE_GLA_BY_ROWS
 #undef FSIE_GLA_LAUNCH
-#undef FSIE_GLA_CHUNKS
     FSIE_CHECK_LAUNCH("gla_scan");
     return 0;
 }

@@ -391,15 +391,14 @@ extern "C" int fsie_mlstm_scan(const void* proj, int64_t stride, int q_off, int 
     const int dp = 16 * scan_waves;
     const dim3 prep_grid(chunks ? max_chunks : 1, heads);
     const size_t prep_lds = 2 * kGlaChunk * (dp + 4) * sizeof(float);
-    const int64_t out_plane = static_cast<int64_t>(n_tokens) * heads * vdim;
 #define FSIE_MLSTM(T, NI, Q)                                                                                              \
     mlstm_scan_kernel<T, NI, Q><<<grid, 64, 0, stream>>>(static_cast<const T*>(proj), stride, q_off, k_off, v_off, q_scale, state, \
                                                       record, n_slots, q_starts, seq_slots, heads, dim, vdim, coef, num, den, \
                                                       col_tiles, skip_from)
 #define FSIE_MLSTM_CHUNKS(T, NW)                                                                                       \
-    gla_chunk_scan_kernel<T, NW, true><<<chunk_grid, 64 * NW, 0, stream>>>(static_cast<const T*>(proj), stride, v_off, chunk_work,    \
-                                                                     state, q_starts, seq_slots, num, out_plane, heads, dim,   \
-                                                                     vdim, dp, 1, n_slots, record, n_at, den)
+    gla_chunk_scan_kernel<T, NW><<<chunk_grid, 64 * NW, 0, stream>>>(static_cast<const T*>(proj), stride, v_off, chunk_work,    \
+                                                                     state, q_starts, seq_slots, num, heads, dim, vdim, dp,    \
+                                                                     n_slots, record, n_at, den)
 #define FSIE_MLSTM_T(T)                                                                                                \
     if (groups == 4 && per_lane <= 8) FSIE_MLSTM(T, 8, 4);                                                             \
     else if (groups == 4 && per_lane <= 16) FSIE_MLSTM(T, 16, 4);                                                      \

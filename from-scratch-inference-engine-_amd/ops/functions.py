@@ -1225,9 +1225,9 @@ def gla_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, z: torch.Te
     q, k (heads x dim) and v (heads x vdim) columns from ``q_off``, ``k_off``, ``v_off``; ``z`` float32
     [T, heads * dim]; ``q_starts`` int32 [n + 1], ``seq_slots`` int32 [n].  Returns o float32 [P, T, heads * vdim]:
     the shares of the P groups of key channels that the kernel deals a head's state to (P follows from the
-    sizes alone); their sum in order is o, and ``gated_headnorm`` takes them as they are.  Long portions are
-    computed chunk by chunk on the matrix cores (the same sums in another order); ``chunked=False`` walks
-    every portion token by token."""
+    sizes, and is one in steps that go chunk by chunk); their sum in order is o, and ``gated_headnorm`` takes them as they are.
+    Steps with portions of prompts are computed chunk by chunk on the matrix cores (the same sums in another order);
+    ``chunked=False`` walks every portion token by token."""
     _need(proj, "gla proj", ndim=2)
     t, w = proj.shape
     if head_decay is not None:
@@ -1260,11 +1260,11 @@ def gla_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, z: torch.Te
     chunk_floats = ctypes.c_int64(0)
     check(load().fsie_gla_scan_shape(heads, dim, vdim, ctypes.byref(per_token), ctypes.byref(planes),
                                      ctypes.byref(chunk_tokens), ctypes.byref(chunk_min), ctypes.byref(chunk_floats)))
-    prep = torch.empty((t * per_token.value,), dtype=torch.float32, device=proj.device)
-    out = torch.empty((planes.value, t, heads * vdim), dtype=torch.float32, device=proj.device)
     # a step of single tokens (t == n, as every captured decode step is) has no portion to cut into chunks
     max_chunks = t // chunk_tokens.value + n if chunked and t > n and t >= chunk_min.value else 0
     work = torch.empty((max_chunks * chunk_floats.value,), dtype=torch.float32, device=proj.device) if max_chunks else None
+    prep = torch.empty((0 if max_chunks else t * per_token.value,), dtype=torch.float32, device=proj.device)
+    out = torch.empty((1 if max_chunks else planes.value, t, heads * vdim), dtype=torch.float32, device=proj.device)
     check(load().fsie_gla_scan(proj.data_ptr(), w, q_off, k_off, v_off, _ptr(z), state.data_ptr(), q_starts.data_ptr(),
                                seq_slots.data_ptr(), n, t, prep.data_ptr(), out.data_ptr(),
                                work.data_ptr() if work is not None else None, max_chunks, heads, dim, vdim, float(q_scale),

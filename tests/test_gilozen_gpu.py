@@ -225,6 +225,30 @@ def test_gla_scan_chunk_by_chunk_and_token_by_token(ops, dtype, heads, dim, vdim
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("heads, dim, vdim", [(2, 128, 72), (3, 16, 16), (1, 200, 40)])
+def test_gla_scan_in_segments(ops, dtype, heads, dim, vdim):
+    """Portions of one chunk, of sixteen (the longest that is one segment), of a token more, of segments of eight and of sixteen
+    chunks, whole and not, side by side and continued: against the walk token by token, from the same states."""
+    lens = [1, 256, 257, 384, 2049, 700, 16]
+    kw, vw = heads * dim, heads * vdim
+    slots = torch.tensor([5, 0, 3, 1, 4, 2, 6], dtype=torch.int32).cuda()
+    states = [rnd((8, heads, dim, vdim), 9).cuda() for _ in range(2)]
+    for step in range(2):
+        mine = lens if step == 0 else lens[::-1]
+        t = sum(mine)
+        proj, z = rnd((t, 2 * kw + vw), 60 + step).to(dtype).cuda(), rnd((t, kw), 70 + step, 4.0)
+        z.view(t, heads, dim)[:, :, 0::3] = 25.0   # keeps everything
+        z.view(t, heads, dim)[:, :, 1::5] = -60.0  # keeps nothing
+        starts = torch.from_numpy(np.cumsum([0] + mine).astype(np.int32)).cuda()
+        outs = [ops.gla_scan(proj, 0, kw, 2 * kw, z.cuda(), state, starts, slots, heads, dim, vdim, dim ** -0.5, 0.5, chunked=chunked).sum(0)
+                for state, chunked in zip(states, (True, False))]
+        for lo, hi in zip(starts.tolist(), starts.tolist()[1:]):
+            assert rel(outs[0][lo:hi].cpu(), outs[1][lo:hi].double().cpu()) <= 2e-5, (step, hi - lo)
+        assert rel(states[0].cpu(), states[1].double().cpu()) <= 2e-5
+    assert torch.equal(states[0][7].cpu(), rnd((8, heads, dim, vdim), 9)[7])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_latent_prep_rope_pairs_and_head_gemm(ops, dtype):
     heads, q_rank, kv_rank, rot_dim, pairs, page, t = 3, 40, 52, 12, 4, 8, 11
     width = 64
