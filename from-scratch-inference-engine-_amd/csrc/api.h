@@ -203,6 +203,8 @@ int fsie_gemm_mfma_fp32_sums(const float* x, const float* w, float* y, int M, in
 // The same for any number of rows (prompts); splits > 1: y = partial sums [splits][M][N] of slices of K, no bias.
 int fsie_gemm_fp32_tile(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int splits,
                         hipStream_t stream);
+int fsie_gemm_fp32_gated(const float* x, const float* w, float* y, int M, int N, int K, int act, float limit, float slope,
+                         hipStream_t stream);
 
 int fsie_gemm_mfma_skinny(const void* x, const void* w, const float* bias, void* y, int M, int N, int K,
                           int out_f32, int waves, int blocks, int epilogue, int splits, hipStream_t stream);

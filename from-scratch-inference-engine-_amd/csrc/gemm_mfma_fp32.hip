@@ -15,13 +15,20 @@ namespace {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// What stands in the place of the plain sums: the rows of W are gate and up in turn and y is [M, N / 2], their product of
+// values (gate_pair), without bias.  As a pass of its own behind the product it was 4.5 us a layer and step of few rows.
+struct Gate {
+    int act;
+    float limit, slope;
+};
+
 // MT tiles of 16 rows of X; WAVES waves split K in steps of 16 values (4 per lane group), U steps in flight.
-template <int MT, int WAVES>
+template <int MT, int WAVES, bool GATED>
 __global__ __launch_bounds__(WAVES * FSIE_WAVE) void gemm_mfma_fp32_kernel(const float* __restrict__ x,
                                                                           const float* __restrict__ w,
                                                                           const float* __restrict__ bias,
                                                                           float* __restrict__ y, int M, int N, int K,
-                                                                          int slice_steps) {
+                                                                          int slice_steps, Gate gate) {
     constexpr int U = MT >= 3 ? 2 : 4;
     __shared__ float red[WAVES > 1 ? (WAVES - 1) * MT * FSIE_WAVE * 4 : 1];
     const int lane = threadIdx.x & (FSIE_WAVE - 1);
@@ -103,6 +110,14 @@ __global__ __launch_bounds__(WAVES * FSIE_WAVE) void gemm_mfma_fp32_kernel(const
     for (int t = 0; t < MT; ++t) {
         const int m = t * 16 + row;
         if (m >= M) continue;
+        if constexpr (GATED) {
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+                const int nn = n0 + kg * 4 + r;
+                if (nn < N) y[static_cast<int64_t>(m) * (N / 2) + nn / 2] = gate_pair(acc[t][r], acc[t][r + 1], gate.act, gate.limit, gate.slope);
+            }
+            continue;
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int nn = n0 + kg * 4 + r;
@@ -111,16 +126,16 @@ __global__ __launch_bounds__(WAVES * FSIE_WAVE) void gemm_mfma_fp32_kernel(const
     }
 }
 
-template <int MT>
-int launch_mt(int waves, const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int splits,
+template <int MT, bool GATED>
+int launch_mt(int waves, const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int splits, Gate gate,
               hipStream_t stream) {
     const int steps = (K + 15) / 16, slice = (steps + splits - 1) / splits;
     const dim3 groups(static_cast<unsigned>((N + 15) / 16), static_cast<unsigned>(splits));
     switch (waves) {
-        case 1: gemm_mfma_fp32_kernel<MT, 1><<<groups, 64, 0, stream>>>(x, w, bias, y, M, N, K, slice); break;
-        case 2: gemm_mfma_fp32_kernel<MT, 2><<<groups, 128, 0, stream>>>(x, w, bias, y, M, N, K, slice); break;
-        case 4: gemm_mfma_fp32_kernel<MT, 4><<<groups, 256, 0, stream>>>(x, w, bias, y, M, N, K, slice); break;
-        default: gemm_mfma_fp32_kernel<MT, 8><<<groups, 512, 0, stream>>>(x, w, bias, y, M, N, K, slice); break;
+        case 1: gemm_mfma_fp32_kernel<MT, 1, GATED><<<groups, 64, 0, stream>>>(x, w, bias, y, M, N, K, slice, gate); break;
+        case 2: gemm_mfma_fp32_kernel<MT, 2, GATED><<<groups, 128, 0, stream>>>(x, w, bias, y, M, N, K, slice, gate); break;
+        case 4: gemm_mfma_fp32_kernel<MT, 4, GATED><<<groups, 256, 0, stream>>>(x, w, bias, y, M, N, K, slice, gate); break;
+        default: gemm_mfma_fp32_kernel<MT, 8, GATED><<<groups, 512, 0, stream>>>(x, w, bias, y, M, N, K, slice, gate); break;
     }
     FSIE_CHECK_LAUNCH("gemm_mfma_fp32");
     return 0;
@@ -138,10 +153,12 @@ int launch_mt(int waves, const float* x, const float* w, const float* bias, floa
 // 211 -> 136 at 682 x 9728 x 896, and in seven slices 822 -> 77 at 682 x 896 x 4864.
 constexpr int kTileEdge = 64, kTileK = 32, kTileFlush = 256;
 
-template <bool SUMS>
+enum Whole { PLAIN = 0, SUMS = 1, GATED = 2 };
+
+template <int RESULT>
 __global__ __launch_bounds__(256) void gemm_fp32_tile_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                             const float* __restrict__ bias, float* __restrict__ y, int M,
-                                                            int N, int K, int k_slice) {
+                                                            int N, int K, int k_slice, Gate gate) {
     __shared__ float4 lds[2][2][kTileEdge][kTileK / 4];
     const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
     const int n0 = blockIdx.x * kTileEdge, m0 = blockIdx.y * kTileEdge;
@@ -212,14 +229,21 @@ __global__ __launch_bounds__(256) void gemm_fp32_tile_kernel(const float* __rest
     for (int t = 0; t < 2; ++t) {
         const int m = m0 + mw + 16 * t + row;
         if (m >= M) continue;
-        float* to = y + ((SUMS ? static_cast<int64_t>(blockIdx.z) * M : 0) + m) * N;
+        float* to = RESULT == GATED ? y + static_cast<int64_t>(m) * (N / 2)
+                                    : y + ((RESULT == SUMS ? static_cast<int64_t>(blockIdx.z) * M : 0) + m) * N;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int n = n0 + nw + 16 * j + 4 * kg;
             const floatx4 v = acc[j][t] + total[j][t];
+            if constexpr (RESULT == GATED) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (n + i < N) to[n + i] = !SUMS && bias ? v[i] + bias[n + i] : v[i];
+                for (int i = 0; i < 4; i += 2)
+                    if (n + i < N) to[(n + i) / 2] = gate_pair(v[i], v[i + 1], gate.act, gate.limit, gate.slope);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (n + i < N) to[n + i] = RESULT == PLAIN && bias ? v[i] + bias[n + i] : v[i];
+            }
         }
     }
 }
@@ -228,8 +252,8 @@ __global__ __launch_bounds__(256) void gemm_fp32_tile_kernel(const float* __rest
 
 // float32 operands and result, any number of rows, K a multiple of 4, x and w 16-byte aligned.  splits > 1: y holds
 // that many partial sums [splits][M][N] of slices of K, without bias.
-extern "C" int fsie_gemm_fp32_tile(const float* x, const float* w, const float* bias, float* y, int M, int N, int K,
-                                   int splits, hipStream_t stream) {
+static int tile_product(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int splits,
+                        const Gate* gate, hipStream_t stream) {
     FSIE_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_fp32_tile: bad sizes M=%d N=%d K=%d", M, N, K);
     FSIE_REQUIRE(K % 4 == 0, "gemm_fp32_tile: K=%d must be a multiple of 4", K);
     FSIE_REQUIRE(splits >= 1 && splits <= 64 && (splits == 1 || !bias), "gemm_fp32_tile: %d slices", splits);
@@ -244,18 +268,25 @@ extern "C" int fsie_gemm_fp32_tile(const float* x, const float* w, const float* 
     FSIE_REQUIRE(splits == 1 || slice * (splits - 1) < K, "gemm_fp32_tile: K=%d does not give %d slices", K, splits);
     const dim3 grid(static_cast<unsigned>((N + kTileEdge - 1) / kTileEdge), static_cast<unsigned>(tiles_m), static_cast<unsigned>(splits));
     if (splits > 1)
-        gemm_fp32_tile_kernel<true><<<grid, 256, 0, stream>>>(x, w, nullptr, y, M, N, K, static_cast<int>(slice));
+        gemm_fp32_tile_kernel<SUMS><<<grid, 256, 0, stream>>>(x, w, nullptr, y, M, N, K, static_cast<int>(slice), Gate{});
+    else if (gate)
+        gemm_fp32_tile_kernel<GATED><<<grid, 256, 0, stream>>>(x, w, nullptr, y, M, N, K, static_cast<int>(ceil_div64(K, kTileK) * kTileK), *gate);
     else
-        gemm_fp32_tile_kernel<false><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K, static_cast<int>(ceil_div64(K, kTileK) * kTileK));
+        gemm_fp32_tile_kernel<PLAIN><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K, static_cast<int>(ceil_div64(K, kTileK) * kTileK), Gate{});
     FSIE_CHECK_LAUNCH("gemm_fp32_tile");
     return 0;
+}
+
+extern "C" int fsie_gemm_fp32_tile(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int splits,
+                                   hipStream_t stream) {
+    return tile_product(x, w, bias, y, M, N, K, splits, nullptr, stream);
 }
 
 // float32 operands and result.  1 <= M <= 64, K a multiple of 4, x and w 16-byte aligned.
 // waves: 1, 2, 4 or 8 waves of a workgroup split K; 0 = choose.  splits > 1: y = partial sums [splits][M][N] of slices of K,
 // no bias.
 static int few_rows(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int waves, int splits,
-                    hipStream_t stream) {
+                    const Gate* gate, hipStream_t stream) {
     FSIE_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_mfma_fp32: bad sizes M=%d N=%d K=%d", M, N, K);
     FSIE_REQUIRE(M <= FSIE_GEMM_MFMA_SKINNY_MAX_M, "gemm_mfma_fp32: at most %d rows, got %d",
                  FSIE_GEMM_MFMA_SKINNY_MAX_M, M);
@@ -278,19 +309,34 @@ static int few_rows(const float* x, const float* w, const float* bias, float* y,
         while (waves > 1 && steps / splits < 4 * waves) waves /= 2;
     }
     switch ((M + 15) / 16) {
-        case 1: return launch_mt<1>(waves, x, w, bias, y, M, N, K, splits, stream);
-        case 2: return launch_mt<2>(waves, x, w, bias, y, M, N, K, splits, stream);
-        case 3: return launch_mt<3>(waves, x, w, bias, y, M, N, K, splits, stream);
-        default: return launch_mt<4>(waves, x, w, bias, y, M, N, K, splits, stream);
+        case 1: return gate ? launch_mt<1, true>(waves, x, w, bias, y, M, N, K, splits, *gate, stream)
+                             : launch_mt<1, false>(waves, x, w, bias, y, M, N, K, splits, Gate{}, stream);
+        case 2: return gate ? launch_mt<2, true>(waves, x, w, bias, y, M, N, K, splits, *gate, stream)
+                             : launch_mt<2, false>(waves, x, w, bias, y, M, N, K, splits, Gate{}, stream);
+        case 3: return gate ? launch_mt<3, true>(waves, x, w, bias, y, M, N, K, splits, *gate, stream)
+                             : launch_mt<3, false>(waves, x, w, bias, y, M, N, K, splits, Gate{}, stream);
+        default: return gate ? launch_mt<4, true>(waves, x, w, bias, y, M, N, K, splits, *gate, stream)
+                             : launch_mt<4, false>(waves, x, w, bias, y, M, N, K, splits, Gate{}, stream);
     }
 }
 
 extern "C" int fsie_gemm_mfma_fp32(const float* x, const float* w, const float* bias, float* y, int M, int N, int K,
                                    int waves, hipStream_t stream) {
-    return few_rows(x, w, bias, y, M, N, K, waves, 1, stream);
+    return few_rows(x, w, bias, y, M, N, K, waves, 1, nullptr, stream);
 }
 
 extern "C" int fsie_gemm_mfma_fp32_sums(const float* x, const float* w, float* y, int M, int N, int K, int splits,
                                         hipStream_t stream) {
-    return few_rows(x, w, nullptr, y, M, N, K, 0, splits, stream);
+    return few_rows(x, w, nullptr, y, M, N, K, 0, splits, nullptr, stream);
+}
+
+// The rows of w are gate and up in turn (N even): y [M, N / 2] is their product of values, act a FsieGateAct or FsieGatePair
+// with its limit and slope.  Any number of rows; otherwise as the two products above, whose bits its sums have.
+extern "C" int fsie_gemm_fp32_gated(const float* x, const float* w, float* y, int M, int N, int K, int act, float limit, float slope,
+                                    hipStream_t stream) {
+    FSIE_REQUIRE(N % 2 == 0, "gemm_fp32_gated: N=%d rows of gate and up in turn", N);
+    FSIE_REQUIRE(FSIE_PAIR_KNOWN(act), "gemm_fp32_gated: unknown activation %d", act);
+    const Gate gate{act, limit, slope};
+    return M <= FSIE_GEMM_MFMA_SKINNY_MAX_M ? few_rows(x, w, nullptr, y, M, N, K, 0, 1, &gate, stream)
+                                            : tile_product(x, w, nullptr, y, M, N, K, 1, &gate, stream);
 }

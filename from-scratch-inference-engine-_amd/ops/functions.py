@@ -458,6 +458,20 @@ def gemm_fp32_tile(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     return out
 
 
+def gemm_fp32_gated(x: torch.Tensor, weight: torch.Tensor, act="silu") -> torch.Tensor:
+    """act(gate) * up (``act``: a ``GateAct`` or its name) [M, N/2] in true float32 of x [M, K] and a weight [N, K] whose rows are
+    gate and up in turn, N even, K a multiple of 4: ``gemm_mfma_fp32`` up to 64 rows, beyond them ``gemm_fp32_tile``."""
+    _need(x, "gemm x", dtype=torch.float32, ndim=2)
+    _need(weight, "gemm weight", dtype=torch.float32, ndim=2)
+    m, k = x.shape
+    n = weight.shape[0]
+    if weight.shape[1] != k:
+        raise KernelError(f"gemm: weight inner size {weight.shape[1]} does not match x's {k}")
+    out = torch.empty((m, n // 2), dtype=torch.float32, device=x.device)
+    check(load().fsie_gemm_fp32_gated(x.data_ptr(), weight.data_ptr(), out.data_ptr(), m, n, k, *gate_act(act).args, _stream()))
+    return out
+
+
 _FP32_TILE_ROWS = 512  # rows of a prompt's step that the slices below are made for
 
 

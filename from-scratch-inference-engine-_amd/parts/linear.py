@@ -85,6 +85,11 @@ class Linear:
         w = self._weight
         return x.is_contiguous() and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
 
+    def takes_f32_matrix(self, x: torch.Tensor) -> bool:
+        """Whether a whole float32 product of these rows runs on the matrix cores."""
+        return (self.float32_on_matrix_cores and x.shape[0] > 2 and self.in_features % 4 == 0
+                and (x.shape[0] <= GEMM_MFMA_SKINNY_MAX_M or self.kernel_reads(x)))
+
     def drop_copy(self) -> int:
         """Forget the fragment-ordered copy (the products then read rows); returns its bytes."""
         if self.streamed is None:

@@ -79,6 +79,8 @@ class SwiGLU(FeedForward):
             act = ops.gemm_mfma_wide_swiglu(x, self.gate_up.weight, act=self._gate_act)
         elif x.dtype == torch.bfloat16 and m <= GEMM_MFMA_SKINNY_BEST_M and self.hidden_size % 8 == 0:
             act = ops.gemm_mfma_skinny_gated(x, self.gate_up.weight, self._gate_act)
+        elif x.dtype == torch.float32 and self.gate_up.takes_f32_matrix(x):
+            act = ops.gemm_fp32_gated(x, self.gate_up.weight, self._gate_act)
         else:
             # prompts: where its tiles fill the chip, the product for many rows with act(gate) * up in its epilogue
             plan = (ops.gemm_tile_plan(m, self.gate_up.out_features, self.hidden_size, ops.GEMM_TILE_PAIR)

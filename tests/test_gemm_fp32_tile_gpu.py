@@ -58,3 +58,15 @@ def test_slices_of_few_rows_are_never_empty():
     for k in list(range(4, 1200, 4)) + [4864, 8192, 18944]:
         slices, steps = ops.gemm_mfma_fp32_splits(k), -(-k // 16)
         assert 1 <= slices <= 8 and -(-steps // slices) * (slices - 1) < steps
+
+
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("m, n, k", [(3, 34, 100), (4, 9728, 896), (16, 18, 2052), (17, 64, 300), (33, 130, 512), (64, 66, 1000), (65, 34, 260),
+                                     (200, 130, 36)])
+def test_gate_and_up_multiplied_in_the_epilogue(m, n, k, act):
+    """The same bits as the product and the pass that multiplies, at the edges of the tiles of rows and of blocks of W."""
+    ops.load(build_if_missing=False)
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn((m, k), generator=g).cuda(), torch.randn((n, k), generator=g).cuda()
+    product = ops.gemm_mfma_fp32(x, w) if m <= 64 else ops.gemm_fp32_tile(x, w)
+    assert torch.equal(ops.gemm_fp32_gated(x, w, act), ops.swiglu(product, act=act))
