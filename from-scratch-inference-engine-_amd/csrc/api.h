@@ -96,14 +96,14 @@ int fsie_gla_scan(const void* proj, int64_t proj_stride, int q_off, int k_off, i
                   const int32_t* q_starts, const int32_t* seq_slots, int n_seqs, int n_tokens, float* prep, float* out,
                   float* chunk_work, int max_chunks, int heads, int dim, int vdim, float q_scale, float inv_tau,
                   int n_slots, int dtype, const float* head_decay, const void* qk, int64_t qk_stride, const float* cos_sin,
-                  int rot_pairs, hipStream_t stream);
+                  int rot_pairs, const void* a, int64_t a_stride, const void* a2, const float* a2_bias, int rank, hipStream_t stream);
 // Its steps that go chunk by chunk (gla_chunks.hip).
 int64_t fsie_gla_chunk_floats(int heads, int dim, int vdim);
 int fsie_gla_chunks(const void* proj, int64_t proj_stride, int q_off, int k_off, int v_off, const float* z, float* state,
                     const int32_t* q_starts, const int32_t* seq_slots, int n_seqs, int n_tokens, float* out, float* work,
                     int max_chunks, int heads, int dim, int vdim, float q_scale, float inv_tau, int n_slots, int dtype,
                     const float* head_decay, const void* qk, int64_t qk_stride, const float* cos_sin, int rot_pairs,
-                    hipStream_t stream);
+                    const void* a, int64_t a_stride, const void* a2, const float* a2_bias, int rank, hipStream_t stream);
 // The same for a step of one token a request (bfloat16), with what stands before and behind it: the decays' second product (the
 // bottleneck's values stand in proj too), the norm of every head's o and its gate.
 int fsie_gla_step_takes(int heads, int dim, int vdim, int rank);

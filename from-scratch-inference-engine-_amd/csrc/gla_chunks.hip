@@ -30,6 +30,7 @@ namespace {
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kChunk = 16;     // tokens of a chunk: one tile of the matrix instruction
 constexpr int kLeastSegment = 8;  // chunks of the shortest segment
@@ -56,6 +57,17 @@ __device__ __forceinline__ int a_place(int t, int j) { return ((j >> 2) * 16 + t
 // ... and of a segment: L as the accumulators lie, and G.
 __host__ __device__ inline int64_t segment_floats_of(int dp, int vdim) { return static_cast<int64_t>(dp) * ((vdim + 15) / 16 * 16) + dp; }
 
+// Where the decays come from a bottleneck (bfloat16), z = W_a2 a + b: the chunk's own kernel multiplies, 16 tokens by a head's channels
+// by rank, where a product of its own and z in memory were 36 us a
+// layer of a prompt of 2,048 tokens (eager, the launch included).  a2 null: z is given.
+struct Bottleneck {
+    const bf16_t* a;      // [n_tokens][a_stride]
+    const bf16_t* a2;     // [heads * dim][rank], rank a multiple of 32
+    const float* bias;    // [heads * dim]
+    int64_t a_stride;
+    int rank;
+};
+
 struct ChunksCall {
     const void *proj, *qk;
     int64_t proj_stride, qk_stride;
@@ -68,6 +80,7 @@ struct ChunksCall {
     const float* head_decay;
     const float2* cos_sin;
     int pairs;
+    Bottleneck from;
     hipStream_t stream;
 };
 
@@ -79,7 +92,7 @@ template <typename T, int DP>
 __global__ __launch_bounds__(kPrepThreads) void gla_chunk_prep_kernel(
     const int32_t* __restrict__ q_starts, const int32_t* __restrict__ seq_slots, const T* __restrict__ rows, int64_t row_stride,
     const float* __restrict__ z, float* __restrict__ work, int n_seqs, int n_slots, int q_off, int k_off, int heads, int dim,
-    const T* __restrict__ v_rows, int64_t v_stride, int vdim, float q_scale, float inv_tau, const float* __restrict__ head_decay, const float2* __restrict__ cos_sin, int pairs) {
+    const T* __restrict__ v_rows, int64_t v_stride, int vdim, float q_scale, float inv_tau, const float* __restrict__ head_decay, const float2* __restrict__ cos_sin, int pairs, Bottleneck from) {
     constexpr int LD = DP + 4, PER = kChunk * DP / kPrepThreads;
     __shared__ __attribute__((aligned(16))) float qs[kChunk * LD], ks[kChunk * LD], bs[kChunk * LD];
     const int h = blockIdx.x, chunk = blockIdx.y, tid = threadIdx.x;
@@ -105,7 +118,28 @@ __global__ __launch_bounds__(kPrepThreads) void gla_chunk_prep_kernel(
         const T* row = rows + static_cast<int64_t>(t) * row_stride + h * dim + c;
         q[i] = to_float(row[q_off]);
         k[i] = to_float(row[k_off]);
-        la[i] = head_decay ? head_decay[h] : z[(static_cast<int64_t>(t) * heads + h) * dim + c];
+        la[i] = head_decay ? head_decay[h] : from.a2 ? 0.f : z[(static_cast<int64_t>(t) * heads + h) * dim + c];
+    }
+    if constexpr (sizeof(T) == 2) {
+        if (from.a2) {
+            // D[channel][token], a tile of sixteen channels a wave at a time
+            const int lane = tid & 63, n = lane & 15, g4 = lane >> 4;
+            const bf16_t* a = from.a + static_cast<int64_t>(t0 + min(n, nt - 1)) * from.a_stride + 8 * g4;
+            for (int tile = tid >> 6; tile < DP / 16; tile += kPrepThreads / 64) {
+                const bf16_t* w2 = from.a2 + static_cast<int64_t>(h * dim + min(16 * tile + n, dim - 1)) * from.rank + 8 * g4;
+                floatx4 sum{0.f, 0.f, 0.f, 0.f}, b4, out;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) b4[i] = from.bias[h * dim + min(16 * tile + 4 * g4 + i, dim - 1)];
+#pragma unroll 2
+                for (int s = 0; s < from.rank; s += 32)
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(w2 + s),
+                                                                 *reinterpret_cast<const bf16x8*>(a + s), sum, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    out[i] = n < nt && 16 * tile + 4 * g4 + i < dim ? to_log2 * log_sigmoid(sum[i] + b4[i]) : 0.f;
+                *reinterpret_cast<floatx4*>(bs + n * LD + 16 * tile + 4 * g4) = out;
+            }
+        }
     }
     if (cos_sin) {
         // the first 2 * pairs channels of a head are turned, channel c with channel c + pairs, by (cos, sin); float32
@@ -140,9 +174,10 @@ __global__ __launch_bounds__(kPrepThreads) void gla_chunk_prep_kernel(
     for (int i = 0; i < PER; ++i) {
         const int e = tid + i * kPrepThreads, t = e / DP, c = e % DP;
         const bool is = t < nt && c < dim;
-        const float log2_alpha = head_decay ? log2f(la[i]) : to_log2 * log_sigmoid(la[i]);
         qs[t * LD + c] = is ? q[i] * q_scale : 0.f;
         ks[t * LD + c] = is ? k[i] : 0.f;
+        if (from.a2) continue;
+        const float log2_alpha = head_decay ? log2f(la[i]) : to_log2 * log_sigmoid(la[i]);
         bs[t * LD + c] = is ? log2_alpha : 0.f;
     }
     __syncthreads();
@@ -429,7 +464,8 @@ int launch(const ChunksCall& c) {
     const T* rows = static_cast<const T*>(c.qk ? c.qk : c.proj);
     gla_chunk_prep_kernel<T, DP><<<dim3(c.heads, c.max_chunks), kPrepThreads, 0, c.stream>>>(
         c.q_starts, c.seq_slots, rows, c.qk ? c.qk_stride : c.proj_stride, c.z, c.work, c.n_seqs, c.n_slots, c.q_off, c.k_off, c.heads,
-        c.dim, static_cast<const T*>(c.proj) + c.v_off, c.proj_stride, c.vdim, c.q_scale, c.inv_tau, c.head_decay, c.cos_sin, c.pairs);
+        c.dim, static_cast<const T*>(c.proj) + c.v_off, c.proj_stride, c.vdim, c.q_scale, c.inv_tau, c.head_decay, c.cos_sin, c.pairs,
+        c.from);
     // segments that are not a portion's last are eight chunks and longer: at most max_chunks / 8 of them, and none where no
     // portion can have more than sixteen chunks
     const int inner = c.n_tokens > kWhole * kChunk ? c.max_chunks / kLeastSegment : 0;
@@ -459,18 +495,22 @@ extern "C" int64_t fsie_gla_chunk_floats(int heads, int dim, int vdim) {
 }
 
 // All portions of the step, chunk by chunk, for fsie_gla_scan (which has checked the operands): work has room for max_chunks
-// chunks, out is [n_tokens][heads * vdim].
+// chunks, out is [n_tokens][heads * vdim].  a2 (or null): the decays before the sigmoid are made here, z is not read.
 extern "C" int fsie_gla_chunks(const void* proj, int64_t proj_stride, int q_off, int k_off, int v_off, const float* z, float* state,
                                const int32_t* q_starts, const int32_t* seq_slots, int n_seqs, int n_tokens, float* out, float* work,
                                int max_chunks, int heads, int dim, int vdim, float q_scale, float inv_tau, int n_slots, int dtype,
                                const float* head_decay, const void* qk, int64_t qk_stride, const float* cos_sin, int rot_pairs,
-                               hipStream_t stream) {
+                               const void* a, int64_t a_stride, const void* a2, const float* a2_bias, int rank, hipStream_t stream) {
     FSIE_REQUIRE(max_chunks >= n_tokens / kChunk + n_seqs, "gla_scan: room for %d chunks, the step may have %d", max_chunks,
                  n_tokens / kChunk + n_seqs);
     FSIE_REQUIRE(n_seqs <= 65535 && heads <= 65535 && (vdim + 63) / 64 <= 65535, "gla_scan: too many requests, heads or columns");
     FSIE_REQUIRE(reinterpret_cast<uintptr_t>(work) % 16 == 0 && dim <= 256, "gla_scan: the work array must be 16-byte aligned");
+    FSIE_REQUIRE(!a2 || (dtype == FSIE_BF16 && !head_decay && a && a2_bias && rank > 0 && rank % 32 == 0 && a_stride >= rank && a_stride % 8 == 0 &&
+                         (reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(a2)) % 16 == 0),
+                 "gla_scan: a bottleneck of %d in rows of %lld: bfloat16, a multiple of 32, on 16 bytes", rank, static_cast<long long>(a_stride));
     const ChunksCall c{proj, qk, proj_stride, qk_stride, q_off, k_off, v_off, z, work, state, out, q_starts, seq_slots, n_seqs,
                        n_tokens, n_tokens / kChunk + n_seqs, heads, dim, vdim, n_slots, q_scale, inv_tau, head_decay,
-                       rot_pairs > 0 ? reinterpret_cast<const float2*>(cos_sin) : nullptr, rot_pairs, stream};
+                       rot_pairs > 0 ? reinterpret_cast<const float2*>(cos_sin) : nullptr, rot_pairs,
+                       Bottleneck{static_cast<const bf16_t*>(a), static_cast<const bf16_t*>(a2), a2_bias, a_stride, rank}, stream};
     return dtype == FSIE_F32 ? launch_dim<float>(c) : launch_dim<bf16_t>(c);
 }

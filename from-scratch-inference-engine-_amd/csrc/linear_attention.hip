@@ -184,11 +184,13 @@ extern "C" int fsie_gla_scan_shape(int heads, int dim, int vdim, int* prep_float
 // is o (fsie_gla_scan_shape gives both numbers).  chunk_work: room for max_chunks chunks, or null: with it every portion of
 // the step goes chunk by chunk, prep is not used and out is one array (max_chunks must be the bound that fsie_gla_scan_shape
 // names, or more); without it every portion is walked token by token.  The two ways differ by rounding only.
+// a2 (or null; with chunk_work and bfloat16): z = a2 [heads * dim][rank] . a [n_tokens][a_stride] + a2_bias is made on the way.
 extern "C" int fsie_gla_scan(const void* proj, int64_t proj_stride, int q_off, int k_off, int v_off, const float* z,
                              float* state, const int32_t* q_starts, const int32_t* seq_slots, int n_seqs, int n_tokens,
                              float* prep, float* out, float* chunk_work, int max_chunks, int heads, int dim, int vdim,
                              float q_scale, float inv_tau, int n_slots, int dtype, const float* head_decay,
-                             const void* qk, int64_t qk_stride, const float* cos_sin, int rot_pairs, hipStream_t stream) {
+                             const void* qk, int64_t qk_stride, const float* cos_sin, int rot_pairs, const void* a, int64_t a_stride,
+                             const void* a2, const float* a2_bias, int rank, hipStream_t stream) {
     FSIE_REQUIRE(rot_pairs >= 0 && 2 * rot_pairs <= dim && (rot_pairs == 0 || cos_sin), "gla_scan: %d rotated pairs in heads of %d",
                  rot_pairs, dim);
     const float2* turn = rot_pairs > 0 ? reinterpret_cast<const float2*>(cos_sin) : nullptr;
@@ -201,7 +203,8 @@ extern "C" int fsie_gla_scan(const void* proj, int64_t proj_stride, int q_off, i
     FSIE_REQUIRE(n_seqs >= 0 && n_tokens >= 0 && heads > 0 && dim > 0 && vdim > 0 && n_slots > 0, "gla_scan: bad sizes");
     FSIE_REQUIRE(dim <= 256, "gla_scan: %d key channels a head are more than the kernel takes (256)", dim);
     FSIE_REQUIRE(dtype == FSIE_F32 || dtype == FSIE_BF16, "gla_scan: unknown dtype %d", dtype);
-    FSIE_REQUIRE(proj && (z || head_decay) && state && q_starts && seq_slots && out && (prep || chunk_work), "gla_scan: missing operand");
+    FSIE_REQUIRE(!a2 || chunk_work, "gla_scan: decays from a bottleneck are made chunk by chunk");
+    FSIE_REQUIRE(proj && (z || head_decay || a2) && state && q_starts && seq_slots && out && (prep || chunk_work), "gla_scan: missing operand");
     FSIE_REQUIRE(q_off >= 0 && k_off >= 0 && v_off >= 0 && (qk || (q_off + heads * dim <= proj_stride &&
                      k_off + heads * dim <= proj_stride)) && v_off + heads * vdim <= proj_stride,
                  "gla_scan: the q, k and v columns do not fit a row of %lld", static_cast<long long>(proj_stride));
@@ -209,7 +212,7 @@ extern "C" int fsie_gla_scan(const void* proj, int64_t proj_stride, int q_off, i
     if (chunk_work)
         return fsie_gla_chunks(proj, proj_stride, q_off, k_off, v_off, z, state, q_starts, seq_slots, n_seqs, n_tokens, out, chunk_work,
                                max_chunks, heads, dim, vdim, q_scale, inv_tau, n_slots, dtype, head_decay, qk, qk_stride, cos_sin,
-                               rot_pairs, stream);
+                               rot_pairs, a, a_stride, a2, a2_bias, rank, stream);
     int rows, splits;
     gla_shape(heads, dim, vdim, &rows, &splits);
     const int dp = kGlaWaves * splits * rows;

@@ -1233,7 +1233,7 @@ def softcap(x: torch.Tensor, cap: float) -> torch.Tensor:
 def gla_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, z: torch.Tensor, state: torch.Tensor,
              q_starts: torch.Tensor, seq_slots: torch.Tensor, heads: int, dim: int, vdim: int, q_scale: float,
              inv_tau: float, chunked: bool = True, head_decay: Optional[torch.Tensor] = None,
-             qk: Optional[torch.Tensor] = None, cos_sin: Optional[torch.Tensor] = None) -> torch.Tensor:
+             qk: Optional[torch.Tensor] = None, cos_sin: Optional[torch.Tensor] = None, bottleneck=None) -> torch.Tensor:
     """S <- diag(sigmoid(z_t)^inv_tau) S + k_t v_t^T, o_t = S^T (q_scale q_t) over the tokens of every
     request of the step, from and to ``state`` float32 [slots, heads, dim, vdim].  ``proj`` [T, W] holds the
     q, k (heads x dim) and v (heads x vdim) columns from ``q_off``, ``k_off``, ``v_off``; ``z`` float32
@@ -1241,13 +1241,14 @@ def gla_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, z: torch.Te
     the shares of the P groups of key channels that the kernel deals a head's state to (P follows from the
     sizes, and is one in steps that go chunk by chunk); their sum in order is o, and ``gated_headnorm`` takes them as they are.
     Steps with portions of prompts are computed chunk by chunk on the matrix cores (the same sums in another order);
-    ``chunked=False`` walks every portion token by token."""
+    ``chunked=False`` walks every portion token by token.  ``bottleneck`` = (a, a2, bias) (bfloat16, in steps of which
+    ``gla_chunked`` says that they go chunk by chunk) in the place of z: z = a [T, rank] . a2 [heads * dim, rank]^T + bias."""
     _need(proj, "gla proj", ndim=2)
     t, w = proj.shape
     if head_decay is not None:
         # a fixed decay a head (float32 [heads]) instead of the decays of every token and key channel
         _need(head_decay, "gla head decay", dtype=torch.float32, shape=(heads,))
-    else:
+    elif bottleneck is None:
         _need(z, "gla z", dtype=torch.float32, shape=(t, heads * dim))
     _need(state, "gla state", dtype=torch.float32, ndim=4)
     if tuple(state.shape[1:]) != (heads, dim, vdim):
@@ -1274,8 +1275,17 @@ def gla_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, z: torch.Te
     chunk_floats = ctypes.c_int64(0)
     check(load().fsie_gla_scan_shape(heads, dim, vdim, ctypes.byref(per_token), ctypes.byref(planes),
                                      ctypes.byref(chunk_tokens), ctypes.byref(chunk_min), ctypes.byref(chunk_floats)))
-    # a step of single tokens (t == n, as every captured decode step is) has no portion to cut into chunks
-    max_chunks = t // chunk_tokens.value + n if chunked and t > n and t >= chunk_min.value else 0
+    max_chunks = t // chunk_tokens.value + n if chunked and gla_chunked(t, n) else 0
+    from_a = (None, 0, None, None, 0)
+    if bottleneck is not None:
+        a, a2, bias = bottleneck
+        _need(a, "gla bottleneck", dtype=torch.bfloat16, ndim=2)
+        rank = a.shape[1]
+        if a.shape[0] != t or not max_chunks:
+            raise KernelError("gla: a bottleneck has a row a token, in a step that goes chunk by chunk")
+        _need(a2, "gla a2", dtype=torch.bfloat16, shape=(heads * dim, rank))
+        _need(bias, "gla a2 bias", dtype=torch.float32, shape=(heads * dim,))
+        from_a = (a.data_ptr(), rank, a2.data_ptr(), bias.data_ptr(), rank)
     work = torch.empty((max_chunks * chunk_floats.value,), dtype=torch.float32, device=proj.device) if max_chunks else None
     prep = torch.empty((0 if max_chunks else t * per_token.value,), dtype=torch.float32, device=proj.device)
     out = torch.empty((1 if max_chunks else planes.value, t, heads * vdim), dtype=torch.float32, device=proj.device)
@@ -1283,8 +1293,14 @@ def gla_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, z: torch.Te
                                seq_slots.data_ptr(), n, t, prep.data_ptr(), out.data_ptr(),
                                work.data_ptr() if work is not None else None, max_chunks, heads, dim, vdim, float(q_scale),
                                float(inv_tau), state.shape[0], dtype_code(proj.dtype), _ptr(head_decay), _ptr(qk),
-                               qk.shape[1] if qk is not None else 0, _ptr(cos_sin), rot_pairs, _stream()))
+                               qk.shape[1] if qk is not None else 0, _ptr(cos_sin), rot_pairs, *from_a, _stream()))
     return out
+
+
+def gla_chunked(tokens: int, requests: int) -> bool:
+    """Whether ``gla_scan`` takes a step of so many tokens of so many requests chunk by chunk: one with a portion of a prompt (a step
+    of single tokens, as every captured decode step is, has nothing to cut into chunks) and sixteen tokens or more."""
+    return tokens > requests and tokens >= 16
 
 
 def gla_step_takes(heads: int, dim: int, vdim: int, rank: int) -> bool:

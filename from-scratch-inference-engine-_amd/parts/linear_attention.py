@@ -24,8 +24,8 @@ class GatedLinearAttention(Mixer):
 
     The projections that read x are one matrix (q, k, v, g rows one after the other; in steps of one token a request W_a1's rows
     too, and one kernel takes it from there to the output projection where it knows the sizes: ``ops.gla_step``).  The state lives in the
-    cache manager's per-request slots: zero when a request starts, carried from step to step; a portion of a
-    prompt and a single decoded token go through the same kernel, which walks a request's tokens in order.
+    cache manager's per-request slots: zero when a request starts, carried from step to step.  Steps with portions of prompts go
+    chunk by chunk (``ops.gla_scan``, which then multiplies by W_a2 itself), others token by token.
     The decays, the state and the sums are float32 whatever the activations' type."""
 
     graph_safe = True  # the step's requests and slots are read from the device tables
@@ -101,9 +101,15 @@ class GatedLinearAttention(Mixer):
                              1.0 / self.tau, self.norm_eps, self.gate_activation)
             return self.o.for_residual(y, ctx)
         p = self.qkvg(x)
-        z = self.a2(self.a1(x), out_dtype=torch.float32)  # the decays before the sigmoid, bias added, float32 from here on
+        a, a2 = self.a1(x), self.a2.weight
+        z, bottleneck = None, None
+        if (a.dtype == torch.bfloat16 and self.decay_rank % 32 == 0 and ops.gla_chunked(x.shape[0], ctx.seq_slots.shape[0])
+                and a.is_contiguous() and a2.is_contiguous() and a.data_ptr() % 16 == 0 and a2.data_ptr() % 16 == 0):
+            bottleneck = (a, a2, self.a2.bias)  # (the scan's first kernel multiplies)
+        else:
+            z = self.a2(a, out_dtype=torch.float32)  # the decays before the sigmoid, bias added, float32 from here on
         o = ops.gla_scan(p, 0, self.k_width, 2 * self.k_width, z, cache.state, ctx.q_starts, ctx.seq_slots, self.n_heads,
-                         self.key_dim, self.value_dim, self.key_dim ** -0.5, 1.0 / self.tau)
+                         self.key_dim, self.value_dim, self.key_dim ** -0.5, 1.0 / self.tau, bottleneck=bottleneck)
         y = ops.gated_headnorm(o, p[:, 2 * self.k_width + self.v_width:], self.norm_weight, self.norm_eps, self.n_heads,
                                self.gate_activation)
         return self.o.for_residual(y, ctx)

@@ -248,6 +248,28 @@ def test_gla_scan_in_segments(ops, dtype, heads, dim, vdim):
     assert torch.equal(states[0][7].cpu(), rnd((8, heads, dim, vdim), 9)[7])
 
 
+@pytest.mark.parametrize("heads, dim, vdim, rank", [(2, 128, 72, 64), (3, 16, 16, 32), (1, 200, 40, 96)])
+def test_gla_scan_makes_the_decays_from_the_bottleneck(ops, heads, dim, vdim, rank):
+    """Against the scan that is given them, made in float32 from the same bfloat16 values."""
+    lens = [1, 35, 16, 3]
+    t, kw, vw = sum(lens), heads * dim, heads * vdim
+    proj = rnd((t, 2 * kw + vw), 1).bfloat16().cuda()
+    a, a2, bias = rnd((t, rank), 2).bfloat16().cuda(), rnd((kw, rank), 3, 0.3).bfloat16().cuda(), rnd((kw,), 4).cuda()
+    z = (a.double() @ a2.double().t() + bias.double()).float()
+    starts = torch.from_numpy(np.cumsum([0] + lens).astype(np.int32)).cuda()
+    slots = torch.tensor([2, 0, 1, 3], dtype=torch.int32).cuda()
+    outs, states = [], []
+    for how in (dict(z=z), dict(z=None, bottleneck=(a, a2, bias))):
+        state = rnd((4, heads, dim, vdim), 9).cuda()
+        outs.append(ops.gla_scan(proj, 0, kw, 2 * kw, how.pop("z"), state, starts, slots, heads, dim, vdim, dim ** -0.5, 0.25, **how)[0])
+        states.append(state)
+    # z: a sum of `rank` products in float32, at most rank + 1 roundings of 2^-24 of magnitudes below 20, in up to 35 decays
+    assert rel(outs[1].cpu(), outs[0].double().cpu()) <= 1e-4 and rel(states[1].cpu(), states[0].double().cpu()) <= 1e-4
+    with pytest.raises(ops.KernelError, match="chunk by chunk"):
+        ops.gla_scan(proj[:4], 0, kw, 2 * kw, None, state, torch.arange(5, dtype=torch.int32).cuda(), slots, heads, dim, vdim, 1.0, 0.25,
+                     bottleneck=(a[:4], a2, bias))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_latent_prep_rope_pairs_and_head_gemm(ops, dtype):
     heads, q_rank, kv_rank, rot_dim, pairs, page, t = 3, 40, 52, 12, 4, 8, 11
