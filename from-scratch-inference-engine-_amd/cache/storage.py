@@ -6,7 +6,7 @@ from dataclasses import dataclass
 from typing import Dict, List, Tuple
 
 from .manager import CacheManager
-from .needs import CacheNeed, LayerCache  # noqa: F401  (LayerCache is also named from here)
+from .needs import CacheNeed, LayerCache, StateNeed  # noqa: F401  (LayerCache is also named from here)
 
 
 @dataclass
@@ -59,9 +59,18 @@ class CacheStorage:
 
     def reset_states(self, ctx) -> None:
         """Zero the per-request memory of the requests that start in this step (queued on the
-        stream like the rest of the step, from the step's own tables)."""
+        stream like the rest of the step, from the step's own tables); plain states all at once."""
+        from .. import ops
+
+        plain = []
         for cid, store in self.state_stores.items():
-            self.layout.state_caches[cid].reset(store, ctx)
+            need = self.layout.state_caches[cid]
+            if type(need).reset is StateNeed.reset:
+                plain.append(store)
+            else:
+                need.reset(store, ctx)
+        if plain:
+            ops.zero_rows_of(plain, ctx.reset_slots)
 
     def clear_fresh(self, ctx) -> None:
         """Zero the pages that this step's requests have just taken from the pools."""

@@ -58,7 +58,8 @@ int fsie_rmsnorm(float* residual, const void* delta, const float* weight, void* 
 int fsie_rmsnorm_plain(const void* x, int64_t x_stride, const float* weight, void* out, int64_t out_stride, int n_rows,
                        int groups, int width, float eps, int dtype, hipStream_t stream);
 // Rows slots[0..n) of a table of n_slots rows of row_bytes set to zero; a negative slot is skipped.
-int fsie_zero_rows(void* table, const int32_t* slots, int n, int64_t row_bytes, int n_slots, hipStream_t stream);
+int fsie_zero_rows(void* const* tables, const int64_t* row_bytes, const int* n_slots, int n_tables, const int32_t* slots, int n,
+                   hipStream_t stream);
 // Pages pages[0..n) (negative: skipped) of two pools of [planes][n_pages][page_bytes] set to zero.
 int fsie_zero_pages(void* pool_a, void* pool_b, const int32_t* pages, int n, int planes, int n_pages,
                     int64_t page_bytes, hipStream_t stream);

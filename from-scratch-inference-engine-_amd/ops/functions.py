@@ -5,7 +5,7 @@ from __future__ import annotations
 import ctypes
 
 from functools import lru_cache
-from typing import Optional
+from typing import Optional, Sequence
 
 import torch
 
@@ -141,15 +141,25 @@ def rmsnorm_plain(x: torch.Tensor, weight: torch.Tensor, eps: float, out: Option
 def zero_rows(table: torch.Tensor, slots: torch.Tensor) -> torch.Tensor:
     """``table[slots[i]] = 0`` for every non-negative entry of ``slots`` (int32); rows are whole
     multiples of four bytes."""
-    _need(table, "zero_rows table")
-    _need(slots, "zero_rows slots", dtype=torch.int32, ndim=1)
-    if table.dim() < 1:
-        raise KernelError("zero_rows: the table needs a first dimension of slots")
-    row_bytes = (table.numel() // max(table.shape[0], 1)) * table.element_size()
-    if row_bytes % 4:
-        raise KernelError(f"zero_rows: rows of {row_bytes} bytes are not whole 4-byte words")
-    check(load().fsie_zero_rows(table.data_ptr(), slots.data_ptr(), slots.shape[0], row_bytes, table.shape[0], _stream()))
+    zero_rows_of([table], slots)
     return table
+
+
+def zero_rows_of(tables: Sequence[torch.Tensor], slots: torch.Tensor) -> None:
+    """``zero_rows`` of every one of ``tables``, sixteen tables a launch."""
+    _need(slots, "zero_rows slots", dtype=torch.int32, ndim=1)
+    sizes = []
+    for table in tables:
+        _need(table, "zero_rows table")
+        if table.dim() < 1:
+            raise KernelError("zero_rows: the table needs a first dimension of slots")
+        row_bytes = (table.numel() // max(table.shape[0], 1)) * table.element_size()
+        if row_bytes % 4:
+            raise KernelError(f"zero_rows: rows of {row_bytes} bytes are not whole 4-byte words")
+        sizes.append(row_bytes)
+    n = len(sizes)
+    check(load().fsie_zero_rows((ctypes.c_void_p * n)(*(t.data_ptr() for t in tables)), (ctypes.c_int64 * n)(*sizes),
+                                (ctypes.c_int * n)(*(t.shape[0] for t in tables)), n, slots.data_ptr(), slots.shape[0], _stream()))
 
 
 def zero_pages(pool_a: torch.Tensor, pool_b: torch.Tensor, pages: torch.Tensor) -> None:

@@ -29,7 +29,7 @@ _SIGNATURES = {
     "fsie_embedding": ([_P, c_int, _P, _P, c_int, c_int, c_int, c_float, _P, _P, c_int, _P], c_int),
     "fsie_rmsnorm": ([_P, _P, _P, _P, _P, c_int, c_int, c_float, c_int, c_int, c_int, c_int, _P], c_int),
     "fsie_rmsnorm_plain": ([_P, c_int64, _P, _P, c_int64, c_int, c_int, c_int, c_float, c_int, _P], c_int),
-    "fsie_zero_rows": ([_P, _P, c_int, c_int64, c_int, _P], c_int),
+    "fsie_zero_rows": ([ctypes.POINTER(c_void_p), ctypes.POINTER(c_int64), ctypes.POINTER(c_int), c_int, _P, c_int, _P], c_int),
     "fsie_zero_pages": ([_P, _P, _P, c_int, c_int, c_int, c_int64, _P], c_int),
     "fsie_random_fill": ([_P, c_int64, ctypes.c_uint64, c_int, c_float, _P], c_int),
     "fsie_swiglu": ([_P, _P, c_int, c_int, c_int, _P], c_int),

@@ -1076,3 +1076,24 @@ def test_gemm_mfma_fp32(ops, m, n, k):
         ops.gemm_mfma_fp32(torch.zeros(2, 6).cuda(), torch.zeros(3, 6).cuda())
     with pytest.raises(ops.KernelError, match="at most 64 rows"):
         ops.gemm_mfma_fp32(torch.zeros(65, 8).cuda(), torch.zeros(3, 8).cuda())
+
+
+@pytest.mark.parametrize("widths", [(3,), (4, 1, 4096), (1030, 0, 70000, 5) + (8,) * 14])
+@pytest.mark.parametrize("slots", [(), (2,), (-1, 0, 7, 4, -1, 1)])
+def test_rows_of_several_tables_set_to_zero(ops, widths, slots):
+    """Rows of one word, of words no multiple of four, of nothing, more tables than a launch takes; tables that start
+    4 bytes past a multiple of 16; slots of none and beyond a table's rows."""
+    tables, want = [], []
+    for k, width in enumerate(widths):
+        rows = 5 + k % 2
+        flat = torch.full((rows * width + 1,), 1.5, device="cuda")
+        table = flat[k % 2:k % 2 + rows * width].view(rows, width)
+        tables.append(table)
+        want.append(table.clone())
+        for slot in slots:
+            if 0 <= slot < rows:
+                want[-1][slot] = 0.0
+    ops.zero_rows_of(tables, torch.tensor(slots, dtype=torch.int32, device="cuda"))
+    for table, expected in zip(tables, want):
+        assert torch.equal(table, expected)
+        assert table.numel() == 0 or (table._base[-1 if table.storage_offset() == 0 else 0] == 1.5)
