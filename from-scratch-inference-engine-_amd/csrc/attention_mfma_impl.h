@@ -190,7 +190,9 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const int n_waves = blockDim.x >> 6;
+    // (one tile: always launched so.  blockDim is a load that the keys of a wave wait for: 1 request of 100 keys of 64 values and 8 of
+    // 64 to 550 of 128, 5.5 and 6.6 us with it, 5.2 and 6.1 without)
+    const int n_waves = NT == 1 ? MAXW : static_cast<int>(blockDim.x) >> 6;
     const int c = lane & 15;  // column of S^T and O^T (query row of a tile); row of the A tiles
     const int G = lane >> 4;  // lane group: which 4 (or 8) of the reduction indices this lane holds
     const int32_t* table = block_tables + static_cast<int64_t>(seq) * max_pages;
@@ -225,7 +227,7 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
     float2 angle = float2{1.f, 0.f};
     int lds_at[NJ];
     const float* col_at[NJ];
-    const int sum_thread = static_cast<int>(threadIdx.x), sum_threads = static_cast<int>(blockDim.x);
+    const int sum_thread = static_cast<int>(threadIdx.x), sum_threads = 64 * n_waves;
     auto issue_sums = [&]() {
         const int q_dim = n_heads * HD, kv_dim = n_kv * HD;
         const int n_cols = (gh_here + 2) * HD;

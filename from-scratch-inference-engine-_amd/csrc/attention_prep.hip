@@ -121,7 +121,7 @@ __global__ __launch_bounds__(kThreads) void attention_prep_kernel(
             if (q_weight || k_weight) {  // (the same for the whole wave; a head without a weight drops the result)
                 float sum = fmaf(a[u][0], a[u][0], fmaf(a[u][1], a[u][1], fmaf(a[u][2], a[u][2], a[u][3] * a[u][3])));
                 for (int o = L >> 1; o > 0; o >>= 1) sum += __shfl_xor(sum, o, FSIE_WAVE);
-                scale = 1.0f / sqrtf(sum / static_cast<float>(dim) + eps);
+                scale = inverse_sqrt(sum / static_cast<float>(dim) + eps);
             }
             float b[4];
 #pragma unroll
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(kThreads) void attention_prep_kernel(
             if (w) {
                 float sum = 0.f;
                 for (int j = lane; j < dim; j += 64) sum = fmaf(to_float(x[j]), to_float(x[j]), sum);
-                scale = 1.0f / sqrtf(wave_sum(sum) / static_cast<float>(dim) + eps);
+                scale = inverse_sqrt(wave_sum(sum) / static_cast<float>(dim) + eps);
             }
             for (int j = lane; j < D; j += 64) o[j] = from_float<T>(j < dim ? normed_turned(x, j, scale, w, pairs, cs) : 0.f);
         }
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(kThreads) void attention_prep_kernel(
                     const float v = value(j);
                     sum = fmaf(v, v, sum);
                 }
-                unit = 1.0f / sqrtf(wave_sum(sum) / static_cast<float>(vdim) + v_eps);
+                unit = inverse_sqrt(wave_sum(sum) / static_cast<float>(vdim) + v_eps);
             }
             for (int j = lane; j < D; j += 64)
                 v_pool[((page * kv_heads + g) * D + j) * page_size + off] = from_float<T>(j < vdim ? value(j) * unit : 0.f);

@@ -22,7 +22,7 @@ __global__ void embedding_kernel(const T* __restrict__ table, const int32_t* __r
     float* dst = out + static_cast<int64_t>(t) * hidden;
     const T* src = id >= 0 && id < vocab ? table + static_cast<int64_t>(id) * hidden : nullptr;
     const T* place = pos >= 0 && pos < n_positions ? pos_table + static_cast<int64_t>(pos) * hidden : nullptr;
-    for (int j = threadIdx.x; j < hidden; j += blockDim.x) {
+    for (int j = threadIdx.x; j < hidden; j += kThreads) {
         const float v = src ? to_float(src[j]) * scale : 0.f;
         dst[j] = place ? v + to_float(place[j]) : v;
     }
@@ -53,16 +53,16 @@ __global__ void rmsnorm_kernel(float* __restrict__ residual, const T* __restrict
     };
     const bool has_delta = del || parts;
     float sum_sq = 0.f;
-    for (int j = threadIdx.x; j < hidden; j += blockDim.x) {
+    for (int j = threadIdx.x; j < hidden; j += kThreads) {
         float v = res[j];
         if (has_delta) v += delta_at(j);
         if (write_back) res[j] = v;
         sum_sq += v * v;
     }
-    const float total = block_sum(sum_sq, scratch);
-    const float scale = 1.0f / sqrtf(total / static_cast<float>(hidden) + eps);
+    const float total = block_sum<kThreads>(sum_sq, scratch);
+    const float scale = inverse_sqrt(total / static_cast<float>(hidden) + eps);
     T* dst = out + static_cast<int64_t>(r) * hidden;
-    for (int j = threadIdx.x; j < hidden; j += blockDim.x) {
+    for (int j = threadIdx.x; j < hidden; j += kThreads) {
         float v = res[j];
         if (has_delta && !write_back) v += delta_at(j);
         dst[j] = from_float<T>((v * scale) * weight[j]);
@@ -87,8 +87,8 @@ struct Pack4<bf16_t> {
     }
     static __device__ __forceinline__ void store(bf16_t* p, float4 v) {
         uint2 w;
-        w.x = static_cast<uint32_t>(float_to_bf16_bits(v.x)) | (static_cast<uint32_t>(float_to_bf16_bits(v.y)) << 16);
-        w.y = static_cast<uint32_t>(float_to_bf16_bits(v.z)) | (static_cast<uint32_t>(float_to_bf16_bits(v.w)) << 16);
+        w.x = pack2_bf16(v.x, v.y);
+        w.y = pack2_bf16(v.z, v.w);
         *reinterpret_cast<uint2*>(p) = w;
     }
 };
@@ -100,7 +100,7 @@ __global__ void embedding_vec_kernel(const T* __restrict__ table, const int32_t*
                                      const T* __restrict__ pos_table, const int32_t* __restrict__ positions,
                                      int n_positions) {
     const int t = blockIdx.x;
-    const int j = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
+    const int j = (blockIdx.y * kThreads + threadIdx.x) * 4;
     if (j >= hidden) return;
     const int id = ids[t];
     const bool ok = id >= 0 && id < vocab;
@@ -182,8 +182,8 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_vec_kernel(float* __restrict_
             sum_sq += v[it].x * v[it].x + v[it].y * v[it].y + v[it].z * v[it].z + v[it].w * v[it].w;
         }
     }
-    const float total = block_sum(sum_sq, scratch);
-    const float scale = 1.0f / sqrtf(total / static_cast<float>(hidden) + eps);
+    const float total = block_sum<THREADS>(sum_sq, scratch);
+    const float scale = inverse_sqrt(total / static_cast<float>(hidden) + eps);
     T* dst = out + static_cast<int64_t>(r) * hidden;
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
@@ -278,7 +278,7 @@ void launch_rmsnorm(const NormCall& c) {
 template <typename T>
 __global__ void swiglu_kernel(const T* __restrict__ x, T* __restrict__ out, int64_t total, int inter, int act, float limit,
                               float slope) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (i >= total) return;
     const float g = to_float(x[2 * i]);
     const float u = to_float(x[2 * i + 1]);
@@ -289,7 +289,7 @@ __global__ void swiglu_kernel(const T* __restrict__ x, T* __restrict__ out, int6
 template <typename T>
 __global__ void swiglu_vec_kernel(const T* __restrict__ x, T* __restrict__ out, int64_t quads, int act, float limit,
                                   float slope) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (i >= quads) return;
     const float4 a = Pack4<T>::load(x + 8 * i), b = Pack4<T>::load(x + 8 * i + 4);
     Pack4<T>::store(out + 4 * i, float4{gate_pair(a.x, a.y, act, limit, slope), gate_pair(a.z, a.w, act, limit, slope),
@@ -300,7 +300,7 @@ __global__ void swiglu_vec_kernel(const T* __restrict__ x, T* __restrict__ out, 
 template <typename T, bool VEC>
 __global__ void round_columns_kernel(const float* __restrict__ x, T* __restrict__ y, int64_t y_stride, int cols) {
     const int64_t row = blockIdx.x;
-    const int j = (blockIdx.y * blockDim.x + threadIdx.x) * (VEC ? 4 : 1);
+    const int j = (blockIdx.y * kThreads + threadIdx.x) * (VEC ? 4 : 1);
     if (j >= cols) return;
     if (VEC) Pack4<T>::store(y + row * y_stride + j, Pack4<float>::load(x + row * cols + j));
     else y[row * y_stride + j] = from_float<T>(x[row * cols + j]);
@@ -308,26 +308,26 @@ __global__ void round_columns_kernel(const float* __restrict__ x, T* __restrict_
 
 template <typename T>
 __global__ void residual_add_kernel(float* __restrict__ residual, const T* __restrict__ delta, int64_t total) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (i < total) residual[i] += to_float(delta[i]);
 }
 
 template <typename T>
 __global__ void round_to_kernel(const float* __restrict__ x, T* __restrict__ y, int64_t total) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (i < total) y[i] = from_float<T>(x[i]);
 }
 
 template <typename T>
 __global__ void scaled_sum_kernel(const T* __restrict__ x1, float a, const T* __restrict__ x2, float b, T* __restrict__ y,
                                   int64_t total) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (i < total) y[i] = from_float<T>(fmaf(a, to_float(x1[i]), b * to_float(x2[i])));
 }
 
 template <typename T>
 __global__ void bias_add_kernel(T* __restrict__ y, const float* __restrict__ bias, int64_t total, int cols) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     if (i < total) y[i] = from_float<T>(to_float(y[i]) + bias[i % cols]);
 }
 
@@ -373,7 +373,7 @@ __global__ void query_temperature_kernel(const int32_t* __restrict__ positions, 
 // y = act(sum of `planes` float32 partial sums, added in their order, + bias), rounded once; four values a thread
 __global__ void sum_round_kernel(const float* __restrict__ parts, int planes, int64_t plane, const float* __restrict__ bias,
                                  bf16_t* __restrict__ y, int64_t total, int cols, int act, float act_pos, float act_neg) {
-    const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
+    const int64_t i = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) * 4;
     if (i >= total) return;
     float4 sum = *reinterpret_cast<const float4*>(parts + i);
     for (int p = 1; p < planes; ++p) {
@@ -410,7 +410,7 @@ __global__ void zero_rows_kernel(ZeroTables t, const int32_t* __restrict__ slots
     if (slot < 0 || slot >= t.n_slots[which]) return;
     const int64_t words = t.row_words[which];
     uint32_t* row = t.table[which] + static_cast<int64_t>(slot) * words;
-    const int64_t first = static_cast<int64_t>(blockIdx.y) * blockDim.x + threadIdx.x, step = static_cast<int64_t>(gridDim.y) * blockDim.x;
+    const int64_t first = static_cast<int64_t>(blockIdx.y) * kThreads + threadIdx.x, step = static_cast<int64_t>(gridDim.y) * kThreads;
     if (words % 4 == 0 && reinterpret_cast<uintptr_t>(t.table[which]) % 16 == 0) {
         for (int64_t i = first; i < words / 4; i += step) reinterpret_cast<uint4*>(row)[i] = make_uint4(0u, 0u, 0u, 0u);
     } else {
@@ -430,8 +430,8 @@ __global__ void zero_pages_kernel(uint32_t* __restrict__ a, uint32_t* __restrict
     const int64_t n = page_words / static_cast<int64_t>(sizeof(V) / 4);
     V zero;
     memset(&zero, 0, sizeof(V));
-    for (int64_t i = static_cast<int64_t>(blockIdx.y) * blockDim.x + threadIdx.x; i < n;
-         i += static_cast<int64_t>(gridDim.y) * blockDim.x)
+    for (int64_t i = static_cast<int64_t>(blockIdx.y) * kThreads + threadIdx.x; i < n;
+         i += static_cast<int64_t>(gridDim.y) * kThreads)
         dst[i] = zero;
 }
 
@@ -445,8 +445,8 @@ __device__ __forceinline__ uint64_t splitmix_output(uint64_t key, uint64_t numbe
 
 __global__ void random_fill_kernel(void* __restrict__ out, int64_t n, uint64_t key, int kind, float std) {
 #pragma clang fp contract(off)  // a product and a sum stay two roundings, as on the host
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-         i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < n;
+         i += static_cast<int64_t>(gridDim.x) * kThreads) {
         const uint64_t a = splitmix_output(key, 2 * static_cast<uint64_t>(i));
         if (kind == 2) {
             static_cast<int32_t*>(out)[i] = static_cast<int32_t>((a >> 17) & 0x7FFF);
@@ -474,7 +474,7 @@ __global__ void rmsnorm_plain_kernel(const T* __restrict__ x, int64_t x_stride, 
                                      T* __restrict__ out, int64_t out_stride, int64_t n_runs, int groups, int width,
                                      float eps) {
     const int lane = threadIdx.x & (FSIE_WAVE - 1);
-    const int64_t run = static_cast<int64_t>(blockIdx.x) * (blockDim.x / FSIE_WAVE) + threadIdx.x / FSIE_WAVE;
+    const int64_t run = static_cast<int64_t>(blockIdx.x) * (kThreads / FSIE_WAVE) + threadIdx.x / FSIE_WAVE;
     if (run >= n_runs) return;
     const int64_t row = run / groups;
     const int g = static_cast<int>(run % groups);
@@ -486,7 +486,7 @@ __global__ void rmsnorm_plain_kernel(const T* __restrict__ x, int64_t x_stride, 
         sum += v * v;
     }
     sum = wave_sum(sum);
-    const float r = 1.0f / sqrtf(sum / static_cast<float>(width) + eps);
+    const float r = inverse_sqrt(sum / static_cast<float>(width) + eps);
     for (int i = lane; i < width; i += FSIE_WAVE) dst[i] = from_float<T>(to_float(src[i]) * r * weight[i]);
 }
 

@@ -148,7 +148,7 @@ __global__ __launch_bounds__(kStepThreads) void gla_step_kernel(
         float total = s_sum[0];
 #pragma unroll
         for (int w = 1; w < CPL; ++w) total += s_sum[w];
-        const float by = 1.0f / sqrtf(total / static_cast<float>(VDIM) + c.eps);
+        const float by = inverse_sqrt(total / static_cast<float>(VDIM) + c.eps);
         c.out[(static_cast<int64_t>(t) * c.heads + h) * VDIM + tid] = from_float<bf16_t>(((sum * by) * weight) * gate_act(gate, c.act));
     }
 }

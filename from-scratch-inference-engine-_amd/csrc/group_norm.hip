@@ -78,7 +78,7 @@ __global__ __launch_bounds__(kThreads) void group_rmsnorm_kernel(
         float sum = 0.f;
         for (int j = lane; j < part; j += 64) sum = fmaf(p[j], p[j], sum);
         sum = wave_sum(sum);
-        if (lane == 0) inv[g] = 1.0f / sqrtf(sum / static_cast<float>(part) + eps);
+        if (lane == 0) inv[g] = inverse_sqrt(sum / static_cast<float>(part) + eps);
     }
     __syncthreads();
     T* o1 = out1 + static_cast<int64_t>(r) * hidden;

@@ -45,7 +45,7 @@ __device__ __forceinline__ float rotated_neighbour(const T* __restrict__ run, in
 //             shared key part, its first 2 * pairs values rotated | zeros up to width]
 // A workgroup a token for the query latent and the gates and, where the layer keeps a cache, one for its row.  Some thousand values
 // a token: what it takes is the trips to memory one after the other, so a thread asks for the first kKept values of its own,
-// their weights, partners, angles and the slot before it adds anything up.  (8 tokens of 768 + 256 + 64 values: one workgroup
+// their weights, partners, angles and the slot before it adds anything up.  (8 tokens of 1,280 + 192 + 64 values: one workgroup
 // with a trip for each of them, one norm behind the other, 7.0 us, this 3.9; 2,048 tokens 10.5 and 10.3, their values' 2-byte stores.)
 constexpr int kKept = 4;
 template <typename T>
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kThreads) void latent_prep_kernel(
         for (int i = 0; i < kKept; ++i)
             if (tid + i * kThreads < q_rank) sum += to_float(own[i]) * to_float(own[i]);
         for (int j = tid + kKept * kThreads; j < q_rank; j += kThreads) sum += to_float(x[j]) * to_float(x[j]);
-        const float scale = 1.0f / sqrtf(block_sum(sum, scratch) / static_cast<float>(q_rank) + eps);
+        const float scale = inverse_sqrt(block_sum<kThreads>(sum, scratch) / static_cast<float>(q_rank) + eps);
         T* dst = cq + static_cast<int64_t>(t) * q_rank;
 #pragma unroll
         for (int i = 0; i < kKept; ++i) {
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kThreads) void latent_prep_kernel(
     for (int i = 0; i < kKept; ++i)
         if (tid + i * kThreads < kv_rank) sum += to_float(own[i]) * to_float(own[i]);
     for (int j = tid + kKept * kThreads; j < kv_rank; j += kThreads) sum += to_float(x[j]) * to_float(x[j]);
-    const float scale = 1.0f / sqrtf(block_sum(sum, scratch) / static_cast<float>(kv_rank) + eps);
+    const float scale = inverse_sqrt(block_sum<kThreads>(sum, scratch) / static_cast<float>(kv_rank) + eps);
     if (slot < 0 || slot >= pool_slots) return;
     const int64_t page = slot / page_size;
     const int off = static_cast<int>(slot - page * page_size);

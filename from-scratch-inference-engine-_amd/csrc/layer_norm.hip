@@ -122,7 +122,7 @@ __global__ __launch_bounds__(1024) void layer_norm_kernel(float* __restrict__ re
             }
         }
     }
-    const float inv = 1.0f / sqrtf(block_sum(sq, scratch) / static_cast<float>(hidden) + eps);
+    const float inv = inverse_sqrt(block_sum(sq, scratch) / static_cast<float>(hidden) + eps);
 #pragma unroll
     for (int k = 0; k < kMaxPer; ++k) {
         const int g = threadIdx.x + k * blockDim.x;

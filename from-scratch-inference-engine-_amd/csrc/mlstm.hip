@@ -314,7 +314,7 @@ __global__ __launch_bounds__(256) void mlstm_out_kernel(const float* __restrict_
         const float v = o[j] * d;
         sum = fmaf(v, v, sum);
     }
-    const float inv = 1.0f / sqrtf(wave_sum(sum) / static_cast<float>(vdim) + eps);
+    const float inv = inverse_sqrt(wave_sum(sum) / static_cast<float>(vdim) + eps);
     const T* g = gate + t * gate_stride + h * vdim;
     T* out = y + unit * vdim;
     for (int j = lane; j < vdim; j += 64) {

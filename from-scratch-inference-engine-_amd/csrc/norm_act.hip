@@ -41,7 +41,7 @@ __global__ __launch_bounds__(kThreads) void sandwich_norm_kernel(
         row_buf[j] = y;
         sum_sq += y * y;
     }
-    const float post_scale = 1.0f / sqrtf(block_sum(sum_sq, scratch) / static_cast<float>(hidden) + post_eps);
+    const float post_scale = inverse_sqrt(block_sum<kThreads>(sum_sq, scratch) / static_cast<float>(hidden) + post_eps);
     sum_sq = 0.f;
     for (int j = threadIdx.x; j < hidden; j += kThreads) {
         const float v = res[j] + (row_buf[j] * post_scale) * post_weight[j];
@@ -49,7 +49,7 @@ __global__ __launch_bounds__(kThreads) void sandwich_norm_kernel(
         if (write_back) res[j] = restart ? restart[j] : v;
         sum_sq += v * v;
     }
-    const float scale = 1.0f / sqrtf(block_sum(sum_sq, scratch) / static_cast<float>(hidden) + eps);
+    const float scale = inverse_sqrt(block_sum<kThreads>(sum_sq, scratch) / static_cast<float>(hidden) + eps);
     T* dst = out + static_cast<int64_t>(r) * out_stride;
     for (int j = threadIdx.x; j < hidden; j += kThreads)
         dst[j] = from_float<T>(weight ? (row_buf[j] * scale) * weight[j] : row_buf[j]);  // (no weight: the stream itself)
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(THREADS) void sandwich_norm_vec_kernel(
         if ((it * THREADS + static_cast<int>(threadIdx.x)) * 4 < hidden)
             sum_sq += y[it].x * y[it].x + y[it].y * y[it].y + y[it].z * y[it].z + y[it].w * y[it].w;
     }
-    const float post_scale = 1.0f / sqrtf(block_sum(sum_sq, scratch) / static_cast<float>(hidden) + post_eps);
+    const float post_scale = inverse_sqrt(block_sum<THREADS>(sum_sq, scratch) / static_cast<float>(hidden) + post_eps);
     sum_sq = 0.f;
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(THREADS) void sandwich_norm_vec_kernel(
         }
     }
     // without a weight the stream itself is the result (a layer whose sublayers read the stream as it is)
-    const float scale = weight ? 1.0f / sqrtf(block_sum(sum_sq, scratch) / static_cast<float>(hidden) + eps) : 1.f;
+    const float scale = weight ? inverse_sqrt(block_sum<THREADS>(sum_sq, scratch) / static_cast<float>(hidden) + eps) : 1.f;
     T* dst = out + static_cast<int64_t>(r) * out_stride;
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(kThreads) void gated_headnorm_kernel(const float* _
 #pragma unroll
         for (int j = 0; j < HELD; ++j)
             if (lane + FSIE_WAVE * j < width) total += x[j] * x[j];
-        const float by = 1.0f / sqrtf(wave_sum(total) / static_cast<float>(width) + eps);
+        const float by = inverse_sqrt(wave_sum(total) / static_cast<float>(width) + eps);
 #pragma unroll
         for (int j = 0; j < HELD; ++j)
             if (lane + FSIE_WAVE * j < width)
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(kThreads) void gated_headnorm_kernel(const float* _
         sum += x * x;
     }
     sum = wave_sum(sum);
-    const float scale = 1.0f / sqrtf(sum / static_cast<float>(width) + eps);
+    const float scale = inverse_sqrt(sum / static_cast<float>(width) + eps);
     for (int i = lane; i < width; i += FSIE_WAVE)
         dst[i] = from_float<T>((((value(i) * scale) * weight[i]) * gate_act(to_float(g[i]), act)) * out_scale);
 }

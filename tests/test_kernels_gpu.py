@@ -1097,3 +1097,26 @@ def test_rows_of_several_tables_set_to_zero(ops, widths, slots):
     for table, expected in zip(tables, want):
         assert torch.equal(table, expected)
         assert table.numel() == 0 or (table._base[-1 if table.storage_offset() == 0 else 0] == 1.5)
+
+
+@pytest.mark.parametrize("size", [1e-18, 3e-16, 1e-15, 1.0, 3e14, 1e15, 1e17])
+def test_norm_factor_at_the_ends_of_its_range(ops, size):
+    """The factor's short form holds between 2^-100 and 2^100 of the mean square; on both sides and beyond, the result is
+    within the rounding of the sum's 300 terms (a mean over lanes: 16 roundings at most in a row), the factor's and two
+    products': 12 units of 2^-24."""
+    x = rnd((4, 300), 5) * size
+    out = ops.rmsnorm_plain(x.cuda(), torch.ones(300, device="cuda"), 0.0).cpu().double()
+    want = x.double() / x.double().pow(2).mean(dim=1, keepdim=True).sqrt()
+    assert ((out - want) / want).abs().max() <= 12 * 2.0 ** -24
+
+
+def test_rounding_to_bfloat16(ops):
+    """Ties, values next to them, subnormal numbers, infinities: to nearest even; NaN stays NaN."""
+    bits = torch.tensor([0x3f808000, 0x3f818000, 0x3f807fff, 0x3f808001, 0x00008000, 0x00018000, 0x007f8000, 0x7f7fffff, 0x7f7f7fff,
+                         0x7f800000, -0x7fffff, 0x7f800001, 0x7fffffff], dtype=torch.int64).to(torch.int32)
+    bits = torch.cat([bits, bits ^ torch.tensor(-2 ** 31, dtype=torch.int32)])
+    x = bits.view(torch.float32)
+    got = ops.round_to(x.view(1, -1).cuda(), torch.bfloat16).view(-1).cpu()
+    want = x.to(torch.bfloat16)
+    nan = x.isnan()
+    assert torch.equal(got.isnan(), nan) and torch.equal(got[~nan].view(torch.int16), want[~nan].view(torch.int16))
