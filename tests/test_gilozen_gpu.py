@@ -248,6 +248,34 @@ def test_gla_scan_in_segments(ops, dtype, heads, dim, vdim):
     assert torch.equal(states[0][7].cpu(), rnd((8, heads, dim, vdim), 9)[7])
 
 
+@pytest.mark.parametrize("heads, dim, vdim, lens", [(1, 16, 16, [8200, 8193, 17]), (2, 96, 70, [256, 300, 33]), (1, 129, 40, [16, 400, 1]), (1, 192, 64, [700, 15]),
+                                                    (3, 256, 130, [257, 2, 140])])
+@pytest.mark.parametrize("how", ["channels", "heads", "heads turned"])
+def test_gla_scan_in_segments_of_every_length_and_width(ops, heads, dim, vdim, lens, how):
+    """Segments of 32 chunks (portions of more than 8,192 tokens), tiles of six sixteens of channels, heads in two halves; decays of
+    every channel, and fixed ones with and without a rotation: against the walk token by token.  Both are float32 sums of the same
+    terms; what a state that forgets nothing has added up over n tokens differs by the root of n roundings of 2^-24 and more."""
+    t, kw, vw = sum(lens), heads * dim, heads * vdim
+    proj, z = rnd((t, 2 * kw + vw), 1).cuda(), rnd((t, kw), 2, 4.0).cuda()
+    z.view(t, heads, dim)[:, :, 0::3] = 25.0  # keeps everything
+    args = dict(head_decay=torch.linspace(0.9, 1.0, heads).cuda()) if how != "channels" else {}
+    if how == "heads turned":
+        angle = rnd((t, dim // 4), 3)
+        args["cos_sin"] = torch.stack([torch.cos(angle), torch.sin(angle)], -1).contiguous().cuda()
+    starts = torch.from_numpy(np.cumsum([0] + lens).astype(np.int32)).cuda()
+    slots = torch.arange(len(lens), dtype=torch.int32).flip(0).contiguous().cuda()
+    outs, states = [], []
+    for chunked in (True, False):
+        state = rnd((len(lens) + 1, heads, dim, vdim), 9).cuda()
+        outs.append(ops.gla_scan(proj, 0, kw, 2 * kw, None if args else z, state, starts, slots, heads, dim, vdim, dim ** -0.5, 0.5,
+                                 chunked=chunked, **args).sum(0))
+        states.append(state)
+    for lo, hi in zip(starts.tolist(), starts.tolist()[1:]):
+        assert rel(outs[0][lo:hi].cpu(), outs[1][lo:hi].double().cpu()) <= 2e-5, hi - lo
+    assert rel(states[0].cpu(), states[1].double().cpu()) <= 2e-5
+    assert torch.equal(states[0][-1], rnd((len(lens) + 1, heads, dim, vdim), 9)[-1].cuda())
+
+
 @pytest.mark.parametrize("heads, dim, vdim, rank", [(2, 128, 72, 64), (3, 16, 16, 32), (1, 200, 40, 96)])
 def test_gla_scan_makes_the_decays_from_the_bottleneck(ops, heads, dim, vdim, rank):
     """Against the scan that is given them, made in float32 from the same bfloat16 values."""
@@ -268,6 +296,26 @@ def test_gla_scan_makes_the_decays_from_the_bottleneck(ops, heads, dim, vdim, ra
     with pytest.raises(ops.KernelError, match="chunk by chunk"):
         ops.gla_scan(proj[:4], 0, kw, 2 * kw, None, state, torch.arange(5, dtype=torch.int32).cuda(), slots, heads, dim, vdim, 1.0, 0.25,
                      bottleneck=(a[:4], a2, bias))
+
+
+@pytest.mark.parametrize("heads, dim, vdim", [(2, 96, 72), (1, 200, 40)])
+def test_decays_from_the_bottleneck_in_segments(ops, heads, dim, vdim):
+    """Portions of several segments and a single token: against the walk token by token with the decays' logits made in 64 bits."""
+    lens, rank = [300, 1, 700], 32
+    t, kw, vw = sum(lens), heads * dim, heads * vdim
+    proj = rnd((t, 2 * kw + vw), 1).bfloat16().cuda()
+    a, a2, bias = rnd((t, rank), 2).bfloat16().cuda(), rnd((kw, rank), 3, 0.3).bfloat16().cuda(), rnd((kw,), 4).cuda()
+    z = (a.double() @ a2.double().t() + bias.double()).float()
+    starts = torch.from_numpy(np.cumsum([0] + lens).astype(np.int32)).cuda()
+    slots = torch.tensor([1, 0, 2], dtype=torch.int32).cuda()
+    outs, states = [], []
+    for how in (dict(z=z, chunked=False), dict(z=None, bottleneck=(a, a2, bias))):
+        state = rnd((3, heads, dim, vdim), 9).cuda()
+        outs.append(ops.gla_scan(proj, 0, kw, 2 * kw, how.pop("z"), state, starts, slots, heads, dim, vdim, dim ** -0.5, 0.25, **how).sum(0))
+        states.append(state)
+    # z: at most rank + 1 roundings of 2^-24 of magnitudes below 20, a factor exp(0.25 dz) a token, and of decays of exp(-0.1) and less on
+    # the average some ten tokens count
+    assert rel(outs[1].cpu(), outs[0].double().cpu()) <= 1e-4 and rel(states[1].cpu(), states[0].double().cpu()) <= 1e-4
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
