@@ -185,6 +185,7 @@ extern "C" int fsie_gemm_mfma_stream_plan(int M, int N, int K, int result, int f
     if (result == SUMS) {
         if (!frags || K < 1024) return -1;
         int splits = (steps + 8 * kMostSteps - 1) / (8 * kMostSteps);
+        if (splits > FSIE_GEMM_MAX_SPLITS) return -1;  // (K beyond 32,768: more partial sums than the norm takes)
         const int blocks = groups * splits > units ? 2 : 1;
         const int across = (groups + blocks - 1) / blocks;
         if (across * splits > units) return -1;

@@ -76,3 +76,34 @@ def test_what_the_plan_takes(ops):
     x = torch.zeros((4, 100), dtype=torch.bfloat16, device="cuda")
     with pytest.raises(ops.KernelError, match="bad sizes"):
         ops.gemm_mfma_stream(x, torch.zeros((8, 100), dtype=torch.bfloat16, device="cuda"), ops.GEMM_STREAM_POINT, 4 + 256 + 65536)
+
+
+def test_every_plan_is_one_that_the_kernel_takes(ops):
+    """Over sizes of all kinds, K beyond what sixteen slices hold among them: the checks of the launch itself, and the residual
+    projections of such sizes."""
+    from from_scratch_inference_engine_amd.parts.linear import Linear
+
+    taken = {r: 0 for r in range(4)}
+    for k in [32 * s for s in (1, 3, 4, 5, 31, 32, 33, 63, 64, 65, 127, 128, 129, 152, 511, 512, 513, 592, 1023, 1024, 1025, 1152, 1280, 2048)]:
+        for n in (4, 16, 20, 36, 64, 100, 256, 272, 896, 1536, 2048, 3584, 4096, 4112, 8192, 11264, 19456, 37888):
+            for result in taken:
+                for m in (1, 2, 3, 8, 9, 16):
+                    for frags in (True, False):
+                        plan = ops.gemm_stream_plan(m, n, k, result, frags)
+                        if plan is None:
+                            continue
+                        taken[result] += 1
+                        waves, blocks, splits = plan & 255, plan >> 8 & 255, plan >> 16
+                        slice_steps = -(-(k // 32) // splits)
+                        assert 1 <= splits <= (16 if result == ops.GEMM_STREAM_SUMS else 1) and slice_steps * (splits - 1) < k // 32, (m, n, k, result)
+                        assert waves in (4, 8, 16) and blocks in (1, 2) and -(-slice_steps // waves) <= 8, (m, n, k, result)
+                        assert frags or result in (ops.GEMM_STREAM_POINT, ops.GEMM_STREAM_PLAN_ACT)
+    assert min(taken.values()) > 100
+    for n, k in ((256, 36864), (64, 40960)):
+        x, w, exact, bound = operands(8, n, k)
+        linear = Linear(k, n)
+        linear.weight = w
+        linear.streamed = ops.fragment_order(w)
+        sums = linear.for_residual(x, type("Step", (), {"partial_sums_ok": True}))
+        got = (sums.double().sum(0) if sums.dim() == 3 else sums.double())
+        assert ((got - exact).abs() <= bound + (0 if sums.dim() == 3 else 2.0 ** -8 * exact.abs())).all(), (n, k)
