@@ -115,12 +115,21 @@ class AttentionPlanner:
     mfma_keeps_first = True  # whether the matrix-core kernels read an item's kept first keys
 
     def _waves_for(self, keys: int, max_waves: int) -> int:
-        """Waves of a workgroup for an item of ``keys`` keys: one per 128 keys, a power of two."""
+        """What a launch is told of items of up to ``keys`` keys: 1, all of them are short (four blocks of 32 keys: the variant
+        with four waves), or more, which is the variant with all the waves that the head size allows."""
         need = max(1, -(-keys // 128))
         w = 1
         while w < need and w < max_waves:
             w *= 2
         return min(w, max_waves)
+
+    def _graph_waves(self, keys: int) -> int:
+        """The same for a captured launch: 1 or all, so that a batch whose items grow from 200 to 2,000 keys keeps its graph.  (Heads
+        with at most as many waves as the variant for short items have that one alone.)"""
+        most = ops.attention_mfma_max_waves(self.head_dim)
+        return 1 if most <= self.short_waves or self._waves_for(keys, most) == 1 else most
+
+    short_waves = 4  # waves of the variant for short items
 
     def _small_keys(self, host, small_tokens):
         """Keys that each small portion of the step reads."""
@@ -253,7 +262,7 @@ class AttentionPlanner:
 
     def graph_bucket(self, host):
         """What a captured graph of this step's shape must fix: the number of (small) work items,
-        the waves per item and the keys per item; None if the step has portions that do not fit
+        the variant of the matrix-core kernel and (of the other one) the keys per item; None if the step has portions that do not fit
         small items."""
         mfma = self.uses_mfma(host.compute_dtype, host.page_size)
         small_tokens = self.geometry(mfma)[0]
@@ -279,7 +288,7 @@ class AttentionPlanner:
             # every request is one whole item: no records, no merge.  A graph of its own: the merge that finds nothing to do costs
             # 1.5 us a layer (one request of the 0.5B shape, 61 tokens and 48 more, 37.3 ms, 35.5 without), the step from whole
             # to cut items one capture more in a batch's life
-            return (n, self._waves_for(longest, ops.attention_mfma_max_waves(self.head_dim)) if mfma else 1, 0 if mfma else split_keys)
+            return (n, self._graph_waves(longest) if mfma else 1, 0 if mfma else split_keys)
         if mfma:
             # items: a multiple of the number of requests and of a quarter of what gives every unit a
             # workgroup, so that one graph serves a batch while its requests grow: their items grow
@@ -289,8 +298,7 @@ class AttentionPlanner:
             group = self.n_heads // self.n_kv
             per_item = self.n_kv * -(-group // min(group, ops.attention_mfma_rows(self.head_dim, False)))
             step = max(host.n_seqs, units // per_item // 4, 1)
-            return (-(-n // step) * step,
-                    self._waves_for(longest, ops.attention_mfma_max_waves(self.head_dim)), 0)
+            return (-(-n // step) * step, self._graph_waves(longest), 0)
         step = host.n_seqs * max(1, 1024 // split_keys)
         return (-(-n // step) * step, 1, split_keys)
 

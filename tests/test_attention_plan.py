@@ -230,3 +230,17 @@ def test_the_short_tile_at_the_end_of_a_long_portion_stays_with_its_group():
     assert covered == list(range(len(tiles))), "every tile, the short one too, is in a group"
     last = max(groups, key=lambda g: int(g[0]) + int(g[1]))
     assert int(last[0]) + int(last[1]) == len(tiles) and int(last[1]) >= 2
+
+
+@pytest.mark.parametrize("head_dim, variants", [(64, [1, 16]), (128, [1, 8]), (256, [1])])
+def test_a_graph_knows_the_variant_of_its_launch_and_no_more(head_dim, variants):
+    """Whole items of 200, 400, 900 and more keys are the same launch, those of up to four blocks of 32 keys another one; wide heads
+    have one variant only."""
+    planner = AttentionPlanner(28, 4, head_dim, None)
+    planner.compute_units = 256
+    seen = []
+    for keys in (20, 100, 128, 129, 200, 300, 400, 512):
+        bucket = planner.graph_bucket(Host([(keys - 1, 1)] * 64, 16, torch.bfloat16))
+        assert bucket[0] == 64
+        seen.append(bucket[1])
+    assert seen == [variants[0]] * 3 + [variants[-1]] * 5
