@@ -131,14 +131,19 @@ class AttentionPlanner:
 
     short_waves = 4  # waves of the variant for short items
 
-    def _small_keys(self, host, small_tokens):
-        """Keys that each small portion of the step reads."""
+    def _cut_from(self, first: int, mfma: bool) -> int:
+        """Where the runs that a portion's keys are cut into are counted from: the matrix-core kernel takes blocks of 32 keys from a
+        multiple of 32 on, so runs from a window's first key would have a block more each than their keys are."""
+        return first & ~31 if mfma else first
+
+    def _small_keys(self, host, small_tokens, mfma: bool):
+        """(Keys that it reads, the same from where its runs are counted) of each small portion of the step."""
         keys = []
         for s in range(host.n_seqs):
             for _, n, p in self._portions(host.past_lens[s], host.q_lens[s]):
                 if n <= small_tokens:
                     first, kept = self._first_key(p)
-                    keys.append(p + n - first + kept)
+                    keys.append((p + n - first + kept, p + n - self._cut_from(first, mfma) + kept))
         return keys
 
     def split_keys(self, host, mfma: bool) -> int:
@@ -156,8 +161,12 @@ class AttentionPlanner:
     def _split_keys(self, host, mfma: bool) -> int:
         small_tokens, _, longest = self.geometry(mfma)
         units = self.compute_units if self.compute_units is not None else ops.compute_units()
-        keys = self._small_keys(host, small_tokens)
+        both = self._small_keys(host, small_tokens, mfma)
+        keys = [k for k, _ in both]
         group = self.n_heads // self.n_kv
+
+        def items_in(length):
+            return sum(self._items_of(k, span, length) for k, span in both)
         # the float32-arithmetic kernel takes 32 keys a pass and up to 16 heads of a group a workgroup:
         # its items shorten to 64 keys (two passes) while compute units are idle
         rows, shortest, room = (ops.attention_mfma_rows(self.head_dim, False), 128, 1) if mfma else (16, 64, 2)
@@ -172,14 +181,14 @@ class AttentionPlanner:
         # share a unit: twice the units.
         # (the matrix-core kernel: up to exactly one workgroup a unit)
         most_groups = units * room + (1 if mfma else 0)
-        while split > shortest and sum(-(-k // (split // 2)) for k in keys) * per_item < most_groups:
+        while split > shortest and items_in(split // 2) * per_item < most_groups:
             split //= 2
         if self.fine_items and mfma and keys and split > shortest:
             # between that length and its half: the shortest multiple of 32 whose workgroups still number at most the units
             lo, hi = 0, (split - split // 2) // 32 - 1
             while lo < hi:
                 mid = (lo + hi + 1) // 2
-                if sum(-(-k // (split - 32 * mid)) for k in keys) * per_item < most_groups:
+                if items_in(split - 32 * mid) * per_item < most_groups:
                     lo = mid
                 else:
                     hi = mid - 1
@@ -221,7 +230,8 @@ class AttentionPlanner:
         # Both in steps of a 64th of the length (at least 32 keys) and to no less than half of it.
         if self.fill_rounds and mfma and keys and units > 0:
             def groups_of(length, least=0):
-                return sum(k // length + (1 if k % length > least else 0) for k in keys) * per_item
+                runs = (span if k > length else k for k, span in both)
+                return sum(k // length + (1 if k % length > least else 0) for k in runs) * per_item
             everyone, large_ones = groups_of(split), groups_of(split, split // 4)
             rounds = -(-large_ones // units)
             room_for = 0
@@ -256,9 +266,10 @@ class AttentionPlanner:
     fine_items = True
 
     @staticmethod
-    def _items_of(keys: int, split_keys: int, longest: int) -> int:
-        """Items that the ``keys`` keys of a small portion are cut into: runs of ``split_keys``."""
-        return max(1, -(-keys // split_keys))
+    def _items_of(keys: int, span: int, split_keys: int) -> int:
+        """Items that the ``keys`` keys of a small portion are cut into, if they are more than ``split_keys``: runs of so many from
+        where they are counted, ``span`` keys before the last."""
+        return 1 if keys <= split_keys else -(-span // split_keys)
 
     def graph_bucket(self, host):
         """What a captured graph of this step's shape must fix: the number of (small) work items,
@@ -267,22 +278,22 @@ class AttentionPlanner:
         mfma = self.uses_mfma(host.compute_dtype, host.page_size)
         small_tokens = self.geometry(mfma)[0]
         split_keys = self.split_keys(host, mfma)
-        most = self.geometry(mfma)[2]
         n, longest = 0, 1
         for s in range(host.n_seqs):
             if host.q_lens[s] > small_tokens:
                 return None
             first_key, kept = self._first_key(host.past_lens[s])
-            keys = host.past_lens[s] + host.q_lens[s] - first_key
-            mine = self._items_of(keys, split_keys, most)
-            longest = max(longest, keys - (mine - 1) * split_keys)  # (the last item; the others have split_keys, if any)
+            total = host.past_lens[s] + host.q_lens[s]
+            span = total - self._cut_from(first_key, mfma)
+            mine = self._items_of(total - first_key, span, split_keys)
+            longest = max(longest, span - (mine - 1) * split_keys)  # (the last item; the others have split_keys, if any)
             if mine > 1:
                 longest = max(longest, split_keys)
                 mine += 1 if kept else 0  # (the kept first keys are an item of their own)
                 if not mfma:  # (and the pooled blocks; the matrix-core geometry keeps them in a table of their own)
                     mine += 1 if self._pooled_seen(host.past_lens[s] + host.q_lens[s] - 1) else 0
             elif kept:
-                longest = max(longest, keys + 32 * -(-kept // 32))
+                longest = max(longest, span + 32 * -(-kept // 32))
             n += mine
         if n == host.n_seqs:
             # every request is one whole item: no records, no merge.  A graph of its own: the merge that finds nothing to do costs
@@ -304,7 +315,7 @@ class AttentionPlanner:
 
     def plan(self, host) -> Dict[str, object]:
         mfma = self.uses_mfma(host.compute_dtype, host.page_size)
-        small_tokens, large_tokens, most = self.geometry(mfma)
+        small_tokens, large_tokens, _ = self.geometry(mfma)
         padded = getattr(host, "pad", None) is not None
         split_keys = self.split_keys(host, mfma)
         small, merges = [], []
@@ -333,7 +344,8 @@ class AttentionPlanner:
                 first_key, kept = self._first_key(p)
                 keep = self.keep_first
                 total = p + n
-                n_splits = self._items_of(total - first_key, split_keys, most) if split_keys is not None else 1
+                cut_from = self._cut_from(first_key, mfma)
+                n_splits = self._items_of(total - first_key, total - cut_from, split_keys) if split_keys is not None else 1
                 pooled = self._pooled_seen(total - 1) > 0
                 if n <= small_tokens and (n_splits > 1 or (two_pass and pooled)):
                     base = n_partial
@@ -347,8 +359,8 @@ class AttentionPlanner:
                         small.append((s, row0, n, p, 0, 0, base, keep | pool_flag))
                         base += n
                     for i in range(n_splits):
-                        kb = first_key + i * split_keys
-                        small.append((s, row0, n, p, kb, total if i == n_splits - 1 else kb + split_keys, base + i * n, keep))
+                        kb = cut_from + i * split_keys
+                        small.append((s, row0, n, p, max(kb, first_key), total if i == n_splits - 1 else kb + split_keys, base + i * n, keep))
                     n_splits += (1 if kept else 0) + (1 if pooled else 0)
                     for t in range(n):
                         merges.append((row0 + t, n_partial + t, n_splits, n))
@@ -400,7 +412,9 @@ class AttentionPlanner:
         large = np.concatenate(large_runs) if large_runs else np.zeros((0, ATTN_ITEM_INTS), dtype=np.int64)
         waves = 1
         if mfma and small:
-            waves = self._waves_for(max(it[5] - it[4] + (32 * -(-min(it[7] & ~(ATTN_KEEP_WALK | ATTN_POOL_WALK), it[4]) // 32)
+            # (in blocks of 32 keys, those of the kept first ones too: the variant for short items has four waves and takes four
+            # blocks, so that how an item's keys are dealt to waves is the same in either variant)
+            waves = self._waves_for(max(it[5] - (it[4] & ~31) + (32 * -(-min(it[7] & ~(ATTN_KEEP_WALK | ATTN_POOL_WALK), it[4]) // 32)
                                                             if it[7] & ATTN_KEEP_WALK else 0) for it in small),
                                     ops.attention_mfma_max_waves(self.head_dim))
         if padded:

@@ -244,3 +244,27 @@ def test_a_graph_knows_the_variant_of_its_launch_and_no_more(head_dim, variants)
         assert bucket[0] == 64
         seen.append(bucket[1])
     assert seen == [variants[0]] * 3 + [variants[-1]] * 5
+
+
+@pytest.mark.parametrize("args", [dict(window=1024), dict(window=128), dict(window=98), dict(window=700, keep_first=40), dict(window=None, chunk=200)])
+def test_short_items_are_four_blocks_of_keys_wherever_a_window_starts(args):
+    """The variant for short items has four waves, a block of 32 keys each, counted from a multiple of 32: an item of more blocks would
+    be dealt otherwise than in the variant with all waves, so that a row's sums would depend on the step's longest item."""
+    rng = random.Random(str(args))
+    planner = AttentionPlanner(16, 4, 128, **args)
+    planner.compute_units = 256
+    short = 0
+    for _ in range(60):
+        host = Host([(rng.choice([rng.randint(0, 300), rng.randint(0, 5000)]), 1) for _ in range(rng.choice([1, 2, 6, 20, 64]))], 16, torch.bfloat16)
+        plan = planner.plan(host)
+        if not args.get("keep_first") and not args.get("chunk"):
+            check_plan(planner, host, plan)
+        blocks = [-(-(int(it[KE]) - (int(it[KB]) & ~31)) // 32) for it in plan["items"]]
+        if args.get("keep_first"):  # (the kept first keys, read as blocks of their own ahead of the item's)
+            kept = [-(-min(args["keep_first"], int(it[KB])) // 32) if it[PARTIAL] < 0 else 0 for it in plan["items"]]
+            blocks = [b + k for b, k in zip(blocks, kept)]
+        assert (plan["waves"] == 1) == (max(blocks) <= 4), blocks
+        assert all(int(it[KB]) % 32 == 0 for it in plan["items"] if it[PARTIAL] >= 0 and int(it[KB]) > planner._first_key(int(it[POS]))[0])
+        assert (planner.graph_bucket(host)[1] == 1) == (plan["waves"] == 1)
+        short += plan["waves"] == 1
+    assert 0 < short < 60

@@ -805,6 +805,26 @@ def test_attention_of_items_by_few_and_by_many_waves(ops, heads, kv, hd, page, w
             assert torch.equal(many[row], few[row]), p
 
 
+@pytest.mark.parametrize("heads, kv, hd, page, window", [(16, 4, 128, 16, 1000), (6, 2, 64, 8, 390), (8, 8, 96, 4, 300)])
+def test_attention_of_cut_items_behind_a_window_by_few_and_by_many_waves(ops, heads, kv, hd, page, window):
+    """Every item that the plan gives the variant for short items leaves the same bits in both variants, wherever its window starts."""
+    from from_scratch_inference_engine_amd.parts.attention import AttentionPlanner
+
+    seqs = [(window + p, 1) for p in (0, 1, 30, 31, 32, 33, 63, 64, 95, 96)] + [(20, 1), (window // 2, 1)]
+    AttentionPlanner.compute_units = 4096  # items of 128 keys
+    try:
+        case = paged_case(seqs, heads, kv, hd, page, torch.bfloat16, seed=hd, window=window)
+    finally:
+        AttentionPlanner.compute_units = None
+    plan = case["plan"]
+    assert plan["waves"] == 1 and plan["n_merges"] >= 10
+    few, many = (run_attention(ops, dict(case, plan=dict(plan, waves=w)), heads, kv, hd, window) for w in (1, 16))
+    assert torch.equal(few, many)
+    for row, ((p, _), q, k, v) in enumerate(zip(seqs, case["qs"], case["ks"], case["vs"])):
+        ref = plain.attention(q, k, v, heads, kv, hd, query_offset=p, window=window)
+        assert (few[row:row + 1] - ref).abs().max() <= 2.0 ** -7 * ref.abs().max(), p
+
+
 @pytest.mark.parametrize("units", [4096, 8])  # items of 128 keys, one wave each, and a merge; whole requests, up to 8 waves
 @pytest.mark.parametrize("heads, kv, hd, page, window, n_parts, bias", [
     (28, 4, 128, 16, None, 8, True),   # a large model's geometry
