@@ -136,28 +136,25 @@ int launch(const StreamCall& c, hipStream_t stream) {
     return 0;
 }
 
-template <int WAVES, int NB, int RESULT, bool FRAGS>
+// LEAST: the fewest steps a wave that a plan asks for with so many waves; fewer are taken as so many (the waves past the last step
+// multiply nothing).
+template <int WAVES, int LEAST, int NB, int RESULT, bool FRAGS>
 int launch_steps(int s, const StreamCall& c, hipStream_t stream) {
-    switch (s) {
-        case 1: return launch<WAVES, 1, NB, RESULT, FRAGS>(c, stream);
-        case 2: return launch<WAVES, 2, NB, RESULT, FRAGS>(c, stream);
-        case 3: return launch<WAVES, 3, NB, RESULT, FRAGS>(c, stream);
-        case 4: return launch<WAVES, 4, NB, RESULT, FRAGS>(c, stream);
-        case 5: return launch<WAVES, 5, NB, RESULT, FRAGS>(c, stream);
-        case 6: return launch<WAVES, 6, NB, RESULT, FRAGS>(c, stream);
-        case 7: return launch<WAVES, 7, NB, RESULT, FRAGS>(c, stream);
-        default: return launch<WAVES, 8, NB, RESULT, FRAGS>(c, stream);
-    }
+    if constexpr (LEAST < kMostSteps)
+        if (s > LEAST) return launch_steps<WAVES, LEAST + 1, NB, RESULT, FRAGS>(s, c, stream);
+    return launch<WAVES, LEAST, NB, RESULT, FRAGS>(c, stream);
 }
 
-// (four waves: one block of rows, whole products; sums: eight waves on a fragment-ordered W)
+// (four waves: whole products; sums: eight waves on a fragment-ordered W.  Two blocks of rows a workgroup: of eight waves, on a
+// fragment-ordered W; what else is asked for in twos goes one by one)
 template <int RESULT, bool FRAGS>
 int launch_waves(int waves, int nb, int s, const StreamCall& c, hipStream_t stream) {
-    if (waves == 8) return nb == 2 ? launch_steps<8, 2, RESULT, FRAGS>(s, c, stream) : launch_steps<8, 1, RESULT, FRAGS>(s, c, stream);
-    if constexpr (RESULT != SUMS) {
-        if (waves == 4) return launch_steps<4, 1, RESULT, FRAGS>(s, c, stream);
-        return nb == 2 ? launch_steps<16, 2, RESULT, FRAGS>(s, c, stream) : launch_steps<16, 1, RESULT, FRAGS>(s, c, stream);
-    }
+    constexpr int LEAST = RESULT == SUMS ? 4 : 5;
+    if constexpr (FRAGS)
+        if (waves == 8 && nb == 2) return launch_steps<8, LEAST, 2, RESULT, FRAGS>(s, c, stream);
+    if (waves == 8) return launch_steps<8, LEAST, 1, RESULT, FRAGS>(s, c, stream);
+    if constexpr (RESULT != SUMS)
+        return waves == 4 ? launch_steps<4, 1, 1, RESULT, FRAGS>(s, c, stream) : launch_steps<16, LEAST, 1, RESULT, FRAGS>(s, c, stream);
     fsie_set_error("gemm_mfma_stream: sums take eight waves a workgroup");
     return 1;
 }

@@ -98,6 +98,9 @@ def test_every_plan_is_one_that_the_kernel_takes(ops):
                         assert 1 <= splits <= (16 if result == ops.GEMM_STREAM_SUMS else 1) and slice_steps * (splits - 1) < k // 32, (m, n, k, result)
                         assert waves in (4, 8, 16) and blocks in (1, 2) and -(-slice_steps // waves) <= 8, (m, n, k, result)
                         assert frags or result in (ops.GEMM_STREAM_POINT, ops.GEMM_STREAM_PLAN_ACT)
+                        # (one of the kernels that are compiled as it is, none rounded up)
+                        assert -(-slice_steps // waves) >= {4: 1, 8: 4 if result == ops.GEMM_STREAM_SUMS else 5, 16: 5}[waves], (m, n, k, result)
+                        assert blocks == 1 or (waves == 8 and frags), (m, n, k, result)
     assert min(taken.values()) > 100
     for n, k in ((256, 36864), (64, 40960)):
         x, w, exact, bound = operands(8, n, k)
