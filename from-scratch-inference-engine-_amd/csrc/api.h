@@ -92,7 +92,7 @@ int fsie_softcap(float* x, int64_t n, float cap, hipStream_t stream);
 
 // Gated linear attention over the tokens of a step, from and to the per-request state (linear_attention.hip).
 int fsie_gla_scan_shape(int heads, int dim, int vdim, int* prep_floats_per_token, int* out_planes, int* chunk_tokens,
-                        int* chunk_min, int64_t* chunk_floats);
+                        int64_t* chunk_floats);
 int fsie_gla_scan(const void* proj, int64_t proj_stride, int q_off, int k_off, int v_off, const float* z, float* state,
                   const int32_t* q_starts, const int32_t* seq_slots, int n_seqs, int n_tokens, float* prep, float* out,
                   float* chunk_work, int max_chunks, int heads, int dim, int vdim, float q_scale, float inv_tau,

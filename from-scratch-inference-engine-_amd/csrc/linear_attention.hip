@@ -29,7 +29,6 @@ constexpr int kGlaThreads = 64 * kGlaWaves;
 constexpr int kGlaCols = 64;
 constexpr int kGlaTokens = 8;  // tokens whose shares of o are added up at once
 constexpr int kGlaChunk = 16;     // tokens of a chunk
-constexpr int kGlaChunkMin = 16;  // steps of fewer tokens walk token by token
 
 // A workgroup barrier that waits for this wave's shared-memory traffic only: __syncthreads also waits for its loads and stores
 // of global memory, and the walk has both in flight at every barrier.
@@ -159,18 +158,16 @@ void gla_shape(int heads, int dim, int vdim, int* rows, int* splits) {
 }  // namespace
 
 // Sizes of the work arrays of fsie_gla_scan for a layer of these sizes: floats of `prep` a token, the planes
-// of `out` (row splits), and for the steps that go chunk by chunk the tokens of a chunk, the least tokens of such a
-// step and the floats of `chunk_work` a chunk.  A step of n_tokens tokens in n_seqs requests has at most
-// n_tokens / chunk_tokens + n_seqs chunks, and none if n_tokens < chunk_min.
+// of `out` (row splits), and for the steps that go chunk by chunk the tokens of a chunk and the floats of `chunk_work` a chunk.  A
+// step of n_tokens tokens in n_seqs requests has at most n_tokens / chunk_tokens + n_seqs chunks.
 extern "C" int fsie_gla_scan_shape(int heads, int dim, int vdim, int* prep_floats_per_token, int* out_planes,
-                                   int* chunk_tokens, int* chunk_min, int64_t* chunk_floats) {
+                                   int* chunk_tokens, int64_t* chunk_floats) {
     FSIE_REQUIRE(heads > 0 && dim > 0 && dim <= 256 && vdim > 0, "gla_scan_shape: bad sizes");
     int rows, splits;
     gla_shape(heads, dim, vdim, &rows, &splits);
     *prep_floats_per_token = 3 * heads * kGlaWaves * splits * rows;
     *out_planes = splits;
     *chunk_tokens = kGlaChunk;
-    *chunk_min = kGlaChunkMin;
     *chunk_floats = fsie_gla_chunk_floats(heads, dim, vdim);
     return 0;
 }

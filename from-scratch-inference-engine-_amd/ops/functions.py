@@ -1281,10 +1281,10 @@ def gla_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, z: torch.Te
         rot_pairs = cos_sin.shape[1]
         if tuple(cos_sin.shape) != (t, rot_pairs, 2) or 2 * rot_pairs > dim:
             raise KernelError(f"gla: cosines and sines {tuple(cos_sin.shape)} do not fit {t} tokens and heads of {dim}")
-    per_token, planes, chunk_tokens, chunk_min = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0)
+    per_token, planes, chunk_tokens = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0)
     chunk_floats = ctypes.c_int64(0)
     check(load().fsie_gla_scan_shape(heads, dim, vdim, ctypes.byref(per_token), ctypes.byref(planes),
-                                     ctypes.byref(chunk_tokens), ctypes.byref(chunk_min), ctypes.byref(chunk_floats)))
+                                     ctypes.byref(chunk_tokens), ctypes.byref(chunk_floats)))
     max_chunks = t // chunk_tokens.value + n if chunked and gla_chunked(t, n) else 0
     from_a = (None, 0, None, None, 0)
     if bottleneck is not None:
@@ -1309,7 +1309,8 @@ def gla_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, z: torch.Te
 
 def gla_chunked(tokens: int, requests: int) -> bool:
     """Whether ``gla_scan`` takes a step of so many tokens of so many requests chunk by chunk: one with a portion of a prompt (a step
-    of single tokens, as every captured decode step is, has nothing to cut into chunks) and sixteen tokens or more."""
+    of single tokens, as every captured decode step is, has nothing to cut into chunks) and sixteen tokens, a chunk, or more.  (The rule
+    stands here alone: the library goes by whether it is given a work array.)"""
     return tokens > requests and tokens >= 16
 
 

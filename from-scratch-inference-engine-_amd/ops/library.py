@@ -88,7 +88,7 @@ _SIGNATURES = {
     "fsie_sandwich_norm": ([_P, _P, _P, _P, c_float, _P, c_float, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P], c_int),
     "fsie_gated_headnorm": ([_P, c_int, _P, c_int64, _P, _P, c_int, c_int, c_int, c_float, c_int, c_int, c_int64, c_float, _P], c_int),
     "fsie_gla_scan_shape": ([c_int, c_int, c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int), ctypes.POINTER(c_int),
-                             ctypes.POINTER(c_int), ctypes.POINTER(c_int64)], c_int),
+                             ctypes.POINTER(c_int64)], c_int),
     "fsie_softcap": ([_P, c_int64, c_float, _P], c_int),
     "fsie_gla_step_takes": ([c_int, c_int, c_int, c_int], c_int),
     "fsie_gla_step": ([_P, c_int64, c_int, c_int, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, c_int, _P, _P, c_int, c_int, c_int,
