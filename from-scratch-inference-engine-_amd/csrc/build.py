@@ -26,8 +26,8 @@ LIB_NAME = "libfsie_kernels.so"
 HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature",
                "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument",
                # a kernel's first arguments (up to 16 registers of them) come with the launch instead of by a trip to memory in
-               # front of everything else: 0.1 to 0.2 us of a kernel (one request of the 0.5B shape, 48 tokens, 32.1 -> 30.9 ms;
-               # eight of the 7B shape 77.4 -> 76.4).  Structs by value are not among them.
+               # front of everything else: 0.1 to 0.2 us of a kernel (one request of the 0.5B shape, 48 tokens, 31.8 ms without,
+               # 30.1 with; eight of Gilozen 18.6 and 18.2, of 14 layers of the 7B shape 77.3 and 76.3).  Structs by value are not among them.
                "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 
 

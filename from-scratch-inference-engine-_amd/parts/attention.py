@@ -28,7 +28,7 @@ class AttentionPlanner:
     or 64 by the same rule as below); for
     the matrix-core kernel, which deals an item's keys to the waves of its workgroup and
     combines those inside, 1,024 keys, or 512, 256 or 128 while that leaves the step with at most
-    as many workgroups as the device has compute units.  Longer portions are cut into *large* tiles of ``large_tokens``; how they are
+    as many workgroups as the device has compute units, in runs that are counted from a multiple of 32 keys.  Longer portions are cut into *large* tiles of ``large_tokens``; how they are
     cut depends on the portion alone, never on what else is in the batch.  The item table lists
     the small items first.
 
@@ -101,7 +101,7 @@ class AttentionPlanner:
                 small = max(1, ops.attention_mfma_rows(self.head_dim, False) // min(group, 16))
                 rows = ops.attention_mfma_rows(self.head_dim, True)
                 large = max(1, rows // min(group, rows))
-                # at most 1,024 keys (eight waves of 128) an item
+                # at most 1,024 keys an item, 512 for heads of more than 128
                 self._geometry[mfma] = (small, large, 128 * min(8, ops.attention_mfma_max_waves(self.head_dim)))
             else:
                 t = ops.attention_tile_tokens(self.n_heads, self.n_kv)
@@ -167,8 +167,10 @@ class AttentionPlanner:
 
         def items_in(length):
             return sum(self._items_of(k, span, length) for k, span in both)
-        # the float32-arithmetic kernel takes 32 keys a pass and up to 16 heads of a group a workgroup:
-        # its items shorten to 64 keys (two passes) while compute units are idle
+        # float32 arithmetic, up to 16 heads of a group a workgroup: items shorten to 64 keys while compute units are idle.  (Lengths
+        # from the kernel on the vector units, 32 keys a pass.  The one on the matrix instruction takes 16 keys a wave, 256 at once for
+        # heads of 64; there, with 256 keys for all against these, 14 heads on 2, ms a step: 4 requests of 250 keys 1.39 / 1.34, of 180
+        # 1.32 / 1.345, 1 of 300 1.43 / 1.37, of 1,500 1.435 / 1.43, 8 of 700 1.50 / 1.51.)
         rows, shortest, room = (ops.attention_mfma_rows(self.head_dim, False), 128, 1) if mfma else (16, 64, 2)
         per_item = self.n_kv * -(-group // min(group, rows))  # workgroups of one item
         split = longest
@@ -177,8 +179,7 @@ class AttentionPlanner:
             # merge at all; the waves of its workgroup deal the keys and combine through LDS
             return longest
         # halved while the halves' workgroups still number at most the compute units: beyond that a
-        # split only adds a merge.  The float32-arithmetic kernel's workgroups are slower and several
-        # share a unit: twice the units.
+        # split only adds a merge.  Float32 arithmetic: several workgroups share a unit, twice the units.
         # (the matrix-core kernel: up to exactly one workgroup a unit)
         most_groups = units * room + (1 if mfma else 0)
         while split > shortest and items_in(split // 2) * per_item < most_groups:
@@ -256,9 +257,9 @@ class AttentionPlanner:
         return split
 
     long_items = True  # items beyond the longest of `geometry` where they still fill the device
-    # Steps of up to so many requests keep items that fit the longest whole (no merge launch).  0:
-    # never, which is faster: the one-wave item asks for all its blocks of keys at once, a wave of the
-    # many-wave workgroup for two at a time.
+    # Steps of up to so many requests keep items that fit the longest whole (no merge launch).  0: never, which is no slower: a
+    # unit draws only so much (ms a step, cut / whole: 14 layers of the 7B shape, 1 request of 400 keys 1.62 / 1.63, of 900 1.62 / 1.71,
+    # 2 of 640 1.64 / 1.68, 4 of 640 1.66 / 1.70; the 0.5B shape, 1 of 300 0.80 / 0.80, 2 of 700 0.84 / 0.87).
     whole_requests = 0
     # items shorten so that the last round of their workgroups is a full one (see split_keys)
     fill_rounds = True
