@@ -47,9 +47,74 @@ constexpr int kWhole = 16;
 __device__ __forceinline__ int segment_of(int n) { return n <= kWhole ? n : n <= 128 ? kLeastSegment : (n <= 512 ? 16 : 32); }
 constexpr int kPrepThreads = 256;
 
-__device__ __forceinline__ int chunks_of(const int32_t* q_starts, const int32_t* seq_slots, int s, int n_slots) {
-    const int len = q_starts[s + 1] - q_starts[s], slot = seq_slots[s];
+__device__ __forceinline__ int chunks_of(int len, int slot, int n_slots) {
     return (len > 0 && slot >= 0 && slot < n_slots) ? (len + kChunk - 1) / kChunk : 0;
+}
+
+// The sum over this lane and those below it, of a wave with all lanes active: within rows of sixteen, then over the rows.
+__device__ __forceinline__ int sum_up_to_lane(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // from one lane below, two, four, eight; zero beyond the row
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // rows 1 and 3: the last lane of the row before
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // rows 2 and 3: lane 31
+    return v;
+}
+
+// The requests' portions laid out one after the other, entries(chunks) places each: the request that has a place.
+struct Place {
+    int seq;     // -1: none
+    int chunks;  // of its portion
+    int before;  // places of the requests before it
+    int first;   // and their chunks
+};
+
+// Every wave for itself, all lanes active, the result the same for all lanes.  More than a few requests are read four a lane and added up
+// by lanes: one after the other, in every workgroup of both kernels, a step in which 255 requests decode beside a portion of two
+// tokens took 960 us a layer of 8 heads of 128 x 256.
+template <typename Entries>
+__device__ __forceinline__ Place place_of(int place, const int32_t* __restrict__ q_starts, const int32_t* __restrict__ seq_slots, int n_seqs,
+                                          int n_slots, Entries entries) {
+    constexpr int kSerial = 8, kEach = 4;
+    int before = 0, first = 0;
+    if (n_seqs <= kSerial) {
+        for (int s = 0; s < n_seqs; ++s) {
+            const int chunks = chunks_of(q_starts[s + 1] - q_starts[s], seq_slots[s], n_slots), here = entries(chunks);
+            if (place < before + here) return Place{s, chunks, before, first};
+            before += here, first += chunks;
+        }
+        return Place{-1, 0, 0, 0};
+    }
+    const int lane = threadIdx.x & 63;
+    for (int s0 = 0; s0 < n_seqs; s0 += 64 * kEach) {
+        int starts[kEach + 1], slots[kEach], chunks[kEach], places = 0, sum = 0;
+#pragma unroll
+        for (int i = 0; i <= kEach; ++i) starts[i] = q_starts[min(s0 + lane * kEach + i, n_seqs)];
+#pragma unroll
+        for (int i = 0; i < kEach; ++i) slots[i] = seq_slots[min(s0 + lane * kEach + i, n_seqs - 1)];
+#pragma unroll
+        for (int i = 0; i < kEach; ++i) {  // (past the last request: no tokens)
+            chunks[i] = chunks_of(starts[i + 1] - starts[i], slots[i], n_slots);
+            places += entries(chunks[i]), sum += chunks[i];
+        }
+        const int places_to = sum_up_to_lane(places), sum_to = sum_up_to_lane(sum);
+        const uint64_t beyond = __ballot(place < before + places_to);
+        if (beyond) {
+            const int at = __builtin_ctzll(beyond);  // the lane that has the request
+            before += __builtin_amdgcn_readlane(places_to - places, at), first += __builtin_amdgcn_readlane(sum_to - sum, at);
+            Place found{-1, 0, 0, 0};
+#pragma unroll
+            for (int i = 0; i < kEach; ++i) {
+                const int n = __builtin_amdgcn_readlane(chunks[i], at), here = entries(n);
+                if (found.seq < 0 && place < before + here) found = Place{s0 + at * kEach + i, n, before, first};
+                before += here, first += n;
+            }
+            return found;
+        }
+        before += __builtin_amdgcn_readlane(places_to, 63), first += __builtin_amdgcn_readlane(sum_to, 63);
+    }
+    return Place{-1, 0, 0, 0};
 }
 
 // Work array of one chunk and head, each operand as the lanes 16 g + n of a wave read it, four floats a lane: q * exp(B_t)
@@ -100,12 +165,8 @@ __global__ __launch_bounds__(kPrepThreads) void gla_chunk_prep_kernel(
     constexpr int LD = DP + 4, PER = kChunk * DP / kPrepThreads;
     __shared__ __attribute__((aligned(16))) float qs[kChunk * LD], ks[kChunk * LD], bs[kChunk * LD];
     const int h = blockIdx.x, chunk = blockIdx.y, tid = threadIdx.x;
-    int first = 0, seq = -1;
-    for (int s = 0; s < n_seqs; ++s) {
-        const int n = chunks_of(q_starts, seq_slots, s, n_slots);
-        if (chunk < first + n) { seq = s; break; }
-        first += n;
-    }
+    const Place at = place_of(chunk, q_starts, seq_slots, n_seqs, n_slots, [](int chunks) { return chunks; });
+    const int seq = at.seq, first = at.first;
     if (seq < 0) return;  // the same for the whole workgroup
     const int t0 = q_starts[seq] + (chunk - first) * kChunk;
     const int nt = min(kChunk, q_starts[seq + 1] - t0);
@@ -320,16 +381,11 @@ __global__ __launch_bounds__(256 * HALVES, 2) void gla_segment_kernel(
     const bool tile_ok = tile0 + column < tiles;  // (waves past the last tile repeat it and write nothing)
     const bool col_ok = tile_ok && col < vdim;
     // the request and the segment
-    int first = 0, before = 0, seq = -1, seg = 0, n_chunks = 0;
-    for (int s = 0; s < n_seqs; ++s) {
-        const int chunks = chunks_of(q_starts, seq_slots, s, n_slots), len = max(1, segment_of(chunks));
-        const int segs = (chunks + len - 1) / len, here = LATER ? max(0, segs - 1) : (segs > 1 ? segs - 1 : segs);
-        if (place < before + here) {
-            seq = s, seg = place - before + (LATER ? 1 : 0), n_chunks = chunks;
-            break;
-        }
-        before += here, first += chunks;
-    }
+    const Place at = place_of(place, q_starts, seq_slots, n_seqs, n_slots, [](int chunks) {
+        const int len = max(1, segment_of(chunks)), segs = (chunks + len - 1) / len;
+        return LATER ? max(0, segs - 1) : (segs > 1 ? segs - 1 : segs);
+    });
+    const int seq = at.seq, seg = place - at.before + (LATER ? 1 : 0), n_chunks = at.chunks, first = at.first;
     if (seq < 0) return;  // the same for the whole workgroup
     const int length = segment_of(n_chunks), begin = seg * length, end = min(n_chunks, begin + length);
     const bool last = end == n_chunks;
@@ -350,9 +406,9 @@ __global__ __launch_bounds__(256 * HALVES, 2) void gla_segment_kernel(
     u32x4 rsrc;
     uint32_t to;
     auto bring_from = [&](int ci, int stage) {
-        const uint64_t at = reinterpret_cast<uint64_t>(w + min(ci, end - 1) * per_chunk);
-        rsrc[0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at));
-        rsrc[1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at >> 32));
+        const uint64_t from_w = reinterpret_cast<uint64_t>(w + min(ci, end - 1) * per_chunk);
+        rsrc[0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(from_w));
+        rsrc[1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(from_w >> 32));
         rsrc[2] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(chunk_floats_of(DP, vdim) * 4));
         rsrc[3] = 0x00020000u;
         to = lds0 + static_cast<uint32_t>(stage) * (St::kFloats * 4) + wave * St::kLoads * 1024u;

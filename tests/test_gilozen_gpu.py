@@ -298,6 +298,32 @@ def test_gla_scan_makes_the_decays_from_the_bottleneck(ops, heads, dim, vdim, ra
                      bottleneck=(a[:4], a2, bias))
 
 
+@pytest.mark.parametrize("n", [8, 9, 63, 64, 65, 255, 256, 257, 700])
+def test_gla_scan_finds_the_portions_of_many_requests(ops, n):
+    """Single tokens, short portions, portions of one segment and of several in any order, requests without a slot among them, the last
+    one's portion long and short: against the walk token by token."""
+    heads, dim, vdim = 2, 16, 20
+    for last in (1, 300):
+        rng = np.random.RandomState(n + last)
+        lens = rng.choice([1, 1, 1, 1, 2, 15, 16, 17, 40], n)
+        lens[rng.choice(n, 3, replace=False)] = [257, 600, 256]
+        lens[-1] = last
+        t, kw, vw = int(lens.sum()), heads * dim, heads * vdim
+        slots = np.where(rng.rand(n) < 0.1, -1, rng.permutation(n + 3)[:n]).astype(np.int32)
+        proj, z = rnd((t, 2 * kw + vw), n).cuda(), rnd((t, kw), n + 1, 2.0).cuda()
+        starts = np.cumsum([0] + list(lens)).astype(np.int32)
+        outs, states = [], []
+        for chunked in (True, False):
+            state = rnd((n + 3, heads, dim, vdim), 9).cuda()
+            outs.append(ops.gla_scan(proj, 0, kw, 2 * kw, z, state, torch.from_numpy(starts).cuda(), torch.from_numpy(slots).cuda(), heads, dim,
+                                     vdim, dim ** -0.5, 0.5, chunked=chunked).sum(0).cpu())
+            states.append(state.cpu())
+        rows = torch.cat([torch.arange(a, b) for a, b, s in zip(starts, starts[1:], slots) if s >= 0])
+        off = (outs[0][rows] - outs[1][rows]).norm(dim=1) / outs[1][rows].norm(dim=1)
+        assert off.max() <= 1e-4 and rel(outs[0][rows], outs[1][rows].double()) <= 2e-5  # (a row by itself may cancel)
+        assert (states[0] - states[1]).abs().max() <= 2e-5 * states[1].abs().max()
+
+
 @pytest.mark.parametrize("heads, dim, vdim", [(2, 96, 72), (1, 200, 40)])
 def test_decays_from_the_bottleneck_in_segments(ops, heads, dim, vdim):
     """Portions of several segments and a single token: against the walk token by token with the decays' logits made in 64 bits."""
