@@ -1308,10 +1308,13 @@ def gla_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, z: torch.Te
 
 
 def gla_chunked(tokens: int, requests: int) -> bool:
-    """Whether ``gla_scan`` takes a step of so many tokens of so many requests chunk by chunk: one with a portion of a prompt (a step
-    of single tokens, as every captured decode step is, has nothing to cut into chunks) and sixteen tokens, a chunk, or more.  (The rule
-    stands here alone: the library goes by whether it is given a work array.)"""
-    return tokens > requests and tokens >= 16
+    """Whether ``gla_scan`` takes a step of so many tokens of so many requests chunk by chunk: one of sixteen tokens, a chunk, and more in
+    which a portion may be longer than eight.  (The rule stands here alone: the library goes by whether it is given a work array.)
+
+    Scan and heads' norm, us, chunks / token by token, heads of 128 x 256 (8) and 256 x 256 (2): 30 single tokens and a portion of 2
+    31.8 / 25.9 and 26.3 / 17.3, of 15 31.8 / 31.1 and 26.4 / 22.3, of 24 33.3 / 34.5 and 28.7 / 25.2; 63 and one of 15 52 / 75 and
+    40 / 44; 8 and one of 8 20.0 / 16.8 and 22.5 / 14.1."""
+    return tokens >= 16 and tokens - requests >= 8
 
 
 def gla_step_takes(heads: int, dim: int, vdim: int, rank: int) -> bool:

@@ -324,6 +324,11 @@ def test_gla_scan_finds_the_portions_of_many_requests(ops, n):
         assert (states[0] - states[1]).abs().max() <= 2e-5 * states[1].abs().max()
 
 
+def test_steps_of_short_portions_go_token_by_token(ops):
+    assert not ops.gla_chunked(4, 4) and not ops.gla_chunked(15, 1) and not ops.gla_chunked(64, 64) and not ops.gla_chunked(70, 63)
+    assert ops.gla_chunked(16, 1) and ops.gla_chunked(71, 63) and ops.gla_chunked(512, 256)
+
+
 @pytest.mark.parametrize("heads, dim, vdim", [(2, 96, 72), (1, 200, 40)])
 def test_decays_from_the_bottleneck_in_segments(ops, heads, dim, vdim):
     """Portions of several segments and a single token: against the walk token by token with the decays' logits made in 64 bits."""
