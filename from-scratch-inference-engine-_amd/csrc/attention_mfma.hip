@@ -27,7 +27,8 @@ extern "C" int fsie_attention_mfma_tiles(int head_dim, int large) {
 
 // bfloat16 only; head_dim a multiple of 16 up to 256; page_size a multiple of 4.
 // large = 0: items of at most 16 rows (tokens x heads of a group); large = 1: up to 16 * tiles rows.
-// `waves` waves of a workgroup split each item's keys (at most 4 for large items).
+// waves: of a workgroup, that split each item's keys.  large = 0: 1, the variant for items of up to four blocks of 32 keys; 0, the same for
+// any items, where more workgroups than units share the memory's rate; more, as many as the head size has.  large = 1: at most 4.
 // slopes [n_heads] (or null): slopes[h] * (query position - key position) is taken off head h's scores, after the cap;
 // row_scale (or null): a factor a token (indexed like the rows of q) on its scores, before the cap.
 extern "C" int fsie_attention_mfma(const void* q, int64_t q_stride, const void* k_pool, const void* v_pool,

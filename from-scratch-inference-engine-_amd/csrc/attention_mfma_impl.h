@@ -30,7 +30,8 @@
 // waves' results meet in LDS, in the fixed order of the waves, behind one barrier.  Decoding against a long context needs
 // neither partial records in memory nor a second kernel, and the result does not depend on timing.
 // Such a step is bound by the chain inside a workgroup: the item, the block table, the keys, one trip to memory each, then
-// products and exponentials that wait for each other.  So no wave takes two blocks where another has none, masks are selects (no
+// products and exponentials that wait for each other.  So no wave takes two blocks where another has none (unless the workgroups are
+// more than the units anyway, where the memory's rate bounds it and fewer waves a workgroup keep more of them under way), masks are selects (no
 // branch a value), and little code is run once: 10 KB of instructions, not 31.  One request of the 0.5B shape and 60 to 110
 // keys 7.2 -> 4.5 us from a workgroup's first instruction to its last, eight of the 7B shape and 64 to 550 6.6 -> 5.0.
 // Several query tiles (NT > 1, up to 4 waves): a wave per 512 keys, combined by the first wave.
@@ -141,7 +142,9 @@ constexpr int kShortWaves = 4;
 
 // BIASED false: no distance bias and no factor a token, known when the kernel is compiled (the QKV variants have no
 // registers to spare for them); true: whatever slopes and row_scale say.
-template <int HDT, int NT, int MAXW, bool V16, bool QKV = false, bool BIASED = true>
+// ONCE: values by streaming loads: where several waves walk long runs of keys, and where more workgroups than units read more than
+// the caches hold; the short items of a few workgroups are slower with them.
+template <int HDT, int NT, int MAXW, bool V16, bool QKV = false, bool BIASED = true, bool ONCE = (MAXW > kShortWaves + 1)>
 __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW == 1 && NT > 1 ? 2 : 1))) void attention_mfma_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_pool,
     const bf16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_pages,
@@ -332,8 +335,8 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
     const int walk_first = kb_first - pre_len;
     const int n_blocks = ((key_end - kb_first + 31) >> 5) + (pre_len >> 5);
     // One query tile: an item's blocks are dealt to as many waves as it has blocks, up to what the head size allows, in runs
-    // of equal length; several tiles: a wave per 16 blocks (512 keys).  How its keys are split depends on the item alone: the
-    // variant for short items has fewer waves, but only where every one of them has a block of its own either way.
+    // of equal length; several tiles: a wave per 16 blocks (512 keys).  By the items' lengths the variant for short items is taken only where
+    // every wave has a block of its own either way: then how an item's keys are split depends on the item alone.
     constexpr int kKeyWaves = QKV && MAXW == kShortWaves + 1 ? kShortWaves : MAXW;
     const int n_run_of = NT == 1 ? (n_blocks + kKeyWaves - 1) / kKeyWaves : 0;
     const int n_active = NT == 1 ? max(1, n_run_of > 0 ? (n_blocks + n_run_of - 1) / n_run_of : 1) : min(n_waves, max(1, (n_blocks + 15) / 16));
@@ -409,9 +412,8 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
         if (V16) {
 #pragma unroll
             for (int dt = 0; dt < HDT; ++dt) {
-                // (streaming loads where several waves walk long runs of keys; the short items of one wave are slower with them)
                 const bf16_t* vp = v0 + static_cast<int64_t>(dt * 16) * page_size;
-                blk.vf[dt].raw = MAXW > kShortWaves + 1 ? ld16_once(vp) : ld16(vp);
+                blk.vf[dt].raw = ONCE ? ld16_once(vp) : ld16(vp);
             }
         } else {
             const bf16_t* v1 = v_pool + at.v[RUN - 1];
@@ -811,19 +813,23 @@ int launch(const void* q, int64_t q_stride, const void* k_pool, const void* v_po
     const dim3 grid(n_items, n_kv, head_chunks);
     scores.group = group;
     scores.page_magic = magic_of(page_size);
+    const bool few = waves == 0;  // (one tile: the variant for short items whatever their length, values by streaming loads)
     if (waves < 1) waves = 1;
     if (waves > MAXW) waves = MAXW;
     // Several query tiles: a launch of one wave per workgroup takes the instantiation without the LDS of the
     // combination, which would otherwise limit how many workgroups a compute unit holds.  One: the variant for short items,
     // or all the waves the kernel has
-#define FSIE_ATTN_LAUNCH(W, THREADS, V)                                                                              \
-    attention_mfma_kernel<HDT, NT, W, V><<<grid, THREADS, 0, stream>>>(                                              \
+#define FSIE_ATTN_LAUNCH(W, THREADS, V) FSIE_ATTN_LAUNCH_ONCE(W, THREADS, V, (W > kShortWaves + 1))
+#define FSIE_ATTN_LAUNCH_ONCE(W, THREADS, V, ONCE)                                                                   \
+    attention_mfma_kernel<HDT, NT, W, V, false, true, ONCE><<<grid, THREADS, 0, stream>>>(                                              \
         static_cast<const bf16_t*>(q), q_stride, static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool), \
         block_tables, max_pages, items, static_cast<bf16_t*>(out), partials, n_heads, n_kv, page_size, window, scale, \
         gh, scores)
     const bool v16 = page_size % 8 == 0;
     if constexpr (NT == 1) {
-        if (waves == 1) {
+        if (few && v16 && HDT <= 8) {  // (wider heads have this many waves and no more)
+            FSIE_ATTN_LAUNCH_ONCE(kShortWaves, 64 * kShortWaves, true, (HDT <= 8));
+        } else if (waves == 1) {
             if (v16) FSIE_ATTN_LAUNCH(kShortWaves, 64 * kShortWaves, true);
             else FSIE_ATTN_LAUNCH(kShortWaves, 64 * kShortWaves, false);
         } else {
@@ -838,6 +844,7 @@ int launch(const void* q, int64_t q_stride, const void* k_pool, const void* v_po
         else FSIE_ATTN_LAUNCH(MAXW, 64 * waves, false);
     }
 #undef FSIE_ATTN_LAUNCH
+#undef FSIE_ATTN_LAUNCH_ONCE
     FSIE_CHECK_LAUNCH("attention_mfma");
     return 0;
 }

@@ -953,7 +953,9 @@ def attention_mfma(q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_pool:
                    row_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Attention of the work items over the paged cache on the matrix cores (bfloat16; head_dim a
     multiple of 16; page size a multiple of 4).  ``items`` may be a view into a longer table.
-    ``waves`` waves of a workgroup split each item's keys and combine inside the workgroup."""
+    The waves of a workgroup split each item's keys and combine inside the workgroup: without ``large`` four where ``waves`` is 1 (items
+    of up to four blocks of 32 keys) or 0 (any items, where their workgroups are more than the compute units), else as many as the head size
+    has; with ``large`` so many, at most four."""
     if not q.is_cuda or q.dtype != torch.bfloat16:
         raise KernelError("attention_mfma q: must be bfloat16 on the GPU")
     _need(k_pool, "k_pool", dtype=q.dtype, ndim=4)

@@ -131,6 +131,18 @@ class AttentionPlanner:
 
     short_waves = 4  # waves of the variant for short items
 
+    def _fills(self, items: int) -> bool:
+        """Whether the matrix-core kernel's workgroups for so many items are more than the compute units.  Queries that are in memory
+        already then go to the variant for short items whatever their length: all the waves of a head size hold so much of a unit that the
+        workgroups go one or two at a time, and what counts is the memory's rate.  Decode attention over keys that no cache holds, us, before items'
+        blocks were dealt to waves / all waves / this: 28 heads on 4 of 128, 200 requests of 300 keys 32.7 / 38.2 / 29.4, of 1,000 99 / 87 / 80;
+        16 on 16 of 64, 64 of 40 8.1 / 14.4 / 6.3, 200 of 500 82 / 98 / 71; 32 on 4 of 32, 200 of 300 12.7 / 17.8 / 10.1.  At as many workgroups
+        as units all waves are faster from 500 keys on (14 on 2 of 64, 128 of 1,000 16.0 / 19.5).  Where attention adds up q/k/v itself, too (64 of 3,000
+        keys, 8 on 8 of 128, 134 / 141)."""
+        units = self.compute_units if self.compute_units is not None else ops.compute_units()
+        group = self.n_heads // self.n_kv
+        return items * self.n_kv * -(-group // min(group, ops.attention_mfma_rows(self.head_dim, False))) > units > 0
+
     def _cut_from(self, first: int, mfma: bool) -> int:
         """Where the runs that a portion's keys are cut into are counted from: the matrix-core kernel takes blocks of 32 keys from a
         multiple of 32 on, so runs from a window's first key would have a block more each than their keys are."""
@@ -274,7 +286,7 @@ class AttentionPlanner:
 
     def graph_bucket(self, host):
         """What a captured graph of this step's shape must fix: the number of (small) work items,
-        the variant of the matrix-core kernel and (of the other one) the keys per item; None if the step has portions that do not fit
+        the variant of the matrix-core kernel, whether its workgroups fill the units and (of the other kernel) the keys per item; None if the step has portions that do not fit
         small items."""
         mfma = self.uses_mfma(host.compute_dtype, host.page_size)
         small_tokens = self.geometry(mfma)[0]
@@ -300,7 +312,7 @@ class AttentionPlanner:
             # every request is one whole item: no records, no merge.  A graph of its own: the merge that finds nothing to do costs
             # 1.5 us a layer (one request of the 0.5B shape, 61 tokens and 48 more, 37.3 ms, 35.5 without), the step from whole
             # to cut items one capture more in a batch's life
-            return (n, self._graph_waves(longest) if mfma else 1, 0 if mfma else split_keys)
+            return (n, self._graph_waves(longest) if mfma else 1, self._fills(n) if mfma else split_keys)
         if mfma:
             # items: a multiple of the number of requests and of a quarter of what gives every unit a
             # workgroup, so that one graph serves a batch while its requests grow: their items grow
@@ -310,7 +322,7 @@ class AttentionPlanner:
             group = self.n_heads // self.n_kv
             per_item = self.n_kv * -(-group // min(group, ops.attention_mfma_rows(self.head_dim, False)))
             step = max(host.n_seqs, units // per_item // 4, 1)
-            return (-(-n // step) * step, self._graph_waves(longest), 0)
+            return (-(-n // step) * step, self._graph_waves(longest), self._fills(n))
         step = host.n_seqs * max(1, 1024 // split_keys)
         return (-(-n // step) * step, 1, split_keys)
 
@@ -411,8 +423,9 @@ class AttentionPlanner:
                     if len(run):
                         large_runs.append(run)
         large = np.concatenate(large_runs) if large_runs else np.zeros((0, ATTN_ITEM_INTS), dtype=np.int64)
-        waves = 1
+        waves, fills = 1, False
         if mfma and small:
+            fills = self._fills(len(small))
             # (in blocks of 32 keys, those of the kept first ones too: the variant for short items has four waves and takes four
             # blocks, so that how an item's keys are dealt to waves is the same in either variant)
             waves = self._waves_for(max(it[5] - (it[4] & ~31) + (32 * -(-min(it[7] & ~(ATTN_KEEP_WALK | ATTN_POOL_WALK), it[4]) // 32)
@@ -420,7 +433,7 @@ class AttentionPlanner:
                                     ops.attention_mfma_max_waves(self.head_dim))
         if padded:
             # a captured graph launches fixed grids: pad with items and merges that do nothing
-            n_items, waves, _ = host.pad[self.key]
+            n_items, waves, fills = host.pad[self.key]
             if len(large) or len(small) > n_items:
                 raise RuntimeError("attention plan does not fit the captured graph")
             small += [(0, 0, 0, 0, 0, 0, -1, 0)] * (n_items - len(small))
@@ -479,7 +492,7 @@ class AttentionPlanner:
             "groups": groups.astype(np.int32), "n_groups": len(groups),
             "n_small": len(small), "n_large": len(large) - n_long, "n_long": n_long, "long_waves": long_waves,
             "n_merges": len(merges) + sum(len(m) for m in merge_runs),
-            "n_partial": n_partial, "mfma": mfma, "waves": waves,
+            "n_partial": n_partial, "mfma": mfma, "waves": waves, "fills": bool(mfma and fills),
             "single": all(host.q_lens[s] == 1 for s in range(host.n_seqs)),  # one token a request
         }
 
@@ -510,7 +523,8 @@ def paged_attention(q: torch.Tensor, q_stride: int, cache, plan, n_heads: int, n
     if plan.mfma:
         if plan.n_small:
             ops.attention_mfma(q, q_stride, cache.k_pool, cache.v_pool, cache.block_tables, plan.items,
-                               plan.n_small, out, *args, large=False, waves=plan.waves, sinks=sinks, softcap=cap, **bias)
+                               plan.n_small, out, *args, large=False, waves=0 if getattr(plan, "fills", False) else plan.waves,
+                               sinks=sinks, softcap=cap, **bias)
         if (plan.n_large and (not plan.n_long or getattr(plan, "long_waves", 4) == 1) and share_keys
                 and ops.attention_mfma_lds_ok(head_dim, cache.page_size)):
             ops.attention_mfma_lds(q, q_stride, cache.k_pool, cache.v_pool, cache.block_tables,

@@ -268,3 +268,18 @@ def test_short_items_are_four_blocks_of_keys_wherever_a_window_starts(args):
         assert (planner.graph_bucket(host)[1] == 1) == (plan["waves"] == 1)
         short += plan["waves"] == 1
     assert 0 < short < 60
+
+
+@pytest.mark.parametrize("heads, kv, n, keys, fills", [(28, 4, 64, 300, False), (28, 4, 65, 300, True), (28, 4, 200, 90, True), (16, 16, 16, 100, False),
+                                                       (16, 16, 17, 100, True), (40, 1, 85, 50, False), (40, 1, 86, 50, True), (28, 4, 8, 3000, False)])
+def test_more_workgroups_than_units(heads, kv, n, keys, fills):
+    """The plan says so by the step's own items, a graph's plan by its bucket: 64 items of 4 kv heads are as many workgroups as units."""
+    planner = AttentionPlanner(heads, kv, 128, None)
+    planner.compute_units = 256
+    host = Host([(keys - 1, 1)] * n, 16, torch.bfloat16)
+    assert planner.plan(host)["fills"] == fills
+    bucket = planner.graph_bucket(host)
+    assert bool(bucket[2]) == fills
+    host.pad = {planner.key: bucket}
+    assert planner.plan(host)["fills"] == fills
+    assert not planner.plan(Host([(keys - 1, 1)] * n, 16, torch.float32))["fills"]

@@ -796,6 +796,7 @@ def test_attention_of_items_by_few_and_by_many_waves(ops, heads, kv, hd, page, w
     assert not plan["n_merges"] and plan["n_small"] == len(seqs)
     many = run_attention(ops, dict(case, plan=dict(plan, waves=16)), heads, kv, hd, window)
     few = run_attention(ops, dict(case, plan=dict(plan, waves=1)), heads, kv, hd, window)
+    assert torch.equal(few, run_attention(ops, dict(case, plan=dict(plan, waves=0)), heads, kv, hd, window))  # (streaming loads only)
     for row, ((p, _), q, k, v) in enumerate(zip(seqs, case["qs"], case["ks"], case["vs"])):
         ref = plain.attention(q, k, v, heads, kv, hd, query_offset=p, window=window)
         for out in (many, few):
@@ -818,8 +819,8 @@ def test_attention_of_cut_items_behind_a_window_by_few_and_by_many_waves(ops, he
         AttentionPlanner.compute_units = None
     plan = case["plan"]
     assert plan["waves"] == 1 and plan["n_merges"] >= 10
-    few, many = (run_attention(ops, dict(case, plan=dict(plan, waves=w)), heads, kv, hd, window) for w in (1, 16))
-    assert torch.equal(few, many)
+    few, many, fills = (run_attention(ops, dict(case, plan=dict(plan, waves=w)), heads, kv, hd, window) for w in (1, 16, 0))
+    assert torch.equal(few, many) and torch.equal(few, fills)
     for row, ((p, _), q, k, v) in enumerate(zip(seqs, case["qs"], case["ks"], case["vs"])):
         ref = plain.attention(q, k, v, heads, kv, hd, query_offset=p, window=window)
         assert (few[row:row + 1] - ref).abs().max() <= 2.0 ** -7 * ref.abs().max(), p
