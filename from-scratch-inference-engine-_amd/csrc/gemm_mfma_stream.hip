@@ -170,7 +170,8 @@ int launch_waves(int waves, int nb, int s, const StreamCall& c, hipStream_t stre
 // the kernel that shares X 11.3, 11.1, 11.1; N = 22016, K = 2048, two rows 16.8 / 16.5), below it not more than two workgroups a unit
 // for nine rows and more (N = 11264, K = 1024, 16 rows 7.9 / 7.4); an activation beyond 64 MB up to four rows (N = 14336,
 // K = 4096, four 23.5 / 23.4, eight 25.9 / 23.3).  Rows of W that are no copy up to a workgroup a unit (against the few-rows kernel,
-// 8 rows, N = 2048, K = 1280 4.6 / 5.2, N = 1552, K = 2048 5.6 / 6.1, N = 4096, K = 896 4.2 / 5.0).
+// 8 rows, N = 2048, K = 1280 4.6 / 5.2, N = 1552, K = 2048 5.6 / 6.1, N = 4096, K = 896 4.2 / 5.0), beyond 28 MB up to eight rows
+// (N = K = 4096, eight 10.4 / 11.1, 13 11.9 / 11.2, 16 12.6 / 11.5; N = K = 3584, 16 9.6 / 10.2).
 // Sums: the fewest slices that a workgroup of eight waves holds, then as many more as leave a wave four steps and the workgroups
 // no more than the units: a second round costs what it hides (N = 4608, K = 3584 8.1 us against 7.0 in seven slices), and the
 // norm pays for every slice.
@@ -198,7 +199,7 @@ extern "C" int fsie_gemm_mfma_stream_plan(int M, int N, int K, int result, int f
     constexpr int64_t MB = 1024 * 1024;
     if (result == GATED && (!frags || (bytes > 24 * MB && (M > 2 || bytes > 72 * MB)) || (M > 8 && groups > 2 * units))) return -1;
     if (result == kPlanActivation && frags && M > 4 && bytes > 64 * MB) return -1;
-    if (result != GATED && !frags && groups > units) return -1;
+    if (result != GATED && !frags && (groups > units || (M > 8 && bytes > 28 * MB))) return -1;
     return waves + 256 * blocks + 65536;
 }
 

@@ -78,6 +78,15 @@ def test_what_the_plan_takes(ops):
         ops.gemm_mfma_stream(x, torch.zeros((8, 100), dtype=torch.bfloat16, device="cuda"), ops.GEMM_STREAM_POINT, 4 + 256 + 65536)
 
 
+def test_the_largest_weights_in_rows_take_up_to_eight_rows(ops):
+    if ops.compute_units() != 256:
+        pytest.skip("the figures are those of 256 units")
+    plan = ops.gemm_stream_plan
+    for result in (ops.GEMM_STREAM_POINT, ops.GEMM_STREAM_PLAN_ACT):
+        assert plan(8, 4096, 4096, result, False) and plan(9, 4096, 4096, result, False) is None
+        assert plan(16, 3584, 3584, result, False) and plan(16, 4096, 4096, result, True)
+
+
 def test_every_plan_is_one_that_the_kernel_takes(ops):
     """Over sizes of all kinds, K beyond what sixteen slices hold among them: the checks of the launch itself, and the residual
     projections of such sizes."""
