@@ -16,6 +16,8 @@
 // this one: 4 requests of 300 keys, 14 heads on 2 of 64 12.1 / 8.3, 28 on 4 of 128 16.9 / 8.6, 16 on 1 of 256 35.0 / 12.5; one
 // of 100 keys 15.1 / 6.9, 23.1 / 7.7, 54 / 13.8; 32 of 700 20.7 / 15.3, 56 / 26, 48 / 24; a prompt of 300 tokens 49 / 16, 88 / 29,
 // 130 / 37, of 1,000 185 / 59, 537 / 155, 636 / 203.
+//
+// More workgroups than units: four waves each whatever the head size (see launch).
 #include "common.h"
 #include "api.h"
 
@@ -43,13 +45,13 @@ struct F32Call {
     const float *sinks, *slopes, *row_scale;
 };
 
-template <int HDT>
-__global__ __launch_bounds__(64 * f32_waves<HDT>()) void attention_f32_kernel(
+template <int HDT, int W>
+__global__ __launch_bounds__(64 * W) void attention_f32_kernel(
     const int32_t* __restrict__ items, const int32_t* __restrict__ block_tables, int max_pages, int page_size, uint32_t page_magic,
     int n_kv, const float* __restrict__ k_pool, const float* __restrict__ v_pool, const float* __restrict__ q, int64_t q_stride,
     float* __restrict__ out, float* __restrict__ partials, int n_heads, int group, int gh, int window, float scale, float softcap,
     const float* __restrict__ sinks, const float* __restrict__ slopes, const float* __restrict__ row_scale) {
-    constexpr int HD = HDT * 16, W = f32_waves<HDT>(), MW = (W + 3) / 4 * 4;
+    constexpr int HD = HDT * 16, MW = (W + 3) / 4 * 4;
     __shared__ floatx4 s_o[W * HDT * 64];
     __shared__ float s_m[16][MW + 4], s_l[16][MW + 4];  // [column][wave]: a lane reads its column's waves four at a time
 
@@ -120,7 +122,7 @@ __global__ __launch_bounds__(64 * f32_waves<HDT>()) void attention_f32_kernel(
     const bool row_ok = tq < n_q && hh < gh_here;
     const int head = h_base + (row_ok ? hh : 0), row = q_row0 + (row_ok ? tq : 0), pos = pos0 + tq;
     floatx4 qf[HDT];
-    {
+    if (W < 16 || any) {  // (of sixteen waves most have no key where items are short, and read nothing; eight are slower with the question)
         const float* qp = q + static_cast<int64_t>(row) * q_stride + static_cast<int64_t>(head) * HD + 4 * G;
 #pragma unroll
         for (int j = 0; j < HDT; ++j) qf[j] = *reinterpret_cast<const floatx4*>(qp + 16 * j);
@@ -205,6 +207,11 @@ __global__ __launch_bounds__(64 * f32_waves<HDT>()) void attention_f32_kernel(
     float m_of_run[MW], l_of_run[MW], factor[MW];
 #pragma unroll
     for (int w = 0; w < MW; w += 4) {
+        if (W == 16 && w >= n_runs) {  // (the same for the whole workgroup, as below; what is left out adds zeros)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) m_of_run[w + i] = -INFINITY, l_of_run[w + i] = 0.f;
+            continue;
+        }
         const floatx4 m4 = *reinterpret_cast<const floatx4*>(&s_m[c][w]), l4 = *reinterpret_cast<const floatx4*>(&s_l[c][w]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -219,9 +226,13 @@ __global__ __launch_bounds__(64 * f32_waves<HDT>()) void attention_f32_kernel(
     const float m_of = m_all == -INFINITY ? 0.f : m_all;
     float denom = 0.f;
 #pragma unroll
-    for (int w = 0; w < MW; ++w) {
-        factor[w] = expf(m_of_run[w] - m_of);
-        denom = fmaf(l_of_run[w], factor[w], denom);
+    for (int w0 = 0; w0 < MW; w0 += 4) {
+        if (W == 16 && w0 >= n_runs) break;
+#pragma unroll
+        for (int w = w0; w < w0 + 4; ++w) {
+            factor[w] = expf(m_of_run[w] - m_of);
+            denom = fmaf(l_of_run[w], factor[w], denom);
+        }
     }
     float inv = 1.f;
     if (partial_base < 0) {
@@ -258,14 +269,25 @@ __global__ __launch_bounds__(64 * f32_waves<HDT>()) void attention_f32_kernel(
     }
 }
 
+template <int HDT, int W>
+void launch_waves(const F32Call& a, dim3 grid, int group, int gh, hipStream_t stream) {
+    attention_f32_kernel<HDT, W><<<grid, 64 * W, 0, stream>>>(
+        a.items, a.block_tables, a.max_pages, a.page_size, 0xFFFFFFFFu / static_cast<uint32_t>(a.page_size) + 1u, a.n_kv, a.k_pool,
+        a.v_pool, a.q, a.q_stride, a.out, a.partials, a.n_heads, group, gh, a.window, a.scale, a.softcap, a.sinks, a.slopes,
+        a.row_scale);
+}
+
 template <int HDT>
 int launch(const F32Call& a, hipStream_t stream) {
     const int group = a.n_heads / a.n_kv, gh = group < 16 ? group : 16;
     const dim3 grid(a.n_items, a.n_kv, (group + gh - 1) / gh);
-    attention_f32_kernel<HDT><<<grid, 64 * f32_waves<HDT>(), 0, stream>>>(
-        a.items, a.block_tables, a.max_pages, a.page_size, 0xFFFFFFFFu / static_cast<uint32_t>(a.page_size) + 1u, a.n_kv, a.k_pool,
-        a.v_pool, a.q, a.q_stride, a.out, a.partials, a.n_heads, group, gh, a.window, a.scale, a.softcap, a.sinks, a.slopes,
-        a.row_scale);
+    constexpr int W = f32_waves<HDT>();
+    // Workgroups of eight and sixteen waves share a unit by twos at most, and short items leave most of their waves without a key: beyond
+    // the units four waves, the same waves in flight in smaller pieces.  Over cold keys, us, the vector units' kernel / all waves / four: 64 requests of 40 keys, 16 heads on 16 of
+    // 64 17.2 / 21.5 / 9.5, 200 of 300 278 / 203 / 130; 200 of 1,000, 14 on 2 of 64 94 / 69 / 50; 64 of 700, 32 on 32 of 128 514 / 308 / 271;
+    // 16 prompts of 60 tokens, 32 on 4 of 32 26.8 / 31.4 / 10.4.  An item of up to four blocks gives the same bits by either.
+    if (W > 4 && static_cast<int64_t>(grid.x) * grid.y * grid.z > fsie_compute_units()) launch_waves<HDT, 4>(a, grid, group, gh, stream);
+    else launch_waves<HDT, W>(a, grid, group, gh, stream);
     FSIE_CHECK_LAUNCH("attention_f32");
     return 0;
 }

@@ -779,6 +779,35 @@ def test_attention_on_the_float32_matrix_instruction(ops, heads, kv, hd, page, w
     assert (other.cpu() - out).abs().max() <= 4e-6
 
 
+@pytest.mark.parametrize("heads, kv, hd, page, window", [(14, 2, 64, 16, None), (4, 4, 16, 4, 21), (6, 3, 128, 24, 70), (20, 1, 80, 8, None)])
+def test_float32_attention_of_more_workgroups_than_units(ops, heads, kv, hd, page, window):
+    """Four waves a workgroup: against the plain product, and against the same items a few at a time (all waves), whose bits are the same
+    up to four blocks of 16 keys."""
+    from from_scratch_inference_engine_amd.parts.attention import AttentionPlanner
+
+    base = [0, 14, 15, 16, 47, 62, 63, 64, 130, 254]
+    seqs = [(p, 1) for p in base] * (ops.compute_units() // (len(base) * kv * -(-heads // kv // 16)) + 1)
+    AttentionPlanner.compute_units = 8
+    try:
+        case = paged_case(seqs, heads, kv, hd, page, torch.float32, seed=hd, window=window)
+    finally:
+        AttentionPlanner.compute_units = None
+    plan = case["plan"]
+    assert not plan["n_merges"] and plan["n_small"] == len(seqs)
+    out = run_attention(ops, case, heads, kv, hd, window)
+    few = torch.zeros_like(out).cuda()
+    q, pools, items = case["q"].cuda(), (case["k_pool"].cuda(), case["v_pool"].cuda(), case["tables"].cuda()), torch.from_numpy(plan["items"]).cuda()
+    for at in range(0, len(seqs), len(base)):
+        ops.attention_scalar(q, heads * hd, *pools, items[at:at + len(base)], len(base), few, None, heads, kv, hd, window, 1.0 / math.sqrt(hd),
+                             len(seqs))
+    few = few.cpu()
+    for row, ((p, _), qs, k, v) in enumerate(zip(seqs, case["qs"], case["ks"], case["vs"])):
+        ref = plain.attention(qs, k, v, heads, kv, hd, query_offset=p, window=window)
+        assert (out[row:row + 1] - ref).abs().max() <= 2e-6 and (few[row:row + 1] - ref).abs().max() <= 2e-6, p
+        if p < 64 or (window and window <= 48):
+            assert torch.equal(out[row], few[row]), p
+
+
 @pytest.mark.parametrize("heads, kv, hd, page, window", [(14, 2, 64, 16, None), (6, 2, 128, 24, 70), (4, 4, 48, 4, None), (20, 1, 256, 8, None)])
 def test_attention_of_items_by_few_and_by_many_waves(ops, heads, kv, hd, page, window):
     """The variant for short items (a wave a block of 32 keys) and the one with all the waves the head size allows: the same bits
