@@ -12,10 +12,10 @@
 // A workgroup takes an item (a tile of up to 16 query rows, a range of keys) of a kv head; the item's blocks of 16 keys are
 // dealt to its waves in runs of equal length, and the waves' sums meet in LDS, in the order of the waves, behind one barrier.
 // What bounds it is the chain: the item, the block table, keys and values, a trip to memory each, then 32 matrix instructions a
-// block and head of 64 at 32 cycles.  With the merge where items are cut, us, the kernel on the vector units (attention_scalar) /
-// this one: 4 requests of 300 keys, 14 heads on 2 of 64 12.1 / 8.3, 28 on 4 of 128 16.9 / 8.6, 16 on 1 of 256 35.0 / 12.5; one
-// of 100 keys 15.1 / 6.9, 23.1 / 7.7, 54 / 13.8; 32 of 700 20.7 / 15.3, 56 / 26, 48 / 24; a prompt of 300 tokens 49 / 16, 88 / 29,
-// 130 / 37, of 1,000 185 / 59, 537 / 155, 636 / 203.
+// block and head of 64 at 32 cycles.  With the merge where items are cut, keys that no cache holds, us, the kernel on the vector
+// units (attention_scalar) / this one: 4 requests of 300 keys, 14 heads on 2 of 64 13.4 / 7.4, 28 on 4 of 128 19.4 / 8.7, 16 on 1
+// of 256 39 / 12.6; one of 100 keys 16.0 / 6.3, 24.0 / 7.7, 60 / 14.1; 32 of 700 26.9 / 12.4, 68 / 26.9, 56 / 25.8; a prompt of 300
+// tokens 54 / 13.2, 94 / 25.6, 137 / 38, of 1,000 202 / 52, 562 / 147, 657 / 202.
 //
 // More workgroups than units: four waves each whatever the head size (see launch).
 #include "common.h"
@@ -282,10 +282,11 @@ int launch(const F32Call& a, hipStream_t stream) {
     const int group = a.n_heads / a.n_kv, gh = group < 16 ? group : 16;
     const dim3 grid(a.n_items, a.n_kv, (group + gh - 1) / gh);
     constexpr int W = f32_waves<HDT>();
-    // Workgroups of eight and sixteen waves share a unit by twos at most, and short items leave most of their waves without a key: beyond
-    // the units four waves, the same waves in flight in smaller pieces.  Over cold keys, us, the vector units' kernel / all waves / four: 64 requests of 40 keys, 16 heads on 16 of
-    // 64 17.2 / 21.5 / 9.5, 200 of 300 278 / 203 / 130; 200 of 1,000, 14 on 2 of 64 94 / 69 / 50; 64 of 700, 32 on 32 of 128 514 / 308 / 271;
-    // 16 prompts of 60 tokens, 32 on 4 of 32 26.8 / 31.4 / 10.4.  An item of up to four blocks gives the same bits by either.
+    // Workgroups of eight and sixteen waves share a unit by twos at most, and short items leave most of their waves without a key:
+    // beyond the units four waves, the same waves in flight in smaller pieces.  Over cold keys, us, the vector units' kernel / all
+    // waves / four: 64 requests of 40 keys, 16 heads on 16 of 64 17.2 / 21.5 / 9.5, 200 of 300 278 / 203 / 130; 200 of 1,000, 14 on 2
+    // of 64 94 / 69 / 50; 64 of 700, 32 on 32 of 128 514 / 308 / 271; 16 prompts of 60 tokens, 32 on 4 of 32 26.8 / 31.4 / 10.4.  An
+    // item of up to four blocks gives the same bits by either.
     if (W > 4 && static_cast<int64_t>(grid.x) * grid.y * grid.z > fsie_compute_units()) launch_waves<HDT, 4>(a, grid, group, gh, stream);
     else launch_waves<HDT, W>(a, grid, group, gh, stream);
     FSIE_CHECK_LAUNCH("attention_f32");
