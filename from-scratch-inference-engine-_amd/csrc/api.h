@@ -271,7 +271,9 @@ int fsie_attention_scalar(const void* q, int64_t q_stride, const void* k_pool, c
                           void* out, float* partials, int n_heads, int n_kv, int head_dim, int page_size,
                           int window, float scale, int dtype, const float* sinks, float softcap, const void* k_pooled,
                           const void* v_pooled, const int32_t* pooled_tables, int pooled_max_pages, int pooled_page_size,
-                          int pooled_tokens, const float* slopes, const float* row_scale, hipStream_t stream);
+                          int pooled_tokens, const float* slopes, const float* row_scale, int all_waves, hipStream_t stream);
+// all_waves (read by the kernel for float32 storage alone): items of more than 64 keys keep all the waves of a head size however many
+// workgroups there are.
 // k_pooled .. pooled_tokens (or null and zeros): pools [units][n_kv][pooled_page_size][head_dim] and
 // [units][n_kv][head_dim][pooled_page_size] that hold one mean key and value for every block of pooled_tokens positions,
 // with their block table [requests][pooled_max_pages]; an item flagged FSIE_ATTN_POOL_WALK reads, beside its own keys,
@@ -293,7 +295,7 @@ int fsie_attention_f32_ok(int head_dim, int page_size);
 int fsie_attention_f32(const float* q, int64_t q_stride, const float* k_pool, const float* v_pool, const int32_t* block_tables,
                        int max_pages, const int32_t* items, int n_items, float* out, float* partials, int n_heads, int n_kv,
                        int head_dim, int page_size, int window, float scale, const float* sinks, float softcap, const float* slopes,
-                       const float* row_scale, hipStream_t stream);
+                       const float* row_scale, int all_waves, hipStream_t stream);
 int fsie_attention_scalar_tile_tokens(int n_heads, int n_kv);
 // The mean key and value of blocks of `block_tokens` consecutive positions, from the pages of keys and values to the
 // pools of pooled blocks: jobs [n_jobs][2] = (request of the step, block), a request of -1: nothing.  Block b's

@@ -15,9 +15,9 @@
 // block and head of 64 at 32 cycles.  With the merge where items are cut, keys that no cache holds, us, the kernel on the vector
 // units (attention_scalar) / this one: 4 requests of 300 keys, 14 heads on 2 of 64 13.4 / 7.4, 28 on 4 of 128 19.4 / 8.7, 16 on 1
 // of 256 39 / 12.6; one of 100 keys 16.0 / 6.3, 24.0 / 7.7, 60 / 14.1; 32 of 700 26.9 / 12.4, 68 / 26.9, 56 / 25.8; a prompt of 300
-// tokens 54 / 13.2, 94 / 25.6, 137 / 38, of 1,000 202 / 52, 562 / 147, 657 / 202.
+// tokens 54 / 14.9, 94 / 30, 137 / 38, of 1,000 202 / 59, 562 / 155, 657 / 202.
 //
-// More workgroups than units: four waves each whatever the head size (see launch).
+// More workgroups than units: four waves each whatever the head size, except over the tiles of long prompts (see launch).
 #include "common.h"
 #include "api.h"
 
@@ -40,7 +40,7 @@ struct F32Call {
     int64_t q_stride;
     const int32_t *block_tables, *items;
     float *out, *partials;
-    int n_items, max_pages, n_heads, n_kv, page_size, window;
+    int n_items, max_pages, n_heads, n_kv, page_size, window, all_waves;
     float scale, softcap;
     const float *sinks, *slopes, *row_scale;
 };
@@ -286,8 +286,10 @@ int launch(const F32Call& a, hipStream_t stream) {
     // beyond the units four waves, the same waves in flight in smaller pieces.  Over cold keys, us, the vector units' kernel / all
     // waves / four: 64 requests of 40 keys, 16 heads on 16 of 64 17.2 / 21.5 / 9.5, 200 of 300 278 / 203 / 130; 200 of 1,000, 14 on 2
     // of 64 94 / 69 / 50; 64 of 700, 32 on 32 of 128 514 / 308 / 271; 16 prompts of 60 tokens, 32 on 4 of 32 26.8 / 31.4 / 10.4.  An
-    // item of up to four blocks gives the same bits by either.
-    if (W > 4 && static_cast<int64_t>(grid.x) * grid.y * grid.z > fsie_compute_units()) launch_waves<HDT, 4>(a, grid, group, gh, stream);
+    // item of up to four blocks gives the same bits by either; a launch with longer tiles of prompts asks for all waves, since a
+    // portion's sums are not to follow from what else is in the step (300 tokens, 14 on 2 of 64, 14.9 us where four took 13.2).
+    const bool many = static_cast<int64_t>(grid.x) * grid.y * grid.z > fsie_compute_units();
+    if (W > 4 && many && !a.all_waves) launch_waves<HDT, 4>(a, grid, group, gh, stream);
     else launch_waves<HDT, W>(a, grid, group, gh, stream);
     FSIE_CHECK_LAUNCH("attention_f32");
     return 0;
@@ -313,7 +315,7 @@ extern "C" int fsie_attention_f32_ok(int head_dim, int page_size) {
 extern "C" int fsie_attention_f32(const float* q, int64_t q_stride, const float* k_pool, const float* v_pool,
                                   const int32_t* block_tables, int max_pages, const int32_t* items, int n_items, float* out,
                                   float* partials, int n_heads, int n_kv, int head_dim, int page_size, int window, float scale,
-                                  const float* sinks, float softcap, const float* slopes, const float* row_scale,
+                                  const float* sinks, float softcap, const float* slopes, const float* row_scale, int all_waves,
                                   hipStream_t stream) {
     FSIE_REQUIRE(n_items >= 0 && n_heads > 0 && n_kv > 0 && n_heads % n_kv == 0,
                  "attention: heads %d must be a positive multiple of kv heads %d", n_heads, n_kv);
@@ -330,6 +332,6 @@ extern "C" int fsie_attention_f32(const float* q, int64_t q_stride, const float*
     a.q = q, a.k_pool = k_pool, a.v_pool = v_pool, a.q_stride = q_stride, a.block_tables = block_tables, a.items = items;
     a.out = out, a.partials = partials, a.n_items = n_items, a.max_pages = max_pages, a.n_heads = n_heads, a.n_kv = n_kv;
     a.page_size = page_size, a.window = window, a.scale = scale, a.softcap = softcap;
-    a.sinks = sinks, a.slopes = slopes, a.row_scale = row_scale;
+    a.sinks = sinks, a.slopes = slopes, a.row_scale = row_scale, a.all_waves = all_waves;
     return launch_from<1>(head_dim / 16, a, stream);
 }

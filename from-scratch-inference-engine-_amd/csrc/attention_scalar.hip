@@ -546,7 +546,7 @@ extern "C" int fsie_attention_scalar(const void* q, int64_t q_stride, const void
                                      int head_dim, int page_size, int window, float scale, int dtype,
                                      const float* sinks, float softcap, const void* k_pooled, const void* v_pooled,
                                      const int32_t* pooled_tables, int pooled_max_pages, int pooled_page_size,
-                                     int pooled_tokens, const float* slopes, const float* row_scale, hipStream_t stream) {
+                                     int pooled_tokens, const float* slopes, const float* row_scale, int all_waves, hipStream_t stream) {
     FSIE_REQUIRE(!(k_pooled && slopes), "attention: a distance bias over pooled blocks has no meaning (a block has no one position)");
     FSIE_REQUIRE(!k_pooled || (v_pooled && pooled_tables && pooled_max_pages > 0 && pooled_page_size > 0 && pooled_tokens > 0 &&
                                window > 0),
@@ -567,7 +567,7 @@ extern "C" int fsie_attention_scalar(const void* q, int64_t q_stride, const void
         return fsie_attention_f32(static_cast<const float*>(q), q_stride, static_cast<const float*>(k_pool),
                                   static_cast<const float*>(v_pool), block_tables, max_pages, items, n_items,
                                   static_cast<float*>(out), partials, n_heads, n_kv, head_dim, page_size, window, scale, sinks,
-                                  softcap, slopes, row_scale, stream);
+                                  softcap, slopes, row_scale, all_waves, stream);
     const int group = n_heads / n_kv;
     const int gh = group < kRows ? group : kRows;
     const int head_chunks = (group + gh - 1) / gh;

@@ -843,7 +843,8 @@ def attention_scalar(q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_poo
                      partials: Optional[torch.Tensor], n_heads: int, n_kv: int, head_dim: int,
                      window: Optional[int], scale: float, n_query_rows: int,
                      sinks: Optional[torch.Tensor] = None, softcap: float = 0.0, pooled=None,
-                     slopes: Optional[torch.Tensor] = None, row_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
+                     slopes: Optional[torch.Tensor] = None, row_scale: Optional[torch.Tensor] = None,
+                     all_waves: bool = False) -> torch.Tensor:
     """Attention of the work items over the paged cache (float32 arithmetic).  ``slopes`` (float32 [n_heads], here and
     in the other attention functions): slopes[h] (query position - key position) is taken off head h's scores, behind
     scale and cap.  ``row_scale`` (float32, one a row of q, here and in the others): a factor on all scores of a row,
@@ -851,7 +852,8 @@ def attention_scalar(q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_poo
     here and in the other attention functions): exp(sinks[h]) is one more term of the denominator of
     head h's softmax, with no key and no value.  ``pooled`` = (k_pool, v_pool, block_tables, block_tokens) of the
     pools of pooled blocks (one mean key and value for every ``block_tokens`` positions): items flagged
-    ``ATTN_POOL_WALK`` also read the blocks that lie wholly before their queries' windows.
+    ``ATTN_POOL_WALK`` also read the blocks that lie wholly before their queries' windows.  ``all_waves``: a plan's, see
+    ``AttentionPlanner``.
 
     ``q`` is a view into rows of stride ``q_stride`` elements whose first n_heads*head_dim columns
     are the queries; ``out`` is [n_query_rows, n_heads*head_dim]."""
@@ -885,7 +887,7 @@ def attention_scalar(q: torch.Tensor, q_stride: int, k_pool: torch.Tensor, v_poo
                                        n_items, out.data_ptr(), _ptr(partials), n_heads, n_kv, head_dim,
                                        page_size, int(window or 0), float(scale), dtype_code(q.dtype),
                                        _sinks_ptr(sinks, n_heads), float(softcap or 0.0), *pooled_args,
-                                       *_bias_ptrs(slopes, row_scale, n_heads, n_query_rows), _stream()))
+                                       *_bias_ptrs(slopes, row_scale, n_heads, n_query_rows), int(all_waves), _stream()))
     return out
 
 

@@ -65,7 +65,7 @@ _SIGNATURES = {
     "fsie_fragment_order_size": ([c_int, c_int], c_int64),
     "fsie_fragment_order": ([_P, _P, c_int, c_int, _P], c_int),
     "fsie_attention_scalar": ([_P, c_int64, _P, _P, _P, c_int, _P, c_int, _P, _P, c_int, c_int, c_int,
-                               c_int, c_int, c_float, c_int, _P, c_float, _P, _P, _P, c_int, c_int, c_int, _P, _P, _P], c_int),
+                               c_int, c_int, c_float, c_int, _P, c_float, _P, _P, _P, c_int, c_int, c_int, _P, _P, c_int, _P], c_int),
     "fsie_attention_mfma": ([_P, c_int64, _P, _P, _P, c_int, _P, c_int, _P, _P, c_int, c_int, c_int,
                              c_int, c_int, c_float, c_int, c_int, _P, c_float, _P, _P, _P], c_int),
     "fsie_attention_mfma_qkv_ok": ([c_int, c_int], c_int),

@@ -493,6 +493,10 @@ class AttentionPlanner:
             "n_small": len(small), "n_large": len(large) - n_long, "n_long": n_long, "long_waves": long_waves,
             "n_merges": len(merges) + sum(len(m) for m in merge_runs),
             "n_partial": n_partial, "mfma": mfma, "waves": waves, "fills": bool(mfma and fills),
+            # tiles of a long portion of more than four blocks of 16 keys: by all waves in float32 whatever else is in the step (up to
+            # four blocks the sums are the same either way; decode items are cut by the batch as it is)
+            "all_waves": not mfma and bool((large[:, 5] - (large[:, 4] & ~15) + np.where(
+                large[:, 7] & ATTN_KEEP_WALK, np.minimum(large[:, 7] & ~(ATTN_KEEP_WALK | ATTN_POOL_WALK), large[:, 4]) + 15 & ~15, 0) > 64).any()),
             "single": all(host.q_lens[s] == 1 for s in range(host.n_seqs)),  # one token a request
         }
 
@@ -543,7 +547,8 @@ def paged_attention(q: torch.Tensor, q_stride: int, cache, plan, n_heads: int, n
                                  plan.n_pool_items, out, *args, softcap=cap, pooled=pooled, **bias)
     else:
         ops.attention_scalar(q, q_stride, cache.k_pool, cache.v_pool, cache.block_tables, plan.items,
-                             plan.n_small + plan.n_large, out, *args, sinks=sinks, softcap=cap, pooled=pooled, **bias)
+                             plan.n_small + plan.n_large, out, *args, sinks=sinks, softcap=cap, pooled=pooled,
+                             all_waves=getattr(plan, "all_waves", False), **bias)
     if plan.n_merges:
         ops.attention_merge(partials, plan.merges, plan.n_merges, out, n_heads, head_dim, sinks=sinks)
     return out

@@ -808,6 +808,32 @@ def test_float32_attention_of_more_workgroups_than_units(ops, heads, kv, hd, pag
             assert torch.equal(out[row], few[row]), p
 
 
+@pytest.mark.parametrize("heads, kv, hd, page, window", [(14, 2, 64, 16, None), (16, 16, 16, 4, None), (6, 3, 128, 24, 70)])
+def test_a_prompt_in_float32_has_the_same_bits_in_any_company(ops, heads, kv, hd, page, window):
+    """Prompts of several tiles, alone (but for the longest fewer workgroups than units) and in one step; up to four blocks of 16 keys
+    by four waves among many, by all alone."""
+    from types import SimpleNamespace
+
+    from from_scratch_inference_engine_amd.parts.attention import paged_attention
+
+    def run(case):
+        plan = SimpleNamespace(**{k: torch.from_numpy(v).cuda() if isinstance(v, np.ndarray) else v for k, v in case["plan"].items()})
+        cache = SimpleNamespace(k_pool=case["k_pool"].cuda(), v_pool=case["v_pool"].cuda(), block_tables=case["tables"].cuda(), page_size=page)
+        return paged_attention(case["q"].cuda(), heads * hd, cache, plan, heads, kv, hd, window, hd ** -0.5, case["q"].shape[0]).cpu()
+
+    for seqs, longest in (([(0, 100), (40, 24), (0, 64), (3, 61), (0, 65), (200, 40), (0, 300)] + [(90, 90)] * 24, True),
+                          ([(0, 30), (0, 64), (20, 44)] * 16, False)):
+        case = paged_case(seqs, heads, kv, hd, page, torch.float32, seed=hd, window=window)
+        assert case["plan"]["all_waves"] == longest
+        together = run(case)
+        row = 0
+        for i, (p, n) in enumerate(seqs[:8]):
+            alone = paged_case([(p, n)], heads, kv, hd, page, torch.float32, seed=hd, window=window, edit=lambda qs, ks, vs: (
+                qs[0].copy_(case["qs"][i]), ks[0].copy_(case["ks"][i]), vs[0].copy_(case["vs"][i])))
+            assert torch.equal(run(alone), together[row:row + n]), (p, n)
+            row += n
+
+
 @pytest.mark.parametrize("heads, kv, hd, page, window", [(14, 2, 64, 16, None), (6, 2, 128, 24, 70), (4, 4, 48, 4, None), (20, 1, 256, 8, None)])
 def test_attention_of_items_by_few_and_by_many_waves(ops, heads, kv, hd, page, window):
     """The variant for short items (a wave a block of 32 keys) and the one with all the waves the head size allows: the same bits
