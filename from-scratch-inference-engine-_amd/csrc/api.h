@@ -358,8 +358,8 @@ int fsie_attention_split_static(const void* q, int64_t q_stride, const void* k_p
 int fsie_sample(const float* logits, int n_rows, int vocab, const float* temperature, const int32_t* top_k,
                 const float* top_p, const double* uniform, int32_t* out, hipStream_t stream);
 // The same at temperatures with every row shared by several workgroups, where fsie_sample_workspace says so:
-// `workspace` = fsie_sample_workspace(n_rows, vocab) bytes on the device (0: the call is fsie_sample's), uninitialised.
-int64_t fsie_sample_workspace(int n_rows, int vocab);
+// `workspace` = fsie_sample_workspace(n_rows, vocab, whether top_k or top_p are given) bytes on the device (0: the call is fsie_sample's), uninitialised.
+int64_t fsie_sample_workspace(int n_rows, int vocab, int thresholds);
 int fsie_sample_split(const float* logits, int n_rows, int vocab, const float* temperature, const int32_t* top_k,
                       const float* top_p, const double* uniform, void* workspace, int32_t* out, hipStream_t stream);
 

@@ -13,8 +13,8 @@
 // is zero or infinite, so that a weight may be a NaN, more than 2,048 tokens in the threshold's bin) are bisected over the order-preserving integer image of the logits, a pass a probe.
 // What bounds it is how often a compute unit reads a row of 600 KB from the caches: one pass for greedy, two at a plain
 // temperature, 4 with a threshold and 5 with two whose bins differ, where the bisection alone took 32 a threshold (64 rows of
-// 152,064, a fifth of them each greedy, at a temperature, top k, top p and both: 152 us, 1,504 with the bisection alone).
-// Long rows are shared by several workgroups where the call has few of them (below): 89 us for the same call.
+// 152,064, a fifth of them each greedy, at a temperature, top k, top p and both: 141 us, 1,504 with the bisection alone).
+// Long rows are shared by several workgroups (below): 45 us for the same call.
 #include "common.h"
 #include "api.h"
 
@@ -46,6 +46,34 @@ __device__ double block_sum_f64(double v, double* scratch) {
     double total = 0.0;
     for (int w = 0; w < kWaves; ++w) total += scratch[w];
     return total;
+}
+
+// A 64-bit value moved between the lanes by the vector unit's data path (a general shuffle is a trip through LDS): lanes that get none
+// have 0.  CTRL: n lanes up within sixteen (0x110 + n), the last of sixteen to the next sixteen (0x142) or to the upper half (0x143).
+template <int CTRL, int ROWS, typename T>
+__device__ __forceinline__ T lanes_up(T v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned int lo = __builtin_amdgcn_update_dpp(0u, static_cast<unsigned int>(u), CTRL, ROWS, 0xf, false);
+    const unsigned int hi = __builtin_amdgcn_update_dpp(0u, static_cast<unsigned int>(u >> 32), CTRL, ROWS, 0xf, false);
+    return __builtin_bit_cast(T, (static_cast<unsigned long long>(hi) << 32) | lo);
+}
+// The sum over this lane and those below it, all 64 active; T: double or unsigned long long.
+template <typename T>
+__device__ __forceinline__ T wave_upto(T v) {
+    v += lanes_up<0x111, 0xf>(v);
+    v += lanes_up<0x112, 0xf>(v);
+    v += lanes_up<0x114, 0xf>(v);
+    v += lanes_up<0x118, 0xf>(v);
+    v += lanes_up<0x142, 0xa>(v);
+    return v + lanes_up<0x143, 0xc>(v);
+}
+// The value of one lane (the same in all), in all of them.
+template <typename T>
+__device__ __forceinline__ T of_lane(T v, int lane) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const unsigned int lo = __builtin_amdgcn_readlane(static_cast<unsigned int>(u), lane);
+    const unsigned int hi = __builtin_amdgcn_readlane(static_cast<unsigned int>(u >> 32), lane);
+    return __builtin_bit_cast(T, (static_cast<unsigned long long>(hi) << 32) | lo);
 }
 
 struct Best {
@@ -384,12 +412,15 @@ __device__ uint32_t cut_by_bisection(const float* row, int vocab, float mx, floa
 }
 
 // The first token, in vocabulary order, at which the running sum of the kept weights passes uniform * their sum, from the
-// sums of the runs: every wave finds the run, and the wave that owns it (`own_runs` runs a wave; -1: there is one wave)
-// walks it.
+// sums of the runs (in LDS): every wave finds the run, whose 64-token lines the waves then walk side by side, one each.  (One
+// wave after all of them is a chain of a trip to memory and six exchanges between lanes a line: 64 rows of 152,064
+// tokens 8.2 us in a kernel of their own; and 2 so.)
 __device__ void draw_from_runs(const float* __restrict__ row, int vocab, Best top, float inv_temp, uint32_t cut, double uniform,
-                               const double* run_sum, int own_runs, int32_t* out) {
+                               const double* run_sum, int32_t* out) {
+    __shared__ double line_sum[kWaves];
+    __shared__ int line_hit[kWaves], line_last[kWaves];
     const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
-    const int rows = ((vocab + FSIE_WAVE - 1) / FSIE_WAVE + kRuns - 1) / kRuns;  // 64 tokens each
+    const int lines = ((vocab + FSIE_WAVE - 1) / FSIE_WAVE + kRuns - 1) / kRuns;
     const float mx = top.value;
     // four neighbouring runs a lane
     double part[kRuns / FSIE_WAVE], upto = 0.0;
@@ -398,12 +429,8 @@ __device__ void draw_from_runs(const float* __restrict__ row, int vocab, Best to
         part[q] = run_sum[lane * (kRuns / FSIE_WAVE) + q];
         upto += part[q];
     }
-#pragma unroll
-    for (int off = 1; off < FSIE_WAVE; off <<= 1) {
-        const double other = __shfl_up(upto, off, FSIE_WAVE);
-        if (lane >= off) upto += other;
-    }
-    const double total = __shfl(upto, FSIE_WAVE - 1, FSIE_WAVE);
+    upto = wave_upto(upto);
+    const double total = of_lane(upto, FSIE_WAVE - 1);
     const double threshold = uniform * total;
     double before = __shfl_up(upto, 1, FSIE_WAVE);
     if (lane == 0) before = 0.0;
@@ -423,29 +450,38 @@ __device__ void draw_from_runs(const float* __restrict__ row, int vocab, Best to
             ++run;
         }
     }
-    run = __shfl(run, owner, FSIE_WAVE);
-    cum = __shfl(cum, owner, FSIE_WAVE);
-    if (own_runs > 0 && wave != run / own_runs) return;
+    run = __builtin_amdgcn_readlane(run, owner);
+    cum = of_lane(cum, owner);
     int last_kept = -1;
-    for (int j = 0; j < rows; ++j) {
-        const int64_t i = (static_cast<int64_t>(run) * rows + j) * FSIE_WAVE + lane;
+    for (int j0 = 0; j0 < lines; j0 += kWaves) {
+        const int64_t i = (static_cast<int64_t>(run) * lines + j0 + wave) * FSIE_WAVE + lane;
         const float v = row[i < vocab ? i : vocab - 1];
-        const bool kept = i < vocab && order_key(v) >= cut;
-        double w = kept ? token_weight(v, mx, inv_temp) : 0.0;
-#pragma unroll
-        for (int off = 1; off < FSIE_WAVE; off <<= 1) {
-            const double other = __shfl_up(w, off, FSIE_WAVE);
-            if (lane >= off) w += other;
+        const bool kept = j0 + wave < lines && i < vocab && order_key(v) >= cut;
+        const double w = wave_upto(kept ? token_weight(v, mx, inv_temp) : 0.0);
+        if (j0 > 0) __syncthreads();
+        if (lane == FSIE_WAVE - 1) line_sum[wave] = w;
+        __syncthreads();
+        double base = cum;
+        for (int q = 0; q < kWaves; ++q) {
+            if (q == wave) base = cum;
+            cum += line_sum[q];
         }
-        const unsigned long long hit = __ballot(kept && threshold < cum + w), any = __ballot(kept);
-        if (hit) {
-            if (lane == __ffsll(hit) - 1) *out = static_cast<int>(i);
-            return;
+        const unsigned long long hit = __ballot(kept && threshold < base + w), any = __ballot(kept);
+        const int64_t first = i - lane;
+        if (lane == 0) {
+            line_hit[wave] = hit ? static_cast<int>(first) + __ffsll(hit) - 1 : -1;
+            line_last[wave] = any ? static_cast<int>(first) + 63 - __clzll(any) : -1;
         }
-        if (any) last_kept = static_cast<int>((static_cast<int64_t>(run) * rows + j) * FSIE_WAVE) + 63 - __clzll(any);
-        cum += __shfl(w, FSIE_WAVE - 1, FSIE_WAVE);
+        __syncthreads();
+        for (int q = 0; q < kWaves; ++q) {
+            if (line_hit[q] >= 0) {
+                if (threadIdx.x == 0) *out = line_hit[q];
+                return;
+            }
+            last_kept = max(last_kept, line_last[q]);
+        }
     }
-    if (lane == 0) *out = last_kept >= 0 ? last_kept : top.index;  // rounding at the run's end
+    if (threadIdx.x == 0) *out = last_kept >= 0 ? last_kept : top.index;  // rounding at the run's end
 }
 
 // Without temperatures: the maximum alone.  A kernel of its own, since the other one's extremes and registers cost this pass
@@ -533,49 +569,58 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
         }
     }
     __syncthreads();
-    draw_from_runs(row, vocab, top, inv_temp, cut, uniform[r], run_sum, kRunsOfWave, out + r);
+    draw_from_runs(row, vocab, top, inv_temp, cut, uniform[r], run_sum, out + r);
 }
 
 // ---- a row shared by several workgroups -------------------------------------------------------
 // One workgroup a row leaves three quarters of the chip idle at 64 rows and all but one unit at one row, and a unit
 // needs some 10 us for every pass over 152,064 tokens (their exponentials and the adds in float64).  From kSplitFrom
-// tokens on the row's runs are dealt to up to 64 workgroups, and the passes become launches: the maximum; bins (or,
-// for rows without a threshold, the draw's sums); the threshold bins' tokens; the cut; the draw's sums; the draw.
-// What a launch leaves for the next lies in a workspace of the row.
-// A workgroup a row takes the same time up to 256 rows and grows with the row; shared, six launches' ends cost some 30 us
-// and the rest grows with the tokens of all rows.  Alone / shared, us, a fifth of the rows each greedy, plain, top k, top p and
-// both, at 1, 8, 32, 64, 128 and 256 rows:
-//    16,384 tokens   34 /  31    34 / 33    35 / 43    35 / 50     35 /  63     36 /  82
-//    32,000          45 /  32    46 / 34    46 / 45    46 / 51     46 /  65     48 /  94
-//    65,536          69 /  34    69 / 39    70 / 49    71 / 58     72 /  77     75 / 114
-//   152,064         137 /  38   138 / 47   144 / 66   152 / 89    153 / 127    159 / 193
-// so rows are shared from kSplitFrom tokens on while each of them has kTokensForRow for every row of the call.  Without
-// thresholds it is three launches, and the same line (32,000 tokens 16 / 9, 17 / 11, 17 / 14, 17 / 17, 17 / 24, 19 / 40).
+// tokens on the row's runs are dealt to up to 32 workgroups, and the passes become launches: the maximum; the row's bins (or,
+// for rows without a threshold, the draw's sums); the tokens about the thresholds, side by side, and the draw's sums of
+// those that are kept for certain; the cut among the listed tokens and the draw.  What a launch leaves for the next lies in
+// a workspace of the row.
+// Alone / shared, us, a fifth of the rows each greedy, plain, top k, top p and both, at 8, 64, 128, 256, 512 and 2,048 rows:
+//    16,384 tokens   34 / 24    35 / 26    35 / 28     36 /  33     66 /  48    206 / 134
+//    32,000          43 / 25    45 / 27    46 / 32     48 /  44     88 /  67    262 / 185
+//    65,536          68 / 25    70 / 32    70 / 42     74 /  61    139 / 102    420 / 343
+//   152,064         130 / 26   141 / 45   145 / 69    155 / 113    289 / 203    847 / 708
+// so where thresholds are given rows are shared up to kMostRows of them (what was measured, twice; their workspaces are 41 KB a row).  Without
+// thresholds it is three launches beside one of two passes, and the line is kMostPlainRows (8, 64, 128, 256, 380 rows of 16,384:
+// 17 / 11, 17 / 13, 17 / 15, 18 / 20, 34 / 26; of 152,064: 42 / 12, 48 / 27, 51 / 43, 61 / 73, 105 / 103).
 // (Without temperatures it is one pass over the row, and a workgroup a row is the faster one; with temperatures that all
 // say greedy too, but that only the device knows.)
 constexpr int kSplitFrom = 16384;
-constexpr int kTokensForRow = 800;
-constexpr int kPart = 256;          // threads of a shared row's workgroups
-constexpr int kMaxParts = 64;
-constexpr int kPairs = 512;         // so many listed tokens are compared with each other, more are bisected
+constexpr int kMostRows = 4096, kMostPlainRows = 160;
+constexpr int kPart = 512;          // threads of a shared row's workgroups
+constexpr int kMaxParts = 32;
+constexpr int kCoarse = 512;        // bins of a shared row
+constexpr int kFine = 1024;         // what the bin of a threshold is cut into
+constexpr int kPairs = 512;         // so many tokens of a fine bin are compared with each other, more are bisected
 constexpr int kKeep = 4096;         // tokens that the list holds
+constexpr int kAllListed = 1024;    // up to this top k the list takes every token down to the bin of the k-th
+static_assert(kRuns / kMaxParts >= kPart / FSIE_WAVE, "every wave of a part has a run");
 
 struct SplitRow {
-    unsigned long long hi[kBins], lo[kBins];
+    unsigned long long sum[kCoarse];  // weights, in units of their bin's own (RowBins)
+    unsigned int count[kCoarse];
+    unsigned int n_listed;            // (behind the bins: cleared with them)
+    int top_index, top_nan;           // the row's, from the parts'
+    float top_max, top_low;
+    int k_bin, from, upto;            // the bin of top k; those that hold the last token of top p
+    double above_k, above, target;    // tokens above k_bin; weight above `from`; what top p's kept weight has to reach (0: no top p alone)
     double run_sum[kRuns];
-    unsigned int count[kBins];
-    unsigned int n_listed, cut;     // (behind the bins: cleared with them)
-    unsigned int pad[2];
     float listed[kKeep];
+    int listed_at[kKeep];
     float part_max[kMaxParts], part_low[kMaxParts];
     int part_index[kMaxParts], part_nan[kMaxParts];
 };
-static_assert(sizeof(SplitRow) % 16 == 0, "rows of the workspace stay aligned");
+static_assert(sizeof(SplitRow) % 8 == 0, "rows of the workspace stay aligned");
 
 struct RowParams {
     float temp, inv_temp, p;
     int k;
     bool cuts;
+    __device__ bool all_listed() const { return 0 < k && k <= kAllListed; }
 };
 __device__ __forceinline__ RowParams row_params(int r, int vocab, const float* temperature, const int32_t* top_k,
                                                 const float* top_p) {
@@ -588,17 +633,44 @@ __device__ __forceinline__ RowParams row_params(int r, int vocab, const float* t
     return q;
 }
 
+// The row's bins: kCoarse equal ones over what it spans, at most kRange or 30 temperatures (43 powers of two in weight).  A bin's weights are
+// summed as integers of a unit of its own, one limb: 2^-(unit + below(bin)), where below(bin) powers of two lie between
+// the largest weight and the bin's.  With at most unit - 25 powers of two a bin nothing of a weight is lost; in the last one,
+// which takes all that lies further down, nothing above 2^-(unit + 42); two limbs of 40 bits lose no less.
+// (Two limbs are twice the additions in LDS and into the row's bins, and thrice the instructions.)
+struct RowBins {
+    float scale, binades;
+    int unit;
+    __device__ int bin(float v, float mx) const { return static_cast<int>(fminf((mx - v) * scale, static_cast<float>(kCoarse - 1))); }
+    __device__ int below(int b) const { return static_cast<int>(static_cast<float>(b) * binades); }
+    __device__ unsigned long long weight(float w, int b) const {
+        const uint32_t u = __float_as_uint(w);
+        const int e = static_cast<int>(u >> 23);
+        const unsigned long long m = e ? (u & 0x7fffffu) | 0x800000u : 0u;
+        return (m << (unit - 22)) >> min(max(128 - e - below(b), 0), 63);  // m * 2^(e - 150) in units
+    }
+    // no token below this lies in bin `b` or above it (a little further down, for what the bins' arithmetic rounds)
+    __device__ float reach(int b, float mx) const {
+        if (b >= kCoarse - 1) return -INFINITY;
+        const float far = static_cast<float>(b + 1) / scale * 1.00001f;
+        return mx - far - fmaxf(fabsf(mx), far) * 1e-6f;
+    }
+    __device__ double value(unsigned long long sum, int b) const { return ldexp(static_cast<double>(sum), -(unit + below(b))); }
+};
+
 // The row's maximum and its place, the smallest value above -inf, whether a NaN is in it: from the parts', by a wave.
 struct RowTop {
     Best best;
     float low;
     bool nan;
-    // whether the row's thresholds can be found by bins, and their scale
-    __device__ bool binned(int vocab, float inv_temp, float* scale) const {
-        const float range = fminf(best.value - low, kRange);
-        if (vocab > kMaxBinned || nan || !(fabsf(best.value) < INFINITY) || !(range > 1e-30f) || !weighs(inv_temp)) return false;
-        *scale = static_cast<float>(kBins - 1) / range;
-        return true;
+    // whether the row's thresholds can be found by bins
+    __device__ bool binned(int vocab, const RowParams& q, RowBins* bins) const {
+        const float range = fminf(best.value - low, fmaxf(kRange, 30.f * q.temp));
+        if (vocab > kMaxBinned || nan || !(fabsf(best.value) < INFINITY) || !(range > 1e-30f) || !weighs(q.inv_temp)) return false;
+        bins->scale = static_cast<float>(kCoarse - 1) / range;
+        bins->binades = q.inv_temp * 1.44269504f / bins->scale;
+        bins->unit = 62 - (32 - __clz(vocab));  // 2^(32 - clz) weights of less than two of a bin's stay below 2^63
+        return bins->binades <= static_cast<float>(bins->unit - 25);
     }
 };
 __device__ RowTop row_top(const SplitRow* w, int parts) {
@@ -616,6 +688,10 @@ __device__ RowTop row_top(const SplitRow* w, int parts) {
     t.low = __shfl(t.low, 0, FSIE_WAVE);
     return t;
 }
+// The same as an earlier launch has left it.
+__device__ __forceinline__ RowTop kept_top(const SplitRow* w) {
+    return RowTop{Best{w->top_max, w->top_index}, w->top_low, w->top_nan != 0};
+}
 
 // 64-token lines of a run, and the tokens of part `part`
 __device__ __forceinline__ int run_lines(int vocab) {
@@ -627,39 +703,61 @@ __device__ __forceinline__ void part_range(int vocab, int parts, int part, int* 
     *end = static_cast<int>(min(static_cast<int64_t>(vocab), tokens * (part + 1)));
 }
 
+constexpr int kAhead = 10;  // loads of a thread in a batch; the next batch is under way while one is worked on
+
 template <typename F>
 __device__ __forceinline__ void for_part(const float* __restrict__ row, int begin, int end, F body) {
-    for (int i0 = begin + threadIdx.x; i0 < end; i0 += kPart * kUnroll) {
-        float v[kUnroll];
+    const auto bring = [&](float (&v)[kAhead], int i0) {
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) v[u] = row[min(i0 + u * kPart, end - 1)];
+        for (int u = 0; u < kAhead; ++u) v[u] = row[min(i0 + static_cast<int>(threadIdx.x) + u * kPart, end - 1)];
+    };
+    if (begin >= end) return;
+    float v[kAhead], next[kAhead];
+    bring(v, begin);
+    for (int i0 = begin; i0 < end; i0 += kPart * kAhead) {
+        if (i0 + kPart * kAhead < end) bring(next, i0 + kPart * kAhead);
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u)
-            if (i0 + u * kPart < end) body(v[u], i0 + u * kPart);
+        for (int u = 0; u < kAhead; ++u) {
+            const int i = i0 + static_cast<int>(threadIdx.x) + u * kPart;
+            if (i < end) body(v[u], i);
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) v[u] = next[u];
     }
 }
 
-// The kept weights of the part's runs, a run a wave at a time, in the order of the lanes.
-__device__ void add_runs(const float* __restrict__ row, int vocab, int parts, int part, float mx, float inv_temp,
-                         uint32_t cut, double* run_sum) {
-    const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
-    const int lines = run_lines(vocab), per_part = kRuns / parts;
-    for (int q = wave; q < per_part; q += kPart / FSIE_WAVE) {
-        const int run = part * per_part + q;
-        const int64_t first = static_cast<int64_t>(run) * lines * FSIE_WAVE + lane;
-        double mine = 0.0;
-        for (int j0 = 0; j0 < lines; j0 += kUnroll) {
-            float v[kUnroll];
+// The sums of body(value, index) over the runs of part `part`, by THREADS threads: every wave takes neighbouring runs, whose
+// lines it goes through as one row of them.  A run's sum does not depend on who adds it up.
+template <int THREADS, typename F>
+__device__ __forceinline__ void add_runs(const float* __restrict__ row, int vocab, int parts, int part, double* run_sum, F body) {
+    const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / FSIE_WAVE);
+    const int lines = run_lines(vocab), runs = kRuns / parts / (THREADS / FSIE_WAVE), all = runs * lines;
+    int run = part * (kRuns / parts) + wave * runs, in_run = 0;
+    const int64_t first = static_cast<int64_t>(run) * lines * FSIE_WAVE + lane;
+    const auto bring = [&](float (&v)[kAhead], int j0) {
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u)
-                v[u] = row[min(first + static_cast<int64_t>(min(j0 + u, lines - 1)) * FSIE_WAVE, static_cast<int64_t>(vocab - 1))];
+        for (int u = 0; u < kAhead; ++u) v[u] = row[min(first + static_cast<int64_t>(j0 + u) * FSIE_WAVE, static_cast<int64_t>(vocab - 1))];
+    };
+    float v[kAhead], next[kAhead];
+    bring(v, 0);
+    double mine = 0.0;
+    for (int j0 = 0; j0 < all; j0 += kAhead) {
+        if (j0 + kAhead < all) bring(next, j0 + kAhead);
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u)
-                if (j0 + u < lines && first + static_cast<int64_t>(j0 + u) * FSIE_WAVE < vocab && order_key(v[u]) >= cut)
-                    mine += token_weight(v[u], mx, inv_temp);
+        for (int u = 0; u < kAhead; ++u) {
+            if (j0 + u >= all) break;
+            const int64_t i = first + static_cast<int64_t>(j0 + u) * FSIE_WAVE;
+            if (i < vocab) mine += body(v[u], static_cast<int>(i));
+            if (++in_run == lines) {
+                mine = wave_upto(mine);
+                if (lane == FSIE_WAVE - 1) run_sum[run] = mine;
+                mine = 0.0;
+                in_run = 0;
+                ++run;
+            }
         }
-        mine = wave_sum_f64(mine);
-        if (lane == 0) run_sum[run] = mine;
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) v[u] = next[u];
     }
 }
 
@@ -668,9 +766,9 @@ __global__ __launch_bounds__(kPart) void split_top_kernel(const float* __restric
     __shared__ int sidx[kPart / FSIE_WAVE], snan[kPart / FSIE_WAVE];
     SplitRow* w = ws + blockIdx.y;
     const int part = blockIdx.x, lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
-    // the bins and counters of the row are this launch's to clear
-    uint32_t* bins = reinterpret_cast<uint32_t*>(w->hi);
-    constexpr int kClear = static_cast<int>(offsetof(SplitRow, listed) / 4);
+    // the row's bins and counter are this launch's to clear
+    uint32_t* bins = reinterpret_cast<uint32_t*>(w->sum);
+    constexpr int kClear = static_cast<int>(offsetof(SplitRow, top_index) / 4);
     for (int i = part * kPart + threadIdx.x; i < kClear; i += parts * kPart) bins[i] = 0;
     int begin, end;
     part_range(vocab, parts, part, &begin, &end);
@@ -708,354 +806,497 @@ __global__ __launch_bounds__(kPart) void split_top_kernel(const float* __restric
     }
 }
 
-__global__ __launch_bounds__(kPart) void split_bins_kernel(const float* __restrict__ logits, int vocab, int parts,
-                                                           const float* __restrict__ temperature,
-                                                           const int32_t* __restrict__ top_k,
-                                                           const float* __restrict__ top_p, SplitRow* ws) {
-    __shared__ unsigned long long hi[kBins], lo[kBins];
-    __shared__ unsigned int count[kBins];
+// Rows without a threshold: the draw's sums.  The others: their bins, counted for top k, weighed for top p (not where the list will
+// hold all that top k keeps).  What bounds it are the weighed rows' instructions, some fifty a token.
+__global__ __launch_bounds__(kPart) void split_weigh_kernel(const float* __restrict__ logits, int vocab, int parts,
+                                                            const float* __restrict__ temperature,
+                                                            const int32_t* __restrict__ top_k,
+                                                            const float* __restrict__ top_p, SplitRow* ws) {
+    __shared__ unsigned long long sum[kCoarse];
+    __shared__ unsigned int count[kCoarse];
     const int r = blockIdx.y;
     const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
-    if (!(q.temp > 0.f)) return;
     SplitRow* w = ws + r;
     const RowTop top = row_top(w, parts);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        w->top_max = top.best.value;
+        w->top_index = top.best.index;
+        w->top_low = top.low;
+        w->top_nan = top.nan;
+    }
+    if (!(q.temp > 0.f)) return;
     const float* row = logits + static_cast<int64_t>(r) * vocab;
     const float mx = top.best.value;
     if (!q.cuts) {
-        add_runs(row, vocab, parts, blockIdx.x, mx, q.inv_temp, 0, w->run_sum);
+        add_runs<kPart>(row, vocab, parts, blockIdx.x, w->run_sum, [&](float v, int) { return token_weight(v, mx, q.inv_temp); });
         return;
     }
-    float scale;
-    if (!top.binned(vocab, q.inv_temp, &scale)) return;
-    for (int b = threadIdx.x; b < kBins; b += kPart) {
-        hi[b] = lo[b] = 0;
+    RowBins bins;
+    if (!top.binned(vocab, q, &bins)) return;
+    const bool weigh = q.p < 1.f && !q.all_listed(), counts = q.k > 0;
+    for (int b = threadIdx.x; b < kCoarse; b += kPart) {
+        sum[b] = 0;
         count[b] = 0;
     }
     __syncthreads();
-    const int hi_bits = 63 - (32 - __clz(vocab));  // vocab < 2^(32 - clz): the sum of all weights stays below 2^63
     int begin, end;
     part_range(vocab, parts, blockIdx.x, &begin, &end);
-    for_part(row, begin, end, [&](float v, int) {
-        const int b = bin_of(v, mx, scale);
-        atomicAdd(&count[b], 1u);
-        if (q.p < 1.f) {
-            const Limbs m = limbs_of(expf((v - mx) * q.inv_temp), hi_bits);
-            if (m.hi) atomicAdd(&hi[b], m.hi);
-            if (m.lo) atomicAdd(&lo[b], m.lo);
-        }
-    });
+    if (weigh) {
+        for_part(row, begin, end, [&](float v, int) {
+            const int b = bins.bin(v, mx);
+            if (counts) atomicAdd(&count[b], 1u);
+            const unsigned long long m = bins.weight(expf((v - mx) * q.inv_temp), b);
+            if (m) atomicAdd(&sum[b], m);
+        });
+    } else {
+        for_part(row, begin, end, [&](float v, int) { atomicAdd(&count[bins.bin(v, mx)], 1u); });
+    }
     __syncthreads();
-    for (int b = threadIdx.x; b < kBins; b += kPart) {
-        if (!count[b]) continue;
-        atomicAdd(&w->count[b], count[b]);
-        if (hi[b]) atomicAdd(&w->hi[b], hi[b]);
-        if (lo[b]) atomicAdd(&w->lo[b], lo[b]);
+    for (int b = threadIdx.x; b < kCoarse; b += kPart) {
+        if (counts && count[b]) atomicAdd(&w->count[b], count[b]);
+        if (weigh && sum[b]) atomicAdd(&w->sum[b], sum[b]);
     }
 }
 
-// The running sums of the bins' values from the maximum down, found by a workgroup of THREADS: where `target` is first
-// reached, and the sum above that bin.
+// The running sums of the bins' values from the maximum down, over a workgroup of THREADS, and the bin in which one first
+// reaches a target.  Fixed order of additions.
 struct Found {
-    int bin;       // -1: nowhere
-    double above, total;
+    int bin;  // -1: nowhere
+    double above;
 };
-// `v`: the values of this thread's own kBins / THREADS neighbouring bins (read from memory once for all searches).
 template <int THREADS>
-__device__ Found find_in_bins(double target, const double (&v)[kBins / THREADS]) {
-    constexpr int PER = kBins / THREADS;
-    __shared__ double wave_sum[THREADS / FSIE_WAVE];
-    __shared__ Found found;
-    const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
-    double run = 0.0;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) run += v[i];
-#pragma unroll
-    for (int off = 1; off < FSIE_WAVE; off <<= 1) {
-        const double other = __shfl_up(run, off, FSIE_WAVE);
-        if (lane >= off) run += other;
-    }
-    __syncthreads();
-    if (lane == FSIE_WAVE - 1) wave_sum[wave] = run;
-    if (threadIdx.x == 0) found.bin = -1;
-    __syncthreads();
-    double base = 0.0, total = 0.0;
-    for (int i = 0; i < THREADS / FSIE_WAVE; ++i) {
-        if (i == wave) base = total;
-        total += wave_sum[i];
-    }
-    const double left = __shfl_up(run, 1, FSIE_WAVE);  // (all lanes together: a shuffle reads active lanes only)
-    double before = base + (lane ? left : 0.0);
-    if (before < target && target <= base + run) {
-        int bin = static_cast<int>(threadIdx.x) * PER;
-#pragma unroll
-        for (int i = 0; i < PER - 1; ++i)
-            if (bin == static_cast<int>(threadIdx.x) * PER + i && target > before + v[i]) {
-                before += v[i];
-                ++bin;
-            }
-        found.bin = bin;
-        found.above = before;
-    }
-    __syncthreads();
-    const Found out{found.bin, found.above, total};
-    __syncthreads();
-    return out;
-}
+struct BinScan {
+    static constexpr int PER = kCoarse > THREADS ? kCoarse / THREADS : 1;  // (threads beyond the bins have none: 0)
+    double v[PER];  // the values of this thread's neighbouring bins
+    double before, upto, total;
 
+    // `wave_sum`: a number a wave, in LDS, of this scan alone
+    __device__ void run(double* wave_sum) {
+        const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
+        double sum = 0.0;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) sum += v[i];
+        sum = wave_upto(sum);
+        if (lane == FSIE_WAVE - 1) wave_sum[wave] = sum;
+        const double left = __shfl_up(sum, 1, FSIE_WAVE);  // (all lanes together: a shuffle reads active lanes only)
+        __syncthreads();
+        double base = 0.0;
+        total = 0.0;
+#pragma unroll
+        for (int i = 0; i < THREADS / FSIE_WAVE; ++i) {
+            if (i == wave) base = total;
+            total += wave_sum[i];
+        }
+        before = base + (lane ? left : 0.0);
+        upto = base + sum;
+    }
+    // `found`: in LDS, of this search alone, its bin set to -1 before the last barrier
+    __device__ Found find(double target, Found* found) const {
+        if (before < target && target <= upto) {
+            int bin = static_cast<int>(threadIdx.x) * PER;
+            double above = before;
+#pragma unroll
+            for (int i = 0; i < PER - 1; ++i)
+                if (bin == static_cast<int>(threadIdx.x) * PER + i && target > above + v[i]) {
+                    above += v[i];
+                    ++bin;
+                }
+            *found = Found{bin, above};
+        }
+        __syncthreads();
+        return *found;
+    }
+    // the sum of the bins above `bin`, and with it
+    __device__ void around(int bin, double* above, double* with) const {
+        __shared__ double shared[2];
+        if (static_cast<int>(threadIdx.x) == bin / PER) {
+            double sum = before;
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                if (bin % PER == i) {
+                    shared[0] = sum;
+                    shared[1] = sum + v[i];
+                }
+                sum += v[i];
+            }
+        }
+        __syncthreads();
+        *above = shared[0];
+        *with = shared[1];
+    }
+};
+
+// Every workgroup of the row finds the bins of its thresholds, lists the part's tokens of them and adds up the draw's sums
+// of those above, which are kept whatever the cut among the listed ones will be.  Most tokens lie below all that: a wave lays those
+// that do not side by side in LDS, so that bins and exponentials are computed of these alone (of all tokens of a line where one of them is kept:
+// 9 us of a top-p row's pass over 19,008 tokens, and 3 so).
+constexpr int kNear = kAhead * FSIE_WAVE + 3 * FSIE_WAVE;
+static_assert(kMaxBinned <= 1 << 23 && kRuns <= 1 << 8, "a token's place and its run within the part fit 32 bits");
 __global__ __launch_bounds__(kPart) void split_list_kernel(const float* __restrict__ logits, int vocab, int parts,
                                                            const float* __restrict__ temperature,
                                                            const int32_t* __restrict__ top_k,
                                                            const float* __restrict__ top_p, SplitRow* ws) {
+    __shared__ float near[kPart / FSIE_WAVE][kNear];
+    __shared__ unsigned int near_at[kPart / FSIE_WAVE][kNear];
+    __shared__ unsigned long long run_hi[kRuns], run_lo[kRuns];
+    __shared__ double wave_sum[2][kPart / FSIE_WAVE];
+    __shared__ Found found[3];
     const int r = blockIdx.y;
     const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
     if (!q.cuts) return;
     SplitRow* w = ws + r;
-    const RowTop top = row_top(w, parts);
-    float scale;
-    if (!top.binned(vocab, q.inv_temp, &scale)) return;
-    const int hi_bits = 63 - (32 - __clz(vocab));
-    constexpr int PER = kBins / kPart;
+    const RowTop top = kept_top(w);
+    RowBins bins;
+    if (!top.binned(vocab, q, &bins)) return;
+    const float mx = top.best.value;
+    constexpr int PER = kCoarse / kPart;
     const int b0 = static_cast<int>(threadIdx.x) * PER;
-    double counts[PER], weights[PER], some[PER];
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        counts[i] = static_cast<double>(w->count[b0 + i]);
-        weights[i] = value_of(Limbs{w->hi[b0 + i], w->lo[b0 + i]}, hi_bits);
-    }
     int k_bin = -1, from = 0, upto = -1;
-    if (q.k > 0) k_bin = find_in_bins<kPart>(q.k, counts).bin;
-    if (q.p < 1.f) {
-        // top p of what top k keeps: all of the bins above its own and some of that one, so the last kept token lies
-        // between the bins that the least and the most of it give
-#pragma unroll
-        for (int i = 0; i < PER; ++i) some[i] = k_bin < 0 || b0 + i <= k_bin ? weights[i] : 0.0;
-        const double most = find_in_bins<kPart>(INFINITY, some).total;
-        double least = most;
-        if (k_bin >= 0) {
-#pragma unroll
-            for (int i = 0; i < PER; ++i) some[i] = b0 + i < k_bin ? weights[i] : 0.0;
-            least = find_in_bins<kPart>(INFINITY, some).total;
-        }
-        const double p = static_cast<double>(q.p);
-        if (p > 0.0) {
-            upto = find_in_bins<kPart>(p * most, weights).bin;
-            from = k_bin < 0 ? upto : find_in_bins<kPart>(p * least, weights).bin;
-            from = max(0, from);
-        }
+    double above_k = 0.0, above = 0.0, target = 0.0;
+    BinScan<kPart> scan;
+    for (int i = threadIdx.x; i < kRuns / parts; i += kPart) run_hi[i] = run_lo[i] = 0;
+    if (threadIdx.x == 0) {
+        found[0].bin = found[1].bin = found[2].bin = -1;
     }
-    int begin, end;
-    part_range(vocab, parts, blockIdx.x, &begin, &end);
-    for_part(logits + static_cast<int64_t>(r) * vocab, begin, end, [&](float v, int) {
-        const int b = bin_of(v, top.best.value, scale);
-        if (b == k_bin || (from <= b && b <= upto)) {
-            const unsigned int at = atomicAdd(&w->n_listed, 1u);
-            if (at < kKeep) w->listed[at] = v;
+    if (q.k > 0) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) scan.v[i] = static_cast<double>(w->count[b0 + i]);
+        scan.run(wave_sum[0]);
+        const Found at = scan.find(q.k, &found[0]);
+        k_bin = at.bin;
+        above_k = at.above;
+        from = upto = k_bin;
+    }
+    if (q.all_listed()) {
+        from = 0;
+    } else if (q.p < 1.f) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) scan.v[i] = bins.value(w->sum[b0 + i], b0 + i);
+        scan.run(wave_sum[1]);
+        const double p = static_cast<double>(q.p);
+        if (k_bin >= 0) {
+            // top p of what top k keeps: all of the bins above its own and some of that one, so the last kept token lies
+            // between the bins that the least and the most of it give
+            double least, most;
+            scan.around(k_bin, &least, &most);
+            upto = scan.find(p * most, &found[1]).bin;
+            from = scan.find(p * least, &found[2]).bin;
+        } else if (q.k == 0) {
+            target = p * scan.total;
+            const Found at = scan.find(target, &found[1]);
+            from = upto = at.bin;
+            above = at.above;
         }
-    });
+        from = max(from, 0);  // (nothing to reach: the largest token, which lies in the first bin)
+        upto = max(upto, 0);
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        w->k_bin = k_bin;
+        w->from = from;
+        w->upto = upto;
+        w->above_k = above_k;
+        w->above = above;
+        w->target = target;
+    }
+    __syncthreads();
+    const float* row = logits + static_cast<int64_t>(r) * vocab;
+    const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / FSIE_WAVE);
+    const int lines = run_lines(vocab), runs = kRuns / parts / (kPart / FSIE_WAVE), all = runs * lines;
+    const int first_run = blockIdx.x * (kRuns / parts), hi_bits = 63 - (32 - __clz(vocab));
+    const int first = (first_run + wave * runs) * lines * FSIE_WAVE + lane;
+    const float reach = bins.reach(max(k_bin, upto), mx);
+    int run = wave * runs, in_run = 0, n = 0;
+    const auto settle = [&]() {
+        for (int at = lane; at < n; at += FSIE_WAVE) {
+            const float v = near[wave][at];
+            const unsigned int place = near_at[wave][at];
+            const int b = bins.bin(v, mx);
+            if (b == k_bin || (from <= b && b <= upto)) {
+                const unsigned int slot = atomicAdd(&w->n_listed, 1u);
+                if (slot < kKeep) {
+                    w->listed[slot] = v;
+                    w->listed_at[slot] = static_cast<int>(place & 0x7fffffu);
+                }
+            } else if (b < from) {
+                const Limbs m = limbs_of(expf((v - mx) * q.inv_temp), hi_bits);
+                if (m.hi) atomicAdd(&run_hi[place >> 23], m.hi);
+                if (m.lo) atomicAdd(&run_lo[place >> 23], m.lo);
+            }
+        }
+        n = 0;
+    };
+    const auto bring = [&](float (&v)[kAhead], int j0) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) v[u] = row[min(first + (j0 + u) * FSIE_WAVE, vocab - 1)];
+    };
+    float v[kAhead], next[kAhead];
+    bring(v, 0);
+    for (int j0 = 0; j0 < all; j0 += kAhead) {
+        if (j0 + kAhead < all) bring(next, j0 + kAhead);
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            if (j0 + u >= all) break;
+            const int i = first + (j0 + u) * FSIE_WAVE;
+            const bool is = v[u] >= reach && i < vocab;
+            const unsigned long long mask = __ballot(is);
+            if (mask) {
+                const int slot = n + __builtin_amdgcn_mbcnt_hi(static_cast<unsigned int>(mask >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<unsigned int>(mask), 0));
+                if (is) {
+                    near[wave][slot] = v[u];
+                    near_at[wave][slot] = static_cast<unsigned int>(run) << 23 | static_cast<unsigned int>(i);
+                }
+                n += __popcll(mask);
+            }
+            if (++in_run == lines) {
+                in_run = 0;
+                ++run;
+            }
+        }
+        if (n > kNear - kAhead * FSIE_WAVE) settle();
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) v[u] = next[u];
+    }
+    settle();
+    __syncthreads();
+    for (int i = threadIdx.x; i < kRuns / parts; i += kPart) w->run_sum[first_run + i] = value_of(Limbs{run_hi[i], run_lo[i]}, hi_bits);
 }
 
-// The key of the first listed token, from the largest down, at which reached(key's tokens and all larger) holds, by
-// bisection over the keys; what is summed are integers, so the list's order does not matter.
-template <typename S, typename F>
-__device__ uint32_t bisect_list(const uint32_t* keys, int n, uint32_t key_max, S value, F reached) {
-    __shared__ unsigned long long sum_hi, sum_lo;
-    uint32_t lo = 0, hi = key_max;
+// What the last launch holds of a row's list: kHeld tokens a thread, in registers.
+constexpr int kHeld = kKeep / kThreads;
+struct Search {  // one of a key, cleared before the last barrier
+    unsigned long long fine[kFine], member[kPairs], wave_sum[kWaves], before, sum;
+    uint32_t member_key[kPairs], cut;
+    unsigned int members, few;
+    int at;
+    __device__ void clear() {
+        fine[threadIdx.x] = 0;
+        if (threadIdx.x == 0) {
+            members = 0;
+            few = 0;
+            cut = 0;
+            at = -1;
+        }
+    }
+};
+struct Cutting {
+    Search search[2];
+    unsigned long long coarse[kCoarse], run_hi[kRuns], run_lo[kRuns];
+    double wave_sum[kWaves];
+    Found found;
+};
+static_assert(kFine == kThreads && kCoarse <= kThreads, "a bin a thread");
+
+constexpr unsigned int kFew = 64;
+// The key of the first token of bin `bin`, from the largest down, at which above + amount(sum of its and all larger
+// tokens' values) reaches `target`; 0: none.  FEW: there may be few tokens in the bin, which are then compared with each other at once
+// (two barriers instead of five, 0.9 us).  Else the bin's tokens (`in`) are dealt to kFine bins, of which one holds it; that one's few
+// tokens are compared with each other, or their keys bisected.  What is summed are integers, so the list's order does not matter.
+template <bool FEW, typename A>
+__device__ uint32_t key_reaching(Search& s, const RowBins& bins, float mx, int bin, const float (&v)[kHeld], const bool (&in)[kHeld],
+                                 const unsigned long long (&value)[kHeld], double above, double target, A amount) {
+    const int lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
+    const auto reaches = [&](unsigned long long sum) { return target <= above + amount(sum); };
+    // among the first n members, with `before` above them
+    const auto compare = [&](unsigned int n, unsigned long long before) {
+        if (threadIdx.x < n) {
+            const uint32_t key = s.member_key[threadIdx.x];
+            unsigned long long over = before, upto = before;
+            for (unsigned int j = 0; j < n; ++j) {
+                if (s.member_key[j] >= key) upto += s.member[j];
+                if (s.member_key[j] > key) over += s.member[j];
+            }
+            if (!reaches(over) && reaches(upto)) s.cut = key;  // (equal keys write the same)
+        }
+        __syncthreads();
+        return s.cut;
+    };
+    const auto join = [&](unsigned int& count, int j, unsigned int most) {
+        const unsigned int m = atomicAdd(&count, 1u);
+        if (m < most) {
+            s.member_key[m] = order_key(v[j]);
+            s.member[m] = value[j];
+        }
+    };
+    if constexpr (FEW) {
+#pragma unroll
+        for (int j = 0; j < kHeld; ++j)
+            if (in[j]) join(s.few, j, kFew);
+        __syncthreads();
+        if (s.few <= kFew) return compare(s.few, 0);
+    }
+    int f[kHeld];
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) {
+        f[j] = -1;
+        if (!in[j]) continue;
+        f[j] = static_cast<int>(fminf(fmaxf(((mx - v[j]) * bins.scale - static_cast<float>(bin)) * kFine, 0.f), static_cast<float>(kFine - 1)));
+        atomicAdd(&s.fine[f[j]], value[j]);
+    }
+    __syncthreads();
+    const unsigned long long mine = s.fine[threadIdx.x];
+    unsigned long long run = wave_upto(mine);
+    if (lane == FSIE_WAVE - 1) s.wave_sum[wave] = run;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) run += i < wave ? s.wave_sum[i] : 0;
+    if (mine && !reaches(run - mine) && reaches(run)) {
+        s.at = static_cast<int>(threadIdx.x);
+        s.before = run - mine;
+    }
+    __syncthreads();
+    const int at = s.at;
+    if (at < 0) return 0;
+    const unsigned long long before = s.before;
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j)
+        if (f[j] == at) join(s.members, j, kPairs);
+    __syncthreads();
+    if (s.members <= kPairs) return compare(s.members, before);
+    uint32_t lo = 0, hi = order_key(mx);
     while (lo < hi) {
         const uint32_t mid = lo + (hi - lo) / 2 + ((hi - lo) & 1);
         __syncthreads();
-        if (threadIdx.x == 0) sum_hi = sum_lo = 0;
+        if (threadIdx.x == 0) s.sum = before;
         __syncthreads();
-        Limbs mine{0, 0};
-        for (int i = threadIdx.x; i < n; i += kThreads)
-            if (keys[i] >= mid) {
-                const Limbs v = value(i);
-                mine.hi += v.hi;
-                mine.lo += v.lo;
-            }
-        if (mine.hi) atomicAdd(&sum_hi, mine.hi);
-        if (mine.lo) atomicAdd(&sum_lo, mine.lo);
+#pragma unroll
+        for (int j = 0; j < kHeld; ++j)
+            if (f[j] == at && order_key(v[j]) >= mid) atomicAdd(&s.sum, value[j]);
         __syncthreads();
-        if (reached(Limbs{sum_hi, sum_lo})) lo = mid; else hi = mid - 1;
+        if (reaches(s.sum)) lo = mid; else hi = mid - 1;
     }
     return lo;
 }
 
-__global__ __launch_bounds__(kThreads) void split_cut_kernel(const float* __restrict__ logits, int vocab, int parts,
-                                                             const float* __restrict__ temperature,
-                                                             const int32_t* __restrict__ top_k,
-                                                             const float* __restrict__ top_p, SplitRow* ws) {
-    __shared__ uint32_t keys[kKeep];
-    __shared__ short bin_of_key[kKeep];
-    __shared__ unsigned long long w_hi[kPairs], w_lo[kPairs];
-    __shared__ double sdbl[kWaves];
-    __shared__ unsigned long long kept_hi, kept_lo;
-    __shared__ uint32_t cut_found;
-    __shared__ unsigned int of_bin;
-    const int r = blockIdx.x;
-    const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
-    if (!q.cuts) return;
-    SplitRow* w = ws + r;
-    const RowTop top = row_top(w, parts);
-    const float* row = logits + static_cast<int64_t>(r) * vocab;
-    const float mx = top.best.value;
-    const uint32_t key_max = order_key(mx);
-    const int n = static_cast<int>(min(w->n_listed, static_cast<unsigned int>(kKeep + 1)));
-    float scale = 0.f;
-    bool fits = top.binned(vocab, q.inv_temp, &scale) && n <= kKeep;  // (the same in every thread)
+// The key at which the row's kept set ends, from its list; 0 where the list does not tell.
+__device__ uint32_t cut_of_list(Cutting& s, const SplitRow* w, const RowParams& q, const RowBins& bins, float mx,
+                                const float (&v)[kHeld], int n) {
     uint32_t cut = 0;
-    if (fits) {
-        const int hi_bits = 63 - (32 - __clz(vocab));
-        for (int i = threadIdx.x; i < n; i += kThreads) {
-            const float v = w->listed[i];
-            keys[i] = order_key(v);
-            bin_of_key[i] = static_cast<short>(bin_of(v, mx, scale));
-            if (i < kPairs) {
-                const Limbs m = limbs_of(expf((v - mx) * q.inv_temp), hi_bits);
-                w_hi[i] = m.hi;
-                w_lo[i] = m.lo;
-            }
-        }
-        const auto listed_weight = [&](int i) {
-            if (i < kPairs) return Limbs{w_hi[i], w_lo[i]};
-            return limbs_of(expf((w->listed[i] - mx) * q.inv_temp), hi_bits);
-        };
-        if (threadIdx.x == 0) {
-            kept_hi = kept_lo = 0;
-            cut_found = 0;
-            of_bin = 0;
-        }
-        __syncthreads();
-        int k_bin = -1;
-        constexpr int PER = kBins / kThreads;
-        const int b0 = static_cast<int>(threadIdx.x) * PER;
-        double values[PER];
-        if (q.k > 0) {
+    int bin[kHeld];
+    bool in[kHeld];
+    unsigned long long value[kHeld];
+    const int k_bin = w->k_bin;
+    Found at{w->from, w->above};
+    double target = w->target;
 #pragma unroll
-            for (int i = 0; i < PER; ++i) values[i] = static_cast<double>(w->count[b0 + i]);
-            const Found at = find_in_bins<kThreads>(q.k, values);
-            k_bin = at.bin;
-            const long long want = q.k - static_cast<long long>(at.above);
-            if (k_bin < 0) {
-                fits = false;
-            } else if (n <= kPairs) {
-                if (static_cast<int>(threadIdx.x) < n && bin_of_key[threadIdx.x] == k_bin) {
-                    const uint32_t mine = keys[threadIdx.x];
-                    int over = 0, upto = 0;
-                    for (int j = 0; j < n; ++j) {
-                        const bool same = bin_of_key[j] == k_bin;
-                        over += same && keys[j] > mine;
-                        upto += same && keys[j] >= mine;
-                    }
-                    if (over < want && want <= upto) cut_found = mine;  // (equal keys write the same)
-                }
-                __syncthreads();
-                cut = cut_found;
-            } else {
-                cut = bisect_list(keys, n, key_max, [&](int i) { return Limbs{bin_of_key[i] == k_bin, 0}; },
-                                  [&](Limbs s) { return static_cast<long long>(s.hi) >= want; });
-            }
-            if (cut == 0) fits = false;
-        }
-        if (fits && q.p < 1.f) {
-            __syncthreads();
-            Limbs kept{0, 0};  // of top k's bin
-            for (int i = threadIdx.x; i < n; i += kThreads)
-                if (bin_of_key[i] == k_bin && keys[i] >= cut) {
-                    const Limbs m = listed_weight(i);
-                    kept.hi += m.hi;
-                    kept.lo += m.lo;
-                }
-            if (kept.hi) atomicAdd(&kept_hi, kept.hi);
-            if (kept.lo) atomicAdd(&kept_lo, kept.lo);
-            if (threadIdx.x == 0) cut_found = 0;
-            __syncthreads();
+    for (int j = 0; j < kHeld; ++j)
+        bin[j] = static_cast<int>(threadIdx.x) + j * kThreads < n ? bins.bin(v[j], mx) : -2;
+    if (q.k > 0) {
+        if (k_bin < 0) return 0;
 #pragma unroll
-            for (int i = 0; i < PER; ++i) {
-                const int b = b0 + i;
-                values[i] = value_of(Limbs{w->hi[b], w->lo[b]}, hi_bits);
-                if (k_bin >= 0 && b >= k_bin) values[i] = b == k_bin ? value_of(Limbs{kept_hi, kept_lo}, hi_bits) : 0.0;
-            }
-            const double target = static_cast<double>(q.p) * find_in_bins<kThreads>(INFINITY, values).total;
-            if (!(target > 0.0)) {
-                cut = key_max;
-            } else {
-                const Found at = find_in_bins<kThreads>(target, values);
-                const auto counts = [&](int i) { return bin_of_key[i] == at.bin && keys[i] >= cut; };
-                const auto reaches = [&](Limbs s) { return target <= at.above + value_of(s, hi_bits); };
-                // (rounding may have put the target outside the bins that were listed)
-                unsigned int mine_of_bin = 0;
-                for (int i = threadIdx.x; i < n; i += kThreads) mine_of_bin += bin_of_key[i] == at.bin;
-                if (mine_of_bin) atomicAdd(&of_bin, mine_of_bin);
-                __syncthreads();
-                uint32_t found = 0;
-                if (at.bin < 0 || of_bin != w->count[max(at.bin, 0)]) {
-                    fits = false;
-                } else if (n <= kPairs) {
-                    if (static_cast<int>(threadIdx.x) < n && counts(threadIdx.x)) {
-                        const uint32_t mine = keys[threadIdx.x];
-                        Limbs over{0, 0}, upto{0, 0};
-                        for (int j = 0; j < n; ++j) {
-                            if (!counts(j) || keys[j] < mine) continue;
-                            upto.hi += w_hi[j];
-                            upto.lo += w_lo[j];
-                            if (keys[j] > mine) {
-                                over.hi += w_hi[j];
-                                over.lo += w_lo[j];
-                            }
-                        }
-                        if (!reaches(over) && reaches(upto)) cut_found = mine;
-                    }
-                    __syncthreads();
-                    found = cut_found;
-                } else {
-                    found = bisect_list(keys, n, key_max, [&](int i) { return counts(i) ? listed_weight(i) : Limbs{0, 0}; }, reaches);
-                }
-                if (found == 0) fits = false;
-                cut = found;
-            }
+        for (int j = 0; j < kHeld; ++j) {
+            in[j] = bin[j] == k_bin;
+            value[j] = 1;
         }
+        cut = key_reaching<true>(s.search[0], bins, mx, k_bin, v, in, value, w->above_k, static_cast<double>(q.k),
+                           [](unsigned long long sum) { return static_cast<double>(sum); });
+        if (cut == 0 || !(q.p < 1.f)) return cut;
     }
-    if (!fits) {
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) value[j] = bin[j] >= 0 ? bins.weight(expf((v[j] - mx) * q.inv_temp), bin[j]) : 0;
+    if (q.k > 0) {
+        // the weights of what top k keeps: of its own bin from the list, of those above from the list or the row's bins
+        const int b = static_cast<int>(threadIdx.x);
+#pragma unroll
+        for (int j = 0; j < kHeld; ++j)
+            if (bin[j] >= 0 && order_key(v[j]) >= cut && (bin[j] == k_bin || q.all_listed())) atomicAdd(&s.coarse[bin[j]], value[j]);
+        const unsigned long long others = !q.all_listed() && b < k_bin ? w->sum[b] : 0;
         __syncthreads();
-        cut = cut_by_bisection(row, vocab, mx, q.inv_temp, q.k, q.p, sdbl);
+        BinScan<kThreads> scan;
+        scan.v[0] = b < kCoarse ? bins.value(s.coarse[b] + others, b) : 0.0;
+        scan.run(s.wave_sum);
+        target = static_cast<double>(q.p) * scan.total;
+        at = scan.find(target, &s.found);
+        // (rounding may have put the target outside the bins that were listed)
+        if (target > 0.0 && !(at.bin == k_bin || (w->from <= at.bin && at.bin <= w->upto))) return 0;
     }
-    if (threadIdx.x == 0) w->cut = cut;
+    if (!(target > 0.0)) return order_key(mx);
+    if (at.bin < 0) return 0;
+#pragma unroll
+    for (int j = 0; j < kHeld; ++j) in[j] = bin[j] == at.bin && order_key(v[j]) >= cut;
+    const auto weight = [&](unsigned long long sum) { return bins.value(sum, at.bin); };
+    return q.k > 0 ? key_reaching<true>(s.search[1], bins, mx, at.bin, v, in, value, at.above, target, weight)
+                   : key_reaching<false>(s.search[1], bins, mx, at.bin, v, in, value, at.above, target, weight);
 }
 
-__global__ __launch_bounds__(kPart) void split_runs_kernel(const float* __restrict__ logits, int vocab, int parts,
-                                                           const float* __restrict__ temperature,
-                                                           const int32_t* __restrict__ top_k,
-                                                           const float* __restrict__ top_p, SplitRow* ws) {
-    const int r = blockIdx.y;
-    const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
-    if (!q.cuts) return;  // (rows without a threshold have their sums already)
-    SplitRow* w = ws + r;
-    add_runs(logits + static_cast<int64_t>(r) * vocab, vocab, parts, blockIdx.x, row_top(w, parts).best.value, q.inv_temp,
-             w->cut, w->run_sum);
-}
-
-__global__ __launch_bounds__(FSIE_WAVE) void split_draw_kernel(const float* __restrict__ logits, int vocab, int parts,
-                                                               const float* __restrict__ temperature,
-                                                               const int32_t* __restrict__ top_k,
-                                                               const float* __restrict__ top_p,
-                                                               const double* __restrict__ uniform, const SplitRow* ws,
-                                                               int32_t* __restrict__ out) {
+__global__ __launch_bounds__(kThreads) void split_draw_kernel(const float* __restrict__ logits, int vocab, int parts,
+                                                              const float* __restrict__ temperature,
+                                                              const int32_t* __restrict__ top_k,
+                                                              const float* __restrict__ top_p,
+                                                              const double* __restrict__ uniform, const SplitRow* ws,
+                                                              int32_t* __restrict__ out) {
+    __shared__ union {
+        Cutting list;
+        Binned bins;
+    } s;
+    __shared__ double run_sum[kRuns], sdbl[kWaves];
     const int r = blockIdx.x;
     const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
     const SplitRow* w = ws + r;
-    const Best top = row_top(w, parts).best;
+    const RowTop top = kept_top(w);
     if (!(q.temp > 0.f)) {
-        if (threadIdx.x == 0) out[r] = top.index;
+        if (threadIdx.x == 0) out[r] = top.best.index;
         return;
     }
-    draw_from_runs(logits + static_cast<int64_t>(r) * vocab, vocab, top, q.inv_temp, q.cuts ? w->cut : 0, uniform[r],
-                   w->run_sum, -1, out + r);
+    const float* row = logits + static_cast<int64_t>(r) * vocab;
+    const float mx = top.best.value;
+    uint32_t cut = 0;  // tokens with key >= cut are kept
+    double sum = threadIdx.x < kRuns ? w->run_sum[threadIdx.x] : 0.0;
+    if (q.cuts) {
+        RowBins bins;
+        const unsigned int listed = w->n_listed;
+        const int n = static_cast<int>(min(listed, static_cast<unsigned int>(kKeep)));
+        float v[kHeld];
+        int at[kHeld];
+#pragma unroll
+        for (int j = 0; j < kHeld; ++j) {
+            const int i = static_cast<int>(threadIdx.x) + j * kThreads;
+            v[j] = i < n ? w->listed[i] : 0.f;
+            at[j] = i < n ? w->listed_at[i] : 0;
+        }
+        s.list.search[0].clear();
+        s.list.search[1].clear();
+        if (threadIdx.x < kCoarse) s.list.coarse[threadIdx.x] = 0;
+        if (threadIdx.x < kRuns) s.list.run_hi[threadIdx.x] = s.list.run_lo[threadIdx.x] = 0;
+        if (threadIdx.x == 0) s.list.found.bin = -1;
+        __syncthreads();
+        // (all of it the same in every thread)
+        if (top.binned(vocab, q, &bins) && listed <= kKeep) cut = cut_of_list(s.list, w, q, bins, mx, v, n);
+        if (cut != 0) {
+            // the kept ones of the listed tokens join the sums of their runs
+            const int hi_bits = 63 - (32 - __clz(vocab)), tokens = run_lines(vocab) * FSIE_WAVE;
+#pragma unroll
+            for (int j = 0; j < kHeld; ++j)
+                if (static_cast<int>(threadIdx.x) + j * kThreads < n && order_key(v[j]) >= cut) {
+                    const Limbs m = limbs_of(expf((v[j] - mx) * q.inv_temp), hi_bits);
+                    const int run = at[j] / tokens;
+                    if (m.hi) atomicAdd(&s.list.run_hi[run], m.hi);
+                    if (m.lo) atomicAdd(&s.list.run_lo[run], m.lo);
+                }
+            __syncthreads();
+            if (threadIdx.x < kRuns) sum += value_of(Limbs{s.list.run_hi[threadIdx.x], s.list.run_lo[threadIdx.x]}, hi_bits);
+        } else {
+            // a row that its list does not settle: as if it were not shared
+            __syncthreads();
+            if (vocab > kMaxBinned || !(fabsf(mx) < INFINITY) ||
+                !cut_by_bins(s.bins, row, vocab, mx, top.low, top.nan, q.inv_temp, q.k, q.p, &cut)) {
+                __syncthreads();
+                cut = cut_by_bisection(row, vocab, mx, q.inv_temp, q.k, q.p, sdbl);
+            }
+            add_runs<kThreads>(row, vocab, 1, 0, run_sum, [&](float v, int) { return order_key(v) >= cut ? token_weight(v, mx, q.inv_temp) : 0.0; });
+            __syncthreads();
+            if (threadIdx.x < kRuns) sum = run_sum[threadIdx.x];
+        }
+    }
+    if (threadIdx.x < kRuns) run_sum[threadIdx.x] = sum;
+    __syncthreads();
+    draw_from_runs(row, vocab, top.best, q.inv_temp, cut, uniform[r], run_sum, out + r);
 }
 
 }  // namespace
 
-extern "C" int64_t fsie_sample_workspace(int n_rows, int vocab) {
-    return vocab >= kSplitFrom && n_rows > 0 && vocab / n_rows >= kTokensForRow ? static_cast<int64_t>(n_rows) * static_cast<int64_t>(sizeof(SplitRow)) : 0;
+extern "C" int64_t fsie_sample_workspace(int n_rows, int vocab, int thresholds) {
+    const bool shared = vocab >= kSplitFrom && vocab <= (1 << 30) && n_rows > 0 && n_rows <= (thresholds ? kMostRows : kMostPlainRows);
+    return shared ? static_cast<int64_t>(n_rows) * static_cast<int64_t>(sizeof(SplitRow)) : 0;
 }
 
 extern "C" int fsie_sample(const float* logits, int n_rows, int vocab, const float* temperature,
@@ -1080,18 +1321,14 @@ extern "C" int fsie_sample_split(const float* logits, int n_rows, int vocab, con
     FSIE_REQUIRE(workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
                  "sample_split: a workspace on 16 bytes is needed");
     SplitRow* ws = static_cast<SplitRow*>(workspace);
-    // a power of two of parts that gives every compute unit about four workgroups
+    // a power of two of parts that gives every compute unit about two workgroups
     int parts = 1;
-    while (parts < kMaxParts && n_rows * parts < 1024) parts *= 2;
+    while (parts < kMaxParts && n_rows * parts < 512) parts *= 2;
     const dim3 grid(parts, n_rows);
     split_top_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, ws);
-    split_bins_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
-    if (top_k || top_p) {
-        split_list_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
-        split_cut_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
-        split_runs_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
-    }
-    split_draw_kernel<<<n_rows, FSIE_WAVE, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, uniform, ws, out);
+    split_weigh_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
+    if (top_k || top_p) split_list_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
+    split_draw_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, uniform, ws, out);
     FSIE_CHECK_LAUNCH("sample_split");
     return 0;
 }

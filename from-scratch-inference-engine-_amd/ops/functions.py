@@ -1118,7 +1118,7 @@ def sample(logits: torch.Tensor, temperature: Optional[torch.Tensor] = None,
     # A large vocabulary in few rows: every row is shared by several workgroups, which meet in a workspace.  Not for the
     # greedy choice alone, which is one pass: 1 row of 151,936 takes 9.5 us so and 12 shared, 64 rows 14 and 13, 256 rows
     # 24 and 33.
-    size = int(load().fsie_sample_workspace(n, v)) if temperature is not None else 0
+    size = 0 if temperature is None else int(load().fsie_sample_workspace(n, v, top_k is not None or top_p is not None))
     if size:
         work = torch.empty((size,), dtype=torch.uint8, device=logits.device)
         check(load().fsie_sample_split(logits.data_ptr(), n, v, _ptr(temperature), _ptr(top_k), _ptr(top_p),

@@ -131,3 +131,30 @@ def test_thresholds_that_no_row_has_are_not_passed(rows, vocab, top_k, top_p, mo
     dev = lambda v, dt: torch.tensor(v, dtype=dt).cuda()
     assert got == sample(x, dev([p.temperature for p in params], torch.float32), dev([top_k] * rows, torch.int32),
                          dev([top_p] * rows, torch.float32), dev(list(uniforms_for(5, range(rows), [3] * rows)), torch.float64)).tolist()
+
+
+@pytest.mark.parametrize("kind", ["plain", "narrow", "wide", "ties", "coarse", "masked"])
+@pytest.mark.parametrize("rows, vocab", [(24, 16384), (24, 16385), (24, 40007), (150, 16447), (600, 16384)])
+def test_shared_rows_choose_what_rows_alone_do(kind, rows, vocab):
+    """Both forms weigh a token by the same float32 and differ by the rounding of float64 sums.  Shared rows have bins of
+    their own (listed whole up to a top k of 1,024; cut into finer ones beyond 64 tokens, whose members are bisected beyond
+    512; lists of more than 4,096 tokens go back to the other form; waves that keep more than a few tokens of a line settle them
+    on the way), in 32 parts, in four and in one."""
+    from from_scratch_inference_engine_amd import ops
+    from from_scratch_inference_engine_amd.ops.functions import _stream, check
+
+    lib = ops.load(build_if_missing=False)
+    cases = [(t, k, p) for t, k, p in [(1.0, 1024, 1.0), (1.0, 1025, 1.0), (1.0, 1025, 0.9), (0.8, 1024, 0.9), (2.0, 6000, 0.95), (1.0, 9000, 1.0),
+                                       (5.0, 0, 0.99), (30.0, 0, 0.5), (0.01, 0, 0.9), (0.0005, 40, 0.9), (0.7, 64, 1.0), (1.0, 0, 0.3)]]
+    x = rows_of(kind, rows, vocab).cuda()
+    t, k, p = zip(*[cases[i % len(cases)] for i in range(rows)])
+    dev = lambda v, dt: torch.tensor(v, dtype=dt).cuda()
+    t, k, p, u = dev(t, torch.float32), dev(k, torch.int32), dev(p, torch.float32), torch.linspace(0.001, 0.999, rows, dtype=torch.float64).cuda()
+    size = lib.fsie_sample_workspace(rows, vocab, 1)
+    work = torch.full((size,), 255, dtype=torch.uint8).cuda()
+    alone, shared = torch.full((rows,), -1, dtype=torch.int32).cuda(), torch.full((rows,), -1, dtype=torch.int32).cuda()
+    args = (x.data_ptr(), rows, vocab, t.data_ptr(), k.data_ptr(), p.data_ptr(), u.data_ptr())
+    check(lib.fsie_sample(*args, alone.data_ptr(), _stream()))
+    check(lib.fsie_sample_split(*args, work.data_ptr(), shared.data_ptr(), _stream()))
+    assert size > 0 and ((alone >= 0) & (alone < vocab)).all()
+    assert torch.equal(alone, shared)
