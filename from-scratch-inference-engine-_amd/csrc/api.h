@@ -359,9 +359,11 @@ int fsie_sample(const float* logits, int n_rows, int vocab, const float* tempera
                 const float* top_p, const double* uniform, int32_t* out, hipStream_t stream);
 // The same at temperatures with every row shared by several workgroups, where fsie_sample_workspace says so:
 // `workspace` = fsie_sample_workspace(n_rows, vocab, whether top_k or top_p are given) bytes on the device (0: the call is fsie_sample's), uninitialised.
+// `on_host`: the four arrays are in host memory, of up to fsie_sample_by_value() rows; they are read before the call returns.
 int64_t fsie_sample_workspace(int n_rows, int vocab, int thresholds);
 int fsie_sample_split(const float* logits, int n_rows, int vocab, const float* temperature, const int32_t* top_k,
-                      const float* top_p, const double* uniform, void* workspace, int32_t* out, hipStream_t stream);
+                      const float* top_p, const double* uniform, int on_host, void* workspace, int32_t* out, hipStream_t stream);
+int fsie_sample_by_value(void);
 
 // ---- RMS norm in groups, over a stream with up to two pending deltas ----------------------------
 // x = residual + delta_scale * (delta1 + delta2) (either delta may be null; each is [total_rows, hidden] in its own

@@ -603,8 +603,11 @@ static_assert(kRuns / kMaxParts >= kPart / FSIE_WAVE, "every wave of a part has 
 struct SplitRow {
     unsigned long long sum[kCoarse];  // weights, in units of their bin's own (RowBins)
     unsigned int count[kCoarse];
-    unsigned int n_listed;            // (behind the bins: cleared with them)
-    int top_index, top_nan;           // the row's, from the parts'
+    unsigned int n_listed, pad;       // (behind the bins: cleared with them)
+    double uniform;                   // the row's parameters, as the first launch brings them
+    float temperature, top_p;
+    int top_k;
+    int top_index, top_nan;           // from the parts'
     float top_max, top_low;
     int k_bin, from, upto;            // the bin of top k; those that hold the last token of top p
     double above_k, above, target;    // tokens above k_bin; weight above `from`; what top p's kept weight has to reach (0: no top p alone)
@@ -622,16 +625,43 @@ struct RowParams {
     bool cuts;
     __device__ bool all_listed() const { return 0 < k && k <= kAllListed; }
 };
-__device__ __forceinline__ RowParams row_params(int r, int vocab, const float* temperature, const int32_t* top_k,
-                                                const float* top_p) {
+__device__ __forceinline__ RowParams row_params(const SplitRow* w, int vocab) {
     RowParams q;
-    q.temp = temperature[r];
+    q.temp = w->temperature;
     q.inv_temp = 1.0f / q.temp;
-    q.k = top_k && top_k[r] > 0 && top_k[r] < vocab ? top_k[r] : 0;
-    q.p = top_p ? top_p[r] : 1.f;
+    q.k = w->top_k > 0 && w->top_k < vocab ? w->top_k : 0;
+    q.p = w->top_p;
     q.cuts = q.temp > 0.f && (q.k > 0 || q.p < 1.f);
     return q;
 }
+
+// The rows' parameters where the first launch finds them: in arrays on the device, or among its own arguments, which the host writes (a
+// copy to the device in front of the launches, with its pinned buffer and the event that guards it, is 20 us of the host, which is what bounds a call of 64 rows, and 2.4 of the device: 68 us and 45 through the sampler).
+struct RowArrays {
+    const float* temperature;
+    const int32_t* top_k;  // or null
+    const float* top_p;    // or null
+    const double* uniform;
+    __device__ void to(SplitRow* w, int r) const {
+        w->temperature = temperature[r];
+        w->top_k = top_k ? top_k[r] : 0;
+        w->top_p = top_p ? top_p[r] : 1.f;
+        w->uniform = uniform[r];
+    }
+};
+constexpr int kByValue = 192;
+struct RowValues {
+    double uniform[kByValue];
+    float temperature[kByValue], top_p[kByValue];
+    int32_t top_k[kByValue];
+    __device__ void to(SplitRow* w, int r) const {
+        w->temperature = temperature[r];
+        w->top_k = top_k[r];
+        w->top_p = top_p[r];
+        w->uniform = uniform[r];
+    }
+};
+static_assert(sizeof(RowValues) + 64 <= 4096, "a launch has room for 4 KB of arguments");
 
 // The row's bins: kCoarse equal ones over what it spans, at most kRange or 30 temperatures (43 powers of two in weight).  A bin's weights are
 // summed as integers of a unit of its own, one limb: 2^-(unit + below(bin)), where below(bin) powers of two lie between
@@ -761,14 +791,16 @@ __device__ __forceinline__ void add_runs(const float* __restrict__ row, int voca
     }
 }
 
-__global__ __launch_bounds__(kPart) void split_top_kernel(const float* __restrict__ logits, int vocab, int parts, SplitRow* ws) {
+template <typename ROWS>
+__global__ __launch_bounds__(kPart) void split_top_kernel(const float* __restrict__ logits, int vocab, int parts, SplitRow* ws, ROWS rows) {
     __shared__ float sval[kPart / FSIE_WAVE], slow[kPart / FSIE_WAVE];
     __shared__ int sidx[kPart / FSIE_WAVE], snan[kPart / FSIE_WAVE];
     SplitRow* w = ws + blockIdx.y;
     const int part = blockIdx.x, lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
+    if (part == 0 && threadIdx.x == 0) rows.to(w, static_cast<int>(blockIdx.y));
     // the row's bins and counter are this launch's to clear
     uint32_t* bins = reinterpret_cast<uint32_t*>(w->sum);
-    constexpr int kClear = static_cast<int>(offsetof(SplitRow, top_index) / 4);
+    constexpr int kClear = static_cast<int>(offsetof(SplitRow, uniform) / 4);
     for (int i = part * kPart + threadIdx.x; i < kClear; i += parts * kPart) bins[i] = 0;
     int begin, end;
     part_range(vocab, parts, part, &begin, &end);
@@ -808,15 +840,12 @@ __global__ __launch_bounds__(kPart) void split_top_kernel(const float* __restric
 
 // Rows without a threshold: the draw's sums.  The others: their bins, counted for top k, weighed for top p (not where the list will
 // hold all that top k keeps).  What bounds it are the weighed rows' instructions, some fifty a token.
-__global__ __launch_bounds__(kPart) void split_weigh_kernel(const float* __restrict__ logits, int vocab, int parts,
-                                                            const float* __restrict__ temperature,
-                                                            const int32_t* __restrict__ top_k,
-                                                            const float* __restrict__ top_p, SplitRow* ws) {
+__global__ __launch_bounds__(kPart) void split_weigh_kernel(const float* __restrict__ logits, int vocab, int parts, SplitRow* ws) {
     __shared__ unsigned long long sum[kCoarse];
     __shared__ unsigned int count[kCoarse];
     const int r = blockIdx.y;
-    const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
     SplitRow* w = ws + r;
+    const RowParams q = row_params(w, vocab);
     const RowTop top = row_top(w, parts);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         w->top_max = top.best.value;
@@ -932,19 +961,16 @@ struct BinScan {
 // 9 us of a top-p row's pass over 19,008 tokens, and 3 so).
 constexpr int kNear = kAhead * FSIE_WAVE + 3 * FSIE_WAVE;
 static_assert(kMaxBinned <= 1 << 23 && kRuns <= 1 << 8, "a token's place and its run within the part fit 32 bits");
-__global__ __launch_bounds__(kPart) void split_list_kernel(const float* __restrict__ logits, int vocab, int parts,
-                                                           const float* __restrict__ temperature,
-                                                           const int32_t* __restrict__ top_k,
-                                                           const float* __restrict__ top_p, SplitRow* ws) {
+__global__ __launch_bounds__(kPart) void split_list_kernel(const float* __restrict__ logits, int vocab, int parts, SplitRow* ws) {
     __shared__ float near[kPart / FSIE_WAVE][kNear];
     __shared__ unsigned int near_at[kPart / FSIE_WAVE][kNear];
     __shared__ unsigned long long run_hi[kRuns], run_lo[kRuns];
     __shared__ double wave_sum[2][kPart / FSIE_WAVE];
     __shared__ Found found[3];
     const int r = blockIdx.y;
-    const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
-    if (!q.cuts) return;
     SplitRow* w = ws + r;
+    const RowParams q = row_params(w, vocab);
+    if (!q.cuts) return;
     const RowTop top = kept_top(w);
     RowBins bins;
     if (!top.binned(vocab, q, &bins)) return;
@@ -1218,11 +1244,7 @@ __device__ uint32_t cut_of_list(Cutting& s, const SplitRow* w, const RowParams& 
                    : key_reaching<false>(s.search[1], bins, mx, at.bin, v, in, value, at.above, target, weight);
 }
 
-__global__ __launch_bounds__(kThreads) void split_draw_kernel(const float* __restrict__ logits, int vocab, int parts,
-                                                              const float* __restrict__ temperature,
-                                                              const int32_t* __restrict__ top_k,
-                                                              const float* __restrict__ top_p,
-                                                              const double* __restrict__ uniform, const SplitRow* ws,
+__global__ __launch_bounds__(kThreads) void split_draw_kernel(const float* __restrict__ logits, int vocab, const SplitRow* ws,
                                                               int32_t* __restrict__ out) {
     __shared__ union {
         Cutting list;
@@ -1230,8 +1252,8 @@ __global__ __launch_bounds__(kThreads) void split_draw_kernel(const float* __res
     } s;
     __shared__ double run_sum[kRuns], sdbl[kWaves];
     const int r = blockIdx.x;
-    const RowParams q = row_params(r, vocab, temperature, top_k, top_p);
     const SplitRow* w = ws + r;
+    const RowParams q = row_params(w, vocab);
     const RowTop top = kept_top(w);
     if (!(q.temp > 0.f)) {
         if (threadIdx.x == 0) out[r] = top.best.index;
@@ -1289,7 +1311,7 @@ __global__ __launch_bounds__(kThreads) void split_draw_kernel(const float* __res
     }
     if (threadIdx.x < kRuns) run_sum[threadIdx.x] = sum;
     __syncthreads();
-    draw_from_runs(row, vocab, top.best, q.inv_temp, cut, uniform[r], run_sum, out + r);
+    draw_from_runs(row, vocab, top.best, q.inv_temp, cut, w->uniform, run_sum, out + r);
 }
 
 }  // namespace
@@ -1313,11 +1335,14 @@ extern "C" int fsie_sample(const float* logits, int n_rows, int vocab, const flo
     return 0;
 }
 
+extern "C" int fsie_sample_by_value(void) { return kByValue; }
+
 extern "C" int fsie_sample_split(const float* logits, int n_rows, int vocab, const float* temperature, const int32_t* top_k,
-                                 const float* top_p, const double* uniform, void* workspace, int32_t* out,
+                                 const float* top_p, const double* uniform, int on_host, void* workspace, int32_t* out,
                                  hipStream_t stream) {
-    FSIE_REQUIRE(n_rows > 0 && n_rows <= 65535 && vocab > 0, "sample_split: bad sizes rows=%d vocab=%d", n_rows, vocab);
+    FSIE_REQUIRE(n_rows > 0 && n_rows <= 65535 && vocab > 0 && vocab <= (1 << 30), "sample_split: bad sizes rows=%d vocab=%d", n_rows, vocab);
     FSIE_REQUIRE(temperature && uniform, "sample_split: temperatures and uniform numbers are needed");
+    FSIE_REQUIRE(!on_host || n_rows <= kByValue, "sample_split: parameters of %d rows from the host, which are %d at most", n_rows, kByValue);
     FSIE_REQUIRE(workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0,
                  "sample_split: a workspace on 16 bytes is needed");
     SplitRow* ws = static_cast<SplitRow*>(workspace);
@@ -1325,10 +1350,21 @@ extern "C" int fsie_sample_split(const float* logits, int n_rows, int vocab, con
     int parts = 1;
     while (parts < kMaxParts && n_rows * parts < 512) parts *= 2;
     const dim3 grid(parts, n_rows);
-    split_top_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, ws);
-    split_weigh_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
-    if (top_k || top_p) split_list_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, ws);
-    split_draw_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, parts, temperature, top_k, top_p, uniform, ws, out);
+    if (on_host) {
+        RowValues rows{};
+        for (int r = 0; r < n_rows; ++r) {
+            rows.uniform[r] = uniform[r];
+            rows.temperature[r] = temperature[r];
+            rows.top_k[r] = top_k ? top_k[r] : 0;
+            rows.top_p[r] = top_p ? top_p[r] : 1.f;
+        }
+        split_top_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, ws, rows);
+    } else {
+        split_top_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, ws, RowArrays{temperature, top_k, top_p, uniform});
+    }
+    split_weigh_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, ws);
+    if (top_k || top_p) split_list_kernel<<<grid, kPart, 0, stream>>>(logits, vocab, parts, ws);
+    split_draw_kernel<<<n_rows, kThreads, 0, stream>>>(logits, vocab, ws, out);
     FSIE_CHECK_LAUNCH("sample_split");
     return 0;
 }

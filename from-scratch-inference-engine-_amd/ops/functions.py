@@ -7,6 +7,7 @@ import ctypes
 from functools import lru_cache
 from typing import Optional, Sequence
 
+import numpy as np
 import torch
 
 from .library import KernelError, check, load
@@ -1096,13 +1097,44 @@ def attention_merge(partials: torch.Tensor, merges: torch.Tensor, n_merges: int,
     return out
 
 
+def sample_takes_arrays(n: int, vocab: int, thresholds: bool) -> bool:
+    """Whether ``sample`` of ``n`` rows takes their parameters as numpy arrays (rows that are shared by workgroups, as many
+    as a launch's arguments have room for)."""
+    return 0 < n <= load().fsie_sample_by_value() and load().fsie_sample_workspace(n, vocab, thresholds) > 0
+
+
+def _sample_arrays(logits, temperature, top_k, top_p, uniform, out):
+    n, v = logits.shape
+    for name, a, dtype in (("temperature", temperature, np.float32), ("top_k", top_k, np.int32), ("top_p", top_p, np.float32),
+                           ("uniform", uniform, np.float64)):
+        if a is None and name.startswith("top"):
+            continue
+        if not isinstance(a, np.ndarray) or a.dtype != dtype or a.shape != (n,) or not a.flags.c_contiguous:
+            raise KernelError(f"{name}: expected a contiguous numpy array of {n} {np.dtype(dtype).name} beside the other parameters")
+    thresholds = top_k is not None or top_p is not None
+    if not sample_takes_arrays(n, v, thresholds):
+        raise KernelError(f"sample: the parameters of {n} rows of {v} tokens must be tensors on the GPU")
+    if out is None:
+        out = torch.empty((n,), dtype=torch.int32, device=logits.device)
+    _need(out, "sample out", dtype=torch.int32, shape=(n,))
+    work = torch.empty((load().fsie_sample_workspace(n, v, thresholds),), dtype=torch.uint8, device=logits.device)
+    at = lambda a: None if a is None else a.ctypes.data
+    check(load().fsie_sample_split(logits.data_ptr(), n, v, at(temperature), at(top_k), at(top_p), at(uniform), 1,
+                                   work.data_ptr(), out.data_ptr(), _stream()))
+    return out
+
+
 def sample(logits: torch.Tensor, temperature: Optional[torch.Tensor] = None,
            top_k: Optional[torch.Tensor] = None, top_p: Optional[torch.Tensor] = None,
            uniform: Optional[torch.Tensor] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """One token id per row of float32 ``logits`` [n, V]: argmax where temperature <= 0 (or no
-    temperatures are given), else temperature/top-k/top-p sampling against ``uniform`` (float64)."""
+    temperatures are given), else temperature/top-k/top-p sampling against ``uniform`` (float64).
+    The rows' parameters are tensors on the device, or numpy arrays where ``sample_takes_arrays`` says so: these are
+    read before the call returns and travel with the launch."""
     _need(logits, "logits", dtype=torch.float32, ndim=2)
     n, v = logits.shape
+    if isinstance(temperature, np.ndarray):
+        return _sample_arrays(logits, temperature, top_k, top_p, uniform, out)
     if temperature is not None:
         _need(temperature, "temperature", dtype=torch.float32, shape=(n,))
         if uniform is None:
@@ -1122,7 +1154,7 @@ def sample(logits: torch.Tensor, temperature: Optional[torch.Tensor] = None,
     if size:
         work = torch.empty((size,), dtype=torch.uint8, device=logits.device)
         check(load().fsie_sample_split(logits.data_ptr(), n, v, _ptr(temperature), _ptr(top_k), _ptr(top_p),
-                                       _ptr(uniform), work.data_ptr(), out.data_ptr(), _stream()))
+                                       _ptr(uniform), 0, work.data_ptr(), out.data_ptr(), _stream()))
         return out
     check(load().fsie_sample(logits.data_ptr(), n, v, _ptr(temperature), _ptr(top_k), _ptr(top_p),
                              _ptr(uniform), out.data_ptr(), _stream()))

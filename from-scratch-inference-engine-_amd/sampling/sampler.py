@@ -102,11 +102,13 @@ class Sampler:
             raise ValueError("sample: one set of parameters, request id and index per row")
         if all(p.greedy for p in params):
             return ops.sample(logits)
-        uniform, temperature, top_k, top_p = self._upload(
-            uniforms_for(self.seed, request_ids, indices),
-            [max(float(p.temperature), 0.0) for p in params], [int(p.top_k) for p in params],
-            [float(p.top_p) for p in params], logits.device)
+        uniform = np.asarray(uniforms_for(self.seed, request_ids, indices), dtype=np.float64)
+        temperature = np.maximum(np.array([p.temperature for p in params], dtype=np.float32), np.float32(0.0))
+        top_k = np.array([p.top_k for p in params], dtype=np.int32)
+        top_p = np.array([p.top_p for p in params], dtype=np.float32)
         # (a threshold that no row has is not passed: the kernels then spare what finds it)
         vocab = logits.shape[1]
-        return ops.sample(logits, temperature, top_k if any(0 < p.top_k < vocab for p in params) else None,
-                          top_p if any(p.top_p < 1.0 for p in params) else None, uniform)
+        k_given, p_given = bool(((top_k > 0) & (top_k < vocab)).any()), bool((top_p < 1.0).any())
+        if not ops.sample_takes_arrays(n, vocab, k_given or p_given):
+            uniform, temperature, top_k, top_p = self._upload(uniform, temperature, top_k, top_p, logits.device)
+        return ops.sample(logits, temperature, top_k if k_given else None, top_p if p_given else None, uniform)

@@ -155,6 +155,8 @@ def test_shared_rows_choose_what_rows_alone_do(kind, rows, vocab):
     alone, shared = torch.full((rows,), -1, dtype=torch.int32).cuda(), torch.full((rows,), -1, dtype=torch.int32).cuda()
     args = (x.data_ptr(), rows, vocab, t.data_ptr(), k.data_ptr(), p.data_ptr(), u.data_ptr())
     check(lib.fsie_sample(*args, alone.data_ptr(), _stream()))
-    check(lib.fsie_sample_split(*args, work.data_ptr(), shared.data_ptr(), _stream()))
+    check(lib.fsie_sample_split(*args, 0, work.data_ptr(), shared.data_ptr(), _stream()))
+    if ops.sample_takes_arrays(rows, vocab, True):  # (the parameters come with the launch instead)
+        assert torch.equal(ops.sample(x, *[v.cpu().numpy() for v in (t, k, p, u)]), shared)
     assert size > 0 and ((alone >= 0) & (alone < vocab)).all()
     assert torch.equal(alone, shared)
