@@ -11,13 +11,13 @@ from one fixed device buffer; a later step of the same shape copies its tables t
 the graph.
 
 The number of requests is rounded up as well (``padded_rows``): a batch that shrinks request by
-request as they finish would otherwise want a new graph, some tens of milliseconds of capture,
-at every size.  The rows that fill a batch up are requests of one token at position 0 whose
-cache is the pools' spare page and the spare state slot; they cost a decode step nothing that
-can be measured, no request reads what they write, and their logits are dropped.
+request as they finish would otherwise want a new graph, some milliseconds of capture, at every
+size.  The rows that fill a batch up are requests of one token at position 0 whose cache is the
+pools' spare page and the spare state slot; they cost a decode step nothing that can be measured,
+no request reads what they write, and their logits are dropped.
 
 A shape is captured when it comes for the third time (``capture_after``); until then its steps
-run eagerly, which costs a few milliseconds of host time each where a capture costs thirty: the
+run eagerly, which costs a few milliseconds of host time each where a capture costs five to ten: the
 shapes a batch passes through while its last requests end, one or two steps each, are not worth
 a graph.
 """
@@ -25,6 +25,7 @@ a graph.
 from __future__ import annotations
 
 import gc
+import threading
 import weakref
 from typing import Dict, List, Optional, Sequence, Tuple
 
@@ -44,6 +45,32 @@ def padded_rows(n: int) -> int:
         return 1 << max(0, n - 1).bit_length()
     step = 16 if n <= 128 else 32
     return -(-n // step) * step
+
+
+class _CollectorOff:
+    """Nothing may free device or pinned memory while a stream is captured, and the collector of reference cycles may come upon
+    dead ones that hold such memory (or other graphs): it stays off while any thread captures.  (What is dead stays where it is
+    until the collector next runs by itself; collecting it in front of every capture took 21 to 39 ms of a capture's 27 to 50.)"""
+
+    def __init__(self):
+        self._lock, self._captures, self._was_on = threading.Lock(), 0, False
+
+    def __enter__(self):
+        with self._lock:
+            if self._captures == 0:
+                self._was_on = gc.isenabled()
+                gc.disable()
+            self._captures += 1
+
+    def __exit__(self, *exc):
+        with self._lock:
+            self._captures -= 1
+            if self._captures == 0 and self._was_on:
+                gc.enable()
+        return False
+
+
+_collector_off = _CollectorOff()
 
 
 class DecodeGraphs:
@@ -137,18 +164,8 @@ class DecodeGraphs:
             if feed is not None:
                 ctx.token_ids[:n].copy_(feed)
             graph = torch.cuda.CUDAGraph()
-            # Nothing may free device or pinned memory while the stream is captured.  Dead cycles
-            # of Python objects that hold such memory (or other graphs) are therefore collected
-            # now, and the collector stays off until the capture has ended.
-            gc.collect()
-            collector_was_on = gc.isenabled()
-            gc.disable()
-            try:
-                with torch.cuda.graph(graph):
-                    logits = runner.model.forward(ctx, runner.storage)
-            finally:
-                if collector_was_on:
-                    gc.enable()
+            with _collector_off, torch.cuda.graph(graph):
+                logits = runner.model.forward(ctx, runner.storage)
             self._graphs[key] = (graph, tables, logits, ctx.token_ids)
             self.captures += 1
             graph.replay()  # the step itself

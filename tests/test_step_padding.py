@@ -34,3 +34,22 @@ def test_the_filler_reads_and_writes_spare_places_only():
     assert e.cache.tables == [[40] * 5, [17] * 3]          # every page of its table is the spare one
     host = HostBatch([e], page_size=8)
     assert host.n_tokens == 37 and host.positions.tolist() == list(range(37)) and host.want_rows.size == 0
+
+
+@pytest.mark.parametrize("was_on", [True, False])
+def test_the_collector_is_off_until_the_last_capture_ends(was_on):
+    import gc
+
+    from from_scratch_inference_engine_amd.engine.graphs import _collector_off
+
+    before = gc.isenabled()
+    (gc.enable if was_on else gc.disable)()
+    try:
+        with _collector_off:
+            with pytest.raises(RuntimeError):
+                with _collector_off:
+                    raise RuntimeError("a capture that fails")
+            assert not gc.isenabled()
+        assert gc.isenabled() == was_on
+    finally:
+        (gc.enable if before else gc.disable)()
