@@ -3,6 +3,8 @@ for a request that does not exist (host logic, no GPU)."""
 
 from types import SimpleNamespace
 
+import pytest
+
 from from_scratch_inference_engine_amd.engine.context import HostBatch, filler_entry, padded_tokens
 from from_scratch_inference_engine_amd.engine.graphs import padded_rows
 
