@@ -365,6 +365,16 @@ int fsie_sample_split(const float* logits, int n_rows, int vocab, const float* t
                       const float* top_p, const double* uniform, int on_host, void* workspace, int32_t* out, hipStream_t stream);
 int fsie_sample_by_value(void);
 
+// ---- a norm and the product behind it, one or two rows ----------------------------------------
+// y = RMSNorm(residual + sums) . w^T: residual float32 [M, K], sums [n_parts, M, K] float32 or none, norm_weight float32 [K]; the sum is
+// written to new_stream [M, K] (another buffer than residual; not where n_parts is 0).  w [N, K] bfloat16 or (frags) its copy in
+// fragment order.  result 0: y float32 [slices, M, N], sums of one or two slices of K; 1: w's rows are gate and up in turn, y bfloat16 [M, N / 2].  Everything
+// 16-byte aligned.
+int fsie_gemm_mfma_normed_takes(int M, int N, int K, int result, int n_parts);
+int fsie_gemm_mfma_normed(const float* residual, const float* sums, int n_parts, const float* norm_weight, float eps, float* new_stream,
+                          const void* w, void* y, int M, int N, int K, int result, int slices, int frags, int act, float pos,
+                          float neg, hipStream_t stream);
+
 // ---- RMS norm in groups, over a stream with up to two pending deltas ----------------------------
 // x = residual + delta_scale * (delta1 + delta2) (either delta may be null; each is [total_rows, hidden] in its own
 // type, FSIE_F32 or FSIE_BF16), written back to `residual` if write_back; the row is cut into `groups` equal

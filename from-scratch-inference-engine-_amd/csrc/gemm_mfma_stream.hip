@@ -37,6 +37,7 @@ constexpr int kMostSteps = 8;  // steps of 32 values of K a wave
 // SUMS: float32 partial sums [slices][M][N]; GATED: bfloat16 [M, N / 2] of gate and up rows in turn; POINT: bfloat16 [M, N],
 // act(sum + bias)
 enum Result { SUMS = 0, GATED = 1, POINT = 2 };
+constexpr int kPlanOne = 4;
 constexpr int kPlanActivation = 3;  // to the plan alone: POINT where the kernel that shares X has the activation in its epilogue too
 struct StreamCall {
     const bf16_t* x;
@@ -155,7 +156,9 @@ int launch_waves(int waves, int nb, int s, const StreamCall& c, hipStream_t stre
     if (waves == 8) return launch_steps<8, LEAST, 1, RESULT, FRAGS>(s, c, stream);
     if constexpr (RESULT != SUMS)
         return waves == 4 ? launch_steps<4, 1, 1, RESULT, FRAGS>(s, c, stream) : launch_steps<16, LEAST, 1, RESULT, FRAGS>(s, c, stream);
-    fsie_set_error("gemm_mfma_stream: sums take eight waves a workgroup");
+    if constexpr (RESULT == SUMS && !FRAGS)
+        if (waves == 4) return launch_steps<4, 5, 1, RESULT, FRAGS>(s, c, stream);
+    fsie_set_error("gemm_mfma_stream: sums take eight waves a workgroup, on rows four");
     return 1;
 }
 
@@ -175,11 +178,14 @@ int launch_waves(int waves, int nb, int s, const StreamCall& c, hipStream_t stre
 // Sums: the fewest slices that a workgroup of eight waves holds, then as many more as leave a wave four steps and the workgroups
 // no more than the units: a second round costs what it hides (N = 4608, K = 3584 8.1 us against 7.0 in seven slices), and the
 // norm pays for every slice.
+// kPlanOne: sums of one slice, for a norm that the next product makes itself (gemm_mfma_normed.hip), whose every workgroup reads them.
+// Rows of W in four waves: N = K = 896, one and two rows 2.9 us, in seven slices 2.4; gate and up with the norm behind them 5.3 and 5.6, 6.1 and 7.3.
 extern "C" int fsie_gemm_mfma_stream_plan(int M, int N, int K, int result, int frags) {
     const int units = fsie_compute_units();
     if (M < 1 || M > 16 || N < 1 || K < 32 || K % 32 || units <= 0) return -1;
     const int steps = K / 32, groups = (N + 15) / 16;
     const int64_t bytes = static_cast<int64_t>(N) * K * 2;
+    if (result == kPlanOne) return !frags && M <= 2 && steps > 4 * 4 && steps <= 4 * kMostSteps && groups <= units ? 4 + 256 + 65536 : -1;
     if (result == SUMS) {
         if (!frags || K < 1024) return -1;
         int splits = (steps + 8 * kMostSteps - 1) / (8 * kMostSteps);
@@ -216,7 +222,7 @@ extern "C" int fsie_gemm_mfma_stream(const void* x, const void* w, const float* 
     FSIE_REQUIRE(result != GATED || FSIE_PAIR_KNOWN(act), "gemm_mfma_stream: unknown activation %d", act);
     FSIE_REQUIRE(result != POINT || FSIE_POINT_KNOWN(act), "gemm_mfma_stream: unknown activation %d", act);
     FSIE_REQUIRE(plan > 0 && (waves == 4 || waves == 8 || waves == 16) && (blocks == 1 || (blocks == 2 && waves > 4)) && splits >= 1 &&
-                     splits <= FSIE_GEMM_MAX_SPLITS && (result != SUMS || (waves == 8 && frags)) && (result != GATED || frags),
+                     splits <= FSIE_GEMM_MAX_SPLITS && (result != SUMS || (frags ? waves == 8 : waves == 4 && splits == 1)) && (result != GATED || frags),
                  "gemm_mfma_stream: no such plan %d for result %d", plan, result);
     const int steps = K / 32, slice = (steps + splits - 1) / splits, s = (slice + waves - 1) / waves;
     FSIE_REQUIRE(slice * (splits - 1) < steps && s <= kMostSteps, "gemm_mfma_stream: K=%d in %d slices of %d waves", K, splits, waves);
@@ -226,6 +232,6 @@ extern "C" int fsie_gemm_mfma_stream(const void* x, const void* w, const float* 
     if (M == 0) return 0;
     const StreamCall c{static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(w), y, M, N, K, slice, act, pos, neg, bias};
     if (result == GATED) return launch_waves<GATED, true>(waves, blocks, s, c, stream);
-    if (result == SUMS) return launch_waves<SUMS, true>(waves, blocks, s, c, stream);
+    if (result == SUMS) return frags ? launch_waves<SUMS, true>(waves, blocks, s, c, stream) : launch_waves<SUMS, false>(waves, blocks, s, c, stream);
     return frags ? launch_waves<POINT, true>(waves, blocks, s, c, stream) : launch_waves<POINT, false>(waves, blocks, s, c, stream);
 }

@@ -161,6 +161,8 @@ class StepContext:
         self.seq_slots = self.q_starts = self.past_lens = self.reset_slots = None
         # set by the model: every norm can add up a delta that comes as float32 partial sums
         self.partial_sums_ok = False
+        # set by a block around its mixer: what it leaves is read whole by every workgroup of the next product
+        self.sums_in_one = False
         self.block_tables: List[torch.Tensor] = []
         self.slots: List[torch.Tensor] = []
         self.fresh_pages: List[Optional[torch.Tensor]] = []  # per group: units just taken from the pool, or None

@@ -637,7 +637,9 @@ def gemm_mfma_wide_swiglu(x: torch.Tensor, weight: torch.Tensor, waves: int = 0,
     """silu(gate) * up, or what ``act`` (a ``GateAct`` or its name) makes of them, [M, N/2] (bfloat16) of x [M, K] and a weight [N, K] whose rows are gate and up
     in turn (or its ``FragmentOrdered`` copy), by the kernel that shares x through LDS; up to 64
     rows, N a multiple of 4, K of 128.  ``few_rows``: up to 16 rows go to ``gemm_mfma_stream`` where that is faster (the same
-    sums in another order)."""
+    sums in another order).  ``x`` may be a norm that waits for its product (``parts.base.PendingNorm``): ``gemm_mfma_normed``."""
+    if not isinstance(x, torch.Tensor):
+        return gemm_mfma_normed(x.residual, x.sums, x.weight, x.eps, x.stream, weight, GEMM_STREAM_GATED, act)
     _need(x, "gemm x", dtype=torch.bfloat16, ndim=2)
     m, k = x.shape
     wptr, n, frags = _wide_weight(weight, k)
@@ -693,7 +695,40 @@ def _gemm_tile(x, weight, result: int, splits: int, tile: int, act) -> torch.Ten
     return out
 
 
-GEMM_STREAM_SUMS, GEMM_STREAM_GATED, GEMM_STREAM_POINT, GEMM_STREAM_PLAN_ACT = 0, 1, 2, 3
+GEMM_STREAM_SUMS, GEMM_STREAM_GATED, GEMM_STREAM_POINT, GEMM_STREAM_PLAN_ACT, GEMM_STREAM_PLAN_ONE = 0, 1, 2, 3, 4
+
+
+@lru_cache(maxsize=4096)
+def gemm_normed_takes(m: int, n: int, k: int, result: int, n_parts: int) -> int:
+    """Whether ``gemm_mfma_normed`` is the faster way to a norm of a stream with ``n_parts`` pending partial sums and the product behind it:
+    the slices of K in which it is (0: it is not)."""
+    return int(load().fsie_gemm_mfma_normed_takes(m, n, k, result, n_parts))
+
+
+def gemm_mfma_normed(residual: torch.Tensor, sums: Optional[torch.Tensor], norm_weight: torch.Tensor, eps: float,
+                     new_stream: Optional[torch.Tensor], weight, result: int, act=None, splits: int = 1) -> torch.Tensor:
+    """RMSNorm(residual + sums) . weight^T of one or two rows, the norm made by the product's own workgroups: ``residual`` float32 [M, K],
+    ``sums`` float32 [S, M, K] (None: no delta), whose total with the residual goes to ``new_stream`` (another buffer);
+    ``weight`` [N, K] bfloat16 or its ``FragmentOrdered`` copy.  GEMM_STREAM_SUMS: float32 [splits, M, N], sums of one or two slices of K; GEMM_STREAM_GATED: [M, N/2] in
+    bfloat16 (``act``: a ``GateAct`` or its name)."""
+    _need(residual, "gemm_mfma_normed residual", dtype=torch.float32, ndim=2)
+    m, k = residual.shape
+    _need(norm_weight, "gemm_mfma_normed norm weight", dtype=torch.float32, shape=(k,))
+    n_parts = 0
+    if sums is not None:
+        n_parts = sums.shape[0]
+        _need(sums, "gemm_mfma_normed sums", dtype=torch.float32, shape=(n_parts, m, k))
+        _need(new_stream, "gemm_mfma_normed new stream", dtype=torch.float32, shape=(m, k))
+    wptr, n, frags = _wide_weight(weight, k)
+    if result == GEMM_STREAM_SUMS:
+        out = torch.empty((splits, m, n), dtype=torch.float32, device=residual.device)
+        args = (0, 0.0, 0.0)
+    else:
+        out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=residual.device)
+        args = gate_act(act).args
+    check(load().fsie_gemm_mfma_normed(residual.data_ptr(), _ptr(sums), n_parts, norm_weight.data_ptr(), float(eps),
+                                       _ptr(new_stream) if n_parts else None, wptr, out.data_ptr(), m, n, k, result, splits, frags, *args, _stream()))
+    return out
 
 
 @lru_cache(maxsize=4096)

@@ -12,7 +12,7 @@ from .. import ops
 from ..cache.manager import PagedNeed, PooledNeed
 from ..ops.functions import ATTN_ITEM_INTS, ATTN_KEEP_WALK, ATTN_MERGE_INTS, ATTN_POOL_WALK
 from ..ops.functions import GEMM_MFMA_SKINNY_BEST_M
-from .base import Mixer, Norm, ParamDecl, Part, PositionEncoding, register_part
+from .base import Mixer, Norm, ParamDecl, Part, PendingNorm, PositionEncoding, register_part
 from .linear import Linear
 
 
@@ -801,14 +801,31 @@ class GQAttention(Mixer):
         # and 14.0, 13.7 and 16.8; 14 of 64 at 640 10.4 and 11.3, 10.3 and 11.1, at 512 10.5 and 11.3, 9.8 and 10.3).
         return self.head_dim > 128 or self.qkv.in_features < 640
 
-    def _from_sums(self, x: torch.Tensor, ctx, cache, plan, fuse: bool, table) -> Optional[torch.Tensor]:
+    def _sums_will_do(self, dtype, cache, plan, fuse: bool) -> bool:
+        """Whether attention of this step may take the q/k/v product as partial sums: one token a request."""
+        return (self.finish_qkv_in_attention and self.sink is None and not self.keep_first and self.softcap is None and fuse and cache.writes and plan.mfma and plan.single
+                and plan.n_small and not plan.n_large and not plan.n_long and dtype == torch.bfloat16
+                and ops.attention_mfma_qkv_ok(self.head_dim, cache.page_size))
+
+    def takes_pending_norm(self, m: int, n_parts: int, ctx, cache) -> bool:
+        qkv = self.qkv
+        if (type(self).forward is not GQAttention.forward or self.prepared or self.wants_long_slices or qkv.weight is None or qkv.weight.dtype != torch.bfloat16 or not qkv.weight.is_contiguous()
+                or qkv.weight.data_ptr() % 16 or not ops.gemm_normed_takes(m, qkv.out_features, qkv.in_features, ops.GEMM_STREAM_SUMS, n_parts)):
+            return False
+        return self._sums_will_do(ctx.compute_dtype, cache, ctx.plan(self.planner()), self._fused_table(ctx)[0])
+
+    def _from_sums(self, x, ctx, cache, plan, fuse: bool, table) -> Optional[torch.Tensor]:
         """Attention of a step of one token a request straight from the q/k/v product's partial sums
         (None: not such a step, or the kernels do not take the sizes)."""
-        if not (self.finish_qkv_in_attention and self.sink is None and not self.keep_first and self.softcap is None and fuse and cache.writes and plan.mfma and plan.single
-                and plan.n_small and not plan.n_large and not plan.n_long and x.dtype == torch.bfloat16
-                and ops.attention_mfma_qkv_ok(self.head_dim, cache.page_size)):
+        if not self._sums_will_do(x.dtype, cache, plan, fuse):
             return None
-        sums = self.qkv.partial_sums(x, few_rows=True, long_slices=self.wants_long_slices)
+        if isinstance(x, PendingNorm):
+            weight = self.qkv.weight if self.qkv.streamed is None else self.qkv.streamed
+            n_parts = 0 if x.sums is None else len(x.sums)
+            splits = ops.gemm_normed_takes(x.shape[0], self.qkv.out_features, self.qkv.in_features, ops.GEMM_STREAM_SUMS, n_parts)
+            sums = ops.gemm_mfma_normed(x.residual, x.sums, x.weight, x.eps, x.stream, weight, ops.GEMM_STREAM_SUMS, splits=splits)
+        else:
+            sums = self.qkv.partial_sums(x, few_rows=True, long_slices=self.wants_long_slices)
         if sums is None:
             return None
         out = torch.empty((x.shape[0], self.q_dim), dtype=x.dtype, device=x.device)

@@ -68,6 +68,20 @@ class HiddenState:
         self.delta_bias = None
 
 
+class PendingNorm:
+    """A norm that the product behind it makes itself (``ops.gemm_mfma_normed``), in the place of its output: the stream as it was,
+    the partial sums to add (or None), the norm's weight and eps, and where the product writes the new stream.  Whoever
+    takes one runs that product once, and first."""
+
+    __slots__ = ("residual", "sums", "weight", "eps", "stream", "dtype")
+
+    def __init__(self, residual, sums, weight, eps, stream, dtype):
+        self.residual, self.sums, self.weight, self.eps, self.stream, self.dtype = residual, sums, weight, eps, stream, dtype
+
+    shape = property(lambda s: s.residual.shape)
+    device = property(lambda s: s.residual.device)
+
+
 class Part:
     kind: str = "part"
     # True if the part takes everything that changes from step to step from device tensors (its
@@ -132,6 +146,14 @@ class Norm(Part):
     def rows(self, hidden: HiddenState, rows: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
         raise NotImplementedError
 
+    def can_wait(self, hidden: HiddenState, out_dtype: torch.dtype) -> bool:
+        """Whether ``wait`` may stand for this call of the norm."""
+        return False
+
+    def wait(self, hidden: HiddenState, out_dtype: torch.dtype) -> PendingNorm:
+        """The norm left to the product behind it; the hidden state already holds the stream that the product will write."""
+        raise NotImplementedError
+
     def plain(self, x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The norm of a plain tensor [T, W], away from the residual stream: a mixer's or a
         feed-forward's output before it is added (sandwich and post-norm arrangements), or the
@@ -149,6 +171,10 @@ class Mixer(Part):
     def planner(self):
         return None
 
+    def takes_pending_norm(self, m: int, n_parts: int, ctx, cache) -> bool:
+        """Whether ``forward`` takes a ``PendingNorm`` of ``m`` rows and ``n_parts`` partial sums as ``x``, and is the faster for it."""
+        return False
+
     def forward(self, x: torch.Tensor, ctx, cache) -> torch.Tensor:
         raise NotImplementedError
 
@@ -158,6 +184,10 @@ class FeedForward(Part):
     # a bias (float32 [H]) that belongs to what ``forward`` returns and that the block hands to the norm that adds it
     # (``HiddenState.delta_bias``); None: what ``forward`` returns is whole
     residual_bias: Optional[torch.Tensor] = None
+
+    def takes_pending_norm(self, m: int, n_parts: int, ctx) -> bool:
+        """As a mixer's."""
+        return False
 
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         raise NotImplementedError

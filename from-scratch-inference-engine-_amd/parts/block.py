@@ -30,10 +30,25 @@ class PreNormBlock(Block):
     def sub_parts(self) -> Dict[str, Part]:
         return {"mixer_norm": self.mixer_norm, "mixer": self.mixer, "ffn_norm": self.ffn_norm, "ffn": self.ffn}
 
+    few_rows = 2  # up to so many a norm may be left to the product behind it
+
+    @staticmethod
+    def _normed(norm: Norm, part: Part, hidden: HiddenState, ctx, *cache):
+        if len(hidden.residual) <= PreNormBlock.few_rows and norm.can_wait(hidden, ctx.compute_dtype):
+            if part.takes_pending_norm(len(hidden.residual), 0 if hidden.delta is None else len(hidden.delta), ctx, *cache):
+                return norm.wait(hidden, ctx.compute_dtype)
+        return norm(hidden, ctx.compute_dtype)
+
     def forward(self, hidden: HiddenState, ctx, cache) -> None:
-        x = self.mixer_norm(hidden, ctx.compute_dtype)
-        hidden.delta = self.mixer.forward(x, ctx, cache)
-        x = self.ffn_norm(hidden, ctx.compute_dtype)
+        few = len(hidden.residual) <= self.few_rows
+        x = self._normed(self.mixer_norm, self.mixer, hidden, ctx, cache)
+        # (the output projection leaves its sums in one slice where every workgroup of the next product is going to read them)
+        ctx.sums_in_one = few and self.ffn_norm.can_wait(hidden, ctx.compute_dtype) and self.ffn.takes_pending_norm(len(hidden.residual), 1, ctx)
+        try:
+            hidden.delta = self.mixer.forward(x, ctx, cache)
+        finally:
+            ctx.sums_in_one = False
+        x = self._normed(self.ffn_norm, self.ffn, hidden, ctx)
         hidden.delta = self.ffn.forward(x, ctx)
 
 

@@ -208,6 +208,10 @@ class Linear:
                     if splits > 1 and self.wide_takes(m, splits) and self.kernel_reads(x) else None)
         if self.in_features % 8:
             return None
+        if getattr(ctx, "sums_in_one", False):
+            plan = ops.gemm_stream_plan(m, self.out_features, self.in_features, ops.GEMM_STREAM_PLAN_ONE, self.streamed is not None)
+            if plan is not None and self.kernel_reads(x):
+                return ops.gemm_mfma_stream(x, self.weight, ops.GEMM_STREAM_SUMS, plan)
         plan = self.stream_plan(m, ops.GEMM_STREAM_SUMS) if m <= GEMM_MFMA_SKINNY_BEST_M else None
         if plan is not None and self.kernel_reads(x):
             return ops.gemm_mfma_stream(x, self.streamed, ops.GEMM_STREAM_SUMS, plan)

@@ -8,7 +8,7 @@ from typing import Dict, Optional
 import torch
 
 from .. import ops
-from .base import FeedForward, ParamDecl, register_part
+from .base import FeedForward, ParamDecl, PendingNorm, register_part
 from ..ops.functions import GEMM_MFMA_SKINNY_BEST_M
 from .linear import Linear
 
@@ -65,9 +65,16 @@ class SwiGLU(FeedForward):
     # has a fragment-ordered copy (beyond: the library's product and a kernel for SiLU*up)
     streamed_swiglu_max_rows = 128
 
+    def takes_pending_norm(self, m: int, n_parts: int, ctx) -> bool:
+        gate_up = self.gate_up
+        return (type(self) is SwiGLU and gate_up.streamed is not None and gate_up.stream_plan(m, ops.GEMM_STREAM_GATED) is not None
+                and ops.gemm_normed_takes(m, gate_up.out_features, self.hidden_size, ops.GEMM_STREAM_GATED, n_parts))
+
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         m = x.shape[0]
-        if (x.dtype == torch.bfloat16 and self.gate_up.copy_for(m) is not None and 0 < m <= self.streamed_swiglu_max_rows
+        if isinstance(x, PendingNorm):
+            act = ops.gemm_mfma_wide_swiglu(x, self.gate_up.streamed, act=self._gate_act)
+        elif (x.dtype == torch.bfloat16 and self.gate_up.copy_for(m) is not None and 0 < m <= self.streamed_swiglu_max_rows
                 and self.gate_up.wide_takes(m, 1, gate_up=True)):
             # from the fragment-ordered copy at any number of rows up to 64, and up to 128 where the
             # kernel has the launch shape for it: SiLU*up in the product's epilogue

@@ -7,7 +7,7 @@ from typing import Dict
 import torch
 
 from .. import ops
-from .base import HiddenState, Norm, ParamDecl, register_part
+from .base import HiddenState, Norm, ParamDecl, PendingNorm, register_part
 
 
 def _no_delta_bias(hidden: HiddenState, name: str) -> None:
@@ -65,6 +65,18 @@ class RMSNorm(Norm):
                                      write_back=True, delta_bias=bias)
         return ops.rmsnorm(hidden.residual, self.weight, self.eps, out_dtype, delta=delta,
                            write_back=delta is not None)
+
+    def can_wait(self, hidden: HiddenState, out_dtype: torch.dtype) -> bool:
+        delta = hidden.delta
+        return (type(self) is RMSNorm and out_dtype == torch.bfloat16 and hidden.delta_norm is None and hidden.delta_bias is None
+                and hidden.delta2 is None and hidden.delta_scale == 1.0
+                and (delta is None or (delta.ndim == 3 and delta.dtype == torch.float32)))
+
+    def wait(self, hidden: HiddenState, out_dtype: torch.dtype) -> PendingNorm:
+        old, sums = hidden.residual, hidden.delta
+        if sums is not None:
+            hidden.residual, hidden.delta = torch.empty_like(old), None
+        return PendingNorm(old, sums, self.weight, self.eps, hidden.residual, out_dtype)
 
     def rows(self, hidden: HiddenState, rows: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
         _no_second_delta(hidden, "rms_norm")

@@ -119,3 +119,63 @@ def test_every_plan_is_one_that_the_kernel_takes(ops):
         sums = linear.for_residual(x, type("Step", (), {"partial_sums_ok": True}))
         got = (sums.double().sum(0) if sums.dim() == 3 else sums.double())
         assert ((got - exact).abs() <= bound + (0 if sums.dim() == 3 else 2.0 ** -8 * exact.abs())).all(), (n, k)
+
+
+# a step of K in each half, as many as four and eight waves hold in 7, 8, 6 and 8 steps each and one fewer; N that ends inside a block of 16 rows;
+# no, one, some and all partial sums that are asked for together
+@pytest.mark.parametrize("m, n, k, parts", [(1, 4, 64, 0), (2, 36, 896, 1), (1, 1152, 896, 4), (2, 52, 864, 3), (1, 20, 1024, 8), (2, 100, 1536, 5), (1, 68, 2048, 7), (2, 48, 2016, 2)])
+@pytest.mark.parametrize("frags", [True, False])
+def test_a_norm_in_the_product_behind_it(ops, m, n, k, parts, frags):
+    gen = torch.Generator().manual_seed(n + k + parts)
+    rand = lambda *s: torch.randn(s, generator=gen).cuda()
+    res, sums, nw, w = rand(m, k), rand(parts, m, k) if parts else None, 1 + 0.1 * rand(k), rand(n, k).to(torch.bfloat16)
+    want_stream, old = res.clone(), res.clone()
+    x = ops.rmsnorm(want_stream, nw, 1e-6, torch.bfloat16, delta=sums, write_back=parts > 0)
+    exact, bound = x.double() @ w.double().t(), k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    weight = ops.fragment_order(w) if frags else w
+    new = torch.full_like(res, float("nan"))
+    for splits in (1, 2):
+        got = ops.gemm_mfma_normed(res, sums, nw, 1e-6, new, weight, ops.GEMM_STREAM_SUMS, splits=splits)
+        assert got.shape == (splits, m, n) and torch.equal(res, old)
+        assert ((got.double().sum(0) - exact).abs() <= bound).all(), splits  # (the normed row is the norm kernel's, bit for bit)
+    assert torch.equal(new, want_stream) if parts else new.isnan().all()
+    gate, up = exact[:, 0::2], exact[:, 1::2]
+    got = ops.gemm_mfma_normed(res, sums, nw, 1e-6, new, weight, ops.GEMM_STREAM_GATED, act="relu").double()
+    want, off = gate.clamp(min=0) * up, bound[:, 0::2] * up.abs() + bound[:, 1::2] * gate.abs()
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2 * off).all()
+
+
+@pytest.mark.parametrize("heads, kv", [(4, 2), (8, 2)])
+def test_steps_of_one_and_two_requests_leave_their_norms_to_the_products(heads, kv, monkeypatch):
+    """Whole steps with and without, eager and replayed: the normed rows are the same bit for bit and the products' float32 sums
+    are made in other slices, which may round to neighbouring bfloat16 values (2^-8 of a value) in each of the layers."""
+    from from_scratch_inference_engine_amd import LLM
+    from from_scratch_inference_engine_amd.engine.context import StepEntry
+    from from_scratch_inference_engine_amd.ops import functions
+    from from_scratch_inference_engine_amd.parts.block import PreNormBlock
+    from from_scratch_inference_engine_amd.parts.linear import Linear
+
+    monkeypatch.setattr(Linear, "streamed_copy_from", 1 << 19)
+    raw = {"architectures": ["Qwen2ForCausalLM"], "model_type": "qwen2", "hidden_size": 64 * heads * 2, "num_hidden_layers": 3,
+           "num_attention_heads": heads, "num_key_value_heads": kv, "head_dim": 128, "intermediate_size": 1024, "vocab_size": 500,
+           "rope_theta": 10000.0, "rms_norm_eps": 1e-6, "tie_word_embeddings": True, "max_position_embeddings": 512}
+    seen, product = [], functions.gemm_mfma_normed
+    counted = lambda *a, **k: (seen.append(a[0].shape[0]), product(*a, **k))[1]
+    for module in ("ops", "ops.functions"):  # (q/k/v asks for it, gate and up come by their own name)
+        monkeypatch.setattr(f"from_scratch_inference_engine_amd.{module}.gemm_mfma_normed", counted)
+    out = {}
+    for rows in (0, 2):
+        monkeypatch.setattr(PreNormBlock, "few_rows", rows)
+        llm = LLM.from_config(raw, weight_seed=3, block_size=16, num_blocks=64, max_batch=4, dtype="bfloat16")
+        runner, steps = llm.engine.runner, []
+        for n in (1, 2, 3):
+            caches = [runner.manager.open((n, r)) for r in range(n)]
+            runner.step([StepEntry(c, list(range(5 + r, 40 + 3 * r)), []) for r, c in enumerate(caches)])
+            for t in range(7):  # (the third of a shape is captured, the others behind it replayed)
+                steps.append(runner.step([StepEntry(c, [7 * t + r], [0]) for r, c in enumerate(caches)]))
+            for c in caches:
+                runner.manager.close(c)
+        out[rows] = torch.cat(steps)
+        assert (len(seen) == 0) if rows == 0 else (set(seen) == {1, 2} and len(seen) % 6 == 0)
+    a, b = out[0].double(), out[2].double()
+    assert ((a - b).norm(dim=1) <= 3 * 2 * 2.0 ** -8 * a.norm(dim=1)).all()
