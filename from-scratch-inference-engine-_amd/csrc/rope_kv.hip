@@ -12,6 +12,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kMaxHalf = 256;  // head_dim <= 512
+constexpr int kBlocksAUnit = 8;
 
 // angle = position * inv_freq in float64, as the plain formula has it, reduced in float64 to
 // [-pi, pi]; there float32 sine and cosine are within a few 1e-7 of the float64 ones.
@@ -182,54 +183,16 @@ __global__ __launch_bounds__(kThreads) void rope_kv_write_table_kernel(
         }
     };
 
-    // ---- values
-    bool run = !PARTS && TOK == 8 && n_here == 8 && slot[0] >= 0 && slot[0] % 8 == 0 && page_size % 8 == 0;
-#pragma unroll
-    for (int j = 1; j < TOK; ++j) run = run && slot[j] == slot[0] + j;
-    if (TOK == 8 && run) {
-        const int64_t page = slot[0] / page_size;
-        const int off = slot[0] % page_size;
-        for (int idx = first; idx < kv_dim; idx += stride) {  // lanes over the dimensions: rows read whole
-            const int kvh = idx / head_dim;
-            const int d = idx - kvh * head_dim;
-            const float b = HAS_BIAS ? bias[q_dim + kv_dim + idx] : 0.f;
-            float x[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                x[j] = to_float(qkv[static_cast<int64_t>(t0 + j) * width + q_dim + kv_dim + idx]) + b;
-            T* dst = v_pool + ((page * n_kv + kvh) * head_dim + d) * page_size + off;
-            Quad<T>::store(dst, float4{x[0], x[1], x[2], x[3]});
-            Quad<T>::store(dst + 4, float4{x[4], x[5], x[6], x[7]});
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < TOK; ++j) {
-            if (slot[j] < 0) continue;
-            const int64_t page = slot[j] / page_size;
-            const int off = slot[j] % page_size;
-            for (int idx = first * 4; idx < kv_dim; idx += stride * 4) {
-                const int kvh = idx / head_dim;
-                const int d = idx - kvh * head_dim;
-                float4 x = load4(t0 + j, q_dim + kv_dim + idx);
-                if (HAS_BIAS) {
-                    const float4 b = *reinterpret_cast<const float4*>(bias + q_dim + kv_dim + idx);
-                    x = float4{x.x + b.x, x.y + b.y, x.z + b.z, x.w + b.w};
-                }
-                T* dst = v_pool + ((page * n_kv + kvh) * head_dim + d) * page_size + off;
-                dst[0] = from_float<T>(x.x);
-                dst[page_size] = from_float<T>(x.y);
-                dst[2 * page_size] = from_float<T>(x.z);
-                dst[3 * page_size] = from_float<T>(x.w);
-            }
-        }
-    }
-
     // ---- q and k heads: unit u of a token = four pairs of one head.  The block's (token, unit) pairs are
     // dealt to the threads of its gridDim.y blocks token by token, so that neighbouring threads take
-    // neighbouring units of one token's row
+    // neighbouring units of one token's row.  The threads behind the last unit begin with the values: what a thread reads of the row
+    // does not wait for its slot, nor the heads' loads for the values' stores (values first and a loop of blocks of a token each: one token of
+    // 40/8 heads of 128 3.5 us, 2.6 so, of 16/16 of 256 6.1 and 2.7; 1,375 tokens of 14/2 of 64 6.2 and 4.5, of 40/8 of 128 23.3 and 15.4;
+    // 150 of 28/4 of 128 4.0 and 3.5; 100 in three partial sums 5.6 and 5.0).
     const int quads = half / 4;
     const int n_units = (n_heads + n_kv) * quads;
-    for (int w = first; w < n_units * n_here; w += stride) {
+    const int heads_items = n_units * n_here;
+    for (int w = first; w < heads_items; w += stride) {
         const int j = TOK == 1 ? 0 : w / n_units;
         const int u = TOK == 1 ? w : w - j * n_units;
         const int h = u / quads;
@@ -266,6 +229,52 @@ __global__ __launch_bounds__(kThreads) void rope_kv_write_table_kernel(
             T* dst = k_pool + ((page * n_kv + (h - n_heads)) * page_size + off) * head_dim;
             Quad<T>::store(dst + i, r1);
             Quad<T>::store(dst + i + half, r2);
+        }
+    }
+    // ---- values
+    if (!write_kv) return;
+    const int behind = first + (heads_items > first ? (heads_items - first + stride - 1) / stride * stride : 0) - heads_items;
+    bool run = !PARTS && TOK == 8 && n_here == 8 && slot[0] >= 0 && slot[0] % 8 == 0 && page_size % 8 == 0;
+#pragma unroll
+    for (int j = 1; j < TOK; ++j) run = run && slot[j] == slot[0] + j;
+    if (TOK == 8 && run) {
+        const int64_t page = slot[0] / page_size;
+        const int off = slot[0] % page_size;
+        for (int idx = behind; idx < kv_dim; idx += stride) {  // lanes over the dimensions: rows read whole
+            const int kvh = idx / head_dim;
+            const int d = idx - kvh * head_dim;
+            const float b = HAS_BIAS ? bias[q_dim + kv_dim + idx] : 0.f;
+            float x[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                x[j] = to_float(qkv[static_cast<int64_t>(t0 + j) * width + q_dim + kv_dim + idx]) + b;
+            T* dst = v_pool + ((page * n_kv + kvh) * head_dim + d) * page_size + off;
+            Quad<T>::store(dst, float4{x[0], x[1], x[2], x[3]});
+            Quad<T>::store(dst + 4, float4{x[4], x[5], x[6], x[7]});
+        }
+    } else {
+        const int per_token = kv_dim / 4;
+        for (int w = behind; w < per_token * n_here; w += stride) {
+            const int j = TOK == 1 ? 0 : w / per_token;
+            const int idx = (TOK == 1 ? w : w - j * per_token) * 4;
+            const int kvh = idx / head_dim;
+            const int d = idx - kvh * head_dim;
+            float4 x = load4(t0 + j, q_dim + kv_dim + idx);
+            if (HAS_BIAS) {
+                const float4 b = *reinterpret_cast<const float4*>(bias + q_dim + kv_dim + idx);
+                x = float4{x.x + b.x, x.y + b.y, x.z + b.z, x.w + b.w};
+            }
+            int sl = slot[0];
+#pragma unroll
+            for (int q = 1; q < TOK; ++q) sl = j == q ? slot[q] : sl;
+            if (sl < 0) continue;
+            const int64_t page = sl / page_size;
+            const int off = sl % page_size;
+            T* dst = v_pool + ((page * n_kv + kvh) * head_dim + d) * page_size + off;
+            dst[0] = from_float<T>(x.x);
+            dst[page_size] = from_float<T>(x.y);
+            dst[2 * page_size] = from_float<T>(x.z);
+            dst[3 * page_size] = from_float<T>(x.w);
         }
     }
 }
@@ -350,15 +359,18 @@ extern "C" int fsie_rope_kv_write_table(void* qkv, const float* cos_sin, const i
     const int write_kv = (k_pool && v_pool && slots) ? 1 : 0;
     FSIE_REQUIRE(!write_kv || (page_size > 0 && pool_slots > 0), "rope_kv_write_table: bad page geometry");
     if (n_tokens == 0) return 0;
-    // eight tokens a block where there are enough blocks left to fill the device, four blocks a run of eight
-    // tokens: the kernel is made of loads that wait for memory, so it wants many waves on every unit
-    // blocks a token: so many that the device's units all have one (64 tokens of 4,608 columns in 7 partial
-    // sums on MI355X: 9.0 us with one block a token)
+    // Eight tokens a block where there are enough blocks left to fill the device.  Blocks a token, or a run of eight: the kernel is made of
+    // loads that wait for memory, so a thread has one item (four pairs, or four values), as long as there are no more than kBlocksAUnit
+    // blocks a unit.
     const int units = fsie_compute_units();
-    const int per_token = n_tokens > 0 && units > n_tokens ? (units / n_tokens > 8 ? 8 : units / n_tokens) : 1;
-    const dim3 parts_grid(static_cast<unsigned>(n_tokens), static_cast<unsigned>(per_token));
+    const int tok = !parts && n_tokens >= 1024 ? 8 : 1, runs = (n_tokens + tok - 1) / tok;
+    const int items = tok * ((n_heads + n_kv) * (head_dim / 8) + n_kv * head_dim / 4);
+    int across = (items + kThreads - 1) / kThreads;
+    if (across > 8) across = 8;
+    while (across > 1 && static_cast<int64_t>(runs) * across > static_cast<int64_t>(kBlocksAUnit) * units) --across;
+    const dim3 grid(static_cast<unsigned>(runs), static_cast<unsigned>(across));
 #define FSIE_ROPE_PARTS(T, B)                                                                                     \
-    rope_kv_write_table_kernel<T, B, 1, true><<<parts_grid, kThreads, 0, stream>>>(                               \
+    rope_kv_write_table_kernel<T, B, 1, true><<<grid, kThreads, 0, stream>>>(                                     \
         static_cast<T*>(qkv), cos_sin, slots, bias, static_cast<T*>(k_pool), static_cast<T*>(v_pool), n_tokens,   \
         n_heads, n_kv, head_dim, page_size, write_kv, pool_slots, parts, n_parts)
     if (parts) {
@@ -373,12 +385,12 @@ extern "C" int fsie_rope_kv_write_table(void* qkv, const float* cos_sin, const i
 #undef FSIE_ROPE_PARTS
 #define FSIE_ROPE_LAUNCH(T, B)                                                                                    \
     do {                                                                                                          \
-        if (n_tokens >= 1024)                                                                                     \
-            rope_kv_write_table_kernel<T, B, 8><<<dim3((n_tokens + 7) / 8, 4), kThreads, 0, stream>>>(            \
+        if (tok == 8)                                                                                             \
+            rope_kv_write_table_kernel<T, B, 8><<<grid, kThreads, 0, stream>>>(                                   \
                 static_cast<T*>(qkv), cos_sin, slots, bias, static_cast<T*>(k_pool), static_cast<T*>(v_pool),     \
                 n_tokens, n_heads, n_kv, head_dim, page_size, write_kv, pool_slots);                              \
         else                                                                                                      \
-            rope_kv_write_table_kernel<T, B, 1><<<n_tokens, kThreads, 0, stream>>>(                               \
+            rope_kv_write_table_kernel<T, B, 1><<<grid, kThreads, 0, stream>>>(                                   \
                 static_cast<T*>(qkv), cos_sin, slots, bias, static_cast<T*>(k_pool), static_cast<T*>(v_pool),     \
                 n_tokens, n_heads, n_kv, head_dim, page_size, write_kv, pool_slots);                              \
     } while (0)
