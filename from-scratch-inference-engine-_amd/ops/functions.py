@@ -695,6 +695,36 @@ def _gemm_tile(x, weight, result: int, splits: int, tile: int, act) -> torch.Ten
     return out
 
 
+GEMM_BLOCK_PLAIN, GEMM_BLOCK_SUMS = 0, 1
+
+
+@lru_cache(maxsize=4096)
+def gemm_block_plan(m: int, n: int, k: int, result: int):
+    """(tile, slices of K) for ``gemm_mfma_block`` at these sizes; None where the library's product (as it chooses by itself) is faster or the
+    kernel does not take them."""
+    choice = int(load().fsie_gemm_mfma_block_plan(m, n, k, result, compute_units()))
+    return None if choice < 0 else (choice % 256, choice // 256)
+
+
+def gemm_mfma_block(x: torch.Tensor, weight: torch.Tensor, result: int, tile: int, splits: int = 1, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x [M, K] . weight [N, K]^T (bfloat16, N a multiple of 16, K of 64) of a hundred to some thousand rows in small tiles.
+    GEMM_BLOCK_PLAIN: [M, N] in bfloat16, ``bias`` (float32) added first; GEMM_BLOCK_SUMS: float32 partial sums [splits, M, N] over slices of K."""
+    _need(x, "gemm x", dtype=torch.bfloat16, ndim=2)
+    _need(weight, "gemm weight", dtype=torch.bfloat16, ndim=2)
+    m, k = x.shape
+    n = weight.shape[0]
+    if weight.shape[1] != k:
+        raise KernelError(f"gemm_mfma_block: x has {k} columns, weight has {weight.shape[1]}")
+    if bias is not None:
+        _need(bias, "gemm bias", dtype=torch.float32, shape=(n,))
+    if result == GEMM_BLOCK_SUMS:
+        out = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+    else:
+        out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    check(load().fsie_gemm_mfma_block(x.data_ptr(), weight.data_ptr(), _ptr(bias), out.data_ptr(), m, n, k, result, splits, tile, _stream()))
+    return out
+
+
 GEMM_STREAM_SUMS, GEMM_STREAM_GATED, GEMM_STREAM_POINT, GEMM_STREAM_PLAN_ACT, GEMM_STREAM_PLAN_ONE = 0, 1, 2, 3, 4
 
 

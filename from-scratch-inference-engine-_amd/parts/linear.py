@@ -58,6 +58,7 @@ class Linear:
         self.streamed = None  # the weight in fragment order (ops.FragmentOrdered), if prepare() made one
         self._wide_splits: dict = {}  # tiles of rows -> slices of K (a property of the sizes alone)
         self._wide_takes: dict = {}   # (tiles, slices, gate/up) -> whether the kernel takes them from this weight
+        self._many_plans: dict = {}   # (rows, result, library tuning) -> how a product of more than 128 rows is taken (of the sizes alone)
 
     @property
     def weight(self) -> Optional[torch.Tensor]:
@@ -116,6 +117,8 @@ class Linear:
         bias = None if skip_bias else self.bias
         w = self.weight
         m = x.shape[0]
+        if m > GEMM_MFMA_WIDE_MAX_M and out_dtype is None and x.dtype == torch.bfloat16 and not (self.in_features % 8 or self.out_features % 8):
+            return self._many_rows(x, bias)
         if x.dtype == torch.float32:
             if self.float32_on_matrix_cores and 2 < m <= GEMM_MFMA_SKINNY_MAX_M and self.in_features % 4 == 0:
                 # decoding in the 32-bit path: W streams once into true float32 matrix instructions
@@ -156,7 +159,32 @@ class Linear:
             # few rows with an odd inner size; float32 results from bfloat16 operands (logits of
             # many rows); and sizes whose rows are not 16-byte aligned, which the library is not given
             return ops.gemm(x, w, bias, out_dtype=out_dtype)
-        y = library_mm(x, w)
+        return self._many_rows(x, bias)
+
+    def _many_plan(self, m: int, result: int):
+        """(tile, slices of K, whether it is the kernel for many rows; else the small tiles') for ``m`` rows, or None where the library's
+        product is the better one.  Remembered by the rows: a property of the sizes alone, asked for in every layer and step."""
+        tuned = library_tuning_enabled()  # (the library's kernels chosen by timing)
+        key = (m, result, tuned)
+        if key not in self._many_plans:
+            if len(self._many_plans) > 1024:
+                self._many_plans.clear()
+            n, k = self.out_features, self.in_features
+            large = ops.gemm_tile_plan(m, n, k, ops.GEMM_TILE_SUMS) if result == ops.GEMM_BLOCK_SUMS and m > GEMM_MFMA_WIDE_MAX_M else None
+            if large is not None:
+                plan = None if large[1] == 1 and tuned else large + (True,)
+            else:
+                plan = None if tuned else ops.gemm_block_plan(m, n, k, result)
+                # (a whole product is better left in bfloat16, half the bytes for the norm)
+                plan = None if plan is None or (result == ops.GEMM_BLOCK_SUMS and plan[1] == 1) else plan + (False,)
+            self._many_plans[key] = plan
+        return self._many_plans[key]
+
+    def _many_rows(self, x: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
+        plan = self._many_plan(x.shape[0], ops.GEMM_BLOCK_PLAIN)
+        if plan is not None and self.kernel_reads(x):
+            return ops.gemm_mfma_block(x, self._weight, ops.GEMM_BLOCK_PLAIN, plan[0], bias=bias)
+        y = library_mm(x, self._weight)
         if bias is not None:
             ops.bias_add(y, bias)
         return y
@@ -191,21 +219,14 @@ class Linear:
         if x.dtype != torch.bfloat16 or m == 0:
             return None
         if m > GEMM_MFMA_WIDE_MAX_M:
-            # prompts and a long K: the product for many rows in slices of K (whole, it is no faster than the library's timed
-            # kernels: 4,096 rows of N = 3584, K = 18944 with the norm 443 us, 401; the library's own choice 567)
-            plan = ops.gemm_tile_plan(m, self.out_features, self.in_features, ops.GEMM_TILE_SUMS)
-            if plan is not None and plan[1] == 1 and library_tuning_enabled():
-                return None
-            return (ops.gemm_mfma_tile(x, self.weight, splits=plan[1], tile=plan[0])
-                    if plan is not None and self.kernel_reads(x) else None)
+            return self._many_sums(x)
         if m > GEMM_MFMA_SKINNY_MAX_M:
             # 65 to 128 rows of a fragment-ordered weight: the same kernel with five to eight tiles of x,
             # where its launch shape has one
-            if self.copy_for(m) is None:
-                return None
-            splits = self.wide_splits(m)
-            return (ops.gemm_mfma_wide(x, self.streamed, splits=splits)
-                    if splits > 1 and self.wide_takes(m, splits) and self.kernel_reads(x) else None)
+            splits = self.wide_splits(m) if self.copy_for(m) is not None else 1
+            if splits > 1 and self.wide_takes(m, splits):
+                return ops.gemm_mfma_wide(x, self.streamed, splits=splits) if self.kernel_reads(x) else None
+            return self._many_sums(x)
         if self.in_features % 8:
             return None
         if getattr(ctx, "sums_in_one", False):
@@ -223,6 +244,17 @@ class Linear:
             return ops.gemm_mfma_wide(x, self.wide_weight(m), splits=splits)
         splits = self.residual_splits(m)
         return ops.gemm_mfma_skinny(x, self.weight, splits=splits) if splits > 1 else None
+
+    def _many_sums(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """Partial sums of more than 64 rows, where slices of K are faster than a whole product: a long K in the kernel for many rows (whole,
+        it is no faster than the library's timed kernels: 4,096 rows of N = 3584, K = 18944 with the norm 443 us, 401; the library's own
+        choice 567), else in the small tiles' one."""
+        plan = self._many_plan(x.shape[0], ops.GEMM_BLOCK_SUMS)
+        if plan is None or not self.kernel_reads(x):
+            return None
+        if plan[2]:
+            return ops.gemm_mfma_tile(x, self._weight, splits=plan[1], tile=plan[0])
+        return ops.gemm_mfma_block(x, self._weight, ops.GEMM_BLOCK_SUMS, plan[0], plan[1])
 
     def partial_sums(self, x: torch.Tensor, few_rows: bool = False, long_slices: bool = False) -> Optional[torch.Tensor]:
         """x . W^T (no bias) of 17 to 64 rows (to 128 from a fragment-ordered copy) as float32 partial
