@@ -5,11 +5,16 @@
 // A workgroup of four waves makes a tile of 64 x 64, 64 x 128 or 128 x 128 rows of X and W, a wave a quarter of it.  Both operands go
 // through LDS, 64 values of K at a time, straight from memory, in three stages: one is read, one has arrived or is about to, one is
 // asked for behind the barrier that says that every wave has read it.  One barrier a step.
-// What bounds it: how much a unit can have under way.  A step takes 0.235, 0.305 and 0.53 us for the three tiles, which is 60 to 79 GB/s a
-// unit of 140 that it draws from its L2 at most; without its loads it takes 0.2 to 0.4, without its products or its reads of LDS as long as
-// with them.  Stages beyond three (eight of 64 x 64) and the next step's fragments read ahead into registers changed nothing, two stages
-// and twice the workgroups a unit lost (0.6 us).  At 1,375 rows, cold weights: N = 1152, K = 896 8.1 us where the library's product takes 9.6, N = K = 896
-// 7.6 and 9.2; at 512 rows 6.0 and 8.3, 5.9 and 8.1; 1,000 of N = K = 2048 14.6 and 16.9.  A call of the library's is 21 us of the host besides, one of this 13.
+// What bounds it: how much a unit can have under way, and where W lies.  Weights are read once a pass and come from HBM, 1.4 us away; the
+// loads of a unit return in order, so that the tiles took 0.34, 0.41 and 0.55 us a step where weights in the caches took 0.24, 0.30 and 0.36.
+// So a workgroup first asks for its share of the W that the workgroups of its die will read (see below): at 1,375 rows, cold weights, N = 1152,
+// K = 896 took 8.7 us without and takes 7.5, 1,000 rows of N = K = 3584 35.2 and 30.4, 1,375 of N = K = 2048 20.7 and 17.0.  Where all tiles of
+// 64 x 64 are on the chip at once six stages fit: 512 rows of N = 1024, K = 4096 15.0 us instead of 18.6, 512 of N = K = 2048 9.7 as with three.
+// A step of 128 x 128 took 0.53 us with its loads, its reads of LDS and its products each in a row, and takes 0.36 with them in turns.
+// Without gain: more stages for the larger tiles, two stages and twice the workgroups a unit, other permutations in LDS, two steps' lines of a row
+// asked for together; a fifth wave that asks for W along the way (it holds up the other four's loads).
+// The library's product takes 11.3 us of the first size above, 36.9 and 21.7 of the others; a call of the library's is 21 us of the host besides,
+// one of this 13.
 #include "common.h"
 #include "api.h"
 
@@ -22,15 +27,18 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kStep = 64;  // values of K a stage
 constexpr int kRowBytes = kStep * 2;
 
+constexpr int kTouched = FSIE_WAVE * 4;  // a wave's values of lines that it only asks for
+
 enum Result { kPlain = 0, kSums = 1 };  // bfloat16 [M, N] with a bias; float32 [splits, M, N]
 
 // A tile: 32 T rows of X by 32 J rows of W, a wave of four a quarter of it.
-template <int T, int J>
+template <int T, int J, int STAGES>
 struct Shape {
     static constexpr int kRows = 32 * T, kCols = 32 * J;
     static constexpr int kStage = (kRows + kCols) * kRowBytes;  // W, then X
     static constexpr int kLoads = T + J;                        // a wave's, of eight rows each: J of W, T of X
-    static constexpr int kStages = 3;
+    static constexpr int kStages = STAGES;
+    static constexpr int kLds = kStages * kStage + 4 * kTouched;
 };
 
 // 16 bytes a lane from memory to LDS, lane i's at lds + 16 i (m0 is an operand; the wait state behind its write is not the compiler's to
@@ -39,6 +47,15 @@ __device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t lds, uint32_t o
     asm volatile(
         "s_nop 0\n\t"
         "buffer_load_dwordx4 %1, %2, %3 offen lds"
+        :
+        : "{m0}"(lds), "v"(offset), "s"(rsrc), "s"(k_offset)
+        : "memory");
+}
+// Four bytes a lane, as above.
+__device__ __forceinline__ void touch(u32x4 rsrc, uint32_t lds, uint32_t offset, uint32_t k_offset) {
+    asm volatile(
+        "s_nop 0\n\t"
+        "buffer_load_dword %1, %2, %3 offen lds"
         :
         : "{m0}"(lds), "v"(offset), "s"(rsrc), "s"(k_offset)
         : "memory");
@@ -61,26 +78,17 @@ template <int J>
 __device__ __forceinline__ int w_key(int row) { return (row >> 1 & 1) | (row % (16 * J) / (4 * J)) << 1; }
 __device__ __forceinline__ int x_key(int row) { return row >> 1 & 7; }
 
-template <int RESULT, int T, int J>
+template <int RESULT, int T, int J, int STAGES>
 __global__ __launch_bounds__(256, 1) void gemm_block_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                             const float* __restrict__ bias, void* __restrict__ y, int M, int N, int K,
-                                                            int m_tiles, int n_tiles, int splits, int n_outside) {
-    using S = Shape<T, J>;
+                                                            int m_tiles, int n_tiles, int splits) {
+    using S = Shape<T, J, STAGES>;
     extern __shared__ char lds[];
-    // a die (the workgroup's number modulo 8) takes neighbouring tiles: of the larger operand its own eighth, of the other one all
+    // a die (the workgroup's number modulo 8) takes neighbouring tiles: of W its own eighth, of X all
     const int tiles = m_tiles * n_tiles * splits, a_die = (tiles + 7) / 8;
     const int id = static_cast<int>(blockIdx.x & 7) * a_die + static_cast<int>(blockIdx.x >> 3);
     if (id >= tiles) return;
-    int m_tile, n_tile, slice;
-    if (n_outside) {
-        m_tile = id % m_tiles;
-        n_tile = id / m_tiles % n_tiles;
-        slice = id / m_tiles / n_tiles;
-    } else {
-        n_tile = id % n_tiles;
-        m_tile = id / n_tiles % m_tiles;
-        slice = id / n_tiles / m_tiles;
-    }
+    const int m_tile = id % m_tiles, n_tile = id / m_tiles % n_tiles, slice = id / m_tiles / n_tiles;
     const int m0 = m_tile * S::kRows, n0 = n_tile * S::kCols;
     const int all_steps = K / kStep;
     const int first_step = static_cast<int>(static_cast<int64_t>(all_steps) * slice / splits);
@@ -108,14 +116,23 @@ __global__ __launch_bounds__(256, 1) void gemm_block_kernel(const bf16_t* __rest
         x_from[i] = static_cast<uint32_t>(min(m0 + r, M - 1)) * static_cast<uint32_t>(K) * 2u + ((lane & 7) ^ x_key(r)) * 16u;
     }
     uint32_t bring_to = 0, read_from = 0;  // the stages' places, in turn
-    const auto bring = [&](int step) {
-        const uint32_t k = static_cast<uint32_t>(first_step + min(step, steps - 1)) * kRowBytes, to = lds0 + bring_to;
-#pragma unroll
-        for (int i = 0; i < J; ++i) load_to_lds(w_rows, to + (wave * J + i) * 1024u, w_from[i], k);
-#pragma unroll
-        for (int i = 0; i < T; ++i) load_to_lds(x_rows, to + S::kCols * kRowBytes + (wave * T + i) * 1024u, x_from[i], k);
-        bring_to = bring_to == (S::kStages - 1) * S::kStage ? 0 : bring_to + S::kStage;
+    const auto next_stage = [](uint32_t at) { return at == (S::kStages - 1) * S::kStage ? 0u : at + S::kStage; };
+    const auto k_of = [&](int step) { return static_cast<uint32_t>(first_step + min(step, steps - 1)) * kRowBytes; };
+    const auto load = [&](int i, uint32_t k) {  // the i-th of this wave's loads of a stage
+        if (i < J) load_to_lds(w_rows, lds0 + bring_to + (wave * J + i) * 1024u, w_from[i], k);
+        else load_to_lds(x_rows, lds0 + bring_to + S::kCols * kRowBytes + (wave * T + i - J) * 1024u, x_from[i - J], k);
     };
+
+    // What of W the stages at the start leave is asked for at once, a value a line, and goes nowhere: the workgroups of this tile of W and
+    // slice, on one die but for few, share its steps.  From HBM a line is 1.4 us away, and three stages would wait for it at every step.
+    if (m_tiles > 2) {
+        for (int step = S::kStages + 4 * m_tile + wave; step < steps; step += 4 * m_tiles) {
+#pragma unroll
+            for (int c = 0; c < S::kCols / FSIE_WAVE; ++c)
+                touch(w_rows, lds0 + S::kStages * S::kStage + wave * kTouched,
+                      static_cast<uint32_t>(min(n0 + c * FSIE_WAVE + lane, N - 1)) * static_cast<uint32_t>(K) * 2u, k_of(step));
+        }
+    }
 
     // Fragments: A = 16 rows of W, B = 16 rows of X, a lane 8 values of K (16 bytes).  Row r of tile j of W is row
     // (r / 4) * 4 J + j * 4 + r % 4 of the wave's 16 J, so that a lane's results of the J tiles are 4 J neighbours.
@@ -129,33 +146,56 @@ __global__ __launch_bounds__(256, 1) void gemm_block_kernel(const bf16_t* __rest
 #pragma unroll
         for (int t = 0; t < T; ++t) acc[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    bring(0);
-    bring(1);
-    for (int step = 0; step < steps; ++step) {
-        // all but the youngest stage's loads have arrived, and what this wave has read of the stage before is in its registers
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(S::kLoads) : "memory");
+    bf16x8 a[2][J][2], b[2][T][2];  // this step's fragments and the next one's
+    const auto read = [&](int i, bf16x8 (&to_a)[J][2], bf16x8 (&to_b)[T][2]) {  // the i-th of a stage's 2 (J + T) fragments
+        const char* stage = lds + read_from;
+        const int h = i / (J + T), f = i % (J + T);
+        if (f < J) to_a[f][h] = *reinterpret_cast<const bf16x8*>(stage + w_at + f * 4 * kRowBytes + (((h * 4 + kg) ^ wk) * 16));
+        else to_b[f - J][h] = *reinterpret_cast<const bf16x8*>(stage + x_at + (f - J) * 16 * kRowBytes + (((h * 4 + kg) ^ xk) * 16));
+    };
+    // A step: the next stage has arrived (all loads but the youngest stage's) and this step's fragments are in every wave's registers,
+    // so its stage is free for the one after the next two.  A load, two fragments of the next step and this step's products go in
+    // turns: eight loads in a row are waited for in the units' address queue as long as the products take, and reads in a row in the LDS's.
+    const auto go = [&](int step, const bf16x8 (&fa)[J][2], const bf16x8 (&fb)[T][2], bf16x8 (&next_a)[J][2], bf16x8 (&next_b)[T][2]) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((S::kStages - 2) * S::kLoads) : "memory");
         FSIE_BLOCK_FENCE();
         __builtin_amdgcn_s_barrier();
         FSIE_BLOCK_FENCE();
-        bring(step + 2);  // into the stage that was read before the barrier
-        const char* stage = lds + read_from;
-        read_from = read_from == (S::kStages - 1) * S::kStage ? 0 : read_from + S::kStage;
-        bf16x8 a[J][2], b[T][2];
+        const uint32_t k = k_of(step + S::kStages);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int c = 0; c < J + T; ++c) {
+            constexpr int kProducts = 2 * J * T;
 #pragma unroll
-            for (int j = 0; j < J; ++j)
-                a[j][h] = *reinterpret_cast<const bf16x8*>(stage + w_at + j * 4 * kRowBytes + (((h * 4 + kg) ^ wk) * 16));
-#pragma unroll
-            for (int t = 0; t < T; ++t)
-                b[t][h] = *reinterpret_cast<const bf16x8*>(stage + x_at + t * 16 * kRowBytes + (((h * 4 + kg) ^ xk) * 16));
+            for (int q = c * kProducts / (J + T); q < (c + 1) * kProducts / (J + T); ++q) {
+                const int h = q / (J * T), t = q / J % T, j = q % J;
+                acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[j][h], fb[t][h], acc[j][t], 0, 0, 0);
+            }
+            read(2 * c, next_a, next_b);
+            read(2 * c + 1, next_a, next_b);
+            load(c, k);
+            FSIE_BLOCK_FENCE();
         }
+        bring_to = next_stage(bring_to);
+        read_from = next_stage(read_from);
+    };
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+    for (int i = 0; i < S::kStages; ++i) {
+        const uint32_t k = k_of(i);
 #pragma unroll
-            for (int t = 0; t < T; ++t)
+        for (int c = 0; c < J + T; ++c) load(c, k);
+        bring_to = next_stage(bring_to);
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S::kStages - 1) * S::kLoads) : "memory");
+    FSIE_BLOCK_FENCE();
+    __builtin_amdgcn_s_barrier();
+    FSIE_BLOCK_FENCE();
 #pragma unroll
-                for (int j = 0; j < J; ++j) acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j][h], b[t][h], acc[j][t], 0, 0, 0);
+    for (int i = 0; i < 2 * (J + T); ++i) read(i, a[0], b[0]);
+    read_from = next_stage(read_from);
+    for (int step = 0; step < steps; step += 2) {
+        go(step, a[0], b[0], a[1], b[1]);
+        if (step + 1 >= steps) break;
+        go(step + 1, a[1], b[1], a[0], b[0]);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (no load may still write LDS when the workgroup's is given away)
 
@@ -198,16 +238,16 @@ struct Call {
     hipStream_t stream;
 };
 
-template <int RESULT, int T, int J>
+template <int RESULT, int T, int J, int STAGES>
 int launch(const Call& c) {
-    using S = Shape<T, J>;
+    using S = Shape<T, J, STAGES>;
     const int m_tiles = (c.M + S::kRows - 1) / S::kRows, n_tiles = (c.N + S::kCols - 1) / S::kCols;
     const unsigned groups = static_cast<unsigned>((m_tiles * n_tiles * c.splits + 7) / 8 * 8);
-    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_block_kernel<RESULT, T, J>),
-                                                          hipFuncAttributeMaxDynamicSharedMemorySize, S::kStages * S::kStage);
-    FSIE_REQUIRE(allowed == hipSuccess, "gemm_mfma_block: %d bytes of LDS: %s", S::kStages * S::kStage, hipGetErrorString(allowed));
-    gemm_block_kernel<RESULT, T, J><<<groups, 256, S::kStages * S::kStage, c.stream>>>(c.x, c.w, c.bias, c.y, c.M, c.N, c.K, m_tiles, n_tiles,
-                                                                                   c.splits, c.N >= c.M);
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_block_kernel<RESULT, T, J, STAGES>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, S::kLds);
+    FSIE_REQUIRE(allowed == hipSuccess, "gemm_mfma_block: %d bytes of LDS: %s", S::kLds, hipGetErrorString(allowed));
+    gemm_block_kernel<RESULT, T, J, STAGES><<<groups, 256, S::kLds, c.stream>>>(c.x, c.w, c.bias, c.y, c.M, c.N, c.K, m_tiles, n_tiles,
+                                                                                   c.splits);
     FSIE_CHECK_LAUNCH("gemm_mfma_block");
     return 0;
 }
@@ -215,9 +255,10 @@ int launch(const Call& c) {
 template <int RESULT>
 int launch_shape(int tile, const Call& c) {
     switch (tile) {
-        case 0: return launch<RESULT, 2, 2>(c);
-        case 1: return launch<RESULT, 2, 4>(c);
-        default: return launch<RESULT, 4, 4>(c);
+        case 0: return launch<RESULT, 2, 2, 3>(c);
+        case 1: return launch<RESULT, 2, 4, 3>(c);
+        case 2: return launch<RESULT, 4, 4, 3>(c);
+        default: return launch<RESULT, 2, 2, 6>(c);
     }
 }
 
@@ -225,29 +266,29 @@ int launch_shape(int tile, const Call& c) {
 
 // Which tile, and in how many slices of K, M rows of this product are best taken; -1: the library's product is faster or the sizes are not
 // the kernel's.  Returns tile + 256 * slices.
-// The rule is the time that a count of steps gives: fixed + steps * a step's, workgroups that share a unit taking turns (0.92 and 1.05 of a
-// step each, as many as the unit's LDS holds), weights that come from HBM, at its latency, up to 1.35 and 1.1 of that; partial sums count their
-// bytes here and in the norm at 4.5 TB/s.  It has to be 0.92 of the library's 6.5 us and 0.95 PFLOP/s, or 3 us and its weights at 2.5 TB/s: the least that
-// it took at 24 matrices of 1 to 33 MB and 19 numbers of rows from 70 to 4,096.  Of these 456 and as many with slices and the norm the rule takes 237,
-// at a median of 0.77 of the library's time, the largest 1.04 (this / the library and the norm: 96 rows of N = 896, K = 4864 8.8 / 12.4, 256 12.0 / 14.6; 96 of
-// N = 2048, K = 8192 17.7 / 24.3, 129 20.6 / 29.6; 96 of N = K = 3584 16.4 / 23.3; whole, 256 of N = 3072, K = 1024 6.6 / 9.1; 850 of N = K = 2048 14.1 / 15.8).
+// The rule is the time that a count of steps gives: fixed + steps * a step's, workgroups that share a unit taking turns (so many as the unit's LDS
+// holds; a second round of 128 x 128 was up to 1.36 of the library's time and is not taken), the weights from HBM at 6.7 to 9 TB/s more; partial sums
+// count their bytes here and in the norm at 4.5 TB/s.  It has to be 0.9 of the library's 9.7 us and 1 PFLOP/s, or 8.2 us and its weights at 2.3 TB/s, as it
+// takes them from HBM at 24 matrices of 1 to 50 MB and 19 numbers of rows from 70 to 4,096.  Of these 456 and as many with slices and the norm the rule takes
+// 392, at a median of 0.74 of the library's time, the largest 1.03 but for 129 rows of N = 8192, K = 2048 (1.13; this / the library, us: 1,375 rows of N = 1152,
+// K = 896 7.5 / 11.3, 1,000 of N = K = 3584 30.4 / 36.9, 2,048 of N = 2048, K = 8192 67.7 / 75.5, 256 of N = 3072, K = 1024 6.9 / 11.9; with the norm, 96 rows of N = 896,
+// K = 4864 in six slices 9.4 / 15.7, 96 of N = 2048, K = 8192 in four 15.3 / 24.0).
 extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int units) {
     if (M <= 0 || N <= 0 || K <= 0 || units <= 0 || N % 16 || K % kStep || (result != kPlain && result != kSums)) return -1;
     if (static_cast<int64_t>(M) * K * 2 >= (int64_t{1} << 31) || static_cast<int64_t>(N) * K * 2 >= (int64_t{1} << 31)) return -1;
-    const int rows[3] = {64, 64, 128}, cols[3] = {64, 128, 128};
-    const double us_a_step[3] = {0.235, 0.305, 0.58}, fixed[3] = {2.3, 2.6, 3.4};
+    const int rows[4] = {64, 64, 128, 64}, cols[4] = {64, 128, 128, 64}, at_once[4] = {3, 2, 1, 1};
+    const double us_a_step[4] = {0.228, 0.295, 0.405, 0.182}, fixed[4] = {2.5, 3.2, 4.2, 3.1}, us_a_mb[4] = {0.15, 0.15, 0.13, 0.11};
+    const double turns[4][4] = {{0, 1, 1.55, 2.6}, {0, 1, 1.9}, {0, 1}, {0, 1}};  // workgroups on a unit: a step's time of one alone
     const int64_t steps = K / kStep;
     const double weights = 2.0 * N * static_cast<double>(K), flops = 2.0 * M * static_cast<double>(N) * K;
     double best = 1e30;
     int choice = -1;
-    for (int tile = 0; tile < 3; ++tile) {
+    for (int tile = 0; tile < 4; ++tile) {
         for (int slices = 1; slices <= (result == kSums ? 8 : 1); ++slices) {
             if (slices > 1 && steps / slices < 4) break;
             const int64_t groups = ceil_div64(M, rows[tile]) * ceil_div64(N, cols[tile]) * slices, deep = ceil_div64(groups, units);
-            if (deep > 3 - tile) continue;  // (so many a unit's LDS holds)
-            const double from_memory = weights < 10e6 ? 0.0 : weights < 16e6 ? 0.7 : 1.0;
-            const double step = us_a_step[tile] * (1.0 + from_memory * (tile == 2 ? 0.1 : 0.35)) * (deep > 1 ? (tile == 0 ? 0.92 : 1.05) * deep : 1.0);
-            double us = fixed[tile] + static_cast<double>(ceil_div64(steps, slices)) * step;
+            if (deep > at_once[tile]) continue;
+            double us = fixed[tile] + static_cast<double>(ceil_div64(steps, slices)) * us_a_step[tile] * turns[tile][deep] + weights * 1e-6 * us_a_mb[tile];
             if (result == kSums) us += 8.0 * slices * M * static_cast<double>(N) / 4.5e6;
             if (us < best) {
                 best = us;
@@ -255,8 +296,8 @@ extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int un
             }
         }
     }
-    const double product = 6.5 + flops / 0.95e9, read = 3.0 + weights / 2.5e6;
-    return choice >= 0 && best <= 0.92 * (product > read ? product : read) ? choice : -1;
+    const double product = 9.7 + flops / 1e9, read = 8.2 + weights / 2.3e6;
+    return choice >= 0 && best <= 0.9 * (product > read ? product : read) ? choice : -1;
 }
 
 extern "C" int fsie_gemm_mfma_block(const void* x, const void* w, const float* bias, void* y, int M, int N, int K, int result, int splits,
@@ -266,7 +307,7 @@ extern "C" int fsie_gemm_mfma_block(const void* x, const void* w, const float* b
     FSIE_REQUIRE(result == kPlain || result == kSums, "gemm_mfma_block: unknown result %d", result);
     FSIE_REQUIRE(splits >= 1 && splits <= K / kStep && (splits == 1 || result == kSums), "gemm_mfma_block: %d slices", splits);
     FSIE_REQUIRE(!bias || result == kPlain, "gemm_mfma_block: partial sums take no bias");
-    FSIE_REQUIRE(tile >= 0 && tile <= 2, "gemm_mfma_block: unknown tile %d", tile);
+    FSIE_REQUIRE(tile >= 0 && tile <= 3, "gemm_mfma_block: unknown tile %d", tile);
     FSIE_REQUIRE(static_cast<int64_t>(M) * K * 2 < (int64_t{1} << 31) && static_cast<int64_t>(N) * K * 2 < (int64_t{1} << 31),
                  "gemm_mfma_block: operands of %d x %d and %d x %d are more than the kernel's 32-bit offsets take", M, K, N, K);
     FSIE_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0 &&

@@ -16,7 +16,7 @@ def ops():
 
 # one step of K, fewer steps than stages, a last tile of one row and one of 16 of N, a whole number of tiles, more tiles than units
 @pytest.mark.parametrize("m, n, k", [(65, 16, 64), (1, 48, 128), (129, 144, 192), (128, 256, 320), (300, 1152, 896), (513, 272, 1088), (1375, 896, 256)])
-@pytest.mark.parametrize("tile", [0, 1, 2])
+@pytest.mark.parametrize("tile", [0, 1, 2, 3])
 def test_products_in_small_tiles(ops, m, n, k, tile):
     gen = torch.Generator().manual_seed(m + n + k)
     x, w = (torch.randn(s, generator=gen).to(torch.bfloat16).cuda() for s in ((m, k), (n, k)))
