@@ -267,12 +267,12 @@ int launch_shape(int tile, const Call& c) {
 // Which tile, and in how many slices of K, M rows of this product are best taken; -1: the library's product is faster or the sizes are not
 // the kernel's.  Returns tile + 256 * slices.
 // The rule is the time that a count of steps gives: fixed + steps * a step's, workgroups that share a unit taking turns (so many as the unit's LDS
-// holds; a second round of 128 x 128 was up to 1.36 of the library's time and is not taken), the weights from HBM at 6.7 to 9 TB/s more; partial sums
-// count their bytes here and in the norm at 4.5 TB/s.  It has to be 0.9 of the library's 9.7 us and 1 PFLOP/s, or 8.2 us and its weights at 2.3 TB/s, as it
-// takes them from HBM at 24 matrices of 1 to 50 MB and 19 numbers of rows from 70 to 4,096.  Of these 456 and as many with slices and the norm the rule takes
-// 392, at a median of 0.74 of the library's time, the largest 1.03 but for 129 rows of N = 8192, K = 2048 (1.13; this / the library, us: 1,375 rows of N = 1152,
-// K = 896 7.5 / 11.3, 1,000 of N = K = 3584 30.4 / 36.9, 2,048 of N = 2048, K = 8192 67.7 / 75.5, 256 of N = 3072, K = 1024 6.9 / 11.9; with the norm, 96 rows of N = 896,
-// K = 4864 in six slices 9.4 / 15.7, 96 of N = 2048, K = 8192 in four 15.3 / 24.0).
+// holds; a second round of 128 x 128 was up to 1.36 of the library's time and is not taken), the weights from HBM at 6.7 to 9 TB/s more; a whole product's
+// bytes or the slices' sums here and in the norm at 3 TB/s.  It has to be 0.95 of the library's 8.9 us, 1.25 PFLOP/s and weights at 3.3 TB/s, as it takes them
+// from HBM at 24 matrices of 1 to 50 MB and 19 numbers of rows from 70 to 4,096.  Of these 456 and as many with slices and the norm the rule takes 426, at a
+// median of 0.75 of the library's time, the largest 1.02 but for 129 rows of N = 8192, K = 2048 (1.13; this / the library, us: 1,375 rows of N = 1152,
+// K = 896 7.5 / 11.3, 512 of N = 4608, K = 3584 28.9 / 33.3, 1,000 of N = K = 3584 30.4 / 36.9, 2,048 of N = 2048, K = 8192 67.7 / 75.5, 256 of N = 3072, K = 1024 6.9 / 11.9; with
+// the norm, 96 rows of N = 896, K = 4864 in six slices 9.4 / 15.7, 96 of N = 2048, K = 8192 in four 15.3 / 24.0).
 extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int units) {
     if (M <= 0 || N <= 0 || K <= 0 || units <= 0 || N % 16 || K % kStep || (result != kPlain && result != kSums)) return -1;
     if (static_cast<int64_t>(M) * K * 2 >= (int64_t{1} << 31) || static_cast<int64_t>(N) * K * 2 >= (int64_t{1} << 31)) return -1;
@@ -281,6 +281,7 @@ extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int un
     const double turns[4][4] = {{0, 1, 1.55, 2.6}, {0, 1, 1.9}, {0, 1}, {0, 1}};  // workgroups on a unit: a step's time of one alone
     const int64_t steps = K / kStep;
     const double weights = 2.0 * N * static_cast<double>(K), flops = 2.0 * M * static_cast<double>(N) * K;
+    const double whole = 4.0 * M * static_cast<double>(N) / 3e6;  // the delta in bfloat16, out and into the norm
     double best = 1e30;
     int choice = -1;
     for (int tile = 0; tile < 4; ++tile) {
@@ -289,15 +290,14 @@ extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int un
             const int64_t groups = ceil_div64(M, rows[tile]) * ceil_div64(N, cols[tile]) * slices, deep = ceil_div64(groups, units);
             if (deep > at_once[tile]) continue;
             double us = fixed[tile] + static_cast<double>(ceil_div64(steps, slices)) * us_a_step[tile] * turns[tile][deep] + weights * 1e-6 * us_a_mb[tile];
-            if (result == kSums) us += 8.0 * slices * M * static_cast<double>(N) / 4.5e6;
+            if (result == kSums) us += (slices == 1 ? whole : 2.0 * slices * whole);
             if (us < best) {
                 best = us;
                 choice = tile + 256 * slices;
             }
         }
     }
-    const double product = 9.7 + flops / 1e9, read = 8.2 + weights / 2.3e6;
-    return choice >= 0 && best <= 0.9 * (product > read ? product : read) ? choice : -1;
+    return choice >= 0 && best <= 0.95 * (8.9 + flops / 1.25e9 + weights / 3.3e6 + (result == kSums ? whole : 0.0)) ? choice : -1;
 }
 
 extern "C" int fsie_gemm_mfma_block(const void* x, const void* w, const float* bias, void* y, int M, int N, int K, int result, int splits,

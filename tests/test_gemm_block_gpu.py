@@ -55,7 +55,7 @@ def test_linear_takes_them(ops, m, n, k, monkeypatch):
     exact = x.double() @ layer.weight.double().t()
     size = exact.abs() + layer.bias.double().abs() + k * 2.0 ** -24 * (x.double().abs() @ layer.weight.double().abs().t())
     assert ((layer(x).double() - exact - layer.bias.double()).abs() <= 2.0 ** -7 * size).all()
-    plain = ops.gemm_block_plan(m, n, k, ops.GEMM_BLOCK_PLAIN) is not None and m > 128
+    plain = ops.gemm_block_plan(m, n, k, ops.GEMM_BLOCK_PLAIN) is not None
     assert (ops.GEMM_BLOCK_PLAIN in seen) == plain
     layer.bias, layer.has_bias = None, False
     delta = layer.for_residual(x, SimpleNamespace(partial_sums_ok=True))
