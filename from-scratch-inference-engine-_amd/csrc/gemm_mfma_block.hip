@@ -17,12 +17,14 @@
 // one of this 13.
 #include "common.h"
 #include "api.h"
+#include "lds_loads.h"
 
 namespace {
 
+using namespace fsie_lds;
+
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kStep = 64;  // values of K a stage
 constexpr int kRowBytes = kStep * 2;
@@ -41,36 +43,7 @@ struct Shape {
     static constexpr int kLds = kStages * kStage + 4 * kTouched;
 };
 
-// 16 bytes a lane from memory to LDS, lane i's at lds + 16 i (m0 is an operand; the wait state behind its write is not the compiler's to
-// put inside an asm statement).
-__device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t lds, uint32_t offset, uint32_t k_offset) {
-    asm volatile(
-        "s_nop 0\n\t"
-        "buffer_load_dwordx4 %1, %2, %3 offen lds"
-        :
-        : "{m0}"(lds), "v"(offset), "s"(rsrc), "s"(k_offset)
-        : "memory");
-}
-// Four bytes a lane, as above.
-__device__ __forceinline__ void touch(u32x4 rsrc, uint32_t lds, uint32_t offset, uint32_t k_offset) {
-    asm volatile(
-        "s_nop 0\n\t"
-        "buffer_load_dword %1, %2, %3 offen lds"
-        :
-        : "{m0}"(lds), "v"(offset), "s"(rsrc), "s"(k_offset)
-        : "memory");
-}
 #define FSIE_BLOCK_FENCE() __builtin_amdgcn_sched_barrier(0)
-
-__device__ __forceinline__ u32x4 rows_from(const bf16_t* base, uint32_t bytes) {
-    const uint64_t at = reinterpret_cast<uint64_t>(base);
-    u32x4 r;
-    r[0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at));
-    r[1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at >> 32));
-    r[2] = __builtin_amdgcn_readfirstlane(bytes);
-    r[3] = 0x00020000u;
-    return r;
-}
 
 // The permutation of a row's eight 16-byte units in LDS: W's rows are read 16 at a time as 4 runs of 4 that lie 4 J apart, X's as 16
 // neighbours; in both any eight lanes in a row meet eight different units.

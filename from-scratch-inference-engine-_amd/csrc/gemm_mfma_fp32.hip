@@ -9,6 +9,7 @@
 // what the other rows hold.
 #include "common.h"
 #include "api.h"
+#include "lds_loads.h"
 
 namespace {
 
@@ -142,18 +143,45 @@ int launch_mt(int waves, const float* x, const float* w, const float* bias, floa
 }
 
 // ---- many rows (prompts) ----------------------------------------------------------------------
-// A workgroup of four waves makes 64 rows of X by 64 of W, a wave 32 by 32; 32 values of K at a time go through two
-// stages of LDS (the next one's loads are under way while this one is multiplied), a row's eight 16-byte units permuted
-// by the row so that eight rows' reads meet different banks.  A wave's read of 16 bytes a lane feeds four instructions
-// of 32 cycles each, so the matrix cores are the bound (busy in 0.71 of the units' cycles at 2,048 x 3584 x 18944, 0.66 at
-// 682 x 9728 x 896, where the LDS is in 0.17, without bank conflicts), and the small tile is what fills the chip: a unit holds
-// five workgroups, and N = 896 at 682 rows still makes 154 of them (in slices of K as many times that).
-// Two levels of float32 sums as above, runs of kTileFlush values of K.  108 TFLOP/s at 2,048 x
-// 3584 x 18944 (154 is what the library reaches at 8,192 cubed); against the vector kernel before it 5,090 -> 2,580 us there,
-// 211 -> 136 at 682 x 9728 x 896, and in seven slices 822 -> 77 at 682 x 896 x 4864.
+// A workgroup of four waves makes 64 rows of X by 64 of W, a wave 32 by 32; 32 values of K at a time go through LDS, a row's eight 16-byte
+// units permuted by the row so that the rows' reads meet different banks.  A wave's read of 16 bytes a lane feeds four instructions of 32
+// cycles each, so the matrix cores are the bound, and the small tile is what fills the chip: N = 896 at 682 rows makes 154 of them (in slices
+// of K as many times that).  Two levels of float32 sums as above, runs of kTileFlush values of K.
+// Through registers and two stages (the first kernel, for K that is no multiple of 32) the matrix cores were busy in 0.66 to 0.71 of the
+// units' cycles: 682 x 9728 x 896 132 us, 682 x 3584 x 18944 1,116, 300 x 1152 x 896 27.8, 128 x 4608 x 3584 102, in seven slices 300 x 896 x 4864
+// 41.7, weights from HBM.  Straight to LDS, the loads, the reads and the products of three stages in turns (the second kernel): 114, 894, 21.2, 74
+// and 34.4; 117 TFLOP/s at 1,500 x 9728 x 896 (96 before), where the library reaches 154 at 8,192 cubed.  Six stages where every workgroup has a unit
+// to itself, whose step of 0.43 us would else not cover the way from HBM; three leave room for three workgroups a unit.
 constexpr int kTileEdge = 64, kTileK = 32, kTileFlush = 256;
+constexpr int kFewTiles = 256;  // so many workgroups have a unit each
 
 enum Whole { PLAIN = 0, SUMS = 1, GATED = 2 };
+
+// A lane holds D[n .. n + 4][m] of a wave's 2 x 2 tiles; m and n: of the first.
+template <int RESULT>
+__device__ __forceinline__ void write_tile(const floatx4 (&acc)[2][2], const floatx4 (&total)[2][2], float* __restrict__ y, const float* __restrict__ bias,
+                                           const Gate& gate, int M, int N, int m_first, int n_first, int slice) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int m = m_first + 16 * t;
+        if (m >= M) continue;
+        float* to = RESULT == GATED ? y + static_cast<int64_t>(m) * (N / 2) : y + (static_cast<int64_t>(RESULT == SUMS ? slice : 0) * M + m) * N;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int n = n_first + 16 * j;
+            const floatx4 v = acc[j][t] + total[j][t];
+            if constexpr (RESULT == GATED) {
+#pragma unroll
+                for (int i = 0; i < 4; i += 2)
+                    if (n + i < N) to[(n + i) / 2] = gate_pair(v[i], v[i + 1], gate.act, gate.limit, gate.slope);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (n + i < N) to[n + i] = RESULT == PLAIN && bias ? v[i] + bias[n + i] : v[i];
+            }
+        }
+    }
+}
 
 template <int RESULT>
 __global__ __launch_bounds__(256) void gemm_fp32_tile_kernel(const float* __restrict__ x, const float* __restrict__ w,
@@ -224,28 +252,133 @@ __global__ __launch_bounds__(256) void gemm_fp32_tile_kernel(const float* __rest
                 }
         }
     }
-    // lane holds D[n .. n + 4][m]
+    write_tile<RESULT>(acc, total, y, bias, gate, M, N, m0 + mw + row, n0 + nw + 4 * kg, static_cast<int>(blockIdx.z));
+}
+
+// The same tiles where K is a whole number of steps: both operands go to LDS straight from memory, STAGES - 1 steps ahead, and a wave reads the
+// next step's fragments, asks for its share of a later stage and multiplies this step's in turns.  The order of every sum is that of the kernel
+// above, and so are its bits.
+template <int RESULT, int STAGES>
+__global__ __launch_bounds__(256) void gemm_fp32_block_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                             const float* __restrict__ bias, float* __restrict__ y, int M, int N, int K,
+                                                             int k_slice, int m_tiles, int n_tiles, int splits, Gate gate) {
+    constexpr int kRowBytes = kTileK * 4, kHalf = kTileEdge * kRowBytes, kStage = 2 * kHalf, kLoads = 4;  // a stage: W, then X
+    extern __shared__ char lds[];
+    // a die (the workgroup's number modulo 8) takes neighbouring tiles: of W its own eighth, of X all
+    const int tiles = m_tiles * n_tiles * splits, a_die = (tiles + 7) / 8;
+    const int id = static_cast<int>(blockIdx.x & 7) * a_die + static_cast<int>(blockIdx.x >> 3);
+    if (id >= tiles) return;
+    const int m_tile = id % m_tiles, n_tile = id / m_tiles % n_tiles, slice = id / m_tiles / n_tiles;
+    const int m0 = m_tile * kTileEdge, n0 = n_tile * kTileEdge;
+    const int first_step = slice * k_slice / kTileK, steps = min(K - slice * k_slice, k_slice) / kTileK;
+    const int lane = threadIdx.x & (FSIE_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / FSIE_WAVE);
+    const int row = lane & 15, kg = lane >> 4;
+    const int nw = (wave & 1) * 32, mw = (wave >> 1) * 32;
+
+    // a wave's loads of a stage: 16 rows of W and of X, eight a load; a row's eight 16-byte units lie permuted by the row
+    const u32x4 w_rows = fsie_lds::rows_from(w, static_cast<uint32_t>(N) * static_cast<uint32_t>(K) * 4u);
+    const u32x4 x_rows = fsie_lds::rows_from(x, static_cast<uint32_t>(M) * static_cast<uint32_t>(K) * 4u);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds);
+    uint32_t from[4];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int m = m0 + mw + 16 * t + row;
-        if (m >= M) continue;
-        float* to = RESULT == GATED ? y + static_cast<int64_t>(m) * (N / 2)
-                                    : y + ((RESULT == SUMS ? static_cast<int64_t>(blockIdx.z) * M : 0) + m) * N;
+    for (int i = 0; i < 2; ++i) {  // rows past the end repeat the last one and are never written
+        const int r = (wave * 2 + i) * 8 + (lane >> 3);
+        const uint32_t unit = ((lane & 7) ^ (r >> 1 & 7)) * 16u;
+        from[i] = static_cast<uint32_t>(min(n0 + r, N - 1)) * static_cast<uint32_t>(K) * 4u + unit;
+        from[2 + i] = static_cast<uint32_t>(min(m0 + r, M - 1)) * static_cast<uint32_t>(K) * 4u + unit;
+    }
+    uint32_t bring_to = 0, read_from = 0;  // the stages' places, in turn
+    const auto next_stage = [](uint32_t at) { return at == (STAGES - 1) * kStage ? 0u : at + kStage; };
+    const auto k_of = [&](int step) { return static_cast<uint32_t>(first_step + min(step, steps - 1)) * kRowBytes; };
+    const auto load = [&](int i, uint32_t k) {
+        fsie_lds::load_to_lds(i < 2 ? w_rows : x_rows, lds0 + bring_to + (i >> 1) * kHalf + (wave * 2 + (i & 1)) * 1024u, from[i], k);
+    };
+    floatx4 acc[2][2], total[2][2];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int n = n0 + nw + 16 * j + 4 * kg;
-            const floatx4 v = acc[j][t] + total[j][t];
-            if constexpr (RESULT == GATED) {
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int i = 0; i < 4; i += 2)
-                    if (n + i < N) to[(n + i) / 2] = gate_pair(v[i], v[i + 1], gate.act, gate.limit, gate.slope);
-            } else {
+        for (int t = 0; t < 2; ++t) acc[j][t] = total[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    floatx4 f[2][4][2];  // this step's fragments and the next one's: [W 0, 1, X 0, 1][half of the step]
+    const auto read = [&](int i, floatx4 (&to)[4][2]) {  // the i-th of a stage's eight
+        const int h = i >> 2, at = i & 3;
+        const int r = (at < 2 ? nw : mw) + (at & 1) * 16 + row;
+        to[at][h] = *reinterpret_cast<const floatx4*>(lds + read_from + (at >> 1) * kHalf + r * kRowBytes + (((4 * h + kg) ^ (row >> 1 & 7)) * 16));
+    };
+    const auto go = [&](int step, const floatx4 (&now)[4][2], floatx4 (&next)[4][2]) {
+        // the next stage has arrived, and this step's fragments are in every wave's registers: its stage is free
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 2) * kLoads) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t k = k_of(step + STAGES);
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (n + i < N) to[n + i] = RESULT == PLAIN && bias ? v[i] + bias[n + i] : v[i];
-            }
+        for (int c = 0; c < 4; ++c) {
+#pragma unroll
+            for (int q = 2 * c; q < 2 * c + 2; ++q)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+                        acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(now[j][q >> 2][q & 3], now[2 + t][q >> 2][q & 3], acc[j][t], 0, 0, 0);
+            read(2 * c, next);
+            read(2 * c + 1, next);
+            load(c, k);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        bring_to = next_stage(bring_to);
+        read_from = next_stage(read_from);
+    };
+#pragma unroll
+    for (int i = 0; i < STAGES; ++i) {
+        const uint32_t k = k_of(i);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) load(c, k);
+        bring_to = next_stage(bring_to);
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * kLoads) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) read(i, f[0]);
+    read_from = next_stage(read_from);
+    constexpr int kRun = kTileFlush / kTileK;
+    for (int step = 0; step < steps; step += 2) {
+        go(step, f[0], f[1]);
+        if (step + 1 < steps) go(step + 1, f[1], f[0]);
+        if ((step + 2) % kRun == 0) {  // (kRun is even; the last run is short of a step where there is an odd number: added below all the same)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    total[j][t] += acc[j][t];
+                    acc[j][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+                }
         }
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (no load may still write LDS when the workgroup's is given away)
+    write_tile<RESULT>(acc, total, y, bias, gate, M, N, m0 + mw + row, n0 + nw + 4 * kg, slice);
+}
+
+struct TileCall {
+    const float *x, *w, *bias;
+    float* y;
+    Gate gate;
+    int M, N, K, slice, m_tiles, n_tiles, splits;
+    hipStream_t stream;
+};
+
+template <int RESULT, int STAGES>
+int launch_block(const TileCall& c) {
+    constexpr int kLds = STAGES * 2 * kTileEdge * kTileK * 4;
+    static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_fp32_block_kernel<RESULT, STAGES>),
+                                                          hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+    FSIE_REQUIRE(allowed == hipSuccess, "gemm_fp32_tile: %d bytes of LDS: %s", kLds, hipGetErrorString(allowed));
+    const unsigned groups = static_cast<unsigned>((static_cast<int64_t>(c.m_tiles) * c.n_tiles * c.splits + 7) / 8 * 8);
+    gemm_fp32_block_kernel<RESULT, STAGES><<<groups, 256, kLds, c.stream>>>(c.x, c.w, c.bias, c.y, c.M, c.N, c.K, c.slice, c.m_tiles, c.n_tiles, c.splits, c.gate);
+    FSIE_CHECK_LAUNCH("gemm_fp32_tile");
+    return 0;
 }
 
 }  // namespace
@@ -266,13 +399,23 @@ static int tile_product(const float* x, const float* w, const float* bias, float
     int64_t slice = ceil_div64(ceil_div64(K, splits), kTileFlush) * kTileFlush;
     if (slice * (splits - 1) >= K) slice = ceil_div64(ceil_div64(K, splits), kTileK) * kTileK;
     FSIE_REQUIRE(splits == 1 || slice * (splits - 1) < K, "gemm_fp32_tile: K=%d does not give %d slices", K, splits);
+    const int64_t tiles_n = ceil_div64(N, kTileEdge), groups = tiles_m * tiles_n * splits;
+    if (splits == 1) slice = ceil_div64(K, kTileK) * kTileK;
+    if (K % kTileK == 0 && static_cast<int64_t>(M) * K * 4 < (int64_t{1} << 31) && static_cast<int64_t>(N) * K * 4 < (int64_t{1} << 31) &&
+        groups < (int64_t{1} << 30)) {
+        const TileCall c{x, w, bias, y, gate ? *gate : Gate{}, M, N, K, static_cast<int>(slice), static_cast<int>(tiles_m), static_cast<int>(tiles_n), splits, stream};
+        const bool few = groups <= kFewTiles;
+        if (splits > 1) return few ? launch_block<SUMS, 6>(c) : launch_block<SUMS, 3>(c);
+        if (gate) return few ? launch_block<GATED, 6>(c) : launch_block<GATED, 3>(c);
+        return few ? launch_block<PLAIN, 6>(c) : launch_block<PLAIN, 3>(c);
+    }
     const dim3 grid(static_cast<unsigned>((N + kTileEdge - 1) / kTileEdge), static_cast<unsigned>(tiles_m), static_cast<unsigned>(splits));
     if (splits > 1)
         gemm_fp32_tile_kernel<SUMS><<<grid, 256, 0, stream>>>(x, w, nullptr, y, M, N, K, static_cast<int>(slice), Gate{});
     else if (gate)
-        gemm_fp32_tile_kernel<GATED><<<grid, 256, 0, stream>>>(x, w, nullptr, y, M, N, K, static_cast<int>(ceil_div64(K, kTileK) * kTileK), *gate);
+        gemm_fp32_tile_kernel<GATED><<<grid, 256, 0, stream>>>(x, w, nullptr, y, M, N, K, static_cast<int>(slice), *gate);
     else
-        gemm_fp32_tile_kernel<PLAIN><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K, static_cast<int>(ceil_div64(K, kTileK) * kTileK), Gate{});
+        gemm_fp32_tile_kernel<PLAIN><<<grid, 256, 0, stream>>>(x, w, bias, y, M, N, K, static_cast<int>(slice), Gate{});
     FSIE_CHECK_LAUNCH("gemm_fp32_tile");
     return 0;
 }

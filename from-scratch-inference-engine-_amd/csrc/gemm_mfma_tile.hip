@@ -22,12 +22,14 @@
 // of 32 x 32 x 16, faster by itself, reads the same bytes in a worse pattern: 1,150.
 #include "common.h"
 #include "api.h"
+#include "lds_loads.h"
 
 namespace {
 
+using namespace fsie_lds;
+
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kStep = 64;  // values of K a stage
 constexpr int kRowBytes = kStep * 2;
@@ -47,27 +49,7 @@ struct Shape {
 
 enum Result { kPair = 1, kSums = 2 };
 
-// 16 bytes a lane from memory to LDS, lane i's at lds + 16 i.  The instruction takes the LDS address from m0, which is an
-// operand here and written by the compiler; the wait state between that and the load is not, inside an asm statement.
-__device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t lds, uint32_t offset, uint32_t k_offset) {
-    asm volatile(
-        "s_nop 0\n\t"
-        "buffer_load_dwordx4 %1, %2, %3 offen lds"
-        :
-        : "{m0}"(lds), "v"(offset), "s"(rsrc), "s"(k_offset)
-        : "memory");
-}
 #define FSIE_TILE_FENCE() __builtin_amdgcn_sched_barrier(0)
-
-__device__ __forceinline__ u32x4 rows_from(const bf16_t* base, uint32_t bytes) {
-    const uint64_t at = reinterpret_cast<uint64_t>(base);
-    u32x4 r;
-    r[0] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at));
-    r[1] = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at >> 32));
-    r[2] = __builtin_amdgcn_readfirstlane(bytes);
-    r[3] = 0x00020000u;
-    return r;
-}
 
 // The permutation of a row's 16-byte units.  W's rows are read 16 at a time as 4 runs of 4 that lie 16 apart (see the
 // fragments below), X's as 16 neighbours: in both any eight lanes in a row see eight values.

@@ -30,6 +30,23 @@ def test_against_64_bits(m, n, k):
         assert got.shape == (slices, m, n) and ((got.double().sum(0) - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("k", [32, 64, 224, 256, 288, 1088])
+@pytest.mark.parametrize("m,n", [(65, 48), (300, 130), (700, 1664)])  # few workgroups and more than 256 of them
+def test_whole_steps_have_the_bits_of_the_others(m, n, k):
+    """K of whole steps goes straight to LDS, four more columns of zeros take the kernel whose loads go through registers: the same sums in the same order."""
+    ops.load(build_if_missing=False)
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn((m, k), generator=g).cuda(), torch.randn((n, k), generator=g).cuda()
+    bias = torch.randn((n,), generator=g).cuda()
+    more = [torch.nn.functional.pad(a, (0, 4)) for a in (x, w)]
+    assert torch.equal(ops.gemm_fp32_tile(x, w), ops.gemm_fp32_tile(*more))
+    assert torch.equal(ops.gemm_fp32_tile(x, w, bias), ops.gemm_fp32_tile(*more, bias))
+    assert torch.equal(ops.gemm_fp32_gated(x, w, "silu"), ops.gemm_fp32_gated(*more, "silu"))
+    if k == 1088:  # (slices of 512 and 768 values, with the four zeros as without)
+        for slices in (3, 2):
+            assert torch.equal(ops.gemm_fp32_tile(x, w, splits=slices), ops.gemm_fp32_tile(*more, splits=slices))
+
+
 def test_slices_are_ones_the_kernel_takes():
     ops.load(build_if_missing=False)
     for m in (65, 200, 682, 2048):
