@@ -24,7 +24,8 @@ class Linear:
     (``for_residual``: 17 to 64 rows, and any number where K is long) and for the partial sums of
     other projections of 17 to 64 rows (``partial_sums``); a third for up to 16 rows and a K so short that all of it is under
     way at once (``ops.gemm_stream_plan``); residual projections of more than 128 rows whose K is 16,384
-    and more the engine's kernel for many rows, in slices of K (``ops.gemm_tile_plan``); everything else
+    and more the engine's kernel for many rows, in slices of K (``ops.gemm_tile_plan``); products of 65 rows
+    and more of matrices of some ten MB the one in small tiles (``ops.gemm_block_plan``); everything else
     the library product (hipBLASLt through torch, where the reference's engine calls cuBLAS) with
     float32 accumulation, the bias added by a kernel of the engine.  A large weight has a second copy in
     the order of the matrix instruction's fragments (``prepare``, ``streamed``), from which the
@@ -182,7 +183,7 @@ class Linear:
 
     def _many_rows(self, x: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
         plan = self._many_plan(x.shape[0], ops.GEMM_BLOCK_PLAIN)
-        if plan is not None and self.kernel_reads(x):
+        if plan is not None and self.kernel_reads(x) and (bias is None or bias.data_ptr() % 16 == 0):
             return ops.gemm_mfma_block(x, self._weight, ops.GEMM_BLOCK_PLAIN, plan[0], bias=bias)
         y = library_mm(x, self._weight)
         if bias is not None:

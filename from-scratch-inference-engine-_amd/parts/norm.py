@@ -68,7 +68,8 @@ class RMSNorm(Norm):
 
     def can_wait(self, hidden: HiddenState, out_dtype: torch.dtype) -> bool:
         delta = hidden.delta
-        return (type(self) is RMSNorm and out_dtype == torch.bfloat16 and hidden.delta_norm is None and hidden.delta_bias is None
+        return (type(self) is RMSNorm and out_dtype == torch.bfloat16 and self.weight.data_ptr() % 16 == 0
+                and hidden.delta_norm is None and hidden.delta_bias is None
                 and hidden.delta2 is None and hidden.delta_scale == 1.0
                 and (delta is None or (delta.ndim == 3 and delta.dtype == torch.float32)))
 

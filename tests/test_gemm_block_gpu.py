@@ -65,3 +65,6 @@ def test_linear_takes_them(ops, m, n, k, monkeypatch):
     odd = wide[:, 4:]
     odd.copy_(x)
     assert ((layer(odd).double() - exact).abs() <= 2.0 ** -7 * size).all() and not seen
+    layer.bias = torch.zeros(n + 1, device="cuda")[1:].copy_(torch.randn(n, generator=gen))  # (four bytes off the 16 that the kernel loads)
+    layer.has_bias = True
+    assert ((layer(x).double() - exact - layer.bias.double()).abs() <= 2.0 ** -7 * (size + layer.bias.double().abs())).all() and not seen
