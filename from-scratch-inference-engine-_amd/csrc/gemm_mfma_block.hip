@@ -241,9 +241,10 @@ int launch_shape(int tile, const Call& c) {
 // the kernel's.  Returns tile + 256 * slices.
 // The rule is the time that a count of steps gives: fixed + steps * a step's, workgroups that share a unit taking turns (so many as the unit's LDS
 // holds; a second round of 128 x 128 was up to 1.36 of the library's time and is not taken), the weights from HBM at 6.7 to 9 TB/s more; a whole product's
-// bytes or the slices' sums here and in the norm at 3 TB/s.  It has to be 0.95 of the library's 8.9 us, 1.25 PFLOP/s and weights at 3.3 TB/s, as it takes them
-// from HBM at 24 matrices of 1 to 50 MB and 19 numbers of rows from 70 to 4,096.  Of these 456 and as many with slices and the norm the rule takes 426, at a
-// median of 0.75 of the library's time, the largest 1.02 but for 129 rows of N = 8192, K = 2048 (1.13; this / the library, us: 1,375 rows of N = 1152,
+// bytes or the slices' sums here and in the norm at 3 TB/s.  It has to be no more than the library's 8.3 us, 1.64 PFLOP/s, weights at 3 TB/s and x at 2.2, the
+// best fit of what it took with weights from HBM at 24 matrices of 1 to 50 MB and 19 numbers of rows from 70 to 4,096 (slices: 0.95 of that and the norm's
+// reading).  Of these 456 and as many with slices and the norm the rule takes 463, at a median of 0.76 of the library's time and at most 1.02 but for 129
+// rows of N = 8192, K = 2048 (1.12; this / the library, us: 1,375 rows of N = 1152,
 // K = 896 7.5 / 11.3, 512 of N = 4608, K = 3584 28.9 / 33.3, 1,000 of N = K = 3584 30.4 / 36.9, 2,048 of N = 2048, K = 8192 67.7 / 75.5, 256 of N = 3072, K = 1024 6.9 / 11.9; with
 // the norm, 96 rows of N = 896, K = 4864 in six slices 9.4 / 15.7, 96 of N = 2048, K = 8192 in four 15.3 / 24.0).
 extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int units) {
@@ -270,7 +271,8 @@ extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int un
             }
         }
     }
-    return choice >= 0 && best <= 0.95 * (8.9 + flops / 1.25e9 + weights / 3.3e6 + (result == kSums ? whole : 0.0)) ? choice : -1;
+    const double library = 8.3 + flops / 1.64e9 + weights / 3e6 + 2.0 * M * static_cast<double>(K) / 2.2e6;
+    return choice >= 0 && best <= (result == kSums ? 0.95 * (library + whole) : library) ? choice : -1;
 }
 
 extern "C" int fsie_gemm_mfma_block(const void* x, const void* w, const float* bias, void* y, int M, int N, int K, int result, int splits,
