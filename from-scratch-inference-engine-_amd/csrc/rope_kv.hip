@@ -133,6 +133,12 @@ struct Quad<bf16_t> {
     }
 };
 
+// A pair turned by (c, s): a1 c - a2 s and a2 c + a1 s, each with one product rounded and the other added to it exactly.  Written out,
+// since which product the compiler rounds follows from how it places registers: it differed between this kernel's variants,
+// from pair to pair, and from one change of the source to the next.
+__device__ __forceinline__ float turned_first(float a1, float a2, float c, float s) { return __builtin_fmaf(a1, c, -(a2 * s)); }
+__device__ __forceinline__ float turned_second(float a1, float a2, float c, float s) { return __builtin_fmaf(a1, s, a2 * c); }
+
 // The same work with the cosines and sines read from the step's table [T][head_dim / 2][2] and four
 // pairs a thread: no trigonometry, 8- and 16-byte accesses.  The whole head is rotated; head_dim is
 // a multiple of 8.  A block takes TOK consecutive tokens: 1, or 8 for long batches (prompt portions).
@@ -162,8 +168,7 @@ __global__ __launch_bounds__(kThreads) void rope_kv_write_table_kernel(
         slot[j] = (write_kv && j < n_here) ? slots[t0 + j] : -1;
         if (slot[j] >= pool_slots) slot[j] = -1;
     }
-    // the blocks of a token (gridDim.y of them; more than one only where the partial sums make a token
-    // heavy) share its columns
+    // the blocks of a token or of a run of eight (gridDim.y of them) share its columns
     const int first = threadIdx.x + blockIdx.y * kThreads;
     const int stride = kThreads * gridDim.y;
     // four consecutive columns of token t
@@ -212,10 +217,10 @@ __global__ __launch_bounds__(kThreads) void rope_kv_write_table_kernel(
             const float4* cs = reinterpret_cast<const float4*>(cos_sin + static_cast<int64_t>(t) * head_dim);
             c01 = cs[i / 2], c23 = cs[i / 2 + 1];
         }
-        const float4 r1{a1.x * c01.x - a2.x * c01.y, a1.y * c01.z - a2.y * c01.w, a1.z * c23.x - a2.z * c23.y,
-                        a1.w * c23.z - a2.w * c23.w};
-        const float4 r2{a2.x * c01.x + a1.x * c01.y, a2.y * c01.z + a1.y * c01.w, a2.z * c23.x + a1.z * c23.y,
-                        a2.w * c23.z + a1.w * c23.w};
+        const float4 r1{turned_first(a1.x, a2.x, c01.x, c01.y), turned_first(a1.y, a2.y, c01.z, c01.w),
+                        turned_first(a1.z, a2.z, c23.x, c23.y), turned_first(a1.w, a2.w, c23.z, c23.w)};
+        const float4 r2{turned_second(a1.x, a2.x, c01.x, c01.y), turned_second(a1.y, a2.y, c01.z, c01.w),
+                        turned_second(a1.z, a2.z, c23.x, c23.y), turned_second(a1.w, a2.w, c23.z, c23.w)};
         if (!PARTS || h < n_heads) {
             Quad<T>::store(head + i, r1);
             Quad<T>::store(head + i + half, r2);

@@ -135,6 +135,30 @@ def test_rope_and_cache_write(ops, dtype, from_table, heads, kv, hd, theta):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("t", [5, 1027])  # a token a block; eight
+def test_a_turned_pair_rounds_the_same_way_in_every_form(ops, dtype, t):
+    """a1 c - (a2 s) and a1 s + (a2 c), the product in brackets rounded and the other added to it exactly: with and without a bias,
+    from the projection or from partial sums, a token or eight of them a block.  (In float64 the exact product and the sum
+    lose at most 2^-53 of it, which the rounding to float32 does not see.)"""
+    heads, kv, hd = 5, 2, 64
+    g = torch.Generator().manual_seed(t)
+    qkv, bias = torch.randn(t, (heads + 2 * kv) * hd, generator=g).to(dtype), torch.randn((heads + 2 * kv) * hd, generator=g)
+    table = ops.rope_table(torch.randint(0, 9000, (t,), generator=g, dtype=torch.int32).cuda(),
+                           torch.tensor([1e4 ** (-2.0 * i / hd) for i in range(hd // 2)], dtype=torch.float64).cuda())
+    c, s = table.cpu().reshape(t, 1, hd // 2, 2).unbind(-1)
+    for add in (None, bias):
+        a = (qkv.float() if add is None else qkv.float() + add)[:, :heads * hd].reshape(t, heads, 2, hd // 2)
+        a1, a2 = a[:, :, 0], a[:, :, 1]
+        first = (a1.double() * c.double() - (a2 * s).double()).float()
+        second = (a1.double() * s.double() + (a2 * c).double()).float()
+        want = torch.stack([first, second], 2).reshape(t, heads * hd).to(dtype)
+        for parts in (None, qkv.float()[None].cuda()):
+            got = ops.rope_kv_write(qkv.clone().cuda(), torch.zeros(t, dtype=torch.int32).cuda(), heads, kv, hd, None,
+                                    bias=None if add is None else add.cuda(), cos_sin=table, parts=parts, by_rows=True)
+            assert torch.equal(got.cpu()[:, :heads * hd], want), (add is None, parts is None)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("page", [16, 8, 4])
 def test_rope_from_table_on_a_long_batch(ops, dtype, page):
     """From 1,024 tokens on a block takes eight tokens and writes the values of eight consecutive
