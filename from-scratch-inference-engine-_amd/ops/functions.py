@@ -633,13 +633,14 @@ def gemm_mfma_wide_splits_ok(k: int, splits: int) -> bool:
 
 
 def gemm_mfma_wide_swiglu(x: torch.Tensor, weight: torch.Tensor, waves: int = 0, blocks: int = 0,
-                          out: Optional[torch.Tensor] = None, act="silu", few_rows: bool = False) -> torch.Tensor:
+                          out: Optional[torch.Tensor] = None, act="silu", few_rows: bool = False, norm: Optional[tuple] = None) -> torch.Tensor:
     """silu(gate) * up, or what ``act`` (a ``GateAct`` or its name) makes of them, [M, N/2] (bfloat16) of x [M, K] and a weight [N, K] whose rows are gate and up
     in turn (or its ``FragmentOrdered`` copy), by the kernel that shares x through LDS; up to 64
     rows, N a multiple of 4, K of 128.  ``few_rows``: up to 16 rows go to ``gemm_mfma_stream`` where that is faster (the same
-    sums in another order).  ``x`` may be a norm that waits for its product (``parts.base.PendingNorm``): ``gemm_mfma_normed``."""
-    if not isinstance(x, torch.Tensor):
-        return gemm_mfma_normed(x.residual, x.sums, x.weight, x.eps, x.stream, weight, GEMM_STREAM_GATED, act)
+    sums in another order).  ``norm`` = (sums, norm weight, eps, new stream): ``x`` is the float32 stream, and the product makes its norm
+    (``gemm_mfma_normed``)."""
+    if norm is not None:
+        return gemm_mfma_normed(x, *norm, weight, GEMM_STREAM_GATED, act)
     _need(x, "gemm x", dtype=torch.bfloat16, ndim=2)
     m, k = x.shape
     wptr, n, frags = _wide_weight(weight, k)

@@ -73,7 +73,7 @@ class SwiGLU(FeedForward):
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         m = x.shape[0]
         if isinstance(x, PendingNorm):
-            act = ops.gemm_mfma_wide_swiglu(x, self.gate_up.streamed, act=self._gate_act)
+            act = ops.gemm_mfma_wide_swiglu(x.residual, self.gate_up.streamed, act=self._gate_act, norm=(x.sums, x.weight, x.eps, x.stream))
         elif (x.dtype == torch.bfloat16 and self.gate_up.copy_for(m) is not None and 0 < m <= self.streamed_swiglu_max_rows
                 and self.gate_up.wide_takes(m, 1, gate_up=True)):
             # from the fragment-ordered copy at any number of rows up to 64, and up to 128 where the
