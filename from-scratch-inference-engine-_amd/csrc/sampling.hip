@@ -1032,7 +1032,13 @@ __global__ __launch_bounds__(kPart) void split_list_kernel(const float* __restri
     const int first = (first_run + wave * runs) * lines * FSIE_WAVE + lane;
     const float reach = bins.reach(max(k_bin, upto), mx);
     int run = wave * runs, in_run = 0, n = 0;
+    // (a wave's tokens change lanes here: what the others wrote is read below, and is read before the next ones are written over it)
+    const auto meet = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
     const auto settle = [&]() {
+        meet();
         for (int at = lane; at < n; at += FSIE_WAVE) {
             const float v = near[wave][at];
             const unsigned int place = near_at[wave][at];
@@ -1049,6 +1055,7 @@ __global__ __launch_bounds__(kPart) void split_list_kernel(const float* __restri
                 if (m.lo) atomicAdd(&run_lo[place >> 23], m.lo);
             }
         }
+        meet();
         n = 0;
     };
     const auto bring = [&](float (&v)[kAhead], int j0) {
