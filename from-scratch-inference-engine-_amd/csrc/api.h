@@ -358,7 +358,8 @@ int fsie_attention_split_static(const void* q, int64_t q_stride, const void* k_p
 int fsie_sample(const float* logits, int n_rows, int vocab, const float* temperature, const int32_t* top_k,
                 const float* top_p, const double* uniform, int32_t* out, hipStream_t stream);
 // The same at temperatures with every row shared by several workgroups, where fsie_sample_workspace says so:
-// `workspace` = fsie_sample_workspace(n_rows, vocab, whether top_k or top_p are given) bytes on the device (0: the call is fsie_sample's), uninitialised.
+// `workspace` = fsie_sample_workspace(n_rows, vocab, whether top_k or top_p are given) bytes on the device (0: the call is fsie_sample's), uninitialised;
+// a row's share begins with the number of tokens that its list got (int32; more than 4,096, or none where thresholds are given: the row was settled by one workgroup).
 // `on_host`: the four arrays are in host memory, of up to fsie_sample_by_value() rows; they are read before the call returns.
 int64_t fsie_sample_workspace(int n_rows, int vocab, int thresholds);
 int fsie_sample_split(const float* logits, int n_rows, int vocab, const float* temperature, const int32_t* top_k,

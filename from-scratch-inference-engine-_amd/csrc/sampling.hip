@@ -579,12 +579,12 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
 // for rows without a threshold, the draw's sums); the tokens about the thresholds, side by side, and the draw's sums of
 // those that are kept for certain; the cut among the listed tokens and the draw.  What a launch leaves for the next lies in
 // a workspace of the row.
-// Alone / shared, us, a fifth of the rows each greedy, plain, top k, top p and both, at 8, 64, 128, 256, 512 and 2,048 rows:
-//    16,384 tokens   34 / 24    35 / 26    35 / 28     36 /  33     66 /  48    206 / 134
-//    32,000          43 / 25    45 / 27    46 / 32     48 /  44     88 /  67    262 / 185
-//    65,536          68 / 25    70 / 32    70 / 42     74 /  61    139 / 102    420 / 343
-//   152,064         130 / 26   141 / 45   145 / 69    155 / 113    289 / 203    847 / 708
-// so where thresholds are given rows are shared up to kMostRows of them (what was measured, twice; their workspaces are 41 KB a row).  Without
+// Alone / shared, us, a fifth of the rows each greedy, plain, top k, top p and both, at 8, 64, 128, 256, 512, 2,048 and 4,096 rows:
+//    16,384 tokens   37 / 23    37 / 27    38 / 29     39 /  34     71 /  51    215 / 134    405 /   243
+//    32,000          46 / 23    48 / 28    48 / 33     51 /  45     96 /  71    269 / 188    516 /   419
+//    65,536          71 / 24    71 / 33    74 / 43     77 /  63    147 / 107    432 / 368    794 /   692
+//   152,064         138 / 25   150 / 46   152 / 70    158 / 116    303 / 211    870 / 759  1,640 / 1,424
+// so where thresholds are given rows are shared up to kMostRows of them (what was measured; their workspaces are 59 KB a row).  Without
 // thresholds it is three launches beside one of two passes, and the line is kMostPlainRows (8, 64, 128, 256, 380 rows of 16,384:
 // 17 / 11, 17 / 13, 17 / 15, 18 / 20, 34 / 26; of 152,064: 42 / 12, 48 / 27, 51 / 43, 61 / 73, 105 / 103).
 // (Without temperatures it is one pass over the row, and a workgroup a row is the faster one; with temperatures that all
@@ -593,7 +593,10 @@ constexpr int kSplitFrom = 16384;
 constexpr int kMostRows = 4096, kMostPlainRows = 160;
 constexpr int kPart = 512;          // threads of a shared row's workgroups
 constexpr int kMaxParts = 32;
-constexpr int kCoarse = 512;        // bins of a shared row
+// Bins of a shared row.  512 are a per cent faster where the thresholds lie among few tokens (64 rows of 152,064 as above 44.7 us, 45.1 with 2,048), but
+// lists then overflow, and one workgroup settles the row, where a threshold lies in a bulk of tokens far below the maximum (64 rows, normal of a
+// width of 0.35, 25 below it: top k of 20,000 230 us, 52 so; top p at a temperature of 4 596 and 84; both 672 and 64).
+constexpr int kCoarse = 2048;
 constexpr int kFine = 1024;         // what the bin of a threshold is cut into
 constexpr int kPairs = 512;         // so many tokens of a fine bin are compared with each other, more are bisected
 constexpr int kKeep = 4096;         // tokens that the list holds
@@ -601,9 +604,9 @@ constexpr int kAllListed = 1024;    // up to this top k the list takes every tok
 static_assert(kRuns / kMaxParts >= kPart / FSIE_WAVE, "every wave of a part has a run");
 
 struct SplitRow {
+    unsigned int n_listed, pad;       // (in front of the bins: cleared with them)
     unsigned long long sum[kCoarse];  // weights, in units of their bin's own (RowBins)
     unsigned int count[kCoarse];
-    unsigned int n_listed, pad;       // (behind the bins: cleared with them)
     double uniform;                   // the row's parameters, as the first launch brings them
     float temperature, top_p;
     int top_k;
@@ -799,7 +802,7 @@ __global__ __launch_bounds__(kPart) void split_top_kernel(const float* __restric
     const int part = blockIdx.x, lane = threadIdx.x & (FSIE_WAVE - 1), wave = threadIdx.x / FSIE_WAVE;
     if (part == 0 && threadIdx.x == 0) rows.to(w, static_cast<int>(blockIdx.y));
     // the row's bins and counter are this launch's to clear
-    uint32_t* bins = reinterpret_cast<uint32_t*>(w->sum);
+    uint32_t* bins = reinterpret_cast<uint32_t*>(w);
     constexpr int kClear = static_cast<int>(offsetof(SplitRow, uniform) / 4);
     for (int i = part * kPart + threadIdx.x; i < kClear; i += parts * kPart) bins[i] = 0;
     int begin, end;
@@ -1117,7 +1120,7 @@ struct Cutting {
     double wave_sum[kWaves];
     Found found;
 };
-static_assert(kFine == kThreads && kCoarse <= kThreads, "a bin a thread");
+static_assert(kFine == kThreads, "a bin a thread");
 
 constexpr unsigned int kFew = 64;
 // The key of the first token of bin `bin`, from the largest down, at which above + amount(sum of its and all larger
@@ -1208,6 +1211,7 @@ __device__ uint32_t cut_of_list(Cutting& s, const SplitRow* w, const RowParams& 
     bool in[kHeld];
     unsigned long long value[kHeld];
     const int k_bin = w->k_bin;
+    const bool all_listed = q.all_listed();
     Found at{w->from, w->above};
     double target = w->target;
 #pragma unroll
@@ -1228,14 +1232,18 @@ __device__ uint32_t cut_of_list(Cutting& s, const SplitRow* w, const RowParams& 
     for (int j = 0; j < kHeld; ++j) value[j] = bin[j] >= 0 ? bins.weight(expf((v[j] - mx) * q.inv_temp), bin[j]) : 0;
     if (q.k > 0) {
         // the weights of what top k keeps: of its own bin from the list, of those above from the list or the row's bins
-        const int b = static_cast<int>(threadIdx.x);
+        using Scan = BinScan<kThreads>;
+        const int b0 = static_cast<int>(threadIdx.x) * Scan::PER;
 #pragma unroll
         for (int j = 0; j < kHeld; ++j)
-            if (bin[j] >= 0 && order_key(v[j]) >= cut && (bin[j] == k_bin || q.all_listed())) atomicAdd(&s.coarse[bin[j]], value[j]);
-        const unsigned long long others = !q.all_listed() && b < k_bin ? w->sum[b] : 0;
+            if (bin[j] >= 0 && order_key(v[j]) >= cut && (bin[j] == k_bin || all_listed)) atomicAdd(&s.coarse[bin[j]], value[j]);
+        unsigned long long others[Scan::PER];
+#pragma unroll
+        for (int i = 0; i < Scan::PER; ++i) others[i] = !all_listed && b0 + i < k_bin ? w->sum[b0 + i] : 0;
         __syncthreads();
-        BinScan<kThreads> scan;
-        scan.v[0] = b < kCoarse ? bins.value(s.coarse[b] + others, b) : 0.0;
+        Scan scan;
+#pragma unroll
+        for (int i = 0; i < Scan::PER; ++i) scan.v[i] = b0 + i < kCoarse ? bins.value(s.coarse[b0 + i] + others[i], b0 + i) : 0.0;
         scan.run(s.wave_sum);
         target = static_cast<double>(q.p) * scan.total;
         at = scan.find(target, &s.found);
@@ -1284,7 +1292,7 @@ __global__ __launch_bounds__(kThreads) void split_draw_kernel(const float* __res
         }
         s.list.search[0].clear();
         s.list.search[1].clear();
-        if (threadIdx.x < kCoarse) s.list.coarse[threadIdx.x] = 0;
+        for (int b = threadIdx.x; b < kCoarse; b += kThreads) s.list.coarse[b] = 0;
         if (threadIdx.x < kRuns) s.list.run_hi[threadIdx.x] = s.list.run_lo[threadIdx.x] = 0;
         if (threadIdx.x == 0) s.list.found.bin = -1;
         __syncthreads();

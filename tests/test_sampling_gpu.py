@@ -160,3 +160,36 @@ def test_shared_rows_choose_what_rows_alone_do(kind, rows, vocab):
         assert torch.equal(ops.sample(x, *[v.cpu().numpy() for v in (t, k, p, u)]), shared)
     assert size > 0 and ((alone >= 0) & (alone < vocab)).all()
     assert torch.equal(alone, shared)
+
+
+# temperature, top k, top p, and the width of a bulk of tokens far below the maximum (0: none)
+BULKS = [(1.0, 20000, 1.0, 0.35), (4.0, 0, 0.9, 0.35), (1.0, 20000, 0.9, 0.5), (4.0, 0, 0.6, 0.2), (1.0, 20000, 1.0, 0.2), (1.0, 20000, 0.9, 1.0)]
+
+
+@pytest.mark.parametrize("cases, vocab", [(BULKS, 152064)], ids=["bulks"])
+def test_lists_settle_cold_rows_and_thresholds_in_a_bulk(cases, vocab):
+    """Rows whose threshold lies where most tokens are choose what they choose alone, and from their lists: not by the slow way that a row takes which its list does not settle (the tokens that a row's list got are the first
+    number of its workspace; an empty or a full list settles nothing)."""
+    from from_scratch_inference_engine_amd import ops
+    from from_scratch_inference_engine_amd.ops.functions import _stream, check
+
+    lib, rows = ops.load(build_if_missing=False), 2 * len(cases)
+    g = torch.Generator().manual_seed(vocab)
+    x = torch.randn((rows, vocab), generator=g) * 2.5
+    for r in range(rows):
+        if cases[r % len(cases)][3]:
+            x[r] = torch.randn(vocab, generator=g) * cases[r % len(cases)][3]
+            x[r, 77], x[r, 5] = 25.0, 20.0
+    x = x.cuda()
+    t, k, p, _ = zip(*[cases[i % len(cases)] for i in range(rows)])
+    dev = lambda v, dt: torch.tensor(v, dtype=dt).cuda()
+    t, k, p, u = dev(t, torch.float32), dev(k, torch.int32), dev(p, torch.float32), torch.linspace(0.001, 0.999, rows, dtype=torch.float64).cuda()
+    size = lib.fsie_sample_workspace(rows, vocab, 1)
+    work = torch.full((size,), 255, dtype=torch.uint8).cuda()
+    alone, shared = torch.full((rows,), -1, dtype=torch.int32).cuda(), torch.full((rows,), -1, dtype=torch.int32).cuda()
+    args = (x.data_ptr(), rows, vocab, t.data_ptr(), k.data_ptr(), p.data_ptr(), u.data_ptr())
+    check(lib.fsie_sample(*args, alone.data_ptr(), _stream()))
+    check(lib.fsie_sample_split(*args, 0, work.data_ptr(), shared.data_ptr(), _stream()))
+    assert torch.equal(alone, shared)
+    listed = work.view(rows, -1)[:, :4].contiguous().view(torch.int32).flatten().tolist()
+    assert all(0 < n <= 4096 for n in listed), listed
