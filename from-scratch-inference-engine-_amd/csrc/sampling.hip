@@ -626,7 +626,6 @@ struct RowParams {
     float temp, inv_temp, p;
     int k;
     bool cuts;
-    __device__ bool all_listed() const { return 0 < k && k <= kAllListed; }
 };
 __device__ __forceinline__ RowParams row_params(const SplitRow* w, int vocab) {
     RowParams q;
@@ -669,11 +668,15 @@ static_assert(sizeof(RowValues) + 64 <= 4096, "a launch has room for 4 KB of arg
 // The row's bins: kCoarse equal ones over what it spans, at most kRange or 30 temperatures (43 powers of two in weight).  A bin's weights are
 // summed as integers of a unit of its own, one limb: 2^-(unit + below(bin)), where below(bin) powers of two lie between
 // the largest weight and the bin's.  With at most unit - 25 powers of two a bin nothing of a weight is lost; in the last one,
-// which takes all that lies further down, nothing above 2^-(unit + 42); two limbs of 40 bits lose no less.
+// which takes all that lies further down, nothing above 2^-(unit + 42); two limbs of 40 bits lose no less.  Rows so cold that a bin would be more (top p
+// below a temperature of some 0.001) end their bins where it is not, far below the last weight that is not zero: what lies further down is the last
+// bin's, and weighs nothing, so that a top k whose token is there binds nothing.  Top k alone weighs nothing and spans as above.  (Settled by one
+// workgroup instead, 64 rows of 152,064 at 0.001: top p 119 us, 44 so, top k 97 and 38, both 138 and 40.)
 // (Two limbs are twice the additions in LDS and into the row's bins, and thrice the instructions.)
 struct RowBins {
     float scale, binades;
     int unit;
+    bool cold;  // what the bins span ends where weights are long zero
     __device__ int bin(float v, float mx) const { return static_cast<int>(fminf((mx - v) * scale, static_cast<float>(kCoarse - 1))); }
     __device__ int below(int b) const { return static_cast<int>(static_cast<float>(b) * binades); }
     __device__ unsigned long long weight(float w, int b) const {
@@ -688,6 +691,8 @@ struct RowBins {
         const float far = static_cast<float>(b + 1) / scale * 1.00001f;
         return mx - far - fmaxf(fabsf(mx), far) * 1e-6f;
     }
+    // whether the list takes every token down to the bin of the k-th
+    __device__ bool all_listed(const RowParams& q) const { return 0 < q.k && q.k <= kAllListed && !cold; }
     __device__ double value(unsigned long long sum, int b) const { return ldexp(static_cast<double>(sum), -(unit + below(b))); }
 };
 
@@ -698,12 +703,15 @@ struct RowTop {
     bool nan;
     // whether the row's thresholds can be found by bins
     __device__ bool binned(int vocab, const RowParams& q, RowBins* bins) const {
-        const float range = fminf(best.value - low, fmaxf(kRange, 30.f * q.temp));
+        bins->unit = 62 - (32 - __clz(vocab));  // 2^(32 - clz) weights of less than two of a bin's stay below 2^63
+        float range = fminf(best.value - low, fmaxf(kRange, 30.f * q.temp));
+        const float most = 0.999f * static_cast<float>(bins->unit - 25) * static_cast<float>(kCoarse - 1) / (q.inv_temp * 1.44269504f);
+        bins->cold = q.p < 1.f && range > most;
+        if (bins->cold) range = most;
         if (vocab > kMaxBinned || nan || !(fabsf(best.value) < INFINITY) || !(range > 1e-30f) || !weighs(q.inv_temp)) return false;
         bins->scale = static_cast<float>(kCoarse - 1) / range;
         bins->binades = q.inv_temp * 1.44269504f / bins->scale;
-        bins->unit = 62 - (32 - __clz(vocab));  // 2^(32 - clz) weights of less than two of a bin's stay below 2^63
-        return bins->binades <= static_cast<float>(bins->unit - 25);
+        return true;
     }
 };
 __device__ RowTop row_top(const SplitRow* w, int parts) {
@@ -865,7 +873,7 @@ __global__ __launch_bounds__(kPart) void split_weigh_kernel(const float* __restr
     }
     RowBins bins;
     if (!top.binned(vocab, q, &bins)) return;
-    const bool weigh = q.p < 1.f && !q.all_listed(), counts = q.k > 0;
+    const bool weigh = q.p < 1.f && !bins.all_listed(q), counts = q.k > 0;
     for (int b = threadIdx.x; b < kCoarse; b += kPart) {
         sum[b] = 0;
         count[b] = 0;
@@ -996,7 +1004,9 @@ __global__ __launch_bounds__(kPart) void split_list_kernel(const float* __restri
         above_k = at.above;
         from = upto = k_bin;
     }
-    if (q.all_listed()) {
+    const bool binds = q.k > 0 && !(bins.cold && k_bin == kCoarse - 1);  // (else top k keeps every token that weighs anything)
+    if (!binds) k_bin = -1;
+    if (bins.all_listed(q)) {
         from = 0;
     } else if (q.p < 1.f) {
 #pragma unroll
@@ -1010,7 +1020,7 @@ __global__ __launch_bounds__(kPart) void split_list_kernel(const float* __restri
             scan.around(k_bin, &least, &most);
             upto = scan.find(p * most, &found[1]).bin;
             from = scan.find(p * least, &found[2]).bin;
-        } else if (q.k == 0) {
+        } else if (!binds) {
             target = p * scan.total;
             const Found at = scan.find(target, &found[1]);
             from = upto = at.bin;
@@ -1211,13 +1221,13 @@ __device__ uint32_t cut_of_list(Cutting& s, const SplitRow* w, const RowParams& 
     bool in[kHeld];
     unsigned long long value[kHeld];
     const int k_bin = w->k_bin;
-    const bool all_listed = q.all_listed();
+    const bool all_listed = bins.all_listed(q), binds = q.k > 0 && !(bins.cold && k_bin < 0);
     Found at{w->from, w->above};
     double target = w->target;
 #pragma unroll
     for (int j = 0; j < kHeld; ++j)
         bin[j] = static_cast<int>(threadIdx.x) + j * kThreads < n ? bins.bin(v[j], mx) : -2;
-    if (q.k > 0) {
+    if (binds) {
         if (k_bin < 0) return 0;
 #pragma unroll
         for (int j = 0; j < kHeld; ++j) {
@@ -1230,7 +1240,7 @@ __device__ uint32_t cut_of_list(Cutting& s, const SplitRow* w, const RowParams& 
     }
 #pragma unroll
     for (int j = 0; j < kHeld; ++j) value[j] = bin[j] >= 0 ? bins.weight(expf((v[j] - mx) * q.inv_temp), bin[j]) : 0;
-    if (q.k > 0) {
+    if (binds) {
         // the weights of what top k keeps: of its own bin from the list, of those above from the list or the row's bins
         using Scan = BinScan<kThreads>;
         const int b0 = static_cast<int>(threadIdx.x) * Scan::PER;
@@ -1255,7 +1265,7 @@ __device__ uint32_t cut_of_list(Cutting& s, const SplitRow* w, const RowParams& 
 #pragma unroll
     for (int j = 0; j < kHeld; ++j) in[j] = bin[j] == at.bin && order_key(v[j]) >= cut;
     const auto weight = [&](unsigned long long sum) { return bins.value(sum, at.bin); };
-    return q.k > 0 ? key_reaching<true>(s.search[1], bins, mx, at.bin, v, in, value, at.above, target, weight)
+    return binds ? key_reaching<true>(s.search[1], bins, mx, at.bin, v, in, value, at.above, target, weight)
                    : key_reaching<false>(s.search[1], bins, mx, at.bin, v, in, value, at.above, target, weight);
 }
 

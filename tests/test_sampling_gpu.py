@@ -163,12 +163,15 @@ def test_shared_rows_choose_what_rows_alone_do(kind, rows, vocab):
 
 
 # temperature, top k, top p, and the width of a bulk of tokens far below the maximum (0: none)
+COLD = [(0.003, 0, 0.9, 0), (0.001, 50, 1.0, 0), (0.001, 50, 0.9, 0), (0.0003, 50, 0.9, 0), (0.0005, 3000, 0.9, 0), (1e-5, 0, 0.5, 0), (1e-5, 9000, 0.9, 0),
+        (0.004, 2000, 0.3, 0), (0.0003, 2, 1.0, 0), (1e-20, 3, 0.9, 0)]
 BULKS = [(1.0, 20000, 1.0, 0.35), (4.0, 0, 0.9, 0.35), (1.0, 20000, 0.9, 0.5), (4.0, 0, 0.6, 0.2), (1.0, 20000, 1.0, 0.2), (1.0, 20000, 0.9, 1.0)]
 
 
-@pytest.mark.parametrize("cases, vocab", [(BULKS, 152064)], ids=["bulks"])
+@pytest.mark.parametrize("cases, vocab", [(COLD, 152064), (COLD, 16385), (BULKS, 152064)], ids=["cold", "cold and few", "bulks"])
 def test_lists_settle_cold_rows_and_thresholds_in_a_bulk(cases, vocab):
-    """Rows whose threshold lies where most tokens are choose what they choose alone, and from their lists: not by the slow way that a row takes which its list does not settle (the tokens that a row's list got are the first
+    """Rows whose weights fall to zero within a bin or two, and rows whose threshold lies where most tokens are, choose what they choose
+    alone, and from their lists: not by the slow way that a row takes which its list does not settle (the tokens that a row's list got are the first
     number of its workspace; an empty or a full list settles nothing)."""
     from from_scratch_inference_engine_amd import ops
     from from_scratch_inference_engine_amd.ops.functions import _stream, check
