@@ -366,9 +366,9 @@ int fsie_sample_split(const float* logits, int n_rows, int vocab, const float* t
                       const float* top_p, const double* uniform, int on_host, void* workspace, int32_t* out, hipStream_t stream);
 int fsie_sample_by_value(void);
 
-// ---- products of a hundred to some thousand rows ------------------------------------------------
+// ---- products of some twenty to some thousand rows ------------------------------------------------
 // x [M, K] . w [N, K]^T, bfloat16, N a multiple of 16, K of 64, everything 16-byte aligned.  result 0: y bfloat16 [M, N] = sum + bias (float32 [N] or
-// null); 1: y float32 [splits, M, N], partial sums of slices of K.  tile 0 to 2: 64 x 64, 64 x 128, 128 x 128 rows of x and w.  The plan: tile + 256 * slices,
+// null); 1: y float32 [splits, M, N], partial sums of slices of K.  tile 0 to 3: 64 x 64, 64 x 128, 128 x 128 rows of x and w, 64 x 64 in six stages of LDS instead of three.  The plan: tile + 256 * slices,
 // or -1 where the library's product is the faster one.
 int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int units);
 int fsie_gemm_mfma_block(const void* x, const void* w, const float* bias, void* y, int M, int N, int K, int result, int splits, int tile,

@@ -1,4 +1,4 @@
-// Y[M, N] = X[M, K] . W[N, K]^T of a hundred to some thousand rows where the tiles of gemm_mfma_tile.hip would leave most of the chip idle: matrices
+// Y[M, N] = X[M, K] . W[N, K]^T of some twenty to some thousand rows where the tiles of gemm_mfma_tile.hip would leave most of the chip idle: matrices
 // of one to some ten MB, a step's portion of a prompt at a time.  bfloat16 operands in rows, on the matrix cores; the result in
 // bfloat16 with the bias added before the one rounding, or float32 partial sums of slices of K for the norm that adds them up.
 //
@@ -240,13 +240,24 @@ int launch_shape(int tile, const Call& c) {
 // Which tile, and in how many slices of K, M rows of this product are best taken; -1: the library's product is faster or the sizes are not
 // the kernel's.  Returns tile + 256 * slices.
 // The rule is the time that a count of steps gives: fixed + steps * a step's, workgroups that share a unit taking turns (so many as the unit's LDS
-// holds; a second round of 128 x 128 was up to 1.36 of the library's time and is not taken), the weights from HBM at 6.7 to 9 TB/s more; a whole product's
-// bytes or the slices' sums here and in the norm at 3 TB/s.  It has to be no more than the library's 8.3 us, 1.64 PFLOP/s, weights at 3 TB/s and x at 2.2, the
-// best fit of what it took with weights from HBM at 24 matrices of 1 to 50 MB and 19 numbers of rows from 70 to 4,096 (slices: 0.95 of that and the norm's
-// reading).  Of these 456 and as many with slices and the norm the rule takes 463, at a median of 0.76 of the library's time and at most 1.02 but for 129
-// rows of N = 8192, K = 2048 (1.12; this / the library, us: 1,375 rows of N = 1152,
+// holds; a second round of 128 x 128 was up to 1.36 of the library's time and is not taken), the weights from HBM at 6.7 to 9 TB/s more; no less than the
+// eight dies' reads of x take; a whole product's bytes or the slices' sums here and in the norm at 3 TB/s.  It has to be no more than the library's 8.3 us, 1.64 PFLOP/s,
+// weights at 3 TB/s and x at 2.2, the best fit of what it took with weights from HBM (slices: 0.95 of that and the norm's reading).
+// Measured with weights from HBM at 2,216 sizes that it takes, 17 to 4,096 rows of 0.02 to 142 MB, it is at a median of 0.7 of the library's time; 34 are beyond 1.02,
+// of which 100 rows of N = K = 4096 1.10, 385 of N = 6144, K = 4096 1.17, 1,009 of N = 160, K = 3072 1.21 (this / the library, us: 17 rows of
+// N = K = 768 5.1 / 5.0, 64 of them 5.2 / 7.0, 64 of N = 512, K = 896 5.0 / 7.7, 1,375 of N = 1152,
 // K = 896 7.5 / 11.3, 512 of N = 4608, K = 3584 28.9 / 33.3, 1,000 of N = K = 3584 30.4 / 36.9, 2,048 of N = 2048, K = 8192 67.7 / 75.5, 256 of N = 3072, K = 1024 6.9 / 11.9; with
-// the norm, 96 rows of N = 896, K = 4864 in six slices 9.4 / 15.7, 96 of N = 2048, K = 8192 in four 15.3 / 24.0).
+// the norm, 96 rows of N = 896, K = 4864 in seven slices 9.2 / 15.4, 96 of N = 2048, K = 8192 in four 16.3 / 24.0).  What it leaves out besides:
+// - beyond kBeyond, where the estimate tells nothing (129 rows of N = K = 8192 66.6 / 46.4, 384 79.9 / 62.1, 96 of N = 16384, K = 2048 22.6 / 20.8), all but slices
+//   of a K longer than N for up to 256 rows (N = 4096, K = 14336 0.44 to 0.79 of the library's time, N = 5120, K = 13824 0.49 to 0.93) and tiles of 128 x 128 that leave few units
+//   idle, K up to 4096 (129 to 256 rows of N = 16384, K = 2048 0.87 to 0.91, of N = 14336, K = 4096 0.88 to 1.00);
+// - 129 to 159 rows of N above 6,400 to 10,240 and K from 2048, where the library is at its best and a third of these tiles' rows are none
+//   (N = 8192, K = 2048 18.3 / 15.9, N = 10240 19.9 / 17.7, N = 7168, K = 3072 24.2 / 22.1; with K = 1536 or N = 6144 0.72);
+// - slices of more than 8,192 rows of W (65 rows of N = 10240, K = 2048 and the norm 59.9 / 50.3).
+// The dies' reads of x: 1,845 rows of N = 512, K = 6656 33.7 / 29.4, 2,284 of N = 432, K = 11776 57.6 / 49.6, which the steps alone put at 22.8 and 37.7.
+constexpr double kBeyond = 53e6;   // bytes of weights
+constexpr double kDiesRead = 6.5e6;  // bytes a us of x by all dies
+
 extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int units) {
     if (M <= 0 || N <= 0 || K <= 0 || units <= 0 || N % 16 || K % kStep || (result != kPlain && result != kSums)) return -1;
     if (static_cast<int64_t>(M) * K * 2 >= (int64_t{1} << 31) || static_cast<int64_t>(N) * K * 2 >= (int64_t{1} << 31)) return -1;
@@ -255,23 +266,35 @@ extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int un
     const double turns[4][4] = {{0, 1, 1.55, 2.6}, {0, 1, 1.9}, {0, 1}, {0, 1}};  // workgroups on a unit: a step's time of one alone
     const int64_t steps = K / kStep;
     const double weights = 2.0 * N * static_cast<double>(K), flops = 2.0 * M * static_cast<double>(N) * K;
+    const double rows_bytes = 2.0 * M * static_cast<double>(K);
+    const bool large = weights > kBeyond;
+    if (large && (result == kSums ? M > 256 || K <= N : M <= 128 || K > 4096)) return -1;
+    if (result == kSums ? N > 8192 : M > 128 && M < 160 && N > 6400 && N <= 10240 && K >= 2048) return -1;
     const double whole = 4.0 * M * static_cast<double>(N) / 3e6;  // the delta in bfloat16, out and into the norm
     double best = 1e30;
     int choice = -1;
+    bool fills = false;  // (nearly all units)
     for (int tile = 0; tile < 4; ++tile) {
         for (int slices = 1; slices <= (result == kSums ? 8 : 1); ++slices) {
             if (slices > 1 && steps / slices < 4) break;
-            const int64_t groups = ceil_div64(M, rows[tile]) * ceil_div64(N, cols[tile]) * slices, deep = ceil_div64(groups, units);
+            const int64_t m_tiles = ceil_div64(M, rows[tile]), n_tiles = ceil_div64(N, cols[tile]), groups = m_tiles * n_tiles * slices;
+            const int64_t deep = ceil_div64(groups, units), a_die = ceil_div64(groups, 8);
             if (deep > at_once[tile]) continue;
             double us = fixed[tile] + static_cast<double>(ceil_div64(steps, slices)) * us_a_step[tile] * turns[tile][deep] + weights * 1e-6 * us_a_mb[tile];
+            // (of one slice's x a die reads the rows of its tiles, of a second one where its tiles go on into that)
+            const double of_slice = a_die < m_tiles ? static_cast<double>(a_die) / m_tiles : 1.0, slices_read = static_cast<double>(a_die) / (m_tiles * n_tiles);
+            const double share = (of_slice > slices_read ? of_slice : slices_read) / slices, read = 8.0 * rows_bytes * (share < 1.0 ? share : 1.0) / kDiesRead;
+            if (us < read) us = read;
             if (result == kSums) us += (slices == 1 ? whole : 2.0 * slices * whole);
             if (us < best) {
                 best = us;
                 choice = tile + 256 * slices;
+                fills = 8 * groups >= 7 * units;
             }
         }
     }
-    const double library = 8.3 + flops / 1.64e9 + weights / 3e6 + 2.0 * M * static_cast<double>(K) / 2.2e6;
+    const double library = 8.3 + flops / 1.64e9 + weights / 3e6 + rows_bytes / 2.2e6;
+    if (large && result == kPlain && (choice % 256 != 2 || !fills)) return -1;
     return choice >= 0 && best <= (result == kSums ? 0.95 * (library + whole) : library) ? choice : -1;
 }
 

@@ -708,7 +708,7 @@ def gemm_block_plan(m: int, n: int, k: int, result: int):
 
 
 def gemm_mfma_block(x: torch.Tensor, weight: torch.Tensor, result: int, tile: int, splits: int = 1, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x [M, K] . weight [N, K]^T (bfloat16, N a multiple of 16, K of 64) of a hundred to some thousand rows in small tiles.
+    """x [M, K] . weight [N, K]^T (bfloat16, N a multiple of 16, K of 64) of some twenty to some thousand rows in small tiles.
     GEMM_BLOCK_PLAIN: [M, N] in bfloat16, ``bias`` (float32) added first; GEMM_BLOCK_SUMS: float32 partial sums [splits, M, N] over slices of K."""
     _need(x, "gemm x", dtype=torch.bfloat16, ndim=2)
     _need(weight, "gemm weight", dtype=torch.bfloat16, ndim=2)

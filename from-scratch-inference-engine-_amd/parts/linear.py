@@ -24,8 +24,9 @@ class Linear:
     (``for_residual``: 17 to 64 rows, and any number where K is long) and for the partial sums of
     other projections of 17 to 64 rows (``partial_sums``); a third for up to 16 rows and a K so short that all of it is under
     way at once (``ops.gemm_stream_plan``); residual projections of more than 128 rows whose K is 16,384
-    and more the engine's kernel for many rows, in slices of K (``ops.gemm_tile_plan``); products of 65 rows
-    and more of matrices of some ten MB the one in small tiles (``ops.gemm_block_plan``); everything else
+    and more the engine's kernel for many rows, in slices of K (``ops.gemm_tile_plan``); products of 17 rows
+    and more that no other of these takes, of matrices up to some 50 MB, the one in small tiles (``ops.gemm_block_plan``, up to 64 rows
+    those of a short K or few rows of W: ``partial_sums``); everything else
     the library product (hipBLASLt through torch, where the reference's engine calls cuBLAS) with
     float32 accumulation, the bias added by a kernel of the engine.  A large weight has a second copy in
     the order of the matrix instruction's fragments (``prepare``, ``streamed``), from which the
@@ -59,7 +60,7 @@ class Linear:
         self.streamed = None  # the weight in fragment order (ops.FragmentOrdered), if prepare() made one
         self._wide_splits: dict = {}  # tiles of rows -> slices of K (a property of the sizes alone)
         self._wide_takes: dict = {}   # (tiles, slices, gate/up) -> whether the kernel takes them from this weight
-        self._many_plans: dict = {}   # (rows, result, library tuning) -> how a product of more than 128 rows is taken (of the sizes alone)
+        self._many_plans: dict = {}   # (rows, result, library tuning) -> how a product of more than 16 rows is taken (of the sizes alone)
 
     @property
     def weight(self) -> Optional[torch.Tensor]:

@@ -37,7 +37,7 @@ def test_products_in_small_tiles(ops, m, n, k, tile):
         assert ((got[-1].double() - last).abs() <= bound).all(), splits
 
 
-@pytest.mark.parametrize("m, n, k", [(200, 896, 896), (300, 128, 512), (96, 896, 2048), (700, 512, 512)])
+@pytest.mark.parametrize("m, n, k", [(200, 896, 896), (300, 128, 512), (96, 896, 2048), (700, 512, 512), (30, 896, 512), (17, 512, 896), (64, 2048, 320)])
 def test_linear_takes_them(ops, m, n, k, monkeypatch):
     """What ``Linear`` makes of them, with the bias in the product and as partial sums, is the library's within their roundings; rows that the
     kernel's loads cannot read go to the library."""
@@ -60,6 +60,9 @@ def test_linear_takes_them(ops, m, n, k, monkeypatch):
     layer.bias, layer.has_bias = None, False
     delta = layer.for_residual(x, SimpleNamespace(partial_sums_ok=True))
     assert ((delta.double().sum(0) if delta.ndim == 3 else delta.double()) - exact).abs().le(2.0 ** -7 * size).all()
+    large = m > 128 and ops.gemm_tile_plan(m, n, k, ops.GEMM_TILE_SUMS) is not None
+    slices = 1 if large or m <= 64 else (ops.gemm_block_plan(m, n, k, ops.GEMM_BLOCK_SUMS) or (0, 1))[1]
+    assert (ops.GEMM_BLOCK_SUMS in seen) == (slices > 1) and (not slices > 1 or delta.shape == (slices, m, n))
     seen.clear()
     wide = torch.zeros((m, k + 4), dtype=torch.bfloat16, device="cuda")
     odd = wide[:, 4:]
