@@ -153,7 +153,6 @@ int launch_mt(int waves, const float* x, const float* w, const float* bias, floa
 // and 34.4; 117 TFLOP/s at 1,500 x 9728 x 896 (96 before), where the library reaches 154 at 8,192 cubed.  Six stages where every workgroup has a unit
 // to itself, whose step of 0.43 us would else not cover the way from HBM; three leave room for three workgroups a unit.
 constexpr int kTileEdge = 64, kTileK = 32, kTileFlush = 256;
-constexpr int kFewTiles = 256;  // so many workgroups have a unit each
 
 enum Whole { PLAIN = 0, SUMS = 1, GATED = 2 };
 
@@ -404,7 +403,7 @@ static int tile_product(const float* x, const float* w, const float* bias, float
     if (K % kTileK == 0 && static_cast<int64_t>(M) * K * 4 < (int64_t{1} << 31) && static_cast<int64_t>(N) * K * 4 < (int64_t{1} << 31) &&
         groups < (int64_t{1} << 30)) {
         const TileCall c{x, w, bias, y, gate ? *gate : Gate{}, M, N, K, static_cast<int>(slice), static_cast<int>(tiles_m), static_cast<int>(tiles_n), splits, stream};
-        const bool few = groups <= kFewTiles;
+        const bool few = groups <= fsie_compute_units();  // (a unit each)
         if (splits > 1) return few ? launch_block<SUMS, 6>(c) : launch_block<SUMS, 3>(c);
         if (gate) return few ? launch_block<GATED, 6>(c) : launch_block<GATED, 3>(c);
         return few ? launch_block<PLAIN, 6>(c) : launch_block<PLAIN, 3>(c);
