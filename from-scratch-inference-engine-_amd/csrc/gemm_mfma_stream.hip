@@ -146,14 +146,15 @@ int launch_steps(int s, const StreamCall& c, hipStream_t stream) {
     return launch<WAVES, LEAST, NB, RESULT, FRAGS>(c, stream);
 }
 
-// (four waves: whole products; sums: eight waves on a fragment-ordered W.  Two blocks of rows a workgroup: of eight waves, on a
+// (four waves: whole products, and sums on rows of W; sums on a fragment-ordered W: eight.  Two blocks of rows a workgroup: of eight waves, on a
 // fragment-ordered W; what else is asked for in twos goes one by one)
 template <int RESULT, bool FRAGS>
 int launch_waves(int waves, int nb, int s, const StreamCall& c, hipStream_t stream) {
     constexpr int LEAST = RESULT == SUMS ? 4 : 5;
     if constexpr (FRAGS)
         if (waves == 8 && nb == 2) return launch_steps<8, LEAST, 2, RESULT, FRAGS>(s, c, stream);
-    if (waves == 8) return launch_steps<8, LEAST, 1, RESULT, FRAGS>(s, c, stream);
+    if constexpr (RESULT != SUMS || FRAGS)
+        if (waves == 8) return launch_steps<8, LEAST, 1, RESULT, FRAGS>(s, c, stream);
     if constexpr (RESULT != SUMS)
         return waves == 4 ? launch_steps<4, 1, 1, RESULT, FRAGS>(s, c, stream) : launch_steps<16, LEAST, 1, RESULT, FRAGS>(s, c, stream);
     if constexpr (RESULT == SUMS && !FRAGS)
