@@ -178,3 +178,23 @@ def test_plans_of_small_tiles_are_ones_the_kernel_takes():
             tile, slices = got % 256, got // 256
             assert 0 <= tile <= 3 and 1 <= slices <= (8 if sums else 1) and slices <= k // 64, (m, n, k, sums)
     assert taken > 1000
+
+
+def test_a_norm_whose_weight_does_not_lie_on_16_bytes_does_not_wait_for_its_product():
+    from from_scratch_inference_engine_amd.parts.base import HiddenState
+    from from_scratch_inference_engine_amd.parts.norm import RMSNorm
+
+    norm, hidden = RMSNorm(64, 1e-6), HiddenState(torch.zeros(1, 64))
+    room = torch.ones(64 + 8)
+    aligned = (-room.data_ptr() // 4) % 4  # (values to the next 16 bytes)
+    for off in range(4):
+        norm.weight = room[aligned + off:aligned + off + 64]
+        assert norm.can_wait(hidden, torch.bfloat16) == (off == 0)
+    norm.weight = room[aligned:aligned + 64]
+    for sums, waits in ((torch.zeros(3, 1, 64), True), (torch.zeros(1, 64, dtype=torch.bfloat16), False), (torch.zeros(3, 1, 64, dtype=torch.bfloat16), False)):
+        hidden.delta = sums
+        assert norm.can_wait(hidden, torch.bfloat16) == waits
+    hidden.delta = None
+    assert not norm.can_wait(hidden, torch.float32)
+    hidden.delta_scale = 0.5
+    assert not norm.can_wait(hidden, torch.bfloat16)
