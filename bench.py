@@ -97,6 +97,7 @@ def kernel_classes(runner, cfg, batch: int, prompt_len: int, itemsize: int) -> d
         "attention_scalar": lambda a, k: "attention", "attention_merge": lambda a, k: "attention",
         "gemm_mfma_skinny": lambda a, k: matrix_class(a[1]), "gemm_mfma_wide": lambda a, k: matrix_class(a[1]),
         "gemm_mfma_wide_swiglu": lambda a, k: "gate_up", "gemm_mfma_stream": lambda a, k: matrix_class(a[1]),
+        "gemm_mfma_block": lambda a, k: matrix_class(a[1]), "gemm_mfma_normed": lambda a, k: matrix_class(a[5]),
         "gemm": lambda a, k: matrix_class(a[1]), "gemm_mfma_fp32": lambda a, k: matrix_class(a[1]),
         "gemm_mfma_fp32_sums": lambda a, k: matrix_class(a[1]), "gemm_fp32_tile": lambda a, k: matrix_class(a[1]),
         "gemm_mfma_tile": lambda a, k: matrix_class(a[1]), "gemm_mfma_tile_gated": lambda a, k: "gate_up",
