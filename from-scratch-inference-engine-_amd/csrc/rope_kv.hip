@@ -366,13 +366,16 @@ extern "C" int fsie_rope_kv_write_table(void* qkv, const float* cos_sin, const i
     if (n_tokens == 0) return 0;
     // Eight tokens a block where there are enough blocks left to fill the device.  Blocks a token, or a run of eight: the kernel is made of
     // loads that wait for memory, so a thread has one item (four pairs, or four values), as long as there are no more than kBlocksAUnit
-    // blocks a unit.
+    // blocks a unit, and two beyond that.  (So many as kBlocksAUnit leaves, as few blocks as one a run: 8,011 tokens of 28/4 heads of 128 41.4 us, 38.4 with two
+    // items; of 40/8 64.2 and 59.9, of 14/2 of 64 11.0 and 11.4 to 12; 16,000 of these 78.7 / 71.1, 125.0 / 118.2, 24.3 / 22.4.  Three items and four: as two, to 5 per
+    // cent more for small heads from 12,000 tokens on.)
     const int units = fsie_compute_units();
     const int tok = !parts && n_tokens >= 1024 ? 8 : 1, runs = (n_tokens + tok - 1) / tok;
     const int items = tok * ((n_heads + n_kv) * (head_dim / 8) + n_kv * head_dim / 4);
     int across = (items + kThreads - 1) / kThreads;
     if (across > 8) across = 8;
-    while (across > 1 && static_cast<int64_t>(runs) * across > static_cast<int64_t>(kBlocksAUnit) * units) --across;
+    const int two_items = (items + 2 * kThreads - 1) / (2 * kThreads), least = two_items < 8 ? two_items : 8;
+    while (across > least && static_cast<int64_t>(runs) * across > static_cast<int64_t>(kBlocksAUnit) * units) --across;
     const dim3 grid(static_cast<unsigned>(runs), static_cast<unsigned>(across));
 #define FSIE_ROPE_PARTS(T, B)                                                                                     \
     rope_kv_write_table_kernel<T, B, 1, true><<<grid, kThreads, 0, stream>>>(                                     \

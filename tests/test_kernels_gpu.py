@@ -135,7 +135,7 @@ def test_rope_and_cache_write(ops, dtype, from_table, heads, kv, hd, theta):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("t", [5, 1027])  # a token a block; eight
+@pytest.mark.parametrize("t", [5, 1027, 9001])  # a token a block; eight; eight in blocks of two items a thread
 def test_a_turned_pair_rounds_the_same_way_in_every_form(ops, dtype, t):
     """a1 c - (a2 s) and a1 s + (a2 c), the product in brackets rounded and the other added to it exactly: with and without a bias,
     from the projection or from partial sums, a token or eight of them a block.  (In float64 the exact product and the sum
