@@ -34,16 +34,20 @@ class PreNormBlock(Block):
 
     @staticmethod
     def _normed(norm: Norm, part: Part, hidden: HiddenState, ctx, *cache):
-        if len(hidden.residual) <= PreNormBlock.few_rows and norm.can_wait(hidden, ctx.compute_dtype):
-            if part.takes_pending_norm(len(hidden.residual), 0 if hidden.delta is None else len(hidden.delta), ctx, *cache):
+        if norm.can_wait(hidden, ctx.compute_dtype):
+            if part.takes_pending_norm(hidden.residual.shape[0], 0 if hidden.delta is None else len(hidden.delta), ctx, *cache):
                 return norm.wait(hidden, ctx.compute_dtype)
         return norm(hidden, ctx.compute_dtype)
 
     def forward(self, hidden: HiddenState, ctx, cache) -> None:
-        few = len(hidden.residual) <= self.few_rows
+        rows = hidden.residual.shape[0]
+        if rows > self.few_rows:  # (asked once: a step of many eager layers is the host's)
+            hidden.delta = self.mixer.forward(self.mixer_norm(hidden, ctx.compute_dtype), ctx, cache)
+            hidden.delta = self.ffn.forward(self.ffn_norm(hidden, ctx.compute_dtype), ctx)
+            return
         x = self._normed(self.mixer_norm, self.mixer, hidden, ctx, cache)
         # (the output projection leaves its sums in one slice where every workgroup of the next product is going to read them)
-        ctx.sums_in_one = few and self.ffn_norm.can_wait(hidden, ctx.compute_dtype) and self.ffn.takes_pending_norm(len(hidden.residual), 1, ctx)
+        ctx.sums_in_one = self.ffn_norm.can_wait(hidden, ctx.compute_dtype) and self.ffn.takes_pending_norm(rows, 1, ctx)
         try:
             hidden.delta = self.mixer.forward(x, ctx, cache)
         finally:

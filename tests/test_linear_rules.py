@@ -198,3 +198,29 @@ def test_a_norm_whose_weight_does_not_lie_on_16_bytes_does_not_wait_for_its_prod
     assert not norm.can_wait(hidden, torch.float32)
     hidden.delta_scale = 0.5
     assert not norm.can_wait(hidden, torch.bfloat16)
+
+
+@pytest.mark.parametrize("rows, asked", [(1, 3), (2, 3), (3, 0), (40, 0)])
+def test_only_steps_of_few_rows_ask_whether_a_norm_may_wait(rows, asked):
+    """An eager step of many layers is bound by the host: a layer of more rows goes through its parts and nothing else (its rows are its shape's:
+    the length of a tensor is four calls)."""
+    from types import SimpleNamespace
+
+    from from_scratch_inference_engine_amd.parts.base import HiddenState
+    from from_scratch_inference_engine_amd.parts.block import PreNormBlock
+
+    questions, order = [], []
+
+    class Norm:
+        def __call__(self, hidden, dtype):
+            order.append("norm")
+            return "x"
+
+        def can_wait(self, hidden, dtype):
+            questions.append(hidden)
+            return False
+
+    part = SimpleNamespace(forward=lambda x, ctx, *cache: order.append("part") or len(order))
+    hidden = HiddenState(SimpleNamespace(shape=(rows, 8)))
+    PreNormBlock(Norm(), part, Norm(), part).forward(hidden, SimpleNamespace(compute_dtype=torch.bfloat16, sums_in_one=False), None)
+    assert order == ["norm", "part", "norm", "part"] and hidden.delta == 4 and len(questions) == asked
