@@ -260,14 +260,15 @@ __global__ __launch_bounds__(256) void gemm_fp32_tile_kernel(const float* __rest
 template <int RESULT, int STAGES>
 __global__ __launch_bounds__(256) void gemm_fp32_block_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                              const float* __restrict__ bias, float* __restrict__ y, int M, int N, int K,
-                                                             int k_slice, int m_tiles, int n_tiles, int splits, Gate gate) {
+                                                             int k_slice, int m_tiles, int n_tiles, int abreast, Gate gate) {
     constexpr int kRowBytes = kTileK * 4, kHalf = kTileEdge * kRowBytes, kStage = 2 * kHalf, kLoads = 4;  // a stage: W, then X
     extern __shared__ char lds[];
-    // a die (the workgroup's number modulo 8) takes neighbouring tiles: of W its own eighth, of X all
-    const int tiles = m_tiles * n_tiles * splits, a_die = (tiles + 7) / 8;
-    const int id = static_cast<int>(blockIdx.x & 7) * a_die + static_cast<int>(blockIdx.x >> 3);
-    if (id >= tiles) return;
-    const int m_tile = id % m_tiles, n_tile = id / m_tiles % n_tiles, slice = id / m_tiles / n_tiles;
+    // A die (the workgroup's number modulo 8) takes neighbouring tiles: of W its own eighth, of X all.  The slices are laid side by side and dealt so, a
+    // die few of them (abreast == splits), or dealt one by one, a die some tiles of each (abreast == 1).
+    const int tiles = m_tiles * n_tiles, dealt = tiles * abreast, a_die = (dealt + 7) / 8, turn = static_cast<int>(blockIdx.x >> 3);
+    const int id = static_cast<int>(blockIdx.x & 7) * a_die + turn % a_die;
+    if (id >= dealt) return;
+    const int slice = turn / a_die + id / tiles, m_tile = id % m_tiles, n_tile = id % tiles / m_tiles;
     const int m0 = m_tile * kTileEdge, n0 = n_tile * kTileEdge;
     const int first_step = slice * k_slice / kTileK, steps = min(K - slice * k_slice, k_slice) / kTileK;
     const int lane = threadIdx.x & (FSIE_WAVE - 1);
@@ -368,14 +369,27 @@ struct TileCall {
     hipStream_t stream;
 };
 
+// Whether slices are dealt to the dies one by one.  Side by side a die reads its slices' part of X alone, which is up to 8 per cent faster (200 rows of N = 2048,
+// K = 8192 in four 74 us, 80 one by one); but a short last slice leaves its dies idle: 2,048 rows of N = 1024, K = 640, slices of 512 and 128,
+// took 42.5 us (35.3 in the kernel above, whose workgroups go to the dies in turn), 512 rows of N = 896, K = 4864 in seven 58.3, 47.6 one by one.  So where
+// a die's workgroups make fewer rounds over its units one by one, and always where two slices are of different lengths.
+bool dealt_one_by_one(const TileCall& c) {
+    if (c.splits == 1 || c.K == static_cast<int64_t>(c.slice) * c.splits) return false;
+    if (c.splits == 2) return true;
+    const int units = fsie_compute_units(), a_die = units > 8 ? units / 8 : 1;
+    const int64_t tiles = static_cast<int64_t>(c.m_tiles) * c.n_tiles;
+    return ceil_div64(ceil_div64(tiles, 8) * c.K, static_cast<int64_t>(c.slice) * a_die) < ceil_div64(ceil_div64(tiles * c.splits, 8), a_die);
+}
+
 template <int RESULT, int STAGES>
 int launch_block(const TileCall& c) {
     constexpr int kLds = STAGES * 2 * kTileEdge * kTileK * 4;
     static const hipError_t allowed = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_fp32_block_kernel<RESULT, STAGES>),
                                                           hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     FSIE_REQUIRE(allowed == hipSuccess, "gemm_fp32_tile: %d bytes of LDS: %s", kLds, hipGetErrorString(allowed));
-    const unsigned groups = static_cast<unsigned>((static_cast<int64_t>(c.m_tiles) * c.n_tiles * c.splits + 7) / 8 * 8);
-    gemm_fp32_block_kernel<RESULT, STAGES><<<groups, 256, kLds, c.stream>>>(c.x, c.w, c.bias, c.y, c.M, c.N, c.K, c.slice, c.m_tiles, c.n_tiles, c.splits, c.gate);
+    const int abreast = dealt_one_by_one(c) ? 1 : c.splits;
+    const unsigned groups = static_cast<unsigned>((static_cast<int64_t>(c.m_tiles) * c.n_tiles * abreast + 7) / 8 * 8 * (c.splits / abreast));
+    gemm_fp32_block_kernel<RESULT, STAGES><<<groups, 256, kLds, c.stream>>>(c.x, c.w, c.bias, c.y, c.M, c.N, c.K, c.slice, c.m_tiles, c.n_tiles, abreast, c.gate);
     FSIE_CHECK_LAUNCH("gemm_fp32_tile");
     return 0;
 }

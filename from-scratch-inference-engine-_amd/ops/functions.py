@@ -491,9 +491,9 @@ def gemm_fp32_tile_splits(m: int, n: int, k: int) -> int:
     """Slices of K for ``gemm_fp32_tile``: whole runs of 256 values (the kernel's own), as many as bring its tiles of 64 x 64
     to four a compute unit at 512 rows.  By N and K alone, whatever ``m``: a row's sums are then the same in a step of any
     number of rows that takes this kernel.  Slices by the step's own rows gain at few rows of a wide W, and at many rows, and lose at others
-    (with the norm, us by 512 rows / by the step's: N = 896, K = 4864 77 / 79 at 700 rows; N = K = 2048 19 / 21 at 65, 69 / 62 at 700, 175 / 154 at
-    2,048; N = K = 5120 109 / 84 at 65).  The kernel of whole steps holds three workgroups a unit; slices that make three are no better (N = 896,
-    K = 4864 in seven / five: 36 / 43 at 300 rows, 62 / 58 at 512, 75 / 78 at 682; N = K = 2048 in four / three: 37 / 36, 48 / 49 and 68 / 76)."""
+    (with the norm, us by 512 rows / by the step's: N = 896, K = 4864 68 / 74 at 700 rows; N = K = 2048 19 / 21 at 65, 69 / 62 at 700, 171 / 150 at
+    2,048; N = K = 5120 104 / 82 at 65).  The kernel of whole steps holds three workgroups a unit; slices that make three are no better (N = 896,
+    K = 4864 in seven / five: 39 / 45 at 300 rows, 53 / 62 at 512, 70 / 75 at 682; N = K = 2048 in four / three: 40 / 39, 51 / 51 and 69 / 68)."""
     tiles = -(-_FP32_TILE_ROWS // 64) * -(-n // 64)
     wanted = min(GEMM_MAX_SPLITS, 4 * compute_units() // tiles, k // 256)
     if wanted < 2:
