@@ -414,7 +414,9 @@ static int tile_product(const float* x, const float* w, const float* bias, float
     FSIE_REQUIRE(splits == 1 || slice * (splits - 1) < K, "gemm_fp32_tile: K=%d does not give %d slices", K, splits);
     const int64_t tiles_n = ceil_div64(N, kTileEdge), groups = tiles_m * tiles_n * splits;
     if (splits == 1) slice = ceil_div64(K, kTileK) * kTileK;
-    if (K % kTileK == 0 && static_cast<int64_t>(M) * K * 4 < (int64_t{1} << 31) && static_cast<int64_t>(N) * K * 4 < (int64_t{1} << 31) &&
+    // (from four steps on: what a workgroup asks for ahead is past the end else, 65 rows of N = 151936, K = 64 59 us, through registers 48; N = 1024 6.1 and 5.6;
+    // K = 128 as fast or faster but for the first of these, 78 and 73)
+    if (K % kTileK == 0 && slice >= 4 * kTileK && static_cast<int64_t>(M) * K * 4 < (int64_t{1} << 31) && static_cast<int64_t>(N) * K * 4 < (int64_t{1} << 31) &&
         groups < (int64_t{1} << 30)) {
         const TileCall c{x, w, bias, y, gate ? *gate : Gate{}, M, N, K, static_cast<int>(slice), static_cast<int>(tiles_m), static_cast<int>(tiles_n), splits, stream};
         const bool few = groups <= fsie_compute_units();  // (a unit each)
