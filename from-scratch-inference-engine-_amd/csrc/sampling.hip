@@ -414,7 +414,8 @@ __device__ uint32_t cut_by_bisection(const float* row, int vocab, float mx, floa
 // The first token, in vocabulary order, at which the running sum of the kept weights passes uniform * their sum, from the
 // sums of the runs (in LDS): every wave finds the run, whose 64-token lines the waves then walk side by side, one each.  (One
 // wave after all of them is a chain of a trip to memory and six exchanges between lanes a line: 64 rows of 152,064
-// tokens 8.2 us in a kernel of their own; and 2 so.)
+// tokens 8.2 us in a kernel of their own; and 2 so.  Up to kLinesOfOne lines are one wave's, with all their loads under way at once.)
+constexpr int kLinesOfOne = 4;
 __device__ void draw_from_runs(const float* __restrict__ row, int vocab, Best top, float inv_temp, uint32_t cut, double uniform,
                                const double* run_sum, int32_t* out) {
     __shared__ double line_sum[kWaves];
@@ -453,6 +454,29 @@ __device__ void draw_from_runs(const float* __restrict__ row, int vocab, Best to
     run = __builtin_amdgcn_readlane(run, owner);
     cum = of_lane(cum, owner);
     int last_kept = -1;
+    if (lines <= kLinesOfOne) {
+        if (wave > 0) return;
+        const int64_t first = static_cast<int64_t>(run) * lines * FSIE_WAVE;
+        float v[kLinesOfOne];
+#pragma unroll
+        for (int q = 0; q < kLinesOfOne; ++q) v[q] = row[min(first + min(q, lines - 1) * FSIE_WAVE + lane, static_cast<int64_t>(vocab - 1))];
+#pragma unroll
+        for (int q = 0; q < kLinesOfOne; ++q) {
+            if (q >= lines) break;
+            const int64_t line = first + q * FSIE_WAVE;
+            const bool kept = line + lane < vocab && order_key(v[q]) >= cut;
+            const double w = wave_upto(kept ? token_weight(v[q], mx, inv_temp) : 0.0);
+            const unsigned long long hit = __ballot(kept && threshold < cum + w), any = __ballot(kept);
+            if (hit) {
+                if (lane == 0) *out = static_cast<int>(line) + __ffsll(hit) - 1;
+                return;
+            }
+            if (any) last_kept = static_cast<int>(line) + 63 - __clzll(any);
+            cum += of_lane(w, FSIE_WAVE - 1);
+        }
+        if (lane == 0) *out = last_kept >= 0 ? last_kept : top.index;
+        return;
+    }
     for (int j0 = 0; j0 < lines; j0 += kWaves) {
         const int64_t i = (static_cast<int64_t>(run) * lines + j0 + wave) * FSIE_WAVE + lane;
         const float v = row[i < vocab ? i : vocab - 1];
