@@ -365,6 +365,8 @@ int64_t fsie_sample_workspace(int n_rows, int vocab, int thresholds);
 int fsie_sample_split(const float* logits, int n_rows, int vocab, const float* temperature, const int32_t* top_k,
                       const float* top_p, const double* uniform, int on_host, void* workspace, int32_t* out, hipStream_t stream);
 int fsie_sample_by_value(void);
+// Whether that is the faster way for parameters on the device, as far as the host can tell: by which of top_k and top_p are given.
+int fsie_sample_shares(int n_rows, int vocab, int top_k, int top_p);
 
 // ---- products of some twenty to some thousand rows ------------------------------------------------
 // x [M, K] . w [N, K]^T, bfloat16, N a multiple of 16, K of 64, everything 16-byte aligned.  result 0: y bfloat16 [M, N] = sum + bias (float32 [N] or

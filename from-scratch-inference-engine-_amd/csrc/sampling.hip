@@ -608,13 +608,18 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(const float* __restric
 //    32,000          46 / 23    48 / 28    48 / 33     51 /  45     96 /  71    269 / 188    516 /   419
 //    65,536          71 / 24    71 / 33    74 / 43     77 /  63    147 / 107    432 / 368    794 /   692
 //   152,064         138 / 25   150 / 46   152 / 70    158 / 116    303 / 211    870 / 759  1,640 / 1,424
-// so where thresholds are given rows are shared up to kMostRows of them (what was measured; their workspaces are 59 KB a row).  Without
-// thresholds it is three launches beside one of two passes, and the line is kMostPlainRows (8, 64, 128, 256, 380 rows of 16,384:
-// 17 / 11, 17 / 13, 17 / 15, 18 / 20, 34 / 26; of 152,064: 42 / 12, 48 / 27, 51 / 43, 61 / 73, 105 / 103).
+// so where both thresholds are given rows are shared up to kMostRows of them (what was measured; their workspaces are 59 KB a row).  Where all rows ask
+// for one kind, a workgroup a row is the faster one below that, up to one round of them: all rows at top k / top p / a temperature alone, alone / shared, us,
+//    16,384 tokens, 16 rows  25 / 24    34 / 28    17 / 14;  40  25 / 28    34 / 33    18 / 15;  100  25 / 32    34 / 38    18 / 18;  256  27 / 29    35 / 36    19 / 22
+//    32,000          40      30 / 29    45 / 35    19 / 16;  80  31 / 30    45 / 37    19 / 18;  192  32 / 36    47 / 46    20 / 24;  320  60 / 52    87 / 67    37 / 38
+//    65,536          80      42 / 35    72 / 46    25 / 23; 128  43 / 37    73 / 49    26 / 28;  224  50 / 56    77 / 72    32 / 40;  512 100 / 91   152 / 121   62 / 72
+//   152,064          64      87 / 40   154 / 55    50 / 29; 128  88 / 59   155 / 82    53 / 46;  224  95 / 96   159 / 128   60 / 72; 1,024 412 / 416 649 / 497 260 / 306
+// and the lines lie where they meet (fsie_sample_shares).  Parameters that the first launch brings spare a copy that is 20 us of the host: such rows are always shared.
 // (Without temperatures it is one pass over the row, and a workgroup a row is the faster one; with temperatures that all
 // say greedy too, but that only the device knows.)
 constexpr int kSplitFrom = 16384;
 constexpr int kMostRows = 4096, kMostPlainRows = 160;
+constexpr int kLongPlain = 98304;
 constexpr int kPart = 512;          // threads of a shared row's workgroups
 constexpr int kMaxParts = 32;
 // Bins of a shared row.  512 are a per cent faster where the thresholds lie among few tokens (64 rows of 152,064 as above 44.7 us, 45.1 with 2,048), but
@@ -1368,6 +1373,13 @@ __global__ __launch_bounds__(kThreads) void split_draw_kernel(const float* __res
 extern "C" int64_t fsie_sample_workspace(int n_rows, int vocab, int thresholds) {
     const bool shared = vocab >= kSplitFrom && vocab <= (1 << 30) && n_rows > 0 && n_rows <= (thresholds ? kMostRows : kMostPlainRows);
     return shared ? static_cast<int64_t>(n_rows) * static_cast<int64_t>(sizeof(SplitRow)) : 0;
+}
+
+extern "C" int fsie_sample_shares(int n_rows, int vocab, int top_k, int top_p) {
+    if (fsie_sample_workspace(n_rows, vocab, top_k || top_p) == 0) return 0;
+    if (top_k && top_p) return 1;
+    if (!top_k && !top_p) return n_rows <= (vocab < kLongPlain ? 96 : 128);
+    return n_rows <= (vocab - 8000) / (top_k ? 450 : 130) || n_rows > fsie_compute_units();
 }
 
 extern "C" int fsie_sample(const float* logits, int n_rows, int vocab, const float* temperature,

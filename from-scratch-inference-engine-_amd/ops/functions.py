@@ -1217,9 +1217,8 @@ def sample(logits: torch.Tensor, temperature: Optional[torch.Tensor] = None,
     # A large vocabulary in few rows: every row is shared by several workgroups, which meet in a workspace.  Not for the
     # greedy choice alone, which is one pass: 1 row of 151,936 takes 9.5 us so and 12 shared, 64 rows 14 and 13, 256 rows
     # 24 and 33.
-    size = 0 if temperature is None else int(load().fsie_sample_workspace(n, v, top_k is not None or top_p is not None))
-    if size:
-        work = torch.empty((size,), dtype=torch.uint8, device=logits.device)
+    if temperature is not None and load().fsie_sample_shares(n, v, top_k is not None, top_p is not None):
+        work = torch.empty((load().fsie_sample_workspace(n, v, top_k is not None or top_p is not None),), dtype=torch.uint8, device=logits.device)
         check(load().fsie_sample_split(logits.data_ptr(), n, v, _ptr(temperature), _ptr(top_k), _ptr(top_p),
                                        _ptr(uniform), 0, work.data_ptr(), out.data_ptr(), _stream()))
         return out

@@ -133,6 +133,7 @@ _SIGNATURES = {
     "fsie_sample_workspace": ([c_int, c_int, c_int], c_int64),
     "fsie_sample_split": ([_P, c_int, c_int, _P, _P, _P, _P, c_int, _P, _P, _P], c_int),
     "fsie_sample_by_value": ([], c_int),
+    "fsie_sample_shares": ([c_int, c_int, c_int, c_int], c_int),
     "fsie_gemm_mfma_block_plan": ([c_int, c_int, c_int, c_int, c_int], c_int),
     "fsie_gemm_mfma_block": ([_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P], c_int),
     "fsie_gemm_mfma_normed_takes": ([c_int, c_int, c_int, c_int, c_int], c_int),

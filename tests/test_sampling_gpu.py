@@ -196,3 +196,15 @@ def test_lists_settle_cold_rows_and_thresholds_in_a_bulk(cases, vocab):
     assert torch.equal(alone, shared)
     listed = work.view(rows, -1)[:, :4].contiguous().view(torch.int32).flatten().tolist()
     assert all(0 < n <= 4096 for n in listed), listed
+
+
+@pytest.mark.parametrize("rows, vocab, top_k, top_p, shared", [
+    (16, 16384, 1, 0, 1), (40, 16384, 1, 0, 0), (256, 16384, 1, 0, 0), (300, 16384, 1, 0, 1), (40, 16384, 0, 1, 1), (100, 16384, 0, 1, 0), (300, 16384, 0, 1, 1),
+    (40, 32000, 1, 0, 1), (100, 32000, 1, 0, 0), (160, 32000, 0, 1, 1), (224, 152064, 1, 0, 1), (256, 152064, 0, 1, 1), (96, 32000, 0, 0, 1), (100, 32000, 0, 0, 0),
+    (128, 152064, 0, 0, 1), (160, 152064, 0, 0, 0), (300, 16384, 0, 0, 0), (4096, 16384, 1, 1, 1), (4097, 16384, 1, 1, 0), (8, 16383, 1, 1, 0), (0, 16384, 1, 1, 0)])
+def test_rows_are_shared_where_that_is_faster(rows, vocab, top_k, top_p, shared):
+    from from_scratch_inference_engine_amd import ops
+
+    lib = ops.load(build_if_missing=False)
+    assert lib.fsie_sample_shares(rows, vocab, top_k, top_p) == shared
+    assert not shared or lib.fsie_sample_workspace(rows, vocab, top_k or top_p) > 0
