@@ -371,7 +371,7 @@ struct TileCall {
 
 // Whether slices are dealt to the dies one by one.  Side by side a die reads its slices' part of X alone, which is up to 8 per cent faster (200 rows of N = 2048,
 // K = 8192 in four 74 us, 80 one by one); but a short last slice leaves its dies idle: 2,048 rows of N = 1024, K = 640, slices of 512 and 128,
-// took 42.5 us (35.3 in the kernel above, whose workgroups go to the dies in turn), 512 rows of N = 896, K = 4864 in seven 58.3, 47.6 one by one.  So where
+// took 42.6 us (36.3 in the kernel above, whose workgroups go to the dies in turn; 32.4 one by one), 512 rows of N = 896, K = 4864 in seven 58.3, 47.6 one by one.  So where
 // a die's workgroups make fewer rounds over its units one by one, and always where two slices are of different lengths.
 bool dealt_one_by_one(const TileCall& c) {
     if (c.splits == 1 || c.K == static_cast<int64_t>(c.slice) * c.splits) return false;
