@@ -243,20 +243,21 @@ int launch_shape(int tile, const Call& c) {
 // holds; a second round of 128 x 128 was up to 1.36 of the library's time and is not taken), the weights from HBM at 6.7 to 9 TB/s more; no less than the
 // eight dies' reads of x take; a whole product's bytes or the slices' sums here and in the norm at 3 TB/s.  It has to be no more than the library's 8.3 us, 1.64 PFLOP/s,
 // weights at 3 TB/s and x at 2.2, the best fit of what it took with weights from HBM (slices: 0.95 of that and the norm's reading).
-// Measured with weights from HBM at 2,241 sizes that it takes, 17 to 4,096 rows of 0.02 to 142 MB, it is at a median of 0.7 of the library's time; 56 are beyond 1.02,
+// Measured with weights from HBM at 2,241 sizes that it takes, 17 to 4,096 rows of 0.02 to 53 MB for the most part, it is at a median of 0.7 of the library's time; 56 are beyond 1.02,
 // of which 100 rows of N = K = 4096 1.10, 385 of N = 6144, K = 4096 1.17, 1,009 of N = 160, K = 3072 1.21 (this / the library, us: 17 rows of
 // N = K = 768 5.1 / 5.0, 64 of them 5.2 / 7.0, 64 of N = 512, K = 896 5.0 / 7.7, 1,375 of N = 1152,
 // K = 896 7.5 / 11.3, 512 of N = 4608, K = 3584 28.9 / 33.3, 1,000 of N = K = 3584 30.4 / 36.9, 2,048 of N = 2048, K = 8192 67.7 / 75.5, 256 of N = 3072, K = 1024 6.9 / 11.9; with
 // the norm, 96 rows of N = 896, K = 4864 in seven slices 9.2 / 15.4, 96 of N = 2048, K = 8192 in four 16.3 / 24.0).  What it leaves out besides:
-// - beyond kBeyond, where the estimate tells nothing (129 rows of N = K = 8192 66.6 / 46.4, 384 79.9 / 62.1, 96 of N = 16384, K = 2048 22.6 / 20.8), all but slices
-//   of a K longer than N for up to 256 rows (N = 4096, K = 14336 0.44 to 0.79 of the library's time, N = 5120, K = 13824 0.49 to 0.93) and tiles of 128 x 128 that leave few units
-//   idle, K up to 4096 (129 to 256 rows of N = 16384, K = 2048 0.87 to 0.91, of N = 14336, K = 4096 0.88 to 1.00);
+// - beyond kBeyond, where the estimate tells nothing (129 rows of N = K = 8192 66.6 / 46.4, 384 79.9 / 62.1), all but slices
+//   of a K no shorter than N for up to 512 rows (N = 4096, K = 14336 0.44 to 0.79 of the library's time, 0.95 to 1.06 from 300 rows on; N = 5120, K = 13824 0.49 to 0.97 and 1.06) and, from 129
+//   rows on, tiles of 128 x 128 that leave few units idle, K up to 8192, 6144 beyond 256 rows (N = 16384, K = 5120 0.90 to 1.01, N = 14336, K = 8192 0.87 to 1.04): 74 sizes,
+//   median 0.90, at most 1.06 (of 53 to 80 MB 170 sizes, median 0.93, 41 beyond 1.02, at most 1.25, 129 rows of N = 8192, K = 4096);
 // - slices of more than 8,192 rows of W (65 rows of N = 10240, K = 2048 and the norm 59.9 / 50.3).
 // 129 to 159 rows of N above 6,400 to 10,240 and K from 2048, where the library is at its best and a third of these tiles' rows are none, are taken all the same
 // (N = 8192, K = 2048 18.3 / 15.9, N = 10240 19.9 / 17.7, N = 7168, K = 3072 24.2 / 22.1; with K = 1536 or N = 6144 0.72): such portions of a prompt are bound by the
 // host, for which the library's call is 21 us and the bias behind it a launch more, this one 13 (Romepel, 9 layers, prompts of 129 to 159 tokens 1.29 ms, 1.43 so).
 // The dies' reads of x: 1,845 rows of N = 512, K = 6656 33.7 / 29.4, 2,284 of N = 432, K = 11776 57.6 / 49.6, which the steps alone put at 22.8 and 37.7.
-constexpr double kBeyond = 53e6;   // bytes of weights
+constexpr double kBeyond = 80e6;   // bytes of weights
 constexpr double kDiesRead = 6.5e6;  // bytes a us of x by all dies
 
 extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int units) {
@@ -269,7 +270,7 @@ extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int un
     const double weights = 2.0 * N * static_cast<double>(K), flops = 2.0 * M * static_cast<double>(N) * K;
     const double rows_bytes = 2.0 * M * static_cast<double>(K);
     const bool large = weights > kBeyond;
-    if (large && (result == kSums ? M > 256 || K <= N : M <= 128 || K > 4096)) return -1;
+    if (large && (result == kSums ? M > 512 || K < N : M <= 128 || K > (M <= 256 ? 8192 : 6144))) return -1;
     if (result == kSums && N > 8192) return -1;
     const double whole = 4.0 * M * static_cast<double>(N) / 3e6;  // the delta in bfloat16, out and into the norm
     double best = 1e30;

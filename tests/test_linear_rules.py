@@ -146,8 +146,8 @@ def _block_plan(m, n, k, sums):
 
 
 @pytest.mark.parametrize("m, n, k, sums", [
-    (129, 8192, 8192, False), (384, 8192, 8192, False), (384, 5120, 13824, False), (96, 16384, 2048, False), (96, 27648, 5120, False), (129, 7168, 5120, False),
-    (96, 14336, 4096, True), (384, 4096, 8192, True),                                                # weights beyond what the estimate was fitted to
+    (129, 8192, 8192, False), (384, 8192, 8192, False), (384, 5120, 13824, False), (96, 27648, 5120, False), (128, 16384, 5120, False), (300, 14336, 8192, False),
+    (100, 14336, 8192, True), (600, 5120, 13824, True),                                              # weights beyond what the estimate was fitted to
     (1845, 512, 6656, False), (2284, 432, 11776, False),                                             # x that every die reads
     (65, 10240, 2048, True),                                                                          # slices of more rows than the norm adds up quickly
     (200, 896, 900, False), (200, 900, 896, False), (0, 896, 896, False), (16 << 20, 896, 64, False), (200, 16 << 20, 64, False)])
@@ -157,7 +157,7 @@ def test_small_tiles_leave_to_the_library(m, n, k, sums):
 
 @pytest.mark.parametrize("m, n, k, sums, plan", [
     (17, 768, 768, False, (0, 1)), (64, 512, 896, False, (3, 1)), (160, 8192, 2048, False, (1, 1)), (136, 6144, 4096, False, (1, 1)), (129, 8192, 2048, False, (1, 1)), (1375, 1152, 896, False, (1, 1)),
-    (256, 16384, 2048, False, (2, 1)), (96, 896, 4864, True, (3, 7)), (192, 4096, 14336, True, (2, 4)), (1000, 3584, 3584, False, (2, 1))])
+    (256, 16384, 2048, False, (2, 1)), (200, 16384, 5120, False, (2, 1)), (200, 16384, 8192, False, (2, 1)), (224, 8192, 8192, True, (2, 2)), (96, 896, 4864, True, (3, 7)), (192, 4096, 14336, True, (2, 4)), (1000, 3584, 3584, False, (2, 1))])
 def test_small_tiles_take(m, n, k, sums, plan):
     got = _block_plan(m, n, k, sums)
     assert (got % 256, got // 256) == plan
