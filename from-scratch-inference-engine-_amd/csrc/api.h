@@ -201,6 +201,11 @@ int fsie_gemm_mfma_fp32(const float* x, const float* w, const float* bias, float
                         hipStream_t stream);
 // The same as partial sums [splits][M][N] of slices of K.
 int fsie_gemm_mfma_fp32_sums(const float* x, const float* w, float* y, int M, int N, int K, int splits, hipStream_t stream);
+// The same for up to 64 rows from a copy of w in the order of the instruction's operands (fsie_fragment_order of it as [N, 2 K] values of 16 bits), K a
+// multiple of 16.  result: 0 whole, 1 gate and up rows in turn, 2 partial sums or whole.  plan: waves + 256 * slices of K, -1: the products above.
+int fsie_gemm_fp32_stream_plan(int M, int N, int K, int result);
+int fsie_gemm_fp32_stream(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int gated, int plan, int act,
+                          float limit, float slope, hipStream_t stream);
 // The same for any number of rows (prompts); splits > 1: y = partial sums [splits][M][N] of slices of K, no bias.
 int fsie_gemm_fp32_tile(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int splits,
                         hipStream_t stream);

@@ -483,6 +483,38 @@ def gemm_fp32_gated(x: torch.Tensor, weight: torch.Tensor, act="silu") -> torch.
     return out
 
 
+GEMM_FP32_WHOLE, GEMM_FP32_GATED, GEMM_FP32_SUMS = 0, 1, 2
+
+
+@lru_cache(maxsize=4096)
+def gemm_fp32_stream_plan(m: int, n: int, k: int, result: int) -> Optional[int]:
+    """How ``gemm_fp32_stream`` takes ``m`` rows (GEMM_FP32_WHOLE, GEMM_FP32_GATED, or GEMM_FP32_SUMS: in slices of K or whole); None where the
+    kernels that read rows of the weight are faster or this one does not take the sizes."""
+    plan = int(load().fsie_gemm_fp32_stream_plan(m, n, k, result))
+    return None if plan < 0 else plan
+
+
+def gemm_fp32_stream(x: torch.Tensor, weight: FragmentOrdered, plan: int, bias: Optional[torch.Tensor] = None, act=None) -> torch.Tensor:
+    """x [M, K] . weight [N, K]^T in true float32 for up to 64 rows, ``weight`` a ``FragmentOrdered`` copy of a float32 matrix.  ``plan``
+    (``gemm_fp32_stream_plan``): one slice of K: [M, N], with ``bias``; several: partial sums [slices, M, N].  ``act`` (a ``GateAct`` or its name): the
+    weight's rows are gate and up in turn, the result is [M, N/2]."""
+    _need(x, "gemm x", dtype=torch.float32, ndim=2)
+    m, k = x.shape
+    if not isinstance(weight, FragmentOrdered):
+        raise KernelError("gemm_fp32_stream: takes a fragment-ordered weight")
+    _need(weight.data, "gemm weight", dtype=torch.float32, ndim=1)
+    n = weight.rows
+    if weight.cols != k:
+        raise KernelError(f"gemm: weight inner size {weight.cols} does not match x's {k}")
+    if bias is not None:
+        _need(bias, "gemm bias", dtype=torch.float32, shape=(n,))
+    slices = plan >> 8
+    out = torch.empty((m, n // 2) if act is not None else (m, n) if slices == 1 else (slices, m, n), dtype=torch.float32, device=x.device)
+    args = gate_act(act).args if act is not None else (0, 0.0, 0.0)
+    check(load().fsie_gemm_fp32_stream(x.data_ptr(), weight.data.data_ptr(), _ptr(bias), out.data_ptr(), m, n, k, int(act is not None), plan, *args, _stream()))
+    return out
+
+
 _FP32_TILE_ROWS = 512  # rows of a prompt's step that the slices below are made for
 
 
@@ -580,7 +612,7 @@ class FragmentOrdered:
     fragments (``fragment_order``): the 64 16-byte units of a block of 16 rows and 32 columns lie
     together in the order of the lanes that hold them, so that a wave's load of the weight is one
     piece of 1 KB and can be a streaming load.  ``gemm_mfma_wide`` and ``gemm_mfma_wide_swiglu``
-    take it in place of the matrix."""
+    take it in place of the matrix.  Of a float32 matrix: blocks of 16 rows and 16 columns, for ``gemm_fp32_stream``."""
 
     __slots__ = ("data", "rows", "cols")
 
@@ -593,15 +625,17 @@ class FragmentOrdered:
 
 
 def fragment_order(weight: torch.Tensor) -> FragmentOrdered:
-    """The copy of ``weight`` [N, K] (bfloat16, K a multiple of 32) in fragment order; the rows that
+    """The copy of ``weight`` [N, K] (bfloat16, K a multiple of 32, or float32, K a multiple of 16) in fragment order; the rows that
     fill N up to a multiple of 16 are zeros."""
-    _need(weight, "fragment_order weight", dtype=torch.bfloat16, ndim=2)
+    wide = isinstance(weight, torch.Tensor) and weight.dtype == torch.float32
+    _need(weight, "fragment_order weight", dtype=torch.float32 if wide else torch.bfloat16, ndim=2)
     n, k = weight.shape
-    size = int(load().fsie_fragment_order_size(n, k))
+    halves = 2 * k if wide else k  # (a 16-byte unit is eight values of 16 bits or four of 32)
+    size = int(load().fsie_fragment_order_size(n, halves))
     if size <= 0:
-        raise KernelError(f"fragment_order: the inner size {k} must be a multiple of 32")
-    data = torch.empty(size, dtype=torch.bfloat16, device=weight.device)
-    check(load().fsie_fragment_order(weight.data_ptr(), data.data_ptr(), n, k, _stream()))
+        raise KernelError(f"fragment_order: the inner size {k} must be a multiple of {16 if wide else 32}")
+    data = torch.empty(size // 2 if wide else size, dtype=weight.dtype, device=weight.device)
+    check(load().fsie_fragment_order(weight.data_ptr(), data.data_ptr(), n, halves, _stream()))
     return FragmentOrdered(data, n, k)
 
 

@@ -127,6 +127,8 @@ _SIGNATURES = {
     "fsie_gemm_mfma_fp32_sums": ([_P, _P, _P, c_int, c_int, c_int, c_int, _P], c_int),
     "fsie_gemm_fp32_tile": ([_P, _P, _P, _P, c_int, c_int, c_int, c_int, _P], c_int),
     "fsie_gemm_fp32_gated": ([_P, _P, _P, c_int, c_int, c_int, c_int, c_float, c_float, _P], c_int),
+    "fsie_gemm_fp32_stream_plan": ([c_int, c_int, c_int, c_int], c_int),
+    "fsie_gemm_fp32_stream": ([_P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, _P], c_int),
     "fsie_gemm_mfma_tile_plan": ([c_int, c_int, c_int, c_int, c_int], c_int),
     "fsie_gemm_mfma_tile": ([_P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, _P], c_int),
     "fsie_sample": ([_P, c_int, c_int, _P, _P, _P, _P, _P, _P], c_int),

@@ -50,6 +50,8 @@ class Linear:
     streamed_copy_from = 8 << 20
     streamed_many_rows_from = 16 << 20
     streamed_copy_reserve = 0.25
+    # A float32 weight from this size on (where copies are made at all): 4 rows of N = K = 896, 3.2 MB, 2.7 us against 3.5; N = 1152 3.1 / 4.1
+    streamed32_copy_from = 2 << 20
 
     def __init__(self, in_features: int, out_features: int, bias: bool = False):
         self.in_features = in_features
@@ -58,6 +60,7 @@ class Linear:
         self._weight: Optional[torch.Tensor] = None
         self.bias: Optional[torch.Tensor] = None
         self.streamed = None  # the weight in fragment order (ops.FragmentOrdered), if prepare() made one
+        self.streamed32 = None  # the same of a float32 weight
         self._wide_splits: dict = {}  # tiles of rows -> slices of K (a property of the sizes alone)
         self._wide_takes: dict = {}   # (tiles, slices, gate/up) -> whether the kernel takes them from this weight
         self._many_plans: dict = {}   # (rows, result, library tuning) -> how a product of more than 16 rows is taken (of the sizes alone)
@@ -69,18 +72,30 @@ class Linear:
     @weight.setter
     def weight(self, t: Optional[torch.Tensor]) -> None:
         self._weight = t
+        self.streamed32 = None
         self.streamed = None  # a copy of the weight that was here says nothing about this one
         self._wide_takes = {}
 
     def prepare(self, copies: bool = True) -> None:
         """Called by the owning part once the weight is set.  ``copies=False``: no second copy."""
         w = self.weight
-        self.streamed = None
-        if (copies and self.streamed_copy_from is not None and w is not None and w.dtype == torch.bfloat16 and w.is_cuda
-                and w.numel() * 2 >= self.streamed_copy_from and ops.gemm_mfma_wide_splits_ok(self.in_features, 1)):
-            free, total = torch.cuda.mem_get_info(w.device)
-            if free - w.numel() * 2 >= self.streamed_copy_reserve * total:
+        self.streamed = self.streamed32 = None
+        if not copies or self.streamed_copy_from is None or w is None or not w.is_cuda:
+            return
+        size = w.numel() * w.element_size()
+        if w.dtype == torch.bfloat16:
+            wanted = size >= self.streamed_copy_from and ops.gemm_mfma_wide_splits_ok(self.in_features, 1)
+        else:
+            wanted = (w.dtype == torch.float32 and size >= self.streamed32_copy_from and w.is_contiguous() and w.data_ptr() % 16 == 0
+                      and ops.gemm_fp32_stream_plan(4, self.out_features, self.in_features, ops.GEMM_FP32_SUMS) is not None)
+        if not wanted:
+            return
+        free, total = torch.cuda.mem_get_info(w.device)
+        if free - size >= self.streamed_copy_reserve * total:
+            if w.dtype == torch.bfloat16:
                 self.streamed = ops.fragment_order(w)
+            else:
+                self.streamed32 = ops.fragment_order(w)
 
     def kernel_reads(self, x: torch.Tensor) -> bool:
         """Whether the engine's 16-byte loads can read ``x`` and the weight as they lie: rows without gaps, on 16 bytes.
@@ -95,12 +110,17 @@ class Linear:
 
     def drop_copy(self) -> int:
         """Forget the fragment-ordered copy (the products then read rows); returns its bytes."""
-        if self.streamed is None:
-            return 0
-        freed = self.streamed.data.numel() * self.streamed.data.element_size()
-        self.streamed = None
+        freed = sum(c.data.numel() * c.data.element_size() for c in (self.streamed, self.streamed32) if c is not None)
+        self.streamed = self.streamed32 = None
         self._wide_takes = {}
         return freed
+
+    def plan32(self, x: torch.Tensor, result: int) -> Optional[int]:
+        """How the float32 kernel of the fragment-ordered copy takes ``x`` (``ops.gemm_fp32_stream``), or None."""
+        m = x.shape[0]
+        if self.streamed32 is None or not 0 < m <= GEMM_MFMA_SKINNY_MAX_M or not self.float32_on_matrix_cores or not self.kernel_reads(x):
+            return None
+        return ops.gemm_fp32_stream_plan(m, self.out_features, self.in_features, result)
 
     def copy_for(self, m: int):
         """The fragment-ordered copy, if there is one that products of ``m`` rows read."""
@@ -122,6 +142,9 @@ class Linear:
         if m > GEMM_MFMA_WIDE_MAX_M and out_dtype is None and x.dtype == torch.bfloat16 and not (self.in_features % 8 or self.out_features % 8):
             return self._many_rows(x, bias)
         if x.dtype == torch.float32:
+            plan = self.plan32(x, ops.GEMM_FP32_WHOLE) if out_dtype in (None, x.dtype) else None
+            if plan is not None:
+                return ops.gemm_fp32_stream(x, self.streamed32, plan, bias)
             if self.float32_on_matrix_cores and 2 < m <= GEMM_MFMA_SKINNY_MAX_M and self.in_features % 4 == 0:
                 # decoding in the 32-bit path: W streams once into true float32 matrix instructions
                 # (several times faster than the vector kernels from 8 rows on, no faster at one or two)
@@ -213,6 +236,10 @@ class Linear:
         m = x.shape[0]
         if x.dtype == torch.float32:
             # the 32-bit path: slices of K where the rows of W alone (or a prompt's tiles) leave the chip idle
+            plan = self.plan32(x, ops.GEMM_FP32_SUMS)
+            if plan is not None:
+                y = ops.gemm_fp32_stream(x, self.streamed32, plan)
+                return y if y.ndim == 3 else y.unsqueeze(0)
             if not self.float32_on_matrix_cores or m <= 2 or self.in_features % 4:
                 return None
             if m <= GEMM_MFMA_SKINNY_MAX_M:

@@ -86,6 +86,8 @@ class SwiGLU(FeedForward):
             act = ops.gemm_mfma_wide_swiglu(x, self.gate_up.weight, act=self._gate_act)
         elif x.dtype == torch.bfloat16 and m <= GEMM_MFMA_SKINNY_BEST_M and self.hidden_size % 8 == 0:
             act = ops.gemm_mfma_skinny_gated(x, self.gate_up.weight, self._gate_act)
+        elif x.dtype == torch.float32 and self.gate_up.plan32(x, ops.GEMM_FP32_GATED) is not None:
+            act = ops.gemm_fp32_stream(x, self.gate_up.streamed32, self.gate_up.plan32(x, ops.GEMM_FP32_GATED), act=self._gate_act)
         elif x.dtype == torch.float32 and self.gate_up.takes_f32_matrix(x):
             act = ops.gemm_fp32_gated(x, self.gate_up.weight, self._gate_act)
         else:
