@@ -17,6 +17,11 @@
 // of 256 39 / 12.6; one of 100 keys 16.0 / 6.3, 24.0 / 7.7, 60 / 14.1; 32 of 700 26.9 / 12.4, 68 / 26.9, 56 / 25.8; a prompt of 300
 // tokens 54 / 14.9, 94 / 30, 137 / 38, of 1,000 202 / 59, 562 / 155, 657 / 202.
 //
+// QKV: steps of one token a request take q, k and v as the partial sums that the product in slices of K leaves, as the bfloat16 kernel's
+// variant does: a workgroup adds up the heads that it needs, with the bias, turns queries and key by the step's table, takes the new key and value from
+// there where its keys end with them, and one workgroup a kv head writes them into the pools.  That spares the launch between product and
+// attention (3.3 us of a layer and step; four requests of the 0.5B shape FIGURES).  The bits are those of the kernels one after the other.
+//
 // More workgroups than units: four waves each whatever the head size, except over the tiles of long prompts (see launch).
 #include "common.h"
 #include "api.h"
@@ -35,6 +40,17 @@ constexpr int f32_waves() {
     return HDT <= 4 ? 16 : (HDT <= 8 ? 8 : 4);  // registers a wave grow with the head size
 }
 
+// What the QKV variant reads and writes beside the kernel's other operands.
+struct F32Sums {
+    const float *sums, *bias, *cos_sin;  // [n_parts][tokens][width]; [width] or null; [tokens][head_dim / 2] pairs of cosine and sine, or null: nothing is turned
+    const int32_t* slots;                // [tokens]: where a token's key and value go (negative, or not below pool_slots: nowhere)
+    float *k_out, *v_out;                // the pools again, to write
+    int64_t part_stride, pool_slots;
+    int n_parts, width;
+};
+
+constexpr int kSumsHdt = 8;  // the QKV variant: heads of up to 128 (its wider ones would have no registers left)
+
 struct F32Call {
     const float *q, *k_pool, *v_pool;
     int64_t q_stride;
@@ -43,16 +59,26 @@ struct F32Call {
     int n_items, max_pages, n_heads, n_kv, page_size, window, all_waves;
     float scale, softcap;
     const float *sinks, *slopes, *row_scale;
+    F32Sums sums;  // sums null: queries from q, keys and values in the pools already
 };
 
-template <int HDT, int W>
+// A pair turned by (c, s), with the roundings of the kernel that turns and writes by itself (rope_kv.hip).
+__device__ __forceinline__ float turned(float first, float second, float c, float s, bool is_second) {
+    return is_second ? __builtin_fmaf(first, s, second * c) : __builtin_fmaf(first, c, -(second * s));
+}
+
+template <int HDT, int W, bool QKV>
 __global__ __launch_bounds__(64 * W) void attention_f32_kernel(
     const int32_t* __restrict__ items, const int32_t* __restrict__ block_tables, int max_pages, int page_size, uint32_t page_magic,
     int n_kv, const float* __restrict__ k_pool, const float* __restrict__ v_pool, const float* __restrict__ q, int64_t q_stride,
     float* __restrict__ out, float* __restrict__ partials, int n_heads, int group, int gh, int window, float scale, float softcap,
-    const float* __restrict__ sinks, const float* __restrict__ slopes, const float* __restrict__ row_scale) {
+    const float* __restrict__ sinks, const float* __restrict__ slopes, const float* __restrict__ row_scale, F32Sums f) {
     constexpr int HD = HDT * 16, MW = (W + 3) / 4 * 4;
     __shared__ floatx4 s_o[W * HDT * 64];
+    // QKV: up to 16 heads of queries, the key and the value (a row four floats longer than a head: 16 rows' reads fall into different banks); the table's pairs
+    constexpr int RS = HD + 4;
+    __shared__ __align__(16) float s_row[QKV ? 18 * RS : 1];
+    __shared__ __align__(16) float2 s_cs[QKV ? HD / 2 : 1];
     __shared__ float s_m[16][MW + 4], s_l[16][MW + 4];  // [column][wave]: a lane reads its column's waves four at a time
 
     typedef int ItemInts __attribute__((ext_vector_type(8), aligned(4)));
@@ -117,12 +143,67 @@ __global__ __launch_bounds__(64 * W) void attention_f32_kernel(
     const bool any = kb_begin < kb_end;
     Asked asked;
     if (any) ask(kb_begin, asked);
+    Block b;
+    // QKV: the heads' sums, all that are asked for at once and before the first keys; a thread has quads of columns of the heads this workgroup needs
+    constexpr int NJ = QKV ? (18 * HD / 4 + 64 * W - 1) / (64 * W) : 1, PC = NJ <= 3 ? 8 : 4;
+    const bool owner = QKV && pos0 >= key_begin && pos0 < key_end;  // the item whose keys end with the new one
+    if constexpr (QKV) {
+        floatx4 part[NJ][PC], bias_of[NJ];
+        float2 angle = float2{1.f, 0.f};
+        const float* at[NJ];
+        const int n_cols = (gh_here + 2) * HD, q_dim = n_heads * HD, kv_dim = n_kv * HD;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int i = (static_cast<int>(threadIdx.x) + j * 64 * W) * 4, ic = i < n_cols ? i : 0;
+            const int seg = ic / HD, d = ic - seg * HD;
+            const int col = seg < gh_here ? (h_base + seg) * HD + d : q_dim + (seg - gh_here) * kv_dim + kvh * HD + d;
+            at[j] = f.sums + static_cast<int64_t>(q_row0) * f.width + col;
+#pragma unroll
+            for (int u = 0; u < PC; ++u) part[j][u] = *reinterpret_cast<const floatx4*>(at[j] + min(u, f.n_parts - 1) * f.part_stride);
+            bias_of[j] = *reinterpret_cast<const floatx4*>(f.bias ? f.bias + col : at[j]);
+        }
+        const float2* table_row = reinterpret_cast<const float2*>(f.cos_sin) + static_cast<int64_t>(q_row0) * (HD / 2);
+        if (f.cos_sin) angle = table_row[min(static_cast<int>(threadIdx.x), HD / 2 - 1)];
+        if (any) load(asked, b);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int i = (static_cast<int>(threadIdx.x) + j * 64 * W) * 4;
+            floatx4 a = part[j][0];
+#pragma unroll
+            for (int u = 1; u < PC; ++u)
+                if (u < f.n_parts) a += part[j][u];
+            for (int s = PC; s < f.n_parts; ++s) a += *reinterpret_cast<const floatx4*>(at[j] + s * f.part_stride);
+            if (f.bias) a += bias_of[j];
+            if (i < n_cols) *reinterpret_cast<floatx4*>(s_row + i / HD * RS + i % HD) = a;
+        }
+        // (four waves, two heads' halves of up to 128 pairs: a thread a pair)
+        if (static_cast<int>(threadIdx.x) < HD / 2) s_cs[threadIdx.x] = angle;
+        __syncthreads();
+    }
+    // four values of a head from d on, turned
+    auto head_values = [&](int seg, int d, bool turn) -> floatx4 {
+        const float* head = s_row + seg * RS;
+        const floatx4 mine = *reinterpret_cast<const floatx4*>(head + d);
+        if (!turn) return mine;
+        const bool second = d >= HD / 2;
+        const int i = second ? d - HD / 2 : d;
+        const floatx4 other = *reinterpret_cast<const floatx4*>(head + (second ? i : i + HD / 2));
+        floatx4 r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = turned(second ? other[e] : mine[e], second ? mine[e] : other[e], s_cs[i + e].x, s_cs[i + e].y, second);
+        return r;
+    };
     // this lane's query row; a row that does not exist reads the item's first one and is masked
     const int tq = c / gh, hh = c - tq * gh;
     const bool row_ok = tq < n_q && hh < gh_here;
     const int head = h_base + (row_ok ? hh : 0), row = q_row0 + (row_ok ? tq : 0), pos = pos0 + tq;
     floatx4 qf[HDT];
-    if (W < 16 || any) {  // (of sixteen waves most have no key where items are short, and read nothing; eight are slower with the question)
+    if constexpr (QKV) {
+        if (any) {
+#pragma unroll
+            for (int j = 0; j < HDT; ++j) qf[j] = head_values(row_ok ? hh : 0, 16 * j + 4 * G, f.cos_sin != nullptr);
+        }
+    } else if (W < 16 || any) {  // (of sixteen waves most have no key where items are short, and read nothing; eight are slower with the question)
         const float* qp = q + static_cast<int64_t>(row) * q_stride + static_cast<int64_t>(head) * HD + 4 * G;
 #pragma unroll
         for (int j = 0; j < HDT; ++j) qf[j] = *reinterpret_cast<const floatx4*>(qp + 16 * j);
@@ -134,9 +215,36 @@ __global__ __launch_bounds__(64 * W) void attention_f32_kernel(
     floatx4 acc[HDT];
 #pragma unroll
     for (int j = 0; j < HDT; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    Block b;
-    if (any) load(asked, b);
+    if constexpr (QKV) {
+        // the new key and value into the pools, by the last wave
+        if (owner && chunk == 0 && wave == W - 1) {
+            const int slot = f.slots[q_row0];
+            if (slot >= 0 && slot < f.pool_slots) {
+                const int page = slot / page_size, off = slot - page * page_size;
+                float* kd = f.k_out + page * page_stride + kv_base + static_cast<int64_t>(off) * HD;
+                float* vd = f.v_out + page * page_stride + kv_base + off;
+                for (int d = 4 * lane; d < HD; d += 256) *reinterpret_cast<floatx4*>(kd + d) = head_values(gh_here, d, f.cos_sin != nullptr);
+                for (int d = lane; d < HD; d += 64) vd[static_cast<int64_t>(d) * page_size] = s_row[(gh_here + 1) * RS + d];
+            }
+        }
+    } else {
+        if (any) load(asked, b);
+    }
     for (int kb = kb_begin; kb < kb_end;) {
+        if constexpr (QKV) {
+            // (what the pools hold at the new key's place is not looked at)
+            if (owner && kb >= kb_first && pos0 >= kb && pos0 < kb + 16) {
+                const int new_i = pos0 - (kb + 4 * G);
+                const float* value = s_row + (gh_here + 1) * RS + c;
+#pragma unroll
+                for (int j = 0; j < HDT; ++j) {
+                    const floatx4 key = head_values(gh_here, 16 * j + 4 * G, f.cos_sin != nullptr);
+                    if (kb + c == pos0) b.k[j] = key;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) b.v[j][i] = i == new_i ? value[16 * j] : b.v[j][i];
+                }
+            }
+        }
         floatx4 st{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < HDT; ++j)
@@ -271,10 +379,15 @@ __global__ __launch_bounds__(64 * W) void attention_f32_kernel(
 
 template <int HDT, int W>
 void launch_waves(const F32Call& a, dim3 grid, int group, int gh, hipStream_t stream) {
-    attention_f32_kernel<HDT, W><<<grid, 64 * W, 0, stream>>>(
-        a.items, a.block_tables, a.max_pages, a.page_size, 0xFFFFFFFFu / static_cast<uint32_t>(a.page_size) + 1u, a.n_kv, a.k_pool,
-        a.v_pool, a.q, a.q_stride, a.out, a.partials, a.n_heads, group, gh, a.window, a.scale, a.softcap, a.sinks, a.slopes,
-        a.row_scale);
+    const uint32_t page_magic = 0xFFFFFFFFu / static_cast<uint32_t>(a.page_size) + 1u;
+    if constexpr (HDT <= kSumsHdt)
+        if (a.sums.sums)
+            return attention_f32_kernel<HDT, W, true><<<grid, 64 * W, 0, stream>>>(
+            a.items, a.block_tables, a.max_pages, a.page_size, page_magic, a.n_kv, a.k_pool, a.v_pool, nullptr, 0, a.out, a.partials, a.n_heads, group,
+                gh, a.window, a.scale, 0.f, nullptr, a.slopes, a.row_scale, a.sums);
+    attention_f32_kernel<HDT, W, false><<<grid, 64 * W, 0, stream>>>(
+            a.items, a.block_tables, a.max_pages, a.page_size, page_magic, a.n_kv, a.k_pool, a.v_pool, a.q, a.q_stride, a.out, a.partials, a.n_heads, group,
+            gh, a.window, a.scale, a.softcap, a.sinks, a.slopes, a.row_scale, a.sums);
 }
 
 template <int HDT>
@@ -333,5 +446,33 @@ extern "C" int fsie_attention_f32(const float* q, int64_t q_stride, const float*
     a.out = out, a.partials = partials, a.n_items = n_items, a.max_pages = max_pages, a.n_heads = n_heads, a.n_kv = n_kv;
     a.page_size = page_size, a.window = window, a.scale = scale, a.softcap = softcap;
     a.sinks = sinks, a.slopes = slopes, a.row_scale = row_scale, a.all_waves = all_waves;
+    return launch_from<1>(head_dim / 16, a, stream);
+}
+
+// The same for a step of one token a request (every item has one query row a head), from the q/k/v product's partial sums [n_parts][n_tokens][(n_heads + 2 n_kv) head_dim]:
+// adds them up, adds `bias` (or null), turns queries and keys by cos_sin [n_tokens][head_dim / 2][2] (or null: not), takes the new key and value from there and
+// writes them to slots[t] of the pools (negative, or not below pool_slots: not).
+extern "C" int fsie_attention_f32_qkv(const float* sums, int n_parts, int n_tokens, const float* bias, const float* cos_sin, const int32_t* slots,
+                                      float* k_pool, float* v_pool, int64_t pool_slots, const int32_t* block_tables, int max_pages,
+                                      const int32_t* items, int n_items, float* out, float* partials, int n_heads, int n_kv, int head_dim,
+                                      int page_size, int window, float scale, const float* slopes, const float* row_scale, hipStream_t stream) {
+    FSIE_REQUIRE(n_items >= 0 && n_heads > 0 && n_kv > 0 && n_heads % n_kv == 0,
+                 "attention_f32_qkv: heads %d must be a positive multiple of kv heads %d", n_heads, n_kv);
+    FSIE_REQUIRE(fsie_attention_f32_ok(head_dim, page_size) && head_dim <= 16 * kSumsHdt,
+                 "attention_f32_qkv: head_dim %d must be a multiple of 16 up to 128 and page_size %d of 4", head_dim, page_size);
+    FSIE_REQUIRE(max_pages > 0 && (static_cast<int64_t>(max_pages) + 8) * page_size * page_size < (int64_t{1} << 32),
+                 "attention_f32_qkv: %d pages of %d keys are more than the kernel can address", max_pages, page_size);
+    FSIE_REQUIRE(n_parts >= 1 && n_parts <= FSIE_GEMM_MAX_SPLITS && n_tokens >= 1 && pool_slots >= 0, "attention_f32_qkv: bad sizes parts=%d T=%d", n_parts, n_tokens);
+    FSIE_REQUIRE(sums && slots && k_pool && v_pool && block_tables && items && out, "attention_f32_qkv: missing operand");
+    FSIE_REQUIRE(reinterpret_cast<uintptr_t>(sums) % 16 == 0 && reinterpret_cast<uintptr_t>(bias) % 16 == 0 && reinterpret_cast<uintptr_t>(cos_sin) % 8 == 0 &&
+                     reinterpret_cast<uintptr_t>(k_pool) % 16 == 0 && reinterpret_cast<uintptr_t>(v_pool) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0,
+                 "attention_f32_qkv: sums, bias, the pools and the result must be 16-byte aligned, the cosines and sines 8-byte");
+    if (n_items == 0) return 0;
+    F32Call a{};
+    a.k_pool = k_pool, a.v_pool = v_pool, a.block_tables = block_tables, a.items = items;
+    a.out = out, a.partials = partials, a.n_items = n_items, a.max_pages = max_pages, a.n_heads = n_heads, a.n_kv = n_kv;
+    a.page_size = page_size, a.window = window, a.scale = scale, a.slopes = slopes, a.row_scale = row_scale;
+    a.sums = F32Sums{sums, bias, cos_sin, slots, k_pool, v_pool, 0, pool_slots, n_parts, (n_heads + 2 * n_kv) * head_dim};
+    a.sums.part_stride = static_cast<int64_t>(n_tokens) * a.sums.width;
     return launch_from<1>(head_dim / 16, a, stream);
 }

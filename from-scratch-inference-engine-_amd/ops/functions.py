@@ -1090,6 +1090,11 @@ def attention_mfma_qkv_ok(head_dim: int, page_size: int) -> bool:
     return bool(load().fsie_attention_mfma_qkv_ok(head_dim, page_size))
 
 
+def attention_f32_qkv_ok(head_dim: int, page_size: int) -> bool:
+    """The same of float32 storage (``attention_qkv`` takes both)."""
+    return 0 < head_dim <= 128 and head_dim % 16 == 0 and page_size > 0 and page_size % 4 == 0
+
+
 def attention_mfma_qkv(sums: torch.Tensor, bias: Optional[torch.Tensor], cos_sin: Optional[torch.Tensor], slots: torch.Tensor,
                        k_pool: torch.Tensor, v_pool: torch.Tensor, block_tables: torch.Tensor, items: torch.Tensor,
                        n_items: int, out: torch.Tensor, partials: Optional[torch.Tensor], n_heads: int, n_kv: int,
@@ -1098,7 +1103,8 @@ def attention_mfma_qkv(sums: torch.Tensor, bias: Optional[torch.Tensor], cos_sin
     """Attention of a step of one token a request (every item: one query row a head) from the q/k/v
     product's float32 partial sums [S, T, (heads + 2 kv heads) head_dim]: the kernel adds them up, adds
     ``bias``, rotates queries and keys by ``cos_sin`` [T, head_dim / 2, 2] (None: no rotation), scores each request's new key
-    from registers and writes it and the value to ``slots[t]`` of the pools (negative: nowhere)."""
+    from registers and writes it and the value to ``slots[t]`` of the pools (negative: nowhere).  Pools and result in bfloat16, or all in
+    float32 (``attention_f32_qkv_ok``; ``waves`` is then the kernel's own choice)."""
     width = (n_heads + 2 * n_kv) * head_dim
     _need(sums, "q/k/v sums", dtype=torch.float32, ndim=3)
     n_parts, t = sums.shape[0], sums.shape[1]
@@ -1111,19 +1117,27 @@ def attention_mfma_qkv(sums: torch.Tensor, bias: Optional[torch.Tensor], cos_sin
         if cos_sin.numel() != t * head_dim:
             raise KernelError(f"cos_sin: {cos_sin.numel()} values for {t} tokens of head_dim {head_dim}")
     _need(slots, "slots", dtype=torch.int32, shape=(t,))
-    _need(k_pool, "k_pool", dtype=torch.bfloat16, ndim=4)
-    _need(v_pool, "v_pool", dtype=torch.bfloat16,
+    wide = isinstance(k_pool, torch.Tensor) and k_pool.dtype == torch.float32
+    dtype = torch.float32 if wide else torch.bfloat16
+    _need(k_pool, "k_pool", dtype=dtype, ndim=4)
+    _need(v_pool, "v_pool", dtype=dtype,
           shape=(k_pool.shape[0], k_pool.shape[1], k_pool.shape[3], k_pool.shape[2]))
     _need(block_tables, "block_tables", dtype=torch.int32, ndim=2)
     _need(items, "attention items", dtype=torch.int32, ndim=2)
     if items.shape[1] != ATTN_ITEM_INTS or items.shape[0] < n_items:
         raise KernelError(f"attention items: shape {tuple(items.shape)} does not hold {n_items} items")
-    _need(out, "attention out", dtype=torch.bfloat16, shape=(t, n_heads * head_dim))
+    _need(out, "attention out", dtype=dtype, shape=(t, n_heads * head_dim))
     pages, kvh, page_size, hd = k_pool.shape
     if kvh != n_kv or hd != head_dim:
         raise KernelError(f"k_pool: shape {tuple(k_pool.shape)} does not match kv heads {n_kv}, head_dim {head_dim}")
     if partials is not None:
         _need(partials, "attention partials", dtype=torch.float32, ndim=1)
+    if wide:
+        check(load().fsie_attention_f32_qkv(sums.data_ptr(), n_parts, t, _ptr(bias), _ptr(cos_sin), slots.data_ptr(), k_pool.data_ptr(),
+                                            v_pool.data_ptr(), pages * page_size, block_tables.data_ptr(), block_tables.shape[1],
+                                            items.data_ptr(), n_items, out.data_ptr(), _ptr(partials), n_heads, n_kv, head_dim, page_size,
+                                            int(window or 0), float(scale), *_bias_ptrs(slopes, row_scale, n_heads, t), _stream()))
+        return out
     check(load().fsie_attention_mfma_qkv(sums.data_ptr(), n_parts, t, _ptr(bias), _ptr(cos_sin), slots.data_ptr(),
                                          k_pool.data_ptr(), v_pool.data_ptr(), pages * page_size,
                                          block_tables.data_ptr(), block_tables.shape[1], items.data_ptr(), n_items,

@@ -803,9 +803,12 @@ class GQAttention(Mixer):
 
     def _sums_will_do(self, dtype, cache, plan, fuse: bool) -> bool:
         """Whether attention of this step may take the q/k/v product as partial sums: one token a request."""
-        return (self.finish_qkv_in_attention and self.sink is None and not self.keep_first and self.softcap is None and fuse and cache.writes and plan.mfma and plan.single
-                and plan.n_small and not plan.n_large and not plan.n_long and dtype == torch.bfloat16
-                and ops.attention_mfma_qkv_ok(self.head_dim, cache.page_size))
+        if not (self.finish_qkv_in_attention and self.sink is None and not self.keep_first and self.softcap is None and fuse and cache.writes and plan.single
+                and plan.n_small and not plan.n_large and not plan.n_long):
+            return False
+        if dtype == torch.float32:
+            return not plan.mfma and not getattr(plan, "all_waves", False) and cache.k_pool.dtype == torch.float32 and ops.attention_f32_qkv_ok(self.head_dim, cache.page_size)
+        return plan.mfma and dtype == torch.bfloat16 and ops.attention_mfma_qkv_ok(self.head_dim, cache.page_size)
 
     def takes_pending_norm(self, m: int, n_parts: int, ctx, cache) -> bool:
         qkv = self.qkv
@@ -824,6 +827,8 @@ class GQAttention(Mixer):
             n_parts = 0 if x.sums is None else len(x.sums)
             splits = ops.gemm_normed_takes(x.shape[0], self.qkv.out_features, self.qkv.in_features, ops.GEMM_STREAM_SUMS, n_parts)
             sums = ops.gemm_mfma_normed(x.residual, x.sums, x.weight, x.eps, x.stream, weight, ops.GEMM_STREAM_SUMS, splits=splits)
+        elif x.dtype == torch.float32:
+            sums = self.qkv.sums32(x)
         else:
             sums = self.qkv.partial_sums(x, few_rows=True, long_slices=self.wants_long_slices)
         if sums is None:

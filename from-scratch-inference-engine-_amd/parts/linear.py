@@ -115,6 +115,14 @@ class Linear:
         self._wide_takes = {}
         return freed
 
+    def sums32(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """x . W^T (no bias) of float32 rows as partial sums [S, T, N] (S = 1 where the product is better left whole) from the copy, or None."""
+        plan = self.plan32(x, ops.GEMM_FP32_SUMS)
+        if plan is None:
+            return None
+        y = ops.gemm_fp32_stream(x, self.streamed32, plan)
+        return y if y.ndim == 3 else y.unsqueeze(0)
+
     def plan32(self, x: torch.Tensor, result: int) -> Optional[int]:
         """How the float32 kernel of the fragment-ordered copy takes ``x`` (``ops.gemm_fp32_stream``), or None."""
         m = x.shape[0]
@@ -236,10 +244,9 @@ class Linear:
         m = x.shape[0]
         if x.dtype == torch.float32:
             # the 32-bit path: slices of K where the rows of W alone (or a prompt's tiles) leave the chip idle
-            plan = self.plan32(x, ops.GEMM_FP32_SUMS)
-            if plan is not None:
-                y = ops.gemm_fp32_stream(x, self.streamed32, plan)
-                return y if y.ndim == 3 else y.unsqueeze(0)
+            sums = self.sums32(x)
+            if sums is not None:
+                return sums
             if not self.float32_on_matrix_cores or m <= 2 or self.in_features % 4:
                 return None
             if m <= GEMM_MFMA_SKINNY_MAX_M:
