@@ -328,6 +328,13 @@ int fsie_attention_mfma_qkv(const float* sums, int n_parts, int n_tokens, const 
                             const int32_t* block_tables, int max_pages, const int32_t* items, int n_items, void* out,
                             float* partials, int n_heads, int n_kv, int head_dim, int page_size, int window,
                             float scale, int waves, const float* slopes, const float* row_scale, hipStream_t stream);
+// the same with the output projection behind it (rows_of_wave: what .._rows says; 0 there: two launches are faster)
+int fsie_attention_mfma_qkv_o_rows(int n_items, int n_heads, int n_kv, int head_dim, int page_size, int o_rows, int units);
+int fsie_attention_mfma_qkv_o(const float* sums, int n_parts, int n_tokens, const float* bias, const float* cos_sin,
+                              const int32_t* slots, void* k_pool, void* v_pool, int64_t pool_slots, const int32_t* block_tables,
+                              int max_pages, const int32_t* items, int n_items, const void* o_weight, int o_rows, float* o_sums,
+                              int rows_of_wave, int n_heads, int n_kv, int head_dim, int page_size, int window, float scale,
+                              hipStream_t stream);
 int fsie_attention_mfma_lds_ok(int head_dim, int page_size);
 int fsie_attention_mfma_lds(const void* q, int64_t q_stride, const void* k_pool, const void* v_pool,
                             const int32_t* block_tables, int max_pages, const int32_t* items, const int32_t* groups,

@@ -22,4 +22,6 @@ LaunchQkvFn table_a_qkv(int hdt) {
     }
 }
 
+LaunchQkvOFn table_a_qkv_o(int hdt) { return hdt == 4 ? launch_qkv_o<4> : nullptr; }
+
 }  // namespace fsie_attn

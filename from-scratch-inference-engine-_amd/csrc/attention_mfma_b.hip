@@ -22,4 +22,6 @@ LaunchQkvFn table_b_qkv(int hdt) {
     }
 }
 
+LaunchQkvOFn table_b_qkv_o(int hdt) { return hdt == 8 ? launch_qkv_o<8> : nullptr; }
+
 }  // namespace fsie_attn

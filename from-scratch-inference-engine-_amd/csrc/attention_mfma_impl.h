@@ -41,6 +41,15 @@
 // heads it needs (its queries, and its kv head's key and value), adds the bias, rotates queries
 // and key, and the workgroup whose keys end with the new one scores it from registers and writes
 // it and its value into the pools.  That spares the launch between the product and attention.
+//
+// OROWS > 0: the same with the output projection behind it, for one or two tokens whose items are short and whole.  Such a step is
+// bound by its launches and by the chain inside each; the projection's own kernel was 3.9 us a layer, of which its chain is a trip for the weight.
+// So every workgroup makes the whole attention of a kv head (a few tens of keys, from the caches) and then multiplies the heads, rounded to
+// 16 bits in LDS, by a few rows of the projection, which it has asked for in front of the first barrier: float32 sums
+// [n_kv][tokens][o_rows], one slice a kv head, for the norm that adds them up.  One request of the 0.5B shape and 30 to 100 keys: attention and
+// projection 8.6 -> 6.8 us a layer, the step 565 -> 520; two requests 591 -> 562.  Where the workgroups are more than the units attention is made
+// in turns and the two launches are faster (the rule is fsie_attention_mfma_qkv_o_rows), and so it is with items of more waves (600
+// keys 17.3 ms for 24 steps, 16.1 cut and merged).
 #pragma once
 
 #include "common.h"
@@ -89,6 +98,11 @@ struct QkvSums {
     const float* slopes;     // [n_heads] or null: slopes[h] * (query position - key position) is taken off the (capped)
                              // scores of head h (any variant)
     const float* row_scale;  // [n_tokens] or null: a factor on all scores of a token, before the cap (any variant)
+    // the variant with the output projection: its weight [o_rows][n_heads head_dim] in rows, and the sums that it leaves [n_kv][n_tokens][o_rows]
+    const bf16_t* o_weight;
+    float* o_sums;
+    int64_t o_part_stride;   // n_tokens * o_rows
+    int o_rows;
     int group;               // heads a kv head (any variant)
     uint32_t page_magic;     // 2^32 / page_size, rounded up: a key's page by one multiplication (any variant)
 };
@@ -144,13 +158,15 @@ constexpr int kShortWaves = 4;
 // registers to spare for them); true: whatever slopes and row_scale say.
 // ONCE: values by streaming loads: where several waves walk long runs of keys, and where more workgroups than units read more than
 // the caches hold; the short items of a few workgroups are slower with them.
-template <int HDT, int NT, int MAXW, bool V16, bool QKV = false, bool BIASED = true, bool ONCE = (MAXW > kShortWaves + 1)>
+// OROWS > 0: each wave multiplies the heads of the workgroup by so many rows of the output projection (below).
+template <int HDT, int NT, int MAXW, bool V16, bool QKV = false, bool BIASED = true, bool ONCE = (MAXW > kShortWaves + 1), int OROWS = 0>
 __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW == 1 && NT > 1 ? 2 : 1))) void attention_mfma_kernel(
     const bf16_t* __restrict__ q, int64_t q_stride, const bf16_t* __restrict__ k_pool,
     const bf16_t* __restrict__ v_pool, const int32_t* __restrict__ block_tables, int max_pages,
     const int32_t* __restrict__ items, bf16_t* __restrict__ out, float* __restrict__ partials, int n_heads,
     int n_kv, int page_size, int window, float scale, int gh, QkvSums f) {
     static_assert(!QKV || (NT == 1 && HDT % 2 == 0), "the QKV variant: one query tile, head_dim a multiple of 32");
+    static_assert(OROWS == 0 || (QKV && HDT <= 8), "the output projection: behind the QKV variant, whose heads in LDS make room for the result");
     constexpr int HD = HDT * 16;
     // scores: 32-wide steps over the head dimension when head_dim is a multiple of 32, else
     // 16-wide steps throughout (the two shapes are never chained on one accumulator)
@@ -160,7 +176,7 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
     constexpr int S32A = S32 > 0 ? S32 : 1;
     constexpr int S16A = S16 > 0 ? S16 : 1;
 
-    const int32_t* item = items + static_cast<int64_t>(blockIdx.x) * FSIE_ATTN_ITEM_INTS;
+    const int32_t* item = items + static_cast<int64_t>(OROWS > 0 ? blockIdx.z : blockIdx.x) * FSIE_ATTN_ITEM_INTS;
     // (the item in one scalar load: its fields one by one are trips of their own, each behind the last one's use)
     typedef int ItemInts __attribute__((ext_vector_type(8), aligned(4)));
     static_assert(FSIE_ATTN_ITEM_INTS == 8, "an item is eight numbers");
@@ -186,7 +202,7 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
     if constexpr (QKV) new_slot = f.slots[q_row0];
 
     const int group = f.group;
-    const int kvh = blockIdx.y, chunk = blockIdx.z;
+    const int kvh = blockIdx.y, chunk = OROWS > 0 ? 0 : blockIdx.z;
     const int gh_here = min(gh, group - chunk * gh);
     const int h_base = kvh * group + chunk * gh;
     const int n_rows = n_q * gh;
@@ -237,7 +253,7 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
         const float* row = f.sums + static_cast<int64_t>(q_row0) * f.width;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            if (j * sum_threads * 4 >= n_cols) {  // (the same for the whole workgroup: no thread has such a column)
+            if (j > 0 && j * sum_threads * 4 >= n_cols) {  // (the same for the whole workgroup: no thread has such a column)
                 lds_at[j] = -1;
                 continue;
             }
@@ -261,7 +277,7 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
     auto finish_sums = [&]() {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            if (j * sum_threads * 4 >= (gh_here + 2) * HD) continue;
+            if (j > 0 && j * sum_threads * 4 >= (gh_here + 2) * HD) continue;
             float4 a{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int u = 0; u < PC; ++u)
@@ -278,6 +294,21 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
             if (i == sum_thread || !f.cos_sin) s_cs[i] = angle;  // (without a table: cosine 1, sine 0)
             else s_cs[i] = (reinterpret_cast<const float2*>(f.cos_sin) + static_cast<int64_t>(q_row0) * (HD / 2))[i];
         }
+    };
+
+    // The output projection's rows of this wave, the columns of this kv head's heads: eight values a lane and load
+    constexpr int OU = OROWS > 0 ? HDT / 2 : 1;  // loads a row (sixteen heads at most)
+    const int o_first = (static_cast<int>(blockIdx.x) * MAXW + wave) * OROWS, o_units = gh_here * (HD / 8);
+    uint4 o_w[OROWS > 0 ? OROWS : 1][OU];
+    auto issue_o = [&]() {
+#pragma unroll
+        for (int r = 0; r < OROWS; ++r) {
+            const bf16_t* w = f.o_weight + (static_cast<int64_t>(min(o_first + r, f.o_rows - 1)) * n_heads + h_base) * HD;
+#pragma unroll
+            for (int u = 0; u < OU; ++u)
+                if (u == 0 || u * 64 < o_units) o_w[r][u] = ld16_once(w + min(u * 64 + lane, o_units - 1) * 8);
+        }
+        __builtin_amdgcn_sched_barrier(0);
     };
 
     // ---- the item's queries: B operands, kept for the whole item
@@ -540,7 +571,7 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
     };
     // ... and into the pools, by a wave that has the least to do
     auto keep_new_key = [&]() {
-        if (!(owner && chunk == 0 && new_slot >= 0 && new_slot < f.pool_slots)) return;
+        if (!(owner && chunk == 0 && (OROWS == 0 || blockIdx.x == 0) && new_slot >= 0 && new_slot < f.pool_slots)) return;
         const float* kh = s_row + gh_here * RS;
         const float* vh = kh + RS;
         const int page = new_slot / page_size;
@@ -562,13 +593,17 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
         // (QKV: the reads of the sums, which come from further away than the table, go out before the
         // wait for the table)
         Asked first;
-        if (any) ask_pages(kb_begin, first);
+        // (a wave without keys asks all the same, for what lies at the start of page 0: behind a branch around these loads the compiler
+        // cannot know how many are under way, and waits for the keys where it needs the sums)
+        const bool ask = QKV || any;
+        if (ask) ask_pages(kb_begin, first);
         if constexpr (QKV) issue_sums();
-        if (any) place(first, at);
-        if (PREFETCH && any) {
+        if (ask) place(first, at);
+        if (PREFETCH && ask) {
             load_block(at, cur);
             if (!SHORT) locate(kb_begin + 32, at);
         }
+        if constexpr (OROWS > 0) issue_o();  // (behind all that attention itself waits for: a wave's loads return in order)
         if constexpr (QKV) {
             finish_sums();
             __syncthreads();
@@ -642,7 +677,7 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
             s_l1[c][wave] = l_w;
         }
         __syncthreads();
-        if (!rvalid[0]) return;
+        if (OROWS == 0 && !rvalid[0]) return;
         float m_of_run[MW], l_of_run[MW], factor[MW];
 #pragma unroll
         for (int w = 0; w < MW; w += 4) {
@@ -667,7 +702,7 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
         float inv = 1.f;
         if (partial_base < 0) {
             float whole = denom;
-            if (f.sinks && m_all != -INFINITY) whole += __builtin_amdgcn_exp2f(f.sinks[rhead[0]] * kLog2e - m_all);
+            if (!QKV && f.sinks && m_all != -INFINITY) whole += __builtin_amdgcn_exp2f(f.sinks[rhead[0]] * kLog2e - m_all);
             inv = whole > 0.f ? 1.0f / whole : 0.f;
         }
         bf16_t* o = out + (static_cast<int64_t>(q_row0 + rtok[0]) * n_heads + rhead[0]) * HD + 4 * G;
@@ -687,12 +722,49 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
 #pragma unroll
                     for (int r = 0; r < 4; ++r) a[r] = w0 + i < n_runs ? fmaf(v[i][r], factor[w0 + i], a[r]) : a[r];
             }
-            if (partial_base < 0) {
+            if constexpr (OROWS > 0) {  // (into the place of the heads in LDS, which were last read in front of the barrier)
+                if (rvalid[0])
+                    *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(s_row) + c * HD + dt * 16 + 4 * G) =
+                        uint2{pack2_bf16(a[0] * inv, a[1] * inv), pack2_bf16(a[2] * inv, a[3] * inv)};
+            } else if (partial_base < 0) {
                 *reinterpret_cast<uint2*>(o + dt * 16) = uint2{pack2_bf16(a[0] * inv, a[1] * inv), pack2_bf16(a[2] * inv, a[3] * inv)};
             } else {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) rec[dt * 16 + 4 * G + r] = a[r];
             }
+        }
+        if constexpr (OROWS > 0) {
+            __syncthreads();
+            float sum[OROWS];
+#pragma unroll
+            for (int r = 0; r < OROWS; ++r) sum[r] = 0.f;
+#pragma unroll
+            for (int u = 0; u < OU; ++u) {
+                if (u > 0 && u * 64 >= o_units) break;  // (the same for the whole workgroup)
+                const int unit = u * 64 + lane;
+                const uint4 x = *reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(s_row) + min(unit, o_units - 1) * 8);
+                const uint32_t xs[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                for (int r = 0; r < OROWS; ++r) {
+                    const uint32_t ws[4] = {o_w[r][u].x, o_w[r][u].y, o_w[r][u].z, o_w[r][u].w};
+                    float more = 0.f;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        more = fmaf(__uint_as_float(xs[i] << 16), __uint_as_float(ws[i] << 16), more);
+                        more = fmaf(__uint_as_float(xs[i] & 0xffff0000u), __uint_as_float(ws[i] & 0xffff0000u), more);
+                    }
+                    sum[r] += unit < o_units ? more : 0.f;
+                }
+            }
+            float mine = 0.f;
+#pragma unroll
+            for (int r = 0; r < OROWS; ++r) {
+                const float all = wave_sum(sum[r]);
+                mine = lane == r ? all : mine;
+            }
+            if (lane < OROWS && o_first + lane < f.o_rows)
+                f.o_sums[kvh * f.o_part_stride + static_cast<int64_t>(q_row0) * f.o_rows + o_first + lane] = mine;
+            return;
         }
         if (partial_base >= 0 && wave == 0 && G == 0) {
             rec[HD] = m_all * kLn2;
@@ -875,6 +947,29 @@ int launch_qkv(const QkvSums& f, const void* k_pool, const void* v_pool, const i
     FSIE_CHECK_LAUNCH("attention_mfma_qkv");
     return 0;
 }
+
+// The same with the output projection: f.o_weight, f.o_sums; o_rows_of_wave rows of it a wave (2, 3 or 4).  No item is cut, none
+// has more than kShortWaves blocks of keys, no group more than 16 heads.
+template <int HDT>
+int launch_qkv_o(const QkvSums& f, const void* k_pool, const void* v_pool, const int32_t* block_tables, int max_pages,
+                 const int32_t* items, int n_items, int o_rows_of_wave, int n_heads, int n_kv, int page_size, int window,
+                 float scale, hipStream_t stream) {
+    constexpr int W = kShortWaves + 1;
+#define FSIE_ATTN_LAUNCH(R)                                                                                          \
+    attention_mfma_kernel<HDT, 1, W, true, true, false, false, R>                                                     \
+        <<<dim3((f.o_rows + W * R - 1) / (W * R), n_kv, n_items), 64 * W, 0, stream>>>(                               \
+            nullptr, 0, static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool), block_tables, max_pages, \
+            items, nullptr, nullptr, n_heads, n_kv, page_size, window, scale, n_heads / n_kv, f)
+    if (o_rows_of_wave == 2) FSIE_ATTN_LAUNCH(2);
+    else if (o_rows_of_wave == 3) FSIE_ATTN_LAUNCH(3);
+    else FSIE_ATTN_LAUNCH(4);
+#undef FSIE_ATTN_LAUNCH
+    FSIE_CHECK_LAUNCH("attention_mfma_qkv_o");
+    return 0;
+}
+
+typedef int (*LaunchQkvOFn)(const QkvSums&, const void*, const void*, const int32_t*, int, const int32_t*, int, int, int, int, int, int,
+                            float, hipStream_t);
 
 typedef int (*LaunchQkvFn)(const QkvSums&, const void*, const void*, const int32_t*, int, const int32_t*, int, void*,
                            float*, int, int, int, int, float, int, hipStream_t);

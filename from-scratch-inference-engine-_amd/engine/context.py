@@ -163,6 +163,7 @@ class StepContext:
         self.partial_sums_ok = False
         # set by a block around its mixer: what it leaves is read whole by every workgroup of the next product
         self.sums_in_one = False
+        self.sums_most = 0  # and how many slices that product takes at most (0: it takes none)
         self.block_tables: List[torch.Tensor] = []
         self.slots: List[torch.Tensor] = []
         self.fresh_pages: List[Optional[torch.Tensor]] = []  # per group: units just taken from the pool, or None

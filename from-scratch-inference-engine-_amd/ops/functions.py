@@ -1090,6 +1090,12 @@ def attention_mfma_qkv_ok(head_dim: int, page_size: int) -> bool:
     return bool(load().fsie_attention_mfma_qkv_ok(head_dim, page_size))
 
 
+def attention_mfma_qkv_o_rows(n_items: int, n_heads: int, n_kv: int, head_dim: int, page_size: int, n: int) -> int:
+    """Rows of an output projection of ``n`` rows a wave, where it is faster in attention's own launch (``attention_mfma_qkv``) for
+    ``n_items`` whole and short items; else 0."""
+    return int(load().fsie_attention_mfma_qkv_o_rows(n_items, n_heads, n_kv, head_dim, page_size, n, compute_units()))
+
+
 def attention_f32_qkv_ok(head_dim: int, page_size: int) -> bool:
     """The same of float32 storage (``attention_qkv`` takes both)."""
     return 0 < head_dim <= 128 and head_dim % 16 == 0 and page_size > 0 and page_size % 4 == 0
@@ -1099,12 +1105,15 @@ def attention_mfma_qkv(sums: torch.Tensor, bias: Optional[torch.Tensor], cos_sin
                        k_pool: torch.Tensor, v_pool: torch.Tensor, block_tables: torch.Tensor, items: torch.Tensor,
                        n_items: int, out: torch.Tensor, partials: Optional[torch.Tensor], n_heads: int, n_kv: int,
                        head_dim: int, window: Optional[int], scale: float, waves: int = 1,
-                       slopes: Optional[torch.Tensor] = None, row_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
+                       slopes: Optional[torch.Tensor] = None, row_scale: Optional[torch.Tensor] = None,
+                       o_weight: Optional[torch.Tensor] = None, o_rows: int = 0) -> torch.Tensor:
     """Attention of a step of one token a request (every item: one query row a head) from the q/k/v
     product's float32 partial sums [S, T, (heads + 2 kv heads) head_dim]: the kernel adds them up, adds
     ``bias``, rotates queries and keys by ``cos_sin`` [T, head_dim / 2, 2] (None: no rotation), scores each request's new key
     from registers and writes it and the value to ``slots[t]`` of the pools (negative: nowhere).  Pools and result in bfloat16, or all in
-    float32 (``attention_f32_qkv_ok``; ``waves`` is then the kernel's own choice)."""
+    float32 (``attention_f32_qkv_ok``; ``waves`` is then the kernel's own choice).
+    ``o_weight`` [N, heads head_dim] (bfloat16): the output projection in the same launch, ``out`` then its float32 partial sums
+    [kv heads, T, N]; ``o_rows``: what ``attention_mfma_qkv_o_rows`` says of the sizes.  Items are whole there."""
     width = (n_heads + 2 * n_kv) * head_dim
     _need(sums, "q/k/v sums", dtype=torch.float32, ndim=3)
     n_parts, t = sums.shape[0], sums.shape[1]
@@ -1126,12 +1135,26 @@ def attention_mfma_qkv(sums: torch.Tensor, bias: Optional[torch.Tensor], cos_sin
     _need(items, "attention items", dtype=torch.int32, ndim=2)
     if items.shape[1] != ATTN_ITEM_INTS or items.shape[0] < n_items:
         raise KernelError(f"attention items: shape {tuple(items.shape)} does not hold {n_items} items")
-    _need(out, "attention out", dtype=dtype, shape=(t, n_heads * head_dim))
+    if o_weight is not None:
+        _need(o_weight, "output projection", dtype=torch.bfloat16, ndim=2)
+        if o_weight.shape[1] != n_heads * head_dim:
+            raise KernelError(f"output projection: {o_weight.shape[1]} columns for {n_heads} heads of {head_dim}")
+        if slopes is not None or row_scale is not None or partials is not None:
+            raise KernelError("attention: the output projection goes with whole items and no bias on the scores")
+        _need(out, "output projection's sums", dtype=torch.float32, shape=(n_kv, t, o_weight.shape[0]))
+    else:
+        _need(out, "attention out", dtype=dtype, shape=(t, n_heads * head_dim))
     pages, kvh, page_size, hd = k_pool.shape
     if kvh != n_kv or hd != head_dim:
         raise KernelError(f"k_pool: shape {tuple(k_pool.shape)} does not match kv heads {n_kv}, head_dim {head_dim}")
     if partials is not None:
         _need(partials, "attention partials", dtype=torch.float32, ndim=1)
+    if o_weight is not None:
+        check(load().fsie_attention_mfma_qkv_o(sums.data_ptr(), n_parts, t, _ptr(bias), _ptr(cos_sin), slots.data_ptr(), k_pool.data_ptr(),
+                                               v_pool.data_ptr(), pages * page_size, block_tables.data_ptr(), block_tables.shape[1],
+                                               items.data_ptr(), n_items, o_weight.data_ptr(), o_weight.shape[0], out.data_ptr(), int(o_rows),
+                                               n_heads, n_kv, head_dim, page_size, int(window or 0), float(scale), _stream()))
+        return out
     if wide:
         check(load().fsie_attention_f32_qkv(sums.data_ptr(), n_parts, t, _ptr(bias), _ptr(cos_sin), slots.data_ptr(), k_pool.data_ptr(),
                                             v_pool.data_ptr(), pages * page_size, block_tables.data_ptr(), block_tables.shape[1],

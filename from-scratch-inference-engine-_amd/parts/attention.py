@@ -817,9 +817,19 @@ class GQAttention(Mixer):
             return False
         return self._sums_will_do(ctx.compute_dtype, cache, ctx.plan(self.planner()), self._fused_table(ctx)[0])
 
+    def _rows_in_attention(self, x, ctx, cache, plan) -> int:
+        """Rows a wave of the output projection where attention's own workgroups make it (a step of one or two requests with short
+        items, whose next norm is made by the product behind it and takes a slice a kv head), or 0."""
+        if (not self.n_kv <= getattr(ctx, "sums_most", 0) or not getattr(ctx, "partial_sums_ok", False) or plan.n_partial or plan.waves != 1
+                or x.dtype != torch.bfloat16 or self._slopes is not None or self.query_temperature is not None or self.o.bias is not None or type(self.o) is not Linear
+                or self.o.weight.dtype != torch.bfloat16 or not self.o.weight.is_contiguous() or self.o.weight.data_ptr() % 16):
+            return 0
+        return ops.attention_mfma_qkv_o_rows(plan.n_small, self.n_heads, self.n_kv, self.head_dim, cache.page_size, self.hidden_size)
+
     def _from_sums(self, x, ctx, cache, plan, fuse: bool, table) -> Optional[torch.Tensor]:
         """Attention of a step of one token a request straight from the q/k/v product's partial sums
-        (None: not such a step, or the kernels do not take the sizes)."""
+        (None: not such a step, or the kernels do not take the sizes); [T, heads], or the output projection's partial sums [kv heads, T, hidden] where that is
+        made in the same launch."""
         if not self._sums_will_do(x.dtype, cache, plan, fuse):
             return None
         if isinstance(x, PendingNorm):
@@ -833,6 +843,12 @@ class GQAttention(Mixer):
             sums = self.qkv.partial_sums(x, few_rows=True, long_slices=self.wants_long_slices)
         if sums is None:
             return None
+        rows = self._rows_in_attention(x, ctx, cache, plan)
+        if rows:
+            out = torch.empty((self.n_kv, x.shape[0], self.hidden_size), dtype=torch.float32, device=x.device)
+            return ops.attention_mfma_qkv(sums, self.qkv.bias, table, cache.slots, cache.k_pool, cache.v_pool, cache.block_tables,
+                                          plan.items, plan.n_small, out, None, self.n_heads, self.n_kv, self.head_dim, self.window,
+                                          self.scale, o_weight=self.o.weight, o_rows=rows)
         out = torch.empty((x.shape[0], self.q_dim), dtype=x.dtype, device=x.device)
         partials = None
         if plan.n_partial:
@@ -953,7 +969,7 @@ class GQAttention(Mixer):
         fuse, table = self._fused_table(ctx)
         out = self._from_sums(x, ctx, cache, plan, fuse, table)
         if out is not None:
-            return self.o.for_residual(out, ctx)
+            return out if out.ndim == 3 else self.o.for_residual(out, ctx)  # (three: the output projection's sums already)
         qkv = self._project_rotate_store(x, ctx, cache, fuse, table)
         out = paged_attention(qkv, qkv.shape[1], cache, plan, self.n_heads, self.n_kv, self.head_dim, self.window,
                               self.scale, x.shape[0], sinks=self.sink, share_keys=self.share_keys, softcap=self.softcap,

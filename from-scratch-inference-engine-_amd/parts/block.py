@@ -48,10 +48,11 @@ class PreNormBlock(Block):
         x = self._normed(self.mixer_norm, self.mixer, hidden, ctx, cache)
         # (the output projection leaves its sums in one slice where every workgroup of the next product is going to read them)
         ctx.sums_in_one = self.ffn_norm.can_wait(hidden, ctx.compute_dtype) and self.ffn.takes_pending_norm(rows, 1, ctx)
+        ctx.sums_most = next((n for n in (8, 4, 2, 1) if self.ffn.takes_pending_norm(rows, n, ctx)), 0) if ctx.sums_in_one else 0
         try:
             hidden.delta = self.mixer.forward(x, ctx, cache)
         finally:
-            ctx.sums_in_one = False
+            ctx.sums_in_one, ctx.sums_most = False, 0
         x = self._normed(self.ffn_norm, self.ffn, hidden, ctx)
         hidden.delta = self.ffn.forward(x, ctx)
 
