@@ -256,6 +256,11 @@ int launch_shape(int tile, const Call& c) {
 // 129 to 159 rows of N above 6,400 to 10,240 and K from 2048, where the library is at its best and a third of these tiles' rows are none, are taken all the same
 // (N = 8192, K = 2048 18.3 / 15.9, N = 10240 19.9 / 17.7, N = 7168, K = 3072 24.2 / 22.1; with K = 1536 or N = 6144 0.72): such portions of a prompt are bound by the
 // host, for which the library's call is 21 us and the bias behind it a launch more, this one 13 (Romepel, 9 layers, prompts of 129 to 159 tokens 1.29 ms, 1.43 so).
+// Of matrices of 8 to 40 MB and 320 to 2,600 rows the fit is some fifth too good to the library, whose choice of a kernel goes by other things than the time
+// counted here: up to 1.3 of it is taken (K to 6 N), in slices up to 1.1 where the fit has no whole product that is as fast.  4,295 sizes from the library to
+// these tiles, weights from HBM: whole 0.82 of its time, with the norm 0.84, slices with the norm 0.80; 107 beyond 1.02, 37 beyond 1.05, at most 1.17 (525 rows of
+// N = 912, K = 5120 19.2 / 16.4).  1,375 rows of N = 896, K = 4864 and the norm 27.7 / 32.1, 513 of N = 2048, K = 8192 39.6 / 47.2, 1,025 of N = K = 2048 21.8 / 24.9, 640 of
+// N = K = 3584 33.8 / 37.8.  200 to 320 rows are the library's at up to 1.4 (251 of N = 880, K = 4608 15.6 / 11.0), and so are a longer K (1,895 of N = 1088, K = 11008 92.5 / 75.5).
 // The dies' reads of x: 1,845 rows of N = 512, K = 6656 33.7 / 29.4, 2,284 of N = 432, K = 11776 57.6 / 49.6, which the steps alone put at 22.8 and 37.7.
 constexpr double kBeyond = 80e6;   // bytes of weights
 constexpr double kDiesRead = 6.5e6;  // bytes a us of x by all dies
@@ -273,7 +278,7 @@ extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int un
     if (large && (result == kSums ? M > 512 || K < N : M <= 128 || K > (M <= 256 ? 8192 : 6144))) return -1;
     if (result == kSums && N > 8192) return -1;
     const double whole = 4.0 * M * static_cast<double>(N) / 3e6;  // the delta in bfloat16, out and into the norm
-    double best = 1e30;
+    double best = 1e30, best_plain = 1e30;
     int choice = -1;
     bool fills = false;  // (nearly all units)
     for (int tile = 0; tile < 4; ++tile) {
@@ -287,6 +292,7 @@ extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int un
             const double of_slice = a_die < m_tiles ? static_cast<double>(a_die) / m_tiles : 1.0, slices_read = static_cast<double>(a_die) / (m_tiles * n_tiles);
             const double share = (of_slice > slices_read ? of_slice : slices_read) / slices, read = 8.0 * rows_bytes * (share < 1.0 ? share : 1.0) / kDiesRead;
             if (us < read) us = read;
+            if (slices == 1 && us < best_plain) best_plain = us;
             if (result == kSums) us += (slices == 1 ? whole : 2.0 * slices * whole);
             if (us < best) {
                 best = us;
@@ -297,7 +303,12 @@ extern "C" int fsie_gemm_mfma_block_plan(int M, int N, int K, int result, int un
     }
     const double library = 8.3 + flops / 1.64e9 + weights / 3e6 + rows_bytes / 2.2e6;
     if (large && result == kPlain && (choice % 256 != 2 || !fills)) return -1;
-    return choice >= 0 && best <= (result == kSums ? 0.95 * (library + whole) : library) ? choice : -1;
+    if (choice < 0) return -1;
+    const bool middle = weights >= 8e6 && weights <= 40e6 && M >= 320 && M <= 2600 && N >= 800;
+    if (result == kSums)
+        return best <= 0.95 * (library + whole) ||
+                       (middle && (N <= 2560 || M >= 500) && best <= 1.1 * (library + whole) && best_plain > library) ? choice : -1;
+    return best <= (middle && K <= 6 * static_cast<int64_t>(N) ? 1.3 : 1.0) * library ? choice : -1;
 }
 
 extern "C" int fsie_gemm_mfma_block(const void* x, const void* w, const float* bias, void* y, int M, int N, int K, int result, int splits,

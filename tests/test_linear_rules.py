@@ -163,6 +163,16 @@ def test_small_tiles_take(m, n, k, sums, plan):
     assert (got % 256, got // 256) == plan
 
 
+@pytest.mark.parametrize("m, n, k, sums, plan", [
+    (1375, 896, 4864, True, (2, 3)), (513, 2048, 8192, True, (2, 3)), (1700, 896, 4864, True, None),   # (the last: a whole product is as fast by the fit)
+    (640, 3584, 3584, False, (2, 1)), (1025, 2048, 2048, False, (2, 1)),
+    (319, 3584, 3584, False, None), (320, 3584, 3584, False, (1, 1)), (2601, 896, 4864, True, None), (400, 3584, 3584, True, None),
+    (1375, 768, 4864, True, None), (700, 1024, 6144, False, (3, 1)), (1895, 1088, 11008, False, None)])
+def test_small_tiles_of_middle_sizes(m, n, k, sums, plan):
+    got = _block_plan(m, n, k, sums)
+    assert (None if got < 0 else (got % 256, got // 256)) == plan
+
+
 def test_plans_of_small_tiles_are_ones_the_kernel_takes():
     import random
 
