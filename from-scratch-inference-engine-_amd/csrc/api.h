@@ -322,7 +322,7 @@ int fsie_attention_mfma_qkv_ok(int head_dim, int page_size);
 int fsie_attention_f32_qkv(const float* sums, int n_parts, int n_tokens, const float* bias, const float* cos_sin, const int32_t* slots,
                            float* k_pool, float* v_pool, int64_t pool_slots, const int32_t* block_tables, int max_pages,
                            const int32_t* items, int n_items, float* out, float* partials, int n_heads, int n_kv, int head_dim,
-                           int page_size, int window, float scale, const float* slopes, const float* row_scale, hipStream_t stream);
+                           int page_size, int window, float scale, int short_items, const float* slopes, const float* row_scale, hipStream_t stream);
 int fsie_attention_mfma_qkv(const float* sums, int n_parts, int n_tokens, const float* bias, const float* cos_sin,
                             const int32_t* slots, void* k_pool, void* v_pool, int64_t pool_slots,
                             const int32_t* block_tables, int max_pages, const int32_t* items, int n_items, void* out,

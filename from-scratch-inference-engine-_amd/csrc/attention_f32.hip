@@ -23,6 +23,8 @@
 // attention (3.3 us of a layer and step; four requests of the 0.5B shape, 16 tokens each, 20.5 ms -> 20.0).  The bits are those of the kernels one after the other.
 //
 // More workgroups than units: four waves each whatever the head size, except over the tiles of long prompts (see launch).
+// So it is for items that are cut to 64 keys: the twelve waves beside them have no keys, and asked in vain for sums (a unit takes 16 cycles for each of a wave's
+// loads).  Four requests of 42 to 316 keys, 14 heads on 2 of 64, 8.1 us -> 6.1 with the loads in straight-line code besides (see `asks`); the step above 20.0 ms -> 19.6.  Longer items are no gain: at 128, 256 and 512 keys 20.7, 22.0 and 21.5 ms.
 #include "common.h"
 #include "api.h"
 
@@ -56,7 +58,7 @@ struct F32Call {
     int64_t q_stride;
     const int32_t *block_tables, *items;
     float *out, *partials;
-    int n_items, max_pages, n_heads, n_kv, page_size, window, all_waves;
+    int n_items, max_pages, n_heads, n_kv, page_size, window, all_waves, few_waves;
     float scale, softcap;
     const float *sinks, *slopes, *row_scale;
     F32Sums sums;  // sums null: queries from q, keys and values in the pools already
@@ -141,12 +143,17 @@ __global__ __launch_bounds__(64 * W) void attention_f32_kernel(
     };
 
     const bool any = kb_begin < kb_end;
+    // QKV with four waves: a wave without keys asks all the same, for what lies at the start of page 0.  Behind a branch around these loads the compiler cannot
+    // know how many are under way, and waits for the keys where it needs the sums.
+    const bool asks = (QKV && W == 4) || any;
     Asked asked;
-    if (any) ask(kb_begin, asked);
+    if (asks) ask(kb_begin, asked);
     Block b;
     // QKV: the heads' sums, all that are asked for at once and before the first keys; a thread has quads of columns of the heads this workgroup needs
     constexpr int NJ = QKV ? (18 * HD / 4 + 64 * W - 1) / (64 * W) : 1, PC = NJ <= 3 ? 8 : 4;
     const bool owner = QKV && pos0 >= key_begin && pos0 < key_end;  // the item whose keys end with the new one
+    int slot = -1;
+    if constexpr (QKV) slot = f.slots[q_row0];
     if constexpr (QKV) {
         floatx4 part[NJ][PC], bias_of[NJ];
         float2 angle = float2{1.f, 0.f};
@@ -154,6 +161,7 @@ __global__ __launch_bounds__(64 * W) void attention_f32_kernel(
         const int n_cols = (gh_here + 2) * HD, q_dim = n_heads * HD, kv_dim = n_kv * HD;
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
+            if (j > 0 && j * 64 * W * 4 >= n_cols) continue;  // (the same for the whole workgroup, as below)
             const int i = (static_cast<int>(threadIdx.x) + j * 64 * W) * 4, ic = i < n_cols ? i : 0;
             const int seg = ic / HD, d = ic - seg * HD;
             const int col = seg < gh_here ? (h_base + seg) * HD + d : q_dim + (seg - gh_here) * kv_dim + kvh * HD + d;
@@ -164,9 +172,10 @@ __global__ __launch_bounds__(64 * W) void attention_f32_kernel(
         }
         const float2* table_row = reinterpret_cast<const float2*>(f.cos_sin) + static_cast<int64_t>(q_row0) * (HD / 2);
         if (f.cos_sin) angle = table_row[min(static_cast<int>(threadIdx.x), HD / 2 - 1)];
-        if (any) load(asked, b);
+        if (asks) load(asked, b);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
+            if (j > 0 && j * 64 * W * 4 >= n_cols) continue;
             const int i = (static_cast<int>(threadIdx.x) + j * 64 * W) * 4;
             floatx4 a = part[j][0];
 #pragma unroll
@@ -199,9 +208,14 @@ __global__ __launch_bounds__(64 * W) void attention_f32_kernel(
     const int head = h_base + (row_ok ? hh : 0), row = q_row0 + (row_ok ? tq : 0), pos = pos0 + tq;
     floatx4 qf[HDT];
     if constexpr (QKV) {
-        if (any) {
+        if (any) {  // (one question for all of them: with one each every read of LDS waited for the last)
+            if (f.cos_sin) {
 #pragma unroll
-            for (int j = 0; j < HDT; ++j) qf[j] = head_values(row_ok ? hh : 0, 16 * j + 4 * G, f.cos_sin != nullptr);
+                for (int j = 0; j < HDT; ++j) qf[j] = head_values(row_ok ? hh : 0, 16 * j + 4 * G, true);
+            } else {
+#pragma unroll
+                for (int j = 0; j < HDT; ++j) qf[j] = head_values(row_ok ? hh : 0, 16 * j + 4 * G, false);
+            }
         }
     } else if (W < 16 || any) {  // (of sixteen waves most have no key where items are short, and read nothing; eight are slower with the question)
         const float* qp = q + static_cast<int64_t>(row) * q_stride + static_cast<int64_t>(head) * HD + 4 * G;
@@ -218,7 +232,6 @@ __global__ __launch_bounds__(64 * W) void attention_f32_kernel(
     if constexpr (QKV) {
         // the new key and value into the pools, by the last wave
         if (owner && chunk == 0 && wave == W - 1) {
-            const int slot = f.slots[q_row0];
             if (slot >= 0 && slot < f.pool_slots) {
                 const int page = slot / page_size, off = slot - page * page_size;
                 float* kd = f.k_out + page * page_stride + kv_base + static_cast<int64_t>(off) * HD;
@@ -402,7 +415,7 @@ int launch(const F32Call& a, hipStream_t stream) {
     // item of up to four blocks gives the same bits by either; a launch with longer tiles of prompts asks for all waves, since a
     // portion's sums are not to follow from what else is in the step (300 tokens, 14 on 2 of 64, 14.9 us where four took 13.2).
     const bool many = static_cast<int64_t>(grid.x) * grid.y * grid.z > fsie_compute_units();
-    if (W > 4 && many && !a.all_waves) launch_waves<HDT, 4>(a, grid, group, gh, stream);
+    if (W > 4 && (many || a.few_waves) && !a.all_waves) launch_waves<HDT, 4>(a, grid, group, gh, stream);
     else launch_waves<HDT, W>(a, grid, group, gh, stream);
     FSIE_CHECK_LAUNCH("attention_f32");
     return 0;
@@ -455,7 +468,7 @@ extern "C" int fsie_attention_f32(const float* q, int64_t q_stride, const float*
 extern "C" int fsie_attention_f32_qkv(const float* sums, int n_parts, int n_tokens, const float* bias, const float* cos_sin, const int32_t* slots,
                                       float* k_pool, float* v_pool, int64_t pool_slots, const int32_t* block_tables, int max_pages,
                                       const int32_t* items, int n_items, float* out, float* partials, int n_heads, int n_kv, int head_dim,
-                                      int page_size, int window, float scale, const float* slopes, const float* row_scale, hipStream_t stream) {
+                                      int page_size, int window, float scale, int short_items, const float* slopes, const float* row_scale, hipStream_t stream) {
     FSIE_REQUIRE(n_items >= 0 && n_heads > 0 && n_kv > 0 && n_heads % n_kv == 0,
                  "attention_f32_qkv: heads %d must be a positive multiple of kv heads %d", n_heads, n_kv);
     FSIE_REQUIRE(fsie_attention_f32_ok(head_dim, page_size) && head_dim <= 16 * kSumsHdt,
@@ -471,7 +484,7 @@ extern "C" int fsie_attention_f32_qkv(const float* sums, int n_parts, int n_toke
     F32Call a{};
     a.k_pool = k_pool, a.v_pool = v_pool, a.block_tables = block_tables, a.items = items;
     a.out = out, a.partials = partials, a.n_items = n_items, a.max_pages = max_pages, a.n_heads = n_heads, a.n_kv = n_kv;
-    a.page_size = page_size, a.window = window, a.scale = scale, a.slopes = slopes, a.row_scale = row_scale;
+    a.page_size = page_size, a.window = window, a.scale = scale, a.slopes = slopes, a.row_scale = row_scale, a.few_waves = short_items;
     a.sums = F32Sums{sums, bias, cos_sin, slots, k_pool, v_pool, 0, pool_slots, n_parts, (n_heads + 2 * n_kv) * head_dim};
     a.sums.part_stride = static_cast<int64_t>(n_tokens) * a.sums.width;
     return launch_from<1>(head_dim / 16, a, stream);

@@ -1106,12 +1106,13 @@ def attention_mfma_qkv(sums: torch.Tensor, bias: Optional[torch.Tensor], cos_sin
                        n_items: int, out: torch.Tensor, partials: Optional[torch.Tensor], n_heads: int, n_kv: int,
                        head_dim: int, window: Optional[int], scale: float, waves: int = 1,
                        slopes: Optional[torch.Tensor] = None, row_scale: Optional[torch.Tensor] = None,
-                       o_weight: Optional[torch.Tensor] = None, o_rows: int = 0) -> torch.Tensor:
+                       o_weight: Optional[torch.Tensor] = None, o_rows: int = 0, short_items: bool = False) -> torch.Tensor:
     """Attention of a step of one token a request (every item: one query row a head) from the q/k/v
     product's float32 partial sums [S, T, (heads + 2 kv heads) head_dim]: the kernel adds them up, adds
     ``bias``, rotates queries and keys by ``cos_sin`` [T, head_dim / 2, 2] (None: no rotation), scores each request's new key
     from registers and writes it and the value to ``slots[t]`` of the pools (negative: nowhere).  Pools and result in bfloat16, or all in
-    float32 (``attention_f32_qkv_ok``; ``waves`` is then the kernel's own choice).
+    float32 (``attention_f32_qkv_ok``; ``waves`` is then the kernel's own choice: four where the items are more than the units or ``short_items`` says that
+    none has more than four blocks of 16 keys).
     ``o_weight`` [N, heads head_dim] (bfloat16): the output projection in the same launch, ``out`` then its float32 partial sums
     [kv heads, T, N]; ``o_rows``: what ``attention_mfma_qkv_o_rows`` says of the sizes.  Items are whole there."""
     width = (n_heads + 2 * n_kv) * head_dim
@@ -1159,7 +1160,7 @@ def attention_mfma_qkv(sums: torch.Tensor, bias: Optional[torch.Tensor], cos_sin
         check(load().fsie_attention_f32_qkv(sums.data_ptr(), n_parts, t, _ptr(bias), _ptr(cos_sin), slots.data_ptr(), k_pool.data_ptr(),
                                             v_pool.data_ptr(), pages * page_size, block_tables.data_ptr(), block_tables.shape[1],
                                             items.data_ptr(), n_items, out.data_ptr(), _ptr(partials), n_heads, n_kv, head_dim, page_size,
-                                            int(window or 0), float(scale), *_bias_ptrs(slopes, row_scale, n_heads, t), _stream()))
+                                            int(window or 0), float(scale), int(short_items), *_bias_ptrs(slopes, row_scale, n_heads, t), _stream()))
         return out
     check(load().fsie_attention_mfma_qkv(sums.data_ptr(), n_parts, t, _ptr(bias), _ptr(cos_sin), slots.data_ptr(),
                                          k_pool.data_ptr(), v_pool.data_ptr(), pages * page_size,

@@ -497,6 +497,8 @@ class AttentionPlanner:
             # four blocks the sums are the same either way; decode items are cut by the batch as it is)
             "all_waves": not mfma and bool((large[:, 5] - (large[:, 4] & ~15) + np.where(
                 large[:, 7] & ATTN_KEEP_WALK, np.minimum(large[:, 7] & ~(ATTN_KEEP_WALK | ATTN_POOL_WALK), large[:, 4]) + 15 & ~15, 0) > 64).any()),
+            # float32: the items are cut, to no more than four blocks of 16 keys
+            "short_items": not mfma and n_partial > 0 and split_keys <= 64,
             "single": all(host.q_lens[s] == 1 for s in range(host.n_seqs)),  # one token a request
         }
 
@@ -856,7 +858,7 @@ class GQAttention(Mixer):
                                    device=x.device)
         ops.attention_mfma_qkv(sums, self.qkv.bias, table, cache.slots, cache.k_pool, cache.v_pool,
                                cache.block_tables, plan.items, plan.n_small, out, partials, self.n_heads, self.n_kv,
-                               self.head_dim, self.window, self.scale, waves=plan.waves, slopes=self._slopes,
+                               self.head_dim, self.window, self.scale, waves=plan.waves, short_items=getattr(plan, "short_items", False), slopes=self._slopes,
                                row_scale=self._row_scale(ctx))
         if plan.n_merges:
             ops.attention_merge(partials, plan.merges, plan.n_merges, out, self.n_heads, self.head_dim)

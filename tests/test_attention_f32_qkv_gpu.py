@@ -89,3 +89,33 @@ def test_refusals(ops):
         ops.attention_mfma_qkv(torch.zeros(1, 1, 192).cuda(), None, None, torch.zeros(1, dtype=torch.int32).cuda(), torch.zeros(2, 1, 16, 64).cuda(),
                                torch.zeros(2, 1, 64, 16).cuda(), torch.zeros(1, 1, dtype=torch.int32).cuda(), torch.zeros(1, 8, dtype=torch.int32).cuda(), 1,
                                torch.zeros(1, 64, dtype=torch.bfloat16).cuda(), None, 1, 1, 64, None, 1.0)
+
+
+@pytest.mark.parametrize("heads, kv, hd, page, n_parts, table", [
+    (14, 2, 64, 16, 7, True), (16, 1, 128, 8, 3, True), (32, 2, 96, 16, 9, True),  # (sixteen heads of 96 and 128: more columns than four waves have threads)
+    (3, 3, 16, 4, 1, False), (20, 1, 64, 16, 2, False)])
+def test_short_items_give_the_same_bits_on_four_waves(ops, heads, kv, hd, page, n_parts, table):
+    from from_scratch_inference_engine_amd.parts.attention import AttentionPlanner
+
+    pasts = [0, 5, 15, 16, 63, 64, 200, 330]
+    t, width = len(pasts), (heads + 2 * kv) * hd
+    AttentionPlanner.compute_units = 4096  # (items of 64 keys)
+    try:
+        case = paged_case([(p, 1) for p in pasts], heads, kv, hd, page, torch.float32, seed=heads)
+    finally:
+        AttentionPlanner.compute_units = None
+    plan = case["plan"]
+    assert plan["short_items"] and plan["n_partial"] and all(it[5] - it[4] <= 64 for it in plan["items"][:plan["n_small"]])
+    g = torch.Generator().manual_seed(9)
+    parts, bias = torch.randn(n_parts, t, width, generator=g).cuda(), torch.randn(width, generator=g).cuda()
+    angles = torch.randn(t, hd, generator=g).cuda() if table else None
+    tables = case["tables"]
+    slots = torch.tensor([int(tables[s, p // page]) * page + p % page for s, p in enumerate(pasts)], dtype=torch.int32).cuda()
+    items, bt = torch.from_numpy(plan["items"]).cuda(), tables.cuda()
+    got = []
+    for short in (False, True):
+        k, v = case["k_pool"].cuda().clone(), case["v_pool"].cuda().clone()
+        out, partials = torch.zeros(t, heads * hd).cuda(), torch.zeros(plan["n_partial"] * heads * (hd + 2)).cuda()
+        ops.attention_mfma_qkv(parts, bias, angles, slots, k, v, bt, items, plan["n_small"], out, partials, heads, kv, hd, None, hd ** -0.5, short_items=short)
+        got.append((out, partials, k, v))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and got[0][1].abs().max() > 0.1
