@@ -45,7 +45,7 @@ constexpr int f32_waves() {
 // What the QKV variant reads and writes beside the kernel's other operands.
 struct F32Sums {
     const float *sums, *bias, *cos_sin;  // [n_parts][tokens][width]; [width] or null; [tokens][head_dim / 2] pairs of cosine and sine, or null: nothing is turned
-    const int32_t* slots;                // [tokens]: where a token's key and value go (negative, or not below pool_slots: nowhere)
+    const int32_t* slots;                // [tokens]: where a token's key and value go (negative, or not below pool_slots: nowhere); the kernel has it in the place of q
     float *k_out, *v_out;                // the pools again, to write
     int64_t part_stride, pool_slots;
     int n_parts, width;
@@ -88,6 +88,10 @@ __global__ __launch_bounds__(64 * W) void attention_f32_kernel(
     const ItemInts it = *reinterpret_cast<const ItemInts*>(items + static_cast<int64_t>(blockIdx.x) * FSIE_ATTN_ITEM_INTS);
     const int seq = it[FSIE_ATTN_ITEM_SEQ], q_row0 = it[FSIE_ATTN_ITEM_QROW], n_q = it[FSIE_ATTN_ITEM_NQ], pos0 = it[FSIE_ATTN_ITEM_POS];
     const int key_begin = it[FSIE_ATTN_ITEM_KBEGIN], key_end = it[FSIE_ATTN_ITEM_KEND], partial_base = it[FSIE_ATTN_ITEM_PARTIAL];
+    // (the arguments that do not come with the launch on the item's trip: left alone, the compiler asks for them behind it, where they are used)
+    if constexpr (QKV)
+        asm volatile("" ::"s"(n_heads), "s"(group), "s"(gh), "s"(window), "s"(scale), "s"(slopes), "s"(row_scale), "s"(f.sums), "s"(f.bias), "s"(f.cos_sin), "s"(f.k_out),
+                     "s"(f.v_out), "s"(f.part_stride), "s"(f.n_parts), "s"(f.width));
     if (n_q <= 0) return;  // padding item
     // the first keys that a window keeps: seen whatever the window says, and read, as blocks ahead of the item's own
     // range, where the item is told to
@@ -153,7 +157,7 @@ __global__ __launch_bounds__(64 * W) void attention_f32_kernel(
     constexpr int NJ = QKV ? (18 * HD / 4 + 64 * W - 1) / (64 * W) : 1, PC = NJ <= 3 ? 8 : 4;
     const bool owner = QKV && pos0 >= key_begin && pos0 < key_end;  // the item whose keys end with the new one
     int slot = -1;
-    if constexpr (QKV) slot = f.slots[q_row0];
+    if constexpr (QKV) slot = reinterpret_cast<const int32_t*>(q)[q_row0];  // (there are no queries: what stands there is where tokens go)
     if constexpr (QKV) {
         floatx4 part[NJ][PC], bias_of[NJ];
         float2 angle = float2{1.f, 0.f};
@@ -396,7 +400,7 @@ void launch_waves(const F32Call& a, dim3 grid, int group, int gh, hipStream_t st
     if constexpr (HDT <= kSumsHdt)
         if (a.sums.sums)
             return attention_f32_kernel<HDT, W, true><<<grid, 64 * W, 0, stream>>>(
-            a.items, a.block_tables, a.max_pages, a.page_size, page_magic, a.n_kv, a.k_pool, a.v_pool, nullptr, 0, a.out, a.partials, a.n_heads, group,
+            a.items, a.block_tables, a.max_pages, a.page_size, page_magic, a.n_kv, a.k_pool, a.v_pool, reinterpret_cast<const float*>(a.sums.slots), 0, a.out, a.partials, a.n_heads, group,
                 gh, a.window, a.scale, 0.f, nullptr, a.slopes, a.row_scale, a.sums);
     attention_f32_kernel<HDT, W, false><<<grid, 64 * W, 0, stream>>>(
             a.items, a.block_tables, a.max_pages, a.page_size, page_magic, a.n_kv, a.k_pool, a.v_pool, a.q, a.q_stride, a.out, a.partials, a.n_heads, group,

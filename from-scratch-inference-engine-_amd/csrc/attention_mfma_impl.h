@@ -87,7 +87,7 @@ struct QkvSums {
     const float* sums;     // [n_parts][n_tokens][width], width = (n_heads + 2 n_kv) head_dim
     const float* bias;     // [width], or null
     const float* cos_sin;  // [n_tokens][head_dim / 2] pairs (cos, sin) of each token's position, or null: no rotation
-    const int32_t* slots;  // [n_tokens] slot of a token's key and value in the pools (negative: nowhere)
+    const int32_t* slots;  // [n_tokens] slot of a token's key and value in the pools (negative: nowhere); the kernel has it in the place of q
     bf16_t* k_out;         // the pools again, to write
     bf16_t* v_out;
     int64_t part_stride;   // n_tokens * width
@@ -181,6 +181,11 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
     typedef int ItemInts __attribute__((ext_vector_type(8), aligned(4)));
     static_assert(FSIE_ATTN_ITEM_INTS == 8, "an item is eight numbers");
     const ItemInts it = *reinterpret_cast<const ItemInts*>(item);
+    // (the arguments beyond those that come with the launch on the same trip: left alone, the compiler asks for them behind the item, where they are used,
+    // on three trips more.  One request of the 0.5B shape 520 us a step, 515 so)
+    if constexpr (QKV)
+        asm volatile("" ::"s"(f.sums), "s"(f.bias), "s"(f.cos_sin), "s"(f.k_out), "s"(f.v_out), "s"(f.part_stride), "s"(f.n_parts), "s"(f.width),
+                     "s"(f.group), "s"(f.page_magic), "s"(n_heads), "s"(n_kv), "s"(page_size), "s"(window), "s"(gh), "s"(scale));
     const int seq = it[FSIE_ATTN_ITEM_SEQ];
     const int q_row0 = it[FSIE_ATTN_ITEM_QROW];
     const int n_q = it[FSIE_ATTN_ITEM_NQ];
@@ -199,7 +204,7 @@ __global__ __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(MAXW 
     const bool owner = QKV && pos0 >= key_begin && pos0 < key_end;
     if (owner) key_end = pos0;
     int new_slot = -1;
-    if constexpr (QKV) new_slot = f.slots[q_row0];
+    if constexpr (QKV) new_slot = reinterpret_cast<const int32_t*>(q)[q_row0];  // (there are no queries: what stands there is where tokens go)
 
     const int group = f.group;
     const int kvh = blockIdx.y, chunk = OROWS > 0 ? 0 : blockIdx.z;
@@ -934,7 +939,7 @@ int launch_qkv(const QkvSums& f, const void* k_pool, const void* v_pool, const i
     if (f.slopes || f.row_scale) FSIE_ATTN_LAUNCH_AS(W, THREADS, true); else FSIE_ATTN_LAUNCH_AS(W, THREADS, false)
 #define FSIE_ATTN_LAUNCH_AS(W, THREADS, B)                                                                           \
     attention_mfma_kernel<HDT, 1, W, true, true, B><<<grid, THREADS, 0, stream>>>(                                      \
-        nullptr, 0, static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool), block_tables, max_pages, \
+        reinterpret_cast<const bf16_t*>(f.slots), 0, static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool), block_tables, max_pages, \
         items, static_cast<bf16_t*>(out), partials, n_heads, n_kv, page_size, window, scale, gh, f)
     constexpr int SHORTW = HDT <= 8 ? kShortWaves + 1 : MAXW;
     if (waves <= 1) {
@@ -958,7 +963,7 @@ int launch_qkv_o(const QkvSums& f, const void* k_pool, const void* v_pool, const
 #define FSIE_ATTN_LAUNCH(R)                                                                                          \
     attention_mfma_kernel<HDT, 1, W, true, true, false, false, R>                                                     \
         <<<dim3((f.o_rows + W * R - 1) / (W * R), n_kv, n_items), 64 * W, 0, stream>>>(                               \
-            nullptr, 0, static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool), block_tables, max_pages, \
+            reinterpret_cast<const bf16_t*>(f.slots), 0, static_cast<const bf16_t*>(k_pool), static_cast<const bf16_t*>(v_pool), block_tables, max_pages, \
             items, nullptr, nullptr, n_heads, n_kv, page_size, window, scale, n_heads / n_kv, f)
     if (o_rows_of_wave == 2) FSIE_ATTN_LAUNCH(2);
     else if (o_rows_of_wave == 3) FSIE_ATTN_LAUNCH(3);
