@@ -6,7 +6,7 @@ computes with torch; a missing kernel library is an error, not a reason to fall 
 """
 
 from .functions import (FragmentOrdered, attention_merge, attention_mfma, attention_mfma_lds, attention_mfma_lds_ok,
-                        attention_mfma_max_waves, attention_mfma_qkv, attention_mfma_qkv_ok, attention_mfma_qkv_o_rows, attention_f32_qkv_ok, attention_mfma_rows, attention_scalar,
+                        attention_mfma_max_waves, attention_mfma_qkv, attention_mfma_qkv_ok, attention_mfma_qkv_o_rows, attention_merge_o, attention_merge_o_rows, attention_f32_qkv_ok, attention_mfma_rows, attention_scalar,
                         attention_tile_tokens, bias_add, compute_units, dtype_code, embedding, fragment_order, gemm, gemm_mfma_fp32, gemm_mfma_fp32_sums, gemm_mfma_fp32_splits, gemm_fp32_gated, gemm_fp32_tile, gemm_fp32_tile_splits, gemm_fp32_stream, gemm_fp32_stream_plan, GEMM_FP32_WHOLE, GEMM_FP32_GATED, GEMM_FP32_SUMS, gemm_mfma_skinny,
                         gemm_mfma_skinny_rope, gemm_mfma_wide, gemm_mfma_wide_best_splits, gemm_mfma_wide_splits_ok,
                         gemm_mfma_wide_swiglu, gemm_mfma_wide_takes, gemm_mfma_stream, gemm_mfma_block, gemm_block_plan, GEMM_BLOCK_PLAIN, GEMM_BLOCK_SUMS, gemm_mfma_normed, gemm_normed_takes, gemm_stream_plan, GEMM_STREAM_SUMS, GEMM_STREAM_GATED, GEMM_STREAM_POINT, GEMM_STREAM_PLAN_ACT, GEMM_STREAM_PLAN_ONE, random_fill,
@@ -20,7 +20,7 @@ from .library import KernelError, KernelLibraryMissing, load
 from .tuning import disable_library_tuning, enable_library_tuning, library_mm, library_tuning_enabled
 
 __all__ = ["FragmentOrdered", "KernelError", "KernelLibraryMissing", "attention_merge", "attention_mfma", "attention_mfma_lds",
-           "attention_mfma_lds_ok", "attention_mfma_max_waves", "attention_mfma_qkv", "attention_mfma_qkv_ok", "attention_mfma_qkv_o_rows", "attention_f32_qkv_ok", "attention_mfma_rows", "attention_scalar",
+           "attention_mfma_lds_ok", "attention_mfma_max_waves", "attention_mfma_qkv", "attention_mfma_qkv_ok", "attention_mfma_qkv_o_rows", "attention_merge_o", "attention_merge_o_rows", "attention_f32_qkv_ok", "attention_mfma_rows", "attention_scalar",
            "attention_tile_tokens", "bias_add", "compute_units", "disable_library_tuning", "dtype_code", "embedding",
            "enable_library_tuning", "fragment_order", "gemm", "gemm_mfma_fp32", "gemm_mfma_fp32_sums", "gemm_mfma_fp32_splits", "gemm_fp32_gated", "gemm_fp32_tile", "gemm_fp32_tile_splits", "gemm_fp32_stream", "gemm_fp32_stream_plan", "GEMM_FP32_WHOLE", "GEMM_FP32_GATED", "GEMM_FP32_SUMS", "gemm_mfma_skinny", "gemm_mfma_skinny_rope", "gemm_mfma_wide",
            "gemm_mfma_tile", "gemm_mfma_tile_gated", "gemm_mfma_stream", "gemm_mfma_block", "gemm_block_plan", "GEMM_BLOCK_PLAIN", "GEMM_BLOCK_SUMS", "gemm_mfma_normed", "gemm_normed_takes", "gemm_stream_plan", "GEMM_STREAM_SUMS", "GEMM_STREAM_GATED", "GEMM_STREAM_POINT", "GEMM_STREAM_PLAN_ACT", "GEMM_STREAM_PLAN_ONE", "gemm_tile_plan", "gemm_mfma_wide_best_splits", "gemm_mfma_wide_splits_ok", "gemm_mfma_wide_swiglu", "gemm_mfma_wide_takes", "library_mm", "library_tuning_enabled", "load", "random_fill", "residual_add",

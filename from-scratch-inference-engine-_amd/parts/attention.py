@@ -819,12 +819,22 @@ class GQAttention(Mixer):
             return False
         return self._sums_will_do(ctx.compute_dtype, cache, ctx.plan(self.planner()), self._fused_table(ctx)[0])
 
+    # Up to so many items a token, or as many as a captured graph has room for at least, the launch that merges them makes the output projection (every workgroup of it merges a kv head's records again): one request of
+    # the 0.5B shape, 24 steps behind 2,000 keys (32 items) 18.06 ms with two launches, 16.70 with one, behind 7,000 (64) 34.95 and 35.04
+    most_records_with_o = 32
+
     def _rows_in_attention(self, x, ctx, cache, plan) -> int:
-        """Rows a wave of the output projection where attention's own workgroups make it (a step of one or two requests with short
-        items, whose next norm is made by the product behind it and takes a slice a kv head), or 0."""
-        if (not self.n_kv <= getattr(ctx, "sums_most", 0) or not getattr(ctx, "partial_sums_ok", False) or plan.n_partial or plan.waves != 1
+        """Rows a wave of the output projection where attention's own workgroups make it, or those that merge its items (a step of one or two
+        requests, whose next norm is made by the product behind it and takes a slice a kv head), or 0."""
+        if (not self.n_kv <= getattr(ctx, "sums_most", 0) or not getattr(ctx, "partial_sums_ok", False)
                 or x.dtype != torch.bfloat16 or self._slopes is not None or self.query_temperature is not None or self.o.bias is not None or type(self.o) is not Linear
                 or self.o.weight.dtype != torch.bfloat16 or not self.o.weight.is_contiguous() or self.o.weight.data_ptr() % 16):
+            return 0
+        if plan.n_partial:
+            # cut items: the launch that merges them makes it, where every token is merged by a few records
+            return (ops.attention_merge_o_rows(plan.n_merges, self.n_heads, self.n_kv, self.head_dim, self.hidden_size)
+                    if plan.n_merges == x.shape[0] and plan.n_small <= max(self.most_records_with_o * x.shape[0], ops.compute_units() // self.n_kv // 4) else 0)
+        if plan.waves != 1:
             return 0
         return ops.attention_mfma_qkv_o_rows(plan.n_small, self.n_heads, self.n_kv, self.head_dim, cache.page_size, self.hidden_size)
 
@@ -846,7 +856,7 @@ class GQAttention(Mixer):
         if sums is None:
             return None
         rows = self._rows_in_attention(x, ctx, cache, plan)
-        if rows:
+        if rows and not plan.n_partial:
             out = torch.empty((self.n_kv, x.shape[0], self.hidden_size), dtype=torch.float32, device=x.device)
             return ops.attention_mfma_qkv(sums, self.qkv.bias, table, cache.slots, cache.k_pool, cache.v_pool, cache.block_tables,
                                           plan.items, plan.n_small, out, None, self.n_heads, self.n_kv, self.head_dim, self.window,
@@ -860,6 +870,8 @@ class GQAttention(Mixer):
                                cache.block_tables, plan.items, plan.n_small, out, partials, self.n_heads, self.n_kv,
                                self.head_dim, self.window, self.scale, waves=plan.waves, short_items=getattr(plan, "short_items", False), slopes=self._slopes,
                                row_scale=self._row_scale(ctx))
+        if rows:
+            return ops.attention_merge_o(partials, plan.merges, plan.n_merges, out, self.o.weight, rows, self.n_heads, self.n_kv, self.head_dim)
         if plan.n_merges:
             ops.attention_merge(partials, plan.merges, plan.n_merges, out, self.n_heads, self.head_dim)
         return out

@@ -1,0 +1,61 @@
+"""The output projection in the launch that merges a decode step's cut items: the heads of the merge alone, times the weight in float32."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from from_scratch_inference_engine_amd import ops
+
+    ops.load()
+    return ops
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 4])
+@pytest.mark.parametrize("heads, kv, hd, n, splits", [
+    (14, 2, 64, 896, [3, 8]), (12, 2, 128, 1536, [1, 9]),
+    (32, 2, 128, 37, [2, 0, 30]),          # sixteen heads a kv head, two a wave; a token that attention has left whole
+    (3, 3, 64, 16, [32, 0]), (1, 1, 64, 1, [5]),
+])
+def test_sums(ops, rows, heads, kv, hd, n, splits):
+    t, g = len(splits), torch.Generator().manual_seed(heads + n)
+    slots = sum(splits)
+    records = torch.randn(slots, heads, hd + 2, generator=g)
+    records[..., hd + 1] = records[..., hd + 1].abs() + 0.5   # the denominators
+    records[:, 0, hd] = -float("inf")                          # a head that has seen no key in any record: nothing, not NaN
+    records[:, 0, :hd] = records[:, 0, hd + 1] = 0
+    if max(splits) > 2:
+        at = sum(splits[:splits.index(max(splits))])
+        records[at + 1, -1, hd] = -float("inf")                # and one that has seen none in one of them
+        records[at + 1, -1, :hd] = records[at + 1, -1, hd + 1] = 0
+    order = list(range(t))[::-1]                                # (the rows in any order, their records one after the other)
+    merges = torch.tensor([(r, sum(splits[:r]), splits[r], 1) for r in order], dtype=torch.int32).cuda()
+    weight = torch.randn(n, heads * hd, generator=g).to(torch.bfloat16).cuda()
+    whole = torch.randn(t, heads * hd, generator=g).to(torch.bfloat16).cuda()
+    partials = records.reshape(-1).cuda()
+    merged = whole.clone()
+    ops.attention_merge(partials, merges, t, merged, heads, hd)
+    got = ops.attention_merge_o(partials, merges, t, whole, weight, rows, heads, kv, hd)
+    x = merged.double().view(t, kv, -1).transpose(0, 1).contiguous()
+    w = weight.double().view(n, kv, -1).permute(1, 2, 0).contiguous()
+    # (the merge's arithmetic is attention_merge's, so its bits; what is left is a float32 sum of heads / kv * head_dim products)
+    bound = torch.bmm(x.abs(), w.abs()) * (heads // kv * hd) * 2.0 ** -24 + 1e-30
+    assert ((got.double() - torch.bmm(x, w)).abs() <= bound).all() and got.isfinite().all()
+
+
+def test_rule_and_refusals(ops):
+    rows = ops.attention_merge_o_rows
+    assert rows(1, 14, 2, 64, 896) == 1 and rows(2, 14, 2, 64, 896) == 2 and rows(ops.compute_units(), 14, 2, 64, 896) == 0
+    assert rows(1, 34, 2, 64, 896) == 0 and rows(1, 14, 2, 96, 896) == 0 and rows(0, 14, 2, 64, 896) == 0 and rows(1, 16, 16, 128, 8192) == 0
+
+    def call(heads=2, hd=64, cols=128, rows=1, n=8):
+        return ops.attention_merge_o(torch.zeros(heads * (hd + 2)).cuda(), torch.zeros(1, 4, dtype=torch.int32).cuda(), 1, torch.zeros(1, heads * hd, dtype=torch.bfloat16).cuda(),
+                                     torch.ones(n, cols, dtype=torch.bfloat16).cuda(), rows, heads, 1, hd)
+
+    assert call().eq(0).all()
+    for bad in (dict(rows=0), dict(rows=5), dict(hd=96, cols=192), dict(heads=17, cols=17 * 64), dict(cols=64)):
+        with pytest.raises(ops.KernelError):
+            call(**bad)
