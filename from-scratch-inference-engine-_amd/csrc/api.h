@@ -335,10 +335,10 @@ int fsie_attention_mfma_qkv_o(const float* sums, int n_parts, int n_tokens, cons
                               int max_pages, const int32_t* items, int n_items, const void* o_weight, int o_rows, float* o_sums,
                               int rows_of_wave, int n_heads, int n_kv, int head_dim, int page_size, int window, float scale,
                               hipStream_t stream);
-// fsie_attention_merge with the output projection behind it (bfloat16; rows_of_wave as above)
+// fsie_attention_merge with the output projection behind it (rows_of_wave as above)
 int fsie_attention_merge_o_rows(int n_merges, int n_heads, int n_kv, int head_dim, int o_rows, int units);
 int fsie_attention_merge_o(const float* partials, const int32_t* merges, int n_merges, int n_tokens, const void* heads, const void* o_weight,
-                           int o_rows, float* o_sums, int rows_of_wave, int n_heads, int n_kv, int head_dim, hipStream_t stream);
+                           int o_rows, float* o_sums, int rows_of_wave, int n_heads, int n_kv, int head_dim, int dtype, hipStream_t stream);
 int fsie_attention_mfma_lds_ok(int head_dim, int page_size);
 int fsie_attention_mfma_lds(const void* q, int64_t q_stride, const void* k_pool, const void* v_pool,
                             const int32_t* block_tables, int max_pages, const int32_t* items, const int32_t* groups,

@@ -1,12 +1,14 @@
-// The merge of a decode step's cut items (attention_merge, attention_scalar.hip) with the output projection behind it, for one or two tokens.
+// The merge of a decode step's cut items (attention_merge, attention_scalar.hip) with the output projection behind it, for a few tokens.
 //
 // Such a step is bound by its launches: the merge of a few records a head is 2.3 to 4 us, nearly all of it the launch and one trip to memory, and the
 // projection behind it as much.  Here a workgroup takes a kv head of a token: a wave merges a head (the arithmetic and the order of attention_merge), the heads, rounded to
-// 16 bits, meet in LDS, and each wave multiplies them by ROWS rows of the projection, which it has asked for behind the records.  Every workgroup of a kv head
+// 16 bits where the heads are, meet in LDS, and each wave multiplies them by ROWS rows of the projection, which it has asked for behind the records.  Every workgroup of a kv head
 // merges the same records again (2 KB a split for seven heads of 64), which costs less than a launch while all workgroups are on the chip at once.
 // The result is float32 sums [n_kv][tokens][o_rows], a slice a kv head, for the norm that adds them up.
 // 24 steps, ms, two launches / this: one request of the 0.5B shape (24 layers) behind 300 keys 16.09 / 15.12, 600 16.28 / 15.04, 2,000 18.06 / 16.70, two behind 400 16.45 / 15.69, behind
 // 2,000 22.49 / 21.39; 12 layers of hidden size 1,536, 12 heads on 2 of 128, one behind 400 12.26 / 11.44; of 1,024, 16 on 4 of 64, behind 600 10.45 / 9.77.
+// In front of a norm of its own (three and four requests, float32): three of the 0.5B shape behind 300 to 500 keys 18.26 / 17.74; in float32 four behind 40 to 301
+// 26.66 / 25.79, one behind 1,500 35.31 / 33.76, four behind 400 to 800 42.13 / 41.23.
 #include "common.h"
 #include "api.h"
 
@@ -17,13 +19,43 @@ namespace {
 constexpr int kMergeWaves = 8;
 constexpr int kAhead = 8;  // records under way
 
-// DIMS = head_dim / 64.
-template <int DIMS, int ROWS>
+// Eight values of the weight or of the heads, and their products added up in order.
+template <typename T>
+struct Eight;
+template <>
+struct Eight<bf16_t> {
+    uint4 raw;
+    __device__ void load(const bf16_t* p) { raw = *reinterpret_cast<const uint4*>(p); }
+    __device__ void store(bf16_t* p) const { *reinterpret_cast<uint4*>(p) = raw; }
+    __device__ float dot(const Eight& o) const {
+        const uint32_t a[4] = {raw.x, raw.y, raw.z, raw.w}, b[4] = {o.raw.x, o.raw.y, o.raw.z, o.raw.w};
+        float z = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            z = fmaf(__uint_as_float(a[i] << 16), __uint_as_float(b[i] << 16), z);
+            z = fmaf(__uint_as_float(a[i] & 0xffff0000u), __uint_as_float(b[i] & 0xffff0000u), z);
+        }
+        return z;
+    }
+};
+template <>
+struct Eight<float> {
+    float4 lo, hi;
+    __device__ void load(const float* p) { lo = *reinterpret_cast<const float4*>(p), hi = *reinterpret_cast<const float4*>(p + 4); }
+    __device__ void store(float* p) const { *reinterpret_cast<float4*>(p) = lo, *reinterpret_cast<float4*>(p + 4) = hi; }
+    __device__ float dot(const Eight& o) const {
+        float z = fmaf(lo.w, o.lo.w, fmaf(lo.z, o.lo.z, fmaf(lo.y, o.lo.y, lo.x * o.lo.x)));
+        return fmaf(hi.w, o.hi.w, fmaf(hi.z, o.hi.z, fmaf(hi.y, o.hi.y, fmaf(hi.x, o.hi.x, z))));
+    }
+};
+
+// T: what the heads and the weight are; DIMS = head_dim / 64.
+template <typename T, int DIMS, int ROWS>
 __global__ __launch_bounds__(64 * kMergeWaves) void attention_merge_o_kernel(
-    const float* __restrict__ partials, const int32_t* __restrict__ merges, const bf16_t* __restrict__ heads, const bf16_t* __restrict__ o_weight,
+    const float* __restrict__ partials, const int32_t* __restrict__ merges, const T* __restrict__ heads, const T* __restrict__ o_weight,
     float* __restrict__ o_sums, int n_heads, int group, int o_rows, int64_t part_stride) {
     constexpr int HD = 64 * DIMS, LOADS = 16 * HD / 8 / 64;  // a row's loads of eight values a lane (sixteen heads at most)
-    __shared__ __align__(16) bf16_t x[16 * HD];
+    __shared__ __align__(16) T x[16 * HD];
     const int32_t* mi = merges + static_cast<int64_t>(blockIdx.z) * FSIE_ATTN_MERGE_INTS;
     const int row = mi[0], first = mi[1], n_splits = mi[2], stride = mi[3];
     const int kvh = blockIdx.y, h0 = kvh * group;
@@ -47,13 +79,13 @@ __global__ __launch_bounds__(64 * kMergeWaves) void attention_merge_o_kernel(
         l = rec0[min(lane, n_splits - 1) * rec_step + HD + 1];
         ask(rec0, 0, n_splits);
     }
-    uint4 w[ROWS][LOADS];
+    Eight<T> w[ROWS][LOADS];
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
-        const bf16_t* at = o_weight + (static_cast<int64_t>(min(o_first + r, o_rows - 1)) * n_heads + h0) * HD;
+        const T* at = o_weight + (static_cast<int64_t>(min(o_first + r, o_rows - 1)) * n_heads + h0) * HD;
 #pragma unroll
         for (int u = 0; u < LOADS; ++u)
-            if (u == 0 || u * 64 < units) w[r][u] = *reinterpret_cast<const uint4*>(at + min(u * 64 + lane, units - 1) * 8);
+            if (u == 0 || u * 64 < units) w[r][u].load(at + min(u * 64 + lane, units - 1) * 8);
     }
     __builtin_amdgcn_sched_barrier(0);
     if (cut) {
@@ -89,11 +121,14 @@ __global__ __launch_bounds__(64 * kMergeWaves) void attention_merge_o_kernel(
             }
             const float inv = denom > 0.f ? 1.0f / denom : 0.f;
 #pragma unroll
-            for (int i = 0; i < DIMS; ++i) x[h * HD + lane + 64 * i] = from_float<bf16_t>(a[i] * inv);
+            for (int i = 0; i < DIMS; ++i) x[h * HD + lane + 64 * i] = from_float<T>(a[i] * inv);
         }
     } else {
-        for (int u = threadIdx.x; u < units; u += 64 * kMergeWaves)
-            *reinterpret_cast<uint4*>(x + u * 8) = *reinterpret_cast<const uint4*>(heads + (static_cast<int64_t>(row) * n_heads + h0) * HD + u * 8);
+        for (int u = threadIdx.x; u < units; u += 64 * kMergeWaves) {
+            Eight<T> e;
+            e.load(heads + (static_cast<int64_t>(row) * n_heads + h0) * HD + u * 8);
+            e.store(x + u * 8);
+        }
     }
     __syncthreads();
     float sum[ROWS];
@@ -103,17 +138,11 @@ __global__ __launch_bounds__(64 * kMergeWaves) void attention_merge_o_kernel(
     for (int u = 0; u < LOADS; ++u) {
         if (u > 0 && u * 64 >= units) break;  // (the same for the whole workgroup)
         const int unit = u * 64 + lane;
-        const uint4 xv = *reinterpret_cast<const uint4*>(x + min(unit, units - 1) * 8);
-        const uint32_t xs[4] = {xv.x, xv.y, xv.z, xv.w};
+        Eight<T> xv;
+        xv.load(x + min(unit, units - 1) * 8);
 #pragma unroll
         for (int r = 0; r < ROWS; ++r) {
-            const uint32_t ws[4] = {w[r][u].x, w[r][u].y, w[r][u].z, w[r][u].w};
-            float more = 0.f;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                more = fmaf(__uint_as_float(xs[i] << 16), __uint_as_float(ws[i] << 16), more);
-                more = fmaf(__uint_as_float(xs[i] & 0xffff0000u), __uint_as_float(ws[i] & 0xffff0000u), more);
-            }
+            const float more = xv.dot(w[r][u]);
             sum[r] += unit < units ? more : 0.f;
         }
     }
@@ -138,28 +167,33 @@ extern "C" int fsie_attention_merge_o_rows(int n_merges, int n_heads, int n_kv, 
     return 0;
 }
 
-// merges [n_merges], records: as fsie_attention_merge.  A token whose merge has no splits: its heads stand whole in `heads` [tokens][n_heads head_dim] (bfloat16).  o_weight
-// [o_rows][n_heads head_dim] (bfloat16, rows without gaps); o_sums [n_kv][n_tokens][o_rows].
+// merges [n_merges], records: as fsie_attention_merge.  A token whose merge has no splits: its heads stand whole in `heads` [tokens][n_heads head_dim].  o_weight
+// [o_rows][n_heads head_dim] (rows without gaps, of the heads' type `dtype`); o_sums [n_kv][n_tokens][o_rows].
 extern "C" int fsie_attention_merge_o(const float* partials, const int32_t* merges, int n_merges, int n_tokens, const void* heads, const void* o_weight,
-                                      int o_rows, float* o_sums, int rows_of_wave, int n_heads, int n_kv, int head_dim, hipStream_t stream) {
+                                      int o_rows, float* o_sums, int rows_of_wave, int n_heads, int n_kv, int head_dim, int dtype, hipStream_t stream) {
     FSIE_REQUIRE(n_merges >= 0 && n_tokens >= 0 && o_rows > 0 && n_heads > 0 && n_kv > 0 && n_heads % n_kv == 0 && n_heads / n_kv <= 16,
                  "attention_merge_o: bad sizes, %d heads on %d, %d rows", n_heads, n_kv, o_rows);
     FSIE_REQUIRE((head_dim == 64 || head_dim == 128) && rows_of_wave >= 1 && rows_of_wave <= 4, "attention_merge_o: heads of %d, %d rows a wave", head_dim, rows_of_wave);
     FSIE_REQUIRE(partials && merges && heads && o_weight && o_sums && reinterpret_cast<uintptr_t>(heads) % 16 == 0 && reinterpret_cast<uintptr_t>(o_weight) % 16 == 0,
                  "attention_merge_o: heads and weight must be 16-byte aligned");
+    FSIE_REQUIRE(dtype == FSIE_F32 || dtype == FSIE_BF16, "attention_merge_o: unknown dtype %d", dtype);
     if (n_merges == 0) return 0;
     const dim3 grid(static_cast<unsigned>(ceil_div64(o_rows, kMergeWaves * rows_of_wave)), n_kv, n_merges);
-#define FSIE_MERGE_O(D, R)                                                                                             \
-    attention_merge_o_kernel<D, R><<<grid, 64 * kMergeWaves, 0, stream>>>(partials, merges, static_cast<const bf16_t*>(heads), static_cast<const bf16_t*>(o_weight), \
-                                                                          o_sums, n_heads, n_heads / n_kv, o_rows, static_cast<int64_t>(n_tokens) * o_rows)
-#define FSIE_MERGE_O_ROWS(D)                                                                                           \
+#define FSIE_MERGE_O(T, D, R)                                                                                          \
+    attention_merge_o_kernel<T, D, R><<<grid, 64 * kMergeWaves, 0, stream>>>(partials, merges, static_cast<const T*>(heads), static_cast<const T*>(o_weight), \
+                                                                             o_sums, n_heads, n_heads / n_kv, o_rows, static_cast<int64_t>(n_tokens) * o_rows)
+#define FSIE_MERGE_O_ROWS(T, D)                                                                                        \
     switch (rows_of_wave) {                                                                                            \
-        case 1: FSIE_MERGE_O(D, 1); break;                                                                             \
-        case 2: FSIE_MERGE_O(D, 2); break;                                                                             \
-        case 3: FSIE_MERGE_O(D, 3); break;                                                                             \
-        default: FSIE_MERGE_O(D, 4); break;                                                                            \
+        case 1: FSIE_MERGE_O(T, D, 1); break;                                                                          \
+        case 2: FSIE_MERGE_O(T, D, 2); break;                                                                          \
+        case 3: FSIE_MERGE_O(T, D, 3); break;                                                                          \
+        default: FSIE_MERGE_O(T, D, 4); break;                                                                         \
     }
-    if (head_dim == 64) FSIE_MERGE_O_ROWS(1) else FSIE_MERGE_O_ROWS(2)
+    if (dtype == FSIE_F32) {
+        if (head_dim == 64) FSIE_MERGE_O_ROWS(float, 1) else FSIE_MERGE_O_ROWS(float, 2)
+    } else {
+        if (head_dim == 64) FSIE_MERGE_O_ROWS(bf16_t, 1) else FSIE_MERGE_O_ROWS(bf16_t, 2)
+    }
 #undef FSIE_MERGE_O_ROWS
 #undef FSIE_MERGE_O
     FSIE_CHECK_LAUNCH("attention_merge_o");

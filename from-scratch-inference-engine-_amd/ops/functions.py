@@ -1243,21 +1243,21 @@ def attention_merge_o_rows(n_merges: int, n_heads: int, n_kv: int, head_dim: int
 
 def attention_merge_o(partials: torch.Tensor, merges: torch.Tensor, n_merges: int, heads: torch.Tensor, o_weight: torch.Tensor, o_rows: int,
                       n_heads: int, n_kv: int, head_dim: int) -> torch.Tensor:
-    """``attention_merge`` and the product with the output projection ``o_weight`` [N, heads head_dim] (bfloat16) in one launch: float32 partial sums
-    [kv heads, T, N], of which the tokens that ``merges`` names are written.  ``heads`` [T, heads head_dim] (bfloat16) holds those of a token without
-    splits.  ``o_rows``: what ``attention_merge_o_rows`` says of the sizes."""
+    """``attention_merge`` and the product with the output projection ``o_weight`` [N, heads head_dim] in one launch: float32 partial sums
+    [kv heads, T, N], of which the tokens that ``merges`` names are written.  ``heads`` [T, heads head_dim] holds those of a token without
+    splits; it and the weight in bfloat16, or both in float32.  ``o_rows``: what ``attention_merge_o_rows`` says of the sizes."""
     _need(partials, "attention partials", dtype=torch.float32, ndim=1)
     _need(merges, "attention merges", dtype=torch.int32, ndim=2)
     if merges.shape[1] != ATTN_MERGE_INTS or merges.shape[0] < n_merges:
         raise KernelError(f"attention merges: shape {tuple(merges.shape)} does not hold {n_merges} items")
-    _need(heads, "attention heads", dtype=torch.bfloat16, ndim=2)
-    _need(o_weight, "output projection", dtype=torch.bfloat16, ndim=2)
+    _need(heads, "attention heads", ndim=2)
+    _need(o_weight, "output projection", dtype=heads.dtype, ndim=2)
     t, width = heads.shape
     if width != n_heads * head_dim or o_weight.shape[1] != width:
         raise KernelError(f"output projection: {o_weight.shape[1]} columns, rows of {width} for {n_heads} heads of {head_dim}")
     out = torch.empty((n_kv, t, o_weight.shape[0]), dtype=torch.float32, device=heads.device)
     check(load().fsie_attention_merge_o(partials.data_ptr(), merges.data_ptr(), n_merges, t, heads.data_ptr(), o_weight.data_ptr(), o_weight.shape[0],
-                                        out.data_ptr(), int(o_rows), n_heads, n_kv, head_dim, _stream()))
+                                        out.data_ptr(), int(o_rows), n_heads, n_kv, head_dim, dtype_code(heads.dtype), _stream()))
     return out
 
 

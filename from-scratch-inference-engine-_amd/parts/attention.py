@@ -824,17 +824,17 @@ class GQAttention(Mixer):
     most_records_with_o = 32
 
     def _rows_in_attention(self, x, ctx, cache, plan) -> int:
-        """Rows a wave of the output projection where attention's own workgroups make it, or those that merge its items (a step of one or two
-        requests, whose next norm is made by the product behind it and takes a slice a kv head), or 0."""
-        if (not self.n_kv <= getattr(ctx, "sums_most", 0) or not getattr(ctx, "partial_sums_ok", False)
-                or x.dtype != torch.bfloat16 or self._slopes is not None or self.query_temperature is not None or self.o.bias is not None or type(self.o) is not Linear
-                or self.o.weight.dtype != torch.bfloat16 or not self.o.weight.is_contiguous() or self.o.weight.data_ptr() % 16):
+        """Rows a wave of the output projection where attention's own workgroups make it, or those that merge its items (a step of few
+        requests, whose next norm takes a slice a kv head), or 0."""
+        most = getattr(ctx, "sums_most", 0) if getattr(ctx, "sums_in_one", False) else 4  # (a norm of its own: what it adds up as fast as it would the projection's own slices)
+        if (self.n_kv > most or not getattr(ctx, "partial_sums_ok", False) or self._slopes is not None or self.query_temperature is not None or self.o.bias is not None or type(self.o) is not Linear
+                or self.o.weight.dtype != x.dtype or not self.o.weight.is_contiguous() or self.o.weight.data_ptr() % 16):
             return 0
         if plan.n_partial:
             # cut items: the launch that merges them makes it, where every token is merged by a few records
             return (ops.attention_merge_o_rows(plan.n_merges, self.n_heads, self.n_kv, self.head_dim, self.hidden_size)
                     if plan.n_merges == x.shape[0] and plan.n_small <= max(self.most_records_with_o * x.shape[0], ops.compute_units() // self.n_kv // 4) else 0)
-        if plan.waves != 1:
+        if plan.waves != 1 or x.dtype != torch.bfloat16:
             return 0
         return ops.attention_mfma_qkv_o_rows(plan.n_small, self.n_heads, self.n_kv, self.head_dim, cache.page_size, self.hidden_size)
 

@@ -14,13 +14,14 @@ def ops():
     return ops
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("rows", [1, 2, 3, 4])
 @pytest.mark.parametrize("heads, kv, hd, n, splits", [
     (14, 2, 64, 896, [3, 8]), (12, 2, 128, 1536, [1, 9]),
     (32, 2, 128, 37, [2, 0, 30]),          # sixteen heads a kv head, two a wave; a token that attention has left whole
     (3, 3, 64, 16, [32, 0]), (1, 1, 64, 1, [5]),
 ])
-def test_sums(ops, rows, heads, kv, hd, n, splits):
+def test_sums(ops, dtype, rows, heads, kv, hd, n, splits):
     t, g = len(splits), torch.Generator().manual_seed(heads + n)
     slots = sum(splits)
     records = torch.randn(slots, heads, hd + 2, generator=g)
@@ -33,8 +34,8 @@ def test_sums(ops, rows, heads, kv, hd, n, splits):
         records[at + 1, -1, :hd] = records[at + 1, -1, hd + 1] = 0
     order = list(range(t))[::-1]                                # (the rows in any order, their records one after the other)
     merges = torch.tensor([(r, sum(splits[:r]), splits[r], 1) for r in order], dtype=torch.int32).cuda()
-    weight = torch.randn(n, heads * hd, generator=g).to(torch.bfloat16).cuda()
-    whole = torch.randn(t, heads * hd, generator=g).to(torch.bfloat16).cuda()
+    weight = torch.randn(n, heads * hd, generator=g).to(dtype).cuda()
+    whole = torch.randn(t, heads * hd, generator=g).to(dtype).cuda()
     partials = records.reshape(-1).cuda()
     merged = whole.clone()
     ops.attention_merge(partials, merges, t, merged, heads, hd)
@@ -51,11 +52,11 @@ def test_rule_and_refusals(ops):
     assert rows(1, 14, 2, 64, 896) == 1 and rows(2, 14, 2, 64, 896) == 2 and rows(ops.compute_units(), 14, 2, 64, 896) == 0
     assert rows(1, 34, 2, 64, 896) == 0 and rows(1, 14, 2, 96, 896) == 0 and rows(0, 14, 2, 64, 896) == 0 and rows(1, 16, 16, 128, 8192) == 0
 
-    def call(heads=2, hd=64, cols=128, rows=1, n=8):
+    def call(heads=2, hd=64, cols=128, rows=1, n=8, dtype=torch.bfloat16):
         return ops.attention_merge_o(torch.zeros(heads * (hd + 2)).cuda(), torch.zeros(1, 4, dtype=torch.int32).cuda(), 1, torch.zeros(1, heads * hd, dtype=torch.bfloat16).cuda(),
-                                     torch.ones(n, cols, dtype=torch.bfloat16).cuda(), rows, heads, 1, hd)
+                                     torch.ones(n, cols, dtype=dtype).cuda(), rows, heads, 1, hd)
 
     assert call().eq(0).all()
-    for bad in (dict(rows=0), dict(rows=5), dict(hd=96, cols=192), dict(heads=17, cols=17 * 64), dict(cols=64)):
+    for bad in (dict(rows=0), dict(rows=5), dict(hd=96, cols=192), dict(heads=17, cols=17 * 64), dict(cols=64), dict(dtype=torch.float32)):
         with pytest.raises(ops.KernelError):
             call(**bad)
