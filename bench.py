@@ -580,7 +580,7 @@ def main() -> int:
             "global_batch": args.batch, "seq_len": context, "prompt_len": args.prompt_len,
             "mean_decode_context": mean_ctx, "kv_block": page, "parallelism": "single GPU",
             "library_gemm_tuning": bool(not args.no_tune and args.dtype == "bf16"),
-            "streamed_weight_copies": bool(not args.no_streamed_copies and args.dtype == "bf16"),
+            "streamed_weight_copies": bool(not args.no_streamed_copies),
         },
         "prefill": prefill,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_BYTES_PER_S / 1e9, "unit": "GB/s",

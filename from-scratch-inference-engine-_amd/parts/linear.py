@@ -17,7 +17,9 @@ class Linear:
 
     float32: the engine's own kernels only (true 32-bit products and sums): vector FMA kernels for 1 and 2
     rows, and from 3 rows on the matrix cores' float32 instruction, which rounds nothing: a kernel that
-    streams W up to 64 rows, one of 64 x 64 tiles beyond; residual projections leave partial sums.
+    streams W up to 64 rows, one of 64 x 64 tiles beyond; residual projections leave partial sums.  A weight of 2 MB and more
+    has a second copy in the order of that instruction's fragments (``streamed32``), from which a third kernel takes up to
+    64 rows, one and two among them (``ops.gemm_fp32_stream_plan``).
     bfloat16: up to 16 rows (decoding) the engine's matrix-core kernel that streams the weight
     once; its sibling that shares x through LDS for float32 results of 8 to 64 rows (the logits;
     beyond 64 rows the library with a float32 result), for the residual projections
