@@ -136,10 +136,12 @@ extern "C" int fsie_attention_mfma_qkv(const float* sums, int n_parts, int n_tok
 // for 32 to 40 steps: 14 heads on 2 of 64, hidden size 896 23.23 / 21.60 with two rows (180 workgroups; with three 21.70, four 21.79), 24.23 / 23.06 with
 // three (240; with two, 360, 24.27); 12 on 2 of 128, hidden size 1,536 14.61 / 13.66 with three (206; with two, 308, 15.42, with four, 154, 13.77), two
 // requests 15.28 / 16.8 to 18.7 (308 and more); 16 on 4 of 64, hidden size 1,024 7.39 / 6.95 with four (208); 8 on 1 of 128, 1,024 7.90 / 7.39.  More rows a wave keep more heads within the units and are slower there: 16 on 8 of 64,
-// hidden size 1,024 12.5 / 12.4 with eight rows (208), 15.1 / 17.0 at 2,048; 12 on 12 at 768 9.4 / 9.9.
+// hidden size 1,024 12.5 / 12.4 with eight rows (208), 15.1 / 17.0 at 2,048; 12 on 12 at 768 9.4 / 9.9.  Every token reads the weight again, which up to some 16 MB of it
+// all costs less than the launch: 20 on 2 of 128, 2,560 (13 MB) 12.30 / 12.04; 16 on 1 of 128, 2,304, one token (9) 10.96 / 10.61, two (19) 11.33 / 11.43.
 extern "C" int fsie_attention_mfma_qkv_o_rows(int n_items, int n_heads, int n_kv, int head_dim, int page_size, int o_rows, int units) {
     if (n_items <= 0 || n_heads <= 0 || n_kv <= 0 || n_heads % n_kv || n_heads / n_kv > 16 || o_rows <= 0 || units <= 0) return 0;
     if ((head_dim != 64 && head_dim != 128) || !fsie_attention_mfma_qkv_ok(head_dim, page_size)) return 0;
+    if (2.0 * n_items * o_rows * n_heads * head_dim > 16e6) return 0;
     for (int rows = 2; rows <= 4; ++rows)
         if (ceil_div64(o_rows, (fsie_attn::kShortWaves + 1) * rows) * n_kv * n_items <= units) return rows;
     return 0;

@@ -68,6 +68,7 @@ def test_rule(ops):
     units, rows = ops.compute_units(), ops.attention_mfma_qkv_o_rows
     assert rows(1, 14, 2, 64, 16, 896) == 2 and rows(2, 14, 2, 64, 16, 896) == 3 and rows(1, 12, 2, 128, 16, 1536) == 3
     assert rows(1, 16, 16, 128, 16, 2048) == 0 and rows(units, 14, 2, 64, 16, 896) == 0  # more workgroups than units
+    assert rows(1, 16, 1, 128, 16, 2304) == 2 and rows(2, 16, 1, 128, 16, 2304) == 0  # 9 MB of weights, and 19
     assert rows(1, 34, 2, 64, 16, 896) == 0 and rows(1, 14, 2, 96, 16, 896) == 0 and rows(1, 14, 2, 64, 12, 896) == 0 and rows(0, 14, 2, 64, 16, 896) == 0
 
 
