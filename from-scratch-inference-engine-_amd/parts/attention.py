@@ -131,6 +131,11 @@ class AttentionPlanner:
 
     short_waves = 4  # waves of the variant for short items
 
+    # Records of a token up to which the launch that merges them may make the output projection as well (every workgroup of it merges a kv head's records
+    # again): one request of the 0.5B shape, 24 steps behind 2,000 keys (32 items) 18.06 ms with two launches, 16.70 with one, behind 7,000
+    # (64) 34.95 and 35.04.  The merge by itself deals more than so many to four waves.
+    few_records = 32
+
     def _fills(self, items: int) -> bool:
         """Whether the matrix-core kernel's workgroups for so many items are more than the compute units.  Queries that are in memory
         already then go to the variant for short items whatever their length: all the waves of a head size hold so much of a unit that the
@@ -286,12 +291,13 @@ class AttentionPlanner:
 
     def graph_bucket(self, host):
         """What a captured graph of this step's shape must fix: the number of (small) work items,
-        the variant of the matrix-core kernel, whether its workgroups fill the units and (of the other kernel) the keys per item; None if the step has portions that do not fit
+        the variant of the matrix-core kernel, whether its workgroups fill the units and (of the other kernel) the keys per item, and where a token
+        has more than ``few_records`` items, a fourth value that says so; None if the step has portions that do not fit
         small items."""
         mfma = self.uses_mfma(host.compute_dtype, host.page_size)
         small_tokens = self.geometry(mfma)[0]
         split_keys = self.split_keys(host, mfma)
-        n, longest = 0, 1
+        n, longest, records = 0, 1, 0
         for s in range(host.n_seqs):
             if host.q_lens[s] > small_tokens:
                 return None
@@ -308,11 +314,13 @@ class AttentionPlanner:
             elif kept:
                 longest = max(longest, span + 32 * -(-kept // 32))
             n += mine
+            records = max(records, mine)
         if n == host.n_seqs:
             # every request is one whole item: no records, no merge.  A graph of its own: the merge that finds nothing to do costs
             # 1.5 us a layer (one request of the 0.5B shape, 61 tokens and 48 more, 37.3 ms, 35.5 without), the step from whole
             # to cut items one capture more in a batch's life
             return (n, self._graph_waves(longest) if mfma else 1, self._fills(n) if mfma else split_keys)
+        many = (True,) if records > self.few_records else ()
         if mfma:
             # items: a multiple of the number of requests and of a quarter of what gives every unit a
             # workgroup, so that one graph serves a batch while its requests grow: their items grow
@@ -322,9 +330,9 @@ class AttentionPlanner:
             group = self.n_heads // self.n_kv
             per_item = self.n_kv * -(-group // min(group, ops.attention_mfma_rows(self.head_dim, False)))
             step = max(host.n_seqs, units // per_item // 4, 1)
-            return (-(-n // step) * step, self._graph_waves(longest), self._fills(n))
+            return (-(-n // step) * step, self._graph_waves(longest), self._fills(n), *many)
         step = host.n_seqs * max(1, 1024 // split_keys)
-        return (-(-n // step) * step, 1, split_keys)
+        return (-(-n // step) * step, 1, split_keys, *many)
 
     def plan(self, host) -> Dict[str, object]:
         mfma = self.uses_mfma(host.compute_dtype, host.page_size)
@@ -431,9 +439,11 @@ class AttentionPlanner:
             waves = self._waves_for(max(it[5] - (it[4] & ~31) + (32 * -(-min(it[7] & ~(ATTN_KEEP_WALK | ATTN_POOL_WALK), it[4]) // 32)
                                                             if it[7] & ATTN_KEEP_WALK else 0) for it in small),
                                     ops.attention_mfma_max_waves(self.head_dim))
+        few_records = all(m[2] <= self.few_records for m in merges)
         if padded:
             # a captured graph launches fixed grids: pad with items and merges that do nothing
-            n_items, waves, fills = host.pad[self.key]
+            n_items, waves, fills, *many = host.pad[self.key]
+            few_records = not many
             if len(large) or len(small) > n_items:
                 raise RuntimeError("attention plan does not fit the captured graph")
             small += [(0, 0, 0, 0, 0, 0, -1, 0)] * (n_items - len(small))
@@ -448,6 +458,8 @@ class AttentionPlanner:
                 merged = {m[0] for m in merges}
                 merges += [(row, 0, 0, 0) for row in range(host.n_tokens) if row not in merged]
                 n_partial = (n_items + (host.n_seqs if two_pass else 0)) * small_tokens
+        single = all(host.q_lens[s] == 1 for s in range(host.n_seqs))  # one token a request
+        extra = {}
         # consecutive large tiles of one request, four at a time, for the kernel that shares the
         # keys of a block among four waves
         groups = np.zeros((0, 2), dtype=np.int64)
@@ -475,7 +487,6 @@ class AttentionPlanner:
             large = np.concatenate([large[~is_long], large[is_long]])
             n_long = int(is_long.sum())
         small_items = np.asarray(small, dtype=np.int64).reshape(-1, ATTN_ITEM_INTS)
-        extra = {}
         if self.pool:
             if padded:  # (a step of single tokens completes at most a block a request)
                 if len(pool_jobs) > host.n_seqs:
@@ -499,7 +510,8 @@ class AttentionPlanner:
                 large[:, 7] & ATTN_KEEP_WALK, np.minimum(large[:, 7] & ~(ATTN_KEEP_WALK | ATTN_POOL_WALK), large[:, 4]) + 15 & ~15, 0) > 64).any()),
             # float32: the items are cut, to no more than four blocks of 16 keys
             "short_items": not mfma and n_partial > 0 and split_keys <= 64,
-            "single": all(host.q_lens[s] == 1 for s in range(host.n_seqs)),  # one token a request
+            "single": single,
+            "few_records": few_records,  # (in a graph: of every step that it stands for)
         }
 
 
@@ -819,10 +831,6 @@ class GQAttention(Mixer):
             return False
         return self._sums_will_do(ctx.compute_dtype, cache, ctx.plan(self.planner()), self._fused_table(ctx)[0])
 
-    # Up to so many items a token, or as many as a captured graph has room for at least, the launch that merges them makes the output projection (every workgroup of it merges a kv head's records again): one request of
-    # the 0.5B shape, 24 steps behind 2,000 keys (32 items) 18.06 ms with two launches, 16.70 with one, behind 7,000 (64) 34.95 and 35.04
-    most_records_with_o = 32
-
     def _rows_in_attention(self, x, ctx, cache, plan) -> int:
         """Rows a wave of the output projection where attention's own workgroups make it, or those that merge its items (a step of few
         requests, whose next norm takes a slice a kv head), or 0."""
@@ -831,9 +839,9 @@ class GQAttention(Mixer):
                 or self.o.weight.dtype != x.dtype or not self.o.weight.is_contiguous() or self.o.weight.data_ptr() % 16):
             return 0
         if plan.n_partial:
-            # cut items: the launch that merges them makes it, where every token is merged by a few records
+            # cut items: the launch that merges them makes it, where every token is merged by few records
             return (ops.attention_merge_o_rows(plan.n_merges, self.n_heads, self.n_kv, self.head_dim, self.hidden_size)
-                    if plan.n_merges == x.shape[0] and plan.n_small <= max(self.most_records_with_o * x.shape[0], ops.compute_units() // self.n_kv // 4) else 0)
+                    if plan.n_merges == x.shape[0] and plan.few_records else 0)
         if plan.waves != 1 or x.dtype != torch.bfloat16:
             return 0
         return ops.attention_mfma_qkv_o_rows(plan.n_small, self.n_heads, self.n_kv, self.head_dim, cache.page_size, self.hidden_size)

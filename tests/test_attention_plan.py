@@ -283,3 +283,19 @@ def test_more_workgroups_than_units(heads, kv, n, keys, fills):
     host.pad = {planner.key: bucket}
     assert planner.plan(host)["fills"] == fills
     assert not planner.plan(Host([(keys - 1, 1)] * n, 16, torch.float32))["fills"]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_many_records_of_one_token_are_many_whatever_the_others_have(dtype):
+    """The launch that merges cut items makes the output projection up to 32 records a token: a long request beside short ones has
+    more than the step's mean.  A graph's plan says the same as its bucket, so that a replay never meets what the capture did not."""
+    planner = AttentionPlanner(14, 2, 64, None)
+    planner.compute_units = 256
+    for lens, few in (([300], True), ([60, 400], True), ([100, 7000], False), ([50, 50, 50, 6000], False), ([6000, 300, 300, 300], False), ([8000], False)):
+        host = Host([(n, 1) for n in lens], 16, dtype)
+        plan = planner.plan(host)
+        assert plan["few_records"] == few == (max(int(m[2]) for m in plan["merges"]) <= 32)
+        bucket = planner.graph_bucket(host)
+        assert bucket[3:] == (() if few else (True,))
+        host.pad = {planner.key: bucket}
+        assert planner.plan(host)["few_records"] == few
