@@ -54,6 +54,16 @@ def padded_tokens(n: int) -> int:
     return up if up - n <= max(64, n // 5) else n
 
 
+def padded_rows(n: int) -> int:
+    """Rows of the graph that serves a decode step of ``n`` requests: 1, 2, 4, 8, then multiples
+    of 16 (a tile of rows in the products) up to 128, which is what the engine's own products
+    take, above that of 32."""
+    if n <= 8:
+        return 1 << max(0, n - 1).bit_length()
+    step = 16 if n <= 128 else 32
+    return -(-n // step) * step
+
+
 class HostBatch:
     """Host view of the step, in the order of the entries."""
 
@@ -157,6 +167,8 @@ class StepContext:
         self.device = device
         self.n_tokens = host.n_tokens
         self.n_seqs = host.n_seqs
+        # rows of the graph that serves, or is going to serve, decode steps of so many requests
+        self.graph_rows = padded_rows(host.n_seqs)
         self.token_ids = self.positions = self.want_rows = None
         self.seq_slots = self.q_starts = self.past_lens = self.reset_slots = None
         # set by the model: every norm can add up a delta that comes as float32 partial sums

@@ -31,20 +31,10 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
-from .context import HostBatch, StepEntry, build_context, filler_entry
+from .context import HostBatch, StepEntry, build_context, filler_entry, padded_rows
 
 PAGE_BUCKET = 32  # block-table widths are at least this many pages (and powers of two)
 CAPTURE_AFTER = 3  # a shape is captured the n-th time it is asked for (read when a runner is made)
-
-
-def padded_rows(n: int) -> int:
-    """Rows of the graph that serves a decode step of ``n`` requests: 1, 2, 4, 8, then multiples
-    of 16 (a tile of rows in the products) up to 128, which is what the engine's own products
-    take, above that of 32."""
-    if n <= 8:
-        return 1 << max(0, n - 1).bit_length()
-    step = 16 if n <= 128 else 32
-    return -(-n // step) * step
 
 
 class _CollectorOff:

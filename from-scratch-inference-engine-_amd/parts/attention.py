@@ -136,6 +136,9 @@ class AttentionPlanner:
     # (64) 34.95 and 35.04.  The merge by itself deals more than so many to four waves.
     few_records = 32
 
+    def _units(self) -> int:
+        return self.compute_units if self.compute_units is not None else ops.compute_units()
+
     def _fills(self, items: int) -> bool:
         """Whether the matrix-core kernel's workgroups for so many items are more than the compute units.  Queries that are in memory
         already then go to the variant for short items whatever their length: all the waves of a head size hold so much of a unit that the
@@ -144,7 +147,7 @@ class AttentionPlanner:
         16 on 16 of 64, 64 of 40 8.1 / 14.4 / 6.3, 200 of 500 82 / 98 / 71; 32 on 4 of 32, 200 of 300 12.7 / 17.8 / 10.1.  At as many workgroups
         as units all waves are faster from 500 keys on (14 on 2 of 64, 128 of 1,000 16.0 / 19.5).  Where attention adds up q/k/v itself, too (64 of 3,000
         keys, 8 on 8 of 128, 134 / 141)."""
-        units = self.compute_units if self.compute_units is not None else ops.compute_units()
+        units = self._units()
         group = self.n_heads // self.n_kv
         return items * self.n_kv * -(-group // min(group, ops.attention_mfma_rows(self.head_dim, False))) > units > 0
 
@@ -177,7 +180,7 @@ class AttentionPlanner:
 
     def _split_keys(self, host, mfma: bool) -> int:
         small_tokens, _, longest = self.geometry(mfma)
-        units = self.compute_units if self.compute_units is not None else ops.compute_units()
+        units = self._units()
         both = self._small_keys(host, small_tokens, mfma)
         keys = [k for k, _ in both]
         group = self.n_heads // self.n_kv
@@ -326,7 +329,7 @@ class AttentionPlanner:
             # workgroup, so that one graph serves a batch while its requests grow: their items grow
             # longer, not more (the captured graph pads with empty items, whose workgroups leave at
             # once).  The length of the items is data of the step, not of the graph.
-            units = self.compute_units if self.compute_units is not None else ops.compute_units()
+            units = self._units()
             group = self.n_heads // self.n_kv
             per_item = self.n_kv * -(-group // min(group, ops.attention_mfma_rows(self.head_dim, False)))
             step = max(host.n_seqs, units // per_item // 4, 1)
@@ -460,6 +463,11 @@ class AttentionPlanner:
                 n_partial = (n_items + (host.n_seqs if two_pass else 0)) * small_tokens
         single = all(host.q_lens[s] == 1 for s in range(host.n_seqs))  # one token a request
         extra = {}
+        if not padded and single and not self.pool and 0 < len(merges) < host.n_tokens and host.n_tokens * self.n_kv <= self._units():
+            # every row once, as a graph merges them (those that need none by an empty merge), for the launch that multiplies by the output
+            # projection too: whether it stands for a step must not follow from whether the step is replayed
+            merged = {m[0] for m in merges}
+            extra["row_merges"] = np.asarray(merges + [(row, 0, 0, 0) for row in range(host.n_tokens) if row not in merged], dtype=np.int32)
         # consecutive large tiles of one request, four at a time, for the kernel that shares the
         # keys of a block among four waves
         groups = np.zeros((0, 2), dtype=np.int64)
@@ -838,13 +846,15 @@ class GQAttention(Mixer):
         if (self.n_kv > most or not getattr(ctx, "partial_sums_ok", False) or self._slopes is not None or self.query_temperature is not None or self.o.bias is not None or type(self.o) is not Linear
                 or self.o.weight.dtype != x.dtype or not self.o.weight.is_contiguous() or self.o.weight.data_ptr() % 16):
             return 0
+        # (by the rows of the graph that takes over from eager steps of this many, so that a request's sums stay what they are)
+        rows = getattr(ctx, "graph_rows", x.shape[0])
         if plan.n_partial:
-            # cut items: the launch that merges them makes it, where every token is merged by few records
-            return (ops.attention_merge_o_rows(plan.n_merges, self.n_heads, self.n_kv, self.head_dim, self.hidden_size)
-                    if plan.n_merges == x.shape[0] and plan.few_records else 0)
+            # cut items: the launch that merges them makes it, where every token has few records
+            every_row = plan.n_merges == x.shape[0] or hasattr(plan, "row_merges")
+            return ops.attention_merge_o_rows(rows, self.n_heads, self.n_kv, self.head_dim, self.hidden_size) if plan.few_records and every_row else 0
         if plan.waves != 1 or x.dtype != torch.bfloat16:
             return 0
-        return ops.attention_mfma_qkv_o_rows(plan.n_small, self.n_heads, self.n_kv, self.head_dim, cache.page_size, self.hidden_size)
+        return ops.attention_mfma_qkv_o_rows(rows, self.n_heads, self.n_kv, self.head_dim, cache.page_size, self.hidden_size)
 
     def _from_sums(self, x, ctx, cache, plan, fuse: bool, table) -> Optional[torch.Tensor]:
         """Attention of a step of one token a request straight from the q/k/v product's partial sums
@@ -879,7 +889,8 @@ class GQAttention(Mixer):
                                self.head_dim, self.window, self.scale, waves=plan.waves, short_items=getattr(plan, "short_items", False), slopes=self._slopes,
                                row_scale=self._row_scale(ctx))
         if rows:
-            return ops.attention_merge_o(partials, plan.merges, plan.n_merges, out, self.o.weight, rows, self.n_heads, self.n_kv, self.head_dim)
+            return ops.attention_merge_o(partials, getattr(plan, "row_merges", plan.merges), x.shape[0], out, self.o.weight, rows, self.n_heads, self.n_kv,
+                                         self.head_dim)
         if plan.n_merges:
             ops.attention_merge(partials, plan.merges, plan.n_merges, out, self.n_heads, self.head_dim)
         return out

@@ -299,3 +299,39 @@ def test_many_records_of_one_token_are_many_whatever_the_others_have(dtype):
         assert bucket[3:] == (() if few else (True,))
         host.pad = {planner.key: bucket}
         assert planner.plan(host)["few_records"] == few
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads, kv, hd", [(14, 2, 64), (12, 2, 128), (16, 1, 128), (16, 4, 64)])
+def test_an_eager_plan_and_a_graphs_plan_agree_on_what_the_output_projection_joins(dtype, heads, kv, hd):
+    """The launch that merges cut items makes the output projection where every row is merged and no token has many records.  Both
+    follow from the requests, not from whether the step is replayed: each row's merge is in either plan, and they say the same of the longest
+    one, by its own records, not by the step's mean (a long request beside short ones has more than its share)."""
+    from from_scratch_inference_engine_amd.engine.graphs import padded_rows
+
+    rng = random.Random(heads * hd)
+    planner = AttentionPlanner(heads, kv, hd, None)
+    planner.compute_units = 256
+    batches = [[60, 400], [600, 40], [2000, 40, 40], [100, 7000], [50, 50, 50, 6000], [6000, 300, 300, 300], [8000], [40], [40, 127, 214, 301]]
+    batches += [[rng.choice([rng.randint(0, 500), rng.randint(0, 8000)]) for _ in range(rng.choice([1, 2, 4]))] for _ in range(40)]
+    seen = set()
+    for lens in batches:
+        eager = planner.plan(Host([(n, 1) for n in lens], 16, dtype))
+        host = Host([(n, 1) for n in lens + [0] * (padded_rows(len(lens)) - len(lens))], 16, dtype)
+        host.pad = {planner.key: planner.graph_bucket(host)}
+        graph = planner.plan(host)
+        cut = eager["n_partial"] > 0
+        assert cut == (graph["n_partial"] > 0) and eager["few_records"] == graph["few_records"], lens
+        if not cut:
+            assert "row_merges" not in eager and not graph["n_merges"]
+            continue
+        mine = eager["row_merges"] if "row_merges" in eager else eager["merges"]
+        rows = [{int(m[0]): int(m[2]) for m in merges} for merges in (mine, graph["merges"])]
+        assert len(mine) == len(lens) and sorted(rows[0]) == list(range(len(lens))) and sorted(rows[1]) == list(range(host.n_tokens))
+        assert all(rows[0][r] == rows[1][r] for r in rows[0]), lens
+        assert eager["few_records"] == (max(rows[0].values()) <= 32), lens
+        seen.add(eager["few_records"])
+    assert seen == {True, False}
+    # portions, and steps whose rows are more than the workgroups that a launch has room for, are left alone
+    assert "row_merges" not in planner.plan(Host([(600, 1), (10, 40)], 16, dtype))
+    assert "row_merges" not in planner.plan(Host([(3, 1)] * 256 + [(9000, 1)], 16, dtype))
