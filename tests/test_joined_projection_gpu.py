@@ -1,10 +1,12 @@
-"""Models whose decode steps make the output projection in attention's launch or in the one that merges its items:
-replayed steps have the bits of eager ones."""
+"""Models whose decode steps make the output projection in attention's launch or in the one that merges its items: the plain model's logits, and
+replayed steps with the bits of eager ones."""
 
+import numpy as np
 import pytest
 import torch
 
 import helpers
+import plain_qwen2 as plain
 
 pytestmark = pytest.mark.gpu
 
@@ -92,3 +94,29 @@ def test_replays_have_the_bits_of_eager_steps(folder, dtype, lengths, joined, mo
     for t, (a, b) in enumerate(zip(*seen)):
         assert torch.equal(a, b), f"step {t}"
     assert calls.only(joined)
+
+
+@pytest.mark.parametrize("graphs", [False, True])
+@pytest.mark.parametrize("dtype, lengths, way", [
+    ("bfloat16", [29], "whole"), ("bfloat16", [29, 62], "whole"), ("bfloat16", [310], "merged"), ("bfloat16", [12, 420, 15], "merged"),
+    ("float32", [140], "merged"), ("float32", [12, 420, 15], "merged"), ("float32", [2200], "apart"),  # (35 records)
+])
+def test_plain_logits_and_nan_in_the_pools(folder, dtype, lengths, way, graphs, monkeypatch):
+    """Every page holds NaN, as an earlier request whose activations overflowed leaves it; decoding crosses the edges of pages, where many workgroups
+    read the lines around a new key and value that one of them writes.  The logits are the plain model's."""
+    from from_scratch_inference_engine_amd import load_model
+    from from_scratch_inference_engine_amd.engine.model import Runner
+
+    model, calls, steps = load_model(folder, dtype=dtype), Counted(monkeypatch), 6
+    tokens = [helpers.token_ids(331, n + steps, 80 + n) for n in lengths]
+    refs = [plain.forward_dir(folder, ids).numpy() for ids in tokens]
+    runner = Runner(model, page_size=16, num_pages=sum(n // 16 + 2 for n in lengths), max_requests=4, use_graphs=graphs)
+    k, v, _ = runner.storage.group_stores[0]
+    k[:, 1:] = float("nan")
+    v[:, 1:] = float("nan")
+    out = decode(runner, [ids[:n] for ids, n in zip(tokens, lengths)], [ids[n:] for ids, n in zip(tokens, lengths)], steps)
+    for i, n in enumerate(lengths):
+        got = np.stack([o[i].float().cpu().numpy() for o in out])
+        helpers.assert_close_to_plain(got, refs[i][n:n + steps], dtype, f"request {i} behind {n} tokens")
+    assert calls.only(way), vars(calls)
+    assert (k[:, 0] == 0).all() and (v[:, 0] == 0).all()
