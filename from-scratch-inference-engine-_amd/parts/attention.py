@@ -463,11 +463,11 @@ class AttentionPlanner:
                 n_partial = (n_items + (host.n_seqs if two_pass else 0)) * small_tokens
         single = all(host.q_lens[s] == 1 for s in range(host.n_seqs))  # one token a request
         extra = {}
-        if not padded and single and not self.pool and 0 < len(merges) < host.n_tokens and host.n_tokens * self.n_kv <= self._units():
+        if not padded and single and not self.pool and 0 < len(merges) < host.n_seqs and host.n_seqs * self.n_kv <= self._units():
             # every row once, as a graph merges them (those that need none by an empty merge), for the launch that multiplies by the output
             # projection too: whether it stands for a step must not follow from whether the step is replayed
             merged = {m[0] for m in merges}
-            extra["row_merges"] = np.asarray(merges + [(row, 0, 0, 0) for row in range(host.n_tokens) if row not in merged], dtype=np.int32)
+            extra["row_merges"] = np.asarray(merges + [(row, 0, 0, 0) for row in range(host.n_seqs) if row not in merged], dtype=np.int32)
         # consecutive large tiles of one request, four at a time, for the kernel that shares the
         # keys of a block among four waves
         groups = np.zeros((0, 2), dtype=np.int64)
