@@ -153,8 +153,8 @@ class AttentionPlanner:
 
     def _cut_from(self, first: int, mfma: bool) -> int:
         """Where the runs that a portion's keys are cut into are counted from: the matrix-core kernel takes blocks of 32 keys from a
-        multiple of 32 on, so runs from a window's first key would have a block more each than their keys are."""
-        return first & ~31 if mfma else first
+        multiple of 32 on and the float32 one of 16, so runs from a window's first key would have a block more each than their keys are."""
+        return first & ~31 if mfma else first & ~15
 
     def _small_keys(self, host, small_tokens, mfma: bool):
         """(Keys that it reads, the same from where its runs are counted) of each small portion of the step."""
@@ -516,8 +516,9 @@ class AttentionPlanner:
             # four blocks the sums are the same either way; decode items are cut by the batch as it is)
             "all_waves": not mfma and bool((large[:, 5] - (large[:, 4] & ~15) + np.where(
                 large[:, 7] & ATTN_KEEP_WALK, np.minimum(large[:, 7] & ~(ATTN_KEEP_WALK | ATTN_POOL_WALK), large[:, 4]) + 15 & ~15, 0) > 64).any()),
-            # float32: the items are cut, to no more than four blocks of 16 keys
-            "short_items": not mfma and n_partial > 0 and split_keys <= 64,
+            # float32: the items are cut, to no more than four blocks of 16 keys (of sizes that a graph fixes, not of the step's own items.  Kept first keys
+            # are one item, however many; a request that is whole starts with a chunk, which may lie across a block)
+            "short_items": not mfma and n_partial > 0 and split_keys <= 64 and self.keep_first <= 64 and (self.chunk or 0) % 16 == 0,
             "single": single,
             "few_records": few_records,  # (in a graph: of every step that it stands for)
         }

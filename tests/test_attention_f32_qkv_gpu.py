@@ -95,13 +95,21 @@ def test_refusals(ops):
     (14, 2, 64, 16, 7, True), (16, 1, 128, 8, 3, True), (32, 2, 96, 16, 9, True),  # (sixteen heads of 96 and 128: more columns than four waves have threads)
     (3, 3, 16, 4, 1, False), (20, 1, 64, 16, 2, False)])
 def test_short_items_give_the_same_bits_on_four_waves(ops, heads, kv, hd, page, n_parts, table):
+    short_items_on_four_waves(ops, heads, kv, hd, page, n_parts, table, [0, 5, 15, 16, 63, 64, 200, 330], None)
+
+
+@pytest.mark.parametrize("window", [200, 263, 320])
+def test_short_items_of_a_window_give_the_same_bits_on_four_waves(ops, window):
+    short_items_on_four_waves(ops, 14, 2, 64, 16, 7, True, [0, 199, 206, 330, 471, 600, 601, 1000], window)
+
+
+def short_items_on_four_waves(ops, heads, kv, hd, page, n_parts, table, pasts, window):
     from from_scratch_inference_engine_amd.parts.attention import AttentionPlanner
 
-    pasts = [0, 5, 15, 16, 63, 64, 200, 330]
     t, width = len(pasts), (heads + 2 * kv) * hd
     AttentionPlanner.compute_units = 4096  # (items of 64 keys)
     try:
-        case = paged_case([(p, 1) for p in pasts], heads, kv, hd, page, torch.float32, seed=heads)
+        case = paged_case([(p, 1) for p in pasts], heads, kv, hd, page, torch.float32, seed=heads, window=window)
     finally:
         AttentionPlanner.compute_units = None
     plan = case["plan"]
@@ -116,6 +124,6 @@ def test_short_items_give_the_same_bits_on_four_waves(ops, heads, kv, hd, page, 
     for short in (False, True):
         k, v = case["k_pool"].cuda().clone(), case["v_pool"].cuda().clone()
         out, partials = torch.zeros(t, heads * hd).cuda(), torch.zeros(plan["n_partial"] * heads * (hd + 2)).cuda()
-        ops.attention_mfma_qkv(parts, bias, angles, slots, k, v, bt, items, plan["n_small"], out, partials, heads, kv, hd, None, hd ** -0.5, short_items=short)
+        ops.attention_mfma_qkv(parts, bias, angles, slots, k, v, bt, items, plan["n_small"], out, partials, heads, kv, hd, window, hd ** -0.5, short_items=short)
         got.append((out, partials, k, v))
     assert all(torch.equal(a, b) for a, b in zip(*got)) and got[0][1].abs().max() > 0.1

@@ -335,3 +335,26 @@ def test_an_eager_plan_and_a_graphs_plan_agree_on_what_the_output_projection_joi
     # portions, and steps whose rows are more than the workgroups that a launch has room for, are left alone
     assert "row_merges" not in planner.plan(Host([(600, 1), (10, 40)], 16, dtype))
     assert "row_merges" not in planner.plan(Host([(3, 1)] * 256 + [(9000, 1)], 16, dtype))
+
+
+@pytest.mark.parametrize("args, short", [(dict(window=1024), True), (dict(window=300), True), (dict(window=203), True), (dict(window=None), True), (dict(window=None, chunk=400), True),
+                                         (dict(window=700, keep_first=40), True), (dict(window=700, keep_first=100), False), (dict(window=None, chunk=200), False)])
+def test_short_float32_items_are_four_blocks_of_keys_wherever_a_window_starts(args, short):
+    """The float32 kernel of four waves takes blocks of 16 keys from a multiple of 16 on, one a wave: items of more blocks would be dealt otherwise than
+    by sixteen waves."""
+    rng = random.Random(str(args))
+    planner = AttentionPlanner(14, 2, 64, **args)
+    planner.compute_units = 256
+    seen = 0
+    for _ in range(80):
+        seqs = [(rng.choice([rng.randint(0, 500), rng.randint(0, 5000)]), 1) for _ in range(rng.choice([1, 2, 4, 8]))]
+        host = Host(seqs, 16, torch.float32)
+        plan = planner.plan(host)
+        if not args.get("keep_first") and not args.get("chunk"):
+            check_plan(planner, host, plan)
+        if plan["short_items"]:
+            seen += 1
+            assert plan["n_partial"] and all(-(-(int(it[KE]) - (int(it[KB]) & ~15)) // 16) <= 4 for it in plan["items"]), seqs
+        host.pad = {planner.key: planner.graph_bucket(host)}
+        assert planner.plan(host)["short_items"] == plan["short_items"]
+    assert (seen > 20) == short and (seen > 0) == short
