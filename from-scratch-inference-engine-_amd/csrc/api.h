@@ -336,7 +336,7 @@ int fsie_attention_mfma_qkv_o(const float* sums, int n_parts, int n_tokens, cons
                               int rows_of_wave, int n_heads, int n_kv, int head_dim, int page_size, int window, float scale,
                               hipStream_t stream);
 // fsie_attention_merge with the output projection behind it (rows_of_wave as above)
-int fsie_attention_merge_o_rows(int n_merges, int n_heads, int n_kv, int head_dim, int o_rows, int units);
+int fsie_attention_merge_o_rows(int n_merges, int n_heads, int n_kv, int head_dim, int o_rows, int dtype, int units);
 int fsie_attention_merge_o(const float* partials, const int32_t* merges, int n_merges, int n_tokens, const void* heads, const void* o_weight,
                            int o_rows, float* o_sums, int rows_of_wave, int n_heads, int n_kv, int head_dim, int dtype, hipStream_t stream);
 int fsie_attention_mfma_lds_ok(int head_dim, int page_size);

@@ -158,10 +158,19 @@ __global__ __launch_bounds__(64 * kMergeWaves) void attention_merge_o_kernel(
 }  // namespace
 
 // Rows of the output projection a wave, for n_merges tokens; 0: the merge and the projection are better two launches, or there is no kernel.  As few as leave
-// no more workgroups than units.
-extern "C" int fsie_attention_merge_o_rows(int n_merges, int n_heads, int n_kv, int head_dim, int o_rows, int units) {
-    if (n_merges <= 0 || n_heads <= 0 || n_kv <= 0 || n_heads % n_kv || n_heads / n_kv > 16 || o_rows <= 0 || units <= 0) return 0;
-    if (head_dim != 64 && head_dim != 128) return 0;
+// no more workgroups than units (which bounds the weight that is read, once a token, to 34 MB for groups of eight heads of 128 in float32).
+// Groups of more than eight heads give a wave two to merge, one after the other, in every workgroup: they gain less, and lose from three tokens on, in float32
+// from two, and beyond 12 heads.  16 steps behind 400 / 1,500 keys, one launch over two:
+//   up to 8 heads   0.92 to 1.00 at every size and number of tokens (1,024 wide, 8 on 1 of 128, one token 0.94 / 0.94, four 0.98 / 0.98; float32 0.98 / 0.98 and 0.99 / 0.99; 2,048
+//                   wide, 16 on 2 of 128, one 0.98 / 0.97; float32 2,560 wide, 8 on 1, two 1.00 / 1.00)
+//   10 and 12       one token 0.93 to 0.99 (1,536 wide, 12 on 1 of 128, 0.93 / 0.94), two 0.94 to 0.99, four 1.01 / 1.01 (1,280 wide, 10 on 1) and 0.99 / 1.00; float32 one 0.98 / 0.99
+//                   to 1.00, two 0.98 / 1.01, four 1.01 / 1.01
+//   16              one token 0.97 to 1.01 (2,048 wide, 16 on 1 of 128, 1.01 / 1.01; 32 on 2 of 64 1.01 / 1.00; 4,096 wide, 32 on 2 of 128, 0.98 / 0.99), four 1.02 / 1.02; float32 0.99 / 1.01 to 1.00 / 1.02
+extern "C" int fsie_attention_merge_o_rows(int n_merges, int n_heads, int n_kv, int head_dim, int o_rows, int dtype, int units) {
+    if (n_merges <= 0 || n_heads <= 0 || n_kv <= 0 || n_heads % n_kv || o_rows <= 0 || units <= 0) return 0;
+    if ((head_dim != 64 && head_dim != 128) || (dtype != FSIE_F32 && dtype != FSIE_BF16)) return 0;
+    const int group = n_heads / n_kv;
+    if (group > kMergeWaves && (group > 12 || n_merges > (dtype == FSIE_F32 ? 1 : 2))) return 0;
     for (int rows = 1; rows <= 4; ++rows)
         if (ceil_div64(o_rows, kMergeWaves * rows) * n_kv * n_merges <= units) return rows;
     return 0;

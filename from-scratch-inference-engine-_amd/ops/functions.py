@@ -1236,9 +1236,10 @@ def attention_merge(partials: torch.Tensor, merges: torch.Tensor, n_merges: int,
     return out
 
 
-def attention_merge_o_rows(n_merges: int, n_heads: int, n_kv: int, head_dim: int, n: int) -> int:
-    """Rows of an output projection of ``n`` rows a wave, where it is faster in the launch of the merge (``attention_merge_o``); else 0."""
-    return int(load().fsie_attention_merge_o_rows(n_merges, n_heads, n_kv, head_dim, n, compute_units()))
+def attention_merge_o_rows(n_merges: int, n_heads: int, n_kv: int, head_dim: int, n: int, dtype: torch.dtype = torch.bfloat16) -> int:
+    """Rows of an output projection of ``n`` rows a wave, where it is faster in the launch of the merge (``attention_merge_o``); else 0.  ``dtype``: the
+    weight's."""
+    return int(load().fsie_attention_merge_o_rows(n_merges, n_heads, n_kv, head_dim, n, dtype_code(dtype), compute_units()))
 
 
 def attention_merge_o(partials: torch.Tensor, merges: torch.Tensor, n_merges: int, heads: torch.Tensor, o_weight: torch.Tensor, o_rows: int,

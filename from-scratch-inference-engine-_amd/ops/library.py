@@ -71,7 +71,7 @@ _SIGNATURES = {
     "fsie_attention_mfma_qkv_ok": ([c_int, c_int], c_int),
     "fsie_attention_mfma_qkv": ([_P, c_int, c_int, _P, _P, _P, _P, _P, c_int64, _P, c_int, _P, c_int, _P, _P, c_int,
                                  c_int, c_int, c_int, c_int, c_float, c_int, _P, _P, _P], c_int),
-    "fsie_attention_merge_o_rows": ([c_int, c_int, c_int, c_int, c_int, c_int], c_int),
+    "fsie_attention_merge_o_rows": ([c_int, c_int, c_int, c_int, c_int, c_int, c_int], c_int),
     "fsie_attention_merge_o": ([_P, _P, c_int, c_int, _P, _P, c_int, _P, c_int, c_int, c_int, c_int, c_int, _P], c_int),
     "fsie_attention_mfma_qkv_o_rows": ([c_int, c_int, c_int, c_int, c_int, c_int, c_int], c_int),
     "fsie_attention_mfma_qkv_o": ([_P, c_int, c_int, _P, _P, _P, _P, _P, c_int64, _P, c_int, _P, c_int, _P, c_int, _P, c_int,

@@ -852,7 +852,7 @@ class GQAttention(Mixer):
         if plan.n_partial:
             # cut items: the launch that merges them makes it, where every token has few records
             every_row = plan.n_merges == x.shape[0] or hasattr(plan, "row_merges")
-            return ops.attention_merge_o_rows(rows, self.n_heads, self.n_kv, self.head_dim, self.hidden_size) if plan.few_records and every_row else 0
+            return ops.attention_merge_o_rows(rows, self.n_heads, self.n_kv, self.head_dim, self.hidden_size, x.dtype) if plan.few_records and every_row else 0
         if plan.waves != 1 or x.dtype != torch.bfloat16:
             return 0
         return ops.attention_mfma_qkv_o_rows(rows, self.n_heads, self.n_kv, self.head_dim, cache.page_size, self.hidden_size)

@@ -60,3 +60,30 @@ def test_rule_and_refusals(ops):
     for bad in (dict(rows=0), dict(rows=5), dict(hd=96, cols=192), dict(heads=17, cols=17 * 64), dict(cols=64), dict(dtype=torch.float32)):
         with pytest.raises(ops.KernelError):
             call(**bad)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads, kv, hd, n, splits", [(14, 2, 64, 40, [65, 4]), (20, 2, 128, 24, [94, 5, 5]), (12, 1, 64, 9, [128]), (9, 1, 128, 8, [64, 0, 33])])
+def test_more_records_than_a_wave_has_lanes(ops, dtype, heads, kv, hd, n, splits):
+    """Sixty-four records are read at a time; the second head of a wave (groups of more than eight) asks for its own.  Against 64 bits: beyond 32 records the merge
+    by itself adds up in another order."""
+    t, g, slots = len(splits), torch.Generator().manual_seed(heads), sum(splits)
+    records = torch.randn(slots, heads, hd + 2, generator=g)
+    records[..., hd + 1] = records[..., hd + 1].abs() + 0.5
+    merges = torch.tensor([(r, sum(splits[:r]), splits[r], 1) for r in range(t)], dtype=torch.int32).cuda()
+    weight = torch.randn(n, heads * hd, generator=g).to(dtype).cuda()
+    whole = torch.randn(t, heads * hd, generator=g).to(dtype)
+    got = ops.attention_merge_o(records.reshape(-1).cuda(), merges, t, whole.cuda(), weight, 1, heads, kv, hd).double().cpu()
+    x, off = whole.double().view(t, heads, hd), torch.zeros(t, heads, hd, dtype=torch.float64)
+    for r, count in enumerate(splits):
+        if count:
+            mine = records[sum(splits[:r]):sum(splits[:r]) + count].double()
+            share = torch.exp(mine[..., hd] - mine[..., hd].amax(0))
+            denom = (share * mine[..., hd + 1]).sum(0)[:, None]
+            x[r] = (share[..., None] * mine[..., :hd]).sum(0) / denom
+            # (float32 sums of `count` products, their factors a few roundings each; then the heads' own rounding)
+            off[r] = (share[..., None] * mine[..., :hd].abs()).sum(0) / denom * (count + 32) * 2.0 ** -23 + x[r].abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 0)
+    by_kv = lambda a: a.reshape(t, kv, -1).transpose(0, 1)
+    w = weight.double().cpu().view(n, kv, -1).permute(1, 2, 0)
+    bound = (by_kv(x.abs() + off) @ w.abs()) * (heads // kv * hd) * 2.0 ** -24 + by_kv(off) @ w.abs() + 1e-30
+    assert ((got - by_kv(x) @ w).abs() <= bound).all()

@@ -233,3 +233,17 @@ def test_only_steps_of_few_rows_ask_whether_a_norm_may_wait(rows, asked):
     hidden = HiddenState(SimpleNamespace(shape=(rows, 8)))
     PreNormBlock(Norm(), part, Norm(), part).forward(hidden, SimpleNamespace(compute_dtype=torch.bfloat16, sums_in_one=False), None)
     assert order == ["norm", "part", "norm", "part"] and hidden.delta == 4 and len(questions) == asked
+
+
+def test_the_merge_makes_the_output_projection_where_a_wave_has_one_head_or_tokens_are_few():
+    """Every workgroup merges its kv head's records again: groups of more heads than a workgroup has waves are slower from three tokens on (float32:
+    two), and beyond 12 heads."""
+    from from_scratch_inference_engine_amd import ops
+    from from_scratch_inference_engine_amd.ops.functions import dtype_code
+
+    rows = lambda t, heads, kv, hd, n, dtype=torch.bfloat16: ops.load().fsie_attention_merge_o_rows(t, heads, kv, hd, n, dtype_code(dtype), 256)
+    assert [rows(t, 14, 2, 64, 896) for t in (1, 2, 3, 4, 5)] == [1, 2, 3, 4, 0]
+    assert [rows(t, 8, 1, 128, 1024) for t in (1, 4, 8)] == [1, 2, 4] and [rows(t, 8, 1, 128, 1024, torch.float32) for t in (1, 4, 8)] == [1, 2, 4]
+    assert [rows(t, 12, 1, 128, 1536) for t in (1, 2, 3, 4)] == [1, 2, 0, 0] and [rows(t, 12, 1, 128, 1536, torch.float32) for t in (1, 2)] == [1, 0]
+    assert rows(1, 16, 1, 128, 2048) == rows(2, 16, 1, 128, 2304) == rows(1, 13, 1, 64, 512) == 0
+    assert rows(1, 14, 2, 96, 896) == rows(0, 14, 2, 64, 896) == 0
