@@ -68,7 +68,8 @@ def kernel_classes(runner, cfg, batch: int, prompt_len: int, itemsize: int) -> d
     """Time of each class of kernels of one decode step: the calls of an eagerly run step are
     recorded (kernel, operands), and each class's calls, over all layers with each layer's own
     weights, are captured into a graph of their own and timed with events around its replays.
-    GB/s = the weights (for attention: the live cache) the class reads once a step / its time."""
+    GB/s = the weights (for attention: the live cache, and the output projection where attention's launches make it) the class reads
+    once a step / its time."""
     import torch
 
     from from_scratch_inference_engine_amd import ops
@@ -94,12 +95,13 @@ def kernel_classes(runner, cfg, batch: int, prompt_len: int, itemsize: int) -> d
         "gemm_mfma_skinny_rope": lambda a, k: "qkv", "rope_kv_write": lambda a, k: "qkv", "bias_add": lambda a, k: "qkv",
         "attention_mfma": lambda a, k: "attention", "attention_mfma_lds": lambda a, k: "attention",
         "attention_mfma_qkv": lambda a, k: "attention",
-        "attention_scalar": lambda a, k: "attention", "attention_merge": lambda a, k: "attention",
+        "attention_scalar": lambda a, k: "attention", "attention_merge": lambda a, k: "attention", "attention_merge_o": lambda a, k: "attention",
         "gemm_mfma_skinny": lambda a, k: matrix_class(a[1]), "gemm_mfma_wide": lambda a, k: matrix_class(a[1]),
         "gemm_mfma_wide_swiglu": lambda a, k: "gate_up", "gemm_mfma_stream": lambda a, k: matrix_class(a[1]),
         "gemm_mfma_block": lambda a, k: matrix_class(a[1]), "gemm_mfma_normed": lambda a, k: matrix_class(a[5]),
         "gemm": lambda a, k: matrix_class(a[1]), "gemm_mfma_fp32": lambda a, k: matrix_class(a[1]),
         "gemm_mfma_fp32_sums": lambda a, k: matrix_class(a[1]), "gemm_fp32_tile": lambda a, k: matrix_class(a[1]),
+        "gemm_fp32_stream": lambda a, k: matrix_class(a[1]), "gemm_fp32_gated": lambda a, k: "gate_up",
         "gemm_mfma_tile": lambda a, k: matrix_class(a[1]), "gemm_mfma_tile_gated": lambda a, k: "gate_up",
         "library_mm": lambda a, k: matrix_class(a[1]),
         "swiglu": lambda a, k: "gate_up", "rmsnorm": lambda a, k: "norms", "embedding": lambda a, k: "other",
@@ -133,9 +135,10 @@ def kernel_classes(runner, cfg, batch: int, prompt_len: int, itemsize: int) -> d
     weights = {"qkv": h * (q + 2 * cfg.num_key_value_heads * cfg.head_dim), "o": q * h, "gate_up": 2 * h * inter,
                "down": h * inter}
     n_layers = sum(1 for c in calls if c[0] == "down")  # (one product a layer, whichever kernel takes it)
+    joined = sum(1 for _, fn, _, k in calls if fn is saved["attention_merge_o"] or k.get("o_weight") is not None)  # layers whose attention makes the output projection
     read = {k: n * itemsize * n_layers for k, n in weights.items()}
     read["lm_head"] = h * v * itemsize
-    read["attention"] = batch * (prompt_len + 1) * 2 * cfg.num_key_value_heads * cfg.head_dim * itemsize * n_layers
+    read["attention"] = batch * (prompt_len + 1) * 2 * cfg.num_key_value_heads * cfg.head_dim * itemsize * n_layers + weights["o"] * itemsize * joined
     out = {}
     # The recorded step and the prompts before it are only queued so far.  Every call below reads that
     # step's tables and intermediate tensors, so they must be complete first; and the calls run on the

@@ -300,6 +300,20 @@ def test_bench_prints_its_line():
     assert two.returncode == 2 and len(two.stdout.strip().splitlines()) == 1
 
 
+@pytest.mark.parametrize("batch, joined", [(4, True), (8, False)])
+def test_bench_knows_the_classes_of_a_float32_step(batch, joined):
+    """Every product of a float32 decode step is in its class, with the weight that it reads: of four requests behind some 500 tokens the output projection is in
+    the merge's launch and so in attention's class, of eight it is a launch of its own."""
+    cmd = [sys.executable, "bench.py", "--shape", "0.5b", "--layers", "2", "--steps", "4", "--warmup", "2", "--dtype", "fp32", "--no-points", "--batch", str(batch)]
+    proc = subprocess.run(cmd, capture_output=True, text=True, timeout=300, cwd=str(helpers.ROOT))
+    assert proc.returncode == 0, proc.stderr[-3000:]
+    kernels = json.loads(proc.stdout.strip().splitlines()[-1])["kernels"]
+    print(kernels)
+    for cls in ["attention", "qkv", "gate_up", "down", "lm_head"] + ([] if joined else ["o"]):
+        assert kernels[cls]["GB/s"] > 0 and kernels[cls]["launches"] > 0, (cls, kernels)
+    assert ("o" in kernels) != joined and "other" in kernels
+
+
 def test_graph_replays_equal_eager_steps(model_dirs):
     """Decode steps run as replayed graphs.  Two runners over the same model, one with graphs and
     one without, decode the same 20 requests (more rows than the engine's own small-matrix kernel
