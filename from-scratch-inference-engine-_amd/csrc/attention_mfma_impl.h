@@ -49,7 +49,9 @@
 // [n_kv][tokens][o_rows], one slice a kv head, for the norm that adds them up.  One request of the 0.5B shape and 30 to 100 keys: attention and
 // projection 8.6 -> 6.8 us a layer, the step 565 -> 520; two requests 591 -> 562.  Where the workgroups are more than the units attention is made
 // in turns and the two launches are faster (the rule is fsie_attention_mfma_qkv_o_rows), and so it is with items of more waves (600
-// keys 17.3 ms for 24 steps, 16.1 cut and merged).
+// keys 17.3 ms for 24 steps, 16.1 cut and merged).  The widest form (heads of 128, four rows a wave: a unit holds five waves, so 256 registers a wave, and 64 of
+// them are the weight's) keeps 16 registers in scratch, 36 bytes a lane; it is faster than the two launches all the same: 16 steps of one request, ms, 2,048 wide, 16 on 2 of
+// 128 6.49 / 6.35, 2,560 wide, 20 on 2 7.03 / 6.89, 1,024 wide, 16 on 4 5.95 / 5.58, two requests 2,560 wide, 8 on 1 6.96 / 6.80.
 #pragma once
 
 #include "common.h"
