@@ -1,8 +1,8 @@
 // The merge of a decode step's cut items (attention_merge, attention_scalar.hip) with the output projection behind it, for a few tokens.
 //
 // Such a step is bound by its launches: the merge of a few records a head is 2.3 to 4 us, nearly all of it the launch and one trip to memory, and the
-// projection behind it as much.  Here a workgroup takes a kv head of a token: a wave merges a head (the arithmetic and the order of attention_merge), the heads, rounded to
-// 16 bits where the heads are, meet in LDS, and each wave multiplies them by ROWS rows of the projection, which it has asked for behind the records.  Every workgroup of a kv head
+// projection behind it as much.  Here a workgroup takes a kv head of a token: a wave merges a head (the arithmetic of attention_merge, and up to 32 records its order: more
+// are dealt to four waves there), the heads, rounded to 16 bits where the heads are, meet in LDS, and each wave multiplies them by ROWS rows of the projection, which it has asked for behind the records.  Every workgroup of a kv head
 // merges the same records again (2 KB a split for seven heads of 64), which costs less than a launch while all workgroups are on the chip at once.
 // The result is float32 sums [n_kv][tokens][o_rows], a slice a kv head, for the norm that adds them up.
 // 24 steps, ms, two launches / this: one request of the 0.5B shape (24 layers) behind 300 keys 16.09 / 15.12, 600 16.28 / 15.04, 2,000 18.06 / 16.70, two behind 400 16.45 / 15.69, behind

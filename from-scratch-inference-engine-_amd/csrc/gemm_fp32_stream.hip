@@ -7,7 +7,7 @@
 // eight steps under way at once: one trip.  A longer K goes four steps at a time with the next four under way.  The waves' shares meet in LDS and are
 // added in the order of the waves; a share is at most eight steps, 128 values, before it is added to the ones behind it, which leaves half the rounding
 // errors of runs of 512 (relative error of K = 896 3.9e-7 -> 2.0e-7, K = 4864 in eight slices 2.2e-7 -> 1.7e-7).
-// As there a row's sums depend on N, K and the number of tiles of 16 rows, never on what the other rows hold.
+// As there a row's sums depend on N, K, the number of tiles of 16 rows and whether the step has one or two rows (the plan below), never on what the other rows hold.
 //
 // MI355X, us, cold weights, rows of W before / this, 4 rows: gate and up with their product N = 9728, K = 896 (35 MB) 11.2 / 9.2, N = 16384, K = 2048 39.3 / 26.2,
 // N = 37888, K = 3584 104 / 91; sums with the norm that adds them up N = 896, K = 4864 9.3 / 7.6, N = 896, K = 896 5.7 / 5.0, N = 2048, K = 8192 22.8 / 15.9,
@@ -163,8 +163,8 @@ int launch_result(bool gated, int waves, int s, const StreamCall& c, hipStream_t
 
 }  // namespace
 
-// How M rows of this product are best taken, or -1 where the kernels that read rows of W are the better ones: waves + 256 * slices of K.  By N, K and
-// the tiles of 16 rows alone.  result 0: whole; 1: gate and up in turn; 2: partial sums for a norm that adds them up, or whole (one slice).
+// How M rows of this product are best taken, or -1 where the kernels that read rows of W are the better ones: waves + 256 * slices of K.  By N, K,
+// the tiles of 16 rows, and of one or two rows whether the vector kernel is the better one.  result 0: whole; 1: gate and up in turn; 2: partial sums for a norm that adds them up, or whole (one slice).
 // Whole: eight waves where they hold K at once (K up to 1,024), else sixteen where the units have no workgroup each (N = 3072, K = 1536 6.0 us, with four 6.5;
 // N = 4096, K = 2048 8.1 / 8.3), else four, of which a unit holds several (N = 16384, K = 2048 26.2, with 16 27.8; N = 37888, K = 3584 91 / 118;
 // N = 3584, K = 3584 11.5 / 13.0).  From 33 rows on the matrix instruction bounds a short K and this is no faster (N = 9728, K = 896 25.8 / 24.7 at 48

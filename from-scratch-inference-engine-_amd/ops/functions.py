@@ -1097,7 +1097,7 @@ def attention_mfma_qkv_o_rows(n_items: int, n_heads: int, n_kv: int, head_dim: i
 
 
 def attention_f32_qkv_ok(head_dim: int, page_size: int) -> bool:
-    """The same of float32 storage (``attention_qkv`` takes both)."""
+    """The same of float32 storage (``attention_mfma_qkv`` takes both)."""
     return 0 < head_dim <= 128 and head_dim % 16 == 0 and page_size > 0 and page_size % 4 == 0
 
 

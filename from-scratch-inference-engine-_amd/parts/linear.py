@@ -32,7 +32,10 @@ class Linear:
     the library product (hipBLASLt through torch, where the reference's engine calls cuBLAS) with
     float32 accumulation, the bias added by a kernel of the engine.  A large weight has a second copy in
     the order of the matrix instruction's fragments (``prepare``, ``streamed``), from which the
-    sibling takes every product of up to 64 rows."""
+    sibling takes every product of up to 64 rows.
+
+    The copies hold what the weight was when ``prepare`` ran: setting ``weight`` drops them, and after a change of the weight's
+    values in place ``prepare`` is called again (or ``drop_copy``), in either precision."""
 
     narrow_to = 64  # float32 results of at most this many outputs from bfloat16 operands: the narrow kernel
     float32_on_matrix_cores = True  # 3 rows of float32 and more: v_mfma_f32_16x16x4_f32 instead of vector FMAs
