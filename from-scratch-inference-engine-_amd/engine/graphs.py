@@ -81,6 +81,7 @@ class DecodeGraphs:
         self.replays = 0
         self.captures = 0
         self._host = None  # the host view that shape_of made, for the step that follows
+        self._copies_dropped = model.copies_dropped
 
     @property
     def runner(self):
@@ -122,6 +123,10 @@ class DecodeGraphs:
         and is not due for one yet (the caller then runs the step eagerly).  ``feed`` (int32, on
         the device) replaces the token ids after the tables have been sent."""
         runner = self.runner
+        if self._copies_dropped != runner.model.copies_dropped:
+            # another runner's cache has taken the memory of the weights' second copies, which the captured products read
+            self._graphs.clear()
+            self._copies_dropped = runner.model.copies_dropped
         n = len(entries)
         entries = self.filled_up(entries)
         host, self._host = self._host, None

@@ -169,6 +169,8 @@ class Model:
             prepare_parts(part, self.device, self.dtype, self.options, seen)
         self.partial_sums_ok = all(norm.adds_partial_sums for norm in self.spec.stream_norms())
 
+    copies_dropped = 0  # how often the second copies have gone: graphs captured before read memory that is no longer theirs
+
     # ---------------------------------------------------------------- cache
     def make_cache(self, page_size: int, num_pages: int, max_requests: int):
         """The cache's host and device side.  The second copies of the large weights were made before
@@ -181,6 +183,7 @@ class Model:
             freed = sum(part.release_optional_memory() for part in self.spec.all_parts())
             if not freed:
                 raise
+            self.copies_dropped += 1
             torch.cuda.empty_cache()
             import warnings
 

@@ -693,6 +693,48 @@ def test_a_cache_that_does_not_fit_beside_the_weight_copies_drops_them(tmp_path,
     assert without == with_copies  # (the products on the copy and on rows give the same bits)
 
 
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_a_runner_whose_graphs_read_copies_that_another_one_has_dropped(tmp_path, monkeypatch, dtype):
+    """Two runners over one model: the second one's cache does not fit beside the copies (made to fail from the host), so they go; the first
+    captures its steps anew, from rows."""
+    import warnings
+
+    from from_scratch_inference_engine_amd import LLM, GenerationConfig
+    from from_scratch_inference_engine_amd.cache import storage as storage_module
+    from from_scratch_inference_engine_amd.engine.model import Runner
+    from from_scratch_inference_engine_amd.parts.linear import Linear
+
+    monkeypatch.setattr(Linear, "streamed_copy_from", 0)
+    monkeypatch.setattr(Linear, "streamed32_copy_from", 0)
+    cfg = dict(helpers.TINY_B, hidden_size=256, num_attention_heads=8, head_dim=32, intermediate_size=384)
+    d = helpers.make_model_dir(tmp_path / "m", cfg, seed=5)
+    llm = LLM(d, dtype=dtype, block_size=8, num_blocks=32, max_batch=4, eos_id=-1)
+    o, graphs = llm.model.spec.layers[0].mixer.o, llm.engine.runner.graphs
+    assert (o.streamed if dtype == "bfloat16" else o.streamed32) is not None
+    prompts = [helpers.token_ids(509, n, 1600 + n) for n in (5, 19)]
+    gen = GenerationConfig(max_tokens=10, temperature=0.0)
+    with_copies = llm.generate_ids_batch(prompts, gen)
+    captures = graphs.captures
+    assert captures and graphs.replays
+    assert llm.generate_ids_batch(prompts, gen) == with_copies and graphs.captures == captures
+
+    real_init, failed = storage_module.CacheStorage.__init__, []
+
+    def init(self, *a, **k):
+        if not failed:
+            failed.append(1)
+            raise torch.cuda.OutOfMemoryError("(the test says so)")
+        real_init(self, *a, **k)
+
+    monkeypatch.setattr(storage_module.CacheStorage, "__init__", init)
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        other = Runner(llm.model, page_size=8, num_pages=32, max_requests=4)
+    assert failed and o.streamed is None and o.streamed32 is None
+    assert llm.generate_ids_batch(prompts, gen) == with_copies and graphs.captures > captures
+    assert other.graphs is not graphs
+
+
 def test_prefill_with_the_library_kernel_selection(model_dirs):
     """With tuning on, a prompt portion of a multiple of 256 rows, and a decode batch of a multiple
     of 16, let torch time the library's candidates for their products; whatever it picks, the

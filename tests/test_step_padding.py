@@ -55,3 +55,27 @@ def test_the_collector_is_off_until_the_last_capture_ends(was_on):
         assert gc.isenabled() == was_on
     finally:
         (gc.enable if before else gc.disable)()
+
+
+def test_graphs_go_with_the_weight_copies_that_they_read():
+    """A second runner whose cache does not fit beside the second copies of the weights takes their memory; what the first runner has captured
+    reads them, so none of it may be replayed again."""
+    from from_scratch_inference_engine_amd.engine.graphs import DecodeGraphs
+
+    class Runner:
+        model = SimpleNamespace(spec=SimpleNamespace(all_parts=lambda: []), planners=[], copies_dropped=0)
+        storage = SimpleNamespace(spare_slot=0, spare_pages=[], tokens_per_page=[])
+
+    class Captured:
+        def replay(self):
+            raise AssertionError("replayed")
+
+    runner = Runner()
+    graphs = DecodeGraphs(runner, capture_after=3)
+    graphs._graphs[(1, ("pages", 32))] = (Captured(), None, None, None)
+    runner.model.copies_dropped += 1
+    entry = SimpleNamespace(tokens=(1,), want=(0,), cache=SimpleNamespace(tables=[], length=3, slot=0))
+    assert graphs.step([entry], {"pages": 32}) is None and not graphs._graphs
+    graphs._graphs[(1, ("pages", 32))] = "a new one"
+    graphs.step([entry] * 2, {"pages": 32})
+    assert graphs._graphs  # (once for each time that they go)
